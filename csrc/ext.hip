@@ -25,11 +25,12 @@ hipError_t lfmq_kv_append(void*, void*, const void*, const void*, int, int,
                           int, int, int, int, hipStream_t);
 hipError_t lfmq_attn_decode(const void*, const void*, const void*, void*,
                             void*, int, int, int, int, int, const void*, int,
-                            float, hipStream_t);
+                            int, float, hipStream_t);
 hipError_t lfmq_attn_decode_fused(const void*, void*, void*, void*, void*,
                                   const void*, int, int, int, int, int,
-                                  const void*, int, float, void*,
+                                  const void*, int, int, float, void*,
                                   hipStream_t);
+int lfmq_attn_decode_splits(int, int, int, int);
 hipError_t lfmq_attn_prefill(const void*, const void*, const void*, void*,
                              int, int, int, int, int, int, int, float,
                              hipStream_t);
@@ -241,8 +242,9 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
   const int b = (int)q.size(0), hq = (int)q.size(1), d = (int)q.size(3);
   const int hkv = (int)kc.size(1), tmax = (int)kc.size(2);
   // graph mode (t_dev set): seq_len is MAX T; grid fixed, T read on device
-  const int nchunks = ((int)seq_len + 255) / 256;
-  auto scratch = torch::empty({(long)b * hq * nchunks * (d + 2)},
+  TORCH_CHECK(hq % hkv == 0, "query heads must share key heads evenly");
+  const int splits = lfmq_attn_decode_splits(b, hq, hkv, (int)seq_len);
+  auto scratch = torch::empty({(long)b * hq * splits * (d + 2)},
                               q.options().dtype(torch::kFloat32));
   auto o = torch::empty_like(q);
   const void* tptr = nullptr;
@@ -252,8 +254,8 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
   }
   CHECK_HIP(lfmq_attn_decode(q.data_ptr(), kc.data_ptr(), vc.data_ptr(),
                              o.data_ptr(), scratch.data_ptr(), b, hq, hkv,
-                             tmax, (int)seq_len, tptr, d, (float)scale,
-                             stream()));
+                             tmax, (int)seq_len, tptr, d, splits,
+                             (float)scale, stream()));
   return o;
 }
 
@@ -449,8 +451,9 @@ torch::Tensor attn_decode_fused(torch::Tensor qkv, torch::Tensor kc,
   check_t(inv_freq, torch::kFloat32, "inv_freq");
   const int b = (int)kc.size(0), hkv = (int)kc.size(1);
   const int tmax = (int)kc.size(2), d = (int)kc.size(3);
-  const int nchunks = ((int)seq_len + 63) / 64;  // fused path: FCH = 64
-  auto scratch = torch::empty({(long)b * hq * nchunks * (d + 2)},
+  TORCH_CHECK(hq % hkv == 0, "query heads must share key heads evenly");
+  const int splits = lfmq_attn_decode_splits(b, (int)hq, hkv, (int)seq_len);
+  auto scratch = torch::empty({(long)b * hq * splits * (d + 2)},
                               qkv.options().dtype(torch::kFloat32));
   auto o = torch::empty({(long)b, 1L, hq * (long)d}, qkv.options());
   const void* tptr = nullptr;
@@ -465,7 +468,7 @@ torch::Tensor attn_decode_fused(torch::Tensor qkv, torch::Tensor kc,
                                    vc.data_ptr(), o.data_ptr(),
                                    scratch.data_ptr(), inv_freq.data_ptr(), b,
                                    (int)hq, hkv, tmax, (int)seq_len, tptr, d,
-                                   (float)scale, tk, stream()));
+                                   splits, (float)scale, tk, stream()));
   return o;
 }
 

@@ -388,6 +388,48 @@ def test_attn_decode_fused_multichunk():
     assert rel_err(o2.reshape(b, hq, 1, d), o_ref) < 2e-2
 
 
+@pytest.mark.parametrize("b,T,hq,hkv,d", [
+    (1, 1, 4, 4, 128), (2, 32, 4, 2, 64), (1, 33, 8, 2, 128),
+    (3, 256, 8, 1, 128), (1, 257, 16, 1, 64), (2, 513, 6, 2, 128),
+    (1, 3000, 12, 1, 128)])
+def test_attn_decode_key_ranges(b, T, hq, hkv, d):
+    """Edges of key tiles, ranges and head tiles, T from the device, twice
+    (tickets).  Rows that a step may not read hold NaN: the later ones and
+    the new key's own, which the launch writes.  Both sides multiply bf16
+    operands in fp32, so they part by the rounding of q, k and o: 3 * 2^-9."""
+    import lfmq_hip
+    torch.manual_seed(T)
+    tmax = T + 70
+    qkv = torch.randn(b, (hq + 2 * hkv) * d).to(torch.bfloat16)
+    kc = torch.randn(b, hkv, tmax, d).to(torch.bfloat16)
+    vc = torch.randn(b, hkv, tmax, d).to(torch.bfloat16)
+    qr, kr, vr = qkv.split([hq * d, hkv * d, hkv * d], dim=-1)
+    pos = torch.tensor([T - 1])
+    q = ref.apply_rope(qr.reshape(b, 1, hq, d).float(), pos)
+    kc[:, :, T - 1] = ref.apply_rope(kr.reshape(b, 1, hkv, d).float(),
+                                     pos)[:, 0].to(torch.bfloat16)
+    vc[:, :, T - 1] = vr.reshape(b, hkv, d)
+    want = ref.attn_decode(q.transpose(1, 2), kc.float(), vc.float(), T,
+                           d ** -0.5)
+    kg, vg = kc.to(DEV), vc.to(DEV)
+    kg[:, :, T - 1:] = float("nan")
+    vg[:, :, T - 1:] = float("nan")
+    inv = ref.rope_freqs(d, 500000.0).to(DEV)
+    tk = torch.zeros(b * hq, dtype=torch.int32, device=DEV)
+    st = torch.tensor([T], dtype=torch.int32, device=DEV)
+    for _ in range(2):
+        o = lfmq_hip.attn_decode_fused(qkv.to(DEV), kg, vg, tmax, d ** -0.5,
+                                       inv, hq, st, tk)
+        assert rel_err(o.reshape(b, hq, 1, d), want) < 6e-3
+    assert int(tk.abs().sum()) == 0
+    assert rel_err(kg[:, :, T - 1], kc[:, :, T - 1]) < 4e-3
+    assert torch.equal(vg[:, :, T - 1].cpu(), vc[:, :, T - 1])
+    o = lfmq_hip.attn_decode(q.transpose(1, 2).to(torch.bfloat16)
+                             .contiguous().to(DEV), kg, vg, T, d ** -0.5,
+                             None)
+    assert rel_err(o, want) < 6e-3
+
+
 @pytest.mark.parametrize("m", [5, 8, 16])
 @pytest.mark.parametrize("n,k,g", [(256, 2048, 128), (100, 512, 64),
                                    (48, 4096, 128)])
