@@ -35,6 +35,9 @@ hipError_t lfmq_attn_prefill(const void*, const void*, const void*, void*,
                              int, int, int, int, int, int, int, float,
                              hipStream_t);
 hipError_t lfmq_hessian_accum(const void*, void*, int, int, hipStream_t);
+hipError_t lfmq_gptq_block(const void*, const void*, void*, void*, void*,
+                           void*, int, int, int, int, int, int, int, bool,
+                           hipStream_t);
 hipError_t lfmq_dq_gemv_gateup(const void*, const void*, const void*,
                                const void*, void*, int, int, int, int, int,
                                float, int, hipStream_t);
@@ -545,6 +548,32 @@ void hessian_accum(torch::Tensor h, torch::Tensor x) {
   CHECK_HIP(lfmq_hessian_accum(x.data_ptr(), h.data_ptr(), t, k, stream()));
 }
 
+// one column block of the GPTQ solve; returns its errors [n, nb]
+torch::Tensor gptq_block(torch::Tensor w, torch::Tensor ub,
+                         torch::Tensor codes, torch::Tensor scales,
+                         torch::Tensor zeros, long i1, long g, long bits,
+                         bool sym) {
+  check_t(w, torch::kFloat32, "w");
+  check_t(ub, torch::kFloat32, "ub");
+  check_t(codes, torch::kInt32, "codes");
+  check_t(scales, torch::kFloat32, "scales");
+  check_t(zeros, torch::kInt32, "zeros");
+  TORCH_CHECK(w.dim() == 2 && ub.dim() == 2 && ub.size(0) == ub.size(1),
+              "w [n, k], ub [nb, nb]");
+  const long n = w.size(0), k = w.size(1), nb = ub.size(0);
+  TORCH_CHECK(codes.sizes() == w.sizes(), "codes must be [n, k]");
+  TORCH_CHECK(g > 0 && k % g == 0 && scales.numel() == n * (k / g) &&
+                  zeros.numel() == n * (k / g),
+              "scales and zeros must be [n, k / g]");
+  auto err = torch::empty({n, nb}, w.options());
+  CHECK_HIP(lfmq_gptq_block(w.data_ptr(), ub.data_ptr(), codes.data_ptr(),
+                            scales.data_ptr(), zeros.data_ptr(),
+                            err.data_ptr(), (int)n, (int)k, (int)(k / g),
+                            (int)i1, (int)nb, (int)g, (int)bits, sym,
+                            stream()));
+  return err;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -562,6 +591,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prefill", &attn_prefill,
         "EXPERIMENTAL flash prefill attention (LFMQ_FLASH_PREFILL)");
   m.def("hessian_accum", &hessian_accum, "H += 2 X^T X");
+  m.def("gptq_block", &gptq_block, "one column block of the GPTQ solve");
   m.def("dq_gemv_gateup", &dq_gemv_gateup, "fused gate_up GEMV + silu*mul");
   m.def("qkv_rope_append", &qkv_rope_append, "fused rope + KV append");
   m.def("greedy_sample", &greedy_sample, "row argmax");

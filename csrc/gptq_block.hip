@@ -1,0 +1,149 @@
+// K13 — GPTQ's inner loop: quantize one block of columns, column by column,
+// each column's rounding error pushed onto the block's later ones.
+//
+//   per group start:  scale, zero from the block's unquantized columns
+//   q_j = clamp(round(w_j / s) + z),  e_j = (w_j - (q_j - z) s) / u_jj
+//   w_c -= e_j u_jc  for the block's c > j
+//
+// Rows do not meet, so a row runs in 16 lanes (four rows a wave), its block
+// in their registers, and the block of U in LDS for all 32 rows of a
+// workgroup.  Lane c of a row holds columns 64 i + 4 c + 0..3: a row of U is
+// read in 16-byte pieces side by side, the same address for all four rows.
+// Bound by the chain column -> division -> broadcast -> update, 128 times:
+// 2048 rows take 56 us a block of 128, where one launch per elementwise
+// operation took 7.2 ms (with the gaps between them).
+//
+// Every operation rounds on its own, in the order of the tensor expressions
+// above, so that results are those of a GPU tensor loop, bit by bit: no
+// contraction, and a division by a constant is a product with its
+// reciprocal.
+#include "common.h"
+
+namespace {
+
+#pragma clang fp contract(off)
+
+constexpr int TPB = 512, RPW = 4;            // rows a wave
+constexpr int ROWS = TPB / LFMQ_WAVE * RPW;  // rows a workgroup
+
+// NaN wins, as in tensor reductions and clamps
+__device__ __forceinline__ float nmin(float a, float b) {
+  return b < a || b != b ? b : a;
+}
+__device__ __forceinline__ float nmax(float a, float b) {
+  return b > a || b != b ? b : a;
+}
+__device__ __forceinline__ float nclamp(float x, float hi) {
+  return x < 0.f ? 0.f : (x > hi ? hi : x);
+}
+
+template <int NC>  // chunks of 64 columns
+__global__ __launch_bounds__(TPB) void gptq_block_kernel(
+    const float* __restrict__ w, const float* __restrict__ ub,
+    i32* __restrict__ codes, float* __restrict__ scales,
+    i32* __restrict__ zeros, float* __restrict__ err, int n, int k, int G,
+    int i1, int nb, int g, float qmax, float inv_range, int sym) {
+  constexpr int BS = NC * 64;
+  extern __shared__ __attribute__((aligned(16))) float us[];   // [nb][BS]
+  for (int t = threadIdx.x; t < nb * BS; t += TPB) {
+    const int r = t / BS, c = t % BS;
+    us[t] = c < nb ? ub[r * nb + c] : 0.f;
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, c16 = lane & 15;
+  const int row = blockIdx.x * ROWS + (threadIdx.x >> 6) * RPW + (lane >> 4);
+  const bool live = row < n;
+  const float* wr = w + (u64)(live ? row : n - 1) * k;
+
+  float v[NC * 4];
+#pragma unroll
+  for (int i = 0; i < NC; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int c = i * 64 + c16 * 4 + r;
+      v[i * 4 + r] = c < nb ? wr[i1 + c] : 0.f;
+    }
+  float s = 1.f, z = 0.f;
+  if (i1 % g != 0) {                       // inside a group begun earlier
+    s = scales[(u64)(live ? row : n - 1) * G + i1 / g];
+    z = (float)zeros[(u64)(live ? row : n - 1) * G + i1 / g];
+  }
+
+#pragma unroll
+  for (int i = 0; i < NC; ++i)
+    for (int c = 0; c < 16; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int j = i * 64 + c * 4 + r;
+        if (j >= nb) break;
+        if ((i1 + j) % g == 0) {
+          float lo = INFINITY, hi = -INFINITY;
+          for (int t = c16; t < g; t += 16) {
+            const float x = wr[i1 + j + t];
+            lo = nmin(lo, x);
+            hi = nmax(hi, x);
+          }
+#pragma unroll
+          for (int o = 8; o > 0; o >>= 1) {
+            lo = nmin(lo, __shfl_xor(lo, o, 64));
+            hi = nmax(hi, __shfl_xor(hi, o, 64));
+          }
+          if (sym) {
+            s = nmax(fabsf(lo), fabsf(hi)) * inv_range;
+            s = s == 0.f ? 1.f : s;
+            z = (qmax + 1.f) * 0.5f;
+          } else {
+            s = (hi - lo) * inv_range;
+            s = s == 0.f ? 1.f : s;
+            z = (float)(i32)nclamp(rintf(-lo / s), qmax);
+          }
+          if (live && c16 == 0) {
+            scales[(u64)row * G + (i1 + j) / g] = s;
+            zeros[(u64)row * G + (i1 + j) / g] = (i32)z;
+          }
+        }
+        const float x = __shfl(v[i * 4 + r], (lane & 48) + c, 64);
+        const float q = nclamp(rintf(x / s) + z, qmax);
+        const float e = (x - (q - z) * s) / us[j * BS + j];
+        if (live && c16 == 0) {
+          codes[(u64)row * k + i1 + j] = (i32)q;
+          err[(u64)row * nb + j] = e;
+        }
+#pragma unroll
+        for (int i2 = i; i2 < NC; ++i2) {
+          const f32x4 u = *(const f32x4*)(us + j * BS + i2 * 64 + c16 * 4);
+#pragma unroll
+          for (int r2 = 0; r2 < 4; ++r2)
+            v[i2 * 4 + r2] = v[i2 * 4 + r2] - e * u[r2];
+        }
+      }
+}
+
+}  // namespace
+
+// w [n, k] fp32 (read only), ub [nb, nb] the block of U on the diagonal,
+// columns i1 .. i1 + nb - 1 (nb <= 128).  Writes codes, err [n, nb] and the
+// scales and zeros of groups that start in the block; a group that began in
+// an earlier block is read from them.
+hipError_t lfmq_gptq_block(const void* w, const void* ub, void* codes,
+                           void* scales, void* zeros, void* err, int n, int k,
+                           int G, int i1, int nb, int g, int bits, bool sym,
+                           hipStream_t stream) {
+  if (nb < 1 || nb > 128 || i1 < 0 || i1 + nb > k || g < 1 || G * (long)g != k)
+    return hipErrorInvalidValue;
+  if (n == 0) return hipSuccess;
+  const float qmax = (float)((1 << bits) - 1);
+  const float inv = sym ? 1.f / ((qmax - 1.f) / 2.f) : 1.f / qmax;
+  const dim3 grid((n + ROWS - 1) / ROWS);
+  const int bs = nb <= 64 ? 64 : 128;
+  const size_t lds = (size_t)nb * bs * sizeof(float);
+#define GO(NC)                                                              \
+  hipLaunchKernelGGL((gptq_block_kernel<NC>), grid, dim3(TPB), lds, stream, \
+                     (const float*)w, (const float*)ub, (i32*)codes,        \
+                     (float*)scales, (i32*)zeros, (float*)err, n, k, G, i1, \
+                     nb, g, qmax, inv, (int)sym)
+  if (bs == 64) GO(1);
+  else GO(2);
+#undef GO
+  return hipGetLastError();
+}

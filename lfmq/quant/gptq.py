@@ -40,6 +40,44 @@ def _hessian_accum(h: torch.Tensor, x: torch.Tensor) -> None:
         ref.hessian_accum(h, x)
 
 
+def _block(w, ub, codes, scales, zeros, i1, cfg, g) -> torch.Tensor:
+    """Quantize the columns from i1 on that ub covers; returns their errors
+    [n, nb].  Groups that start here fit w as it was before the block."""
+    qmax = (1 << cfg.bits) - 1
+    nb = ub.shape[0]
+    wb = w[:, i1:i1 + nb].clone()
+    err = torch.zeros_like(wb)
+    for j in range(nb):
+        col = i1 + j
+        gi = col // g
+        if col % g == 0:
+            # (re)fit scale/zero on the error-compensated group slice
+            _, s_, z_ = ref.quant_groupwise(w[:, col:col + g], cfg.bits, g,
+                                            cfg.sym)
+            scales[:, gi] = s_[:, 0]
+            zeros[:, gi] = z_[:, 0]
+        scale, zero = scales[:, gi], zeros[:, gi]
+        wj = wb[:, j]
+        q = torch.clamp(torch.round(wj / scale) + zero, 0, qmax)
+        codes[:, col] = q.to(torch.int32)
+        dq = (q - zero) * scale
+        e = (wj - dq) / ub[j, j]
+        if j + 1 < nb:
+            wb[:, j + 1:] -= torch.outer(e, ub[j, j + 1:])
+        err[:, j] = e
+    return err
+
+
+GPU_BLOCK = 128        # widest block of the HIP kernel: its U fits in LDS
+
+
+def _gpu_block(w, ub, codes, scales, zeros, i1, cfg, g) -> torch.Tensor:
+    """_block in one launch (csrc/gptq_block.hip), the same bit by bit."""
+    from ..ops import hip_ext
+    return hip_ext().gptq_block(w, ub.contiguous(), codes, scales, zeros, i1,
+                                g, cfg.bits, cfg.sym)
+
+
 @torch.no_grad()
 def gptq_quantize_layer(
     w: torch.Tensor, h: torch.Tensor, cfg: QuantConfig
@@ -67,7 +105,7 @@ def gptq_quantize_layer(
     perm = None
     if cfg.act_order:
         perm = torch.argsort(torch.diag(h), descending=True)
-        w = w[:, perm]
+        w = w[:, perm].contiguous()
         h = h[perm][:, perm]
 
     damp = cfg.damp_percent * torch.diag(h).mean()
@@ -81,36 +119,11 @@ def gptq_quantize_layer(
     codes = torch.zeros(n, k, dtype=torch.int32, device=dev)
     scales = torch.zeros(n, G, dtype=torch.float32, device=dev)
     zeros = torch.zeros(n, G, dtype=torch.int32, device=dev)
-    qmax = (1 << cfg.bits) - 1
 
-    bs = cfg.block_size
-    scale_cur = torch.ones(n, device=dev)
-    zero_cur = torch.zeros(n, dtype=torch.int32, device=dev)
-    for i1 in range(0, k, bs):
-        i2 = min(i1 + bs, k)
-        wb = w[:, i1:i2].clone()
-        err = torch.zeros_like(wb)
-        ub = U[i1:i2, i1:i2]
-        for j in range(i2 - i1):
-            col = i1 + j
-            if col % g == 0:
-                # (re)fit scale/zero on the error-compensated group slice
-                grp = w[:, col:col + g]
-                _, s_, z_ = ref.quant_groupwise(grp, cfg.bits, g, cfg.sym)
-                gi = col // g
-                scales[:, gi] = s_[:, 0]
-                zeros[:, gi] = z_[:, 0]
-                scale_cur = s_[:, 0].to(dev)
-                zero_cur = z_[:, 0].to(dev)
-            wj = wb[:, j]
-            q = torch.clamp(torch.round(wj / scale_cur) + zero_cur, 0, qmax)
-            codes[:, col] = q.to(torch.int32)
-            dq = (q - zero_cur) * scale_cur
-            e = (wj - dq) / ub[j, j]
-            if j + 1 < i2 - i1:
-                wb[:, j + 1:] -= torch.outer(e, ub[j, j + 1:])
-            err[:, j] = e
-        w[:, i1:i2] = wb
+    block = _gpu_block if w.is_cuda and cfg.block_size <= GPU_BLOCK else _block
+    for i1 in range(0, k, cfg.block_size):
+        i2 = min(i1 + cfg.block_size, k)
+        err = block(w, U[i1:i2, i1:i2], codes, scales, zeros, i1, cfg, g)
         if i2 < k:
             w[:, i2:] -= err @ U[i1:i2, i2:]
 

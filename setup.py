@@ -33,6 +33,7 @@ SOURCES = [
     "csrc/dq_gemv_mfma.hip",
     "csrc/dq_gemm.hip",
     "csrc/hessian.hip",
+    "csrc/gptq_block.hip",
     "csrc/attn_decode.hip",
     "csrc/attn_prefill.hip",
     "csrc/qkv_rope_append.hip",

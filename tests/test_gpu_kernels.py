@@ -430,6 +430,36 @@ def test_attn_decode_key_ranges(b, T, hq, hkv, d):
     assert rel_err(o, want) < 6e-3
 
 
+@pytest.mark.parametrize("n,k,nb,i1,g,bits,sym", [
+    (1, 128, 128, 0, 128, 4, False), (33, 256, 128, 128, 64, 4, True),
+    (70, 384, 128, 128, 384, 8, False), (32, 200, 64, 64, 40, 8, True),
+    (5, 133, 5, 128, 19, 4, False), (64, 512, 100, 200, 256, 4, False)])
+def test_gptq_block_is_the_tensor_loop(n, k, nb, i1, g, bits, sym):
+    """Bit by bit: partial blocks, groups longer and shorter than a block,
+    an all-zero group, a row that is not finite."""
+    from lfmq import QuantConfig
+    from lfmq.quant.gptq import _block, _gpu_block
+    torch.manual_seed(n + k)
+    cfg = QuantConfig(scheme="gptq", bits=bits, group_size=g, sym=sym)
+    w = torch.randn(n, k, device=DEV)
+    w[0, i1:i1 + nb] = 0
+    if n > 4:
+        w[4, i1] = float("inf")
+    ub = torch.randn(nb, nb, device=DEV).mul_(0.1).triu_()
+    ub.diagonal().uniform_(0.5, 2.0)
+    got = []
+    for fn in (_block, _gpu_block):
+        out = [torch.zeros(n, k, dtype=torch.int32, device=DEV),
+               torch.full((n, k // g), 0.4, device=DEV),
+               torch.full((n, k // g), 5, dtype=torch.int32, device=DEV)]
+        got.append(out + [fn(w, ub, *out, i1, cfg, g)])
+    fine = torch.isfinite(got[0][3]).all(1)
+    assert int(fine.sum()) >= n - 1
+    for a, b in zip(*got):
+        assert torch.equal(a[fine], b[fine])
+    assert torch.equal(torch.isfinite(got[0][3]), torch.isfinite(got[1][3]))
+
+
 @pytest.mark.parametrize("m", [5, 8, 16])
 @pytest.mark.parametrize("n,k,g", [(256, 2048, 128), (100, 512, 64),
                                    (48, 4096, 128)])
