@@ -1,0 +1,37 @@
+// Packed weights as matrix-core operands: eight codes of one weight row as
+// the exact bf16 numbers 128 + c (int4, one dword) or c (int8, two dwords).
+// With a group's scale s and zero z,
+//   sum s (c - z) x = s (sum code x) - s zb sum x,  zb = z + 128 or z.
+#pragma once
+#include "common.h"
+
+template <int BITS>
+__device__ __forceinline__ s16x8 codes8(const u32* w) {
+  if constexpr (BITS == 4) {
+    const DequantPairs4 d = dequant4_pairs(w[0]);
+    return __builtin_bit_cast(s16x8, u32x4{d.p01, d.p23, d.p45, d.p67});
+  } else {
+    u32x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      // at most 8 significant bits: the upper half of the float is exact
+      const u32 p = w[i >> 1] >> (16 * (i & 1));
+      const float lo = (float)(p & 0xFFu), hi = (float)((p >> 8) & 0xFFu);
+      o[i] = __builtin_amdgcn_perm(__builtin_bit_cast(u32, hi),
+                                   __builtin_bit_cast(u32, lo), 0x07060302u);
+    }
+    return __builtin_bit_cast(s16x8, o);
+  }
+}
+
+// zb of group gi from its word of packed zeros
+template <int BITS>
+__device__ __forceinline__ float zero_bias(u32 word, int gi) {
+  return BITS == 4 ? (float)(unpack4(word, gi & 7) + 128u)
+                   : (float)unpack8(word, gi & 3);
+}
+
+__device__ __forceinline__ s16x8 bf16_ones() {
+  return __builtin_bit_cast(
+      s16x8, u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
+}

@@ -1,0 +1,344 @@
+// K3c/K4c — W4A16 / W8A16 product for a few to a few hundred rows of x:
+// y[m, n] = x[m, k] · dequant(W)[n, k]^T (+ bias) (+ residual).
+//
+// Between the GEMV (m <= 4) and the large product the packed weights are
+// still most of the traffic, so they are read once, straight into
+// registers, and turned into matrix-core operands there: int4 as the exact
+// bf16 numbers 128 + c, int8 as c.  Scale and zero are applied per group to
+// the fp32 result:  sum s (c - z) x = s (sum c x - z sum x), the second sum
+// from one more product, with ones.
+//
+// A wave computes MT x 16 rows by NT x 16 columns over a share of k.  Its
+// lanes read 16 bytes of a packed row at a time (a chunk of KC values of k
+// is split over the four lane groups, x is read in the same order), the next
+// chunk's weights are on their way during this one's products, and no
+// barrier is needed until the four waves of a workgroup, which share k, add
+// their results in LDS.  Where the columns do not fill the chip, k is also
+// split over workgroups; their fp32 sums meet in dq_rows_sum.
+//
+// us a call, before (16-column GEMV tiles up to 16 rows, 128 x 128 tiles
+// above) and now:
+//                       8 rows       24 rows       48 rows
+//   n 28672, k 4096   70.0 -> 24.1  108 -> 31.6   107 -> 49.3
+//   n 4096, k 14336   45.0 -> 17.8  362 -> 20.6   366 -> 29.7   (4 bits)
+//   n 4096, k 4096    13.7 ->  9.0  101 -> 11.9   101 -> 14.4
+//   n 16384, k 2048   75.5 -> 13.8   57 -> 16.1    58 -> 19.9   (8 bits,
+//   n 2048, k 8192    25.5 -> 12.0  203 -> 14.1   203 -> 16.6    group 64)
+#include "dq_frag.h"
+
+namespace {
+
+constexpr int NW = 4, TPB = NW * LFMQ_WAVE;
+
+struct RArgs {
+  const char* w;                 // [n, k * BITS / 8] bytes
+  const unsigned short* scales;  // [n, G]
+  const u32* zeros;              // [n, zw]
+  const unsigned short* x;       // [m, k]
+  unsigned short* y;             // [m, n]
+  const unsigned short *bias, *resid;
+  float* part;                   // [splits, m, n], splits > 1
+  int m, n, k, g, splits;
+};
+
+__device__ __forceinline__ float epilogue(const RArgs& A, float v, int row,
+                                          int col) {
+  if (A.bias != nullptr) v += bf16_bits_to_f32(A.bias[col]);
+  if (A.resid != nullptr)
+    v += bf16_bits_to_f32(A.resid[(u64)row * A.n + col]);
+  return v;
+}
+
+template <int BITS, int MT, int NT, int KC>
+__global__ __launch_bounds__(TPB) void dq_rows_kernel(RArgs A) {
+  constexpr int J = KC / 32;                 // products a chunk
+  constexpr int WD = J * BITS / 4;           // packed dwords a lane, a chunk
+  constexpr int BM = MT * 16, BN = NT * 16, LD = BN + 4;
+  // first [groups][BN] scales and zeros, then [NW][BM][LD] results
+  extern __shared__ __attribute__((aligned(16))) float red[];
+  u32* meta = (u32*)red;
+  const int lane = threadIdx.x & 63, l15 = lane & 15, l4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = blockIdx.x * BN, m0 = blockIdx.z * BM;
+  const int C = A.k / KC;
+  // this wave's chunks: workgroups, then waves, share them evenly
+  const int u = blockIdx.y * NW + wave, U = gridDim.y * NW;
+  const int c0 = (int)((long)C * u / U), c1 = (int)((long)C * (u + 1) / U);
+  const int G = A.k / A.g, zw = (G + 32 / BITS - 1) / (32 / BITS);
+
+  // one word a column and group of this workgroup: scale (bf16) above,
+  // zero bias below.  Read from memory once; per chunk, its lines of 2-byte
+  // scales would be most of the traffic.
+  const int w0 = (int)((long)C * blockIdx.y * NW / U);
+  const int w1 = (int)((long)C * (blockIdx.y + 1) * NW / U);
+  const int g0 = w0 * KC / A.g, ng = w1 > w0 ? (w1 - 1) * KC / A.g - g0 + 1 : 0;
+  for (int i = threadIdx.x; i < BN * ng; i += TPB) {
+    const int col = i / ng, gi = g0 + i % ng;
+    const u64 r = min(n0 + col, A.n - 1);
+    const u32 z = A.zeros[r * zw + gi / (32 / BITS)];
+    meta[(gi - g0) * BN + col] =
+        (u32)A.scales[r * G + gi] << 16 |
+        (BITS == 4 ? unpack4(z, gi & 7) + 128u : unpack8(z, gi & 3));
+  }
+  const char* wr[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int col = min(n0 + t * 16 + l15, A.n - 1);
+    wr[t] = A.w + (u64)col * (A.k * BITS / 8) + l4 * (WD * 4);
+  }
+  u32 xo[MT];                                // byte offsets into x
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+    xo[t] = ((u32)min(m0 + t * 16 + l15, A.m - 1) * A.k + l4 * (KC / 4)) * 2;
+
+  const s16x8 ones = bf16_ones();
+  f32x4 acc[MT][NT] = {};
+  // WR chunks of weights and XR of x are on their way
+  constexpr int WR = MT == 1 ? 4 : 2, XR = MT <= 2 ? 2 : 1;
+  u32 wq[WR][NT][WD];
+  s16x8 xq[XR][MT][J];
+  auto fetch_w = [&](int c, u32 (&w)[NT][WD]) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const u32* p = (const u32*)(wr[t] + (u64)c * (KC * BITS / 8));
+      if constexpr (WD >= 4) {
+#pragma unroll
+        for (int i = 0; i < WD / 4; ++i) {
+          const u32x4 v = __builtin_nontemporal_load((const u32x4*)p + i);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[t][i * 4 + e] = v[e];
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < WD; ++e) w[t][e] = p[e];
+      }
+    }
+  };
+  auto fetch_x = [&](int c, s16x8 (&x)[MT][J]) {
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        x[t][j] = *(const s16x8*)((const char*)A.x + xo[t] +
+                                  (u32)(c * KC + j * 8) * 2);
+  };
+  auto multiply = [&](int c, const u32 (&w)[NT][WD], const s16x8 (&x)[MT][J]) {
+    const u32* mt = meta + (c * KC / A.g - g0) * BN + l15;
+    f32x4 xs[MT] = {};
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        xs[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[t][j], ones, xs[t],
+                                                        0, 0, 0);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      f32x4 a[MT] = {};
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        const s16x8 b = codes8<BITS>(&w[nt][j * BITS / 4]);
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+          a[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[t][j], b, a[t], 0,
+                                                         0, 0);
+      }
+      const u32 e = mt[nt * 16];
+      const float s = __builtin_bit_cast(float, e & 0xFFFF0000u);
+      const float sz = s * (float)(e & 0xFFu);
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc[t][nt][i] = fmaf(-sz, xs[t][i], fmaf(s, a[t][i], acc[t][nt][i]));
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < WR; ++i) {
+    if (c0 + i < c1) fetch_w(c0 + i, wq[i]);
+    if (i < XR && XR > 1 && c0 + i < c1) fetch_x(c0 + i, xq[i]);
+  }
+  __syncthreads();                           // meta is there
+  for (int c = c0; c < c1; c += WR) {
+#pragma unroll
+    for (int i = 0; i < WR; ++i) {
+      if (c + i >= c1) break;
+      if constexpr (XR == 1) fetch_x(c + i, xq[0]);
+      multiply(c + i, wq[i], xq[i % XR]);
+      if (c + i + WR < c1) fetch_w(c + i + WR, wq[i]);
+      if (XR > 1 && c + i + XR < c1) fetch_x(c + i + XR, xq[i % XR]);
+    }
+  }
+
+  // ---- the waves' shares of k ----
+  __syncthreads();                           // meta is read
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        red[((u32)wave * BM + t * 16 + l4 * 4 + r) * LD + nt * 16 + l15] =
+            acc[t][nt][r];
+  __syncthreads();
+  const bool wide = A.n % 4 == 0;
+  for (int id = threadIdx.x; id < BM * BN / 4; id += TPB) {
+    const int row = id / (BN / 4), c4 = id % (BN / 4) * 4;
+    const int gr = m0 + row, gc = n0 + c4;
+    if (gr >= A.m || gc >= A.n) continue;
+    f32x4 v = *(const f32x4*)(red + (u32)row * LD + c4);
+#pragma unroll
+    for (int w = 1; w < NW; ++w)
+      v += *(const f32x4*)(red + ((u32)w * BM + row) * LD + c4);
+    if (gridDim.y > 1) {
+      float* p = A.part + ((u64)blockIdx.y * A.m + gr) * A.n + gc;
+      if (wide) {
+        *(f32x4*)p = v;
+      } else {
+        for (int e = 0; e < 4 && gc + e < A.n; ++e) p[e] = v[e];
+      }
+      continue;
+    }
+    unsigned short* p = A.y + (u64)gr * A.n + gc;
+    for (int e = 0; e < 4; ++e)
+      if (gc + e < A.n) v[e] = epilogue(A, v[e], gr, gc + e);
+    if (wide) {
+      *(u64*)p = pack_bf16x2(v[0], v[1]) | (u64)pack_bf16x2(v[2], v[3]) << 32;
+    } else {
+      for (int e = 0; e < 4 && gc + e < A.n; ++e)
+        p[e] = (unsigned short)f32_to_bf16_bits_rne(v[e]);
+    }
+  }
+}
+
+// y = sum of the splits' parts (+ bias) (+ residual)
+__global__ __launch_bounds__(256) void dq_rows_sum(RArgs A) {
+  const u64 total = (u64)A.m * A.n;
+  if (A.n % 4 == 0) {
+    for (u64 id = ((u64)blockIdx.x * 256 + threadIdx.x) * 4; id < total;
+         id += (u64)gridDim.x * 1024) {
+      f32x4 v = *(const f32x4*)(A.part + id);
+#pragma unroll 4
+      for (int s = 1; s < A.splits; ++s)
+        v += *(const f32x4*)(A.part + s * total + id);
+      const int row = id / A.n, col = id % A.n;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = epilogue(A, v[e], row, col + e);
+      *(u64*)(A.y + id) =
+          pack_bf16x2(v[0], v[1]) | (u64)pack_bf16x2(v[2], v[3]) << 32;
+    }
+    return;
+  }
+  for (u64 id = (u64)blockIdx.x * 256 + threadIdx.x; id < total;
+       id += (u64)gridDim.x * 256) {
+    float v = 0.f;
+    for (int s = 0; s < A.splits; ++s) v += A.part[s * total + id];
+    A.y[id] = (unsigned short)f32_to_bf16_bits_rne(
+        epilogue(A, v, id / A.n, id % A.n));
+  }
+}
+
+void sum_parts(const RArgs& A, hipStream_t stream) {
+  const u64 items = (u64)A.m * A.n / (A.n % 4 == 0 ? 4 : 1);
+  hipLaunchKernelGGL(dq_rows_sum,
+                     dim3((u32)min((items + 255) / 256, (u64)1024)),
+                     dim3(256), 0, stream, A);
+}
+
+struct Tile { int mt, nt; };
+
+// rows and columns (in 16s) of a wave
+Tile tile_of(int m) {
+  if (m <= 16) return {1, 2};
+  if (m <= 32) return {2, 4};
+  return {3, 4};
+}
+
+int chunk_of(int g) { return g % 128 == 0 ? 128 : (g % 64 == 0 ? 64 : 32); }
+
+// scales and zeros of a workgroup: its share of the chunks, which may begin
+// and end inside a group
+size_t meta_bytes(int k, int g, int splits, int nt) {
+  const int kc = chunk_of(g), chunks = (k / kc + splits - 1) / splits + 1;
+  return ((size_t)chunks * kc / g + 2) * nt * 16 * 4;
+}
+
+template <int BITS, int MT, int NT, int KC>
+hipError_t go(const RArgs& A, hipStream_t stream) {
+  const size_t sums = (size_t)NW * MT * 16 * (NT * 16 + 4) * 4;
+  const size_t lds = max(sums, meta_bytes(A.k, A.g, A.splits, NT));
+  if (lds > 64 * 1024) return hipErrorInvalidValue;
+  const dim3 grid(ceil_div_u32(A.n, NT * 16), A.splits,
+                  ceil_div_u32(A.m, MT * 16));
+  hipLaunchKernelGGL((dq_rows_kernel<BITS, MT, NT, KC>), grid, dim3(TPB), lds,
+                     stream, A);
+  if (A.splits > 1) sum_parts(A, stream);
+  return hipGetLastError();
+}
+
+template <int BITS, int KC>
+hipError_t go_tile(const RArgs& A, hipStream_t stream) {
+  const Tile t = tile_of(A.m);
+  if (t.mt == 1) return go<BITS, 1, 2, KC>(A, stream);
+  if (t.mt == 2) return go<BITS, 2, 4, KC>(A, stream);
+  return go<BITS, 3, 4, KC>(A, stream);
+}
+
+}  // namespace
+
+// false: the shape belongs to another kernel
+bool lfmq_dq_rows_ok(int m, int n, int k, int g) {
+  return g % 32 == 0 && g <= k && k % g == 0 && (u64)m * k * 2 < (1ull << 32);
+}
+
+// workgroups that share k
+int lfmq_dq_rows_splits(int m, int n, int k, int g) {
+  const Tile t = tile_of(m);
+  const int wgs = (int)(ceil_div_u32(n, t.nt * 16) * ceil_div_u32(m, t.mt * 16));
+  const int C = k / chunk_of(g);
+  // 256 workgroups, or 512 where a wave keeps six chunks (us at 8 rows, 2 / 4
+  // splits: n 4096, k 4096 9.0 / 9.7, k 14336 18.3 / 17.8)
+  int s = max(1, min(256 / wgs, C / (NW * 2)));
+  if (512 / wgs <= C / (NW * 6)) s = max(s, 512 / wgs);
+  while (meta_bytes(k, g, s, t.nt) > 64 * 1024) ++s;     // LDS of a workgroup
+  return s;
+}
+
+// part: splits > 1 only, [splits, m, n] fp32
+hipError_t lfmq_dq_rows(const void* qweight, const void* scales,
+                        const void* qzeros, const void* x, void* y,
+                        const void* bias, const void* resid, void* part,
+                        int m, int n, int k, int g, int bits, int splits,
+                        hipStream_t stream) {
+  if (!lfmq_dq_rows_ok(m, n, k, g)) return hipErrorInvalidValue;
+  if (bits != 4 && bits != 8) return hipErrorInvalidValue;
+  const RArgs A{(const char*)qweight, (const unsigned short*)scales,
+                (const u32*)qzeros, (const unsigned short*)x,
+                (unsigned short*)y, (const unsigned short*)bias,
+                (const unsigned short*)resid, (float*)part, m, n, k, g,
+                splits};
+  const int kc = chunk_of(g);
+  if (bits == 4) {
+    if (kc == 128) return go_tile<4, 128>(A, stream);
+    if (kc == 64) return go_tile<4, 64>(A, stream);
+    return go_tile<4, 32>(A, stream);
+  }
+  if (kc == 128) return go_tile<8, 128>(A, stream);
+  if (kc == 64) return go_tile<8, 64>(A, stream);
+  return go_tile<8, 32>(A, stream);
+}
+
+// y = sum of part [splits, m, n] (+ bias) (+ residual)
+hipError_t lfmq_dq_rows_sum(const void* part, void* y, const void* bias,
+                            const void* resid, int m, int n, int splits,
+                            hipStream_t stream) {
+  RArgs A{};
+  A.part = (float*)part;
+  A.y = (unsigned short*)y;
+  A.bias = (const unsigned short*)bias;
+  A.resid = (const unsigned short*)resid;
+  A.m = m;
+  A.n = n;
+  A.splits = splits;
+  sum_parts(A, stream);
+  return hipGetLastError();
+}

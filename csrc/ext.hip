@@ -10,9 +10,16 @@ hipError_t lfmq_unpack(const void*, void*, long, int, int, hipStream_t);
 hipError_t lfmq_dq_gemv(const void*, const void*, const void*, const void*,
                         void*, const void*, const void*, int, int, int, int,
                         int, float, int, hipStream_t);
-hipError_t lfmq_dq_gemm(const void*, const void*, const void*, const void*,
-                        void*, const void*, int, int, int, int, int,
-                        hipStream_t);
+bool lfmq_dq_rows_ok(int, int, int, int);
+int lfmq_dq_rows_splits(int, int, int, int);
+hipError_t lfmq_dq_rows(const void*, const void*, const void*, const void*,
+                        void*, const void*, const void*, void*, int, int, int,
+                        int, int, int, hipStream_t);
+bool lfmq_dq_tile_ok(int, int);
+int lfmq_dq_tile_splits(int, int, int, int);
+hipError_t lfmq_dq_tile(const void*, const void*, const void*, const void*,
+                        void*, const void*, void*, int, int, int, int, int,
+                        int, hipStream_t);
 hipError_t lfmq_rmsnorm(const void*, const void*, const void*, void*, void*,
                         int, int, float, hipStream_t);
 hipError_t lfmq_rope(void*, void*, const void*, const void*, int, int, int,
@@ -126,17 +133,47 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
     rptr = resid->data_ptr();
   }
   auto y = torch::empty({m, n}, x.options());
-  if (m <= 16) {
+  // Which kernel: a wave a few columns (GEMV), rows of x in registers, or x
+  // through LDS.  us of the first two, n 28672, k 4096, 4 bits: 24.6 / 21.5 at
+  // 2 rows but 8.5 / 9.6 at n 6144; 36 / 22 and 11.9 / 9.8 at 4.  8 bits,
+  // n 32000, k 2048: 18.5 / 18.7 at 1 row, 29 / 19 at 2.  The last two, 4
+  // bits, n 28672 and 4096: 49 / 50 and 14.4 / 19 at 48 rows, 66 / 51 and
+  // 17 / 20 at 64.
+  const bool by_rows = (cols_hint == 0 ? m >= (bits == 8 ? 2 : 3)
+                                       : cols_hint == 6 && m > 4) &&
+                       m <= 48 && rms_eps < 0 &&
+                       lfmq_dq_rows_ok(m, n, k, (int)g);
+  if (m > 16) {
+    TORCH_CHECK(rptr == nullptr && rms_eps < 0,
+                "fused rms/resid is a decode (m<=16) path");
+    TORCH_CHECK(lfmq_dq_tile_ok(k, (int)g),
+                "more than 16 rows need groups of a multiple of 64 that "
+                "divide k");
+  }
+  torch::Tensor part;
+  auto parts = [&](int splits) -> void* {
+    if (splits == 1) return nullptr;
+    part = torch::empty({(long)splits * m * n},
+                        x.options().dtype(torch::kFloat32));
+    return part.data_ptr();
+  };
+  if (by_rows) {
+    const int splits = lfmq_dq_rows_splits(m, n, k, (int)g);
+    CHECK_HIP(lfmq_dq_rows(qweight.data_ptr(), scales.data_ptr(),
+                           qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
+                           rptr, parts(splits), m, n, k, (int)g, (int)bits,
+                           splits, stream()));
+  } else if (m <= 16) {
     CHECK_HIP(lfmq_dq_gemv(qweight.data_ptr(), scales.data_ptr(),
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                            rptr, m, n, k, (int)g, (int)bits, (float)rms_eps,
                            (int)cols_hint, stream()));
   } else {
-    TORCH_CHECK(rptr == nullptr && rms_eps < 0,
-                "fused rms/resid is a decode (m<=16) path");
-    CHECK_HIP(lfmq_dq_gemm(qweight.data_ptr(), scales.data_ptr(),
+    const int splits = lfmq_dq_tile_splits(m, n, k, (int)g);
+    CHECK_HIP(lfmq_dq_tile(qweight.data_ptr(), scales.data_ptr(),
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
-                           m, n, k, (int)g, (int)bits, stream()));
+                           parts(splits), m, n, k, (int)g, (int)bits, splits,
+                           stream()));
   }
   return y;
 }

@@ -30,8 +30,8 @@ SOURCES = [
     "csrc/rope.hip",
     "csrc/elementwise.hip",
     "csrc/dq_gemv.hip",
-    "csrc/dq_gemv_mfma.hip",
-    "csrc/dq_gemm.hip",
+    "csrc/dq_rows.hip",
+    "csrc/dq_tile.hip",
     "csrc/hessian.hip",
     "csrc/gptq_block.hip",
     "csrc/attn_decode.hip",

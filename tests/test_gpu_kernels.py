@@ -477,6 +477,49 @@ def test_dq_gemv_mfma_variant(m, n, k, g):
     assert rel_err(y, y_ref) < 2e-2, f"rel={rel_err(y, y_ref)}"
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,n,k,g", [
+    (3, 33, 384, 128), (5, 37, 96, 32), (16, 96, 640, 64), (17, 130, 640, 64),
+    (33, 65, 512, 512), (48, 32, 8192, 64), (49, 36, 1024, 128),
+    (127, 129, 640, 64), (129, 40, 8192, 128), (260, 257, 2048, 2048)])
+def test_dq_linear_rows_and_tiles(bits, m, n, k, g):
+    """Edges of row, column and key tiles, groups that are no multiple of
+    eight a row, splits of k, ragged n, bias and residual.  Products of bf16
+    and codes are exact and summed in fp32, so the result is off by its own
+    rounding, 2^-9 of a value."""
+    torch.manual_seed(m + n)
+    codes, scales, zeros = ref.quant_groupwise(torch.randn(n, k), bits, g,
+                                               False)
+    qw, qz = ref.pack_codes(codes, bits), ref.pack_zeros(zeros, bits)
+    s16 = scales.to(torch.bfloat16)
+    x = torch.randn(m, k).to(torch.bfloat16)
+    bias = torch.randn(n).to(torch.bfloat16)
+    resid = torch.randn(m, n).to(torch.bfloat16) if m <= 16 else None
+    w = ref.dequant_groupwise(codes, s16.float(), zeros, g).double()
+    want = x.double() @ w.t() + bias.double()
+    if resid is not None:
+        want += resid.double()
+    y = ext().dq_linear(x.to(DEV), qw.to(DEV), s16.to(DEV), qz.to(DEV), bits,
+                        g, bias.to(DEV), None if resid is None
+                        else resid.to(DEV), -1.0, 0)
+    assert y.shape == (m, n)
+    err = (y.cpu().double() - want).abs()
+    assert float((err / (want.abs() + 1e-3 * want.abs().max())).max()) < 5e-3
+
+
+def test_dq_linear_refuses():
+    """More than 16 rows: groups of 32 and fused epilogues, as ever."""
+    x = torch.zeros(17, 96, dtype=torch.bfloat16, device=DEV)
+    qw = torch.zeros(8, 12, dtype=torch.int32, device=DEV)
+    qz = torch.zeros(8, 1, dtype=torch.int32, device=DEV)
+    s = torch.ones(8, 3, dtype=torch.bfloat16, device=DEV)
+    r = torch.zeros(17, 8, dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(RuntimeError):
+        ext().dq_linear(x, qw, s, qz, 4, 32, None, None, -1.0, 0)
+    with pytest.raises(RuntimeError):
+        ext().dq_linear(x, qw, s, qz, 4, 32, None, r, -1.0, 0)
+
+
 # ------------------------------------------------ flash prefill
 def _prefill_oracle(q, kc, vc, pos0, T, scale):
     """fp32 attention of queries at positions [pos0, T) against cache
