@@ -21,6 +21,7 @@
 //   n 16384, k 2048    58 -> 28.3    59 -> 45.9    501 -> 377   (8 bits,
 //   n 2048, k 8192    203 -> 24.5   203 -> 32.5    343 -> 233    group 64)
 #include "dq_frag.h"
+#include "lds_dma.h"
 
 namespace {
 
@@ -36,19 +37,6 @@ struct TArgs {
   float* part;                   // [splits, m, n], splits > 1
   int m, n, k, g, splits;
 };
-
-// 16 bytes a lane from base + off to LDS byte `lds` + 16 lane.  The compiler
-// does not see these loads: whoever reads waits for them (vmcnt) first.
-__device__ __forceinline__ void load_to_lds(const void* base, u32 off,
-                                            u32 lds) {
-  asm volatile(
-      "s_mov_b32 m0, %0\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, %2"
-      :
-      : "s"(lds), "v"(off), "s"(base)
-      : "memory", "m0");
-}
 
 template <int BITS, int KC>
 __global__ __launch_bounds__(TPB, 2) void dq_tile_kernel(TArgs A) {
@@ -72,7 +60,7 @@ __global__ __launch_bounds__(TPB, 2) void dq_tile_kernel(TArgs A) {
   const int c0 = (int)((long)C * sp / A.splits);
   const int c1 = (int)((long)C * (sp + 1) / A.splits);
   const int G = A.k / A.g, zw = (G + 32 / BITS - 1) / (32 / BITS);
-  auto key = [](int row) { return SL == 16 ? row & 15 : (row >> 1) & 7; };
+  auto key = [](int row) { return slot_key<SL>(row); };
 
   // staging: a wave's load writes 1 KiB of LDS in lane order, so the lane
   // picks the slot that belongs there; rows past m repeat the last one
@@ -158,8 +146,7 @@ __global__ __launch_bounds__(TPB, 2) void dq_tile_kernel(TArgs A) {
     const char* buf = smem + par * XB;
     // this chunk's loads have landed (a wave waits for its own), the other
     // buffer is consumed
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
+    lds_loads_done();
     s16x8 b[NT][J], xa[2][J];
     float s[NT], sz[NT];
     const int gi = c * KC / A.g;

@@ -122,6 +122,7 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
   const int m = (int)x.size(0), k = (int)x.size(1);
   const int n = (int)qweight.size(0);
   TORCH_CHECK(qweight.size(1) == (long)k * bits / 32, "qweight/k mismatch");
+  if ((uintptr_t)x.data_ptr() % 16) x = x.clone();  // 16-byte loads to LDS
   const void* bptr = nullptr;
   if (bias.has_value()) {
     check_t(*bias, torch::kBFloat16, "bias");
@@ -582,6 +583,7 @@ void hessian_accum(torch::Tensor h, torch::Tensor x) {
   check_t(x, torch::kBFloat16, "x");
   const int t = (int)x.size(0), k = (int)x.size(1);
   TORCH_CHECK(h.size(0) == k && h.size(1) == k, "H must be [k, k]");
+  if ((uintptr_t)x.data_ptr() % 16) x = x.clone();  // 16-byte loads to LDS
   CHECK_HIP(lfmq_hessian_accum(x.data_ptr(), h.data_ptr(), t, k, stream()));
 }
 

@@ -1,111 +1,200 @@
-// K1 — GPTQ Hessian accumulate: H += 2·XᵀX (X bf16 [t, k], H fp32 [k, k]).
+// K1 — GPTQ Hessian accumulate: H += 2·XᵀX (X bf16 [t, k], H fp32 [k, k];
+// SURVEY.md §2.3 K1).
 //
-// MFMA rank-k update: both operands of the (I,J)
-// output tile are column-slices of the SAME X, staged into LDS
-// TRANSPOSED ([col][t] rows, +16-ushort pad for conflict-free
-// ds_read_b128 fragment reads) so A- and B-fragments are contiguous.
-// Full matrix is computed (no triangle+mirror pass: the mirror would
-// re-stream the 822 MB fp32 H of a 14336-wide layer for no win —
-// MFMA flops are free at calibration scale).  One workgroup per 128x128
-// tile; read-modify-write accumulate (one WG owns each tile).
-#include "common.h"
+// Both operands of a product are columns of X, consecutive tokens a lane.
+// Rows of X go from memory straight into LDS as they are, and the transposing
+// LDS read (16 lanes get the 16 columns of a 4 x 16 block) makes operands of
+// them.  H is symmetric but for what it held before: only tiles on and below
+// the diagonal are computed, and each is added to its own place and to its
+// mirror image.
+//
+// A workgroup = 128 x 128, 4 waves of 64 x 64, tokens in steps of 64 through
+// two LDS buffers.  Tiles run in blocks of 8 x 8, one block to an XCD at a
+// time, whose L2 then serves a row of tiles eight times.  Bound by the LDS
+// reads of the fragments and by reading and writing H (in whole lines,
+// through LDS), one after the other.  2048 x 14336: 770 us (547 TFLOP/s of
+// the half computed), against 2102 for the full square staged through
+// transposing 2-byte LDS writes; 2048 x 2048: 33 (70), 64 x 512: 9.3 (8.5).
+#include "lds_dma.h"
 
 namespace {
 
-constexpr int BC = 128;   // columns per tile side
-constexpr int BT = 64;    // token rows per staging step
-constexpr int TPB = 512;
-constexpr int LDT = BT + 16;  // padded [col][t] row length (ushorts)
-typedef s16x8 frag_ab;
+constexpr int TPB = 256, NW = 4;
+constexpr int BC = 128, BK = 64;             // tile side, tokens a step
+constexpr int SB = 8;                        // tiles a side of a block
+constexpr int BUF = 2 * BC * BK * 2;         // both operands of a step
+constexpr int LD = BC + 1;                   // of the result in LDS
 
-__global__ __launch_bounds__(TPB, 1) void hessian_kernel(
-    const u32* __restrict__ x, float* __restrict__ h, int t, int k) {
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
+
+// a step's operand in LDS: [BK tokens][BC columns], 32-byte chunks of a row
+// (16 columns) XOR-swizzled by the token so that the four tokens of a
+// transposing read, and those of neighbouring lane groups, use other banks
+__device__ __forceinline__ int chunk_key(int token) {
+  return (token & 7) ^ ((token >> 1) & 4);
+}
+
+__global__ __launch_bounds__(TPB, 2) void hessian_kernel(
+    const unsigned short* __restrict__ x, float* __restrict__ h, int t,
+    int k, bool direct) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  unsigned short* ldsI = (unsigned short*)smem;             // [BC][LDT]
-  unsigned short* ldsJ = ldsI + BC * LDT;
+  // block (bi, bj) of the lower triangle, tile (r, c) of it
+  const u32 id = xcd_swizzle(blockIdx.x, gridDim.x);
+  const u32 blk = id / (SB * SB);
+  u32 bi = (u32)((sqrtf(8.f * blk + 1.f) - 1.f) * 0.5f);
+  while (bi * (bi + 1) / 2 > blk) --bi;
+  while ((bi + 1) * (bi + 2) / 2 <= blk) ++bi;
+  const u32 bj = blk - bi * (bi + 1) / 2;
+  const int ti = bi * SB + id / SB % SB, tj = bj * SB + id % SB;
+  const int i0 = ti * BC, j0 = tj * BC;
+  if (tj > ti || i0 >= k) return;
 
-  const u32 nbx = (k + BC - 1) / BC;
-  const int cI = (blockIdx.x / nbx) * BC;
-  const int cJ = (blockIdx.x % nbx) * BC;
-
-  const int tid = threadIdx.x;
-  const int lane = tid % LFMQ_WAVE;
-  const int wave = tid / LFMQ_WAVE;
-  const int wm = wave / 4, wn = wave % 4;
-
-  f32x4 acc[4][2];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wi = wave >> 1, wj = wave & 1;
+  const int l15 = lane & 15, l4 = lane >> 4;
+  // staging: a wave's load fills 4 tokens of 256 bytes; tokens past the end
+  // repeat the last one and are cleared below, columns past k are not stored
+  constexpr int NL = BC * BK * 2 / 1024 / NW;          // loads an operand
+  u32 ci[NL], cj[NL];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NL; ++i) {
+    const int tok = (i * NW + wave) * 4 + (lane >> 4);
+    const int c = (((lane & 15) >> 1) ^ chunk_key(tok)) * 16 + (lane & 1) * 8;
+    ci[i] = (i0 + c < k ? c : 0) * 2;
+    cj[i] = (j0 + c < k ? c : 0) * 2;
+  }
+  auto stage = [&](int t0, int buf) {
+    const unsigned short* a = x + (u64)t0 * k + i0;
+    const unsigned short* b = x + (u64)t0 * k + j0;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = {0.f, 0.f, 0.f, 0.f};
-
-  const unsigned short* xs = (const unsigned short*)x;
-  const int tsteps = (t + BT - 1) / BT;
-  for (int ts = 0; ts < tsteps; ++ts) {
-    // stage transposed: thread -> (t_row, 8-col slot); 64 x 16 slots,
-    // each thread handles 2 slots of 8 ushort scattered writes.
-    for (int sl = tid; sl < BT * 16; sl += TPB) {
-      const int tr = sl % BT;          // lanes 0..31 span t -> ~2-way banks
-      const int c8 = (sl / BT) * 8;
-      const int tg = ts * BT + tr;
-#pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        unsigned short* lds = half ? ldsJ : ldsI;
-        const int cbase = half ? cJ : cI;
-        u32x4 v = {0, 0, 0, 0};
-        if (tg < t && cbase + c8 < k) {
-          const unsigned short* src = xs + (u64)tg * k + cbase + c8;
-          v = *(const u32x4*)src;  // 8 cols (16B); k%8==0 required
-        }
-        const unsigned short* vs = (const unsigned short*)&v;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) lds[(c8 + i) * LDT + tr] = vs[i];
-      }
+    for (int i = 0; i < NL; ++i) {
+      const int tok = (i * NW + wave) * 4 + (lane >> 4);
+      const u32 row = (u32)min(tok, t - 1 - t0) * (u32)(k * 2);
+      load_to_lds(a, row + ci[i], buf * BUF + (i * NW + wave) * 1024);
+      load_to_lds(b, row + cj[i], buf * BUF + BUF / 2 + (i * NW + wave) * 1024);
     }
-    __syncthreads();
-
-    // MFMA over this 64-token slab: A rows = cI cols, B cols = cJ cols
+  };
+  // operand: 8 tokens of column c * 16 + l15, in two reads of four
+  auto frag = [&](const char* buf, int ks, int c) {
+    s16x8 f;
 #pragma unroll
-    for (int ks = 0; ks < BT / 32; ++ks) {
-      const int t8 = ks * 32 + (lane >> 4) * 8;
-      frag_ab a[4], b[2];
+    for (int e = 0; e < 2; ++e) {
+      const int tok = ks * 32 + l4 * 8 + e * 4 + (l15 >> 2);
+      const char* p = buf + tok * (BC * 2) + ((c ^ chunk_key(tok)) << 5) +
+                      (l15 & 3) * 8;
+      const s16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) f[e * 4 + i] = v[i];
+    }
+    return f;
+  };
+  f32x4 acc[4][4] = {};
+  stage(0, 0);
+  for (int t0 = 0, par = 0; t0 < t; t0 += BK, par ^= 1) {
+    lds_loads_done();
+    if (t0 + BK < t) {
+      stage(t0 + BK, par ^ 1);
+    } else if (t0 + BK > t) {
+      const u32x4 z = {0, 0, 0, 0};
+      for (int i = (t - t0) * 16 + tid; i < BK * 16; i += TPB) {
+        *(u32x4*)(smem + par * BUF + i * 16) = z;
+        *(u32x4*)(smem + par * BUF + BUF / 2 + i * 16) = z;
+      }
+      __syncthreads();
+    }
+    const char* la = smem + par * BUF;
+    const char* lb = la + BUF / 2;
+#pragma unroll
+    for (int ks = 0; ks < BK / 32; ++ks) {
+      s16x8 a[4], b[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int row = wm * 64 + i * 16 + (lane & 15);
-        a[i] = *(frag_ab*)(ldsI + row * LDT + t8);
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int col = wn * 32 + j * 16 + (lane & 15);
-        b[j] = *(frag_ab*)(ldsJ + col * LDT + t8);
+        a[i] = frag(la, ks, wi * 4 + i);
+        b[i] = frag(lb, ks, wj * 4 + i);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < 4; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
               a[i], b[j], acc[i][j], 0, 0, 0);
     }
-    __syncthreads();
   }
-
-  // epilogue: H[cI+row][cJ+col] += 2*acc
-  const int ccol = cJ + wn * 32 + (lane & 15);
+  // H += 2 acc, here and mirrored.  A single round of workgroups waits for
+  // memory once, straight from the fragments (64 x 512: 9.3 us, 13.9 through
+  // LDS) ...
+  if (direct) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 4; ++i) {
+      const int row = i0 + wi * 64 + i * 16 + l4 * 4;
+      float v[4][4];
+      f32x4 u[4];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = ccol + j * 16;
-      if (col >= k) continue;
+      for (int j = 0; j < 4; ++j) {
+        const int col = j0 + wj * 64 + j * 16 + l15;
+        if (row >= k || col >= k) continue;  // k in eights: four rows alike
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = cI + wm * 64 + i * 16 + (lane >> 4) * 4 + r;
-        if (row < k) {
-          float* p = h + (u64)row * k + col;
-          *p = fmaf(2.f, acc[i][j][r], *p);
+        for (int r = 0; r < 4; ++r) v[j][r] = h[(u64)(row + r) * k + col];
+        if (ti != tj) u[j] = *(const f32x4*)(h + (u64)col * k + row);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int col = j0 + wj * 64 + j * 16 + l15;
+        if (row >= k || col >= k) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          h[(u64)(row + r) * k + col] = fmaf(2.f, acc[i][j][r], v[j][r]);
+          u[j][r] = fmaf(2.f, acc[i][j][r], u[j][r]);
         }
+        if (ti != tj) *(f32x4*)(h + (u64)col * k + row) = u[j];
       }
     }
+    return;
+  }
+  // ... more are bound by the traffic: 64 rows at a time through LDS, so that
+  // whole cache lines are read and written either way (128 x 14336: 346 us,
+  // 707 from the fragments; LD: rows and columns both spread over the banks)
+  float* out = (float*)smem;
+  for (int half = 0; half < 2; ++half) {
+    __syncthreads();
+    if (wi == half) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            out[(i * 16 + l4 * 4 + r) * LD + wj * 64 + j * 16 + l15] =
+                acc[i][j][r];
+    }
+    __syncthreads();
+    // W x (64 BC / W) results at (row0, col0) of H, U of a thread at once
+    auto add = [&](int row0, int col0, int W, int ro, int co) {
+      constexpr int U = 16;
+      const int c = tid & (W - 1), rs = TPB / W;
+      if (col0 + c >= k) return;
+      const int R = min(64 * BC / W, k - row0);
+      float* p = h + (u64)row0 * k + col0;
+      for (int r = tid / W; r < R; r += rs * U) {
+        float v[U];
+#pragma unroll
+        for (int e = 0; e < U; ++e) {
+          const int rr = r + e * rs;
+          if (rr < R) v[e] = p[(u32)(rr * k + c)];
+        }
+#pragma unroll
+        for (int e = 0; e < U; ++e) {
+          const int rr = r + e * rs;
+          if (rr < R)
+            p[(u32)(rr * k + c)] = fmaf(2.f, out[rr * ro + c * co], v[e]);
+        }
+      }
+    };
+    add(i0 + half * 64, j0, BC, LD, 1);
+    if (ti != tj) add(j0, i0 + half * 64, 64, 1, LD);
+  }
 }
 
 }  // namespace
@@ -113,10 +202,12 @@ __global__ __launch_bounds__(TPB, 1) void hessian_kernel(
 hipError_t lfmq_hessian_accum(const void* x, void* h, int t, int k,
                               hipStream_t stream) {
   if (k % 8) return hipErrorInvalidValue;
-  const u32 nb = ceil_div_u32(k, BC);
-  dim3 grid(nb * nb), block(TPB);
-  const size_t lds = 2 * BC * (BT + 16) * sizeof(unsigned short);
-  hipLaunchKernelGGL(hessian_kernel, grid, block, lds, stream, (const u32*)x,
-                     (float*)h, t, k);
+  if (t == 0 || k == 0) return hipSuccess;
+  const u32 n = ceil_div_u32(k, BC * SB), tiles = ceil_div_u32(k, BC);
+  constexpr int lds = 2 * BUF;               // half a result fits
+  static_assert(64 * LD * 4 <= lds, "");
+  hipLaunchKernelGGL(hessian_kernel, dim3(n * (n + 1) / 2 * SB * SB),
+                     dim3(TPB), lds, stream, (const unsigned short*)x,
+                     (float*)h, t, k, tiles * (tiles + 1) / 2 <= 256);
   return hipGetLastError();
 }

@@ -1,0 +1,32 @@
+// Loads from global memory straight into LDS.
+#pragma once
+#include "common.h"
+
+// 16 bytes a lane from base + off (both as the lane sees them; base uniform)
+// to LDS byte `lds` (uniform) + 16 lane.  The compiler does not see these
+// loads: whoever reads the bytes waits for vmcnt first, then for the other
+// waves at a barrier.
+__device__ __forceinline__ void load_to_lds(const void* base, u32 off,
+                                            u32 lds) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2"
+      :
+      : "s"(lds), "v"(off), "s"(base)
+      : "memory", "m0");
+}
+
+// own loads have landed, everybody's after the barrier
+__device__ __forceinline__ void lds_loads_done() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
+// Swizzle of rows of 4, 8 or 16 16-byte slots: the slots of 16 consecutive
+// rows at one column fall into different banks.
+template <int SLOTS>
+__device__ __forceinline__ int slot_key(int row) {
+  static_assert(SLOTS == 4 || SLOTS == 8 || SLOTS == 16, "");
+  return SLOTS == 16 ? row & 15 : (SLOTS == 8 ? (row >> 1) & 7 : (row >> 2) & 3);
+}

@@ -388,6 +388,22 @@ def test_attn_decode_fused_multichunk():
     assert rel_err(o2.reshape(b, hq, 1, d), o_ref) < 2e-2
 
 
+@pytest.mark.parametrize("t,k", [(1, 8), (63, 136), (64, 1024), (129, 1160),
+                                 (70, 2952)])
+def test_hessian_accum_tiles(t, k):
+    """Edges of tiles and steps, both ways to add a tile, an H that is not
+    symmetric.  fp32 sums of t + 1 terms: 2^-24 each."""
+    torch.manual_seed(t + k)
+    x = torch.randn(t, k).to(torch.bfloat16)
+    h = torch.randn(k, k)
+    got = h.to(DEV)
+    ext().hessian_accum(got, x.to(DEV))
+    want = h.double() + 2 * x.double().t() @ x.double()
+    bound = (h.abs() + 2 * x.float().abs().t() @ x.float().abs()) * 2 ** -24
+    assert bool(((got.cpu().double() - want).abs()
+                 <= (t + 1) * bound.double()).all())
+
+
 @pytest.mark.parametrize("b,T,hq,hkv,d", [
     (1, 1, 4, 4, 128), (2, 32, 4, 2, 64), (1, 33, 8, 2, 128),
     (3, 256, 8, 1, 128), (1, 257, 16, 1, 64), (2, 513, 6, 2, 128),
