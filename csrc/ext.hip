@@ -300,7 +300,7 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
   return o;
 }
 
-// EXPERIMENTAL flash prefill (csrc/attn_prefill.hip): q [b,s,hq*d] roped,
+// flash prefill (csrc/attn_prefill.hip): q [b,s,hq*d] roped,
 // caches [b,hkv,tmax,d] holding rows [0, pos0+s).  d == 128 only.
 torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor kc,
                            torch::Tensor vc, long hq, long pos0,
@@ -313,6 +313,9 @@ torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor kc,
   const int d = (int)kc.size(3);
   TORCH_CHECK(q.size(2) == hq * d, "q last dim != hq*d");
   TORCH_CHECK(pos0 + s <= tmax, "cache too small");
+  // 16-byte loads to LDS
+  if ((uintptr_t)kc.data_ptr() % 16) kc = kc.clone();
+  if ((uintptr_t)vc.data_ptr() % 16) vc = vc.clone();
   auto o = torch::empty_like(q);
   CHECK_HIP(lfmq_attn_prefill(q.data_ptr(), kc.data_ptr(), vc.data_ptr(),
                               o.data_ptr(), b, s, (int)hq, hkv, tmax,
@@ -628,7 +631,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("kv_append", &kv_append, "KV cache append");
   m.def("attn_decode", &attn_decode, "GQA decode attention");
   m.def("attn_prefill", &attn_prefill,
-        "EXPERIMENTAL flash prefill attention (LFMQ_FLASH_PREFILL)");
+        "flash prefill attention (LFMQ_FLASH_PREFILL)");
   m.def("hessian_accum", &hessian_accum, "H += 2 X^T X");
   m.def("gptq_block", &gptq_block, "one column block of the GPTQ solve");
   m.def("dq_gemv_gateup", &dq_gemv_gateup, "fused gate_up GEMV + silu*mul");

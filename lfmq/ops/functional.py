@@ -161,8 +161,8 @@ def attn_prefill_fused(q: torch.Tensor, k_cache: torch.Tensor,
                        v_cache: torch.Tensor, pos0: int,
                        scale: Optional[float] = None) -> torch.Tensor:
     """GPU flash prefill (csrc/attn_prefill.hip): one MFMA kernel instead
-    of the rocBLAS matmul chain (measured 3.3-6.3x faster at s 256-2048,
-    rel_err ~4e-3 vs fp32; tools/prefill_flash_bench.py).  q [b, s, hq, d]
+    of the rocBLAS matmul chain (rel_err ~4e-3 vs fp32;
+    tools/prefill_flash_bench.py).  q [b, s, hq, d]
     already roped (the qkv_rope_append output); caches [b, hkv, Tmax, d]
     hold rows [0, pos0+s).  d == 128 only.  Default GPU prefill path;
     LFMQ_FLASH_PREFILL=0 restores the matmul chain."""

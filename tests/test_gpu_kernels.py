@@ -574,6 +574,35 @@ def test_attn_prefill_flash(b, s, pos0):
     assert rel_err(o, o_ref) < 3e-2
 
 
+@pytest.mark.parametrize("b,s,pos0,hq,hkv", [
+    (1, 65, 63, 8, 1), (2, 129, 0, 4, 4), (6, 257, 5, 32, 8)])
+def test_attn_prefill_tiles(b, s, pos0, hq, hkv):
+    """Edges of query and key tiles at both widths of a workgroup (64 and,
+    for the largest, 128 queries); rows that no query may see hold NaN, in
+    the cache and behind a misaligned view of it.  Weights are rounded to
+    bf16 (2^-9 of each, in both terms of the quotient one of them) and so is
+    the result: below 2^-7 of the largest value."""
+    from lfmq.ops import functional as F
+    torch.manual_seed(s)
+    d, T = 128, pos0 + s
+    q = torch.randn(b, s, hq, d).to(torch.bfloat16)
+    kc = torch.randn(b, hkv, T, d).to(torch.bfloat16)
+    vc = torch.randn(b, hkv, T, d).to(torch.bfloat16)
+    want = _prefill_oracle(q, kc, vc, pos0, T, d ** -0.5)
+
+    def cache(c, shift):
+        n = b * hkv * (T + 3) * d
+        t = torch.full((n + shift,), float("nan"), dtype=torch.bfloat16,
+                       device=DEV)[shift:].view(b, hkv, T + 3, d)
+        t[:, :, :T] = c.to(DEV)
+        return t
+
+    for shift in (0, 2):
+        o = F.attn_prefill_fused(q.to(DEV), cache(kc, shift),
+                                 cache(vc, shift), pos0, d ** -0.5)
+        assert rel_err(o, want) < 2 ** -7
+
+
 def test_moe_route_kernel():
     """One-kernel MoE routing vs the torch reference chain."""
     import lfmq_hip
