@@ -35,3 +35,28 @@ __device__ __forceinline__ s16x8 bf16_ones() {
   return __builtin_bit_cast(
       s16x8, u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
 }
+
+// what the packed-product kernels (dq_rows, dq_tile) take
+struct DqArgs {
+  const char* w;                 // [n, k * BITS / 8] bytes
+  const unsigned short* scales;  // [n, G]
+  const u32* zeros;              // [n, zw]
+  const unsigned short* x;       // [m, k]
+  unsigned short* y;             // [m, n]
+  const unsigned short *bias, *resid;
+  float* part;                   // [splits, m, n], splits > 1
+  int m, n, k, g, splits;
+  // experts: w, scales and zeros have one [n, ..] each; a row tile is {expert
+  // (-1: none), first slot, slots}
+  const i32* tiles;
+  const i32* src;                // row of x for a slot, or null: the slot
+  float* y32;                    // [slots, n]
+};
+
+// DENSE: y = x W^T (+ bias) (+ residual).  Of an expert's rows, GLU: W is
+// [gate | up], y [slots, n / 2] = silu(gate) * up; SLOTS: y32 in fp32.
+enum DqMode { DENSE, GLU, SLOTS };
+
+__device__ __forceinline__ float silu_mul_f(float g, float u) {
+  return g / (1.f + __expf(-g)) * u;
+}

@@ -30,18 +30,7 @@ namespace {
 
 constexpr int NW = 4, TPB = NW * LFMQ_WAVE;
 
-struct RArgs {
-  const char* w;                 // [n, k * BITS / 8] bytes
-  const unsigned short* scales;  // [n, G]
-  const u32* zeros;              // [n, zw]
-  const unsigned short* x;       // [m, k]
-  unsigned short* y;             // [m, n]
-  const unsigned short *bias, *resid;
-  float* part;                   // [splits, m, n], splits > 1
-  int m, n, k, g, splits;
-};
-
-__device__ __forceinline__ float epilogue(const RArgs& A, float v, int row,
+__device__ __forceinline__ float epilogue(const DqArgs& A, float v, int row,
                                           int col) {
   if (A.bias != nullptr) v += bf16_bits_to_f32(A.bias[col]);
   if (A.resid != nullptr)
@@ -49,8 +38,8 @@ __device__ __forceinline__ float epilogue(const RArgs& A, float v, int row,
   return v;
 }
 
-template <int BITS, int MT, int NT, int KC>
-__global__ __launch_bounds__(TPB) void dq_rows_kernel(RArgs A) {
+template <int BITS, int MT, int NT, int KC, DqMode MODE>
+__global__ __launch_bounds__(TPB) void dq_rows_kernel(DqArgs A) {
   constexpr int J = KC / 32;                 // products a chunk
   constexpr int WD = J * BITS / 4;           // packed dwords a lane, a chunk
   constexpr int BM = MT * 16, BN = NT * 16, LD = BN + 4;
@@ -59,12 +48,28 @@ __global__ __launch_bounds__(TPB) void dq_rows_kernel(RArgs A) {
   u32* meta = (u32*)red;
   const int lane = threadIdx.x & 63, l15 = lane & 15, l4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n0 = blockIdx.x * BN, m0 = blockIdx.z * BM;
+  // this workgroup's rows, from row0 of x (or slot) on
+  int row0 = blockIdx.z * BM, rows = A.m - row0, expert = 0;
+  if constexpr (MODE != DENSE) {
+    expert = A.tiles[3 * blockIdx.z];
+    if (expert < 0) return;
+    row0 = A.tiles[3 * blockIdx.z + 1];
+    rows = A.tiles[3 * blockIdx.z + 2];
+  }
+  // columns; GLU: the first half of the 16s is gate, the second up
+  constexpr int HT = MODE == GLU ? NT / 2 : NT;
+  const int n0 = blockIdx.x * (HT * 16), half = A.n / 2;
+  auto column = [&](int c) {               // of this workgroup -> of W
+    if (MODE == GLU && c >= HT * 16)
+      return half + min(n0 + c - HT * 16, half - 1);
+    return min(n0 + c, (MODE == GLU ? half : A.n) - 1);
+  };
   const int C = A.k / KC;
   // this wave's chunks: workgroups, then waves, share them evenly
   const int u = blockIdx.y * NW + wave, U = gridDim.y * NW;
   const int c0 = (int)((long)C * u / U), c1 = (int)((long)C * (u + 1) / U);
   const int G = A.k / A.g, zw = (G + 32 / BITS - 1) / (32 / BITS);
+  const u64 first = (u64)expert * A.n;     // the expert's rows of W
 
   // one word a column and group of this workgroup: scale (bf16) above,
   // zero bias below.  Read from memory once; per chunk, its lines of 2-byte
@@ -74,7 +79,7 @@ __global__ __launch_bounds__(TPB) void dq_rows_kernel(RArgs A) {
   const int g0 = w0 * KC / A.g, ng = w1 > w0 ? (w1 - 1) * KC / A.g - g0 + 1 : 0;
   for (int i = threadIdx.x; i < BN * ng; i += TPB) {
     const int col = i / ng, gi = g0 + i % ng;
-    const u64 r = min(n0 + col, A.n - 1);
+    const u64 r = first + column(col);
     const u32 z = A.zeros[r * zw + gi / (32 / BITS)];
     meta[(gi - g0) * BN + col] =
         (u32)A.scales[r * G + gi] << 16 |
@@ -83,13 +88,16 @@ __global__ __launch_bounds__(TPB) void dq_rows_kernel(RArgs A) {
   const char* wr[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const int col = min(n0 + t * 16 + l15, A.n - 1);
-    wr[t] = A.w + (u64)col * (A.k * BITS / 8) + l4 * (WD * 4);
+    const u64 r = first + column(t * 16 + l15);
+    wr[t] = A.w + r * (A.k * BITS / 8) + l4 * (WD * 4);
   }
   u32 xo[MT];                                // byte offsets into x
 #pragma unroll
-  for (int t = 0; t < MT; ++t)
-    xo[t] = ((u32)min(m0 + t * 16 + l15, A.m - 1) * A.k + l4 * (KC / 4)) * 2;
+  for (int t = 0; t < MT; ++t) {
+    int r = row0 + min(t * 16 + l15, rows - 1);
+    if (MODE != DENSE && A.src != nullptr) r = A.src[r];
+    xo[t] = ((u32)r * A.k + l4 * (KC / 4)) * 2;
+  }
 
   const s16x8 ones = bf16_ones();
   f32x4 acc[MT][NT] = {};
@@ -180,38 +188,51 @@ __global__ __launch_bounds__(TPB) void dq_rows_kernel(RArgs A) {
         red[((u32)wave * BM + t * 16 + l4 * 4 + r) * LD + nt * 16 + l15] =
             acc[t][nt][r];
   __syncthreads();
-  const bool wide = A.n % 4 == 0;
-  for (int id = threadIdx.x; id < BM * BN / 4; id += TPB) {
-    const int row = id / (BN / 4), c4 = id % (BN / 4) * 4;
-    const int gr = m0 + row, gc = n0 + c4;
-    if (gr >= A.m || gc >= A.n) continue;
-    f32x4 v = *(const f32x4*)(red + (u32)row * LD + c4);
+  const int nout = MODE == GLU ? half : A.n;
+  const bool wide = nout % 4 == 0;
+  for (int id = threadIdx.x; id < BM * HT * 4; id += TPB) {
+    const int row = id / (HT * 4), c4 = id % (HT * 4) * 4;
+    const int gr = row0 + row, gc = n0 + c4;
+    if (row >= rows || gc >= nout) continue;
+    auto sum = [&](int c) {
+      f32x4 v = *(const f32x4*)(red + (u32)row * LD + c);
 #pragma unroll
-    for (int w = 1; w < NW; ++w)
-      v += *(const f32x4*)(red + ((u32)w * BM + row) * LD + c4);
-    if (gridDim.y > 1) {
-      float* p = A.part + ((u64)blockIdx.y * A.m + gr) * A.n + gc;
+      for (int w = 1; w < NW; ++w)
+        v += *(const f32x4*)(red + ((u32)w * BM + row) * LD + c);
+      return v;
+    };
+    f32x4 v = sum(c4);
+    if constexpr (MODE == GLU) {
+      const f32x4 up = sum(HT * 16 + c4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = silu_mul_f(v[e], up[e]);
+    }
+    if (MODE == SLOTS || (MODE == DENSE && gridDim.y > 1)) {
+      float* p = (MODE == SLOTS ? A.y32 : A.part + (u64)blockIdx.y * A.m * nout)
+                 + (u64)gr * nout + gc;
       if (wide) {
         *(f32x4*)p = v;
       } else {
-        for (int e = 0; e < 4 && gc + e < A.n; ++e) p[e] = v[e];
+        for (int e = 0; e < 4 && gc + e < nout; ++e) p[e] = v[e];
       }
       continue;
     }
-    unsigned short* p = A.y + (u64)gr * A.n + gc;
-    for (int e = 0; e < 4; ++e)
-      if (gc + e < A.n) v[e] = epilogue(A, v[e], gr, gc + e);
+    unsigned short* p = A.y + (u64)gr * nout + gc;
+    if constexpr (MODE == DENSE) {
+      for (int e = 0; e < 4; ++e)
+        if (gc + e < nout) v[e] = epilogue(A, v[e], gr, gc + e);
+    }
     if (wide) {
       *(u64*)p = pack_bf16x2(v[0], v[1]) | (u64)pack_bf16x2(v[2], v[3]) << 32;
     } else {
-      for (int e = 0; e < 4 && gc + e < A.n; ++e)
+      for (int e = 0; e < 4 && gc + e < nout; ++e)
         p[e] = (unsigned short)f32_to_bf16_bits_rne(v[e]);
     }
   }
 }
 
 // y = sum of the splits' parts (+ bias) (+ residual)
-__global__ __launch_bounds__(256) void dq_rows_sum(RArgs A) {
+__global__ __launch_bounds__(256) void dq_rows_sum(DqArgs A) {
   const u64 total = (u64)A.m * A.n;
   if (A.n % 4 == 0) {
     for (u64 id = ((u64)blockIdx.x * 256 + threadIdx.x) * 4; id < total;
@@ -237,7 +258,7 @@ __global__ __launch_bounds__(256) void dq_rows_sum(RArgs A) {
   }
 }
 
-void sum_parts(const RArgs& A, hipStream_t stream) {
+void sum_parts(const DqArgs& A, hipStream_t stream) {
   const u64 items = (u64)A.m * A.n / (A.n % 4 == 0 ? 4 : 1);
   hipLaunchKernelGGL(dq_rows_sum,
                      dim3((u32)min((items + 255) / 256, (u64)1024)),
@@ -262,25 +283,34 @@ size_t meta_bytes(int k, int g, int splits, int nt) {
   return ((size_t)chunks * kc / g + 2) * nt * 16 * 4;
 }
 
-template <int BITS, int MT, int NT, int KC>
-hipError_t go(const RArgs& A, hipStream_t stream) {
+template <int BITS, int MT, int NT, int KC, DqMode MODE = DENSE>
+hipError_t go(const DqArgs& A, int tiles, hipStream_t stream) {
   const size_t sums = (size_t)NW * MT * 16 * (NT * 16 + 4) * 4;
   const size_t lds = max(sums, meta_bytes(A.k, A.g, A.splits, NT));
-  if (lds > 64 * 1024) return hipErrorInvalidValue;
-  const dim3 grid(ceil_div_u32(A.n, NT * 16), A.splits,
-                  ceil_div_u32(A.m, MT * 16));
-  hipLaunchKernelGGL((dq_rows_kernel<BITS, MT, NT, KC>), grid, dim3(TPB), lds,
-                     stream, A);
+  if (lds > 160 * 1024) return hipErrorInvalidValue;
+  static size_t set = 64 * 1024;
+  if (lds > set) {
+    LFMQ_CHECK_HIP(hipFuncSetAttribute(
+        (const void*)dq_rows_kernel<BITS, MT, NT, KC, MODE>,
+        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    set = 160 * 1024;
+  }
+  const int cols = MODE == GLU ? NT * 8 : NT * 16;
+  const dim3 grid(ceil_div_u32(MODE == GLU ? A.n / 2 : A.n, cols), A.splits,
+                  tiles);
+  hipLaunchKernelGGL((dq_rows_kernel<BITS, MT, NT, KC, MODE>), grid, dim3(TPB),
+                     lds, stream, A);
   if (A.splits > 1) sum_parts(A, stream);
   return hipGetLastError();
 }
 
 template <int BITS, int KC>
-hipError_t go_tile(const RArgs& A, hipStream_t stream) {
+hipError_t go_tile(const DqArgs& A, hipStream_t stream) {
   const Tile t = tile_of(A.m);
-  if (t.mt == 1) return go<BITS, 1, 2, KC>(A, stream);
-  if (t.mt == 2) return go<BITS, 2, 4, KC>(A, stream);
-  return go<BITS, 3, 4, KC>(A, stream);
+  const int tiles = ceil_div_u32(A.m, t.mt * 16);
+  if (t.mt == 1) return go<BITS, 1, 2, KC>(A, tiles, stream);
+  if (t.mt == 2) return go<BITS, 2, 4, KC>(A, tiles, stream);
+  return go<BITS, 3, 4, KC>(A, tiles, stream);
 }
 
 }  // namespace
@@ -311,11 +341,11 @@ hipError_t lfmq_dq_rows(const void* qweight, const void* scales,
                         hipStream_t stream) {
   if (!lfmq_dq_rows_ok(m, n, k, g)) return hipErrorInvalidValue;
   if (bits != 4 && bits != 8) return hipErrorInvalidValue;
-  const RArgs A{(const char*)qweight, (const unsigned short*)scales,
-                (const u32*)qzeros, (const unsigned short*)x,
-                (unsigned short*)y, (const unsigned short*)bias,
-                (const unsigned short*)resid, (float*)part, m, n, k, g,
-                splits};
+  const DqArgs A{(const char*)qweight, (const unsigned short*)scales,
+                 (const u32*)qzeros, (const unsigned short*)x,
+                 (unsigned short*)y, (const unsigned short*)bias,
+                 (const unsigned short*)resid, (float*)part, m, n, k, g,
+                 splits, nullptr, nullptr, nullptr};
   const int kc = chunk_of(g);
   if (bits == 4) {
     if (kc == 128) return go_tile<4, 128>(A, stream);
@@ -331,7 +361,7 @@ hipError_t lfmq_dq_rows(const void* qweight, const void* scales,
 hipError_t lfmq_dq_rows_sum(const void* part, void* y, const void* bias,
                             const void* resid, int m, int n, int splits,
                             hipStream_t stream) {
-  RArgs A{};
+  DqArgs A{};
   A.part = (float*)part;
   A.y = (unsigned short*)y;
   A.bias = (const unsigned short*)bias;
@@ -341,4 +371,42 @@ hipError_t lfmq_dq_rows_sum(const void* part, void* y, const void* bias,
   A.splits = splits;
   sum_parts(A, stream);
   return hipGetLastError();
+}
+
+// rows of x (or slots) by expert, tiles of up to 16 of them (DqArgs); glu: y
+// bf16 [slots, n / 2], else fp32 [slots, n]
+hipError_t lfmq_dq_rows_experts(const void* qweight, const void* scales,
+                                const void* qzeros, const void* x,
+                                const void* src, const void* tiles, void* y,
+                                int n_tiles, int n, int k, int g, int bits,
+                                bool glu, hipStream_t stream) {
+  if (g % 32 || g > k || k % g || n % 2) return hipErrorInvalidValue;
+  DqArgs A{};
+  A.w = (const char*)qweight;
+  A.scales = (const unsigned short*)scales;
+  A.zeros = (const u32*)qzeros;
+  A.x = (const unsigned short*)x;
+  A.y = (unsigned short*)y;
+  A.y32 = (float*)y;
+  A.src = (const i32*)src;
+  A.tiles = (const i32*)tiles;
+  A.n = n;
+  A.k = k;
+  A.g = g;
+  A.splits = 1;
+  const int kc = chunk_of(g);
+#define GO(B, KC)                                             \
+  return glu ? go<B, 1, 2, KC, GLU>(A, n_tiles, stream)       \
+             : go<B, 1, 2, KC, SLOTS>(A, n_tiles, stream)
+#define GOB(B)              \
+  do {                      \
+    if (kc == 128) GO(B, 128); \
+    if (kc == 64) GO(B, 64);   \
+    GO(B, 32);              \
+  } while (0)
+  if (bits == 4) GOB(4);
+  if (bits == 8) GOB(8);
+#undef GOB
+#undef GO
+  return hipErrorInvalidValue;
 }

@@ -15,11 +15,11 @@
 // TFLOP/s at 3001 x 28672 x 4096 (4 bits, groups of 128), where 128 x 128
 // tiles of weights unpacked into LDS reached 418.  us a call, before and now:
 //                       64 rows      256 rows      3001 rows
-//   n 28672, k 4096   107 -> 50.7   178 -> 87.9   1690 -> 918
-//   n 4096, k 14336   369 -> 33.1   361 -> 53.7    890 -> 496   (4 bits)
-//   n 6144, k 4096    101 -> 25.2   103 -> 34.4    422 -> 230
-//   n 16384, k 2048    58 -> 28.3    59 -> 45.9    501 -> 377   (8 bits,
-//   n 2048, k 8192    203 -> 24.5   203 -> 32.5    343 -> 233    group 64)
+//   n 28672, k 4096   107 -> 40.2   178 -> 87.9   1690 -> 918
+//   n 4096, k 14336   369 -> 26.4   361 -> 53.7    890 -> 496   (4 bits)
+//   n 6144, k 4096    101 -> 19.5   103 -> 34.4    422 -> 230
+//   n 16384, k 2048    58 -> 24.2    59 -> 45.9    501 -> 377   (8 bits,
+//   n 2048, k 8192    203 -> 20.8   203 -> 32.5    343 -> 233    group 64)
 #include "dq_frag.h"
 #include "lds_dma.h"
 
@@ -27,66 +27,69 @@ namespace {
 
 constexpr int NW = 4, TPB = NW * LFMQ_WAVE;
 
-struct TArgs {
-  const char* w;                 // [n, k * BITS / 8] bytes
-  const unsigned short* scales;  // [n, G]
-  const u32* zeros;              // [n, zw]
-  const unsigned short* x;       // [m, k]
-  unsigned short* y;             // [m, n]
-  const unsigned short* bias;
-  float* part;                   // [splits, m, n], splits > 1
-  int m, n, k, g, splits;
-};
+constexpr int ROWS = 128;                        // of a tile, at most
 
-template <int BITS, int KC>
-__global__ __launch_bounds__(TPB, 2) void dq_tile_kernel(TArgs A) {
-  constexpr int MT = 8, NT = 2, BM = MT * 16, BN = NW * NT * 16;
+// rows row0 .. of x (or slots), MT * 16 of them at most
+template <int BITS, int KC, DqMode MODE, int MT>
+__device__ __forceinline__ void dq_tile_body(const DqArgs& A, char* smem,
+                                             int row0, int rows, int expert,
+                                             int nblk, int sp) {
+  constexpr int NT = 2, BM = MT * 16, BN = NW * NT * 16;
   constexpr int J = KC / 32, WD = J * BITS / 4;
   constexpr int SL = KC / 8;                     // 16-byte slots a row
   constexpr int NX = BM * SL / TPB;              // staged slots a thread
-  constexpr int XB = BM * KC * 2;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+  constexpr int XB = ROWS * KC * 2;
   float* xsum = (float*)(smem + 2 * XB);         // [2][BM]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l15 = lane & 15, l4 = lane >> 4;
-  // an XCD's workgroups share columns: rows run fastest
-  const u32 mb = (A.m + BM - 1) / BM, nb = (A.n + BN - 1) / BN;
-  u32 id = xcd_swizzle(blockIdx.x, gridDim.x);
-  const int m0 = (int)(id % mb) * BM;
-  id /= mb;
-  const int n0 = (int)(id % nb) * BN, sp = (int)(id / nb);
   const int C = A.k / KC;
   const int c0 = (int)((long)C * sp / A.splits);
   const int c1 = (int)((long)C * (sp + 1) / A.splits);
   const int G = A.k / A.g, zw = (G + 32 / BITS - 1) / (32 / BITS);
   auto key = [](int row) { return slot_key<SL>(row); };
+  // columns of this workgroup; GLU: a wave's first 16 are gate, the others up
+  const int half = A.n / 2, n0 = nblk * (MODE == GLU ? BN / 2 : BN);
 
   // staging: a wave's load writes 1 KiB of LDS in lane order, so the lane
-  // picks the slot that belongs there; rows past m repeat the last one
-  u32 xo[NX];
+  // picks the slot that belongs there; rows past the end repeat the last one
+  const unsigned short* xb = MODE == DENSE ? A.x + (u64)row0 * A.k : A.x;
+  constexpr int RS = NW * 64 / SL;               // rows between a lane's slots
+  static_assert(RS % 16 == 0, "which share one swizzle key");
+  const int xrow = wave * 64 / SL + lane / SL;
+  const u32 xslot = ((lane % SL) ^ key(xrow)) * 16, pitch = A.k * 2;
+  u32 xo[MODE == DENSE ? 1 : NX];                // experts: rows by src
+  if constexpr (MODE == DENSE) {
+    xo[0] = xrow * pitch;
+  } else {
 #pragma unroll
-  for (int i = 0; i < NX; ++i) {
-    const int p = (i * NW + wave) * 64 + lane, row = p / SL;
-    xo[i] = ((u32)min(row, A.m - 1 - m0) * A.k +
-             ((p % SL) ^ key(row)) * 8) * 2;
+    for (int i = 0; i < NX; ++i) {
+      int r = row0 + min(xrow + i * RS, rows - 1);
+      if (A.src != nullptr) r = A.src[r];
+      xo[i] = (u32)r * pitch + xslot;
+    }
   }
   auto stage = [&](int c, int buf) {
-    const char* base = (const char*)(A.x + (u64)m0 * A.k + c * KC);
+    const char* base = (const char*)(xb + c * KC);
 #pragma unroll
-    for (int i = 0; i < NX; ++i)
-      load_to_lds(base, xo[i], buf * XB + (i * NW + wave) * 1024);
+    for (int i = 0; i < NX; ++i) {
+      const u32 off = MODE == DENSE ? min(xo[0] + (u32)(i * RS) * pitch,
+                                          (u32)(rows - 1) * pitch) + xslot
+                                    : xo[MODE == DENSE ? 0 : i];
+      load_to_lds(base, off, buf * XB + (i * NW + wave) * 1024);
+    }
   };
-  // weights: rows of this workgroup's columns, within 4 GiB of the first
+  // weights: a matrix is below 4 GiB
   const int wrow = A.k * BITS / 8;
-  const char* wb = A.w + (u64)n0 * wrow;
-  u32 wo[NT], so[NT], zo[NT];
+  const char* wb = A.w + (u64)expert * A.n * wrow;
+  const unsigned short* sb = A.scales + (u64)expert * A.n * G;
+  const u32* zb = A.zeros + (u64)expert * A.n * zw;
+  u32 wo[NT], col[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const int col = min(n0 + (wave * NT + t) * 16 + l15, A.n - 1);
-    wo[t] = (u32)(col - n0) * wrow + l4 * (WD * 4);
-    so[t] = (u32)col * G;
-    zo[t] = (u32)col * zw;
+    col[t] = MODE == GLU ? t * half + min(n0 + wave * 16 + l15, half - 1)
+                         : min(n0 + (wave * NT + t) * 16 + l15, A.n - 1);
+    wo[t] = col[t] * wrow + l4 * (WD * 4);
   }
 
   u32 wn[NT][WD];
@@ -102,16 +105,16 @@ __global__ __launch_bounds__(TPB, 2) void dq_tile_kernel(TArgs A) {
     if (!by8) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        sq[t][0] = A.scales[so[t] + gi];
-        zq[t][0] = A.zeros[zo[t] + gi / (32 / BITS)];
+        sq[t][0] = sb[col[t] * G + gi];
+        zq[t][0] = zb[col[t] * zw + gi / (32 / BITS)];
       }
     } else if (next8) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        sq[t] = *(const u32x4*)(A.scales + so[t] + (gi & ~7));
+        sq[t] = *(const u32x4*)(sb + col[t] * G + (gi & ~7));
 #pragma unroll
         for (int i = 0; i < BITS / 4; ++i)
-          zq[t][i] = A.zeros[zo[t] + (gi & ~7) / (32 / BITS) + i];
+          zq[t][i] = zb[col[t] * zw + (gi & ~7) / (32 / BITS) + i];
       }
     }
 #pragma unroll
@@ -238,70 +241,111 @@ __global__ __launch_bounds__(TPB, 2) void dq_tile_kernel(TArgs A) {
   }
 
   // C fragment: column l15, rows l4 * 4 + r
-  if (A.splits > 1) {
-    float* part = A.part + (u64)sp * A.m * A.n;
+  if (MODE == SLOTS || (MODE == DENSE && A.splits > 1)) {
+    float* part = MODE == SLOTS ? A.y32 : A.part + (u64)sp * A.m * A.n;
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = m0 + t * 16 + l4 * 4 + r;
+        const int row = t * 16 + l4 * 4 + r;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
           const int col = n0 + (wave * NT + nt) * 16 + l15;
-          if (row < A.m && col < A.n)
-            part[(u64)row * A.n + col] = acc[t][nt][r];
+          if (row < rows && col < A.n)
+            part[(u64)(row0 + row) * A.n + col] = acc[t][nt][r];
         }
       }
     return;
   }
   // through LDS, so that rows are written in 16-byte pieces
-  constexpr int LD = BN + 8;
+  constexpr int BO = MODE == GLU ? BN / 2 : BN, LD = BO + 8;
+  const int nout = MODE == GLU ? half : A.n;
   unsigned short* out = (unsigned short*)smem;
+  __syncthreads();
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int c = (wave * NT + nt) * 16 + l15;
-    const float bias = A.bias != nullptr && n0 + c < A.n
+  for (int nt = 0; nt < (MODE == GLU ? 1 : NT); ++nt) {
+    const int c = (MODE == GLU ? wave : wave * NT + nt) * 16 + l15;
+    const float bias = MODE == DENSE && A.bias != nullptr && n0 + c < A.n
                            ? bf16_bits_to_f32(A.bias[n0 + c])
                            : 0.f;
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
+      for (int r = 0; r < 4; ++r) {
+        const float v = MODE == GLU ? silu_mul_f(acc[t][0][r], acc[t][1][r])
+                                    : acc[t][nt][r] + bias;
         out[(t * 16 + l4 * 4 + r) * LD + c] =
-            (unsigned short)f32_to_bf16_bits_rne(acc[t][nt][r] + bias);
+            (unsigned short)f32_to_bf16_bits_rne(v);
+      }
   }
   __syncthreads();
-  const bool wide = A.n % 8 == 0;
-  for (int i = tid; i < BM * BN / 8; i += TPB) {
-    const int row = i / (BN / 8), c = i % (BN / 8) * 8;
-    const int gr = m0 + row, gc = n0 + c;
-    if (gr >= A.m || gc >= A.n) continue;
-    unsigned short* p = A.y + (u64)gr * A.n + gc;
+  const bool wide = nout % 8 == 0;
+  for (int i = tid; i < BM * BO / 8; i += TPB) {
+    const int row = i / (BO / 8), c = i % (BO / 8) * 8;
+    const int gc = n0 + c;
+    if (row >= rows || gc >= nout) continue;
+    unsigned short* p = A.y + (u64)(row0 + row) * nout + gc;
     const unsigned short* q = out + row * LD + c;
     if (wide) {
       *(u32x4*)p = *(const u32x4*)q;
     } else {
-      for (int e = 0; e < 8 && gc + e < A.n; ++e) p[e] = q[e];
+      for (int e = 0; e < 8 && gc + e < nout; ++e) p[e] = q[e];
     }
   }
 }
 
-template <int BITS, int KC>
-hipError_t go(const TArgs& A, hipStream_t stream) {
+// SMALL: tiles of up to 64 rows may occur (experts) or are all (dense)
+template <int BITS, int KC, DqMode MODE, bool SMALL>
+__global__ __launch_bounds__(TPB, 2) void dq_tile_kernel(DqArgs A, int mb) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  // an XCD's workgroups share columns: row tiles run fastest
+  const u32 nb = MODE == GLU ? (A.n / 2 + 63) / 64 : (A.n + 127) / 128;
+  u32 id = xcd_swizzle(blockIdx.x, gridDim.x);
+  const int mt = (int)(id % mb);
+  id /= mb;
+  const int nblk = (int)(id % nb), sp = (int)(id / nb);
+  int row0 = mt * ROWS, rows = min(A.m - row0, ROWS), expert = 0;
+  if constexpr (MODE != DENSE) {
+    expert = A.tiles[3 * mt];
+    if (expert < 0) return;
+    row0 = A.tiles[3 * mt + 1];
+    rows = A.tiles[3 * mt + 2];
+  }
+  if (SMALL && (MODE == DENSE || rows <= 64))
+    dq_tile_body<BITS, KC, MODE, 4>(A, smem, row0, rows, expert, nblk, sp);
+  else
+    dq_tile_body<BITS, KC, MODE, 8>(A, smem, row0, rows, expert, nblk, sp);
+}
+
+template <int BITS, int KC, DqMode MODE, bool SMALL>
+hipError_t go(const DqArgs& A, int mb, hipStream_t stream) {
   // two buffers and the sums; the result, padded, takes a little more
-  constexpr size_t bufs = 2 * 128 * KC * 2 + 2 * 128 * 4, out = 128 * 136 * 2;
+  constexpr size_t bufs = 2 * ROWS * KC * 2 + 2 * ROWS * 4;
+  constexpr size_t out = ROWS * 136 * 2;
   constexpr size_t lds = bufs > out ? bufs : out;
   static bool set = false;
   if (!set && lds > 64 * 1024) {
     LFMQ_CHECK_HIP(hipFuncSetAttribute(
-        (const void*)dq_tile_kernel<BITS, KC>,
+        (const void*)dq_tile_kernel<BITS, KC, MODE, SMALL>,
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     set = true;
   }
-  const u32 grid = ceil_div_u32(A.m, 128) * ceil_div_u32(A.n, 128) * A.splits;
-  hipLaunchKernelGGL((dq_tile_kernel<BITS, KC>), dim3(grid), dim3(TPB), lds,
-                     stream, A);
+  const u32 nb = MODE == GLU ? ceil_div_u32(A.n / 2, 64)
+                             : ceil_div_u32(A.n, 128);
+  hipLaunchKernelGGL((dq_tile_kernel<BITS, KC, MODE, SMALL>),
+                     dim3(mb * nb * A.splits), dim3(TPB), lds, stream, A, mb);
   return hipGetLastError();
+}
+
+template <DqMode MODE, bool SMALL>
+hipError_t go_bits(const DqArgs& A, int bits, int mb, hipStream_t stream) {
+  if (bits == 4)
+    return A.g % 128 == 0 ? go<4, 128, MODE, SMALL>(A, mb, stream)
+                          : go<4, 64, MODE, SMALL>(A, mb, stream);
+  if (bits == 8)
+    return A.g % 128 == 0 ? go<8, 128, MODE, SMALL>(A, mb, stream)
+                          : go<8, 64, MODE, SMALL>(A, mb, stream);
+  return hipErrorInvalidValue;
 }
 
 }  // namespace
@@ -328,18 +372,41 @@ hipError_t lfmq_dq_tile(const void* qweight, const void* scales,
                         const void* qzeros, const void* x, void* y,
                         const void* bias, void* part, int m, int n, int k,
                         int g, int bits, int splits, hipStream_t stream) {
-  if (!lfmq_dq_tile_ok(k, g)) return hipErrorInvalidValue;
-  const TArgs A{(const char*)qweight, (const unsigned short*)scales,
-                (const u32*)qzeros, (const unsigned short*)x,
-                (unsigned short*)y, (const unsigned short*)bias, (float*)part,
-                m, n, k, g, splits};
-  hipError_t e;
-  if (bits == 4)
-    e = g % 128 == 0 ? go<4, 128>(A, stream) : go<4, 64>(A, stream);
-  else if (bits == 8)
-    e = g % 128 == 0 ? go<8, 128>(A, stream) : go<8, 64>(A, stream);
-  else
+  if (!lfmq_dq_tile_ok(k, g) || (u64)n * k * bits / 8 >= 1ull << 32)
     return hipErrorInvalidValue;
+  const DqArgs A{(const char*)qweight, (const unsigned short*)scales,
+                 (const u32*)qzeros, (const unsigned short*)x,
+                 (unsigned short*)y, (const unsigned short*)bias, nullptr,
+                 (float*)part, m, n, k, g, splits, nullptr, nullptr, nullptr};
+  const hipError_t e =
+      m <= 64 ? go_bits<DENSE, true>(A, bits, 1, stream)
+              : go_bits<DENSE, false>(A, bits, ceil_div_u32(m, ROWS), stream);
   if (e != hipSuccess || splits == 1) return e;
   return lfmq_dq_rows_sum(part, y, bias, nullptr, m, n, splits, stream);
+}
+
+// rows of x (or slots) by expert, tiles of up to 128 of them (DqArgs); glu:
+// y bf16 [slots, n / 2], else fp32 [slots, n]
+hipError_t lfmq_dq_tile_experts(const void* qweight, const void* scales,
+                                const void* qzeros, const void* x,
+                                const void* src, const void* tiles, void* y,
+                                int n_tiles, int n, int k, int g, int bits,
+                                bool glu, hipStream_t stream) {
+  if (!lfmq_dq_tile_ok(k, g) || n % 2 || (u64)n * k * bits / 8 >= 1ull << 32)
+    return hipErrorInvalidValue;
+  DqArgs A{};
+  A.w = (const char*)qweight;
+  A.scales = (const unsigned short*)scales;
+  A.zeros = (const u32*)qzeros;
+  A.x = (const unsigned short*)x;
+  A.y = (unsigned short*)y;
+  A.y32 = (float*)y;
+  A.src = (const i32*)src;
+  A.tiles = (const i32*)tiles;
+  A.n = n;
+  A.k = k;
+  A.g = g;
+  A.splits = 1;
+  return glu ? go_bits<GLU, true>(A, bits, n_tiles, stream)
+             : go_bits<SLOTS, true>(A, bits, n_tiles, stream);
 }

@@ -53,17 +53,17 @@ hipError_t lfmq_qkv_rope_append(const void*, void*, void*, void*, const void*,
                                 int, const void*, hipStream_t);
 hipError_t lfmq_advance_record(void*, void*, const void*, void*, int, int,
                                hipStream_t);
-hipError_t lfmq_grouped_dq_gemv(const void*, const void*, const void*,
-                                const void*, void*, const void*, const void*,
-                                const void*, int, int, int, int, int, int,
-                                int, bool, hipStream_t);
-hipError_t lfmq_grouped_dq_gemv_scatter(const void*, const void*, const void*,
-                                        const void*, void*, const void*,
-                                        const void*, const void*, const void*,
-                                        int, int, int, int, int, int,
-                                        hipStream_t);
-hipError_t lfmq_moe_route(const void*, void*, void*, void*, void*, int, int,
-                          int, hipStream_t);
+hipError_t lfmq_moe_route(const void*, void*, void*, void*, void*, void*,
+                          void*, void*, int, int, int, int, int, hipStream_t);
+hipError_t lfmq_moe_tiles(const void*, void*, int, int, int, hipStream_t);
+hipError_t lfmq_moe_sum(const void*, const void*, const void*, void*, int, int,
+                        int, hipStream_t);
+hipError_t lfmq_dq_rows_experts(const void*, const void*, const void*,
+                                const void*, const void*, const void*, void*,
+                                int, int, int, int, int, bool, hipStream_t);
+hipError_t lfmq_dq_tile_experts(const void*, const void*, const void*,
+                                const void*, const void*, const void*, void*,
+                                int, int, int, int, int, bool, hipStream_t);
 hipError_t lfmq_argmax_rows(const void*, void*, void*, void*, int, int,
                             hipStream_t);
 hipError_t lfmq_read_probe(const void*, void*, long, long, int, int, int,
@@ -138,11 +138,13 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
   // through LDS.  us of the first two, n 28672, k 4096, 4 bits: 24.6 / 21.5 at
   // 2 rows but 8.5 / 9.6 at n 6144; 36 / 22 and 11.9 / 9.8 at 4.  8 bits,
   // n 32000, k 2048: 18.5 / 18.7 at 1 row, 29 / 19 at 2.  The last two, 4
-  // bits, n 28672 and 4096: 49 / 50 and 14.4 / 19 at 48 rows, 66 / 51 and
-  // 17 / 20 at 64.
+  // bits, k 4096: n 28672 35.0 / 35.4 at 32 rows, 42 / 35 at 33; n 6144
+  // 15.8 / 16.1 and 18.1 / 16.4; n 4096 still 14.5 / 15.4 at 48.  k 2048, n
+  // 16384 (8 bits): 19.9 / 21.6 at 48.
+  const bool large = k >= 4096 && (long)n * k >= 24l << 20;
   const bool by_rows = (cols_hint == 0 ? m >= (bits == 8 ? 2 : 3)
                                        : cols_hint == 6 && m > 4) &&
-                       m <= 48 && rms_eps < 0 &&
+                       m <= (large ? 32 : 48) && rms_eps < 0 &&
                        lfmq_dq_rows_ok(m, n, k, (int)g);
   if (m > 16) {
     TORCH_CHECK(rptr == nullptr && rms_eps < 0,
@@ -384,94 +386,137 @@ void read_probe(torch::Tensor src, torch::Tensor sink, long row_bytes,
                             stream()));
 }
 
+// one-kernel MoE routing: logits [t, E] bf16 -> (token of a slot, slot
+// weights, first slots of the experts, experts that have any)
+std::vector<torch::Tensor> moe_route(torch::Tensor logits, long topk) {
+  check_t(logits, torch::kBFloat16, "logits");
+  const int t = (int)logits.size(0), E = (int)logits.size(1);
+  TORCH_CHECK(t <= 64, "moe_route takes up to 64 tokens");
+  const auto i32 = logits.options().dtype(torch::kInt32);
+  const auto f32 = logits.options().dtype(torch::kFloat32);
+  auto src_tok = torch::empty({(long)t * topk}, i32);
+  auto slot_w = torch::empty({(long)t * topk}, f32);
+  auto pos = torch::empty({(long)t * topk}, i32);
+  auto w = torch::empty({(long)t * topk}, f32);
+  auto offsets = torch::empty({(long)E + 1}, i32);
+  auto active = torch::empty({(long)E}, i32);
+  CHECK_HIP(lfmq_moe_route(logits.data_ptr(), src_tok.data_ptr(),
+                           slot_w.data_ptr(), pos.data_ptr(), w.data_ptr(),
+                           offsets.data_ptr(), active.data_ptr(), nullptr, t,
+                           E, (int)topk, 1, 0, stream()));
+  return {src_tok, slot_w, offsets, active};
+}
+
+// Rows a tile of the grouped products for `slots` rows over E experts.  us of
+// a layer of 8 experts (4096, 14336, 4 bits) with 16 / 128: 280 / 377 at 12
+// rows an expert, 418 / 397 at 16, 669 / 403 at 32.
+long moe_tile(long slots, long E, long k_in, long g_in, long k_out,
+              long g_out) {
+  return slots > 14 * E && lfmq_dq_tile_ok((int)k_in, (int)g_in) &&
+                 lfmq_dq_tile_ok((int)k_out, (int)g_out)
+             ? 128
+             : 16;
+}
+
+// routing for the grouped products: (token of a slot, slot and weight of a
+// token's choice [t, topk], tiles of bm rows)
+std::vector<torch::Tensor> moe_plan(torch::Tensor logits, long topk, long bm) {
+  check_t(logits, torch::kBFloat16, "logits");
+  const int t = (int)logits.size(0), E = (int)logits.size(1);
+  const long slots = (long)t * topk;
+  const int n_tiles = (int)(slots / bm + std::min((long)E, slots));
+  const auto i32 = logits.options().dtype(torch::kInt32);
+  auto src = torch::empty({slots}, i32);
+  auto pos = torch::empty({t, topk}, i32);
+  auto w = torch::empty({t, topk}, logits.options().dtype(torch::kFloat32));
+  auto tiles = torch::empty({n_tiles, 3}, i32);
+  CHECK_HIP(lfmq_moe_route(logits.data_ptr(), src.data_ptr(), nullptr,
+                           pos.data_ptr(), w.data_ptr(), nullptr, nullptr,
+                           tiles.data_ptr(), t, E, (int)topk, (int)bm, n_tiles,
+                           stream()));
+  return {src, pos, w, tiles};
+}
+
+// rows of x by expert (src: the row of a slot, else the slot itself): glu:
+// bf16 [slots, n / 2] silu(gate) * up of W = [gate | up], else fp32 [slots, n]
+torch::Tensor moe_linear(torch::Tensor x, c10::optional<torch::Tensor> src,
+                         torch::Tensor tiles, torch::Tensor qweight,
+                         torch::Tensor scales, torch::Tensor qzeros, long bits,
+                         long g, bool glu, long bm) {
+  check_t(x, torch::kBFloat16, "x");
+  check_t(tiles, torch::kInt32, "tiles");
+  check_t(qweight, torch::kInt32, "qweight");
+  check_t(scales, torch::kBFloat16, "scales");
+  check_t(qzeros, torch::kInt32, "qzeros");
+  const int n = (int)qweight.size(1), k = (int)x.size(1);
+  TORCH_CHECK(qweight.size(2) == (long)k * bits / 32, "qweight/k mismatch");
+  TORCH_CHECK(x.numel() * 2 < 1l << 32, "x of 4 GiB or more");
+  if ((uintptr_t)x.data_ptr() % 16) x = x.clone();  // 16-byte loads to LDS
+  const void* sptr = nullptr;
+  long slots = x.size(0);
+  if (src.has_value()) {
+    check_t(*src, torch::kInt32, "src");
+    sptr = src->data_ptr();
+    slots = src->numel();
+  }
+  auto y = glu ? torch::empty({slots, (long)n / 2}, x.options())
+               : torch::empty({slots, (long)n},
+                              x.options().dtype(torch::kFloat32));
+  TORCH_CHECK(bm == 16 || bm == 128, "tiles of 16 or 128 rows");
+  const int nt = (int)tiles.size(0);
+  if (nt == 0) return y;
+  if (bm == 128)
+    CHECK_HIP(lfmq_dq_tile_experts(
+        qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
+        sptr, tiles.data_ptr(), y.data_ptr(), nt, n, k, (int)g, (int)bits, glu,
+        stream()));
+  else
+    CHECK_HIP(lfmq_dq_rows_experts(
+        qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
+        sptr, tiles.data_ptr(), y.data_ptr(), nt, n, k, (int)g, (int)bits, glu,
+        stream()));
+  return y;
+}
+
+// y[t] = sum of a token's rows, weighted
+torch::Tensor moe_sum(torch::Tensor rows, torch::Tensor pos, torch::Tensor w) {
+  check_t(rows, torch::kFloat32, "rows");
+  check_t(pos, torch::kInt32, "pos");
+  check_t(w, torch::kFloat32, "w");
+  const long t = pos.size(0), topk = pos.size(1), n = rows.size(1);
+  auto y = torch::empty({t, n}, rows.options().dtype(torch::kBFloat16));
+  CHECK_HIP(lfmq_moe_sum(rows.data_ptr(), pos.data_ptr(), w.data_ptr(),
+                         y.data_ptr(), (int)t, (int)n, (int)topk, stream()));
+  return y;
+}
+
+// slots already sorted by expert: `offsets` [E + 1] says where each begins
+torch::Tensor grouped_tiles(torch::Tensor offsets, long slots) {
+  check_t(offsets, torch::kInt32, "offsets");
+  const int E = (int)offsets.numel() - 1;
+  const int n_tiles = (int)(slots / 16 + std::min((long)E, slots));
+  auto tiles = torch::empty({n_tiles, 3}, offsets.options());
+  if (n_tiles > 0)
+    CHECK_HIP(lfmq_moe_tiles(offsets.data_ptr(), tiles.data_ptr(), E, 16,
+                             n_tiles, stream()));
+  return tiles;
+}
+
 torch::Tensor grouped_dq_gateup(torch::Tensor x, torch::Tensor src_tok,
                                 torch::Tensor offsets, torch::Tensor qweight,
                                 torch::Tensor scales, torch::Tensor qzeros,
                                 long bits, long g,
                                 c10::optional<torch::Tensor> active) {
-  check_t(x, torch::kBFloat16, "x");
-  check_t(qweight, torch::kInt32, "qweight");
-  check_t(src_tok, torch::kInt32, "src_tok");
-  check_t(offsets, torch::kInt32, "offsets");
-  const int E = (int)qweight.size(0), n = (int)qweight.size(1);
-  const int k = (int)x.size(1);
-  const long slots = src_tok.numel();
-  const void* act = nullptr;
-  int grid_e = E;
-  if (active.has_value()) {
-    act = active->data_ptr();
-    grid_e = (int)std::min((long)E, slots);
-  }
-  auto y = torch::empty({slots, (long)(n / 2)}, x.options());
-  CHECK_HIP(lfmq_grouped_dq_gemv(qweight.data_ptr(), scales.data_ptr(),
-                                 qzeros.data_ptr(), x.data_ptr(), y.data_ptr(),
-                                 src_tok.data_ptr(), offsets.data_ptr(), act,
-                                 grid_e, E, n, k, (int)g, (int)bits,
-                                 (int)x.size(0), true, stream()));
-  return y;
-}
-
-// one-kernel MoE routing: logits [t, E] bf16 -> (src_tok, slot_w, offsets)
-std::vector<torch::Tensor> moe_route(torch::Tensor logits, long topk) {
-  check_t(logits, torch::kBFloat16, "logits");
-  const int t = (int)logits.size(0), E = (int)logits.size(1);
-  auto src_tok = torch::empty({(long)t * topk},
-                              logits.options().dtype(torch::kInt32));
-  auto slot_w = torch::empty({(long)t * topk},
-                             logits.options().dtype(torch::kFloat32));
-  auto offsets = torch::empty({(long)E + 1},
-                              logits.options().dtype(torch::kInt32));
-  auto active = torch::empty({(long)E},
-                             logits.options().dtype(torch::kInt32));
-  CHECK_HIP(lfmq_moe_route(logits.data_ptr(), src_tok.data_ptr(),
-                           slot_w.data_ptr(), offsets.data_ptr(),
-                           active.data_ptr(), t, E, (int)topk, stream()));
-  return {src_tok, slot_w, offsets, active};
-}
-
-// w2 grouped GEMV + fused weighted scatter into y_f32 [t, n] (caller zeroed)
-void grouped_dq_linear_scatter(torch::Tensor x, torch::Tensor offsets,
-                               torch::Tensor dst_tok, torch::Tensor slot_w,
-                               torch::Tensor y_f32, torch::Tensor qweight,
-                               torch::Tensor scales, torch::Tensor qzeros,
-                               long bits, long g,
-                               c10::optional<torch::Tensor> active) {
-  check_t(x, torch::kBFloat16, "x");
-  check_t(y_f32, torch::kFloat32, "y_f32");
-  check_t(dst_tok, torch::kInt32, "dst_tok");
-  check_t(slot_w, torch::kFloat32, "slot_w");
-  check_t(offsets, torch::kInt32, "offsets");
-  const int E = (int)qweight.size(0), n = (int)qweight.size(1);
-  const int k = (int)x.size(1);
-  TORCH_CHECK(y_f32.size(1) == n, "y_f32 width mismatch");
-  const void* act = nullptr;
-  int grid_e = E;
-  if (active.has_value()) {
-    act = active->data_ptr();
-    grid_e = std::min((long)E, dst_tok.numel());
-  }
-  CHECK_HIP(lfmq_grouped_dq_gemv_scatter(
-      qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
-      y_f32.data_ptr(), offsets.data_ptr(), dst_tok.data_ptr(),
-      slot_w.data_ptr(), act, grid_e, n, k, (int)g, (int)bits,
-      (int)x.size(0), stream()));
+  return moe_linear(x, src_tok, grouped_tiles(offsets, src_tok.numel()),
+                    qweight, scales, qzeros, bits, g, true, 16);
 }
 
 torch::Tensor grouped_dq_linear(torch::Tensor x, torch::Tensor offsets,
                                 torch::Tensor qweight, torch::Tensor scales,
                                 torch::Tensor qzeros, long bits, long g) {
-  check_t(x, torch::kBFloat16, "x");
-  check_t(qweight, torch::kInt32, "qweight");
-  check_t(offsets, torch::kInt32, "offsets");
-  const int E = (int)qweight.size(0), n = (int)qweight.size(1);
-  const int k = (int)x.size(1);
-  auto y = torch::empty({x.size(0), (long)n}, x.options());
-  CHECK_HIP(lfmq_grouped_dq_gemv(qweight.data_ptr(), scales.data_ptr(),
-                                 qzeros.data_ptr(), x.data_ptr(), y.data_ptr(),
-                                 nullptr, offsets.data_ptr(), nullptr, E, E,
-                                 n, k, (int)g, (int)bits, (int)x.size(0),
-                                 false, stream()));
-  return y;
+  return moe_linear(x, c10::nullopt, grouped_tiles(offsets, x.size(0)),
+                    qweight, scales, qzeros, bits, g, false, 16)
+      .to(torch::kBFloat16);
 }
 
 void advance_record(torch::Tensor state, torch::Tensor tok_buf,
@@ -644,7 +689,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("grouped_dq_gateup", &grouped_dq_gateup, "MoE grouped gate_up+silu");
   m.def("grouped_dq_linear", &grouped_dq_linear, "MoE grouped linear");
   m.def("moe_route", &moe_route, "one-kernel MoE top-k routing");
-  m.def("grouped_dq_linear_scatter", &grouped_dq_linear_scatter,
-        "MoE w2 grouped GEMV + fused weighted scatter");
+  m.def("moe_tile", &moe_tile, "rows a tile of the grouped products");
+  m.def("moe_plan", &moe_plan, "MoE routing with tiles");
+  m.def("moe_linear", &moe_linear, "MoE grouped product over tiles");
+  m.def("moe_sum", &moe_sum, "MoE weighted sum of a token's rows");
   m.def("engine_step", &engine_step, "persistent decode engine step");
 }

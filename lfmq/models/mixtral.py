@@ -117,8 +117,14 @@ class MixtralMoE(nn.Module):
                 "bits": mods[0].bits, "g": mods[0].group_size,
                 "n": mods[0].out_features, "k": mods[0].in_features,
             }
-        self._grouped = g
+        self._grouped, self._grouped_of = g, self._packed_state()
         return g
+
+    def _packed_state(self) -> list:
+        """Which buffers, and which writes to them, consolidate() copied."""
+        return [(t.data_ptr(), t._version) for e in self.experts
+                for m in (e.w13, e.w2) for t in (m.qweight, m.scales,
+                                                 m.qzeros)]
 
     def forward(self, x):
         b, s, h = x.shape
@@ -127,13 +133,27 @@ class MixtralMoE(nn.Module):
         if (x.is_cuda and self._grouped is None
                 and isinstance(self.experts[0].w13, QLinear)):
             self.consolidate()  # lazy one-time stacking for the grouped kernel
-        if x.is_cuda and self._grouped is not None and t * self.top_k <= 64:
-            # routing runs inside _forward_grouped (one moe_route kernel)
-            y2 = self._forward_grouped(x2, None, None)
+        # up to 64 rows always went through the grouped kernels; more do
+        # where the experts are nothing but their packed matrices
+        if x.is_cuda and self._grouped is not None and (
+                t * self.top_k <= 64 or self._plain()):
+            y2 = self._forward_grouped(x2)
         else:
             weights, ids = self.route(x2)
             y2 = self._forward_loop(x2, weights, ids)
         return y2.reshape(b, s, h)
+
+    def _plain(self) -> bool:
+        """The experts are what consolidate() copied, with no act-order
+        gather, bias or hook that their own forward would run, and of shapes
+        that the grouped kernels take."""
+        return self.n_experts <= 64 and self.top_k <= 4 and not any(
+            m._forward_hooks or m._forward_pre_hooks
+            for e in self.experts for m in (e, e.w13, e.w2)) and all(
+            type(m) is QLinear and not hasattr(m, "perm") and m.bias is None
+            and m.group_size % 32 == 0
+            for e in self.experts for m in (e.w13, e.w2)) and \
+            self._grouped_of == self._packed_state()
 
     def _forward_loop(self, x2, weights, ids):
         y = torch.zeros_like(x2)
@@ -148,31 +168,23 @@ class MixtralMoE(nn.Module):
             y[tok_mask] += ye * w.unsqueeze(-1).to(ye.dtype)
         return y
 
-    def _forward_grouped(self, x2, weights, ids):
-        """GPU decode: ONE routing kernel (moe_route: topk+softmax+counting
-        sort), grouped gateup GEMV, then the w2 grouped GEMV with the
-        weighted token scatter FUSED into its epilogue.  5 launches per MoE
-        layer vs ~16 with the round-1 aten chain; all
-        device-side (graph-capturable).  weights/ids args are unused here —
-        routing runs on the raw router logits."""
-        del weights, ids
+    def _forward_grouped(self, x2):
+        """On the device from logits to sum, any number of tokens: routing
+        and row tiles in one kernel, grouped products with silu·mul in the
+        first one's epilogue, weighted sum of a token's rows."""
         from ..ops import hip_ext
-        t = x2.shape[0]
+        ext = hip_ext()
+        a, b = self._grouped["w13"], self._grouped["w2"]
+        bm = ext.moe_tile(x2.shape[0] * self.top_k, self.n_experts, a["k"],
+                          a["g"], b["k"], b["g"])
         logits16 = self.gate(x2)  # dense bf16 router GEMV
-        src_tok, slot_w, offsets, active = hip_ext().moe_route(
-            logits16.contiguous(), self.top_k)
-
-        gg = self._grouped
-        h = hip_ext().grouped_dq_gateup(
-            x2, src_tok, offsets, gg["w13"]["qweight"], gg["w13"]["scales"],
-            gg["w13"]["qzeros"], gg["w13"]["bits"], gg["w13"]["g"], active)
-        y = torch.zeros(t, x2.shape[1], dtype=torch.float32,
-                        device=x2.device)
-        hip_ext().grouped_dq_linear_scatter(
-            h, offsets, src_tok, slot_w, y, gg["w2"]["qweight"],
-            gg["w2"]["scales"], gg["w2"]["qzeros"], gg["w2"]["bits"],
-            gg["w2"]["g"], active)
-        return y.to(x2.dtype)
+        src, pos, w, tiles = ext.moe_plan(logits16.contiguous(), self.top_k,
+                                          bm)
+        h = ext.moe_linear(x2, src, tiles, a["qweight"], a["scales"],
+                           a["qzeros"], a["bits"], a["g"], True, bm)
+        rows = ext.moe_linear(h, None, tiles, b["qweight"], b["scales"],
+                              b["qzeros"], b["bits"], b["g"], False, bm)
+        return ext.moe_sum(rows, pos, w)
 
 
 class MixtralDecoderLayer(nn.Module):

@@ -39,7 +39,6 @@ SOURCES = [
     "csrc/qkv_rope_append.hip",
     "csrc/sample.hip",
     "csrc/probe.hip",
-    "csrc/grouped_dq_gemm.hip",
     "csrc/engine.hip",
     "csrc/moe_route.hip",
 ]

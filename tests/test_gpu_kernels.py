@@ -603,6 +603,81 @@ def test_attn_prefill_tiles(b, s, pos0, hq, hkv):
         assert rel_err(o, want) < 2 ** -7
 
 
+@pytest.mark.parametrize("bits,t,E,top,k,g,inter", [
+    (4, 1, 8, 2, 256, 64, 96), (4, 13, 4, 1, 128, 32, 64),
+    (8, 40, 5, 3, 192, 64, 136), (4, 66, 3, 2, 256, 128, 128),
+    (4, 301, 4, 2, 128, 64, 192), (8, 65, 64, 4, 64, 64, 64)])
+def test_moe_grouped_products(bits, t, E, top, k, g, inter):
+    """Plan, both grouped products and the sum, at both tile heights where
+    the groups allow: experts without rows, tiles with few rows, up to 64
+    experts.  Codes are exact and sums in fp32, so the result is off by the
+    rounding of the activations between the products and its own, 2^-8 in
+    all of the largest value."""
+    torch.manual_seed(t)
+
+    def packed(n, kk):
+        c, s, z = ref.quant_groupwise(torch.randn(E * n, kk), bits, g, False)
+        s = s.to(torch.bfloat16)
+        w = ref.dequant_groupwise(c, s.float(), z, g).view(E, n, kk)
+        return w, [ref.pack_codes(c, bits).view(E, n, -1).to(DEV),
+                   s.view(E, n, -1).to(DEV),
+                   ref.pack_zeros(z, bits).view(E, n, -1).to(DEV)]
+
+    w13, p13 = packed(2 * inter, k)
+    w2, p2 = packed(k, inter) if inter % g == 0 else (None, None)
+    x = torch.randn(t, k).to(torch.bfloat16)
+    # distinct in every row: no ties
+    logits = torch.stack([torch.randperm(E) for _ in range(t)]) \
+        .to(torch.bfloat16) * 0.25
+    logits[:, E // 2] = -9.0 if top < E else 0.1
+    top_l, ids = torch.topk(logits.float(), top, -1)
+    wt = torch.softmax(top_l, -1)
+    x64 = x.double()
+    for bm in (16, 128) if g % 64 == 0 else (16,):
+        src, pos, w, tiles = ext().moe_plan(logits.to(DEV), top, bm)
+        assert torch.equal(src.cpu()[pos.cpu().long()],
+                           torch.arange(t, dtype=torch.int32)
+                           .unsqueeze(1).expand(t, top))
+        assert rel_err(w, wt) < 1e-5
+        h = ext().moe_linear(x.to(DEV), src, tiles, *p13, bits, g, True, bm)
+        want = torch.empty(t, top, inter, dtype=torch.float64)
+        for j in range(top):
+            gu = torch.einsum("tk,tnk->tn", x64, w13[ids[:, j]].double())
+            want[:, j] = torch.nn.functional.silu(gu[:, :inter]) \
+                * gu[:, inter:]
+        assert rel_err(h.cpu()[pos.cpu().long()], want) < 5e-3
+        if p2 is None:
+            continue
+        rows = ext().moe_linear(h, None, tiles, *p2, bits, g, False, bm)
+        y = ext().moe_sum(rows, pos, w)
+        out = sum(wt[:, j:j + 1].double() * torch.einsum(
+            "tk,tnk->tn", want[:, j], w2[ids[:, j]].double())
+            for j in range(top))
+        assert rel_err(y, out) < 2 ** -7
+
+
+def test_mixtral_prompt_sees_new_weights():
+    """A prompt after the experts' packed weights were written again."""
+    from lfmq import QuantConfig
+    from lfmq.models.mixtral import MixtralConfig, MixtralMoE
+    from lfmq.models.qlinear import QLinear
+    torch.manual_seed(3)
+    cfg = MixtralConfig.tiny(hidden_size=256, intermediate_size=256)
+    moe = MixtralMoE(cfg, torch.bfloat16)
+    qc = QuantConfig(scheme="rtn", bits=4, group_size=64)
+    for e in moe.experts:
+        e.w13, e.w2 = QLinear.from_rtn(e.w13, qc), QLinear.from_rtn(e.w2, qc)
+    moe = moe.to(DEV)
+    x = torch.randn(1, 70, 256, device=DEV).to(torch.bfloat16)
+    with torch.no_grad():
+        first = moe(x)
+        assert moe._plain()
+        for e in moe.experts:
+            e.w2.scales.mul_(2)
+        again = moe(x)
+    assert rel_err(again, 2 * first.float()) < 2e-2
+
+
 def test_moe_route_kernel():
     """One-kernel MoE routing vs the torch reference chain."""
     import lfmq_hip
