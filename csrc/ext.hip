@@ -42,6 +42,9 @@ hipError_t lfmq_attn_prefill(const void*, const void*, const void*, void*,
                              int, int, int, int, int, int, int, float,
                              hipStream_t);
 hipError_t lfmq_hessian_accum(const void*, void*, int, int, hipStream_t);
+int lfmq_chol_pad(int n);
+hipError_t lfmq_chol_inverse(const void*, void*, void*, void*, void*, void*,
+                             int, hipStream_t);
 hipError_t lfmq_gptq_block(const void*, const void*, void*, void*, void*,
                            void*, int, int, int, int, int, int, int, bool,
                            hipStream_t);
@@ -635,6 +638,24 @@ void hessian_accum(torch::Tensor h, torch::Tensor x) {
   CHECK_HIP(lfmq_hessian_accum(x.data_ptr(), h.data_ptr(), t, k, stream()));
 }
 
+// U upper triangular, U^T U = h^-1, and [1]: not 0 if h (its lower triangle)
+// is not positive definite in fp32
+std::vector<torch::Tensor> chol_inverse(torch::Tensor h) {
+  check_t(h, torch::kFloat32, "h");
+  TORCH_CHECK(h.dim() == 2 && h.size(0) == h.size(1) && h.size(0) > 0,
+              "h must be [n, n]");
+  const int n = (int)h.size(0);
+  const long np = lfmq_chol_pad(n);
+  auto u = torch::zeros_like(h);
+  auto m = torch::empty({np, np}, h.options());
+  auto s = torch::empty({np + 64, 64}, h.options());
+  auto info = torch::empty({1}, h.options().dtype(torch::kInt32));
+  CHECK_HIP(lfmq_chol_inverse(h.data_ptr(), u.data_ptr(), m.data_ptr(),
+                              s.data_ptr(), s.data_ptr<float>() + np * 64,
+                              info.data_ptr(), n, stream()));
+  return {u, info};
+}
+
 // one column block of the GPTQ solve; returns its errors [n, nb]
 torch::Tensor gptq_block(torch::Tensor w, torch::Tensor ub,
                          torch::Tensor codes, torch::Tensor scales,
@@ -678,6 +699,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prefill", &attn_prefill,
         "flash prefill attention (LFMQ_FLASH_PREFILL)");
   m.def("hessian_accum", &hessian_accum, "H += 2 X^T X");
+  m.def("chol_inverse", &chol_inverse,
+        "upper Cholesky factor of the inverse, and whether there is none");
   m.def("gptq_block", &gptq_block, "one column block of the GPTQ solve");
   m.def("dq_gemv_gateup", &dq_gemv_gateup, "fused gate_up GEMV + silu*mul");
   m.def("qkv_rope_append", &qkv_rope_append, "fused rope + KV append");

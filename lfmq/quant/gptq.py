@@ -4,7 +4,7 @@ inverse, column-blocked quantize-then-error-propagate loop.
 Math (the north star's inventory, BASELINE.json:5):
   H   = Σ 2·XᵀX                      (ops.hessian_accum — HIP K1 on GPU)
   H_d = H + λ·mean(diag H)·I          (λ = damp_percent)
-  U   = chol(H_d⁻¹, upper)            (torch.linalg → rocSOLVER on GPU)
+  U   = chol(H_d⁻¹, upper)            (csrc/chol_inverse.hip on GPU)
   for each column j (in blocks):      q_j = quant(w_j)
       err = (w_j − dq_j) / U_jj ;  w_{j+1..} −= err ⊗ U_{j, j+1..}
 Scales/zeros are recomputed at every group boundary from the
@@ -68,6 +68,19 @@ def _block(w, ub, codes, scales, zeros, i1, cfg, g) -> torch.Tensor:
     return err
 
 
+def _inverse_factor(h: torch.Tensor) -> torch.Tensor:
+    """U upper triangular with UᵀU = h⁻¹."""
+    if h.is_cuda:
+        from ..ops import hip_ext
+        U, failed = hip_ext().chol_inverse(h.contiguous())
+        if not failed.item():
+            return U
+        # a pivot is not positive in this order of elimination
+    L = torch.linalg.cholesky(h)
+    hinv = torch.cholesky_inverse(L)
+    return torch.linalg.cholesky(hinv, upper=True)
+
+
 GPU_BLOCK = 128        # widest block of the HIP kernel: its U fits in LDS
 
 
@@ -111,10 +124,7 @@ def gptq_quantize_layer(
     damp = cfg.damp_percent * torch.diag(h).mean()
     h += torch.eye(k, device=dev) * damp
 
-    # U = chol(H^-1, upper) via the standard two-step (robust on rocSOLVER):
-    L = torch.linalg.cholesky(h)
-    hinv = torch.cholesky_inverse(L)
-    U = torch.linalg.cholesky(hinv, upper=True)
+    U = _inverse_factor(h)
 
     codes = torch.zeros(n, k, dtype=torch.int32, device=dev)
     scales = torch.zeros(n, G, dtype=torch.float32, device=dev)

@@ -34,6 +34,7 @@ SOURCES = [
     "csrc/dq_tile.hip",
     "csrc/hessian.hip",
     "csrc/gptq_block.hip",
+    "csrc/chol_inverse.hip",
     "csrc/attn_decode.hip",
     "csrc/attn_prefill.hip",
     "csrc/qkv_rope_append.hip",

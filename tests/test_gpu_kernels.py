@@ -476,6 +476,39 @@ def test_gptq_block_is_the_tensor_loop(n, k, nb, i1, g, bits, sym):
     assert torch.equal(torch.isfinite(got[0][3]), torch.isfinite(got[1][3]))
 
 
+@pytest.mark.parametrize("n", [1, 17, 64, 65, 130, 300, 513])
+def test_chol_inverse(n):
+    """U of U^T U = H^-1 against 64 bits; only H's lower triangle is read;
+    a matrix that is not positive definite is reported, wherever it fails."""
+    torch.manual_seed(n)
+    x = torch.randn(2 * n + 1, n, device=DEV) + torch.randn(n, device=DEV)
+    h = x.t() @ x + n * torch.eye(n, device=DEV)
+    u, failed = ext().chol_inverse(
+        h.tril() + torch.randn(n, n, device=DEV).triu(1))
+    h64 = h.double().cpu()
+    w = torch.linalg.cholesky(torch.linalg.inv(h64), upper=True)
+    # first-order bound: each rounding (2^-24) moves U by cond(H) at most;
+    # sums of n of them in random directions
+    tol = 2 * math.sqrt(n) * 2 ** -24 * float(torch.linalg.cond(h64))
+    assert failed.item() == 0
+    assert float((u.double().cpu() - w).norm() / w.norm()) <= tol
+    assert float(u.tril(-1).abs().max()) == 0.0
+    for i in {0, n // 2, n - 1}:
+        bad = h.clone()
+        bad[i, i] = -bad[i, i]
+        assert ext().chol_inverse(bad)[1].item() == 1
+
+
+def test_gptq_solve_refuses_what_is_not_positive_definite():
+    from lfmq import QuantConfig
+    from lfmq.quant.gptq import gptq_quantize_layer
+    cfg = QuantConfig(scheme="gptq", bits=4, group_size=32)
+    h = torch.eye(128, device=DEV)
+    h[40, 40] = -3.0
+    with pytest.raises(torch.linalg.LinAlgError):
+        gptq_quantize_layer(torch.randn(16, 128, device=DEV), h, cfg)
+
+
 @pytest.mark.parametrize("m", [5, 8, 16])
 @pytest.mark.parametrize("n,k,g", [(256, 2048, 128), (100, 512, 64),
                                    (48, 4096, 128)])
