@@ -45,6 +45,7 @@ __global__ __launch_bounds__(TPB, 2) void hessian_kernel(
   u32 bi = (u32)((sqrtf(8.f * blk + 1.f) - 1.f) * 0.5f);
   while (bi * (bi + 1) / 2 > blk) --bi;
   while ((bi + 1) * (bi + 2) / 2 <= blk) ++bi;
+  bi = __builtin_amdgcn_readfirstlane(bi);   // the root is a vector operation
   const u32 bj = blk - bi * (bi + 1) / 2;
   const int ti = bi * SB + id / SB % SB, tj = bj * SB + id % SB;
   const int i0 = ti * BC, j0 = tj * BC;
@@ -153,48 +154,46 @@ __global__ __launch_bounds__(TPB, 2) void hessian_kernel(
     }
     return;
   }
-  // ... more are bound by the traffic: 64 rows at a time through LDS, so that
-  // whole cache lines are read and written either way (128 x 14336: 346 us,
-  // 707 from the fragments; LD: rows and columns both spread over the banks)
+  // ... more are bound by the traffic: through LDS, so that 512 bytes of a row
+  // are read and written together either way, 32 elements a thread in flight
+  // (128 x 14336: 341 us, 707 from the fragments; 102 x 7416, whose rows do
+  // not start lines: 100, 105 with halves of the tile and 256 bytes of the
+  // mirror.  LD: rows and columns both spread over the banks)
   float* out = (float*)smem;
-  for (int half = 0; half < 2; ++half) {
-    __syncthreads();
-    if (wi == half) {
+  __syncthreads();
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            out[(i * 16 + l4 * 4 + r) * LD + wj * 64 + j * 16 + l15] =
-                acc[i][j][r];
-    }
-    __syncthreads();
-    // W x (64 BC / W) results at (row0, col0) of H, U of a thread at once
-    auto add = [&](int row0, int col0, int W, int ro, int co) {
-      constexpr int U = 16;
-      const int c = tid & (W - 1), rs = TPB / W;
-      if (col0 + c >= k) return;
-      const int R = min(64 * BC / W, k - row0);
-      float* p = h + (u64)row0 * k + col0;
-      for (int r = tid / W; r < R; r += rs * U) {
-        float v[U];
+      for (int r = 0; r < 4; ++r)
+        out[(wi * 64 + i * 16 + l4 * 4 + r) * LD + wj * 64 + j * 16 + l15] =
+            acc[i][j][r];
+  __syncthreads();
+  // BC x BC results at (row0, col0) of H, U of a thread at once
+  auto add = [&](int row0, int col0, int ro, int co) {
+    constexpr int U = 32;
+    const int c = tid & (BC - 1), rs = TPB / BC;
+    if (col0 + c >= k) return;
+    const int R = min(BC, k - row0);
+    float* p = h + (u64)row0 * k + col0;
+    for (int r = tid / BC; r < R; r += rs * U) {
+      float v[U];
 #pragma unroll
-        for (int e = 0; e < U; ++e) {
-          const int rr = r + e * rs;
-          if (rr < R) v[e] = p[(u32)(rr * k + c)];
-        }
-#pragma unroll
-        for (int e = 0; e < U; ++e) {
-          const int rr = r + e * rs;
-          if (rr < R)
-            p[(u32)(rr * k + c)] = fmaf(2.f, out[rr * ro + c * co], v[e]);
-        }
+      for (int e = 0; e < U; ++e) {
+        const int rr = r + e * rs;
+        if (rr < R) v[e] = p[(u32)(rr * k + c)];
       }
-    };
-    add(i0 + half * 64, j0, BC, LD, 1);
-    if (ti != tj) add(j0, i0 + half * 64, 64, 1, LD);
-  }
+#pragma unroll
+      for (int e = 0; e < U; ++e) {
+        const int rr = r + e * rs;
+        if (rr < R)
+          p[(u32)(rr * k + c)] = fmaf(2.f, out[rr * ro + c * co], v[e]);
+      }
+    }
+  };
+  add(i0, j0, LD, 1);
+  if (ti != tj) add(j0, i0, 1, LD);
 }
 
 }  // namespace
@@ -204,10 +203,10 @@ hipError_t lfmq_hessian_accum(const void* x, void* h, int t, int k,
   if (k % 8) return hipErrorInvalidValue;
   if (t == 0 || k == 0) return hipSuccess;
   const u32 n = ceil_div_u32(k, BC * SB), tiles = ceil_div_u32(k, BC);
-  constexpr int lds = 2 * BUF;               // half a result fits
-  static_assert(64 * LD * 4 <= lds, "");
+  const bool direct = tiles * (tiles + 1) / 2 <= 256;
+  const int lds = direct ? 2 * BUF : max(2 * BUF, BC * LD * 4);
   hipLaunchKernelGGL(hessian_kernel, dim3(n * (n + 1) / 2 * SB * SB),
                      dim3(TPB), lds, stream, (const unsigned short*)x,
-                     (float*)h, t, k, tiles * (tiles + 1) / 2 <= 256);
+                     (float*)h, t, k, direct);
   return hipGetLastError();
 }
