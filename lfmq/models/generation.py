@@ -14,6 +14,7 @@ import torch
 
 from ..config import GenerationConfig
 from ..ops import functional as F
+from .seqcache import upload
 
 
 def _next_token(logits_last: torch.Tensor, gc: Optional[GenerationConfig],
@@ -100,8 +101,8 @@ class PackedStepper:
         batch = self.cache.batch([self.slots[r] for r in ids],
                                  [len(e[1]) for e in entries])
         return self.model.forward_tokens(
-            torch.tensor(flat, device=self.device), batch, self.cache,
-            torch.tensor(select, dtype=torch.int64, device=self.device))
+            upload(flat, None, self.device), batch, self.cache,
+            upload(select, torch.int64, self.device))
 
     def end(self, ids: Sequence[Hashable]) -> None:
         """These requests are finished; their slots are given back."""

