@@ -300,9 +300,15 @@ hipError_t lfmq_latent_ring(const SeqView& sv, const void* own_row,
   return hipGetLastError();
 }
 
-// as many sequences as there are and LDS has room for
-static int sequences_per_pass(int b, int nc, int per_seq) {
-  int nb = b == 1 ? 1 : (b <= 4 ? 4 : 8);
+// Sequences that share a pass over the weights: one, a workgroup each, until
+// that makes `most` workgroups (the weights come from L2 then, and a merge of
+// several sequences is a chain); then as many as there are and LDS has room
+// for.  us with one / with 4 or 8, 16 heads, rank 512, 128 wide: expand 6.4 /
+// 16 for 3 sequences, 14 / 33 for 48, 42 / 29 for 256 (from 2048 workgroups
+// on slower); absorb 3.5 / 3.8 and 4.0 / 5.3 for 8, no faster from 16 on.
+static int sequences_per_pass(int b, int nc, int per_seq, int groups,
+                              int most) {
+  int nb = groups * b <= most ? 1 : (b <= 4 ? 4 : 8);
   while (nb > 1 && (size_t)nb * (per_seq + PW * nc * 64) * 4 > 64 * 1024)
     nb = nb == 8 ? 4 : 1;
   return nb;
@@ -325,7 +331,8 @@ hipError_t lfmq_latent_absorb(const void* q, const void* w, const SeqView& sv,
                               int dim, int rot, int rot_dims, int rank,
                               bool f32, hipStream_t stream) {
   const int nc = rank % 2 == 0 ? 2 : 1;
-  const int nb = sequences_per_pass(sv.b, nc, dim);
+  const int nb = sequences_per_pass(
+      sv.b, nc, dim, heads * ((rank + 64 * nc - 1) / (64 * nc)), 512);
   const dim3 grid((rank + 64 * nc - 1) / (64 * nc), heads,
                   (sv.b + nb - 1) / nb), block(PTPB);
   const size_t lds = (nb * (size_t)dim + PW * nb * nc * 64) * sizeof(float);
@@ -345,7 +352,8 @@ hipError_t lfmq_latent_expand(const void* part, int splits, const void* sink,
                               void* out, int b, int heads, int rank, int vdim,
                               bool f32, hipStream_t stream) {
   const int nc = vdim % 2 == 0 ? 2 : 1;
-  const int nb = sequences_per_pass(b, nc, rank + splits);
+  const int nb = sequences_per_pass(
+      b, nc, rank + splits, heads * ((vdim + 64 * nc - 1) / (64 * nc)), 2048);
   const dim3 grid((vdim + 64 * nc - 1) / (64 * nc), heads, (b + nb - 1) / nb),
       block(PTPB);
   const size_t lds = (nb * (size_t)rank + PW * nb * nc * 64 +

@@ -413,6 +413,30 @@ def test_window_attention_decode(dtype, general, H, dim, rot, rank, dv,
     close(y, want, 3e-5 if dtype == torch.float32 else 3e-2)
 
 
+@pytest.mark.parametrize("nb", [1, 2, 3, 9])
+@pytest.mark.parametrize("H", [4, 700])
+def test_latent_products_do_not_depend_on_the_batch(H, nb):
+    """One sequence a workgroup or several: the same sums in one order."""
+    g = gen(H + nb)
+    dim, rot, rank, dv, splits = 8, 4, 12, 6, 3
+    lens = [5 * i + 1 for i in range(nb)]
+    c = make_cache({"ring": ((64, rank + rot), torch.bfloat16)}, lens)
+    dev = lambda *s: randn(*s, g=g).to(DEV)
+    uk, uv = (dev(H, *s).bfloat16() for s in ((dim, rank), (rank, dv)))
+    q, gate = (dev(nb, H * n).bfloat16() for n in (dim + rot, dv))
+    part, sink = dev(nb, splits, H, rank + 2).abs_(), dev(H)
+    inv = F().rope_inv_freq(rot, 300.0, DEV)
+
+    def both(rows):
+        b = c.batch(rows, [1] * len(rows))
+        return (F().latent_absorb(q[rows], uk, b, c, inv, rot),
+                F().latent_expand(part[rows], sink, uv, gate[rows]))
+
+    for got, one in zip(both(list(range(nb))),
+                        zip(*(both([i]) for i in range(nb)))):
+        assert torch.equal(got, torch.cat(one).view_as(got))
+
+
 # ---------------------------------------------------------------------------
 # models
 # ---------------------------------------------------------------------------
