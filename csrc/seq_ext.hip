@@ -115,6 +115,10 @@ hipError_t lfmq_argmax_rows_any(const void*, void*, void*, void*, int, int,
 hipError_t lfmq_advance_record(void*, void*, const void*, void*, int, int,
                                hipStream_t);
 
+bool lfmq_linear_rows_ok(const void*, long, const void*, int, int, int);
+hipError_t lfmq_linear_rows(const void*, long, const void*, void*, int, int,
+                            int, bool, hipStream_t);
+
 namespace {
 
 #define CHECK_HIP(call)                                                     \
@@ -816,6 +820,29 @@ T_ silu_mul_fused(T_ gu) {
   return y;
 }
 
+// x [..., k] w^T, or silu(gate) * up of it; undefined where the kernel does
+// not take it (its sizes, strides, types)
+c10::optional<T_> linear_rows(T_ x, T_ w, bool glu) {
+  if (!x.is_cuda() || x.device() != w.device() || x.dim() < 1 ||
+      x.scalar_type() != torch::kBFloat16 ||
+      w.scalar_type() != torch::kBFloat16 || w.dim() != 2 ||
+      !w.is_contiguous() || x.size(-1) != w.size(1) ||
+      (x.dim() == 2 ? x.stride(1) != 1 : !x.is_contiguous()))
+    return c10::nullopt;
+  const long k = w.size(1), n = w.size(0), m = k ? x.numel() / k : 0;
+  const long ldx = x.dim() == 2 && m > 1 ? x.stride(0) : k;
+  if (m > 48 || n > INT32_MAX || k > INT32_MAX || (glu && n % 2) ||
+      !lfmq_linear_rows_ok(x.data_ptr(), ldx, w.data_ptr(), (int)m, (int)n,
+                           (int)k))
+    return c10::nullopt;
+  auto sizes = x.sizes().vec();
+  sizes.back() = glu ? n / 2 : n;
+  auto y = torch::empty(sizes, x.options());
+  CHECK_HIP(lfmq_linear_rows(x.data_ptr(), ldx, w.data_ptr(), y.data_ptr(),
+                             (int)m, (int)n, (int)k, glu, stream()));
+  return y;
+}
+
 T_ greedy_sample(T_ logits) {
   const bool f32 = storage(logits, "logits");
   check(logits, logits.scalar_type(), "logits");
@@ -875,6 +902,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_down", &moe_down, "down products of the experts");
   m.def("clamped_glu", &clamped_glu, "clamped GLU on fused gate_up");
   m.def("silu_mul_fused", &silu_mul_fused, "silu-mul on fused gate_up");
+  m.def("linear_rows", &linear_rows, "16-bit product for a few rows, or None");
   m.def("greedy_sample", &greedy_sample, "row argmax");
   m.def("advance_record", &advance_record, "graph decode-state advance");
 }

@@ -35,6 +35,25 @@ def _fp32(n: int, value: float = 0.0) -> nn.Parameter:
     return nn.Parameter(torch.full((n,), value, dtype=torch.float32))
 
 
+class Linear(nn.Linear):
+    """nn.Linear without a bias whose decode steps run on the kernel for a
+    few rows."""
+
+    def __init__(self, n_in: int, n_out: int, dtype):
+        super().__init__(n_in, n_out, bias=False, dtype=dtype)
+
+    def forward(self, x):
+        if self.bias is not None:
+            return super().forward(x)
+        return F.linear(x, self.weight)
+
+    def hooked(self) -> bool:
+        """Whether anyone watches this module's calls."""
+        m = nn.modules.module
+        return bool(self._forward_hooks or self._forward_pre_hooks
+                    or m._global_forward_hooks or m._global_forward_pre_hooks)
+
+
 class ResidualNorm(nn.Module):
     """RMS norm on the fp32 residual stream, fused with adding the previous
     sublayer's output.  centred: the weight is an offset from one."""
@@ -60,13 +79,12 @@ class MLSTMMixer(nn.Module):
         self.heads, self.dim, self.vdim = heads, dim, vdim
         self.cap, self.eps = gate_cap, eps
         # [q | k | v | output gate]
-        self.in_proj = nn.Linear(width, 2 * heads * (dim + vdim), bias=False,
-                                 dtype=dtype)
+        self.in_proj = Linear(width, 2 * heads * (dim + vdim), dtype)
         # [input gate | forget gate], one of each per head
         self.gate_w = nn.Parameter(torch.zeros(2 * heads, width, dtype=dtype))
         self.gate_b = _fp32(2 * heads)
         self.norm_w = _fp32(heads * vdim, 1.0)
-        self.o_proj = nn.Linear(heads * vdim, width, bias=False, dtype=dtype)
+        self.o_proj = Linear(heads * vdim, width, dtype)
 
     def state_spec(self, max_seq: int) -> dict:
         return {"S": ((self.heads, self.dim, self.vdim), torch.float32),
@@ -103,18 +121,16 @@ class LatentAttention(nn.Module):
         self.scale, self.eps = scale, eps
         self.rot_base, self.rot_dims = rot_base, rot_dims
         # [query latent | kv latent | rotated key | output gate]
-        self.in_proj = nn.Linear(
-            width, q_rank + kv_rank + rot_dim + heads * vdim, bias=False,
-            dtype=dtype)
+        self.in_proj = Linear(
+            width, q_rank + kv_rank + rot_dim + heads * vdim, dtype)
         self.q_norm = _fp32(q_rank, 1.0)
         self.kv_norm = _fp32(kv_rank, 1.0)
-        self.q_up = nn.Linear(q_rank, heads * (dim + rot_dim), bias=False,
-                              dtype=dtype)
+        self.q_up = Linear(q_rank, heads * (dim + rot_dim), dtype)
         # rows [keys of all heads | values of all heads]
         self.kv_up = nn.Parameter(torch.zeros(heads * (dim + vdim), kv_rank,
                                               dtype=dtype))
         self.sink = _fp32(heads)
-        self.o_proj = nn.Linear(heads * vdim, width, bias=False, dtype=dtype)
+        self.o_proj = Linear(heads * vdim, width, dtype)
         self._absorbed = None
 
     def state_spec(self, max_seq: int) -> dict:
@@ -248,8 +264,8 @@ class ParallelMixer(nn.Module):
         bs = self.branches.values()
         self.rows_in = sum(b.rows_in for b in bs)
         self.rows_out = sum(b.rows_out for b in bs)
-        self.in_proj = nn.Linear(width, self.rows_in, bias=False, dtype=dtype)
-        self.o_proj = nn.Linear(self.rows_out, width, bias=False, dtype=dtype)
+        self.in_proj = Linear(width, self.rows_in, dtype)
+        self.o_proj = Linear(self.rows_out, width, dtype)
 
     def state_spec(self, max_seq: int) -> dict:
         return {f"{n}.{k}": v for n, b in self.branches.items()
@@ -278,11 +294,17 @@ class DenseMLP(nn.Module):
     def __init__(self, width: int, ff: int, dtype):
         super().__init__()
         self.ff = ff
-        self.gate_up_proj = nn.Linear(width, 2 * ff, bias=False, dtype=dtype)
-        self.down_proj = nn.Linear(ff, width, bias=False, dtype=dtype)
+        self.gate_up_proj = Linear(width, 2 * ff, dtype)
+        self.down_proj = Linear(ff, width, dtype)
 
     def forward(self, h):
-        return self.down_proj(F.silu_mul_gateup(self.gate_up_proj(h), self.ff))
+        g = self.gate_up_proj
+        y = (F.linear_silu_mul(h, g.weight)
+             if type(g) is Linear and g.bias is None and not g.hooked()
+             else None)
+        if y is None:
+            y = F.silu_mul_gateup(g(h), self.ff)
+        return self.down_proj(y)
 
 
 class ExpertSum(NamedTuple):
@@ -302,8 +324,8 @@ class ClampedGLU(nn.Module):
                  beta: float, dtype):
         super().__init__()
         self.act = (limit, alpha, beta)
-        self.gate_up_proj = nn.Linear(width, 2 * ff, bias=False, dtype=dtype)
-        self.down_proj = nn.Linear(ff, width, bias=False, dtype=dtype)
+        self.gate_up_proj = Linear(width, 2 * ff, dtype)
+        self.down_proj = Linear(ff, width, dtype)
 
     def forward(self, h):
         return self.down_proj(F.clamped_glu(self.gate_up_proj(h), *self.act))

@@ -16,8 +16,8 @@ import torch
 import torch.nn as nn
 
 from ..ops import functional as F
-from .mixers import (DenseMLP, LatentAttention, MixerBlock, MLSTMMixer,
-                     ResidualNorm)
+from .mixers import (DenseMLP, LatentAttention, Linear, MixerBlock,
+                     MLSTMMixer, ResidualNorm)
 from .packed import PackedCausalLM
 from .seqcache import SequenceCache, StepBatch
 
@@ -156,7 +156,7 @@ class RapivikForCausalLM(PackedCausalLM):
                     _make_mixer(e, w, eps, dtype), mlp, w, eps, True, dtype)
         self.order = [f"l{cfg.owner(i)}" for i in range(cfg.n_layers)]
         self.norm = ResidualNorm(w, eps, True, dtype)
-        self.lm_head = nn.Linear(w, cfg.vocab_size, bias=False, dtype=dtype)
+        self.lm_head = Linear(w, cfg.vocab_size, dtype)
 
     def layer_mixers(self) -> list:
         return [self.blocks[b].mixer for b in self.order]

@@ -170,7 +170,7 @@ class ZatasunForCausalLM(PackedCausalLM):
             h = h[select]
             if h.shape[0] == 0:
                 return h.new_empty(0, self.cfg.vocab_size)
-        return nn.functional.linear(h, table)
+        return F.linear(h, table)
 
 
 # ---------------------------------------------------------------------------

@@ -104,6 +104,31 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     return ref.silu_mul(gate, up)
 
 
+def _plain(x, w) -> bool:
+    """Tensors that only the values of matter of: no gradient, no subclass,
+    no other dtype wanted."""
+    return (type(x) is torch.Tensor and not torch.is_autocast_enabled()
+            and not (torch.is_grad_enabled()
+                     and (x.requires_grad or w.requires_grad)))
+
+
+def linear(x, w):
+    """x wᵀ.  A few rows of 16-bit values: the kernel for decode steps."""
+    if x.is_cuda and _plain(x, w):
+        y = seq_ext().linear_rows(x, w, False)
+        if y is not None:
+            return y
+    return torch.nn.functional.linear(x, w)
+
+
+def linear_silu_mul(x, w):
+    """silu_mul_gateup(x wᵀ) in one launch, or None where the kernel for
+    decode steps does not take it."""
+    if x.is_cuda and _plain(x, w):
+        return seq_ext().linear_rows(x, w, True)
+    return None
+
+
 def silu_mul_gateup(gate_up: torch.Tensor, inter: int) -> torch.Tensor:
     """silu(gu[..., :inter]) * gu[..., inter:] without materializing the
     split halves (one fused kernel on GPU)."""

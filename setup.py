@@ -59,6 +59,7 @@ SEQ_SOURCES = [
     "csrc/gated_lru.hip",
     "csrc/moe_experts.hip",
     "csrc/post_norm.hip",
+    "csrc/linear_rows.hip",
     "csrc/elementwise.hip",
     "csrc/sample.hip",
 ]

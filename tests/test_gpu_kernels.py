@@ -735,6 +735,50 @@ def test_moe_route_kernel():
                            float(w_ref[tok, j[0, 0]])) < 1e-3
 
 
+# ----------------------------------------------------------- linear_rows
+@pytest.mark.parametrize("m,n,k,glu", [
+    (1, 1, 128, False), (3, 17, 256, False), (16, 33, 1152, False),
+    (5, 6144 + 20, 1152, False), (16, 6144, 2048, False),
+    (8, 37, 2176, False), (7, 2048, 2304, False), (9, 40, 2304, False),
+    (4, 7000, 4224, False), (3, 2 * 23, 1152, True), (16, 2 * 100, 128, True),
+    (2, 2 * 16, 4224, True)])
+def test_linear_rows(m, n, k, glu):
+    from lfmq.ops import functional as F
+    torch.manual_seed(m * n + k)
+    buf = torch.randn(m, k + 64, device=DEV).bfloat16()
+    x = buf[:, 32:32 + k]                      # rows further apart than long
+    w = torch.randn(n, k, device=DEV).bfloat16() / k ** 0.5
+    want = x.double() @ w.double().t()
+    # the result's rounding, and a sum of k products in 32 bits
+    slack = 2 ** -24 * k ** 0.5 * (x.double().abs() @ w.double().abs().t())
+    if glu:
+        (g, u), (sg, su) = want.chunk(2, 1), slack.chunk(2, 1)
+        want = torch.nn.functional.silu(g) * u
+        slack = 1.1 * (sg * u.abs() + su * g.abs()) + 2 ** -20 * want.abs()
+        got = F.linear_silu_mul(x, w)
+    else:
+        from lfmq.ops import seq_ext
+        got = seq_ext().linear_rows(x, w, False)
+        assert torch.equal(got, F.linear(x, w))
+    assert bool(((got.double() - want).abs()
+                 <= 2 ** -8 * want.abs() + slack + 1e-30).all())
+
+
+def test_linear_rows_leaves_the_rest_to_the_library():
+    from lfmq.ops import functional as F
+    from lfmq.ops import seq_ext
+    w = torch.randn(64, 256, device=DEV).bfloat16()
+    x = torch.randn(17, 260, device=DEV).bfloat16()
+    for a, b in ((x[:, :256], w), (x[:4, 4:260], w), (x[:4, :200], w[:, :200]),
+                 (x[:0, :256], w), (x[:4, :256].float(), w.float()),
+                 (x[:4, :256], w.t().contiguous().t())):
+        assert seq_ext().linear_rows(a, b, False) is None
+        assert F.linear(a, b).shape == (a.shape[0], 64)
+    p = torch.nn.Parameter(w)
+    assert F.linear(x[:4, :256].contiguous(), p).requires_grad
+    assert F.linear_silu_mul(x[:4, :256].contiguous(), p) is None
+
+
 # ------------------------------------------------------------- seqcache
 def test_uploads_behind_queued_work_keep_their_numbers():
     """Pinned copies are used again only once they have been read."""
