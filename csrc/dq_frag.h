@@ -51,6 +51,7 @@ struct DqArgs {
   const i32* tiles;
   const i32* src;                // row of x for a slot, or null: the slot
   float* y32;                    // [slots, n]
+  float rms_eps = -1.f;          // >= 0: rows of x over their root mean square
 };
 
 // DENSE: y = x W^T (+ bias) (+ residual).  Of an expert's rows, GLU: W is

@@ -12,23 +12,25 @@
 // lanes read 16 bytes of a packed row at a time (a chunk of KC values of k
 // is split over the four lane groups, x is read in the same order), the next
 // chunk's weights are on their way during this one's products, and no
-// barrier is needed until the four waves of a workgroup, which share k, add
-// their results in LDS.  Where the columns do not fill the chip, k is also
-// split over workgroups; their fp32 sums meet in dq_rows_sum.
+// barrier is needed until the waves of a workgroup, which share k, add
+// their results in LDS.  Where that does not fill the chip, k is also split
+// over workgroups; their fp32 sums meet in dq_rows_sum.
+//
+// What a decode layer has around its products rides along: the root mean
+// square of a row of x is the diagonal of x xT, one more product a chunk,
+// and scales the sums; silu(gate) * up; bias and residual.
 //
 // us a call, before (16-column GEMV tiles up to 16 rows, 128 x 128 tiles
 // above) and now:
 //                       8 rows       24 rows       48 rows
 //   n 28672, k 4096   70.0 -> 24.1  108 -> 31.6   107 -> 49.3
-//   n 4096, k 14336   45.0 -> 17.8  362 -> 20.6   366 -> 29.7   (4 bits)
-//   n 4096, k 4096    13.7 ->  9.0  101 -> 11.9   101 -> 14.4
-//   n 16384, k 2048   75.5 -> 13.8   57 -> 16.1    58 -> 19.9   (8 bits,
+//   n 4096, k 14336   45.0 -> 17.4  362 -> 20.6   366 -> 29.7   (4 bits)
+//   n 4096, k 4096    13.7 ->  8.0  101 -> 11.6   101 -> 14.4
+//   n 16384, k 2048   75.5 -> 12.9   57 -> 15.1    58 -> 18.2   (8 bits,
 //   n 2048, k 8192    25.5 -> 12.0  203 -> 14.1   203 -> 16.6    group 64)
 #include "dq_frag.h"
 
 namespace {
-
-constexpr int NW = 4, TPB = NW * LFMQ_WAVE;
 
 __device__ __forceinline__ float epilogue(const DqArgs& A, float v, int row,
                                           int col) {
@@ -38,8 +40,9 @@ __device__ __forceinline__ float epilogue(const DqArgs& A, float v, int row,
   return v;
 }
 
-template <int BITS, int MT, int NT, int KC, DqMode MODE>
-__global__ __launch_bounds__(TPB) void dq_rows_kernel(DqArgs A) {
+template <int BITS, int MT, int NT, int NW, int KC, DqMode MODE>
+__global__ __launch_bounds__(NW * 64) void dq_rows_kernel(DqArgs A) {
+  constexpr int TPB = NW * 64;
   constexpr int J = KC / 32;                 // products a chunk
   constexpr int WD = J * BITS / 4;           // packed dwords a lane, a chunk
   constexpr int BM = MT * 16, BN = NT * 16, LD = BN + 4;
@@ -50,12 +53,13 @@ __global__ __launch_bounds__(TPB) void dq_rows_kernel(DqArgs A) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // this workgroup's rows, from row0 of x (or slot) on
   int row0 = blockIdx.z * BM, rows = A.m - row0, expert = 0;
-  if constexpr (MODE != DENSE) {
+  if (MODE != DENSE && A.tiles != nullptr) {
     expert = A.tiles[3 * blockIdx.z];
     if (expert < 0) return;
     row0 = A.tiles[3 * blockIdx.z + 1];
     rows = A.tiles[3 * blockIdx.z + 2];
   }
+  const bool rms = MODE != SLOTS && A.rms_eps >= 0.f;
   // columns; GLU: the first half of the 16s is gate, the second up
   constexpr int HT = MODE == GLU ? NT / 2 : NT;
   const int n0 = blockIdx.x * (HT * 16), half = A.n / 2;
@@ -101,6 +105,7 @@ __global__ __launch_bounds__(TPB) void dq_rows_kernel(DqArgs A) {
 
   const s16x8 ones = bf16_ones();
   f32x4 acc[MT][NT] = {};
+  f32x4 sq[MT] = {};                         // x xT: its diagonal
   // WR chunks of weights and XR of x are on their way
   constexpr int WR = MT == 1 ? 4 : 2, XR = MT <= 2 ? 2 : 1;
   u32 wq[WR][NT][WD];
@@ -139,6 +144,13 @@ __global__ __launch_bounds__(TPB) void dq_rows_kernel(DqArgs A) {
       for (int t = 0; t < MT; ++t)
         xs[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[t][j], ones, xs[t],
                                                         0, 0, 0);
+    if (rms)
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+          sq[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[t][j], x[t][j],
+                                                          sq[t], 0, 0, 0);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
       f32x4 a[MT] = {};
@@ -187,7 +199,24 @@ __global__ __launch_bounds__(TPB) void dq_rows_kernel(DqArgs A) {
       for (int r = 0; r < 4; ++r)
         red[((u32)wave * BM + t * 16 + l4 * 4 + r) * LD + nt * 16 + l15] =
             acc[t][nt][r];
+  float* rs = red + NW * BM * LD;            // [BM], after [NW][BM]
+  if (rms) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (l15 == l4 * 4 + r) rs[BM + wave * BM + t * 16 + l15] = sq[t][r];
+  }
   __syncthreads();
+  if (rms) {
+    if (threadIdx.x < BM) {
+      float v = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) v += rs[BM + w * BM + threadIdx.x];
+      rs[threadIdx.x] = rsqrtf(v / (float)A.k + A.rms_eps);
+    }
+    __syncthreads();
+  }
   const int nout = MODE == GLU ? half : A.n;
   const bool wide = nout % 4 == 0;
   for (int id = threadIdx.x; id < BM * HT * 4; id += TPB) {
@@ -202,10 +231,15 @@ __global__ __launch_bounds__(TPB) void dq_rows_kernel(DqArgs A) {
       return v;
     };
     f32x4 v = sum(c4);
+    const float scale = rms ? rs[row] : 1.f;
     if constexpr (MODE == GLU) {
       const f32x4 up = sum(HT * 16 + c4);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = silu_mul_f(v[e], up[e]);
+      for (int e = 0; e < 4; ++e)
+        v[e] = silu_mul_f(v[e] * scale, up[e] * scale);
+    } else if (rms) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] *= scale;
     }
     if (MODE == SLOTS || (MODE == DENSE && gridDim.y > 1)) {
       float* p = (MODE == SLOTS ? A.y32 : A.part + (u64)blockIdx.y * A.m * nout)
@@ -265,15 +299,6 @@ void sum_parts(const DqArgs& A, hipStream_t stream) {
                      dim3(256), 0, stream, A);
 }
 
-struct Tile { int mt, nt; };
-
-// rows and columns (in 16s) of a wave
-Tile tile_of(int m) {
-  if (m <= 16) return {1, 2};
-  if (m <= 32) return {2, 4};
-  return {3, 4};
-}
-
 int chunk_of(int g) { return g % 128 == 0 ? 128 : (g % 64 == 0 ? 64 : 32); }
 
 // scales and zeros of a workgroup: its share of the chunks, which may begin
@@ -283,78 +308,147 @@ size_t meta_bytes(int k, int g, int splits, int nt) {
   return ((size_t)chunks * kc / g + 2) * nt * 16 * 4;
 }
 
-template <int BITS, int MT, int NT, int KC, DqMode MODE = DENSE>
+template <int BITS, int MT, int NT, int NW, int KC, DqMode MODE = DENSE>
 hipError_t go(const DqArgs& A, int tiles, hipStream_t stream) {
-  const size_t sums = (size_t)NW * MT * 16 * (NT * 16 + 4) * 4;
+  const size_t sums =
+      ((size_t)NW * MT * 16 * (NT * 16 + 4) + (NW + 1) * MT * 16) * 4;
   const size_t lds = max(sums, meta_bytes(A.k, A.g, A.splits, NT));
   if (lds > 160 * 1024) return hipErrorInvalidValue;
   static size_t set = 64 * 1024;
   if (lds > set) {
     LFMQ_CHECK_HIP(hipFuncSetAttribute(
-        (const void*)dq_rows_kernel<BITS, MT, NT, KC, MODE>,
+        (const void*)dq_rows_kernel<BITS, MT, NT, NW, KC, MODE>,
         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     set = 160 * 1024;
   }
   const int cols = MODE == GLU ? NT * 8 : NT * 16;
   const dim3 grid(ceil_div_u32(MODE == GLU ? A.n / 2 : A.n, cols), A.splits,
                   tiles);
-  hipLaunchKernelGGL((dq_rows_kernel<BITS, MT, NT, KC, MODE>), grid, dim3(TPB),
+  hipLaunchKernelGGL((dq_rows_kernel<BITS, MT, NT, NW, KC, MODE>), grid, dim3(NW * 64),
                      lds, stream, A);
   if (A.splits > 1) sum_parts(A, stream);
   return hipGetLastError();
 }
 
+// rows and columns (in 16s) of a wave, waves of a workgroup; whole: they
+// take all of k, else it is also split over workgroups
+struct Tile {
+  int mt, nt, nw;
+  bool whole;
+};
+
+// fused: norm or gate, which need whole sums.  us per call, whole / split and
+// summed by a second launch (4 bits but for the last):
+//   n 6144, k 4096        8 rows  9.4 / 10.2    24 rows 13.1 / 14.3
+//   n 4096, k 4096                8.0 /  9.0            11.6 / 12.0
+//   n 4096, k 14336              17.4 / 17.9  16 rows   21.8 / 19.0
+//   n 2048, k 8192               10.9 /  9.7            18.3 / 12.2
+//   n 3072, k 2048                5.6 /  7.5             7.4 / 10.2
+//   n 2048, k 2048 (8 bits)       6.5 /  7.5             8.3 /  9.8
+// 48 rows: n 3072, k 2048 10.0 / 11.9, n 4096, k 4096 18.2 / 14.5; n 16384,
+// k 2048 four or eight waves 17.8 / 14.9.
+Tile tile_of(int m, int n, int k, int g, bool glu, bool fused) {
+  const int mt = m <= 16 ? 1 : (m <= 32 ? 2 : 3);
+  if (g % 64 != 0) return {mt, mt == 1 ? 2 : 4, 4, fused};
+  const bool few = n < 6144 && !glu;         // columns: tiles of 16
+  if (mt == 1) {
+    if (!few) return {1, 2, n >= 16384 ? 4 : 8, true};
+    if (fused || (n >= 2048 && (k <= 4096 || (n >= 4096 && m <= 8))))
+      return {1, 1, 8, true};
+    return {1, 2, 4, false};
+  }
+  if (mt == 2) {
+    if (few && (fused || (n >= 2048 && k <= 4096))) return {2, 1, 8, true};
+    if (!few && !glu && n < 16384 && (fused || k <= 4096))
+      return {2, 2, 4, true};
+    return {2, 4, 4, fused};
+  }
+  if (few && (fused || (n >= 2048 && k <= 2048))) return {3, 1, 8, true};
+  if (glu || n >= 16384) return {3, 4, 8, true};
+  if (fused) return {3, 2, 8, true};
+  return {3, 4, 4, false};
+}
+
 template <int BITS, int KC>
-hipError_t go_tile(const DqArgs& A, hipStream_t stream) {
-  const Tile t = tile_of(A.m);
+hipError_t go_tile(const DqArgs& A, bool glu, hipStream_t stream) {
+  const Tile t = tile_of(A.m, A.n, A.k, A.g, glu, glu || A.rms_eps >= 0.f);
   const int tiles = ceil_div_u32(A.m, t.mt * 16);
-  if (t.mt == 1) return go<BITS, 1, 2, KC>(A, tiles, stream);
-  if (t.mt == 2) return go<BITS, 2, 4, KC>(A, tiles, stream);
-  return go<BITS, 3, 4, KC>(A, tiles, stream);
+#define V(MT, NT, NW)                              \
+  if (t.mt == MT && t.nt == NT && t.nw == NW) \
+    return go<BITS, MT, NT, NW, KC>(A, tiles, stream)
+#define VG(MT, NT, NW)                                                 \
+  if (t.mt == MT && t.nt == NT && t.nw == NW)                          \
+    return glu ? go<BITS, MT, NT, NW, KC, GLU>(A, tiles, stream)       \
+               : go<BITS, MT, NT, NW, KC>(A, tiles, stream)
+  VG(1, 2, 4);
+  VG(2, 4, 4);
+  if constexpr (KC == 32) {
+    VG(3, 4, 4);
+  } else {
+    V(3, 4, 4);
+    VG(1, 2, 8);
+    V(1, 1, 8);
+    V(2, 1, 8);
+    V(2, 2, 4);
+    V(3, 1, 8);
+    V(3, 2, 8);
+    VG(3, 4, 8);
+  }
+#undef V
+#undef VG
+  return hipErrorInvalidValue;
 }
 
 }  // namespace
 
-// false: the shape belongs to another kernel
-bool lfmq_dq_rows_ok(int m, int n, int k, int g) {
-  return g % 32 == 0 && g <= k && k % g == 0 && (u64)m * k * 2 < (1ull << 32);
+// false: the shape belongs to another kernel.  fused: norm or gate
+bool lfmq_dq_rows_ok(int m, int n, int k, int g, bool fused) {
+  if (g % 32 || g > k || k % g || (u64)m * k * 2 >= 1ull << 32) return false;
+  // whole sums: scales and zeros of all groups in LDS
+  return !fused || (m <= 48 && meta_bytes(k, g, 1, 4) <= 96 * 1024);
 }
 
 // workgroups that share k
 int lfmq_dq_rows_splits(int m, int n, int k, int g) {
-  const Tile t = tile_of(m);
+  const Tile t = tile_of(m, n, k, g, false, false);
+  if (t.whole && meta_bytes(k, g, 1, t.nt) <= 64 * 1024) return 1;
   const int wgs = (int)(ceil_div_u32(n, t.nt * 16) * ceil_div_u32(m, t.mt * 16));
   const int C = k / chunk_of(g);
   // 256 workgroups, or 512 where a wave keeps six chunks (us at 8 rows, 2 / 4
   // splits: n 4096, k 4096 9.0 / 9.7, k 14336 18.3 / 17.8)
-  int s = max(1, min(256 / wgs, C / (NW * 2)));
-  if (512 / wgs <= C / (NW * 6)) s = max(s, 512 / wgs);
+  int s = max(1, min(256 / wgs, C / (t.nw * 2)));
+  if (512 / wgs <= C / (t.nw * 6)) s = max(s, 512 / wgs);
   while (meta_bytes(k, g, s, t.nt) > 64 * 1024) ++s;     // LDS of a workgroup
   return s;
 }
 
-// part: splits > 1 only, [splits, m, n] fp32
+// part: splits > 1 only, [splits, m, n] fp32.  rms_eps >= 0: rows of x are
+// scaled by 1 / sqrt(mean x^2 + eps) first; glu: y [m, n / 2] = silu(gate)
+// up of W = [gate | up].  Both with splits 1.
 hipError_t lfmq_dq_rows(const void* qweight, const void* scales,
                         const void* qzeros, const void* x, void* y,
                         const void* bias, const void* resid, void* part,
                         int m, int n, int k, int g, int bits, int splits,
-                        hipStream_t stream) {
-  if (!lfmq_dq_rows_ok(m, n, k, g)) return hipErrorInvalidValue;
+                        float rms_eps, bool glu, hipStream_t stream) {
+  const bool fused = glu || rms_eps >= 0.f;
+  if (!lfmq_dq_rows_ok(m, n, k, g, fused) || (fused && splits != 1) ||
+      (glu && n % 2))
+    return hipErrorInvalidValue;
   if (bits != 4 && bits != 8) return hipErrorInvalidValue;
   const DqArgs A{(const char*)qweight, (const unsigned short*)scales,
                  (const u32*)qzeros, (const unsigned short*)x,
                  (unsigned short*)y, (const unsigned short*)bias,
                  (const unsigned short*)resid, (float*)part, m, n, k, g,
-                 splits, nullptr, nullptr, nullptr};
+                 splits, nullptr, nullptr, nullptr, rms_eps};
   const int kc = chunk_of(g);
   if (bits == 4) {
-    if (kc == 128) return go_tile<4, 128>(A, stream);
-    if (kc == 64) return go_tile<4, 64>(A, stream);
-    return go_tile<4, 32>(A, stream);
+    if (kc == 128) return go_tile<4, 128>(A, glu, stream);
+    if (kc == 64) return go_tile<4, 64>(A, glu, stream);
+    return go_tile<4, 32>(A, glu, stream);
   }
-  if (kc == 128) return go_tile<8, 128>(A, stream);
-  if (kc == 64) return go_tile<8, 64>(A, stream);
-  return go_tile<8, 32>(A, stream);
+  if (kc == 128) return go_tile<8, 128>(A, glu, stream);
+  if (kc == 64) return go_tile<8, 64>(A, glu, stream);
+  return go_tile<8, 32>(A, glu, stream);
 }
 
 // y = sum of part [splits, m, n] (+ bias) (+ residual)
@@ -396,8 +490,8 @@ hipError_t lfmq_dq_rows_experts(const void* qweight, const void* scales,
   A.splits = 1;
   const int kc = chunk_of(g);
 #define GO(B, KC)                                             \
-  return glu ? go<B, 1, 2, KC, GLU>(A, n_tiles, stream)       \
-             : go<B, 1, 2, KC, SLOTS>(A, n_tiles, stream)
+  return glu ? go<B, 1, 2, 4, KC, GLU>(A, n_tiles, stream)       \
+             : go<B, 1, 2, 4, KC, SLOTS>(A, n_tiles, stream)
 #define GOB(B)              \
   do {                      \
     if (kc == 128) GO(B, 128); \

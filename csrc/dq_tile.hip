@@ -370,8 +370,10 @@ hipError_t lfmq_dq_rows_sum(const void* part, void* y, const void* bias,
 
 hipError_t lfmq_dq_tile(const void* qweight, const void* scales,
                         const void* qzeros, const void* x, void* y,
-                        const void* bias, void* part, int m, int n, int k,
-                        int g, int bits, int splits, hipStream_t stream) {
+                        const void* bias, const void* resid, void* part,
+                        int m, int n, int k, int g, int bits, int splits,
+                        hipStream_t stream) {
+  if (resid != nullptr && splits == 1) return hipErrorInvalidValue;
   if (!lfmq_dq_tile_ok(k, g) || (u64)n * k * bits / 8 >= 1ull << 32)
     return hipErrorInvalidValue;
   const DqArgs A{(const char*)qweight, (const unsigned short*)scales,
@@ -382,7 +384,7 @@ hipError_t lfmq_dq_tile(const void* qweight, const void* scales,
       m <= 64 ? go_bits<DENSE, true>(A, bits, 1, stream)
               : go_bits<DENSE, false>(A, bits, ceil_div_u32(m, ROWS), stream);
   if (e != hipSuccess || splits == 1) return e;
-  return lfmq_dq_rows_sum(part, y, bias, nullptr, m, n, splits, stream);
+  return lfmq_dq_rows_sum(part, y, bias, resid, m, n, splits, stream);
 }
 
 // rows of x (or slots) by expert, tiles of up to 128 of them (DqArgs); glu:

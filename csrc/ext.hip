@@ -10,16 +10,17 @@ hipError_t lfmq_unpack(const void*, void*, long, int, int, hipStream_t);
 hipError_t lfmq_dq_gemv(const void*, const void*, const void*, const void*,
                         void*, const void*, const void*, int, int, int, int,
                         int, float, int, hipStream_t);
-bool lfmq_dq_rows_ok(int, int, int, int);
+bool lfmq_dq_rows_ok(int, int, int, int, bool);
 int lfmq_dq_rows_splits(int, int, int, int);
 hipError_t lfmq_dq_rows(const void*, const void*, const void*, const void*,
                         void*, const void*, const void*, void*, int, int, int,
-                        int, int, int, hipStream_t);
+                        int, int, int, float,
+                        bool, hipStream_t);
 bool lfmq_dq_tile_ok(int, int);
 int lfmq_dq_tile_splits(int, int, int, int);
 hipError_t lfmq_dq_tile(const void*, const void*, const void*, const void*,
-                        void*, const void*, void*, int, int, int, int, int,
-                        int, hipStream_t);
+                        void*, const void*, const void*, void*, int, int, int,
+                        int, int, int, hipStream_t);
 hipError_t lfmq_rmsnorm(const void*, const void*, const void*, void*, void*,
                         int, int, float, hipStream_t);
 hipError_t lfmq_rope(void*, void*, const void*, const void*, int, int, int,
@@ -144,14 +145,20 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
   // bits, k 4096: n 28672 35.0 / 35.4 at 32 rows, 42 / 35 at 33; n 6144
   // 15.8 / 16.1 and 18.1 / 16.4; n 4096 still 14.5 / 15.4 at 48.  k 2048, n
   // 16384 (8 bits): 19.9 / 21.6 at 48.
-  const bool large = k >= 4096 && (long)n * k >= 24l << 20;
-  const bool by_rows = (cols_hint == 0 ? m >= (bits == 8 ? 2 : 3)
+  // With the norm, GEMV / rows (n 6144, k 4096, 4 bits): 8.8 / 9.1 at 2 rows,
+  // 12.9 / 9.8 at 4, and norm and product apart: 13.6 / 10.0 at 8, 23.8 /
+  // 20.2 at 48.
+  const bool rms = rms_eps >= 0;
+  const bool large = !rms && k >= 4096 && (long)n * k >= 24l << 20 &&
+                     (rptr == nullptr ||
+                      lfmq_dq_tile_splits(m, n, k, (int)g) > 1);
+  const bool by_rows = (cols_hint == 0 ? m >= (bits == 8 || n >= 16384 ? 2 : 3)
                                        : cols_hint == 6 && m > 4) &&
-                       m <= (large ? 32 : 48) && rms_eps < 0 &&
-                       lfmq_dq_rows_ok(m, n, k, (int)g);
+                       m <= (large ? 32 : 48) &&
+                       lfmq_dq_rows_ok(m, n, k, (int)g, rms);
   if (m > 16) {
-    TORCH_CHECK(rptr == nullptr && rms_eps < 0,
-                "fused rms/resid is a decode (m<=16) path");
+    TORCH_CHECK((by_rows || !rms) && (m <= 48 || rptr == nullptr),
+                "fused rms/resid is a decode (m <= 48) path");
     TORCH_CHECK(lfmq_dq_tile_ok(k, (int)g),
                 "more than 16 rows need groups of a multiple of 64 that "
                 "divide k");
@@ -164,11 +171,11 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
     return part.data_ptr();
   };
   if (by_rows) {
-    const int splits = lfmq_dq_rows_splits(m, n, k, (int)g);
+    const int splits = rms ? 1 : lfmq_dq_rows_splits(m, n, k, (int)g);
     CHECK_HIP(lfmq_dq_rows(qweight.data_ptr(), scales.data_ptr(),
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                            rptr, parts(splits), m, n, k, (int)g, (int)bits,
-                           splits, stream()));
+                           splits, (float)rms_eps, false, stream()));
   } else if (m <= 16) {
     CHECK_HIP(lfmq_dq_gemv(qweight.data_ptr(), scales.data_ptr(),
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
@@ -178,8 +185,8 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
     const int splits = lfmq_dq_tile_splits(m, n, k, (int)g);
     CHECK_HIP(lfmq_dq_tile(qweight.data_ptr(), scales.data_ptr(),
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
-                           parts(splits), m, n, k, (int)g, (int)bits, splits,
-                           stream()));
+                           rptr, parts(splits), m, n, k, (int)g, (int)bits,
+                           splits, stream()));
   }
   return y;
 }
@@ -336,7 +343,21 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
   check_t(qweight, torch::kInt32, "qweight");
   const int m = (int)x.size(0), k = (int)x.size(1);
   const int n = (int)qweight.size(0);
+  TORCH_CHECK(qweight.size(1) == (long)k * bits / 32, "qweight/k mismatch");
   auto y = torch::empty({m, n / 2}, x.options());
+  // as dq_linear.  us with the norm, GEMV / rows, n 28672, k 4096, 4 bits:
+  // 37.5 / 24.0 at 4 rows; norm, product and gate apart / rows: 32.5 / 26.4 at
+  // 8, 44.0 / 37.6 at 32, 46.5 / 49.6 at 48 (n 16384, k 2048: 21.4 / 15.6)
+  if (cols_hint == 0 && m >= (bits == 8 || n >= 16384 ? 2 : 3) && m <= 48 &&
+      n % 2 == 0 &&
+      lfmq_dq_rows_ok(m, n, k, (int)g, true)) {
+    if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
+    CHECK_HIP(lfmq_dq_rows(qweight.data_ptr(), scales.data_ptr(),
+                           qzeros.data_ptr(), x.data_ptr(), y.data_ptr(),
+                           nullptr, nullptr, nullptr, m, n, k, (int)g,
+                           (int)bits, 1, (float)rms_eps, true, stream()));
+    return y;
+  }
   CHECK_HIP(lfmq_dq_gemv_gateup(qweight.data_ptr(), scales.data_ptr(),
                                 qzeros.data_ptr(), x.data_ptr(), y.data_ptr(),
                                 m, n, k, (int)g, (int)bits, (float)rms_eps,

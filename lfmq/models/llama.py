@@ -23,6 +23,7 @@ import torch.nn as nn
 
 from ..ops import functional as F
 from .kvcache import KVCache
+from .qlinear import FEW_ROWS, QLinear, hooked, rows_fused
 
 
 @dataclass
@@ -184,12 +185,13 @@ class LlamaMLP(nn.Module):
         self.inter = cfg.intermediate_size
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        from .qlinear import QLinear
         gp = self.gate_up_proj
         m = x.numel() // x.shape[-1]
-        if (x.is_cuda and m <= 4 and type(gp).forward is QLinear.forward
-                and isinstance(gp, QLinear) and not hasattr(gp, "perm")):
-            # fused gate_up GEMV + silu·mul epilogue (no separate pass)
+        if (x.is_cuda and m <= FEW_ROWS and isinstance(gp, QLinear)
+                and type(gp).forward is QLinear.forward
+                and not hasattr(gp, "perm")
+                and (m <= 4 or (gp.bias is None and rows_fused(gp)))):
+            # fused gate_up product + silu·mul epilogue (no separate pass)
             h = F.dq_gemv_gateup(x, gp.qweight, gp.scales, gp.qzeros,
                                  gp.bits, gp.group_size)
             return self.down_proj(h)
@@ -329,7 +331,6 @@ class LlamaForCausalLM(nn.Module):
         return True
 
     def _decode_fused_ready(self) -> bool:
-        from .qlinear import QLinear
         for layer in self.layers:
             if not (getattr(layer, "_in_norm_folded", False)
                     and getattr(layer, "_post_norm_folded", False)):
@@ -345,6 +346,25 @@ class LlamaForCausalLM(nn.Module):
                     return False
         return True
 
+    def _rows_fused(self) -> bool:
+        """Whether the products of a larger batch may take norm, gate and
+        residual with them."""
+        for layer in self.layers:
+            mlp, att = layer.mlp, layer.self_attn
+            ins, outs = (att.qkv_proj, mlp.gate_up_proj), \
+                        (att.o_proj, mlp.down_proj)
+            if not all(rows_fused(p) for p in ins) or \
+                    mlp.gate_up_proj.bias is not None:
+                return False
+            if not all(isinstance(p, QLinear) and p.group_size % 64 == 0
+                       and not hooked(p) for p in outs):
+                return False
+            if type(mlp).forward is not LlamaMLP.forward or hooked(
+                    layer.input_layernorm, layer.post_attention_layernorm,
+                    mlp):
+                return False
+        return True
+
     def forward_decode_step(self, input_ids, cache, state, max_seq):
         """One hipGraph-capturable decode step: [b,1] ids -> [b,1,vocab]."""
         # persistent weight-streaming engine: the whole layer stack in ONE
@@ -355,8 +375,9 @@ class LlamaForCausalLM(nn.Module):
         x = self.embed_tokens(input_ids)
         if getattr(self, "_fused_decode", None) is None:
             self._fused_decode = self._decode_fused_ready()
-        # the rms/silu-fused GEMV variants are m <= 4 kernels
-        if self._fused_decode and input_ids.shape[0] <= 4:
+        b = input_ids.shape[0]
+        if self._fused_decode and (b <= 4 or (b <= FEW_ROWS
+                                              and self._rows_fused())):
             for i, layer in enumerate(self.layers):
                 x = layer.forward_decode_fused(x, cache.k[i], cache.v[i],
                                                state, max_seq)

@@ -29,6 +29,7 @@ import torch
 import torch.nn as nn
 
 from ..ops import functional as F
+from .qlinear import hooked
 
 
 def _fp32(n: int, value: float = 0.0) -> nn.Parameter:
@@ -46,12 +47,6 @@ class Linear(nn.Linear):
         if self.bias is not None:
             return super().forward(x)
         return F.linear(x, self.weight)
-
-    def hooked(self) -> bool:
-        """Whether anyone watches this module's calls."""
-        m = nn.modules.module
-        return bool(self._forward_hooks or self._forward_pre_hooks
-                    or m._global_forward_hooks or m._global_forward_pre_hooks)
 
 
 class ResidualNorm(nn.Module):
@@ -300,7 +295,7 @@ class DenseMLP(nn.Module):
     def forward(self, h):
         g = self.gate_up_proj
         y = (F.linear_silu_mul(h, g.weight)
-             if type(g) is Linear and g.bias is None and not g.hooked()
+             if type(g) is Linear and g.bias is None and not hooked(g)
              else None)
         if y is None:
             y = F.silu_mul_gateup(g(h), self.ff)

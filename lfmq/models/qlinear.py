@@ -129,6 +129,27 @@ class QLinear(nn.Module):
                            self.bits, self.group_size, self.bias, resid=resid)
 
 
+FEW_ROWS = 48        # rows of the kernel that has norm and gate epilogues
+
+
+def hooked(*modules) -> bool:
+    """Whether anyone watches calls of these modules."""
+    m = nn.modules.module
+    return bool(m._global_forward_hooks or m._global_forward_pre_hooks
+                or any(p._forward_hooks or p._forward_pre_hooks
+                       for p in modules))
+
+
+def rows_fused(p: nn.Module) -> bool:
+    """Whether that kernel may take the norm in front of p, or the gate
+    behind it, for 5 to FEW_ROWS rows: a packed layer as it is, groups that
+    the kernel takes, calls that nobody watches."""
+    return (isinstance(p, QLinear) and type(p).forward is QLinear.forward
+            and not hasattr(p, "perm") and p.group_size % 64 == 0
+            and p.in_features % p.group_size == 0
+            and p.in_features // p.group_size <= 256 and not hooked(p))
+
+
 class Int8PerTensorLinear(nn.Module):
     """Per-tensor symmetric int8 linear — the OPT-125m CPU decode path
     (BASELINE.json config #1).  int8 codes + one fp32 scale."""

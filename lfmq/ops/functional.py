@@ -87,7 +87,8 @@ def dq_linear(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor,
               resid: Optional[torch.Tensor] = None,
               rms_eps: float = -1.0) -> torch.Tensor:
     """Fused dequant-GEMM y = x @ dequant(W)^T (+bias) (+residual)
-    (rms_eps >= 0: fused-RMSNorm input, decode m<=4 GPU path only)."""
+    (rms_eps >= 0: fused-RMSNorm input; with resid, at most 48 rows, on
+    the GPU only)."""
     if x.is_cuda:
         x2 = x.reshape(-1, x.shape[-1])
         r2 = resid.reshape(-1, resid.shape[-1]).contiguous() if resid is not None else None
@@ -251,7 +252,8 @@ def attn_decode_fused(qkv, k_cache, v_cache, state_or_T, max_t: int,
 def dq_gemv_gateup(x: torch.Tensor, qweight: torch.Tensor,
                    scales: torch.Tensor, qzeros: torch.Tensor, bits: int,
                    group_size: int, rms_eps: float = -1.0) -> torch.Tensor:
-    """GPU-only fused gate_up GEMV + silu·mul epilogue (m <= 4);
+    """GPU-only fused gate_up product + silu·mul epilogue (m <= 48;
+    above 4 in groups of a multiple of 32);
     rms_eps >= 0 additionally fuses the RMSNorm of the input."""
     x2 = x.reshape(-1, x.shape[-1])
     y = hip_ext().dq_gemv_gateup(x2, qweight, scales, qzeros, bits,

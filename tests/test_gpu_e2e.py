@@ -137,6 +137,37 @@ def test_fused_fold_decode_matches_unfused():
     assert agree >= 0.75, f"fused vs unfused token agreement {agree}"
 
 
+@pytest.mark.parametrize("b", [2, 6, 20, 48])
+def test_fused_decode_of_a_batch_matches_apart(b):
+    """Norm, gate and residual inside the products of a few rows against
+    kernels of their own, same weights and cache: logits agree to the
+    rounding of the values in between; a hook on a layer is still called."""
+    cfg = LlamaConfig(vocab_size=512, hidden_size=512, intermediate_size=1024,
+                      n_layers=2, n_heads=8, n_kv_heads=2, head_dim=64,
+                      max_seq=64)
+    qcfg = lfmq.QuantConfig(scheme="rtn", bits=4, group_size=64,
+                            fold_rms=True)
+    m = lfmq.quantize(lfmq.build_model(cfg, seed=7), qcfg).to(DEV)
+    ids = torch.randint(0, cfg.vocab_size, (b, 5), device=DEV)
+    out = []
+    calls = []
+    for fused in (True, False):
+        if not fused:
+            assert m._fused_decode and m._rows_fused()
+            h = m.layers[0].mlp.gate_up_proj.register_forward_hook(
+                lambda *a: calls.append(1))
+            assert not m._rows_fused()
+            m._fused_decode = False
+        c = m.make_cache(b, 32)
+        with torch.no_grad():
+            m(ids, c)
+            state = torch.tensor([5, 6, 0], dtype=torch.int32, device=DEV)
+            out.append(m.forward_decode_step(ids[:, :1], c, state, 32).float())
+    assert calls or b <= 4
+    d = (out[0] - out[1]).norm() / out[1].norm()
+    assert float(d) < 0.02, float(d)     # 2 layers of 2^-9 roundings
+
+
 def test_mixtral_gpu_decode():
     """Mixtral on GPU: grouped-kernel decode vs CPU reference logits."""
     from lfmq.models.mixtral import MixtralConfig

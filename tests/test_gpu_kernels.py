@@ -556,6 +556,52 @@ def test_dq_linear_rows_and_tiles(bits, m, n, k, g):
     assert float((err / (want.abs() + 1e-3 * want.abs().max())).max()) < 5e-3
 
 
+@pytest.mark.parametrize("bits,m,n,k,g", [
+    (4, 3, 48, 256, 128), (8, 2, 17, 192, 64), (4, 16, 6208, 256, 64),
+    (4, 5, 72, 96, 32), (4, 2, 16400, 128, 128), (8, 16, 3072, 2048, 128),
+    (4, 17, 100, 384, 128), (8, 32, 6144, 256, 128), (4, 31, 16384, 128, 64),
+    (4, 33, 200, 256, 64), (8, 47, 6150, 128, 128), (4, 48, 16384, 192, 64),
+    (4, 40, 6144, 4096, 128)])
+def test_dq_rows_norm_gate_residual(bits, m, n, k, g):
+    """A few rows with everything a decode layer fuses: the norm of x in
+    front (a row of zeros, one of large values), silu(gate) * up or the
+    residual behind.  Same bound as without: rounding of the result."""
+    torch.manual_seed(m + n)
+    gate = n % 2 == 0
+    codes = torch.randint(0, 1 << bits, (n, k), dtype=torch.int32)
+    zeros = torch.randint(0, 1 << bits, (n, k // g), dtype=torch.int32)
+    s16 = (torch.rand(n, k // g) * 0.02 + 0.01).to(torch.bfloat16)
+    packed = (ref.pack_codes(codes, bits).to(DEV), s16.to(DEV),
+              ref.pack_zeros(zeros, bits).to(DEV))
+    x = torch.randn(m, k).to(torch.bfloat16)
+    x[0] = 0
+    x[m - 1] *= 3000
+    w = ref.dequant_groupwise(codes, s16.float(), zeros, g).double().to(DEV)
+    bias = torch.randn(n).to(torch.bfloat16)
+    resid = torch.randn(m, n).to(torch.bfloat16)
+    xd, b, r = x.to(DEV), bias.to(DEV), resid.to(DEV)
+    eps = 1e-5
+    x64 = xd.double()
+    normed = x64 * torch.rsqrt((x64 ** 2).mean(1, keepdim=True) + eps) @ w.t()
+
+    def close(y, want):
+        err = (y.double() - want).abs()
+        floor = 1e-3 * want.abs().amax(1, keepdim=True) + 1e-30
+        assert float((err / (want.abs() + floor)).max()) < 5e-3
+
+    close(ext().dq_linear(xd, *packed, bits, g, b, None, eps, 0),
+          normed + b.double())
+    close(ext().dq_linear(xd, *packed, bits, g, None, r, -1.0, 0),
+          x64 @ w.t() + r.double())
+    if gate:
+        for e, h in ((eps, normed), (-1.0, x64[:m - 1] @ w.t())):
+            h = h[:m - 1] if e > 0 else h     # one row less: another tile
+            a, u = h.chunk(2, 1)
+            # the gate turns the sums' 2^-24 sqrt(k) into at most its slope
+            close(ext().dq_gemv_gateup(xd[:m - 1], *packed, bits, g, e, 0),
+                  torch.nn.functional.silu(a) * u)
+
+
 def test_dq_linear_refuses():
     """More than 16 rows: groups of 32 and fused epilogues, as ever."""
     x = torch.zeros(17, 96, dtype=torch.bfloat16, device=DEV)
