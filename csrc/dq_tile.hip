@@ -11,15 +11,17 @@
 // The sums of x that the zeros need are shared out: a wave makes a quarter
 // of the rows' with products by ones, and all waves apply them a chunk later.
 //
-// Bound by the issue of products, unpacking and scaling together: 768
-// TFLOP/s at 3001 x 28672 x 4096 (4 bits, groups of 128), where 128 x 128
-// tiles of weights unpacked into LDS reached 418.  us a call, before and now:
+// Bound by latencies between the stages of two waves a SIMD (matrix cores
+// busy 41 % of the time, vector units 46 %, LDS half): 777 TFLOP/s at 3001 x
+// 28672 x 4096 (4 bits, groups of 128), where 128 x 128 tiles of weights
+// unpacked into LDS reached 418.  128 x 256 tiles with one wave a SIMD: 570.
+// LDS slots without bank conflicts: the same time.  us a call, before and now:
 //                       64 rows      256 rows      3001 rows
-//   n 28672, k 4096   107 -> 40.2   178 -> 87.9   1690 -> 918
-//   n 4096, k 14336   369 -> 26.4   361 -> 53.7    890 -> 496   (4 bits)
-//   n 6144, k 4096    101 -> 19.5   103 -> 34.4    422 -> 230
-//   n 16384, k 2048    58 -> 24.2    59 -> 45.9    501 -> 377   (8 bits,
-//   n 2048, k 8192    203 -> 20.8   203 -> 32.5    343 -> 233    group 64)
+//   n 28672, k 4096   107 -> 40.2   178 -> 87.5   1690 -> 907
+//   n 4096, k 14336   369 -> 26.4   361 -> 52.2    890 -> 506   (4 bits)
+//   n 6144, k 4096    101 -> 19.5   103 -> 32.6    422 -> 216
+//   n 16384, k 2048    58 -> 24.2    59 -> 46.2    501 -> 360   (8 bits,
+//   n 2048, k 8192    203 -> 20.8   203 -> 31.1    343 -> 233    group 64)
 #include "dq_frag.h"
 #include "lds_dma.h"
 
@@ -186,6 +188,11 @@ __device__ __forceinline__ void dq_tile_body(const DqArgs& A, char* smem,
         for (int r = 0; r < 4; ++r)
           acc[t][nt][r] = fmaf(s[nt], a[t & 1][nt][r],
                                fmaf(-szp[nt], xp[t & 1][r], acc[t][nt][r]));
+      // here: sunk behind all products, as the compiler likes it, they leave
+      // the matrix cores idle and take 256 registers (3001 x 28672 x 4096: 951
+      // us, 907 so; 3001 x 6144 x 4096: 242, 216)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) asm volatile("" : "+v"(acc[t][nt]));
     };
 #pragma unroll
     for (int j = 0; j < J; ++j) xa[0][j] = load(l15, j);
@@ -207,24 +214,25 @@ __device__ __forceinline__ void dq_tile_body(const DqArgs& A, char* smem,
           a[t & 1][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
               xa[t & 1][j], b[nt][j], a[t & 1][nt], 0, 0, 0);
       if (t > 0) fold(t - 1);
-      // kept apart, the stages fit 256 registers (W4: 774 against 731 TFLOP/s
-      // at 3001 x 28672 x 4096; W8 spills so: 672 against 687)
-      if constexpr (BITS == 4) __builtin_amdgcn_sched_barrier(0);
+      // row tiles kept apart (free, W8 loses 2 %)
+      __builtin_amdgcn_sched_barrier(0);
     }
     // this wave's share of the chunk's sums
-    f32x4 xs[MT / NW] = {};
+    constexpr int XS = (MT + NW - 1) / NW;
+    f32x4 xs[XS] = {};
 #pragma unroll
-    for (int i = 0; i < MT / NW; ++i)
+    for (int i = 0; i < XS; ++i)
+      if (MT % NW == 0 || i * NW + wave < MT)
 #pragma unroll
-      for (int j = 0; j < J; ++j)
-        xs[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            load((wave * (MT / NW) + i) * 16 + l15, j), ones, xs[i], 0, 0, 0);
+        for (int j = 0; j < J; ++j)
+          xs[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              load((i * NW + wave) * 16 + l15, j), ones, xs[i], 0, 0, 0);
     fold(MT - 1);
     if (l15 == 0) {
 #pragma unroll
-      for (int i = 0; i < MT / NW; ++i)
-        *(f32x4*)(xsum + par * BM + (wave * (MT / NW) + i) * 16 + l4 * 4) =
-            xs[i];
+      for (int i = 0; i < XS; ++i)
+        if (MT % NW == 0 || i * NW + wave < MT)
+          *(f32x4*)(xsum + par * BM + (i * NW + wave) * 16 + l4 * 4) = xs[i];
     }
 #pragma unroll
     for (int t = 0; t < NT; ++t) szp[t] = sz[t];
@@ -294,9 +302,11 @@ __device__ __forceinline__ void dq_tile_body(const DqArgs& A, char* smem,
   }
 }
 
-// SMALL: tiles of up to 64 rows may occur (experts) or are all (dense)
-template <int BITS, int KC, DqMode MODE, bool SMALL>
-__global__ __launch_bounds__(TPB, 2) void dq_tile_kernel(DqArgs A, int mb) {
+// step: rows from tile to tile (DENSE).  A tile takes the smallest body of 64,
+// 96 or 128 rows that holds it; LARGE: there is none below 97.
+template <int BITS, int KC, DqMode MODE, bool LARGE>
+__global__ __launch_bounds__(TPB, 2) void dq_tile_kernel(DqArgs A, int mb,
+                                                         int step) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   // an XCD's workgroups share columns: row tiles run fastest
   const u32 nb = MODE == GLU ? (A.n / 2 + 63) / 64 : (A.n + 127) / 128;
@@ -304,21 +314,23 @@ __global__ __launch_bounds__(TPB, 2) void dq_tile_kernel(DqArgs A, int mb) {
   const int mt = (int)(id % mb);
   id /= mb;
   const int nblk = (int)(id % nb), sp = (int)(id / nb);
-  int row0 = mt * ROWS, rows = min(A.m - row0, ROWS), expert = 0;
+  int row0 = mt * step, rows = min(A.m - row0, step), expert = 0;
   if constexpr (MODE != DENSE) {
     expert = A.tiles[3 * mt];
     if (expert < 0) return;
     row0 = A.tiles[3 * mt + 1];
     rows = A.tiles[3 * mt + 2];
   }
-  if (SMALL && (MODE == DENSE || rows <= 64))
+  if (!LARGE && rows <= 64)
     dq_tile_body<BITS, KC, MODE, 4>(A, smem, row0, rows, expert, nblk, sp);
+  else if (!LARGE && rows <= 96)
+    dq_tile_body<BITS, KC, MODE, 6>(A, smem, row0, rows, expert, nblk, sp);
   else
     dq_tile_body<BITS, KC, MODE, 8>(A, smem, row0, rows, expert, nblk, sp);
 }
 
-template <int BITS, int KC, DqMode MODE, bool SMALL>
-hipError_t go(const DqArgs& A, int mb, hipStream_t stream) {
+template <int BITS, int KC, DqMode MODE, bool LARGE>
+hipError_t go(const DqArgs& A, int mb, int step, hipStream_t stream) {
   // two buffers and the sums; the result, padded, takes a little more
   constexpr size_t bufs = 2 * ROWS * KC * 2 + 2 * ROWS * 4;
   constexpr size_t out = ROWS * 136 * 2;
@@ -326,25 +338,27 @@ hipError_t go(const DqArgs& A, int mb, hipStream_t stream) {
   static bool set = false;
   if (!set && lds > 64 * 1024) {
     LFMQ_CHECK_HIP(hipFuncSetAttribute(
-        (const void*)dq_tile_kernel<BITS, KC, MODE, SMALL>,
+        (const void*)dq_tile_kernel<BITS, KC, MODE, LARGE>,
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     set = true;
   }
   const u32 nb = MODE == GLU ? ceil_div_u32(A.n / 2, 64)
                              : ceil_div_u32(A.n, 128);
-  hipLaunchKernelGGL((dq_tile_kernel<BITS, KC, MODE, SMALL>),
-                     dim3(mb * nb * A.splits), dim3(TPB), lds, stream, A, mb);
+  hipLaunchKernelGGL((dq_tile_kernel<BITS, KC, MODE, LARGE>),
+                     dim3(mb * nb * A.splits), dim3(TPB), lds, stream, A, mb,
+                     step);
   return hipGetLastError();
 }
 
-template <DqMode MODE, bool SMALL>
-hipError_t go_bits(const DqArgs& A, int bits, int mb, hipStream_t stream) {
+template <DqMode MODE, bool LARGE>
+hipError_t go_bits(const DqArgs& A, int bits, int mb, int step,
+                   hipStream_t stream) {
   if (bits == 4)
-    return A.g % 128 == 0 ? go<4, 128, MODE, SMALL>(A, mb, stream)
-                          : go<4, 64, MODE, SMALL>(A, mb, stream);
+    return A.g % 128 == 0 ? go<4, 128, MODE, LARGE>(A, mb, step, stream)
+                          : go<4, 64, MODE, LARGE>(A, mb, step, stream);
   if (bits == 8)
-    return A.g % 128 == 0 ? go<8, 128, MODE, SMALL>(A, mb, stream)
-                          : go<8, 64, MODE, SMALL>(A, mb, stream);
+    return A.g % 128 == 0 ? go<8, 128, MODE, LARGE>(A, mb, step, stream)
+                          : go<8, 64, MODE, LARGE>(A, mb, step, stream);
   return hipErrorInvalidValue;
 }
 
@@ -380,9 +394,12 @@ hipError_t lfmq_dq_tile(const void* qweight, const void* scales,
                  (const u32*)qzeros, (const unsigned short*)x,
                  (unsigned short*)y, (const unsigned short*)bias, nullptr,
                  (float*)part, m, n, k, g, splits, nullptr, nullptr, nullptr};
-  const hipError_t e =
-      m <= 64 ? go_bits<DENSE, true>(A, bits, 1, stream)
-              : go_bits<DENSE, false>(A, bits, ceil_div_u32(m, ROWS), stream);
+  // row tiles alike, in sixteens: 129 rows are two of 80
+  const int mb = (int)ceil_div_u32(m, ROWS);
+  const int step = (int)ceil_div_u32(ceil_div_u32(m, mb), 16) * 16;
+  const hipError_t e = step <= 96
+                           ? go_bits<DENSE, false>(A, bits, mb, step, stream)
+                           : go_bits<DENSE, true>(A, bits, mb, step, stream);
   if (e != hipSuccess || splits == 1) return e;
   return lfmq_dq_rows_sum(part, y, bias, resid, m, n, splits, stream);
 }
@@ -409,6 +426,6 @@ hipError_t lfmq_dq_tile_experts(const void* qweight, const void* scales,
   A.k = k;
   A.g = g;
   A.splits = 1;
-  return glu ? go_bits<GLU, true>(A, bits, n_tiles, stream)
-             : go_bits<SLOTS, true>(A, bits, n_tiles, stream);
+  return glu ? go_bits<GLU, false>(A, bits, n_tiles, 0, stream)
+             : go_bits<SLOTS, false>(A, bits, n_tiles, 0, stream);
 }

@@ -152,9 +152,12 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
   const bool large = !rms && k >= 4096 && (long)n * k >= 24l << 20 &&
                      (rptr == nullptr ||
                       lfmq_dq_tile_splits(m, n, k, (int)g) > 1);
+  // a product that a few workgroups do whole: n 2048, k 2048 11.2 / 14.7 at 77
+  // rows, 15.1 / 17.0 at 120, but 21 / 16.6 at 129; n 3072 15.6 / 16.0
+  const bool small = !rms && rptr == nullptr && (long)n * k <= 4l << 20;
   const bool by_rows = (cols_hint == 0 ? m >= (bits == 8 || n >= 16384 ? 2 : 3)
                                        : cols_hint == 6 && m > 4) &&
-                       m <= (large ? 32 : 48) &&
+                       m <= (large ? 32 : small ? 96 : 48) &&
                        lfmq_dq_rows_ok(m, n, k, (int)g, rms);
   if (m > 16) {
     TORCH_CHECK((by_rows || !rms) && (m <= 48 || rptr == nullptr),

@@ -556,6 +556,25 @@ def test_dq_linear_rows_and_tiles(bits, m, n, k, g):
     assert float((err / (want.abs() + 1e-3 * want.abs().max())).max()) < 5e-3
 
 
+@pytest.mark.parametrize("m", [64, 65, 96, 97, 129, 160, 193, 300])
+@pytest.mark.parametrize("bits,n,k,g", [(4, 2100, 2048, 128), (8, 130, 192, 64)])
+def test_dq_tile_bodies(bits, m, n, k, g):
+    """Row tiles of 64, 96 and 128, one to three of them, whole and split k;
+    products whose result is off by its own rounding."""
+    torch.manual_seed(m)
+    codes = torch.randint(0, 1 << bits, (n, k), dtype=torch.int32)
+    zeros = torch.randint(0, 1 << bits, (n, k // g), dtype=torch.int32)
+    s16 = (torch.rand(n, k // g) * 0.02 + 0.01).to(torch.bfloat16)
+    w = ref.dequant_groupwise(codes, s16.float(), zeros, g).double().to(DEV)
+    x = torch.randn(m, k).to(torch.bfloat16).to(DEV)
+    y = ext().dq_linear(x, ref.pack_codes(codes, bits).to(DEV), s16.to(DEV),
+                        ref.pack_zeros(zeros, bits).to(DEV), bits, g, None,
+                        None, -1.0, 0)
+    want = x.double() @ w.t()
+    err = (y.double() - want).abs()
+    assert float((err / (want.abs() + 1e-3 * want.abs().max())).max()) < 5e-3
+
+
 @pytest.mark.parametrize("bits,m,n,k,g", [
     (4, 3, 48, 256, 128), (8, 2, 17, 192, 64), (4, 16, 6208, 256, 64),
     (4, 5, 72, 96, 32), (4, 2, 16400, 128, 128), (8, 16, 3072, 2048, 128),
