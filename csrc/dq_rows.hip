@@ -265,19 +265,33 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(DqArgs A) {
   }
 }
 
-// y = sum of the splits' parts (+ bias) (+ residual)
+// y = sum of the splits' parts (+ bias) (+ residual); GLU: silu(gate) * up of
+// the sums, y half as wide
+template <bool GLU>
 __global__ __launch_bounds__(256) void dq_rows_sum(DqArgs A) {
-  const u64 total = (u64)A.m * A.n;
-  if (A.n % 4 == 0) {
-    for (u64 id = ((u64)blockIdx.x * 256 + threadIdx.x) * 4; id < total;
-         id += (u64)gridDim.x * 1024) {
-      f32x4 v = *(const f32x4*)(A.part + id);
+  const u64 part = (u64)A.m * A.n;
+  const int nout = GLU ? A.n / 2 : A.n;
+  const u64 total = (u64)A.m * nout;
+  if (nout % 4 == 0) {
+    auto sum = [&](u64 at) {
+      f32x4 v = *(const f32x4*)(A.part + at);
 #pragma unroll 4
       for (int s = 1; s < A.splits; ++s)
-        v += *(const f32x4*)(A.part + s * total + id);
-      const int row = id / A.n, col = id % A.n;
+        v += *(const f32x4*)(A.part + s * part + at);
+      return v;
+    };
+    for (u64 id = ((u64)blockIdx.x * 256 + threadIdx.x) * 4; id < total;
+         id += (u64)gridDim.x * 1024) {
+      const int row = id / nout, col = id % nout;
+      f32x4 v = sum((u64)row * A.n + col);
+      if constexpr (GLU) {
+        const f32x4 up = sum((u64)row * A.n + nout + col);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = epilogue(A, v[e], row, col + e);
+        for (int e = 0; e < 4; ++e) v[e] = silu_mul_f(v[e], up[e]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = epilogue(A, v[e], row, col + e);
+      }
       *(u64*)(A.y + id) =
           pack_bf16x2(v[0], v[1]) | (u64)pack_bf16x2(v[2], v[3]) << 32;
     }
@@ -285,18 +299,25 @@ __global__ __launch_bounds__(256) void dq_rows_sum(DqArgs A) {
   }
   for (u64 id = (u64)blockIdx.x * 256 + threadIdx.x; id < total;
        id += (u64)gridDim.x * 256) {
-    float v = 0.f;
-    for (int s = 0; s < A.splits; ++s) v += A.part[s * total + id];
+    const int row = id / nout, col = id % nout;
+    float v = 0.f, up = 0.f;
+    for (int s = 0; s < A.splits; ++s) {
+      v += A.part[s * part + (u64)row * A.n + col];
+      if (GLU) up += A.part[s * part + (u64)row * A.n + nout + col];
+    }
     A.y[id] = (unsigned short)f32_to_bf16_bits_rne(
-        epilogue(A, v, id / A.n, id % A.n));
+        GLU ? silu_mul_f(v, up) : epilogue(A, v, row, col));
   }
 }
 
-void sum_parts(const DqArgs& A, hipStream_t stream) {
-  const u64 items = (u64)A.m * A.n / (A.n % 4 == 0 ? 4 : 1);
-  hipLaunchKernelGGL(dq_rows_sum,
-                     dim3((u32)min((items + 255) / 256, (u64)1024)),
-                     dim3(256), 0, stream, A);
+void sum_parts(const DqArgs& A, bool glu, hipStream_t stream) {
+  const int nout = glu ? A.n / 2 : A.n;
+  const u64 items = (u64)A.m * nout / (nout % 4 == 0 ? 4 : 1);
+  const dim3 grid((u32)min((items + 255) / 256, (u64)1024));
+  if (glu)
+    hipLaunchKernelGGL(dq_rows_sum<true>, grid, dim3(256), 0, stream, A);
+  else
+    hipLaunchKernelGGL(dq_rows_sum<false>, grid, dim3(256), 0, stream, A);
 }
 
 int chunk_of(int g) { return g % 128 == 0 ? 128 : (g % 64 == 0 ? 64 : 32); }
@@ -326,7 +347,7 @@ hipError_t go(const DqArgs& A, int tiles, hipStream_t stream) {
                   tiles);
   hipLaunchKernelGGL((dq_rows_kernel<BITS, MT, NT, NW, KC, MODE>), grid, dim3(NW * 64),
                      lds, stream, A);
-  if (A.splits > 1) sum_parts(A, stream);
+  if (A.splits > 1) sum_parts(A, false, stream);
   return hipGetLastError();
 }
 
@@ -451,10 +472,10 @@ hipError_t lfmq_dq_rows(const void* qweight, const void* scales,
   return go_tile<8, 32>(A, glu, stream);
 }
 
-// y = sum of part [splits, m, n] (+ bias) (+ residual)
+// y = sum of part [splits, m, n] (+ bias) (+ residual), or the gate of it
 hipError_t lfmq_dq_rows_sum(const void* part, void* y, const void* bias,
                             const void* resid, int m, int n, int splits,
-                            hipStream_t stream) {
+                            bool glu, hipStream_t stream) {
   DqArgs A{};
   A.part = (float*)part;
   A.y = (unsigned short*)y;
@@ -463,7 +484,7 @@ hipError_t lfmq_dq_rows_sum(const void* part, void* y, const void* bias,
   A.m = m;
   A.n = n;
   A.splits = splits;
-  sum_parts(A, stream);
+  sum_parts(A, glu, stream);
   return hipGetLastError();
 }
 

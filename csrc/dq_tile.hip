@@ -302,7 +302,7 @@ __device__ __forceinline__ void dq_tile_body(const DqArgs& A, char* smem,
   }
 }
 
-// step: rows from tile to tile (DENSE).  A tile takes the smallest body of 64,
+// step: rows from tile to tile (without a list of them).  A tile takes the smallest body of 64,
 // 96 or 128 rows that holds it; LARGE: there is none below 97.
 template <int BITS, int KC, DqMode MODE, bool LARGE>
 __global__ __launch_bounds__(TPB, 2) void dq_tile_kernel(DqArgs A, int mb,
@@ -315,7 +315,7 @@ __global__ __launch_bounds__(TPB, 2) void dq_tile_kernel(DqArgs A, int mb,
   id /= mb;
   const int nblk = (int)(id % nb), sp = (int)(id / nb);
   int row0 = mt * step, rows = min(A.m - row0, step), expert = 0;
-  if constexpr (MODE != DENSE) {
+  if (MODE != DENSE && A.tiles != nullptr) {
     expert = A.tiles[3 * mt];
     if (expert < 0) return;
     row0 = A.tiles[3 * mt + 1];
@@ -380,14 +380,19 @@ int lfmq_dq_tile_splits(int m, int n, int k, int g) {
 
 hipError_t lfmq_dq_rows_sum(const void* part, void* y, const void* bias,
                             const void* resid, int m, int n, int splits,
-                            hipStream_t stream);
+                            bool glu, hipStream_t stream);
 
+// glu: y [m, n / 2] = silu(gate) up of W = [gate | up], without bias and
+// residual
 hipError_t lfmq_dq_tile(const void* qweight, const void* scales,
                         const void* qzeros, const void* x, void* y,
                         const void* bias, const void* resid, void* part,
                         int m, int n, int k, int g, int bits, int splits,
-                        hipStream_t stream) {
+                        bool glu, hipStream_t stream) {
   if (resid != nullptr && splits == 1) return hipErrorInvalidValue;
+  if (glu && (n % 2 || bias != nullptr || resid != nullptr ||
+              (u64)m * k * 2 >= 1ull << 32))
+    return hipErrorInvalidValue;
   if (!lfmq_dq_tile_ok(k, g) || (u64)n * k * bits / 8 >= 1ull << 32)
     return hipErrorInvalidValue;
   const DqArgs A{(const char*)qweight, (const unsigned short*)scales,
@@ -397,11 +402,15 @@ hipError_t lfmq_dq_tile(const void* qweight, const void* scales,
   // row tiles alike, in sixteens: 129 rows are two of 80
   const int mb = (int)ceil_div_u32(m, ROWS);
   const int step = (int)ceil_div_u32(ceil_div_u32(m, mb), 16) * 16;
-  const hipError_t e = step <= 96
-                           ? go_bits<DENSE, false>(A, bits, mb, step, stream)
-                           : go_bits<DENSE, true>(A, bits, mb, step, stream);
+  hipError_t e;
+  if (glu && splits == 1)
+    e = step <= 96 ? go_bits<GLU, false>(A, bits, mb, step, stream)
+                   : go_bits<GLU, true>(A, bits, mb, step, stream);
+  else
+    e = step <= 96 ? go_bits<DENSE, false>(A, bits, mb, step, stream)
+                   : go_bits<DENSE, true>(A, bits, mb, step, stream);
   if (e != hipSuccess || splits == 1) return e;
-  return lfmq_dq_rows_sum(part, y, bias, resid, m, n, splits, stream);
+  return lfmq_dq_rows_sum(part, y, bias, resid, m, n, splits, glu, stream);
 }
 
 // rows of x (or slots) by expert, tiles of up to 128 of them (DqArgs); glu:

@@ -20,7 +20,7 @@ bool lfmq_dq_tile_ok(int, int);
 int lfmq_dq_tile_splits(int, int, int, int);
 hipError_t lfmq_dq_tile(const void*, const void*, const void*, const void*,
                         void*, const void*, const void*, void*, int, int, int,
-                        int, int, int, hipStream_t);
+                        int, int, int, bool, hipStream_t);
 hipError_t lfmq_rmsnorm(const void*, const void*, const void*, void*, void*,
                         int, int, float, hipStream_t);
 hipError_t lfmq_rope(void*, void*, const void*, const void*, int, int, int,
@@ -189,7 +189,7 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
     CHECK_HIP(lfmq_dq_tile(qweight.data_ptr(), scales.data_ptr(),
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                            rptr, parts(splits), m, n, k, (int)g, (int)bits,
-                           splits, stream()));
+                           splits, false, stream()));
   }
   return y;
 }
@@ -350,10 +350,26 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
   auto y = torch::empty({m, n / 2}, x.options());
   // as dq_linear.  us with the norm, GEMV / rows, n 28672, k 4096, 4 bits:
   // 37.5 / 24.0 at 4 rows; norm, product and gate apart / rows: 32.5 / 26.4 at
-  // 8, 44.0 / 37.6 at 32, 46.5 / 49.6 at 48 (n 16384, k 2048: 21.4 / 15.6)
+  // 8, 44.0 / 37.6 at 32 (n 16384, k 2048 at 48: 21.4 / 15.6)
+  const bool large = rms_eps < 0 && k >= 4096 && (long)n * k >= 24l << 20;
+  if (cols_hint == 0 && n % 2 == 0 && m > (large ? 32 : 48) &&
+      lfmq_dq_tile_ok(k, (int)g)) {
+    TORCH_CHECK(rms_eps < 0, "fused rms is a decode (m <= 48) path");
+    if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
+    const int splits = lfmq_dq_tile_splits(m, n, k, (int)g);
+    torch::Tensor part;
+    if (splits > 1)
+      part = torch::empty({(long)splits * m * n},
+                          x.options().dtype(torch::kFloat32));
+    CHECK_HIP(lfmq_dq_tile(qweight.data_ptr(), scales.data_ptr(),
+                           qzeros.data_ptr(), x.data_ptr(), y.data_ptr(),
+                           nullptr, nullptr,
+                           splits > 1 ? part.data_ptr() : nullptr, m, n, k,
+                           (int)g, (int)bits, splits, true, stream()));
+    return y;
+  }
   if (cols_hint == 0 && m >= (bits == 8 || n >= 16384 ? 2 : 3) && m <= 48 &&
-      n % 2 == 0 &&
-      lfmq_dq_rows_ok(m, n, k, (int)g, true)) {
+      n % 2 == 0 && lfmq_dq_rows_ok(m, n, k, (int)g, true)) {
     if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
     CHECK_HIP(lfmq_dq_rows(qweight.data_ptr(), scales.data_ptr(),
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(),

@@ -187,7 +187,7 @@ class LlamaMLP(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         gp = self.gate_up_proj
         m = x.numel() // x.shape[-1]
-        if (x.is_cuda and m <= FEW_ROWS and isinstance(gp, QLinear)
+        if (x.is_cuda and isinstance(gp, QLinear)
                 and type(gp).forward is QLinear.forward
                 and not hasattr(gp, "perm")
                 and (m <= 4 or (gp.bias is None and rows_fused(gp)))):
@@ -252,11 +252,15 @@ class LlamaDecoderLayer(nn.Module):
         o = self.self_attn.decode_qkv_attn(x, cache_k, cache_v, state,
                                            max_seq, rms_eps=eps)
         x = self.self_attn.o_proj.forward_resid(o, x)
-        mlp = self.mlp
-        h = F.dq_gemv_gateup(x, mlp.gate_up_proj.qweight,
-                             mlp.gate_up_proj.scales, mlp.gate_up_proj.qzeros,
-                             mlp.gate_up_proj.bits, mlp.gate_up_proj.group_size,
-                             rms_eps=self.post_attention_layernorm.eps)
+        mlp, gp = self.mlp, self.mlp.gate_up_proj
+        h, eps = x, self.post_attention_layernorm.eps
+        if x.shape[0] > 32 and gp.in_features >= 4096 and \
+                gp.in_features * gp.out_features >= 24 << 20:
+            # the product for prompts, which takes normed rows, is faster
+            # (28672 x 4096 at 48 rows: 41 us with its norm, 50)
+            h, eps = self.post_attention_layernorm(x), -1.0
+        h = F.dq_gemv_gateup(h, gp.qweight, gp.scales, gp.qzeros, gp.bits,
+                             gp.group_size, rms_eps=eps)
         x = mlp.down_proj.forward_resid(h, x)
         return x
 

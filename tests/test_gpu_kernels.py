@@ -576,6 +576,30 @@ def test_dq_tile_bodies(bits, m, n, k, g):
 
 
 @pytest.mark.parametrize("bits,m,n,k,g", [
+    (4, 49, 260, 256, 128), (8, 97, 2 * 67, 128, 64), (4, 130, 1026, 2048, 64),
+    (8, 300, 4096, 256, 128), (4, 3000, 2 * 1030, 128, 128),
+    (4, 40, 6144, 4096, 128), (8, 77, 2 * 5, 192, 64)])
+def test_dq_tile_gate(bits, m, n, k, g):
+    """silu(gate) * up behind the product of a prompt: in its epilogue, and
+    behind the sum of a split k; gates that end inside a tile."""
+    torch.manual_seed(m)
+    codes = torch.randint(0, 1 << bits, (n, k), dtype=torch.int32)
+    zeros = torch.randint(0, 1 << bits, (n, k // g), dtype=torch.int32)
+    s16 = (torch.rand(n, k // g) * 0.02 + 0.01).to(torch.bfloat16)
+    w = ref.dequant_groupwise(codes, s16.float(), zeros, g).double().to(DEV)
+    x = torch.randn(m, k).to(torch.bfloat16).to(DEV)
+    y = ext().dq_gemv_gateup(x, ref.pack_codes(codes, bits).to(DEV),
+                             s16.to(DEV), ref.pack_zeros(zeros, bits).to(DEV),
+                             bits, g, -1.0, 0)
+    a, u = (x.double() @ w.t()).chunk(2, 1)
+    want = torch.nn.functional.silu(a) * u
+    err = (y.double() - want).abs()
+    floor = 1e-3 * want.abs().amax(1, keepdim=True)
+    assert y.shape == (m, n // 2)
+    assert float((err / (want.abs() + floor)).max()) < 5e-3
+
+
+@pytest.mark.parametrize("bits,m,n,k,g", [
     (4, 3, 48, 256, 128), (8, 2, 17, 192, 64), (4, 16, 6208, 256, 64),
     (4, 5, 72, 96, 32), (4, 2, 16400, 128, 128), (8, 16, 3072, 2048, 128),
     (4, 17, 100, 384, 128), (8, 32, 6144, 256, 128), (4, 31, 16384, 128, 64),
