@@ -46,7 +46,7 @@ hipError_t lfmq_hessian_accum(const void*, void*, int, int, hipStream_t);
 int lfmq_chol_pad(int n);
 hipError_t lfmq_chol_inverse(const void*, void*, void*, void*, void*, void*,
                              int, hipStream_t);
-hipError_t lfmq_gptq_block(const void*, const void*, void*, void*, void*,
+hipError_t lfmq_gptq_block(const void*, const void*, int, void*, void*, void*,
                            void*, int, int, int, int, int, int, int, bool,
                            hipStream_t);
 hipError_t lfmq_dq_gemv_gateup(const void*, const void*, const void*,
@@ -702,7 +702,10 @@ torch::Tensor gptq_block(torch::Tensor w, torch::Tensor ub,
                          torch::Tensor zeros, long i1, long g, long bits,
                          bool sym) {
   check_t(w, torch::kFloat32, "w");
-  check_t(ub, torch::kFloat32, "ub");
+  TORCH_CHECK(ub.is_cuda() && ub.scalar_type() == torch::kFloat32 &&
+                  ub.dim() == 2 && ub.stride(1) == 1 &&
+                  ub.stride(0) >= ub.size(1) && ub.stride(0) <= INT32_MAX,
+              "ub must be rows of fp32 on GPU");
   check_t(codes, torch::kInt32, "codes");
   check_t(scales, torch::kFloat32, "scales");
   check_t(zeros, torch::kInt32, "zeros");
@@ -714,7 +717,8 @@ torch::Tensor gptq_block(torch::Tensor w, torch::Tensor ub,
                   zeros.numel() == n * (k / g),
               "scales and zeros must be [n, k / g]");
   auto err = torch::empty({n, nb}, w.options());
-  CHECK_HIP(lfmq_gptq_block(w.data_ptr(), ub.data_ptr(), codes.data_ptr(),
+  CHECK_HIP(lfmq_gptq_block(w.data_ptr(), ub.data_ptr(),
+                            (int)ub.stride(0), codes.data_ptr(),
                             scales.data_ptr(), zeros.data_ptr(),
                             err.data_ptr(), (int)n, (int)k, (int)(k / g),
                             (int)i1, (int)nb, (int)g, (int)bits, sym,

@@ -87,7 +87,9 @@ GPU_BLOCK = 128        # widest block of the HIP kernel: its U fits in LDS
 def _gpu_block(w, ub, codes, scales, zeros, i1, cfg, g) -> torch.Tensor:
     """_block in one launch (csrc/gptq_block.hip), the same bit by bit."""
     from ..ops import hip_ext
-    return hip_ext().gptq_block(w, ub.contiguous(), codes, scales, zeros, i1,
+    if ub.stride(1) != 1:
+        ub = ub.contiguous()
+    return hip_ext().gptq_block(w, ub, codes, scales, zeros, i1,
                                 g, cfg.bits, cfg.sym)
 
 
@@ -135,7 +137,8 @@ def gptq_quantize_layer(
         i2 = min(i1 + cfg.block_size, k)
         err = block(w, U[i1:i2, i1:i2], codes, scales, zeros, i1, cfg, g)
         if i2 < k:
-            w[:, i2:] -= err @ U[i1:i2, i2:]
+            # in one pass over w, of the products' sums in fp32
+            w[:, i2:].addmm_(err, U[i1:i2, i2:], alpha=-1)
 
     aperm = None
     if perm is not None:
