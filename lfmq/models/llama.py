@@ -23,7 +23,8 @@ import torch.nn as nn
 
 from ..ops import functional as F
 from .kvcache import KVCache
-from .qlinear import FEW_ROWS, QLinear, hooked, rows_fused
+from .linear import Linear, hooked
+from .qlinear import FEW_ROWS, QLinear, rows_fused
 
 
 @dataclass
@@ -274,7 +275,7 @@ class LlamaForCausalLM(nn.Module):
         self.layers = nn.ModuleList(LlamaDecoderLayer(cfg, dtype)
                                     for _ in range(cfg.n_layers))
         self.norm = RMSNorm(cfg.hidden_size, cfg.rms_eps, dtype)
-        self.lm_head = nn.Linear(cfg.hidden_size, cfg.vocab_size, bias=False, dtype=dtype)
+        self.lm_head = Linear(cfg.hidden_size, cfg.vocab_size, dtype)
         if cfg.tie_embeddings:
             self.lm_head.weight = self.embed_tokens.weight
 
@@ -302,6 +303,8 @@ class LlamaForCausalLM(nn.Module):
         pos0 = cache.seq_len
         if positions is None:
             positions = torch.arange(pos0, pos0 + s, device=input_ids.device)
+        if positions.is_cuda:
+            positions = positions.to(torch.int32)    # once, not in every layer
         seq_after = pos0 + s
         x = self.embed_tokens(input_ids)
         residual = None

@@ -29,24 +29,11 @@ import torch
 import torch.nn as nn
 
 from ..ops import functional as F
-from .qlinear import hooked
+from .linear import Linear, hooked
 
 
 def _fp32(n: int, value: float = 0.0) -> nn.Parameter:
     return nn.Parameter(torch.full((n,), value, dtype=torch.float32))
-
-
-class Linear(nn.Linear):
-    """nn.Linear without a bias whose decode steps run on the kernel for a
-    few rows."""
-
-    def __init__(self, n_in: int, n_out: int, dtype):
-        super().__init__(n_in, n_out, bias=False, dtype=dtype)
-
-    def forward(self, x):
-        if self.bias is not None:
-            return super().forward(x)
-        return F.linear(x, self.weight)
 
 
 class ResidualNorm(nn.Module):

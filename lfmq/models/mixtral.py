@@ -22,6 +22,7 @@ import torch.nn as nn
 
 from ..ops import functional as F
 from .kvcache import KVCache
+from .linear import Linear
 from .llama import LlamaAttention, LlamaConfig, RMSNorm
 from .qlinear import QLinear
 
@@ -89,8 +90,7 @@ class MixtralMoE(nn.Module):
         self.cfg = cfg
         self.n_experts = cfg.n_experts
         self.top_k = cfg.top_k
-        self.gate = nn.Linear(cfg.hidden_size, cfg.n_experts, bias=False,
-                              dtype=dtype)  # router stays dense bf16
+        self.gate = Linear(cfg.hidden_size, cfg.n_experts, dtype)  # router stays dense bf16
         self.experts = nn.ModuleList(MixtralExpert(cfg, dtype)
                                      for _ in range(cfg.n_experts))
         self._grouped = None  # set by consolidate()
@@ -241,8 +241,7 @@ class MixtralForCausalLM(nn.Module):
         self.layers = nn.ModuleList(MixtralDecoderLayer(cfg, dtype)
                                     for _ in range(cfg.n_layers))
         self.norm = RMSNorm(cfg.hidden_size, cfg.rms_eps, dtype)
-        self.lm_head = nn.Linear(cfg.hidden_size, cfg.vocab_size, bias=False,
-                                 dtype=dtype)
+        self.lm_head = Linear(cfg.hidden_size, cfg.vocab_size, dtype)
 
     @torch.no_grad()
     def init_random(self, seed: int = 0):
@@ -270,6 +269,8 @@ class MixtralForCausalLM(nn.Module):
         pos0 = cache.seq_len
         if positions is None:
             positions = torch.arange(pos0, pos0 + s, device=input_ids.device)
+        if positions.is_cuda:
+            positions = positions.to(torch.int32)    # once, not in every layer
         x = self.embed_tokens(input_ids)
         residual = None
         for i, layer in enumerate(self.layers):

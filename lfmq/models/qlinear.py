@@ -16,6 +16,7 @@ from .. import dist as lfmq_dist
 from ..config import QuantConfig
 from ..ops import functional as F
 from ..ops import ref
+from .linear import hooked
 
 
 class QLinear(nn.Module):
@@ -130,14 +131,6 @@ class QLinear(nn.Module):
 
 
 FEW_ROWS = 48        # rows of the kernel that has norm and gate epilogues
-
-
-def hooked(*modules) -> bool:
-    """Whether anyone watches calls of these modules."""
-    m = nn.modules.module
-    return bool(m._global_forward_hooks or m._global_forward_pre_hooks
-                or any(p._forward_hooks or p._forward_pre_hooks
-                       for p in modules))
 
 
 def rows_fused(p: nn.Module) -> bool:

@@ -16,8 +16,9 @@ import torch
 import torch.nn as nn
 
 from ..ops import functional as F
-from .mixers import (DenseMLP, LatentAttention, Linear, MixerBlock,
-                     MLSTMMixer, ResidualNorm)
+from .linear import Linear
+from .mixers import (DenseMLP, LatentAttention, MixerBlock, MLSTMMixer,
+                     ResidualNorm)
 from .packed import PackedCausalLM
 from .seqcache import SequenceCache, StepBatch
 
