@@ -113,6 +113,16 @@ torch::Tensor unpack(torch::Tensor packed, long bits, long k) {
   return out;
 }
 
+// rows from which the rows kernel is taken and not the GEMV, whose lanes hold
+// the scales of 128 groups at most.  us of both at 2 rows: 8 bits 12.5 / 13.3
+// (n 6144, k 4096), 22.9 / 20.5 (4096, 14336), 44.6 / 32.7 (28672, 4096); 4
+// bits 8.8 / 9.3, 17.0 / 15.1 and 27.3 / 22.0.  At 1 row the GEMV: 6.9 / 9.2,
+// 13.5 / 15.1, 18.1 / 22.5 (4 bits).
+int rows_from(long bits, long n, long k, long g) {
+  if (k > 128 * g) return 1;
+  return bits == 8 || n * k >= 32l << 20 ? 2 : 3;
+}
+
 torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
                         torch::Tensor scales, torch::Tensor qzeros, long bits,
                         long g, c10::optional<torch::Tensor> bias,
@@ -155,7 +165,7 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
   // a product that a few workgroups do whole: n 2048, k 2048 11.2 / 14.7 at 77
   // rows, 15.1 / 17.0 at 120, but 21 / 16.6 at 129; n 3072 15.6 / 16.0
   const bool small = !rms && rptr == nullptr && (long)n * k <= 4l << 20;
-  const bool by_rows = (cols_hint == 0 ? m >= (bits == 8 || n >= 16384 ? 2 : 3)
+  const bool by_rows = (cols_hint == 0 ? m >= rows_from(bits, n, k, g)
                                        : cols_hint == 6 && m > 4) &&
                        m <= (large ? 32 : small ? 96 : 48) &&
                        lfmq_dq_rows_ok(m, n, k, (int)g, rms);
@@ -368,7 +378,7 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
                            (int)g, (int)bits, splits, true, stream()));
     return y;
   }
-  if (cols_hint == 0 && m >= (bits == 8 || n >= 16384 ? 2 : 3) && m <= 48 &&
+  if (cols_hint == 0 && m >= rows_from(bits, n, k, g) && m <= 48 &&
       n % 2 == 0 && lfmq_dq_rows_ok(m, n, k, (int)g, true)) {
     if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
     CHECK_HIP(lfmq_dq_rows(qweight.data_ptr(), scales.data_ptr(),

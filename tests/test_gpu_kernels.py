@@ -645,6 +645,27 @@ def test_dq_rows_norm_gate_residual(bits, m, n, k, g):
                   torch.nn.functional.silu(a) * u)
 
 
+@pytest.mark.parametrize("m", [1, 2, 4])
+def test_dq_linear_of_many_groups(m):
+    """More groups a row than the GEMV's lanes hold scales of."""
+    torch.manual_seed(m)
+    n, k, g = 64, 8320, 64
+    codes = torch.randint(0, 16, (n, k), dtype=torch.int32)
+    zeros = torch.randint(0, 16, (n, k // g), dtype=torch.int32)
+    s16 = (torch.rand(n, k // g) * 0.02 + 0.01).to(torch.bfloat16)
+    packed = (ref.pack_codes(codes, 4).to(DEV), s16.to(DEV),
+              ref.pack_zeros(zeros, 4).to(DEV), 4, g)
+    x = torch.randn(m, k).to(torch.bfloat16).to(DEV)
+    want = x.double() @ ref.dequant_groupwise(
+        codes, s16.float(), zeros, g).double().to(DEV).t()
+    a, u = want.chunk(2, 1)
+    for y, w in ((ext().dq_linear(x, *packed, None, None, -1.0, 0), want),
+                 (ext().dq_gemv_gateup(x, *packed, -1.0, 0),
+                  torch.nn.functional.silu(a) * u)):
+        err = (y.double() - w).abs()
+        assert float((err / (w.abs() + 1e-3 * w.abs().max())).max()) < 5e-3
+
+
 def test_dq_linear_refuses():
     """More than 16 rows: groups of 32 and fused epilogues, as ever."""
     x = torch.zeros(17, 96, dtype=torch.bfloat16, device=DEV)
