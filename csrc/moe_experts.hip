@@ -15,6 +15,7 @@
 // Three forms of the two products: 128-row tiles through LDS (prompts),
 // 16-row tiles whose waves split the inner dimension and stream the weights
 // past registers (few rows an expert: decoding), and any size, 16 or 32 bit.
+#include "lds_dma.h"
 #include "seq_common.h"
 
 namespace {
@@ -281,10 +282,14 @@ __global__ __launch_bounds__(NW * 64) void moe_rows16(GemmArgs A) {
   stf((bf16_t*)A.out + (u64)(row0 + i) * A.N + n0 + c, o);
 }
 
-// 128 rows x 128 weight rows (GLU: 64 gate and 64 up), 4 waves of 64 x 64,
-// K in steps of 64 through two LDS buffers; 16-byte blocks of a 128-byte LDS
-// row are XOR-swizzled by the row so that fragment reads spread over banks
-constexpr int BM = 128, BN = 128, BK = 64;
+// 128 rows x 128 weight rows (GLU: 64 gate and 64 up), 4 waves of 64 x 64, K
+// in steps of 64 through two LDS buffers.  Both operands go from memory
+// straight into LDS, 16-byte blocks of a 128-byte row XOR-swizzled by the row
+// so that fragment reads spread over banks.  us of routing and both products,
+// 16 experts of 2048 x 2048, two a token, against staging through registers:
+// 2977 tokens 273 (310), 800 tokens 128 (135); 6000 tokens, 4096 x 3584: 1289
+// (1498).  Consecutive workgroups on one XCD: 293, 161, 1751.
+constexpr int BM = 128, BN = 128, BK = 64, BUF = (BM + BN) * BK * 2;
 
 template <bool GLU>
 __global__ __launch_bounds__(256, 2) void moe_rows128(GemmArgs A) {
@@ -293,66 +298,62 @@ __global__ __launch_bounds__(256, 2) void moe_rows128(GemmArgs A) {
   const int ex = tile[0];
   if (ex < 0) return;
   const int row0 = tile[1], rows = tile[2];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l15 = lane & 15, l4 = lane >> 4;
   const int wm = wave >> 1, wn = wave & 1;
   const int n0 = blockIdx.x * (GLU ? 64 : 128);
   const int wrows = GLU ? 2 * A.N : A.N;
-  const bf16_t* w = (const bf16_t*)A.w + (u64)ex * wrows * A.K;
-  // staging role: 16-byte column sc of rows sr + 32 i
-  const int sr = tid >> 3, sc = tid & 7;
-  const bf16_t *ap[4], *bp[4];
+  const char* w = (const char*)A.w + (u64)ex * wrows * A.K * 2;
+  // a wave's load fills 8 rows, a lane the block that belongs there; rows past
+  // the end repeat the last one, columns past K are cleared below
+  u32 ao[4], bo[4];
+  const int at = (lane & 7) ^ slot_key<8>(wave * 8 + (lane >> 3));
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int r = sr + 32 * i;
-    const int slot = row0 + min(r, rows - 1);
-    ap[i] = (const bf16_t*)A.a +
-            (u64)(A.src != nullptr ? A.src[slot] : slot) * A.K;
-    int n;
-    if constexpr (GLU)
-      n = (r < 64 ? 0 : A.N) + min(n0 + (r & 63), A.N - 1);
-    else
-      n = min(n0 + r, A.N - 1);
-    bp[i] = w + (u64)n * A.K;
+    const int r = (i * 4 + wave) * 8 + (lane >> 3);
+    int slot = row0 + min(r, rows - 1);
+    if (A.src != nullptr) slot = A.src[slot];
+    ao[i] = (u32)slot * (u32)(A.K * 2);
+    const int n = GLU ? (r < 64 ? 0 : A.N) + min(n0 + (r & 63), A.N - 1)
+                      : min(n0 + r, A.N - 1);
+    bo[i] = (u32)n * (u32)(A.K * 2);
   }
-  u32x4 xa[4], xb[4];
-  auto fetch = [&](int k0) {
-    const int k = k0 + sc * 8;
-    const u32x4 z = {0, 0, 0, 0};
+  auto stage = [&](int k0, int buf) {
+    // K in eights: a block is inside a row or past it
+    const u32 off = (k0 + at * 8 < A.K ? k0 + at * 8 : 0) * 2;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      xa[i] = k < A.K ? *(const u32x4*)(ap[i] + k) : z;
-      xb[i] = k < A.K ? *(const u32x4*)(bp[i] + k) : z;
-    }
-  };
-  auto stage = [&](char* buf) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = sr + 32 * i, o = r * 128 + ((sc ^ (r & 7)) << 4);
-      *(u32x4*)(buf + o) = xa[i];
-      *(u32x4*)(buf + BM * 128 + o) = xb[i];
+      load_to_lds(A.a, ao[i] + off, buf * BUF + (i * 4 + wave) * 1024);
+      load_to_lds(w, bo[i] + off, buf * BUF + BUF / 2 + (i * 4 + wave) * 1024);
     }
   };
   f32x4 acc[4][4] = {};
-  fetch(0);
-  stage(smem);
-  __syncthreads();
-  int cur = 0;
-  for (int k0 = 0; k0 < A.K; k0 += BK) {
-    const bool more = k0 + BK < A.K;
-    if (more) fetch(k0 + BK);
-    const char* la = smem + cur * (BM + BN) * 128;
-    const char* lb = la + BM * 128;
+  stage(0, 0);
+  for (int k0 = 0, cur = 0; k0 < A.K; k0 += BK, cur ^= 1) {
+    lds_loads_done();
+    char* la = smem + cur * BUF;
+    char* lb = la + BUF / 2;
+    if (k0 + BK < A.K) {
+      stage(k0 + BK, cur ^ 1);
+    } else if (k0 + BK > A.K) {
+      const u32x4 z = {0, 0, 0, 0};
+      for (int i = tid; i < (BM + BN) * 8; i += 256)
+        if (k0 + ((i & 7) ^ slot_key<8>(i >> 3 & 127)) * 8 >= A.K)
+          *(u32x4*)(la + i * 16) = z;
+      __syncthreads();
+    }
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       s16x8 af[4], bf[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int r = wm * 64 + i * 16 + l15;
-        af[i] = *(const s16x8*)(la + r * 128 + (((ks * 4 + l4) ^ (r & 7)) << 4));
         const int c = GLU ? (i >> 1) * 64 + wn * 32 + (i & 1) * 16 + l15
                           : wn * 64 + i * 16 + l15;
-        bf[i] = *(const s16x8*)(lb + c * 128 + (((ks * 4 + l4) ^ (c & 7)) << 4));
+        const int s = ((ks * 4 + l4) ^ slot_key<8>(l15)) << 4;
+        af[i] = *(const s16x8*)(la + r * 128 + s);
+        bf[i] = *(const s16x8*)(lb + c * 128 + s);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i)
@@ -361,9 +362,6 @@ __global__ __launch_bounds__(256, 2) void moe_rows128(GemmArgs A) {
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
               af[i], bf[j], acc[i][j], 0, 0, 0);
     }
-    cur ^= 1;
-    if (more) stage(smem + cur * (BM + BN) * 128);
-    __syncthreads();
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -447,7 +445,7 @@ hipError_t gemm(const GemmArgs& A, int max_tiles, int bm, bool f32,
                 hipStream_t stream) {
   if (max_tiles < 1 || max_tiles > 65535) return hipErrorInvalidValue;
   if (bm == 128 && !f32) {
-    const size_t lds = 2 * (BM + BN) * 128;
+    const size_t lds = 2 * BUF;
     const int per = GLU ? 64 : 128;
     hipLaunchKernelGGL(moe_rows128<GLU>,
                        dim3((A.N + per - 1) / per, max_tiles), dim3(256), lds,

@@ -760,7 +760,8 @@ T_ moe_glu(T_ h, T_ gu, T_ src, T_ weight, T_ tiles, double limit,
   check(tiles, torch::kInt32, "tiles");
   const long pairs = src.numel(), ff = gu.size(1) / 2, K = h.size(1);
   TORCH_CHECK(gu.dim() == 3 && gu.size(2) == K && gu.size(1) == 2 * ff &&
-                  (bm < 16 || (!f32 && K % 8 == 0 && al16(h) && al16(gu))),
+                  (bm < 16 || (!f32 && K % 8 == 0 && al16(h) && al16(gu))) &&
+                  (bm < 128 || (h.numel() < 1l << 31 && ff * K < 1l << 30)),
               "moe_glu: shape mismatch");
   auto out = torch::empty({pairs, ff}, h.options());
   CHECK_HIP(lfmq_moe_glu(h.data_ptr(), gu.data_ptr(), src.data_ptr(),
@@ -779,7 +780,8 @@ T_ moe_down(T_ act, T_ down, T_ tiles, long bm) {
   check(tiles, torch::kInt32, "tiles");
   const long K = act.size(1), N = down.size(1);
   TORCH_CHECK(down.dim() == 3 && down.size(2) == K &&
-                  (bm < 16 || (!f32 && K % 8 == 0 && al16(act) && al16(down))),
+                  (bm < 16 || (!f32 && K % 8 == 0 && al16(act) && al16(down))) &&
+                  (bm < 128 || (act.numel() < 1l << 31 && N * K < 1l << 31)),
               "moe_down: shape mismatch");
   auto out = torch::empty({act.size(0), N}, act.options());
   CHECK_HIP(lfmq_moe_down(act.data_ptr(), down.data_ptr(), tiles.data_ptr(),

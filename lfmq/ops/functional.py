@@ -469,8 +469,11 @@ def moe(h, router, gate_up, down, top: int, act, general: bool = False):
     the router has its row).  Stays on the device."""
     ext = seq_ext()
     E, ff2, width = gate_up.shape
+    # the tiled products address 4 GiB of rows and of an expert's weights
+    n = h.shape[0]
     aligned = not general and h.dtype == torch.bfloat16 and \
-        width % 8 == 0 and ff2 % 16 == 0
+        width % 8 == 0 and ff2 % 16 == 0 and \
+        max(n * width, n * top * ff2 // 2, ff2 * width) < 1 << 31
     bm = ext.moe_tile(h.shape[0] * top, E, aligned)
     src, weight, pos, tiles, sgate = ext.moe_route(h, router, E, top, bm)
     a = ext.moe_glu(h, gate_up, src, weight, tiles, *act, bm)
