@@ -12,16 +12,16 @@
 // of the rows' with products by ones, and all waves apply them a chunk later.
 //
 // Bound by latencies between the stages of two waves a SIMD (matrix cores
-// busy 41 % of the time, vector units 46 %, LDS half): 777 TFLOP/s at 3001 x
+// busy 41 % of the time, vector units 46 %, LDS half): 832 TFLOP/s at 3001 x
 // 28672 x 4096 (4 bits, groups of 128), where 128 x 128 tiles of weights
 // unpacked into LDS reached 418.  128 x 256 tiles with one wave a SIMD: 570.
 // LDS slots without bank conflicts: the same time.  us a call, before and now:
 //                       64 rows      256 rows      3001 rows
-//   n 28672, k 4096   107 -> 40.2   178 -> 87.5   1690 -> 907
-//   n 4096, k 14336   369 -> 26.4   361 -> 52.2    890 -> 506   (4 bits)
-//   n 6144, k 4096    101 -> 19.5   103 -> 32.6    422 -> 216
-//   n 16384, k 2048    58 -> 24.2    59 -> 46.2    501 -> 360   (8 bits,
-//   n 2048, k 8192    203 -> 20.8   203 -> 31.1    343 -> 233    group 64)
+//   n 28672, k 4096   107 -> 40.2   178 -> 87.5   1690 -> 847
+//   n 4096, k 14336   369 -> 26.4   361 -> 52.2    890 -> 459   (4 bits)
+//   n 6144, k 4096    101 -> 19.5   103 -> 32.6    422 -> 210
+//   n 16384, k 2048    58 -> 24.2    59 -> 46.2    501 -> 336   (8 bits,
+//   n 2048, k 8192    203 -> 20.8   203 -> 31.1    343 -> 213    group 64)
 #include "dq_frag.h"
 #include "lds_dma.h"
 
@@ -308,14 +308,30 @@ template <int BITS, int KC, DqMode MODE, bool LARGE>
 __global__ __launch_bounds__(TPB, 2) void dq_tile_kernel(DqArgs A, int mb,
                                                          int step) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  // an XCD's workgroups share columns: row tiles run fastest
+  // Up to eight row tiles: an XCD takes a range of columns, row tiles fastest
+  // (n 28672, k 4096, 256 rows: 94 us, 97 columns fastest over all XCDs; 8
+  // bits, n 32000: 96, 102).  More: columns fastest (2600 rows: 809, 765; 660
+  // tokens through 8 experts 924, 869), or, where every eighth row tile is the
+  // same XCD's, row tiles (3001 rows: 924 / 865 / 847 in this order).
   const u32 nb = MODE == GLU ? (A.n / 2 + 63) / 64 : (A.n + 127) / 128;
-  u32 id = xcd_swizzle(blockIdx.x, gridDim.x);
-  const int mt = (int)(id % mb);
-  id /= mb;
-  const int nblk = (int)(id % nb), sp = (int)(id / nb);
-  int row0 = mt * step, rows = min(A.m - row0, step), expert = 0;
-  if (MODE != DENSE && A.tiles != nullptr) {
+  const bool list = MODE != DENSE && A.tiles != nullptr;
+  const bool ranges = !list && mb <= 8;
+  u32 id = ranges ? xcd_swizzle(blockIdx.x, gridDim.x) : blockIdx.x;
+  u32 mt, nblk;
+  if (ranges || (!list && mb % 8 == 0)) {
+    mt = id % mb;
+    id /= mb;
+    nblk = id % nb;
+    id /= nb;
+  } else {
+    nblk = id % nb;
+    id /= nb;
+    mt = id % mb;
+    id /= mb;
+  }
+  const int sp = (int)id;
+  int row0 = (int)mt * step, rows = min(A.m - row0, step), expert = 0;
+  if (list) {
     expert = A.tiles[3 * mt];
     if (expert < 0) return;
     row0 = A.tiles[3 * mt + 1];
