@@ -378,6 +378,27 @@ hipError_t go_bits(const DqArgs& A, int bits, int mb, int step,
   return hipErrorInvalidValue;
 }
 
+// Rows of the tiles of a whole k.  Two workgroups a CU take a round, one
+// alone 0.69 of it; a tile of 96 rows 0.9 of one of 128, of 64 rows 0.75 (less
+// where the rounds are many, but then the last one does not matter).  us with
+// 128 / 96 / 64, 4 bits, k 4096: n 6144, 1300 rows 131 / 118 / 103, 1500 rows
+// 133 / 118 / 136, 1024 rows 73 / 106 / 92; n 4096, 1500 rows 78 / 70 / 92; n
+// 28672, 800 rows 277 / 268 / 302.
+int tile_rows(int m, int n, int cols) {
+  int best = ROWS;
+  float least = INFINITY;
+  for (int r = ROWS; r >= 64; r -= 32) {
+    const u32 u = ceil_div_u32(ceil_div_u32(m, r) * ceil_div_u32(n, cols), 256);
+    const float t = ((u / 2) + (u & 1) * 0.69f) *
+                    (r == 128 ? 1.f : (r == 96 ? 0.9f : 0.75f));
+    if (t < least * 0.99f) {
+      least = t;
+      best = r;
+    }
+  }
+  return best;
+}
+
 }  // namespace
 
 bool lfmq_dq_tile_ok(int k, int g) {
@@ -416,7 +437,9 @@ hipError_t lfmq_dq_tile(const void* qweight, const void* scales,
                  (unsigned short*)y, (const unsigned short*)bias, nullptr,
                  (float*)part, m, n, k, g, splits, nullptr, nullptr, nullptr};
   // row tiles alike, in sixteens: 129 rows are two of 80
-  const int mb = (int)ceil_div_u32(m, ROWS);
+  const int most = splits == 1 ? tile_rows(m, glu ? n / 2 : n, glu ? 64 : 128)
+                               : ROWS;
+  const int mb = (int)ceil_div_u32(m, most);
   const int step = (int)ceil_div_u32(ceil_div_u32(m, mb), 16) * 16;
   hipError_t e;
   if (glu && splits == 1)
