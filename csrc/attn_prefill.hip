@@ -19,9 +19,9 @@
 // Bound by the LDS reads of both operands and the softmax's vector work.
 // 32 heads on 8, us before (values transposed by 2-byte LDS writes, weights
 // through LDS) and now:
-//   1 x 512          32.2 ->  14.9    1 x 3001 after 1000   866 -> 207
-//   2 x 330          33.9 ->  13.6    1 x 8192             3785 -> 861
-//   1 x 2048          367 ->  79      (594 and 639 TFLOP/s)
+//   1 x 512          32.2 ->  15.1    1 x 3001 after 1000   866 -> 186
+//   2 x 330          33.9 ->  12.8    1 x 8192             3785 -> 620
+//   1 x 2048          367 ->  65      (663 and 887 TFLOP/s)
 #include "lds_dma.h"
 
 namespace {
@@ -39,7 +39,7 @@ typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
 struct PArgs {
   const unsigned short *q, *kc, *vc;
   unsigned short* o;
-  int s, hq, hkv, tmax, pos0, T;
+  int s, b, hq, hkv, tmax, pos0, T;
   float scale;
 };
 
@@ -52,8 +52,17 @@ template <int QT>
 __global__ __launch_bounds__(TPB, 2) void attn_prefill_kernel(PArgs A) {
   constexpr int BM = NW * QT * 16;
   extern __shared__ __attribute__((aligned(16))) char smem[];  // [2][K | V]
-  const int q0 = (gridDim.x - 1 - blockIdx.x) * BM;
-  const int h = blockIdx.y, bb = blockIdx.z, hk = h / (A.hq / A.hkv);
+  // An XCD (every eighth workgroup) takes an eighth of the heads, if that
+  // divides them, so that its L2 holds the keys and values they share: heads
+  // fastest, last queries first (8192 queries 851 us, so 620)
+  const u32 nq = (A.s + BM - 1) / BM, all = A.hq * A.b, per = all / 8;
+  u32 id = blockIdx.x, hb = id / nq, qt = id % nq;
+  if (all % 8 == 0) {
+    hb = id % 8 * per + id / 8 % per;
+    qt = id / 8 / per;
+  }
+  const int q0 = (int)(nq - 1 - qt) * BM;
+  const int h = hb % A.hq, bb = hb / A.hq, hk = h / (A.hq / A.hkv);
   const int lane = threadIdx.x & 63, l15 = lane & 15, l4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned short* K = A.kc + ((u64)bb * A.hkv + hk) * A.tmax * HD;
@@ -207,7 +216,7 @@ __global__ __launch_bounds__(TPB, 2) void attn_prefill_kernel(PArgs A) {
 template <int QT>
 hipError_t launch(const PArgs& A, int b, hipStream_t stream) {
   constexpr int lds = 4 * TILE;
-  const dim3 grid((A.s + NW * QT * 16 - 1) / (NW * QT * 16), A.hq, b);
+  const dim3 grid((A.s + NW * QT * 16 - 1) / (NW * QT * 16) * A.hq * A.b);
   hipLaunchKernelGGL(attn_prefill_kernel<QT>, grid, dim3(TPB), lds, stream, A);
   return hipGetLastError();
 }
@@ -225,10 +234,10 @@ hipError_t lfmq_attn_prefill(const void* q, const void* kc, const void* vc,
   const int T = pos0 + s;
   if (T > tmax) return hipErrorInvalidValue;
   const PArgs A{(const unsigned short*)q, (const unsigned short*)kc,
-                (const unsigned short*)vc, (unsigned short*)o, s, hq, hkv,
+                (const unsigned short*)vc, (unsigned short*)o, s, b, hq, hkv,
                 tmax, pos0, T, scale};
   // 128 queries a workgroup where they fill the chip, else 64 (us of 64 / 128:
-  // 512 queries 14.9 / 17.4, 1024 32.1 / 33.4, 2048 109 / 79)
+  // 512 queries 14.9 / 17.4, 1024 32.1 / 33.4, 2048 109 / 79, heads in turn)
   if ((long)((s + 127) / 128) * hq * b >= 384) return launch<2>(A, b, stream);
   return launch<1>(A, b, stream);
 }
