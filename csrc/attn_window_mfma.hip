@@ -33,6 +33,7 @@ struct PArgs {
   u64 ldo;
   float gain;
   bool v4;               // four columns of g and out may be moved at once
+  int max_count = 0;     // tokens of the longest sequence
 };
 
 __device__ __forceinline__ u32 swz(u32 row) { return (row ^ (row >> 3)) & 7; }
@@ -52,9 +53,23 @@ __global__ __launch_bounds__(TPB, 2) void attn_window_prompt_mfma(SeqView sv,
   extern __shared__ __attribute__((aligned(16))) char smem[];
   char* ldsK = smem;
   char* ldsV = ldsK + BN * KROW;
-  // the last queries see the most keys: they start first
-  const int q0 = (gridDim.x - 1 - blockIdx.x) * BM;
-  const int s = blockIdx.z, h = blockIdx.y, kh = h / A.group;
+  // The last queries see the most keys: they start first.  Where eight divides
+  // the heads, an XCD (every eighth workgroup) takes an eighth of them, whose
+  // keys and values its L2 then holds.
+  const u32 nq = (A.max_count + BM - 1) / BM, per = A.heads / 8;
+  u32 id = blockIdx.x, qi, s, h;
+  if (A.heads % 8 == 0) {
+    h = id % 8 * per + id / 8 % per;
+    id /= A.heads;
+    s = id % sv.b;
+    qi = id / sv.b;
+  } else {
+    qi = id % nq;
+    h = id / nq % A.heads;
+    s = id / nq / A.heads;
+  }
+  const int q0 = (int)(nq - 1 - qi) * BM;
+  const int kh = h / A.group;
   const int row0 = sv.cu[s], cnt = sv.cu[s + 1] - row0;
   if (q0 >= cnt) return;
   const int slot = sv.slots[s], len0 = sv.lens[slot];
@@ -302,9 +317,12 @@ hipError_t launch(const SeqView& sv, const PArgs& A, int max_count,
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     set = true;
   }
-  hipLaunchKernelGGL((attn_window_prompt_mfma<KS, VT, QT>),
-                     dim3((max_count + 64 * QT - 1) / (64 * QT), A.heads, sv.b),
-                     dim3(TPB), lds, stream, sv, A);
+  PArgs B = A;
+  B.max_count = max_count;
+  const u64 wgs = (u64)((max_count + 64 * QT - 1) / (64 * QT)) * A.heads * sv.b;
+  if (wgs >= 1ull << 31) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((attn_window_prompt_mfma<KS, VT, QT>), dim3((u32)wgs),
+                     dim3(TPB), lds, stream, sv, B);
   return hipGetLastError();
 }
 
