@@ -9,10 +9,11 @@
 // mirror image.
 //
 // A workgroup = 128 x 128, 4 waves of 64 x 64, tokens in steps of 64 through
-// two LDS buffers.  Tiles run in blocks of 8 x 8, one block to an XCD at a
-// time, whose L2 then serves a row of tiles eight times.  Bound by the LDS
+// two LDS buffers.  Tiles run in blocks of 4 x 4, a range of blocks to an XCD,
+// whose L2 then serves a row of tiles four times (8 x 8 leave more of the
+// triangle's edge empty: 102 x 7416 99 us, 82 so).  Bound by the LDS
 // reads of the fragments and by reading and writing H (in whole lines,
-// through LDS), one after the other.  2048 x 14336: 770 us (547 TFLOP/s of
+// through LDS), one after the other.  2048 x 14336: 653 us (645 TFLOP/s of
 // the half computed), against 2102 for the full square staged through
 // transposing 2-byte LDS writes; 2048 x 2048: 33 (70), 64 x 512: 9.3 (8.5).
 #include "lds_dma.h"
@@ -21,7 +22,7 @@ namespace {
 
 constexpr int TPB = 256, NW = 4;
 constexpr int BC = 128, BK = 64;             // tile side, tokens a step
-constexpr int SB = 8;                        // tiles a side of a block
+constexpr int SB = 4;                        // tiles a side of a block
 constexpr int BUF = 2 * BC * BK * 2;         // both operands of a step
 constexpr int LD = BC + 1;                   // of the result in LDS
 
@@ -156,9 +157,9 @@ __global__ __launch_bounds__(TPB, 2) void hessian_kernel(
   }
   // ... more are bound by the traffic: through LDS, so that 512 bytes of a row
   // are read and written together either way, 32 elements a thread in flight
-  // (128 x 14336: 341 us, 707 from the fragments; 102 x 7416, whose rows do
-  // not start lines: 100, 105 with halves of the tile and 256 bytes of the
-  // mirror.  LD: rows and columns both spread over the banks)
+  // (128 x 14336: 350 us, 707 from the fragments; with halves of the tile and
+  // 256 bytes of the mirror, 102 x 7416, whose rows do not start lines, is 5 %
+  // slower.  LD: rows and columns both spread over the banks)
   float* out = (float*)smem;
   __syncthreads();
 #pragma unroll
