@@ -825,7 +825,9 @@ T_ silu_mul_fused(T_ gu) {
 // x [..., k] w^T, or silu(gate) * up of it; undefined where the kernel does
 // not take it (its sizes, strides, types)
 c10::optional<T_> linear_rows(T_ x, T_ w, bool glu) {
+  // (the library also runs on a device that is not the current one)
   if (!x.is_cuda() || x.device() != w.device() || x.dim() < 1 ||
+      x.get_device() != at::cuda::getCurrentCUDAStream().device_index() ||
       x.scalar_type() != torch::kBFloat16 ||
       w.scalar_type() != torch::kBFloat16 || w.dim() != 2 ||
       !w.is_contiguous() || x.size(-1) != w.size(1) ||

@@ -72,7 +72,8 @@ def _inverse_factor(h: torch.Tensor) -> torch.Tensor:
     """U upper triangular with UᵀU = h⁻¹."""
     if h.is_cuda:
         from ..ops import hip_ext
-        U, failed = hip_ext().chol_inverse(h.contiguous())
+        with torch.cuda.device(h.device):
+            U, failed = hip_ext().chol_inverse(h.contiguous())
         if not failed.item():
             return U
         # a pivot is not positive in this order of elimination
@@ -89,8 +90,9 @@ def _gpu_block(w, ub, codes, scales, zeros, i1, cfg, g) -> torch.Tensor:
     from ..ops import hip_ext
     if ub.stride(1) != 1:
         ub = ub.contiguous()
-    return hip_ext().gptq_block(w, ub, codes, scales, zeros, i1,
-                                g, cfg.bits, cfg.sym)
+    with torch.cuda.device(w.device):
+        return hip_ext().gptq_block(w, ub, codes, scales, zeros, i1, g,
+                                    cfg.bits, cfg.sym)
 
 
 @torch.no_grad()
@@ -108,7 +110,7 @@ def gptq_quantize_layer(
     n, k = w.shape
     g = k if cfg.group_size == -1 else cfg.group_size
     G = k // g
-    w = w.float().clone()
+    w = w.float().clone(memory_format=torch.contiguous_format)
     h = h.float().clone()
     dev = w.device
 

@@ -499,6 +499,23 @@ def test_chol_inverse(n):
         assert ext().chol_inverse(bad)[1].item() == 1
 
 
+def test_gptq_solve_takes_any_strides():
+    from lfmq import QuantConfig
+    from lfmq.quant.gptq import gptq_quantize_layer
+    torch.manual_seed(3)
+    cfg = QuantConfig(scheme="gptq", bits=4, group_size=32)
+    x = torch.randn(300, 128, device=DEV)
+    h = x.t() @ x
+    wide = torch.randn(128, 48, device=DEV)
+    want = gptq_quantize_layer(wide.t().contiguous(), h, cfg)
+    big = torch.zeros(128, 256, device=DEV)
+    big[:, ::2] = h
+    for got in (gptq_quantize_layer(wide.t(), h, cfg),
+                gptq_quantize_layer(wide.t(), big[:, ::2], cfg)):
+        for a, b in zip(got[:3], want[:3]):
+            assert torch.equal(a, b)
+
+
 def test_gptq_solve_refuses_what_is_not_positive_definite():
     from lfmq import QuantConfig
     from lfmq.quant.gptq import gptq_quantize_layer
