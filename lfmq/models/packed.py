@@ -56,6 +56,7 @@ class PackedCausalLM(nn.Module):
         or of the `select`ed ones (int64 row numbers).  Advances the cache.
         trace collects the residual stream after every layer run."""
         self._check(tokens)
+        batch.arrive()
         logits = self._run(tokens, batch, cache, select, trace)
         cache.advance(tokens, batch)
         return logits

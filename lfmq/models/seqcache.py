@@ -36,7 +36,8 @@ class StepBatch:
     """counts[i] tokens of slot slots[i], rows packed in that order."""
 
     def __init__(self, slots: Sequence[int], counts: Sequence[int],
-                 len0: Sequence[int], device):
+                 len0: Sequence[int], device, lasting: bool = False):
+        """lasting: for more than the step it is made for, on any stream."""
         if len(slots) != len(counts) or not slots:
             raise ValueError("a step needs slots, and one count for each")
         if min(counts) < 1:
@@ -44,6 +45,9 @@ class StepBatch:
         if len(set(slots)) != len(slots):
             raise ValueError("a slot may appear once in a step")
         self.device = device
+        self._lasting = lasting
+        self._stream = None if lasting or torch.device(device).type != "cuda" \
+            else torch.cuda.current_stream(device)
         self.slot_ids, self.counts = list(slots), list(counts)
         self.len0 = list(len0)
         self.b, self.n = len(slots), sum(counts)
@@ -62,7 +66,17 @@ class StepBatch:
         self._chunks: Dict[int, tuple] = {}
 
     def _dev(self, ints) -> torch.Tensor:
+        if self._lasting:
+            return torch.tensor(ints, dtype=torch.int32).to(self.device)
         return upload(ints, torch.int32, self.device)
+
+    def arrive(self) -> None:
+        """The numbers' copies are queued on the stream that the batch was
+        made on; a step on another stream waits for them."""
+        if self._stream is not None:
+            now = torch.cuda.current_stream(self.device)
+            if now != self._stream:
+                now.wait_stream(self._stream)
 
     def view(self, cache):
         return self.seq, self.cu, self.slots, cache.lens
@@ -171,7 +185,7 @@ class SequenceCache:
         same from step to step (hipGraph capture)."""
         if b not in self._decode:
             self._decode[b] = StepBatch(range(b), [1] * b, [1] * b,
-                                        self.device)
+                                        self.device, lasting=True)
         return self._decode[b]
 
     def advance(self, tokens: torch.Tensor, batch: StepBatch) -> None:

@@ -918,3 +918,24 @@ def test_uploads_behind_queued_work_keep_their_numbers():
     for j, t in enumerate(got):
         i = j // 2
         assert t.tolist() == [i, i + 1] * (1 + i % 7)
+
+
+def test_batch_made_on_one_stream_steps_on_another():
+    """The step waits for the batch's numbers, which are queued behind work
+    of the stream that it was made on."""
+    from lfmq.models.rapivik import RapivikConfig
+    import lfmq
+    m = lfmq.build_model(RapivikConfig.tiny(n_layers=2), seed=1).to(DEV)
+    tok = torch.randint(0, 512, (7,), device=DEV)
+    want = m.forward_tokens(tok, (c := m.make_cache(2, 32)).batch([1], [7]), c)
+    cache = m.make_cache(2, 32)
+    x = torch.randn(4096, 4096, device=DEV)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(20):
+        x = (x @ x).clamp_(-1, 1)
+    batch = cache.batch([1], [7])
+    with torch.cuda.stream(side):
+        got = m.forward_tokens(tok, batch, cache)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
