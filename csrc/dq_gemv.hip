@@ -95,9 +95,8 @@ __global__ __launch_bounds__(WAVES_PER_WG * LFMQ_WAVE) void dq_gemv_kernel(
       }
       const int gg = lane + 64 * half;
       const u64 sidx = (u64)cc * G + gg;
-      const u32 sraw = __builtin_amdgcn_raw_buffer_load_b32(
-          s_rsrc, (u32)(sidx * 2) & ~3u, 0, 0);
-      const float s = bf16_bits_to_f32((sidx & 1) ? (sraw >> 16) : (sraw & 0xFFFF));
+      const float s = bf16_bits_to_f32((unsigned short)
+          __builtin_amdgcn_raw_buffer_load_b16(s_rsrc, (u32)(sidx * 2), 0, 0));
       const u32 zword = __builtin_amdgcn_raw_buffer_load_b32(
           z_rsrc, (u32)(((u64)cc * zw + gg / per_z) * 4), 0, 0);
       const u32 z = BITS == 4 ? unpack4(zword, gg % 8) : unpack8(zword, gg % 4);

@@ -662,6 +662,30 @@ def test_dq_rows_norm_gate_residual(bits, m, n, k, g):
                   torch.nn.functional.silu(a) * u)
 
 
+@pytest.mark.parametrize("m,n,k,g", [
+    (1, 37, 2048, 64), (1, 3073, 4224, 128), (1, 66, 14336, 128)])
+@pytest.mark.parametrize("eps", [-1.0, 1e-5])
+def test_dq_gemv_splits(m, n, k, g, eps):
+    """One or two rows: columns a wave, and k shared by a workgroup's waves;
+    n and k that end inside their tiles, with norm, bias and residual."""
+    torch.manual_seed(n + k)
+    codes = torch.randint(0, 16, (n, k), dtype=torch.int32)
+    zeros = torch.randint(0, 16, (n, k // g), dtype=torch.int32)
+    s16 = (torch.rand(n, k // g) * 0.02 + 0.01).to(torch.bfloat16)
+    w = ref.dequant_groupwise(codes, s16.float(), zeros, g).double().to(DEV)
+    x = torch.randn(m, k).to(torch.bfloat16).to(DEV)
+    b, r = (torch.randn(*t).to(torch.bfloat16).to(DEV) for t in ((n,), (m, n)))
+    y = ext().dq_linear(x, ref.pack_codes(codes, 4).to(DEV), s16.to(DEV),
+                        ref.pack_zeros(zeros, 4).to(DEV), 4, g, b, r, eps, 0)
+    want = x.double() @ w.t()
+    if eps > 0:
+        want *= torch.rsqrt((x.double() ** 2).mean(1, keepdim=True) + eps)
+    want += b.double() + r.double()
+    err = (y.double() - want).abs()
+    # sums of k products of bf16 pairs in 32 bits beside the result's rounding
+    assert float((err / (want.abs() + 1e-3 * want.abs().max())).max()) < 5e-3
+
+
 @pytest.mark.parametrize("m", [1, 2, 4])
 def test_dq_linear_of_many_groups(m):
     """More groups a row than the GEMV's lanes hold scales of."""
