@@ -111,6 +111,12 @@ __global__ __launch_bounds__(WAVES_PER_WG * LFMQ_WAVE) void dq_gemv_kernel(
     }
   }
 
+  // past the row: past all of x too, which reads as zeros (the next row's
+  // values would count in the norm)
+  auto x_at = [&](int mm, int k0) {
+    return k0 < k ? (u32)(mm * k + k0) * 2 : 0x7FFFFF00u;
+  };
+
   float acc[COLS][M];
 #pragma unroll
   for (int c = 0; c < COLS; ++c)
@@ -155,7 +161,7 @@ __global__ __launch_bounds__(WAVES_PER_WG * LFMQ_WAVE) void dq_gemv_kernel(
 #pragma unroll
       for (int mm = 0; mm < M; ++mm) {
         if (mm >= m) break;
-        const u32 xbyte = (u32)(mm * k * 2 + it * 4096 + lane * 64);
+        const u32 xbyte = x_at(mm, it * 2048 + lane * 32);
         u32x4 xq0 = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xbyte, 0, 0);
         u32x4 xq1 = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xbyte + 16, 0, 0);
         u32x4 xq2 = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xbyte + 32, 0, 0);
@@ -232,7 +238,7 @@ __global__ __launch_bounds__(WAVES_PER_WG * LFMQ_WAVE) void dq_gemv_kernel(
 #pragma unroll
       for (int mm = 0; mm < M; ++mm) {
         if (mm >= m) break;
-        const u32 xbyte = (u32)(mm * k * 2 + it * 4096 + lane * 64);
+        const u32 xbyte = x_at(mm, it * 2048 + lane * 32);
         u32x4 xq0 = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xbyte, 0, 0);
         u32x4 xq1 = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xbyte + 16, 0, 0);
         u32x4 xq2 = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xbyte + 32, 0, 0);
@@ -290,7 +296,7 @@ __global__ __launch_bounds__(WAVES_PER_WG * LFMQ_WAVE) void dq_gemv_kernel(
 #pragma unroll
       for (int mm = 0; mm < M; ++mm) {
         if (mm >= m) break;
-        const u32 xbyte = (u32)(mm * k * 2 + it * 4096 + lane * 64);
+        const u32 xbyte = x_at(mm, it * 2048 + lane * 32);
         float xv[32];
 #pragma unroll
         for (int h = 0; h < 4; ++h) {
