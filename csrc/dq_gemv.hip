@@ -485,11 +485,17 @@ hipError_t launch_bits(const void* qweight, const void* scales,
     // sustains >6 TB/s at large grids).  cols_hint 0 = auto.
     int cols = cols_hint;
     const int kiters = (k + 2047) / 2048;
-    // measured: wg-internal split-k does NOT beat the multi-column wave
-    // layout on the decode shapes (LDS combine + fewer weight streams
-    // offset the shorter latency chain) — kept behind hint 5 for A/B.
-    const bool want_ksplit = !GATEUP && BITS == 4 && kiters >= 2 &&
-                             cols_hint == 5;
+    // One row of 4-bit weights, us with 1 / 2 columns a wave and with four
+    // columns whose k the workgroup's waves share: n 2048, k 2048 3.6 / 3.9 /
+    // 3.8, n 2048, k 8192 6.2 / 6.7 / 6.2, n 4096, k 4096 5.6 / 5.8 / 6.6, n
+    // 4096, k 11008 10.3 / 10.3 / 11, k 14336 13.9 / 13.2 / 12.5, n 5120, k
+    // 13824 16 / 16 / 13.4, n 6144, k 14336 17.9 / 16.8 / 17.1.  Two rows: n
+    // 2048, k 4096 5.5 / 5.6, k 8192 8.4 / 8.2.
+    const bool narrow = !GATEUP && BITS == 4 && m <= 2;
+    const bool want_ksplit =
+        !GATEUP && BITS == 4 &&
+        ((cols_hint == 5 && kiters >= 2) ||
+         (cols_hint == 0 && m == 1 && kiters >= 7 && n < 6144));
     if (want_ksplit) {
       // wg-internal split-k: the 4 waves share 4 columns
       dim3 gridk(ceil_div_u32(n, 4));
@@ -501,6 +507,9 @@ hipError_t launch_bits(const void* qweight, const void* scales,
         launch_ksplit<BITS, 4, false, 4, RMS>(gridk, block, stream, qweight, scales, qzeros, x, y, bias, resid, m, n, k, g, eps);
       return hipGetLastError();
     }
+    if (cols == 0 && narrow &&
+        (k <= 4096 ? n <= (m == 1 ? 4096 : 3072) : m == 1 && n <= 3072))
+      cols = 1;
     if (cols == 0 || cols == 5) cols = (GATEUP || n >= 16384) ? 4 : 2;
     const int per_wg = WAVES_PER_WG * (GATEUP ? cols / 2 : cols);
     dim3 grid(ceil_div_u32(GATEUP ? n / 2 : n, per_wg));

@@ -664,7 +664,8 @@ def test_dq_rows_norm_gate_residual(bits, m, n, k, g):
 
 @pytest.mark.parametrize("m,n,k,g", [
     (1, 37, 2048, 64), (2, 3071, 256, 128), (1, 3073, 4224, 128),
-    (2, 130, 4224, 128), (1, 66, 14336, 128)])
+    (2, 130, 4224, 128), (1, 61, 12416, 128), (1, 66, 14336, 128),
+    (1, 4097, 512, 128)])
 @pytest.mark.parametrize("eps", [-1.0, 1e-5])
 def test_dq_gemv_splits(m, n, k, g, eps):
     """One or two rows: columns a wave, and k shared by a workgroup's waves;
