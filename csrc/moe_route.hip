@@ -81,7 +81,8 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(RouteArgs A) {
       for (int j = na; j < E; ++j) A.active[j] = -1;
   }
   __syncthreads();
-  if (A.offsets != nullptr && tid <= E) A.offsets[tid] = offs[tid];
+  if (A.offsets != nullptr)                // one more than there may be threads
+    for (int e = tid; e <= E; e += blockDim.x) A.offsets[e] = offs[e];
   if (A.tiles != nullptr) {
     for (int i = tid; i < A.n_tiles; i += blockDim.x) {
       int e = -1;
