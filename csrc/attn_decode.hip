@@ -364,7 +364,7 @@ hipError_t launch(const DArgs& A, int b, hipStream_t stream) {
 int lfmq_attn_decode_splits(int b, int hq, int hkv, int T) {
   const int group = hq / hkv, gh = head_tile(group);
   const int wgs = b * hkv * ((group + gh - 1) / gh);
-  const int n = FULL_WGS / wgs;
+  const int n = FULL_WGS / max(wgs, 1);
   const int most = (T + LEAST_KEYS - 1) / LEAST_KEYS;
   return max(1, min(min(n, most), MAX_SPLITS));
 }

@@ -16,6 +16,19 @@ def ext():
     return hip_ext()
 
 
+# ------------------------------------------------------------- attention
+def test_decode_attention_of_no_sequences():
+    """Refused, as a launch of nothing is."""
+    kc = torch.zeros(0, 8, 64, 128, dtype=BF, device=DEV)
+    with pytest.raises(RuntimeError, match="invalid configuration"):
+        ext().attn_decode(torch.zeros(0, 32, 1, 128, dtype=BF, device=DEV),
+                          kc, kc, 33, 0.1, None)
+    with pytest.raises(RuntimeError, match="invalid configuration"):
+        ext().attn_decode_fused(
+            torch.zeros(0, 48 * 128, dtype=BF, device=DEV), kc, kc, 33, 0.1,
+            torch.ones(64, device=DEV), 32, None, None)
+
+
 # --------------------------------------------------------------- routing
 @pytest.mark.parametrize("t", [1, 2, 63, 64])
 def test_route_to_as_many_experts_as_lanes(t):
