@@ -433,7 +433,8 @@ bool lfmq_dq_rows_ok(int m, int n, int k, int g, bool fused) {
 int lfmq_dq_rows_splits(int m, int n, int k, int g) {
   const Tile t = tile_of(m, n, k, g, false, false);
   if (t.whole && meta_bytes(k, g, 1, t.nt) <= 64 * 1024) return 1;
-  const int wgs = (int)(ceil_div_u32(n, t.nt * 16) * ceil_div_u32(m, t.mt * 16));
+  const int wgs = max(1, (int)(ceil_div_u32(n, t.nt * 16) *
+                               ceil_div_u32(m, t.mt * 16)));
   const int C = k / chunk_of(g);
   // 256 workgroups, or 512 where a wave keeps six chunks (us at 8 rows, 2 / 4
   // splits: n 4096, k 4096 9.0 / 9.7, k 14336 18.3 / 17.8)

@@ -406,7 +406,7 @@ bool lfmq_dq_tile_ok(int k, int g) {
 }
 
 int lfmq_dq_tile_splits(int m, int n, int k, int g) {
-  const int wgs = (int)(ceil_div_u32(n, 128) * ceil_div_u32(m, 128));
+  const int wgs = max(1, (int)(ceil_div_u32(n, 128) * ceil_div_u32(m, 128)));
   const int C = k / (g % 128 == 0 ? 128 : 64);
   // 256 workgroups, or 512 where six chunks are left to each (us at 64 rows,
   // 4 bits: n 28672, k 4096 57 / 48, n 6144 21.8 / 23.8, n 4096, k 14336

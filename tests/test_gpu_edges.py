@@ -29,6 +29,26 @@ def test_decode_attention_of_no_sequences():
             torch.ones(64, device=DEV), 32, None, None)
 
 
+# ------------------------------------------------------- packed products
+def test_packed_product_of_nothing():
+    """No rows: no rows, however large the matrix; no columns: refused, as a
+    launch of nothing is."""
+    n, k, g = 6144, 4096, 128
+    p = [torch.zeros(n, k // 8, dtype=torch.int32, device=DEV),
+         torch.ones(n, k // g, dtype=BF, device=DEV),
+         torch.zeros(n, k // g // 8, dtype=torch.int32, device=DEV)]
+    x, r = (torch.zeros(0, c, dtype=BF, device=DEV) for c in (k, n))
+    for resid, eps in ((None, -1.0), (r, -1.0), (None, 1e-5)):
+        y = ext().dq_linear(x, *p, 4, g, None, resid, eps, 0)
+        assert y.shape == (0, n)
+    assert ext().dq_gemv_gateup(x, *p, 4, g, -1.0, 0).shape == (0, n // 2)
+    empty = [t[:0] for t in p]
+    for m in (1, 8, 64):
+        with pytest.raises(RuntimeError, match="invalid configuration"):
+            ext().dq_linear(torch.zeros(m, k, dtype=BF, device=DEV), *empty, 4,
+                            g, None, None, -1.0, 0)
+
+
 # --------------------------------------------------------------- routing
 @pytest.mark.parametrize("t", [1, 2, 63, 64])
 def test_route_to_as_many_experts_as_lanes(t):
