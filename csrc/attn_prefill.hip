@@ -40,7 +40,7 @@ struct PArgs {
   const unsigned short *q, *kc, *vc;
   unsigned short* o;
   int s, b, hq, hkv, tmax, pos0, T;
-  float scale;
+  float scale, sign;       // scale > 0; what queries are multiplied by first
 };
 
 __device__ __forceinline__ u32 pack2(float a, float b) {
@@ -93,6 +93,16 @@ __global__ __launch_bounds__(TPB, 2) void attn_prefill_kernel(PArgs A) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
       qf[qt][ks] = *(const s16x8*)(p + ks * 32 + l4 * 8);
+  }
+  if (A.sign != 1.f) {
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          qf[qt][ks][e] = (short)f32_to_bf16_bits_rne(
+              bf16_bits_to_f32((unsigned short)qf[qt][ks][e]) * A.sign);
   }
   const float sc2 = A.scale * LOG2E;             // softmax in powers of two
   const int w_lo = A.pos0 + w0, w_hi = w_lo + QT * 16 - 1;   // positions
@@ -233,9 +243,14 @@ hipError_t lfmq_attn_prefill(const void* q, const void* kc, const void* vc,
   if (hq % hkv) return hipErrorInvalidValue;
   const int T = pos0 + s;
   if (T > tmax) return hipErrorInvalidValue;
+  // The kernel compares scores before it scales them.  A scale that turns
+  // their order or makes them equal goes to the queries instead: -1 and 0 are
+  // exact there, and NaN makes all of them NaN.
+  const bool up = scale > 0.f;
   const PArgs A{(const unsigned short*)q, (const unsigned short*)kc,
                 (const unsigned short*)vc, (unsigned short*)o, s, b, hq, hkv,
-                tmax, pos0, T, scale};
+                tmax, pos0, T, up ? scale : (scale < 0.f ? -scale : 1.f),
+                up ? 1.f : (scale < 0.f ? -1.f : scale)};
   // 128 queries a workgroup where they fill the chip, else 64 (us of 64 / 128:
   // 512 queries 14.9 / 17.4, 1024 32.1 / 33.4, 2048 109 / 79, heads in turn)
   if ((long)((s + 127) / 128) * hq * b >= 384) return launch<2>(A, b, stream);

@@ -1,6 +1,7 @@
 """The edges of what the GPU calls take: nothing at all, more than a counter
 or an address holds, infinities, numbers below the normal range, tensors that
 stand for more than their values, streams and graphs."""
+import math
 
 import pytest
 import torch
@@ -17,6 +18,28 @@ def ext():
 
 
 # ------------------------------------------------------------- attention
+@pytest.mark.parametrize("scale", [0.0, -0.125])
+@pytest.mark.parametrize("s,pos0", [(70, 0), (130, 33)])
+def test_prompt_attention_takes_any_scale(scale, s, pos0):
+    """A scale of 0 weighs all visible keys alike, a negative one prefers
+    the least scores.  Weights are rounded to 8 bits, as the result is."""
+    torch.manual_seed(s)
+    hq, hkv, d, T = 4, 2, 128, pos0 + s
+    q = torch.randn(1, s, hq, d).to(BF)
+    kc, vc = (torch.randn(1, hkv, T + 9, d).to(BF) for _ in range(2))
+    got = ext().attn_prefill(q.view(1, s, -1).to(DEV), kc.to(DEV), vc.to(DEV),
+                             hq, pos0, scale)
+    k, v = (t[0, :, :T].double().repeat_interleave(hq // hkv, 0)
+            for t in (kc, vc))
+    sc = q[0].double().transpose(0, 1) @ k.transpose(1, 2) * scale
+    seen = torch.arange(T) <= pos0 + torch.arange(s).unsqueeze(1)
+    w = torch.softmax(sc.masked_fill(~seen, -math.inf), -1)
+    want = (w @ v).transpose(0, 1).reshape(s, hq * d)
+    got = got.double().cpu().view(s, hq * d)
+    assert bool(got.isfinite().all())
+    assert float((got - want).abs().max() / want.abs().max()) < 2 ** -7
+
+
 def test_decode_attention_of_no_sequences():
     """Refused, as a launch of nothing is."""
     kc = torch.zeros(0, 8, 64, 128, dtype=BF, device=DEV)
