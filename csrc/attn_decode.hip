@@ -205,9 +205,16 @@ __global__ __launch_bounds__(TPB) void attn_decode_kernel(DArgs A) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc[h][e] *= a;
     }
+    // rows past the range are the last one again: 0, which their weight of 0
+    // leaves 0 (an infinite value would be NaN)
+    if (t0 + KT > hi) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i)
+        if (t0 + i * RPP + vrow >= hi) vv[i] = u32x4{0, 0, 0, 0};
+    }
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-      if (FUSED && min(t0 + i * RPP + vrow, hi - 1) == pos) vv[i] = v_new;
+      if (FUSED && t0 + i * RPP + vrow == pos) vv[i] = v_new;
       float v[8];
 #pragma unroll
       for (int e = 0; e < 4; ++e)

@@ -40,6 +40,28 @@ def test_prompt_attention_takes_any_scale(scale, s, pos0):
     assert float((got - want).abs().max() / want.abs().max()) < 2 ** -7
 
 
+@pytest.mark.parametrize("T", [1, 33, 70, 300])
+@pytest.mark.parametrize("fused", [False, True])
+def test_decode_attention_of_an_infinite_value(T, fused):
+    """An infinite value in the last row of the cache is weighed once."""
+    torch.manual_seed(T)
+    hq, hkv, d = 4, 2, 128
+    kc, vc = (torch.randn(1, hkv, T + 5, d).to(BF).to(DEV) for _ in range(2))
+    qkv = torch.randn(1, (hq + 2 * hkv) * d).to(BF).to(DEV)
+    if fused:
+        qkv.view(1, hq + 2 * hkv, d)[:, hq + hkv:, 7] = math.inf
+        o = ext().attn_decode_fused(qkv, kc, vc, T, d ** -0.5,
+                                    torch.ones(d // 2, device=DEV), hq, None,
+                                    None)
+    else:
+        vc[:, :, T - 1, 7] = math.inf
+        o = ext().attn_decode(qkv[:, :hq * d].view(1, hq, 1, d), kc, vc, T,
+                              d ** -0.5, None)
+    o = o.float().view(hq, d)
+    assert bool((o[:, 7] == math.inf).all())
+    assert bool(o[:, :7].isfinite().all() and o[:, 8:].isfinite().all())
+
+
 def test_decode_attention_of_no_sequences():
     """Refused, as a launch of nothing is."""
     kc = torch.zeros(0, 8, 64, 128, dtype=BF, device=DEV)
