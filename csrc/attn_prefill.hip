@@ -117,6 +117,14 @@ __global__ __launch_bounds__(TPB, 2) void attn_prefill_kernel(PArgs A) {
   for (int t0 = 0, par = 0; t0 < hi; t0 += BN, par ^= 1) {
     lds_loads_done();
     if (t0 + BN < hi) stage(t0 + BN, par ^ 1);
+    if (t0 + BN > hi) {
+      // values past the end: 0, which their weight of 0 leaves 0 (an infinite
+      // one would be NaN)
+      const u32x4 z = {0, 0, 0, 0};
+      for (int i = (hi - t0) * (ROW / 16) + threadIdx.x; i < TILE / 16; i += TPB)
+        *(u32x4*)(smem + par * 2 * TILE + TILE + i * 16) = z;
+      __syncthreads();
+    }
     if (t0 > w_hi) continue;                     // none seen
     const char* lk = smem + par * 2 * TILE;
     const char* lv = lk + TILE;

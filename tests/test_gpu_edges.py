@@ -62,6 +62,21 @@ def test_decode_attention_of_an_infinite_value(T, fused):
     assert bool(o[:, :7].isfinite().all() and o[:, 8:].isfinite().all())
 
 
+@pytest.mark.parametrize("s,pos0", [(1, 0), (70, 0), (130, 33)])
+def test_prompt_attention_of_an_infinite_value(s, pos0):
+    """The same for a prompt's last query."""
+    from lfmq.ops import functional as F
+    torch.manual_seed(s)
+    hq, hkv, d, T = 4, 2, 128, pos0 + s
+    q = torch.randn(1, s, hq, d).to(BF).to(DEV)
+    kc, vc = (torch.randn(1, hkv, T + 9, d).to(BF).to(DEV) for _ in range(2))
+    vc[:, :, T - 1, 7] = math.inf
+    o = F.attn_prefill_fused(q, kc, vc, pos0, d ** -0.5)
+    o = o.float().view(s, hq, d)[-1]
+    assert bool((o[:, 7] == math.inf).all())
+    assert bool(o[:, :7].isfinite().all() and o[:, 8:].isfinite().all())
+
+
 def test_decode_attention_of_no_sequences():
     """Refused, as a launch of nothing is."""
     kc = torch.zeros(0, 8, 64, 128, dtype=BF, device=DEV)
