@@ -10,14 +10,18 @@
 // workgroup.  Lane c of a row holds columns 64 i + 4 c + 0..3: a row of U is
 // read in 16-byte pieces side by side, the same address for all four rows.
 // Bound by the chain broadcast -> quotients -> update, 128 times 0.25 us:
-// 2048 rows take 37 us a block of 128 (56 with divisions and a search for
+// 2048 rows take 34.7 us a block of 128 (56 with divisions and a search for
 // the groups' starts in the chain), where one launch per elementwise
-// operation took 7.2 ms (with the gaps between them).
+// operation took 7.2 ms (with the gaps between them).  Four rows that meet
+// numbers whose quotients need a division are done again with divisions: 65
+// us (tested column by column: 37 for all).
 //
 // Every operation rounds on its own, in the order of the tensor expressions
 // above, so that results are those of a GPU tensor loop, bit by bit: no
 // contraction, and a division by a constant is a product with its
 // reciprocal.
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -38,14 +42,21 @@ __device__ __forceinline__ float nclamp(float x, float hi) {
   return x < 0.f ? 0.f : (x > hi ? hi : x);
 }
 
+// 1 / d, or NaN where quotient() is not x / d to the last bit: its remainders
+// leave the normal range, or there is no reciprocal
+__device__ __forceinline__ float inverse(float d) {
+  const float r = 1.f / d;
+  return fabsf(r) > 0x1p-40f && fabsf(r) < 0x1p100f ? r : NAN;
+}
+
 // x / d given r = 1 / d, both rounded to nearest: the product corrected twice
 // by its remainder is the rounded quotient (Markstein), in half the steps of a
-// division that starts from d alone.  Infinite and NaN stay what they are.
+// division that starts from d alone.  NaN where the product is not finite; x
+// from 2^-80 on (below, the last bit of a quotient below it may differ).
 __device__ __forceinline__ float quotient(float x, float d, float r) {
   const float q0 = x * r;
   const float q1 = fmaf(fmaf(-q0, d, x), r, q0);
-  const float q2 = fmaf(fmaf(-q1, d, x), r, q1);
-  return fabsf(q0) < INFINITY ? q2 : q0;
+  return fmaf(fmaf(-q1, d, x), r, q1);
 }
 
 template <int NC>  // chunks of 64 columns
@@ -71,80 +82,94 @@ __global__ __launch_bounds__(TPB) void gptq_block_kernel(
       if (t0 + i * TPB < nb * BS) us[t0 + i * TPB] = v[i];
   }
   __syncthreads();
-  for (int j = threadIdx.x; j < nb; j += TPB) ru[j] = 1.f / us[j * BS + j];
+  for (int j = threadIdx.x; j < nb; j += TPB) ru[j] = inverse(us[j * BS + j]);
   __syncthreads();
   const int lane = threadIdx.x & 63, c16 = lane & 15;
   const int row = blockIdx.x * ROWS + (threadIdx.x >> 6) * RPW + (lane >> 4);
   const bool live = row < n;
   const float* wr = w + (u64)(live ? row : n - 1) * k;
 
-  float v[NC * 4];
+  // the block's columns; EXACT: with divisions.  Whether the quotients were
+  // those of divisions.
+  auto columns = [&](auto exact) {
+    constexpr bool EXACT = decltype(exact)::value;
+    float v[NC * 4];
 #pragma unroll
-  for (int i = 0; i < NC; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int c = i * 64 + c16 * 4 + r;
-      v[i * 4 + r] = c < nb ? wr[i1 + c] : 0.f;
-    }
-  float s = 1.f, z = 0.f, rs;
-  int start = (g - i1 % g) % g;            // column where the next group starts
-  if (i1 % g != 0) {                       // inside a group begun earlier
-    s = scales[(u64)(live ? row : n - 1) * G + i1 / g];
-    z = (float)zeros[(u64)(live ? row : n - 1) * G + i1 / g];
-  }
-  rs = 1.f / s;
-
-#pragma unroll
-  for (int i = 0; i < NC; ++i)
-    for (int c = 0; c < 16; ++c)
+    for (int i = 0; i < NC; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int j = i * 64 + c * 4 + r;
-        if (j >= nb) break;
-        if (j == start) {
-          start += g;
-          float lo = INFINITY, hi = -INFINITY;
-          for (int t = c16; t < g; t += 16) {
-            const float x = wr[i1 + j + t];
-            lo = nmin(lo, x);
-            hi = nmax(hi, x);
-          }
-#pragma unroll
-          for (int o = 8; o > 0; o >>= 1) {
-            lo = nmin(lo, __shfl_xor(lo, o, 64));
-            hi = nmax(hi, __shfl_xor(hi, o, 64));
-          }
-          if (sym) {
-            s = nmax(fabsf(lo), fabsf(hi)) * inv_range;
-            s = s == 0.f ? 1.f : s;
-            z = (qmax + 1.f) * 0.5f;
-          } else {
-            s = (hi - lo) * inv_range;
-            s = s == 0.f ? 1.f : s;
-            z = (float)(i32)nclamp(rintf(-lo / s), qmax);
-          }
-          rs = 1.f / s;
-          if (live && c16 == 0) {
-            scales[(u64)row * G + (i1 + j) / g] = s;
-            zeros[(u64)row * G + (i1 + j) / g] = (i32)z;
-          }
-        }
-        const float x = __shfl(v[i * 4 + r], (lane & 48) + c, 64);
-        const float q = nclamp(rintf(quotient(x, s, rs)) + z, qmax);
-        const float e =
-            quotient(x - (q - z) * s, us[j * BS + j], ru[j]);
-        if (live && c16 == 0) {
-          codes[(u64)row * k + i1 + j] = (i32)q;
-          err[(u64)row * nb + j] = e;
-        }
-#pragma unroll
-        for (int i2 = i; i2 < NC; ++i2) {
-          const f32x4 u = *(const f32x4*)(us + j * BS + i2 * 64 + c16 * 4);
-#pragma unroll
-          for (int r2 = 0; r2 < 4; ++r2)
-            v[i2 * 4 + r2] = v[i2 * 4 + r2] - e * u[r2];
-        }
+        const int c = i * 64 + c16 * 4 + r;
+        v[i * 4 + r] = c < nb ? wr[i1 + c] : 0.f;
       }
+    float s = 1.f, z = 0.f, rs;
+    int start = (g - i1 % g) % g;          // column where the next group starts
+    if (i1 % g != 0) {                     // inside a group begun earlier
+      s = scales[(u64)(live ? row : n - 1) * G + i1 / g];
+      z = (float)zeros[(u64)(live ? row : n - 1) * G + i1 / g];
+    }
+    rs = inverse(s);
+    u32 least = ~0u;                       // dividend but 0, as bits
+    float finite = 0.f;                    // NaN if an error was not
+
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      for (int c = 0; c < 16; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int j = i * 64 + c * 4 + r;
+          if (j >= nb) break;
+          if (j == start) {
+            start += g;
+            float lo = INFINITY, hi = -INFINITY;
+            for (int t = c16; t < g; t += 16) {
+              const float x = wr[i1 + j + t];
+              lo = nmin(lo, x);
+              hi = nmax(hi, x);
+            }
+#pragma unroll
+            for (int o = 8; o > 0; o >>= 1) {
+              lo = nmin(lo, __shfl_xor(lo, o, 64));
+              hi = nmax(hi, __shfl_xor(hi, o, 64));
+            }
+            if (sym) {
+              s = nmax(fabsf(lo), fabsf(hi)) * inv_range;
+              s = s == 0.f ? 1.f : s;
+              z = (qmax + 1.f) * 0.5f;
+            } else {
+              s = (hi - lo) * inv_range;
+              s = s == 0.f ? 1.f : s;
+              z = (float)(i32)nclamp(rintf(-lo / s), qmax);
+            }
+            rs = inverse(s);
+            if (live && c16 == 0) {
+              scales[(u64)row * G + (i1 + j) / g] = s;
+              zeros[(u64)row * G + (i1 + j) / g] = (i32)z;
+            }
+          }
+          const float x = __shfl(v[i * 4 + r], (lane & 48) + c, 64);
+          const float u_jj = us[j * BS + j];
+          const float q = nclamp(
+              rintf(EXACT ? x / s : quotient(x, s, rs)) + z, qmax);
+          const float y = x - (q - z) * s;
+          const float e = EXACT ? y / u_jj : quotient(y, u_jj, ru[j]);
+          least = min(least, (__builtin_bit_cast(u32, y) << 1) - 1u);
+          finite = fmaf(e, 0.f, finite);
+          if (live && c16 == 0) {
+            codes[(u64)row * k + i1 + j] = (i32)q;
+            err[(u64)row * nb + j] = e;
+          }
+#pragma unroll
+          for (int i2 = i; i2 < NC; ++i2) {
+            const f32x4 u = *(const f32x4*)(us + j * BS + i2 * 64 + c16 * 4);
+#pragma unroll
+            for (int r2 = 0; r2 < 4; ++r2)
+              v[i2 * 4 + r2] = v[i2 * 4 + r2] - e * u[r2];
+          }
+        }
+    return least >= (0x17800000u << 1) - 1u && finite == 0.f;
+  };
+  // no ordinary weights need the second
+  if (__any(!columns(std::false_type{}))) columns(std::true_type{});
 }
 
 }  // namespace

@@ -109,6 +109,36 @@ def test_packed_product_of_nothing():
                             g, None, None, -1.0, 0)
 
 
+# ------------------------------------------------------------------ gptq
+@pytest.mark.parametrize("tiny", [1e-40, 3e-38, 2e-36, 1e-33])
+def test_gptq_block_of_numbers_below_the_normal_range(tiny):
+    """Groups whose scale has no finite reciprocal, and remainders that leave
+    the normal range: still the tensor loop's quotients."""
+    from lfmq import QuantConfig
+    from lfmq.quant import gptq
+    torch.manual_seed(5)
+    n, k, g = 40, 128, 64
+    w = torch.randn(n, k, device=DEV)
+    w[0] = 0
+    w[0, 3] = tiny
+    w[1, :g] *= tiny
+    w[2] *= tiny
+    w[3] = 0
+    w[4, g:] = tiny
+    u = torch.randn(k, k, device=DEV).triu_() * 0.05
+    u.diagonal().copy_(torch.rand(k, device=DEV) + 0.5)
+    cfg = QuantConfig(scheme="gptq", bits=4, group_size=g)
+
+    def solve(f):
+        out = (torch.zeros(n, k, dtype=torch.int32, device=DEV),
+               torch.zeros(n, k // g, device=DEV),
+               torch.zeros(n, k // g, dtype=torch.int32, device=DEV))
+        return (*out, f(w, u, *out, 0, cfg, g))
+
+    for got, want in zip(solve(gptq._gpu_block), solve(gptq._block)):
+        assert torch.equal(got, want)
+
+
 # --------------------------------------------------------------- routing
 @pytest.mark.parametrize("t", [1, 2, 63, 64])
 def test_route_to_as_many_experts_as_lanes(t):
