@@ -496,7 +496,7 @@ hipError_t lfmq_dq_rows_experts(const void* qweight, const void* scales,
                                 const void* src, const void* tiles, void* y,
                                 int n_tiles, int n, int k, int g, int bits,
                                 bool glu, hipStream_t stream) {
-  if (g % 32 || g > k || k % g || n % 2) return hipErrorInvalidValue;
+  if (g % 32 || g > k || k % g || (glu && n % 2)) return hipErrorInvalidValue;
   DqArgs A{};
   A.w = (const char*)qweight;
   A.scales = (const unsigned short*)scales;

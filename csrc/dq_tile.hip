@@ -459,7 +459,8 @@ hipError_t lfmq_dq_tile_experts(const void* qweight, const void* scales,
                                 const void* src, const void* tiles, void* y,
                                 int n_tiles, int n, int k, int g, int bits,
                                 bool glu, hipStream_t stream) {
-  if (!lfmq_dq_tile_ok(k, g) || n % 2 || (u64)n * k * bits / 8 >= 1ull << 32)
+  if (!lfmq_dq_tile_ok(k, g) || (glu && n % 2) ||
+      (u64)n * k * bits / 8 >= 1ull << 32)
     return hipErrorInvalidValue;
   DqArgs A{};
   A.w = (const char*)qweight;

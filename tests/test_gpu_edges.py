@@ -6,6 +6,8 @@ import math
 import pytest
 import torch
 
+from lfmq.ops import ref
+
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
@@ -15,6 +17,17 @@ BF = torch.bfloat16
 def ext():
     from lfmq.ops import hip_ext
     return hip_ext()
+
+
+def packed(n, k, g, bits=4, seed=0):
+    """(dequantized weights, [qweight, scales, qzeros] on the GPU)"""
+    gen = torch.Generator().manual_seed(seed)
+    c, s, z = ref.quant_groupwise(torch.randn(n, k, generator=gen), bits, g,
+                                  False)
+    s = s.to(BF)
+    return (ref.dequant_groupwise(c, s.float(), z, g),
+            [ref.pack_codes(c, bits).to(DEV), s.to(DEV),
+             ref.pack_zeros(z, bits).to(DEV)])
 
 
 # ------------------------------------------------------------- attention
@@ -161,3 +174,28 @@ def test_route_to_as_many_experts_as_lanes(t):
         at = slice(int(want[e]), int(want[e + 1]))
         assert sorted(src[at].tolist()) == \
             (ids == e).any(1).nonzero().flatten().tolist()
+
+
+# ---------------------------------------------------------- grouped calls
+def grouped_case(t, E, n, k, g, seed):
+    torch.manual_seed(seed)
+    w, p = packed(E * n, k, g)
+    ids = torch.randint(0, E, (t,)).sort().values
+    off = torch.zeros(E + 1, dtype=torch.int32)
+    off[1:] = torch.bincount(ids, minlength=E).cumsum(0)
+    x = torch.randn(t, k).to(BF)
+    rows = torch.stack([x[i].double() @ w.view(E, n, k)[ids[i]].double().t()
+                        for i in range(t)])
+    return (x.to(DEV), off.to(DEV), [a.view(E, n, -1) for a in p], rows)
+
+
+@pytest.mark.parametrize("n", [1, 37, 66])
+def test_grouped_linear_of_any_width(n):
+    x, off, p, rows = grouped_case(23, 5, n, 128, 32, n)
+    got = ext().grouped_dq_linear(x, off, *p, 4, 32).double().cpu()
+    assert float((got - rows).abs().max() / rows.abs().max()) < 2 ** -8
+    x, off, p, rows = grouped_case(130, 3, n, 128, 64, n)
+    tiles = torch.tensor([[e, int(a), int(b - a)] for e, (a, b) in enumerate(
+        zip(off[:-1], off[1:]))], dtype=torch.int32, device=DEV)
+    got = ext().moe_linear(x, None, tiles, *p, 4, 64, False, 128)
+    assert float((got.cpu() - rows).abs().max() / rows.abs().max()) < 1e-5
