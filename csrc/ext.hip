@@ -572,6 +572,29 @@ torch::Tensor grouped_dq_linear(torch::Tensor x, torch::Tensor offsets,
       .to(torch::kBFloat16);
 }
 
+// y_f32[dst_tok[s]] += slot_w[s] * (x[s] W_e^T)
+void grouped_dq_linear_scatter(torch::Tensor x, torch::Tensor offsets,
+                               torch::Tensor dst_tok, torch::Tensor slot_w,
+                               torch::Tensor y_f32, torch::Tensor qweight,
+                               torch::Tensor scales, torch::Tensor qzeros,
+                               long bits, long g,
+                               c10::optional<torch::Tensor> active) {
+  check_t(y_f32, torch::kFloat32, "y_f32");
+  check_t(dst_tok, torch::kInt32, "dst_tok");
+  check_t(slot_w, torch::kFloat32, "slot_w");
+  TORCH_CHECK(y_f32.size(1) == qweight.size(1), "y_f32 width mismatch");
+  const long slots = x.size(0);
+  TORCH_CHECK(dst_tok.numel() >= slots && slot_w.numel() >= slots,
+              "a token and a weight for every slot");
+  auto rows = moe_linear(x, c10::nullopt, grouped_tiles(offsets, slots),
+                         qweight, scales, qzeros, bits, g, false, 16);
+  rows.mul_(slot_w.view({-1}).narrow(0, 0, slots).unsqueeze(1));
+  // no expert's: not written
+  auto none = at::arange(slots, offsets.options()).ge(offsets.select(0, -1));
+  rows.masked_fill_(none.unsqueeze(1), 0);
+  y_f32.index_add_(0, dst_tok.view({-1}).narrow(0, 0, slots), rows);
+}
+
 void advance_record(torch::Tensor state, torch::Tensor tok_buf,
                     torch::Tensor sampled, torch::Tensor ring) {
   check_t(state, torch::kInt32, "state");
@@ -765,6 +788,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "fused rope+KV-append+attention decode");
   m.def("grouped_dq_gateup", &grouped_dq_gateup, "MoE grouped gate_up+silu");
   m.def("grouped_dq_linear", &grouped_dq_linear, "MoE grouped linear");
+  m.def("grouped_dq_linear_scatter", &grouped_dq_linear_scatter,
+        "MoE grouped linear, weighted rows added to their tokens'");
   m.def("moe_route", &moe_route, "one-kernel MoE top-k routing");
   m.def("moe_tile", &moe_tile, "rows a tile of the grouped products");
   m.def("moe_plan", &moe_plan, "MoE routing with tiles");

@@ -199,3 +199,20 @@ def test_grouped_linear_of_any_width(n):
         zip(off[:-1], off[1:]))], dtype=torch.int32, device=DEV)
     got = ext().moe_linear(x, None, tiles, *p, 4, 64, False, 128)
     assert float((got.cpu() - rows).abs().max() / rows.abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("n", [37, 64])
+def test_grouped_linear_scatter(n):
+    """Adds a slot's row, weighted, to its token's."""
+    x, off, p, rows = grouped_case(24, 5, n, 128, 64, n)
+    off[-1] = rest = max(int(off[-2]), 20)     # the slots after it: nobody's
+    dst = torch.randperm(24).to(torch.int32) % 12
+    wt = torch.rand(24)
+    y = torch.randn(12, n)
+    want = y.double().index_add(0, dst[:rest].long(),
+                                (rows * wt.double()[:, None])[:rest])
+    y = y.to(DEV)
+    ext().grouped_dq_linear_scatter(x, off, dst.to(DEV), wt.to(DEV), y, *p, 4,
+                                    64, None)
+    assert float((y.double().cpu() - want).abs().max()
+                 / want.abs().max()) < 1e-5
