@@ -76,6 +76,10 @@ class MixtralExpert(nn.Module):
         return self.w2(F.silu_mul_gateup(gu, self.inter))
 
 
+_PACKED = ("qweight", "scales", "qzeros")
+_STACKS = [(name, key) for name in ("w13", "w2") for key in _PACKED]
+
+
 class MixtralMoE(nn.Module):
     """Top-k router + experts.  Forward modes:
       - dense loop (CPU / prefill): per-expert masked forward
@@ -101,41 +105,59 @@ class MixtralMoE(nn.Module):
         weights = torch.softmax(weights, dim=-1)
         return weights, ids
 
-    @torch.no_grad()
+    def _packed(self) -> bool:
+        return all(isinstance(m, QLinear) for e in self.experts
+                   for m in (e.w13, e.w2))
+
     def consolidate(self):
         """Stack the quantized experts' packed buffers for the grouped
-        kernel: qweight [E, n, kw], scales [E, n, G], qzeros [E, n, zw]."""
-        if not isinstance(self.experts[0].w13, QLinear):
+        kernels: qweight [E, n, kw], scales [E, n, G], qzeros [E, n, zw].
+        The experts' buffers become the stacks' parts: the weights are there
+        once, and what is written to an expert is what the kernels read."""
+        if not self._packed():
             return None
         g = {}
-        for name in ("w13", "w2"):
-            mods = [getattr(e, name) for e in self.experts]
-            g[name] = {
-                "qweight": torch.stack([m.qweight for m in mods]),
-                "scales": torch.stack([m.scales for m in mods]),
-                "qzeros": torch.stack([m.qzeros for m in mods]),
-                "bits": mods[0].bits, "g": mods[0].group_size,
-                "n": mods[0].out_features, "k": mods[0].in_features,
-            }
-        self._grouped, self._grouped_of = g, self._packed_state()
+        # (ordinary tensors, which may be written to, in any mode)
+        with torch.inference_mode(False), torch.no_grad():
+            for name in ("w13", "w2"):
+                mods = [getattr(e, name) for e in self.experts]
+                g[name] = {key: torch.stack([getattr(m, key) for m in mods])
+                           for key in _PACKED}
+                g[name].update(bits=mods[0].bits, g=mods[0].group_size,
+                               n=mods[0].out_features, k=mods[0].in_features)
+        device = g["w2"]["qweight"].device
+        if device.type == "cuda":
+            if torch.cuda.is_current_stream_capturing():
+                return g         # the graph's: filled whenever it runs
+            # before another stream reads the stacks
+            torch.cuda.current_stream(device).synchronize()
+        for name, key in _STACKS:
+            for e, part in zip(self.experts, g[name][key]):
+                setattr(getattr(e, name), key, part)
+        self._grouped = g
         return g
 
-    def _packed_state(self) -> list:
-        """Which buffers, and which writes to them, consolidate() copied."""
-        return [(t.data_ptr(), t._version) for e in self.experts
-                for m in (e.w13, e.w2) for t in (m.qweight, m.scales,
-                                                 m.qzeros)]
+    def _stacks(self) -> dict:
+        """The stacks of the experts' buffers as they are now: replaced or
+        moved ones are stacked again."""
+        g = self._grouped
+        if g is None:
+            return self.consolidate()
+        for name, key in _STACKS:
+            t = g[name][key]
+            at, step = t.data_ptr(), t.stride(0) * t.element_size()
+            for i, e in enumerate(self.experts):
+                if getattr(getattr(e, name), key).data_ptr() != at + i * step:
+                    return self.consolidate()
+        return g
 
     def forward(self, x):
         b, s, h = x.shape
         x2 = x.reshape(-1, h)
         t = x2.shape[0]
-        if (x.is_cuda and self._grouped is None
-                and isinstance(self.experts[0].w13, QLinear)):
-            self.consolidate()  # lazy one-time stacking for the grouped kernel
         # up to 64 rows always went through the grouped kernels; more do
         # where the experts are nothing but their packed matrices
-        if x.is_cuda and self._grouped is not None and (
+        if x.is_cuda and self._packed() and (
                 t * self.top_k <= 64 or self._plain()):
             y2 = self._forward_grouped(x2)
         else:
@@ -144,16 +166,15 @@ class MixtralMoE(nn.Module):
         return y2.reshape(b, s, h)
 
     def _plain(self) -> bool:
-        """The experts are what consolidate() copied, with no act-order
-        gather, bias or hook that their own forward would run, and of shapes
-        that the grouped kernels take."""
+        """The experts are their packed matrices, with no act-order gather,
+        bias or hook that their own forward would run, and of shapes that the
+        grouped kernels take."""
         return self.n_experts <= 64 and self.top_k <= 4 and not any(
             m._forward_hooks or m._forward_pre_hooks
             for e in self.experts for m in (e, e.w13, e.w2)) and all(
             type(m) is QLinear and not hasattr(m, "perm") and m.bias is None
             and m.group_size % 32 == 0
-            for e in self.experts for m in (e.w13, e.w2)) and \
-            self._grouped_of == self._packed_state()
+            for e in self.experts for m in (e.w13, e.w2))
 
     def _forward_loop(self, x2, weights, ids):
         y = torch.zeros_like(x2)
@@ -174,7 +195,8 @@ class MixtralMoE(nn.Module):
         first one's epilogue, weighted sum of a token's rows."""
         from ..ops import hip_ext
         ext = hip_ext()
-        a, b = self._grouped["w13"], self._grouped["w2"]
+        g = self._stacks()
+        a, b = g["w13"], g["w2"]
         bm = ext.moe_tile(x2.shape[0] * self.top_k, self.n_experts, a["k"],
                           a["g"], b["k"], b["g"])
         logits16 = self.gate(x2)  # dense bf16 router GEMV

@@ -216,3 +216,88 @@ def test_grouped_linear_scatter(n):
                                     64, None)
     assert float((y.double().cpu() - want).abs().max()
                  / want.abs().max()) < 1e-5
+
+
+# --------------------------------------------------------------- mixtral
+def quantized_moe(hidden, inter, group=64, seed=3, **kw):
+    from lfmq import QuantConfig
+    from lfmq.models.mixtral import MixtralConfig, MixtralMoE
+    from lfmq.models.qlinear import QLinear
+    torch.manual_seed(seed)
+    cfg = MixtralConfig.tiny(hidden_size=hidden, intermediate_size=inter, **kw)
+    moe = MixtralMoE(cfg, BF).to(DEV)
+    qc = QuantConfig(scheme="rtn", bits=4, group_size=group)
+    for e in moe.experts:
+        e.w13, e.w2 = QLinear.from_rtn(e.w13, qc), QLinear.from_rtn(e.w2, qc)
+    return moe
+
+
+def by_loop(moe, x):
+    x2 = x.reshape(-1, x.shape[-1])
+    return moe._forward_loop(x2, *moe.route(x2)).reshape(x.shape)
+
+
+def close(a, b):
+    a, b = a.double(), b.double()
+    return float((a - b).abs().max() / b.abs().max()) < 2 ** -6
+
+
+@pytest.mark.parametrize("t", [2, 70])
+def test_mixtral_made_in_inference_mode(t):
+    with torch.inference_mode():
+        moe = quantized_moe(256, 256)
+        x = torch.randn(1, t, 256, device=DEV).to(BF)
+        assert close(moe(x), by_loop(moe, x))
+    with torch.no_grad():
+        moe.consolidate()
+        assert close(moe(x.clone()), by_loop(moe, x.clone()))
+
+
+@pytest.mark.parametrize("t", [1, 4, 70])
+def test_mixtral_uses_the_weights_that_are_there(t):
+    """Written in place, written past the version counters, replaced (the
+    new ones at the old addresses, too), loaded, moved."""
+    moe, other = quantized_moe(256, 256), quantized_moe(256, 256, seed=9)
+    x = torch.randn(1, t, 256, device=DEV).to(BF)
+    with torch.no_grad():
+        moe(x)
+        before = moe.experts[0].w2.scales
+        for e in moe.experts:
+            e.w2.scales.mul_(2)
+        assert close(moe(x), by_loop(moe, x))
+        for e in moe.experts:
+            e.w2.scales.data.mul_(2)
+        assert close(moe(x), by_loop(moe, x))
+        assert before.data_ptr() == moe.experts[0].w2.scales.data_ptr()
+        for e in moe.experts:
+            new = e.w2.scales.flip(0).cpu()
+            e.w2.scales = None
+            e.w2.scales = new.to(DEV)
+        assert close(moe(x), by_loop(moe, x))
+        moe.load_state_dict(other.state_dict())
+        assert close(moe(x), by_loop(moe, x))
+        assert close(moe(x), other(x))
+        moe = moe.cpu().to(DEV)
+        assert close(moe(x), by_loop(moe, x))
+
+
+def test_mixtral_weights_replaced_and_then_captured():
+    """A graph that has to lay the experts out itself does so whenever it
+    runs, and leaves nothing of its memory to later calls."""
+    moe, other = quantized_moe(256, 256), quantized_moe(256, 256, seed=9)
+    x = torch.randn(1, 2, 256, device=DEV).to(BF)
+    with torch.no_grad():
+        moe(x)
+        moe.load_state_dict(other.state_dict(), assign=True)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = moe(x)
+        want = by_loop(other, x)
+        assert close(moe(x), want)
+        for _ in range(3):
+            got.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert close(got, want)
+            assert close(moe(x), want)

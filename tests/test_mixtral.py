@@ -191,3 +191,41 @@ def _ep_paths_worker(rank, world, port, tmpdir):
 def test_ep_gloo_static_and_dynamic_paths(tmp_path):
     mp.spawn(_ep_paths_worker, args=(2, 29815, str(tmp_path)), nprocs=2,
              join=True)
+
+
+def test_consolidated_experts_are_parts_of_the_stacks(tmp_path):
+    """One copy of the weights: writes meet, what is replaced is stacked
+    again, and models are saved, loaded and copied as before."""
+    import copy
+    cfg = MixtralConfig.tiny()
+    qcfg = lfmq.QuantConfig(scheme="rtn", bits=4, group_size=32)
+    qm = lfmq.quantize(lfmq.build_model(cfg, seed=8), qcfg)
+    want = {k: v.clone() for k, v in qm.state_dict().items()}
+    qm.consolidate_moe()
+    moe = qm.layers[0].moe
+    w = moe.experts[1].w2
+    g = moe._stacks()
+    w.scales.data.mul_(2)
+    assert torch.equal(g["w2"]["scales"][1], w.scales)
+    assert moe._stacks() is g
+    w.scales = w.scales / 2
+    assert moe._stacks() is not g
+    assert torch.equal(moe._stacks()["w2"]["scales"][1], w.scales)
+    p = str(tmp_path / "mx")
+    lfmq.save(qm, p, qcfg)
+    for m in (qm, copy.deepcopy(qm), lfmq.load(p)):
+        got = m.state_dict()
+        assert got.keys() == want.keys()
+        assert all(torch.equal(got[k], want[k]) for k in want)
+
+
+@pytest.mark.parametrize("later", [False, True])
+def test_experts_made_in_inference_mode_consolidate(later):
+    cfg = MixtralConfig.tiny()
+    qcfg = lfmq.QuantConfig(scheme="rtn", bits=4, group_size=32)
+    with torch.inference_mode():
+        qm = lfmq.quantize(lfmq.build_model(cfg, seed=8), qcfg)
+        if not later:
+            qm.consolidate_moe()
+    qm.consolidate_moe()
+    assert qm.layers[0].moe._stacks()["w13"]["qweight"].shape[0] == 4
