@@ -125,20 +125,21 @@ __global__ __launch_bounds__(64) void moe_tiles_kernel(
 // y[t] = sum over a token's choices of w * rows[pos], fp32 -> bf16
 __global__ __launch_bounds__(256) void moe_sum_kernel(
     const float* __restrict__ rows, const i32* __restrict__ pos,
-    const float* __restrict__ w, unsigned short* __restrict__ y, int n,
+    const float* __restrict__ w, unsigned short* __restrict__ y, int t, int n,
     int topk) {
-  const u64 tok = blockIdx.y;
   const int c = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (c >= n) return;
-  f32x4 v = {0.f, 0.f, 0.f, 0.f};
-  for (int j = 0; j < topk; ++j) {
-    const float wj = w[tok * topk + j];
-    const f32x4 r = *(const f32x4*)(rows + (u64)pos[tok * topk + j] * n + c);
+  for (u64 tok = blockIdx.y; tok < (u64)t; tok += gridDim.y) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < topk; ++j) {
+      const float wj = w[tok * topk + j];
+      const f32x4 r = *(const f32x4*)(rows + (u64)pos[tok * topk + j] * n + c);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = fmaf(wj, r[e], v[e]);
+      for (int e = 0; e < 4; ++e) v[e] = fmaf(wj, r[e], v[e]);
+    }
+    *(u64*)(y + tok * n + c) =
+        pack_bf16x2(v[0], v[1]) | (u64)pack_bf16x2(v[2], v[3]) << 32;
   }
-  *(u64*)(y + tok * n + c) =
-      pack_bf16x2(v[0], v[1]) | (u64)pack_bf16x2(v[2], v[3]) << 32;
 }
 
 }  // namespace
@@ -168,8 +169,9 @@ hipError_t lfmq_moe_sum(const void* rows, const void* pos, const void* w,
                         void* y, int t, int n, int topk, hipStream_t stream) {
   if (n % 4) return hipErrorInvalidValue;
   if (t == 0) return hipSuccess;
-  hipLaunchKernelGGL(moe_sum_kernel, dim3((n / 4 + 255) / 256, t), dim3(256),
-                     0, stream, (const float*)rows, (const i32*)pos,
-                     (const float*)w, (unsigned short*)y, n, topk);
+  hipLaunchKernelGGL(moe_sum_kernel,
+                     dim3((n / 4 + 255) / 256, min(t, 65535)), dim3(256), 0,
+                     stream, (const float*)rows, (const i32*)pos,
+                     (const float*)w, (unsigned short*)y, t, n, topk);
   return hipGetLastError();
 }

@@ -76,6 +76,8 @@ class MixtralExpert(nn.Module):
         return self.w2(F.silu_mul_gateup(gu, self.inter))
 
 
+# the grouped kernels address 4 GiB of 16-bit rows
+_ROWS_ELEMENTS = (1 << 31) - 1
 _PACKED = ("qweight", "scales", "qzeros")
 _STACKS = [(name, key) for name in ("w13", "w2") for key in _PACKED]
 
@@ -197,16 +199,25 @@ class MixtralMoE(nn.Module):
         ext = hip_ext()
         g = self._stacks()
         a, b = g["w13"], g["w2"]
-        bm = ext.moe_tile(x2.shape[0] * self.top_k, self.n_experts, a["k"],
-                          a["g"], b["k"], b["g"])
-        logits16 = self.gate(x2)  # dense bf16 router GEMV
-        src, pos, w, tiles = ext.moe_plan(logits16.contiguous(), self.top_k,
-                                          bm)
-        h = ext.moe_linear(x2, src, tiles, a["qweight"], a["scales"],
-                           a["qzeros"], a["bits"], a["g"], True, bm)
-        rows = ext.moe_linear(h, None, tiles, b["qweight"], b["scales"],
-                              b["qzeros"], b["bits"], b["g"], False, bm)
-        return ext.moe_sum(rows, pos, w)
+        logits16 = self.gate(x2).contiguous()  # dense bf16 router GEMV
+
+        def part(x, logits):
+            bm = ext.moe_tile(x.shape[0] * self.top_k, self.n_experts, a["k"],
+                              a["g"], b["k"], b["g"])
+            src, pos, w, tiles = ext.moe_plan(logits, self.top_k, bm)
+            h = ext.moe_linear(x, src, tiles, a["qweight"], a["scales"],
+                               a["qzeros"], a["bits"], a["g"], True, bm)
+            rows = ext.moe_linear(h, None, tiles, b["qweight"], b["scales"],
+                                  b["qzeros"], b["bits"], b["g"], False, bm)
+            return ext.moe_sum(rows, pos, w)
+
+        t = x2.shape[0]
+        most = _ROWS_ELEMENTS // max(a["k"], self.top_k * b["k"])
+        if t <= most:
+            return part(x2, logits16)
+        n = -(-t // most)
+        return torch.cat([part(x, z) for x, z in zip(
+            x2.tensor_split(n), logits16.tensor_split(n))])
 
 
 class MixtralDecoderLayer(nn.Module):

@@ -301,3 +301,22 @@ def test_mixtral_weights_replaced_and_then_captured():
             torch.cuda.synchronize()
             assert close(got, want)
             assert close(moe(x), want)
+
+
+def test_mixtral_prompt_past_four_gibibytes():
+    """75000 tokens' activations in the experts are more than 4 GiB."""
+    moe = quantized_moe(64, 14336)
+    x = torch.randn(1, 75000, 64, device=DEV).to(BF)
+    at = torch.tensor([0, 1, 37499, 37500, 65535, 65536, 74999], device=DEV)
+    with torch.no_grad():
+        y = moe(x)
+        assert y.shape == x.shape
+        assert close(y[:, at], by_loop(moe, x[:, at]))
+
+
+def test_mixtral_prompt_of_more_tokens_than_a_grid_has_rows():
+    moe = quantized_moe(64, 64)
+    x = torch.randn(1, 70000, 64, device=DEV).to(BF)
+    at = torch.tensor([0, 1, 65534, 65535, 65536, 69999], device=DEV)
+    with torch.no_grad():
+        assert close(moe(x)[:, at], by_loop(moe, x[:, at]))
