@@ -20,8 +20,9 @@ class Linear(nn.Linear):
 
 
 def hooked(*modules) -> bool:
-    """Whether anyone watches calls of these modules."""
+    """Whether anyone watches calls of these modules, or has put a forward of
+    an instance's own in their way."""
     m = nn.modules.module
     return bool(m._global_forward_hooks or m._global_forward_pre_hooks
                 or any(p._forward_hooks or p._forward_pre_hooks
-                       for p in modules))
+                       or "forward" in p.__dict__ for p in modules))

@@ -320,3 +320,17 @@ def test_mixtral_prompt_of_more_tokens_than_a_grid_has_rows():
     at = torch.tensor([0, 1, 65534, 65535, 65536, 69999], device=DEV)
     with torch.no_grad():
         assert close(moe(x)[:, at], by_loop(moe, x[:, at]))
+
+
+# ---------------------------------------------------------------- linear
+def test_dense_layer_calls_an_instance_s_own_forward():
+    from lfmq.models.mixers import DenseMLP
+    torch.manual_seed(2)
+    mlp = DenseMLP(256, 128, BF).to(DEV).requires_grad_(False)
+    x = torch.randn(3, 256, device=DEV).to(BF)
+    want = mlp(x)
+    mlp.gate_up_proj.forward = lambda v: torch.zeros(3, 256, device=DEV,
+                                                     dtype=BF)
+    assert float(mlp(x).abs().max()) == 0
+    del mlp.gate_up_proj.forward
+    assert torch.equal(mlp(x), want)
