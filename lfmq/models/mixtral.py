@@ -22,7 +22,7 @@ import torch.nn as nn
 
 from ..ops import functional as F
 from .kvcache import KVCache
-from .linear import Linear
+from .linear import Linear, hooked
 from .llama import LlamaAttention, LlamaConfig, RMSNorm
 from .qlinear import QLinear
 
@@ -168,15 +168,19 @@ class MixtralMoE(nn.Module):
         return y2.reshape(b, s, h)
 
     def _plain(self) -> bool:
-        """The experts are their packed matrices, with no act-order gather,
-        bias or hook that their own forward would run, and of shapes that the
-        grouped kernels take."""
-        return self.n_experts <= 64 and self.top_k <= 4 and not any(
-            m._forward_hooks or m._forward_pre_hooks
-            for e in self.experts for m in (e, e.w13, e.w2)) and all(
-            type(m) is QLinear and not hasattr(m, "perm") and m.bias is None
-            and m.group_size % 32 == 0
-            for e in self.experts for m in (e.w13, e.w2))
+        """Routing and experts are what the grouped kernels do: no act-order
+        gather, bias, hook, class or forward of their own, and shapes that
+        the kernels take."""
+        cls = type(self)
+        return (self.n_experts <= 64 and self.top_k <= 4
+                and cls.route is MixtralMoE.route
+                and cls._forward_loop is MixtralMoE._forward_loop
+                and not {"route", "_forward_loop"} & self.__dict__.keys()
+                and all(type(e) is MixtralExpert
+                        and not hooked(e, e.w13, e.w2) for e in self.experts)
+                and all(type(m) is QLinear and not hasattr(m, "perm")
+                        and m.bias is None and m.group_size % 32 == 0
+                        for e in self.experts for m in (e.w13, e.w2)))
 
     def _forward_loop(self, x2, weights, ids):
         y = torch.zeros_like(x2)

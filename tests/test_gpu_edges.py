@@ -303,6 +303,52 @@ def test_mixtral_weights_replaced_and_then_captured():
             assert close(moe(x), want)
 
 
+def test_mixtral_prompt_calls_what_was_put_in_its_way():
+    """Hooks on all modules, an expert's own forward or class, routing of a
+    subclass."""
+    from lfmq.models import mixtral
+    moe = quantized_moe(256, 256)
+    x = torch.randn(1, 70, 256, device=DEV).to(BF)
+    seen = []
+    with torch.no_grad():
+        want = moe(x)
+        h = torch.nn.modules.module.register_module_forward_hook(
+            lambda m, i, o: seen.append(m))
+        try:
+            got = moe(x)
+        finally:
+            h.remove()
+        assert close(got, want)
+        assert {id(e) for e in moe.experts} <= {id(m) for m in seen}
+
+        e = moe.experts[0]
+        e.forward = lambda v: torch.zeros_like(v)
+        assert close(moe(x), by_loop(moe, x)) and not close(moe(x), want)
+        del e.forward
+        e.w2.forward = lambda v: torch.zeros(v.shape[0], 256, device=DEV,
+                                             dtype=BF)
+        assert close(moe(x), by_loop(moe, x)) and not close(moe(x), want)
+        del e.w2.forward
+        assert close(moe(x), want)
+
+        class Twice(mixtral.MixtralExpert):
+            def forward(self, v):
+                return 2 * super().forward(v)
+
+        e.__class__ = Twice
+        assert close(moe(x), by_loop(moe, x)) and not close(moe(x), want)
+        e.__class__ = mixtral.MixtralExpert
+
+        class Last(mixtral.MixtralMoE):
+            def route(self, x2):
+                w, ids = super().route(x2)
+                return w, torch.zeros_like(ids) + torch.arange(
+                    2, device=DEV)
+
+        moe.__class__ = Last
+        assert close(moe(x), by_loop(moe, x)) and not close(moe(x), want)
+
+
 def test_mixtral_prompt_past_four_gibibytes():
     """75000 tokens' activations in the experts are more than 4 GiB."""
     moe = quantized_moe(64, 14336)
