@@ -822,11 +822,29 @@ T_ silu_mul_fused(T_ gu) {
   return y;
 }
 
+// Whether a call on t is about its values alone: no tangent, batch or gradient
+// of a transform, no class or mode that takes calls over, nothing that records
+// them.  Tensors and threads of that kind carry dispatch keys of their own.
+bool values_only(const T_& t) {
+  const uint64_t usual =
+      c10::full_backend_mask |
+      c10::DispatchKeySet({c10::DispatchKey::Dense,
+                           c10::DispatchKey::AutogradFunctionality,
+                           c10::DispatchKey::ADInplaceOrView})
+          .raw_repr() |
+      c10::autocast_dispatch_keyset.raw_repr();
+  const auto thread = c10::impl::tls_local_dispatch_key_set().included_;
+  return !(t.key_set().raw_repr() & ~usual) &&
+         !(thread.raw_repr() &
+           ~(c10::default_included_set.raw_repr() | c10::full_backend_mask)) &&
+         !t._fw_grad(0).defined();
+}
+
 // x [..., k] w^T, or silu(gate) * up of it; undefined where the kernel does
-// not take it (its sizes, strides, types)
+// not take it (its sizes, strides, types, more than values)
 c10::optional<T_> linear_rows(T_ x, T_ w, bool glu) {
   // (the library also runs on a device that is not the current one)
-  if (!x.is_cuda() || x.device() != w.device() || x.dim() < 1 ||
+  if (!values_only(x) || !values_only(w) || !x.is_cuda() || x.device() != w.device() || x.dim() < 1 ||
       x.get_device() != at::cuda::getCurrentCUDAStream().device_index() ||
       x.scalar_type() != torch::kBFloat16 ||
       w.scalar_type() != torch::kBFloat16 || w.dim() != 2 ||
@@ -906,6 +924,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_down", &moe_down, "down products of the experts");
   m.def("clamped_glu", &clamped_glu, "clamped GLU on fused gate_up");
   m.def("silu_mul_fused", &silu_mul_fused, "silu-mul on fused gate_up");
+  m.def("values_only", &values_only, "whether only t's values matter now");
   m.def("linear_rows", &linear_rows, "16-bit product for a few rows, or None");
   m.def("greedy_sample", &greedy_sample, "row argmax");
   m.def("advance_record", &advance_record, "graph decode-state advance");

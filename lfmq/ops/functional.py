@@ -13,6 +13,8 @@ import os
 from typing import Optional
 
 import torch
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import hip_ext, ref, seq_ext
 
@@ -105,17 +107,26 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     return ref.silu_mul(gate, up)
 
 
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
+
+
 def _plain(x, w) -> bool:
-    """Tensors that only the values of matter of: no gradient, no subclass,
-    no other dtype wanted."""
-    return (type(x) is torch.Tensor and not torch.is_autocast_enabled()
-            and not (torch.is_grad_enabled()
-                     and (x.requires_grad or w.requires_grad)))
+    """Tensors that only the values of matter of, as far as Python knows: no
+    gradient, no subclass, no other dtype wanted, calls that nobody takes over
+    (a default device has no say in these).  The kernel's own check sees
+    transforms, tracing and dispatch modes."""
+    if type(x) is not torch.Tensor or type(w) not in _TENSORS or \
+            torch.compiler.is_compiling() or torch.is_autocast_enabled():
+        return False
+    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
+        return False
+    return not torch._C._len_torch_function_stack() or all(
+        type(m) is DeviceContext for m in _get_current_function_mode_stack())
 
 
 def linear(x, w):
     """x wᵀ.  A few rows of 16-bit values: the kernel for decode steps."""
-    if x.is_cuda and _plain(x, w):
+    if _plain(x, w) and x.is_cuda:
         y = seq_ext().linear_rows(x, w, False)
         if y is not None:
             return y
@@ -125,7 +136,7 @@ def linear(x, w):
 def linear_silu_mul(x, w):
     """silu_mul_gateup(x wᵀ) in one launch, or None where the kernel for
     decode steps does not take it."""
-    if x.is_cuda and _plain(x, w):
+    if _plain(x, w) and x.is_cuda:
         return seq_ext().linear_rows(x, w, True)
     return None
 

@@ -369,6 +369,59 @@ def test_mixtral_prompt_of_more_tokens_than_a_grid_has_rows():
 
 
 # ---------------------------------------------------------------- linear
+def test_linear_of_more_than_values():
+    """Forward-mode tangents, vmap, tracing, a weight of another class, modes
+    that watch calls: what the library's product gives."""
+    import torch.autograd.forward_ad as fwAD
+    from lfmq.models.linear import Linear
+    torch.manual_seed(2)
+    m = Linear(256, 64, BF).to(DEV).requires_grad_(False)
+    x, dx = (torch.randn(3, 256, device=DEV).to(BF) for _ in range(2))
+    want = torch.nn.functional.linear
+    with fwAD.dual_level():
+        t = fwAD.unpack_dual(m(fwAD.make_dual(x, dx))).tangent
+        assert torch.equal(t, want(dx, m.weight))
+        m2 = Linear(256, 64, BF).to(DEV).requires_grad_(False)
+        del m2.weight
+        m2.weight = fwAD.make_dual(m.weight.detach(), m.weight.detach())
+        t = fwAD.unpack_dual(m2(x)).tangent
+        assert torch.equal(t, want(x, m.weight))
+    traced = torch.jit.trace(m, (x,), check_trace=False)
+    assert torch.equal(traced(dx), want(dx, m.weight))
+
+    class Scaled(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            r = super().__torch_function__(func, types, args, kwargs or {})
+            return r * 2 if func is want else r
+
+    m.weight = torch.nn.Parameter(m.weight.detach().as_subclass(Scaled),
+                                  requires_grad=False)
+    w = m.weight.detach().as_subclass(torch.Tensor)
+    assert torch.equal(m(x).as_subclass(torch.Tensor), 2 * want(x, w))
+    m.weight = torch.nn.Parameter(w, requires_grad=False)
+
+    from torch.utils.flop_counter import FlopCounterMode
+    with FlopCounterMode(display=False) as count:
+        m(x)
+    assert count.get_total_flops() == 2 * 3 * 256 * 64
+
+
+def test_linear_under_transforms():
+    from lfmq.models.linear import Linear
+    torch.manual_seed(2)
+    m = Linear(256, 64, BF).to(DEV).requires_grad_(False)
+    x = torch.randn(3, 256, device=DEV).to(BF)
+    want = torch.nn.functional.linear(x, m.weight).float()
+    got = torch.func.vmap(m)(x)
+    assert float((got.float() - want).abs().max()) < 2 ** -6
+    _, t = torch.func.jvp(m, (x,), (x,))
+    assert float((t.float() - want).abs().max()) < 2 ** -6
+    with torch.device(DEV):                    # still the kernel
+        from lfmq.ops import seq_ext
+        assert torch.equal(m(x), seq_ext().linear_rows(x, m.weight, False))
+
+
 def test_dense_layer_calls_an_instance_s_own_forward():
     from lfmq.models.mixers import DenseMLP
     torch.manual_seed(2)
