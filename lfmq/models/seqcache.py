@@ -46,8 +46,7 @@ class StepBatch:
             raise ValueError("a slot may appear once in a step")
         self.device = device
         self._lasting = lasting
-        self._stream = None if lasting or torch.device(device).type != "cuda" \
-            else torch.cuda.current_stream(device)
+        self._queued: List[tuple] = []          # uploads and their streams
         self.slot_ids, self.counts = list(slots), list(counts)
         self.len0 = list(len0)
         self.b, self.n = len(slots), sum(counts)
@@ -68,15 +67,22 @@ class StepBatch:
     def _dev(self, ints) -> torch.Tensor:
         if self._lasting:
             return torch.tensor(ints, dtype=torch.int32).to(self.device)
-        return upload(ints, torch.int32, self.device)
+        t = upload(ints, torch.int32, self.device)
+        if t.is_cuda:
+            self._queued.append((t, torch.cuda.current_stream(t.device)))
+        return t
 
     def arrive(self) -> None:
-        """The numbers' copies are queued on the stream that the batch was
-        made on; a step on another stream waits for them."""
-        if self._stream is not None:
-            now = torch.cuda.current_stream(self.device)
-            if now != self._stream:
-                now.wait_stream(self._stream)
+        """The numbers' copies are queued on the streams that asked for them.
+        A step on another stream waits for them, and their memory is not given
+        out again before that step has read it."""
+        if not self._queued:
+            return
+        now = torch.cuda.current_stream(self.device)
+        for t, made_on in self._queued:
+            if made_on != now:
+                now.wait_stream(made_on)
+                t.record_stream(now)
 
     def view(self, cache):
         return self.seq, self.cu, self.slots, cache.lens

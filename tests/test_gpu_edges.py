@@ -433,3 +433,61 @@ def test_dense_layer_calls_an_instance_s_own_forward():
     assert float(mlp(x).abs().max()) == 0
     del mlp.gate_up_proj.forward
     assert torch.equal(mlp(x), want)
+
+
+# -------------------------------------------------------------- seqcache
+def busy(n=20):
+    """Work that is queued for a while."""
+    x = torch.randn(4096, 4096, device=DEV)
+    for _ in range(n):
+        x = (x @ x).clamp_(-1, 1)
+
+
+def tiny_packed():
+    import lfmq
+    from lfmq.models.rapivik import RapivikConfig
+    return lfmq.build_model(RapivikConfig.tiny(n_layers=2), seed=1).to(DEV)
+
+
+@torch.no_grad()
+def test_batch_is_kept_for_a_step_on_another_stream():
+    """A batch is dropped while the step that reads its numbers is queued on
+    another stream; batches of the same sizes are made meanwhile."""
+    m = tiny_packed()
+    tok = torch.randint(0, 512, (80,), device=DEV)
+
+    def step(cache, slots, counts):
+        return m.forward_tokens(tok, cache.batch(slots, counts), cache)
+
+    want = step(m.make_cache(4, 96), [1, 3], [70, 10])
+    cache, side = m.make_cache(4, 96), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        busy(40)
+    batch = cache.batch([1, 3], [70, 10])
+    with torch.cuda.stream(side):
+        got = m.forward_tokens(tok, batch, cache)
+    del batch
+    other = m.make_cache(4, 96)
+    for _ in range(8):
+        other.batch([2, 0], [10, 70])
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+
+
+@torch.no_grad()
+def test_step_waits_for_numbers_that_another_stream_asked_for():
+    """The layouts that a batch makes when they are asked for are queued on
+    that step's stream."""
+    m = tiny_packed()
+    tok = torch.randint(0, 512, (80,), device=DEV)
+    cache, side = m.make_cache(2, 96), torch.cuda.Stream()
+    want = m.forward_tokens(tok, cache.batch([0, 1], [70, 10]), cache)
+    cache, again = m.make_cache(2, 96), m.make_cache(2, 96)
+    batch = cache.batch([0, 1], [70, 10])
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        busy()
+        m.forward_tokens(tok, batch, cache)
+    assert torch.equal(m.forward_tokens(tok, batch, again), want)
+    assert {s for _, s in batch._queued} == {torch.cuda.current_stream(), side}
