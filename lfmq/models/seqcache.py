@@ -75,8 +75,10 @@ class StepBatch:
     def arrive(self) -> None:
         """The numbers' copies are queued on the streams that asked for them.
         A step on another stream waits for them, and their memory is not given
-        out again before that step has read it."""
-        if not self._queued:
+        out again before that step has read it.  A capture knows no streams
+        outside of it: torch.cuda.graph() waits for all of them when it begins,
+        and who replays a graph keeps its batch."""
+        if not self._queued or torch.cuda.is_current_stream_capturing():
             return
         now = torch.cuda.current_stream(self.device)
         for t, made_on in self._queued:

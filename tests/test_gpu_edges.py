@@ -491,3 +491,27 @@ def test_step_waits_for_numbers_that_another_stream_asked_for():
         m.forward_tokens(tok, batch, cache)
     assert torch.equal(m.forward_tokens(tok, batch, again), want)
     assert {s for _, s in batch._queued} == {torch.cuda.current_stream(), side}
+
+
+@torch.no_grad()
+def test_step_of_a_batch_made_before_its_capture():
+    m = tiny_packed()
+    tok = torch.randint(0, 512, (80,), device=DEV)
+    cache = m.make_cache(2, 96)
+    fresh = cache.snapshot()
+    batch = cache.batch([0, 1], [70, 10])
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        want = m.forward_tokens(tok, batch, cache)
+    torch.cuda.synchronize()
+    cache.restore(fresh)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = m.forward_tokens(tok, batch, cache)
+    for _ in range(3):
+        cache.restore(fresh)
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
