@@ -13,7 +13,8 @@ import torch
 
 class KVCache:
     def __init__(self, n_layers: int, batch: int, n_kv_heads: int,
-                 max_seq: int, head_dim: int, device, dtype=torch.bfloat16):
+                 max_seq: int, head_dim: int, device, dtype=torch.bfloat16,
+                 n_heads: int = 0):
         self.max_seq = max_seq
         self.seq_len = 0
         self.k_all = torch.zeros(n_layers, batch, n_kv_heads, max_seq,
@@ -22,6 +23,11 @@ class KVCache:
                                  head_dim, device=device, dtype=dtype)
         self.k = [self.k_all[i] for i in range(n_layers)]
         self.v = [self.v_all[i] for i in range(n_layers)]
+        # arrivals of the key ranges of a query head (decode attention), back
+        # at zero after every layer.  The cache's, as its rows are: steps that
+        # overlap, or that two graphs hold, run on caches of their own.
+        self.tickets = torch.zeros(batch * (n_heads or n_kv_heads),
+                                   dtype=torch.int32, device=device)
 
     def reset(self) -> None:
         self.seq_len = 0

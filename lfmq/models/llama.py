@@ -140,14 +140,16 @@ class LlamaAttention(nn.Module):
         o = o.transpose(1, 2).reshape(b, s, hq * d)
         return self.o_proj(o)
 
-    def forward_decode_graph(self, x, cache_k, cache_v, state, max_seq):
+    def forward_decode_graph(self, x, cache_k, cache_v, state, max_seq,
+                             tickets=None):
         """hipGraph-capturable decode step (s == 1, GPU only)."""
         b, s, _ = x.shape
-        o = self.decode_qkv_attn(x, cache_k, cache_v, state, max_seq)
+        o = self.decode_qkv_attn(x, cache_k, cache_v, state, max_seq,
+                                 tickets=tickets)
         return self.o_proj(o)
 
     def decode_qkv_attn(self, x, cache_k, cache_v, state, max_seq,
-                        rms_eps: float = -1.0):
+                        rms_eps: float = -1.0, tickets=None):
         """qkv GEMV -> ONE fused rope+KV-append+attention launch; returns
         [b, s, hq*d] (pre o_proj).  rms_eps >= 0 additionally fuses the
         input RMSNorm into the qkv GEMV (norm weight pre-folded)."""
@@ -158,7 +160,7 @@ class LlamaAttention(nn.Module):
             qkv = self.qkv_proj(x)
         o = F.attn_decode_fused(qkv.view(b, -1), cache_k, cache_v, state,
                                 max_seq, self.scale, self.n_heads,
-                                self.cfg.rope_theta)
+                                self.cfg.rope_theta, tickets)
         return o.view(b, s, self.n_heads * self.head_dim)
 
     def _chunk_attn(self, q, cache_k, cache_v, pos0, seq_len_after):
@@ -228,7 +230,7 @@ class LlamaDecoderLayer(nn.Module):
         return h, residual
 
     def forward_decode_step(self, x, cache_k, cache_v, state, max_seq,
-                            residual=None):
+                            residual=None, tickets=None):
         if residual is None:
             residual = x
             h = self.input_layernorm(x)
@@ -237,21 +239,22 @@ class LlamaDecoderLayer(nn.Module):
                                              self.input_layernorm.weight,
                                              self.input_layernorm.eps)
         h = self.self_attn.forward_decode_graph(h, cache_k, cache_v, state,
-                                                max_seq)
+                                                max_seq, tickets)
         h, residual = F.rmsnorm_residual(h, residual,
                                          self.post_attention_layernorm.weight,
                                          self.post_attention_layernorm.eps)
         h = self.mlp(h)
         return h, residual
 
-    def forward_decode_fused(self, x, cache_k, cache_v, state, max_seq):
+    def forward_decode_fused(self, x, cache_k, cache_v, state, max_seq,
+                             tickets=None):
         """Folded-norm decode step: both RMSNorms ride inside the GEMVs
         and both residual adds ride in the o/down epilogues — 6 kernels
         per layer, no separate norm/add launches.  Requires
         _in_norm_folded and _post_norm_folded (lfmq.quant.fold)."""
         eps = self.input_layernorm.eps
         o = self.self_attn.decode_qkv_attn(x, cache_k, cache_v, state,
-                                           max_seq, rms_eps=eps)
+                                           max_seq, eps, tickets)
         x = self.self_attn.o_proj.forward_resid(o, x)
         mlp, gp = self.mlp, self.mlp.gate_up_proj
         h, eps = x, self.post_attention_layernorm.eps
@@ -291,10 +294,10 @@ class LlamaForCausalLM(nn.Module):
                    device=None) -> KVCache:
         dev = device or next(self.parameters()).device
         # TP: layers may hold a KV-head shard; size the cache from the module
-        hkv = self.layers[0].self_attn.n_kv_heads
-        return KVCache(self.cfg.n_layers, batch, hkv,
+        att = self.layers[0].self_attn
+        return KVCache(self.cfg.n_layers, batch, att.n_kv_heads,
                        max_seq or self.cfg.max_seq, self.cfg.head_dim, dev,
-                       dtype=self.dtype)
+                       dtype=self.dtype, n_heads=att.n_heads)
 
     def forward(self, input_ids: torch.Tensor, cache: KVCache,
                 positions: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -382,18 +385,19 @@ class LlamaForCausalLM(nn.Module):
         x = self.embed_tokens(input_ids)
         if getattr(self, "_fused_decode", None) is None:
             self._fused_decode = self._decode_fused_ready()
-        b = input_ids.shape[0]
+        b, tickets = input_ids.shape[0], getattr(cache, "tickets", None)
         if self._fused_decode and (b <= 4 or (b <= FEW_ROWS
                                               and self._rows_fused())):
             for i, layer in enumerate(self.layers):
                 x = layer.forward_decode_fused(x, cache.k[i], cache.v[i],
-                                               state, max_seq)
+                                               state, max_seq, tickets)
             x = self.norm(x)
         else:
             residual = None
             for i, layer in enumerate(self.layers):
                 x, residual = layer.forward_decode_step(
-                    x, cache.k[i], cache.v[i], state, max_seq, residual)
+                    x, cache.k[i], cache.v[i], state, max_seq, residual,
+                    tickets)
             x = self.norm(x, residual=residual)
         return self.lm_head(x)
 

@@ -252,7 +252,7 @@ class MixtralDecoderLayer(nn.Module):
         return h, residual
 
     def forward_decode_step(self, x, cache_k, cache_v, state, max_seq,
-                            residual=None):
+                            residual=None, tickets=None):
         if residual is None:
             residual = x
             h = self.input_layernorm(x)
@@ -261,7 +261,7 @@ class MixtralDecoderLayer(nn.Module):
                                              self.input_layernorm.weight,
                                              self.input_layernorm.eps)
         h = self.self_attn.forward_decode_graph(h, cache_k, cache_v, state,
-                                                max_seq)
+                                                max_seq, tickets)
         h, residual = F.rmsnorm_residual(h, residual,
                                          self.post_attention_layernorm.weight,
                                          self.post_attention_layernorm.eps)
@@ -296,10 +296,10 @@ class MixtralForCausalLM(nn.Module):
 
     def make_cache(self, batch: int, max_seq: Optional[int] = None, device=None):
         dev = device or next(self.parameters()).device
-        hkv = self.layers[0].self_attn.n_kv_heads
-        return KVCache(self.cfg.n_layers, batch, hkv,
+        att = self.layers[0].self_attn
+        return KVCache(self.cfg.n_layers, batch, att.n_kv_heads,
                        max_seq or self.cfg.max_seq, self.cfg.head_dim, dev,
-                       dtype=self.dtype)
+                       dtype=self.dtype, n_heads=att.n_heads)
 
     def forward(self, input_ids, cache: KVCache, positions=None):
         b, s = input_ids.shape
@@ -320,10 +320,10 @@ class MixtralForCausalLM(nn.Module):
 
     def forward_decode_step(self, input_ids, cache, state, max_seq):
         x = self.embed_tokens(input_ids)
-        residual = None
+        residual, tickets = None, getattr(cache, "tickets", None)
         for i, layer in enumerate(self.layers):
             x, residual = layer.forward_decode_step(
-                x, cache.k[i], cache.v[i], state, max_seq, residual)
+                x, cache.k[i], cache.v[i], state, max_seq, residual, tickets)
         x = self.norm(x, residual=residual)
         return self.lm_head(x)
 

@@ -47,19 +47,6 @@ def rmsnorm_residual(x: torch.Tensor, residual: torch.Tensor,
 
 
 _INV_FREQ_CACHE: dict = {}
-# zero-initialized arrival tickets for the in-launch attention combine:
-# the winning chunk resets its entry, so one buffer per (n, device) stays
-# valid across steps and graph replays
-_TICKETS_CACHE: dict = {}
-
-
-def _tickets(n: int, device) -> "torch.Tensor":
-    key = (n, str(device))
-    t = _TICKETS_CACHE.get(key)
-    if t is None:
-        t = torch.zeros(n, dtype=torch.int32, device=device)
-        _TICKETS_CACHE[key] = t
-    return t
 
 
 def _inv_freq(d: int, theta: float, device) -> torch.Tensor:
@@ -244,20 +231,24 @@ def attn_decode_graph(q, k_cache, v_cache, state, max_t: int, scale: float):
 
 
 def attn_decode_fused(qkv, k_cache, v_cache, state_or_T, max_t: int,
-                      scale: float, hq: int, theta: float = 500000.0):
+                      scale: float, hq: int, theta: float = 500000.0,
+                      tickets: Optional[torch.Tensor] = None):
     """One launch: rope(q,k) off the raw qkv buffer, KV-cache append,
     chunked decode attention.  state_or_T: device state tensor (graph
-    mode, T = state[1]) or a host int T."""
+    mode, T = state[1]) or a host int T.  tickets: zeros that no other step
+    uses at the same time (KVCache.tickets), at least one for every query head
+    of the batch; without them a second launch merges the chunks."""
     d = k_cache.shape[-1]
     inv = _inv_freq(d, theta, qkv.device)
-    tk = _tickets(k_cache.shape[0] * hq, qkv.device)
+    if tickets is not None and tickets.numel() < k_cache.shape[0] * hq:
+        tickets = None
     if torch.is_tensor(state_or_T):
         return hip_ext().attn_decode_fused(qkv.contiguous(), k_cache, v_cache,
                                            max_t, scale, inv, hq,
-                                           state_or_T[1:2], tk)
+                                           state_or_T[1:2], tickets)
     return hip_ext().attn_decode_fused(qkv.contiguous(), k_cache, v_cache,
                                        int(state_or_T), scale, inv, hq, None,
-                                       tk)
+                                       tickets)
 
 
 def dq_gemv_gateup(x: torch.Tensor, qweight: torch.Tensor,

@@ -143,3 +143,14 @@ def test_per_channel_quant_e2e(tmp_path):
     ids = torch.arange(8).remainder(cfg.vocab_size).reshape(1, 8)
     assert torch.equal(qm(ids, qm.make_cache(1, 16)),
                        back(ids, back.make_cache(1, 16)))
+
+
+def test_caches_own_their_arrival_counters():
+    """Steps on two caches may overlap: nothing of theirs is shared, and there
+    is a counter for every query head."""
+    from lfmq.models.mixtral import MixtralConfig
+    for cfg in (LlamaConfig.tiny(), MixtralConfig.tiny()):
+        m = lfmq.build_model(cfg, seed=0)
+        a, b = m.make_cache(3, 16), m.make_cache(3, 16)
+        assert a.tickets.data_ptr() != b.tickets.data_ptr()
+        assert a.tickets.tolist() == [0] * 3 * cfg.n_heads

@@ -102,6 +102,49 @@ def test_decode_attention_of_no_sequences():
             torch.ones(64, device=DEV), 32, None, None)
 
 
+@torch.no_grad()
+def test_decode_steps_that_overlap_on_two_streams():
+    """Two captured steps of one model and one shape, each with a cache of
+    its own and many key ranges a head, replayed at the same time."""
+    import lfmq
+    from lfmq.models.llama import LlamaConfig
+    T = 2500
+    cfg = LlamaConfig(vocab_size=512, hidden_size=512, intermediate_size=512,
+                      n_layers=4, n_heads=8, n_kv_heads=2, head_dim=64)
+    m = lfmq.quantize(lfmq.build_model(cfg, seed=0), lfmq.QuantConfig(
+        scheme="rtn", bits=4, group_size=64)).to(DEV)
+    runs = []
+    for seed in range(2):
+        torch.manual_seed(seed)
+        cache = m.make_cache(1, max_seq=T + 8)
+        for t in (cache.k_all, cache.v_all):
+            t.normal_()
+        tok = torch.randint(0, 512, (1, 1), device=DEV)
+        state = torch.tensor([T - 1, T, 0], dtype=torch.int32, device=DEV)
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            want = m.forward_decode_step(tok, cache, state, T + 8).clone()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = m.forward_decode_step(tok, cache, state, T + 8)
+        runs.append((graph, side, got, want, (cache, tok, state)))
+    a, b = (r[4][0].tickets for r in runs)
+    assert a.data_ptr() != b.data_ptr() and not a.any() and not b.any()
+    for _ in range(30):
+        for graph, side, *_ in runs:
+            with torch.cuda.stream(side):
+                for _ in range(4):
+                    graph.replay()
+        torch.cuda.synchronize()
+        for *_, got, want, _ in runs:
+            assert torch.equal(got, want)
+            got.zero_()
+        torch.cuda.synchronize()
+    assert not a.any() and not b.any()
+
+
 # ------------------------------------------------------- packed products
 def test_packed_product_of_nothing():
     """No rows: no rows, however large the matrix; no columns: refused, as a
