@@ -150,7 +150,7 @@ def test_caches_own_their_arrival_counters():
     is a counter for every query head."""
     from lfmq.models.mixtral import MixtralConfig
     for cfg in (LlamaConfig.tiny(), MixtralConfig.tiny()):
-        m = lfmq.build_model(cfg, seed=0)
+        m = build_model(cfg, seed=0)
         a, b = m.make_cache(3, 16), m.make_cache(3, 16)
         assert a.tickets.data_ptr() != b.tickets.data_ptr()
         assert a.tickets.tolist() == [0] * 3 * cfg.n_heads
