@@ -34,6 +34,7 @@
 namespace {
 
 constexpr int WAVES_PER_WG = 4;
+constexpr int MAX_GROUPS = 128;    // a lane holds two groups' scales
 constexpr u32 ONE2_BF16 = 0x3F803F80u;  // bf16x2 (1.0, 1.0)
 
 template <int M, int BITS, int COLS, bool GATEUP, int KI, bool RMS,
@@ -548,7 +549,8 @@ hipError_t lfmq_dq_gemv(const void* qweight, const void* scales,
                         const void* bias, const void* resid, int m, int n,
                         int k, int g, int bits, float rms_eps, int cols_hint,
                         hipStream_t stream) {
-  if (m > 16 || k % 8 != 0 || g % 32 != 0 || g > k) return hipErrorInvalidValue;
+  if (m > 16 || k % 8 != 0 || g % 32 != 0 || g > k || k > MAX_GROUPS * (long)g)
+    return hipErrorInvalidValue;
   const bool rms = rms_eps >= 0.f;
   if (rms && m > 4) return hipErrorInvalidValue;
   if (bits == 4) {
@@ -571,7 +573,8 @@ hipError_t lfmq_dq_gemv_gateup(const void* qweight, const void* scales,
                                int m, int n, int k, int g, int bits,
                                float rms_eps, int cols_hint,
                                hipStream_t stream) {
-  if (m > 4 || k % 8 != 0 || g % 32 != 0 || g > k || n % 2)
+  if (m > 4 || k % 8 != 0 || g % 32 != 0 || g > k || n % 2 ||
+      k > MAX_GROUPS * (long)g)
     return hipErrorInvalidValue;
   const bool rms = rms_eps >= 0.f;
   if (bits == 4) {

@@ -123,6 +123,10 @@ int rows_from(long bits, long n, long k, long g) {
   return bits == 8 || n * k >= 32l << 20 ? 2 : 3;
 }
 
+torch::Tensor rmsnorm(torch::Tensor x, torch::Tensor w, double eps,
+                      c10::optional<torch::Tensor> residual);
+torch::Tensor silu_mul_fused(torch::Tensor gate_up);
+
 torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
                         torch::Tensor scales, torch::Tensor qzeros, long bits,
                         long g, c10::optional<torch::Tensor> bias,
@@ -136,6 +140,13 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
   const int m = (int)x.size(0), k = (int)x.size(1);
   const int n = (int)qweight.size(0);
   TORCH_CHECK(qweight.size(1) == (long)k * bits / 32, "qweight/k mismatch");
+  // more groups than either kernel with the norm in it holds scales of (381
+  // and 128): the norm apart
+  if (rms_eps >= 0 && m <= 4 && k > 128 * g &&
+      !lfmq_dq_rows_ok(m, n, k, (int)g, true)) {
+    x = rmsnorm(x, torch::ones({k}, x.options()), rms_eps, c10::nullopt);
+    rms_eps = -1;
+  }
   if ((uintptr_t)x.data_ptr() % 16) x = x.clone();  // 16-byte loads to LDS
   const void* bptr = nullptr;
   if (bias.has_value()) {
@@ -387,6 +398,9 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
                            (int)bits, 1, (float)rms_eps, true, stream()));
     return y;
   }
+  if (k > 128 * g)                         // the GEMV's limit: the gate apart
+    return silu_mul_fused(dq_linear(x, qweight, scales, qzeros, bits, g,
+                                    c10::nullopt, c10::nullopt, rms_eps, 0));
   CHECK_HIP(lfmq_dq_gemv_gateup(qweight.data_ptr(), scales.data_ptr(),
                                 qzeros.data_ptr(), x.data_ptr(), y.data_ptr(),
                                 m, n, k, (int)g, (int)bits, (float)rms_eps,

@@ -165,6 +165,36 @@ def test_packed_product_of_nothing():
                             g, None, None, -1.0, 0)
 
 
+@pytest.mark.parametrize("m", [1, 2, 4])
+@pytest.mark.parametrize("k,g", [(12416, 32), (28672, 64)])
+def test_norm_and_gate_of_more_groups_than_kernels_hold(m, k, g):
+    """388 and 448 groups a row.  The norm's result is rounded to 8 bits (each
+    of k terms by 2^-9: of their sum's size, 2^-9 in the root mean square),
+    then sums, gate and result."""
+    torch.manual_seed(m)
+    n = 64
+    codes = torch.randint(0, 16, (n, k), dtype=torch.int32)
+    zeros = torch.randint(0, 16, (n, k // g), dtype=torch.int32)
+    s16 = (torch.rand(n, k // g) * 0.02 + 0.01).to(BF)
+    p = (ref.pack_codes(codes, 4).to(DEV), s16.to(DEV),
+         ref.pack_zeros(zeros, 4).to(DEV), 4, g)
+    w = ref.dequant_groupwise(codes, s16.float(), zeros, g).double()
+    x = torch.randn(m, k).to(BF)
+    xn = x.double() * torch.rsqrt(x.double().square().mean(1, True) + 1e-5)
+    for v, eps in ((x.double(), -1.0), (xn, 1e-5)):
+        want = v @ w.t()
+        a, u = want.chunk(2, 1)
+        for y, z in ((ext().dq_linear(x.to(DEV), *p, None, None, eps, 0),
+                      want),
+                     (ext().dq_gemv_gateup(x.to(DEV), *p, eps, 0),
+                      torch.nn.functional.silu(a) * u)):
+            err = (y.double().cpu() - z).square().mean().sqrt()
+            assert float(err / z.square().mean().sqrt()) < 2 ** -7
+    for hint in (1, 2, 4, 5):                  # the GEMV by name: refused
+        with pytest.raises(RuntimeError):
+            ext().dq_linear(x.to(DEV), *p, None, None, -1.0, hint)
+
+
 # ------------------------------------------------------------------ gptq
 @pytest.mark.parametrize("tiny", [1e-40, 3e-38, 2e-36, 1e-33])
 def test_gptq_block_of_numbers_below_the_normal_range(tiny):
