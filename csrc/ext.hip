@@ -137,6 +137,7 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
   check_t(scales, torch::kBFloat16, "scales");
   check_t(qzeros, torch::kInt32, "qzeros");
   TORCH_CHECK(x.dim() == 2, "x must be [m, k]");
+  TORCH_CHECK(g > 0, "groups have at least one column");
   const int m = (int)x.size(0), k = (int)x.size(1);
   const int n = (int)qweight.size(0);
   TORCH_CHECK(qweight.size(1) == (long)k * bits / 32, "qweight/k mismatch");
@@ -365,6 +366,7 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
                              long cols_hint) {
   check_t(x, torch::kBFloat16, "x");
   check_t(qweight, torch::kInt32, "qweight");
+  TORCH_CHECK(g > 0, "groups have at least one column");
   const int m = (int)x.size(0), k = (int)x.size(1);
   const int n = (int)qweight.size(0);
   TORCH_CHECK(qweight.size(1) == (long)k * bits / 32, "qweight/k mismatch");
@@ -479,6 +481,7 @@ std::vector<torch::Tensor> moe_route(torch::Tensor logits, long topk) {
 // rows an expert, 418 / 397 at 16, 669 / 403 at 32.
 long moe_tile(long slots, long E, long k_in, long g_in, long k_out,
               long g_out) {
+  TORCH_CHECK(g_in > 0 && g_out > 0, "groups have at least one column");
   return slots > 14 * E && lfmq_dq_tile_ok((int)k_in, (int)g_in) &&
                  lfmq_dq_tile_ok((int)k_out, (int)g_out)
              ? 128
@@ -489,6 +492,7 @@ long moe_tile(long slots, long E, long k_in, long g_in, long k_out,
 // token's choice [t, topk], tiles of bm rows)
 std::vector<torch::Tensor> moe_plan(torch::Tensor logits, long topk, long bm) {
   check_t(logits, torch::kBFloat16, "logits");
+  TORCH_CHECK(bm > 0, "tiles have at least one row");
   const int t = (int)logits.size(0), E = (int)logits.size(1);
   const long slots = (long)t * topk;
   const int n_tiles = (int)(slots / bm + std::min((long)E, slots));
@@ -517,6 +521,7 @@ torch::Tensor moe_linear(torch::Tensor x, c10::optional<torch::Tensor> src,
   check_t(qzeros, torch::kInt32, "qzeros");
   const int n = (int)qweight.size(1), k = (int)x.size(1);
   TORCH_CHECK(qweight.size(2) == (long)k * bits / 32, "qweight/k mismatch");
+  TORCH_CHECK(g > 0, "groups have at least one column");
   TORCH_CHECK(x.numel() * 2 < 1l << 32, "x of 4 GiB or more");
   if ((uintptr_t)x.data_ptr() % 16) x = x.clone();  // 16-byte loads to LDS
   const void* sptr = nullptr;

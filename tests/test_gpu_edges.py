@@ -195,6 +195,23 @@ def test_norm_and_gate_of_more_groups_than_kernels_hold(m, k, g):
             ext().dq_linear(x.to(DEV), *p, None, None, -1.0, hint)
 
 
+def test_packed_product_of_no_group():
+    """Groups of nothing are refused by name (a division by their size would
+    end the process)."""
+    x = torch.zeros(2, 128, dtype=BF, device=DEV)
+    p = [t[None] for t in packed(8, 128, 64)[1]]
+    tiles = torch.zeros(1, 3, dtype=torch.int32, device=DEV)
+    for call in (
+            lambda: ext().dq_linear(x, *(t[0] for t in p), 4, 0, None, None,
+                                    -1.0, 0),
+            lambda: ext().dq_gemv_gateup(x, *(t[0] for t in p), 4, 0, -1.0, 0),
+            lambda: ext().moe_linear(x, None, tiles, *p, 4, 0, False, 16),
+            lambda: ext().moe_tile(64, 2, 128, 0, 128, 0),
+            lambda: ext().moe_plan(x[:, :8].contiguous(), 2, 0)):
+        with pytest.raises(RuntimeError, match="at least one"):
+            call()
+
+
 # ------------------------------------------------------------------ gptq
 @pytest.mark.parametrize("tiny", [1e-40, 3e-38, 2e-36, 1e-33])
 def test_gptq_block_of_numbers_below_the_normal_range(tiny):
