@@ -123,6 +123,11 @@ int rows_from(long bits, long n, long k, long g) {
   return bits == 8 || n * k >= 32l << 20 ? 2 : 3;
 }
 
+// the product through LDS addresses a matrix below 4 GiB, the others any
+bool tile_addresses(long n, long k, long bits) {
+  return n * k / 8 * bits < 1l << 32;
+}
+
 torch::Tensor rmsnorm(torch::Tensor x, torch::Tensor w, double eps,
                       c10::optional<torch::Tensor> residual);
 torch::Tensor silu_mul_fused(torch::Tensor gate_up);
@@ -171,7 +176,8 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
   // 12.9 / 9.8 at 4, and norm and product apart: 13.6 / 10.0 at 8, 23.8 /
   // 20.2 at 48.
   const bool rms = rms_eps >= 0;
-  const bool large = !rms && k >= 4096 && (long)n * k >= 24l << 20 &&
+  const bool tile = tile_addresses(n, k, bits);
+  const bool large = tile && !rms && k >= 4096 && (long)n * k >= 24l << 20 &&
                      (rptr == nullptr ||
                       lfmq_dq_tile_splits(m, n, k, (int)g) > 1);
   // a product that a few workgroups do whole: n 2048, k 2048 11.2 / 14.7 at 77
@@ -179,7 +185,7 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
   const bool small = !rms && rptr == nullptr && (long)n * k <= 4l << 20;
   const bool by_rows = (cols_hint == 0 ? m >= rows_from(bits, n, k, g)
                                        : cols_hint == 6 && m > 4) &&
-                       m <= (large ? 32 : small ? 96 : 48) &&
+                       (!tile || m <= (large ? 32 : small ? 96 : 48)) &&
                        lfmq_dq_rows_ok(m, n, k, (int)g, rms);
   if (m > 16) {
     TORCH_CHECK((by_rows || !rms) && (m <= 48 || rptr == nullptr),
@@ -374,8 +380,10 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
   // as dq_linear.  us with the norm, GEMV / rows, n 28672, k 4096, 4 bits:
   // 37.5 / 24.0 at 4 rows; norm, product and gate apart / rows: 32.5 / 26.4 at
   // 8, 44.0 / 37.6 at 32 (n 16384, k 2048 at 48: 21.4 / 15.6)
-  const bool large = rms_eps < 0 && k >= 4096 && (long)n * k >= 24l << 20;
-  if (cols_hint == 0 && n % 2 == 0 && m > (large ? 32 : 48) &&
+  const bool tile = tile_addresses(n, k, bits) && (long)m * k < 1l << 31;
+  const bool large =
+      tile && rms_eps < 0 && k >= 4096 && (long)n * k >= 24l << 20;
+  if (cols_hint == 0 && tile && n % 2 == 0 && m > (large ? 32 : 48) &&
       lfmq_dq_tile_ok(k, (int)g)) {
     TORCH_CHECK(rms_eps < 0, "fused rms is a decode (m <= 48) path");
     if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
@@ -400,7 +408,8 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
                            (int)bits, 1, (float)rms_eps, true, stream()));
     return y;
   }
-  if (k > 128 * g)                         // the GEMV's limit: the gate apart
+  // what no kernel with the gate in it takes (the GEMV: 128 groups)
+  if (k > 128 * g || (cols_hint == 0 && !tile && m > 48))
     return silu_mul_fused(dq_linear(x, qweight, scales, qzeros, bits, g,
                                     c10::nullopt, c10::nullopt, rms_eps, 0));
   CHECK_HIP(lfmq_dq_gemv_gateup(qweight.data_ptr(), scales.data_ptr(),

@@ -212,6 +212,48 @@ def test_packed_product_of_no_group():
             call()
 
 
+def test_packed_product_with_a_matrix_past_four_gibibytes():
+    """More rows than the kernel that addresses any matrix takes otherwise."""
+    n, k, g, m = 131072 + 64, 65536, 128, 99
+    gen = torch.Generator(DEV).manual_seed(0)
+    p = [torch.randint(-2 ** 31, 2 ** 31 - 1, (n, k // 8), dtype=torch.int32,
+                       generator=gen, device=DEV),
+         torch.rand(n, k // g, generator=gen, device=DEV).to(BF),
+         torch.randint(-2 ** 31, 2 ** 31 - 1, (n, k // g // 8),
+                       dtype=torch.int32, generator=gen, device=DEV)]
+    x = torch.randn(m, k, generator=gen, device=DEV).to(BF)
+    at = torch.tensor([0, 1, n // 2 - 1, n // 2, 65600, 131071, 131072, n - 1],
+                      device=DEV)
+
+    def columns(i):
+        w = ref.dequant_weight(*(t[i].cpu() for t in p), 4, g, k)
+        return x.double() @ w.double().t().to(DEV)
+
+    want = columns(at)
+    y = ext().dq_linear(x, *p, 4, g, None, None, -1.0, 0)
+    assert float((y[:, at].double() - want).abs().max()
+                 / want.abs().max()) < 2 ** -8
+    at = at[:3]
+    want = torch.nn.functional.silu(columns(at)) * columns(at + n // 2)
+    y = ext().dq_gemv_gateup(x, *p, 4, g, -1.0, 0)
+    assert float((y[:, at].double() - want).abs().max()
+                 / want.abs().max()) < 2 ** -6
+
+
+def test_gate_of_rows_past_four_gibibytes():
+    m, n, k, g = 524288 + 70, 128, 4096, 128
+    w, p = packed(n, k, g)
+    x = torch.randn(m, k, device=DEV, dtype=BF)
+    y = ext().dq_gemv_gateup(x, *p, 4, g, -1.0, 0)
+    assert y.shape == (m, n // 2)
+    at = torch.tensor([0, 63, 64, 262143, 262144, 524287, 524288, m - 1],
+                      device=DEV)
+    a, u = (x[at].double() @ w.double().t().to(DEV)).chunk(2, 1)
+    want = torch.nn.functional.silu(a) * u
+    assert float((y[at].double() - want).abs().max()
+                 / want.abs().max()) < 2 ** -6
+
+
 # ------------------------------------------------------------------ gptq
 @pytest.mark.parametrize("tiny", [1e-40, 3e-38, 2e-36, 1e-33])
 def test_gptq_block_of_numbers_below_the_normal_range(tiny):
