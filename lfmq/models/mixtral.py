@@ -157,9 +157,9 @@ class MixtralMoE(nn.Module):
         b, s, h = x.shape
         x2 = x.reshape(-1, h)
         t = x2.shape[0]
-        # up to 64 rows always went through the grouped kernels; more do
-        # where the experts are nothing but their packed matrices
-        if x.is_cuda and self._packed() and (
+        # up to 64 rows go through the grouped kernels whoever watches the
+        # experts; more do where the experts are nothing but their matrices
+        if x.is_cuda and self._packed() and not self._gathers() and (
                 t * self.top_k <= 64 or self._plain()):
             y2 = self._forward_grouped(x2)
         else:
@@ -167,10 +167,15 @@ class MixtralMoE(nn.Module):
             y2 = self._forward_loop(x2, weights, ids)
         return y2.reshape(b, s, h)
 
+    def _gathers(self) -> bool:
+        """Experts have an act-order gather or a bias, which the grouped
+        kernels know nothing of."""
+        return any(hasattr(m, "perm") or m.bias is not None
+                   for e in self.experts for m in (e.w13, e.w2))
+
     def _plain(self) -> bool:
-        """Routing and experts are what the grouped kernels do: no act-order
-        gather, bias, hook, class or forward of their own, and shapes that
-        the kernels take."""
+        """Routing and experts are what the grouped kernels do: no hook, class
+        or forward of their own, and shapes that the kernels take."""
         cls = type(self)
         return (self.n_experts <= 64 and self.top_k <= 4
                 and cls.route is MixtralMoE.route
@@ -178,12 +183,18 @@ class MixtralMoE(nn.Module):
                 and not {"route", "_forward_loop"} & self.__dict__.keys()
                 and all(type(e) is MixtralExpert
                         and not hooked(e, e.w13, e.w2) for e in self.experts)
-                and all(type(m) is QLinear and not hasattr(m, "perm")
-                        and m.bias is None and m.group_size % 32 == 0
+                and all(type(m) is QLinear and m.group_size % 32 == 0
                         for e in self.experts for m in (e.w13, e.w2)))
 
     def _forward_loop(self, x2, weights, ids):
         y = torch.zeros_like(x2)
+        if x2.is_cuda and torch.cuda.is_current_stream_capturing():
+            # every token through every expert: the host may not wait for
+            # the routing
+            for e, expert in enumerate(self.experts):
+                w = (weights * (ids == e)).sum(dim=-1, keepdim=True)
+                y += expert(x2) * w.to(y.dtype)
+            return y
         for e in range(self.n_experts):
             mask = (ids == e)
             tok_mask = mask.any(dim=-1)

@@ -435,6 +435,34 @@ def test_mixtral_weights_replaced_and_then_captured():
             assert close(moe(x), want)
 
 
+@pytest.mark.parametrize("t", [1, 5, 70])
+def test_mixtral_experts_with_a_gather(t):
+    """Act-order experts take their columns in an order of their own, in a
+    captured step too."""
+    moe = quantized_moe(256, 256)
+    x = torch.randn(1, t, 256, device=DEV).to(BF)
+    with torch.no_grad():
+        plain = moe(x)
+        for i, e in enumerate(moe.experts):
+            for m in (e.w13, e.w2):
+                m.register_buffer("perm", torch.randperm(256).to(DEV))
+        want = by_loop(moe, x)
+        assert not close(plain, want)
+        assert close(moe(x), want)
+        if t > 5:
+            return
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = moe(x)
+        for _ in range(3):
+            got.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert close(got, want)
+            assert close(moe(x), want)
+
+
 def test_mixtral_prompt_calls_what_was_put_in_its_way():
     """Hooks on all modules, an expert's own forward or class, routing of a
     subclass."""
