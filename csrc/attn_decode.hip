@@ -383,7 +383,7 @@ hipError_t lfmq_attn_decode(const void* q, const void* kc, const void* vc,
                             int tmax, int T, const void* T_dev, int d,
                             int splits, float scale, hipStream_t stream) {
   if (d != 128 && d != 64) return hipErrorInvalidValue;
-  if (hq % hkv) return hipErrorInvalidValue;
+  if (hq % hkv || T < 1) return hipErrorInvalidValue;
   const DArgs A{(const unsigned short*)q, (unsigned short*)kc,
                 (unsigned short*)vc, (float*)scratch, (u32*)o, nullptr,
                 (const i32*)T_dev, nullptr, hq, hkv, tmax, T, splits,
@@ -402,7 +402,7 @@ hipError_t lfmq_attn_decode_fused(const void* qkv, void* kc, void* vc,
                                   int d, int splits, float scale,
                                   void* tickets, hipStream_t stream) {
   if (d != 128 && d != 64) return hipErrorInvalidValue;
-  if (hq % hkv) return hipErrorInvalidValue;
+  if (hq % hkv || T < 1) return hipErrorInvalidValue;
   const DArgs A{(const unsigned short*)qkv, (unsigned short*)kc,
                 (unsigned short*)vc, (float*)scratch, (u32*)o,
                 (const float*)inv_freq, (const i32*)T_dev, (u32*)tickets, hq,

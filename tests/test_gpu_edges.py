@@ -102,6 +102,19 @@ def test_decode_attention_of_no_sequences():
             torch.ones(64, device=DEV), 32, None, None)
 
 
+def test_decode_attention_of_no_keys():
+    """Refused: there is nothing to take a mean of."""
+    kc = torch.zeros(1, 8, 64, 128, dtype=BF, device=DEV)
+    for T in (0, -3):
+        with pytest.raises(RuntimeError):
+            ext().attn_decode(torch.zeros(1, 32, 1, 128, dtype=BF, device=DEV),
+                              kc, kc, T, 0.1, None)
+        with pytest.raises(RuntimeError):
+            ext().attn_decode_fused(
+                torch.zeros(1, 48 * 128, dtype=BF, device=DEV), kc, kc, T, 0.1,
+                torch.ones(64, device=DEV), 32, None, None)
+
+
 @torch.no_grad()
 def test_decode_steps_that_overlap_on_two_streams():
     """Two captured steps of one model and one shape, each with a cache of
