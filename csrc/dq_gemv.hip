@@ -512,6 +512,7 @@ hipError_t launch_bits(const void* qweight, const void* scales,
         (k <= 4096 ? n <= (m == 1 ? 4096 : 3072) : m == 1 && n <= 3072))
       cols = 1;
     if (cols == 0 || cols == 5) cols = (GATEUP || n >= 16384) ? 4 : 2;
+    if (cols != 4 && (GATEUP || cols != 1)) cols = 2;      // bodies there are
     const int per_wg = WAVES_PER_WG * (GATEUP ? cols / 2 : cols);
     dim3 grid(ceil_div_u32(GATEUP ? n / 2 : n, per_wg));
 #define LFMQ_M(CC)                                                            \
@@ -524,7 +525,7 @@ hipError_t launch_bits(const void* qweight, const void* scales,
         launch_one<BITS, CC, GATEUP, 4, RMS>(grid, block, stream, qweight, scales, qzeros, x, y, bias, resid, m, n, k, g, eps); \
     } while (0)
     if (cols == 4) LFMQ_M(4);
-    else if (cols == 1) LFMQ_M(GATEUP ? 2 : 1);
+    else if (cols == 1) LFMQ_M(GATEUP ? 2 : 1);            // (no gate with 1)
     else LFMQ_M(2);
 #undef LFMQ_M
   } else {

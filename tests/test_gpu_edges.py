@@ -267,6 +267,23 @@ def test_gate_of_rows_past_four_gibibytes():
                  / want.abs().max()) < 2 ** -6
 
 
+@pytest.mark.parametrize("hint", [0, 1, 2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("m", [1, 3])
+def test_gemv_takes_any_number_of_columns_for_a_hint(hint, m):
+    """Numbers that it has no body for are another one's, whole."""
+    n, k, g = 130, 4096, 128
+    w, p = packed(n, k, g)
+    x = torch.randn(m, k).to(BF)
+    want = x.double() @ w.double().t()
+    a, u = want.chunk(2, 1)
+    for y, z in ((ext().dq_linear(x.to(DEV), *p, 4, g, None, None, -1.0, hint),
+                  want),
+                 (ext().dq_gemv_gateup(x.to(DEV), *p, 4, g, -1.0, hint),
+                  torch.nn.functional.silu(a) * u)):
+        assert float((y.double().cpu() - z).abs().max()
+                     / z.abs().max()) < 2 ** -7
+
+
 # ------------------------------------------------------------------ gptq
 @pytest.mark.parametrize("tiny", [1e-40, 3e-38, 2e-36, 1e-33])
 def test_gptq_block_of_numbers_below_the_normal_range(tiny):
