@@ -260,7 +260,7 @@ def dq_gemv_gateup(x: torch.Tensor, qweight: torch.Tensor,
     x2 = x.reshape(-1, x.shape[-1])
     y = hip_ext().dq_gemv_gateup(x2, qweight, scales, qzeros, bits,
                                  group_size, rms_eps, 0)
-    return y.reshape(*x.shape[:-1], y.shape[-1])
+    return _guard(y, "dq_gemv_gateup").reshape(*x.shape[:-1], y.shape[-1])
 
 
 def greedy_sample(logits: torch.Tensor) -> torch.Tensor:

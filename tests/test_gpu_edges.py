@@ -284,6 +284,19 @@ def test_gemv_takes_any_number_of_columns_for_a_hint(hint, m):
                      / z.abs().max()) < 2 ** -7
 
 
+@pytest.mark.parametrize("m", [1, 40])
+def test_guard_names_the_gate(m, monkeypatch):
+    """LFMQ_NANCHECK finds the operation that made a value infinite."""
+    from lfmq.ops import functional as F
+    monkeypatch.setattr(F, "_NANCHECK", True)
+    _, p = packed(64, 128, 64)
+    x = torch.ones(m, 128, device=DEV, dtype=BF)
+    F.dq_gemv_gateup(x, *p, 4, 64)
+    x[0, 3] = math.inf
+    with pytest.raises(FloatingPointError, match="dq_gemv_gateup"):
+        F.dq_gemv_gateup(x, *p, 4, 64)
+
+
 # ------------------------------------------------------------------ gptq
 @pytest.mark.parametrize("tiny", [1e-40, 3e-38, 2e-36, 1e-33])
 def test_gptq_block_of_numbers_below_the_normal_range(tiny):
