@@ -583,6 +583,8 @@ torch::Tensor grouped_tiles(torch::Tensor offsets, long slots) {
   return tiles;
 }
 
+// For callers with sorted slots of their own.  `active`, the experts that have
+// any, says nothing that `offsets` does not: not read.
 torch::Tensor grouped_dq_gateup(torch::Tensor x, torch::Tensor src_tok,
                                 torch::Tensor offsets, torch::Tensor qweight,
                                 torch::Tensor scales, torch::Tensor qzeros,

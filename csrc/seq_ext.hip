@@ -853,7 +853,7 @@ c10::optional<T_> linear_rows(T_ x, T_ w, bool glu) {
     return c10::nullopt;
   const long k = w.size(1), n = w.size(0), m = k ? x.numel() / k : 0;
   const long ldx = x.dim() == 2 && m > 1 ? x.stride(0) : k;
-  if (m > 48 || n > INT32_MAX || k > INT32_MAX || (glu && n % 2) ||
+  if (m > 16 || n > INT32_MAX || k > INT32_MAX || (glu && n % 2) ||
       !lfmq_linear_rows_ok(x.data_ptr(), ldx, w.data_ptr(), (int)m, (int)n,
                            (int)k))
     return c10::nullopt;

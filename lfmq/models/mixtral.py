@@ -1,16 +1,16 @@
-"""Mixtral 8x7B MoE (BASELINE.json config #5).
+"""Mixtral 8x7B MoE.
 
 Same attention/backbone as Llama (GQA, RoPE θ=1e6, RMSNorm) with the MLP
 replaced by a top-2 router over 8 experts.  Experts use the fused
 w13 (gate|up) + w2 (down) projections like the Llama MLP, so GPTQ/AWQ/RTN
 quantize each expert Linear exactly like any other layer.
 
-GPU decode path: tokens are routed, sorted by expert on-device, and run
-through the grouped dequant-GEMM (csrc/grouped_dq_gemm.hip) — one launch
-for all experts' w13 (with the silu·mul epilogue fused) and one for w2 —
-instead of 8 per-expert launches.  With expert
-parallelism (lfmq/dist/ep.py) tokens go through the all-to-all dispatch/
-combine pair instead.
+GPU path, decode and prompts: tokens are routed and sorted by expert on the
+device (csrc/moe_route.hip) and run through the grouped packed products
+(csrc/dq_rows.hip, csrc/dq_tile.hip) — one launch for all experts' w13 (with
+the silu·mul epilogue fused) and one for w2 — instead of launches per expert.
+With expert parallelism (lfmq/dist/ep.py) tokens go through the all-to-all
+dispatch/combine pair instead.
 """
 from __future__ import annotations
 
@@ -84,9 +84,10 @@ _STACKS = [(name, key) for name in ("w13", "w2") for key in _PACKED]
 
 class MixtralMoE(nn.Module):
     """Top-k router + experts.  Forward modes:
-      - dense loop (CPU / prefill): per-expert masked forward
-      - grouped (GPU decode, consolidated buffers): one grouped
-        dequant-GEMM launch pair for all experts
+      - loop (CPU; experts that are more than their packed matrices):
+        per-expert forward of the tokens that chose it
+      - grouped (GPU, stacked buffers): one launch pair of packed products
+        for all experts
       - EP (world > 1): token all-to-all to the rank owning the expert
         (installed by lfmq.dist.ep.apply_expert_parallel)
     """

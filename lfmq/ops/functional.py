@@ -18,7 +18,7 @@ from torch.utils._device import DeviceContext
 
 from . import hip_ext, ref, seq_ext
 
-# Debug numeric guard (SURVEY.md §5.2): LFMQ_NANCHECK=1 asserts every op
+# Debug numeric guard: LFMQ_NANCHECK=1 asserts every op
 # output is finite — catches kernel-layout or quantization bugs at the
 # op that produced them instead of 30 layers later.
 _NANCHECK = os.environ.get("LFMQ_NANCHECK", "0") == "1"
@@ -254,9 +254,10 @@ def attn_decode_fused(qkv, k_cache, v_cache, state_or_T, max_t: int,
 def dq_gemv_gateup(x: torch.Tensor, qweight: torch.Tensor,
                    scales: torch.Tensor, qzeros: torch.Tensor, bits: int,
                    group_size: int, rms_eps: float = -1.0) -> torch.Tensor:
-    """GPU-only fused gate_up product + silu·mul epilogue (m <= 48;
-    above 4 in groups of a multiple of 32);
-    rms_eps >= 0 additionally fuses the RMSNorm of the input."""
+    """GPU-only fused gate_up product + silu·mul epilogue, any number of
+    rows (above 4 in groups of a multiple of 32 that divide k, above 48 of 64);
+    rms_eps >= 0 additionally fuses the RMSNorm of the input (up to 48
+    rows)."""
     x2 = x.reshape(-1, x.shape[-1])
     y = hip_ext().dq_gemv_gateup(x2, qweight, scales, qzeros, bits,
                                  group_size, rms_eps, 0)
