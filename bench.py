@@ -1,13 +1,11 @@
 #!/usr/bin/env python3
-"""Driver bench contract: flagship quantized decode on N GPUs of one node.
+"""Flagship quantized decode on N GPUs of one node.
 
     python bench.py --gpus N --steps K --warmup W
-    (N>1: launched by the driver via torch.distributed.run, one rank/GPU,
-     RCCL over xGMI)
+    (N>1: launched via torch.distributed.run, one rank/GPU, RCCL over xGMI)
 
-Measures the BASELINE.json headline metric — Llama-3-8B W4A16 group-size
-128 greedy-decode tokens/sec — on synthetic data and random-init weights
-(no network; BASELINE.md protocol).  value = whole-job tokens/s (batch ×
+Measures Llama-3-8B W4A16 group-size 128 greedy-decode tokens/sec on
+synthetic data and random-init weights (no network).  value = whole-job tokens/s (batch ×
 steps ÷ max-over-ranks elapsed).  TP keeps total work fixed as N grows
 => scaling "strong".
 """
@@ -95,8 +93,8 @@ def main():
     r = bench_decode(model, cfg, args.batch, args.prompt, args.steps,
                      args.warmup, device)
 
-    # Fidelity field of the contract metric ("decode tok/s + delta-ppl vs
-    # fp16", BASELINE.json:2): teacher-forced ppl + logit KL of the
+    # Fidelity field of the metric ("decode tok/s + delta-ppl vs
+    # fp16"): teacher-forced ppl + logit KL of the
     # quantized model vs the same-seed bf16 reference on a fixed synthetic
     # stream.  Measured at world==1 (the sharded model's fidelity is the
     # same weights; TP changes only the execution plan).

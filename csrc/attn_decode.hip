@@ -1,5 +1,5 @@
 // K8 — GQA decode attention: o = softmax(q·Kᵀ·scale)·V over the KV cache,
-// one query token per sequence (SURVEY.md §2.3 K8).
+// one query token per sequence.
 //
 // Bound by the read of the cache, so a key/value row is read once for all
 // the query heads that share it: a workgroup = one key range x up to GH

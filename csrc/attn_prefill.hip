@@ -1,6 +1,5 @@
 // Flash-style prefill attention on MFMA: o = softmax(q·Kᵀ·scale + causal)·V
-// against the KV cache, s >= 1 queries at positions [pos0, pos0+s)
-// (SURVEY.md §2.3 K8 prefill note).
+// against the KV cache, s >= 1 queries at positions [pos0, pos0+s).
 //
 //   q   [b, s, hq*128] bf16, already roped (qkv_rope_append output view)
 //   k/v [b, hkv, tmax, 128] bf16 caches holding positions [0, pos0+s)

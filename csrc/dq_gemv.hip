@@ -1,7 +1,6 @@
 // K3a/K4a — W4A16 / W8A16 dequant-fused GEMV for decode (m <= 16).
 //
-// The decode hot kernel: y[m,n] = x[m,k] · W[n,k]^T,
-// W int4/int8 group-quantized (layout: lfmq/ops/ref.py).  Memory-bound on
+// The decode hot kernel: y[m,n] = x[m,k] · W[n,k]^T, W int4/int8 group-quantized (layout: lfmq/ops/ref.py).  Memory-bound on
 // the packed weight stream; measured design history on MI355X:
 //   - per-wave buffer descriptors MUST be readfirstlane-uniform
 //     (csrc/common.h make_rsrc_uniform) or hipcc waterfalls every load

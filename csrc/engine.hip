@@ -1,5 +1,5 @@
 // Persistent weight-streaming decode engine for Llama-family W4A16 decode
-// on MI355X (round-2 headline work; design: docs/persistent_decode_design.md,
+// on MI355X (design: docs/persistent_decode_design.md,
 // structure: cdna_hip_programming.md §5.6 + Guideline 16,
 // prices: MI355X_MICROARCH.md persistent-kernel table).
 //
@@ -7,8 +7,8 @@
 // embedding read, per layer [norm+qkv GEMV] -> [rope+append+attention] ->
 // [o GEMV+resid] -> [norm+gate_up GEMV+silu] -> [down GEMV+resid], and the
 // final RMSNorm.  Replaces ~194 launches/step whose ~3-4 us fixed cost was
-// measured as ~0.7 ms of the 1.97 ms round-1 step (profiles/decode_profile_
-// r01.md).  lm_head + sampling remain separate launches.
+// measured as ~0.7 ms of a 1.97 ms step (profiles/decode_profile_r01.md).
+// lm_head + sampling remain separate launches.
 //
 // Geometry: grid = 256 workgroups (one per CU, all co-resident — verified
 // by csrc/engine_probe.hip census), 4 waves each:
@@ -20,7 +20,7 @@
 //                      vmcnt(0) drains — see engine_common.h).
 //   waves 0-2        = consumers: dequant+dot records out of the ring
 //                      (v_perm nibble dequant + v_dot2 bf16, the proven
-//                      round-1 GEMV inner idioms), attention units, and
+//                      inner idioms of the GEMV), attention units, and
 //                      3-way-split granule gathers; wave 0 leads (norm
 //                      scalars, phase publication).
 //
@@ -101,7 +101,7 @@ __device__ __forceinline__ u64 cursor_next(Cursor& c, int rec, u32 ring_bytes) {
 // one conflict-free ds_read_b128 (stride 16 B across lanes).  Math matches
 // csrc/dq_gemv.hip: s*( sum (128+c)*x ) - s*(z+128)*sum x, fp32 accumulate.
 // Chunked two-phase pipeline: issue a whole chunk's LDS loads up front
-// (independent), then compute — the round-1 GEMV lesson (csrc/dq_gemv.hip
+// (independent), then compute — the GEMV's lesson (csrc/dq_gemv.hip
 // KI-unroll): per-iteration loads make the compiler reuse registers and
 // serialize the loop on LDS latency.  CHUNK=8 covers k=4096 ops in one
 // chunk; k=14336 (down) runs 3.5 chunks.

@@ -1,5 +1,4 @@
-// K1 — GPTQ Hessian accumulate: H += 2·XᵀX (X bf16 [t, k], H fp32 [k, k];
-// SURVEY.md §2.3 K1).
+// K1 — GPTQ Hessian accumulate: H += 2·XᵀX (X bf16 [t, k], H fp32 [k, k]).
 //
 // Both operands of a product are columns of X, consecutive tokens a lane.
 // Rows of X go from memory straight into LDS as they are, and the transposing

@@ -1,6 +1,6 @@
 // K6 — fused RMSNorm: y = x · rsqrt(mean(x²)+ε) · w, optional fused
 // residual add in the same pass (one read, one write — the op is
-// HBM-bound; SURVEY.md §2.3 K6).
+// HBM-bound).
 // One workgroup per row; bf16 loaded 8-wide (G13: scalar bf16 is 2×
 // slower); wave shuffle + LDS cross-wave reduction.
 #include "common.h"

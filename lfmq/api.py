@@ -1,4 +1,4 @@
-"""Public API: quantize() / save() / load() (BASELINE.json north star).
+"""Public API: quantize() / save() / load().
 
     from lfmq import quantize, save, load, QuantConfig
     qm = quantize(model, QuantConfig(scheme="gptq"))     # in-place swap to QLinear
@@ -152,7 +152,7 @@ def load(path: str, device: str = "cpu", tp_rank: int = 0, tp_world: int = 1,
         state["lm_head.weight"] = state["embed_tokens.weight"]
     if dtype is not None:
         # assign=True would otherwise let the checkpoint dtype override an
-        # explicitly requested one (ADVICE.md r1): cast float tensors here.
+        # explicitly requested one: cast float tensors here.
         keep = _fp32_names(model)
         state = {k: (v.to(torch.float32 if k in keep else dtype)
                      if v.is_floating_point() else v)
@@ -160,7 +160,7 @@ def load(path: str, device: str = "cpu", tp_rank: int = 0, tp_world: int = 1,
     model.load_state_dict(state, strict=True, assign=True)
     model = model.to(device)  # anything not in the checkpoint (none today)
     # assign=True unties tied embeddings (two independent tensors after the
-    # load, ADVICE.md r1): re-tie so memory and semantics match build time.
+    # load): re-tie so memory and semantics match build time.
     if getattr(model.cfg, "tie_embeddings", False) and \
             isinstance(getattr(model, "lm_head", None), nn.Linear):
         model.lm_head.weight = model.embed_tokens.weight

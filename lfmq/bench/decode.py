@@ -1,7 +1,7 @@
-"""Decode tok/s harness (the BASELINE.json headline metric).
+"""Decode tok/s harness.
 
 Greedy decode on synthetic data / random-init weights (no network => no
-pretrained checkpoints; BASELINE.md).  Timing protocol: untimed prefill +
+pretrained checkpoints).  Timing protocol: untimed prefill +
 warmup decode steps, then barrier + synchronize, time EXACTLY K decode
 steps, synchronize + barrier, MAX over ranks.  Nothing is skipped inside
 the timed region: every step runs all layers + lm_head + argmax and feeds
@@ -55,7 +55,7 @@ def _bench_config(model_name: str, n_layers: Optional[int] = None):
     elif model_name == "tiny-debug-tp8":
         # contract-test shape that shards at TP 4 and 8 (8 q/kv heads,
         # row-shard k dims divisible by 8 ranks x group 32) — exercises
-        # the N=4/8 rank math of the driver's scale run on CPU/gloo
+        # the rank math of 4 and 8 GPUs on CPU/gloo
         cfg = LlamaConfig(vocab_size=512, hidden_size=512,
                           intermediate_size=1024, n_layers=2, n_heads=8,
                           n_kv_heads=8, head_dim=64, max_seq=256)

@@ -1,8 +1,8 @@
-"""Delta-perplexity harness (BASELINE.md): teacher-forced NLL on an
+"""Delta-perplexity harness: teacher-forced NLL on an
 identical fixed-seed synthetic stream through the bf16 model and the
 quantized model; delta_ppl = ppl_quant − ppl_bf16.  Random-init weights
 make ppl noisy, so logit KL and per-layer weight MSE are reported
-alongside as fidelity checks (SURVEY.md §3.4)."""
+alongside as fidelity checks."""
 from __future__ import annotations
 
 import math

@@ -1,4 +1,4 @@
-"""BASELINE.md results-row emitter (SURVEY.md §2 bench inventory)."""
+"""Rows of measured results as a markdown table."""
 from __future__ import annotations
 
 import json
@@ -6,7 +6,7 @@ from typing import List
 
 
 def rows_to_markdown(rows: List[dict]) -> str:
-    """baseline_rows.json entries -> BASELINE.md table rows."""
+    """baseline_rows.json entries -> table rows."""
     out = ["| config | TP | decode tok/s (b=1) | delta-ppl | logit KL | notes |",
            "|---|---|---|---|---|---|"]
     for r in rows:

@@ -1,4 +1,4 @@
-"""rocprofv3 wrapper (SURVEY.md §5.1): capture kernel traces/stats for a
+"""rocprofv3 wrapper: capture kernel traces/stats for a
 bench command and summarize per-kernel totals from the result DB.
 
     from lfmq.bench.rocprof import profile_command, summarize_db
@@ -81,7 +81,7 @@ def summarize_db(db_path: str, top: int = 20, tail_frac: float = 0.5) -> list:
 
 
 def torch_profile(fn, steps: int = 8, out_trace: str = None):
-    """torch.profiler wrapper for launch-gap analysis (SURVEY.md §5.1):
+    """torch.profiler wrapper for launch-gap analysis:
     runs fn() `steps` times under the ROCm-aware profiler and returns the
     key-averages table; optionally exports a chrome trace."""
     import torch

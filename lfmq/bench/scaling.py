@@ -1,9 +1,8 @@
-"""TP scaling-curve runner (SURVEY.md §1 bench inventory).
+"""TP scaling-curve runner.
 
 Launches `bench.py` via torch.distributed.run for each N in gpus and
-collects the JSON lines — the same protocol the driver uses for
-SCALE_rNN.json (weak/strong efficiency is computed by the consumer from
-the per-N values, never reported by us).
+collects the JSON lines (weak/strong efficiency is computed by the consumer
+from the per-N values, never reported here).
 
     python -m lfmq.bench.scaling --gpus 1,2,4,8 --steps 128
 """

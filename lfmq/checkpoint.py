@@ -15,7 +15,7 @@ Format (FORMAT_VERSION 1, layout doc in lfmq/ops/ref.py):
 
 Writes are atomic (tmp file + os.replace).  load_packed(tp_rank, tp_world)
 reads ONLY each rank's shard slices via safetensors lazy slicing — no
-full-tensor read, no weight broadcast (SURVEY.md §3.2).
+full-tensor read, no weight broadcast.
 """
 from __future__ import annotations
 

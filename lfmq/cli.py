@@ -152,7 +152,7 @@ def eval(ckpt: str = typer.Option(...),
                                         "model was built with (quantize "
                                         "--seed); the bf16 reference must "
                                         "match it or delta-ppl is noise")):
-    """Delta-perplexity vs the bf16 model (BASELINE.md protocol):
+    """Delta-perplexity vs the bf16 model:
     teacher-forced NLL on an identical fixed-seed synthetic stream,
     plus logit KL and per-layer weight MSE (random-init caveat)."""
     import lfmq
@@ -211,7 +211,7 @@ def bench(ckpt: Optional[str] = typer.Option(None),
           lm_head: str = typer.Option("w8", help="bf16 | w8 | w4 "
                                       "(profiles/lm_head_decision_r02.md)"),
           no_graph: bool = typer.Option(False)):
-    """Decode tok/s (the BASELINE.json headline metric)."""
+    """Decode tok/s."""
     import lfmq
     from lfmq.bench.decode import bench_decode, build_quantized_llama
 
@@ -266,8 +266,7 @@ def generate(ckpt: str = typer.Option(...),
 def serve(ckpt: str = typer.Option(...),
           host: str = typer.Option("127.0.0.1"),
           port: int = typer.Option(8000)):
-    """Minimal generation server (fastapi/uvicorn) with prometheus
-    counters."""
+    """Minimal generation server (fastapi/uvicorn) with prometheus counters."""
     import lfmq
     from lfmq.obs.serve import make_app
 

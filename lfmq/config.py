@@ -1,8 +1,7 @@
 """Quantization and run configuration.
 
-The reference tree is empty; the binding spec is the north
-star in BASELINE.json:5 — scheme ∈ {rtn, gptq, awq}, bits ∈ {4, 8},
-group-wise scale/zero-point, int4 packing. QuantConfig is the single
+scheme ∈ {rtn, gptq, awq}, bits ∈ {4, 8}, group-wise scale/zero-point,
+int4 packing.  QuantConfig is the single
 source of truth for those knobs and round-trips to/from the packed
 checkpoint's quant_config.json (lfmq/checkpoint.py).
 """
@@ -30,7 +29,7 @@ class QuantConfig:
     group_size:  per-group quantization along the input (k) dimension;
                  -1 means per-channel (one group = whole row).
                  0 plus per_tensor=True means a single scale for the tensor
-                 (config #1: OPT-125m per-tensor int8 RTN).
+                 (OPT-125m: per-tensor int8 RTN).
     sym:         symmetric (no zero-point) vs asymmetric quantization.
     per_tensor:  per-tensor scale (int8 RTN CPU path only).
     """

@@ -3,7 +3,7 @@
 One process per GPU, torch.distributed; the "nccl" backend string IS RCCL
 on ROCm.  The same code path runs under gloo with world_size>1 on a CPU
 host (tests/test_tp_gloo.py) — the only difference is the backend string,
-so multi-rank numerics are testable without a GPU cluster (SURVEY.md §4.3).
+so multi-rank numerics are testable without a GPU cluster.
 """
 from __future__ import annotations
 
@@ -26,7 +26,7 @@ def init_dist(backend: Optional[str] = None) -> tuple[int, int]:
     if world <= 1 and "RANK" not in os.environ:
         return 0, 1
     # under torchrun (RANK set) we initialise even at world 1 so a 1-GPU
-    # run exercises the real RCCL init path (VERDICT r1 #2)
+    # run exercises the real RCCL init path
     if not dist.is_initialized():
         if backend is None:
             backend = "nccl" if torch.cuda.is_available() else "gloo"

@@ -1,6 +1,5 @@
 """Expert parallelism for Mixtral: experts partitioned across ranks,
-token dispatch/return by all_to_all (BASELINE.json
-config #5).
+token dispatch/return by all_to_all.
 
 Two dispatch protocols per MoE layer (ranks hold replicated activations;
 each rank owns the MoE compute for its token shard and n_experts/world
@@ -20,7 +19,7 @@ dispatch).  3 collectives/layer total: dispatch, combine, re-replicate.
 
 DYNAMIC (prefill / large t): ragged all_to_all with an up-front count
 exchange.  The exchange tensors live on the computing device (RCCL
-requires device tensors; round-1 had them on CPU) and
+requires device tensors) and
 the single .tolist() on the counts is the one host sync.
 
   1. shard tokens: rank r takes its slice of the flattened tokens

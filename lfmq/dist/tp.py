@@ -1,6 +1,6 @@
 """Tensor-parallel sharding of packed quantized Llama models.
 
-Plan (SURVEY.md §2.4): column-parallel qkv_proj / gate_up_proj / lm_head,
+Plan: column-parallel qkv_proj / gate_up_proj / lm_head,
 row-parallel o_proj / down_proj with an all-reduce on RCCL over xGMI.
 Packed-tensor slicing rules (layout: lfmq/ops/ref.py):
   - column (n) shard: slice rows of qweight/scales/qzeros.
@@ -165,7 +165,7 @@ def shard_llama(model: nn.Module, rank: int, world: int) -> nn.Module:
 
 @torch.no_grad()
 def shard_mixtral(model: nn.Module, rank: int, world: int) -> nn.Module:
-    """TP-only Mixtral fallback (SURVEY.md §2.4): attention column/row
+    """TP-only Mixtral fallback: attention column/row
     sharded exactly like Llama, experts REPLICATED (the mandated
     expert-parallel path is lfmq.dist.ep; this keeps memory higher but
     needs no all-to-all).  The row-parallel o_proj all-reduce makes the
@@ -211,7 +211,7 @@ class _GatheredLinear(nn.Module):
 def load_tp(path: str, meta: dict, device: str, rank: int, world: int,
             dtype=None) -> nn.Module:
     """Build this rank's sharded model, reading only its slices from the
-    packed checkpoint (no broadcast, lazy slices)."""
+    packed checkpoint."""
     from ..api import _build_quantized_skeleton
     from ..checkpoint import load_packed
 

@@ -1,4 +1,4 @@
-"""hipGraph-captured decode (SURVEY.md §7 M6).
+"""hipGraph-captured decode.
 
 The eager decode step is ~260 kernel launches; at ~1.2-3 µs of
 launch/gap each that overhead rivals the weight-stream time.  The whole

@@ -2,7 +2,7 @@
 
 One stacked [L, b, hkv, T_max, d] bf16 allocation per side; `k[i]`/`v[i]`
 are contiguous per-layer views (static addresses so the whole decode step
-can be captured into a hipGraph — SURVEY.md §3.3).  The stacked base
+can be captured into a hipGraph).  The stacked base
 tensors (`k_all`/`v_all`) give the persistent decode engine a single
 pointer + layer stride (lfmq/models/engine.py).
 """

@@ -1,10 +1,9 @@
 """Llama-3 family architecture, built natively for the MI355X decode path.
 
-Random-init from a local config (no network => no pretrained weights,
-BASELINE.md protocol).  MI355X-first choices:
+Random-init from a local config (no network => no pretrained weights).
+MI355X-first choices:
   - fused qkv_proj and gate_up_proj Linears (one GEMV launch each at
-    decode instead of 3/2 — launch overhead is the TP=8 risk,
-    SURVEY.md §2.5)
+    decode instead of 3/2 — launch overhead is the TP=8 risk)
   - static KV cache + pure-tensor decode step, hipGraph-capturable
   - attention decode / rmsnorm / rope / silu·mul via the gfx950 HIP
     kernels (lfmq.ops.functional)
@@ -56,7 +55,7 @@ class LlamaConfig:
 
     @classmethod
     def tiny(cls, **kw):
-        """2-layer 8B-shaped-per-layer test model (SURVEY.md §4.5)."""
+        """2-layer 8B-shaped-per-layer test model."""
         return cls(**{**dict(vocab_size=512, hidden_size=256,
                              intermediate_size=512, n_layers=2, n_heads=4,
                              n_kv_heads=2, head_dim=64, max_seq=512), **kw})

@@ -1,5 +1,5 @@
-"""OPT-125m — the plumbing model for BASELINE.json config #1:
-per-tensor int8 RTN quantize + CPU matmul decode (no GPU involved).
+"""OPT-125m — the plumbing model: per-tensor int8 RTN quantize + CPU matmul
+decode (no GPU involved).
 
 LayerNorm / ReLU architecture, learned positional embeddings (offset 2,
 as OPT does), pre-LN.  Random-init; runs entirely in local pytest.

@@ -101,9 +101,7 @@ class QLinear(nn.Module):
         if perm is not None:
             # act-order layout v2: the packed weight keeps QUANT order
             # (groups contiguous — every fused kernel works unchanged);
-            # the input is gathered once instead (x[perm]).  GPU act-order
-            # decode was a loud NotImplementedError in round 1 (VERDICT
-            # item 5).
+            # the input is gathered once instead (x[perm]).
             x = x.index_select(-1, perm)
         return F.dq_linear(x, self.qweight, self.scales, self.qzeros,
                            self.bits, self.group_size, self.bias)
@@ -144,8 +142,8 @@ def rows_fused(p: nn.Module) -> bool:
 
 
 class Int8PerTensorLinear(nn.Module):
-    """Per-tensor symmetric int8 linear — the OPT-125m CPU decode path
-    (BASELINE.json config #1).  int8 codes + one fp32 scale."""
+    """Per-tensor symmetric int8 linear — the OPT-125m CPU decode path.
+    int8 codes + one fp32 scale."""
 
     def __init__(self, in_features: int, out_features: int, bias: bool = True):
         super().__init__()
@@ -197,7 +195,7 @@ class GatherColumnParallelQLinear(QLinear):
     crosses k-shard boundaries, so instead the (k-sharded) input is
     all-gathered to full width, the OUTPUT dim is column-sharded, and the
     shard outputs are all-gathered — two all-gathers instead of one
-    all-reduce, for the act-order quality mode only (VERDICT r1 item 5)."""
+    all-reduce, for the act-order quality mode only."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         x = lfmq_dist.all_gather_cat(x, dim=-1)
@@ -213,8 +211,7 @@ class GatherColumnParallelQLinear(QLinear):
 
 
 class RowParallelQLinear(QLinear):
-    """Input dimension sharded; partial outputs all-reduced (RCCL/xGMI —
-    the collective call site of SURVEY.md §2.5)."""
+    """Input dimension sharded; partial outputs all-reduced (RCCL/xGMI)."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         y = super().forward(x)

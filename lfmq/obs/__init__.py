@@ -1,4 +1,4 @@
-"""Observability: structured logging + per-phase timers (SURVEY.md §5.5)."""
+"""Observability: structured logging + per-phase timers."""
 from __future__ import annotations
 
 import contextlib

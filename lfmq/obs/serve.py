@@ -1,6 +1,6 @@
 """Minimal FastAPI generation server with prometheus counters.
 
-Not on the benchmark critical path (SURVEY.md §5.5) — a thin serving
+Not on the benchmark critical path — a thin serving
 front for the quantized decode engine:
     POST /generate  {"input_ids": [[...]], "max_new_tokens": 32}
     GET  /metrics   prometheus text (tokens generated, requests, tok/s)

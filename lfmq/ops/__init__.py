@@ -1,9 +1,9 @@
 """Op bindings: the single compute backend is PyTorch-ROCm + the in-tree
 HIP extensions (csrc/ -> lfmq_hip.so and lfmq_seq.so, gfx950 only).
 
-There is deliberately NO multi-backend dispatch:
-on a GPU device the HIP extension is the only path and a missing extension
-raises immediately instead of silently falling back to eager PyTorch.  The
+There is deliberately NO multi-backend dispatch: on a GPU device the HIP
+extension is the only path and a missing extension raises immediately instead
+of silently falling back to eager PyTorch.  The
 CPU twins in lfmq.ops.ref exist for unit tests and for the OPT-125m int8
 CPU decode config, which is spec'd as a CPU path.
 """

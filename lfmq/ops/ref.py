@@ -2,8 +2,7 @@
 
 Exact, simple torch-CPU (fp32) implementations.  Every HIP kernel's GPU
 parity test (tests/test_gpu_kernels.py, -m gpu) compares against one of
-these.  The OPT-125m int8 CPU decode path (BASELINE.json config #1) also
-runs on these — that is a spec'd CPU path, not a dispatch fallback.
+these.  The OPT-125m int8 CPU decode path also runs on these — that is a spec'd CPU path, not a dispatch fallback.
 
 Packed layout v1 (FORMAT_VERSION = 1, lfmq/config.py):
   qweight: uint32 [n, k/8]   — nibble i (little-endian: bits 4i..4i+3) of
@@ -69,7 +68,7 @@ def quant_groupwise(
 
 
 def quant_per_tensor_int8(w: torch.Tensor) -> Tuple[torch.Tensor, float]:
-    """Per-tensor symmetric int8 (config #1).  Returns (codes int8, scale)."""
+    """Per-tensor symmetric int8.  Returns (codes int8, scale)."""
     w = w.float()
     absmax = float(w.abs().max())
     scale = absmax / 127.0 if absmax > 0 else 1.0

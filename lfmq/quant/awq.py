@@ -3,8 +3,7 @@
 Per scale-group (linears sharing one input), grid-search α ∈ [0,1] for
 per-channel scales s = a_absmean^α (normalized), fold s into the producing
 op (RMSNorm/LayerNorm weight, or the previous Linear's output rows), then
-group-wise RTN int4/int8 on the scaled weights (BASELINE.json:5 inventory:
-"group-wise scale/zero-point search").
+group-wise RTN int4/int8 on the scaled weights.
 
 Scale groups (fused-projection Llama arch):
   input_layernorm        -> qkv_proj

@@ -1,8 +1,7 @@
 """Calibration data pipeline: fixed-seed synthetic token streams.
 
-No network anywhere in this environment, so calibration
-runs on seeded synthetic token sequences — matching the BASELINE.json
-protocol ("on synthetic data / random-init weights").  Batches stream
+No network anywhere in this environment, so calibration runs on seeded
+synthetic token sequences.  Batches stream
 through the model block-by-block (sequential per-block calibration keeps
 peak memory at one decoder block, which is what lets a 70B quantize fit).
 """

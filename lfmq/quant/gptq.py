@@ -1,7 +1,7 @@
 """GPTQ calibration: per-channel Hessian accumulate, damped Cholesky
 inverse, column-blocked quantize-then-error-propagate loop.
 
-Math (the north star's inventory, BASELINE.json:5):
+Math:
   H   = Σ 2·XᵀX                      (ops.hessian_accum — HIP K1 on GPU)
   H_d = H + λ·mean(diag H)·I          (λ = damp_percent)
   U   = chol(H_d⁻¹, upper)            (csrc/chol_inverse.hip on GPU)
@@ -16,7 +16,7 @@ GPU kernel serves act-order checkpoints unchanged.
 Calibration is sequential per decoder block: only one block's Hessians
 (≈1 GB fp32 for 8B, ≈4 GB for 70B) are live at a time, and the next
 block's inputs are produced by the already-quantized block, so error
-propagates realistically (SURVEY.md §3.1).
+propagates realistically.
 """
 from __future__ import annotations
 
@@ -159,7 +159,7 @@ class GPTQQuantizer:
     def run(self, model: nn.Module, calib: Optional[CalibStream] = None,
             device: Optional[torch.device] = None,
             resume_dir: Optional[str] = None) -> nn.Module:
-        """resume_dir: per-block completion checkpoints (SURVEY.md §5.4) —
+        """resume_dir: per-block completion checkpoints —
         a 70B calibration is long; `quantize --resume` skips blocks whose
         quantized state was already written (atomic tmp+rename)."""
         import os
@@ -214,7 +214,6 @@ class GPTQQuantizer:
                         if meta.get("perm"):
                             # act_order checkpoints carry a perm buffer;
                             # register it so load_state_dict finds the key
-                            # (resume of act_order=True failed).
                             q.register_buffer("perm", torch.zeros(
                                 meta["in"], dtype=torch.int64, device=device))
                         replace_module(block, lname, q)

@@ -1,4 +1,4 @@
-"""Round-to-nearest quantizer: per-tensor int8 (config #1) and per-group
+"""Round-to-nearest quantizer: per-tensor int8 and per-group
 int4/int8 (the RTN baseline for GPTQ/AWQ comparisons)."""
 from __future__ import annotations
 

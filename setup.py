@@ -17,7 +17,7 @@ from torch.utils.cpp_extension import BuildExtension, CUDAExtension
 os.environ.setdefault("PYTORCH_ROCM_ARCH", "gfx950")
 
 # LFMQ_ASAN=1: address-sanitized build of the HOST side of the extension
-# (binding/launch logic; SURVEY.md §5.2).  Run with
+# (binding/launch logic).  Run with
 # LD_PRELOAD=$(clang -print-file-name=libclang_rt.asan-x86_64.so).
 _ASAN = os.environ.get("LFMQ_ASAN", "0") == "1"
 _CXX_FLAGS = ["-O3", "-std=c++17"] + (
