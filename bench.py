@@ -34,7 +34,7 @@ def main():
     # profiles/lm_head_decision_r02.md
     ap.add_argument("--lm-head", default="w8", choices=["bf16", "w4", "w8"],
                     help="lm_head path: HIP W8 GEMV (default; KL-neutral), "
-                         "rocBLAS bf16, or HIP W4 (fastest, +6% logit KL)")
+                         "rocBLAS bf16, or HIP W4 (fastest, +6%% logit KL)")
     ap.add_argument("--quant-lm-head", action="store_true",
                     help="legacy alias for --lm-head w4")
     ap.add_argument("--no-fidelity", action="store_true",
