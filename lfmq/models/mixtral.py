@@ -14,6 +14,7 @@ dispatch/combine pair instead.
 """
 from __future__ import annotations
 
+import threading
 from dataclasses import dataclass, asdict
 from typing import Optional
 
@@ -24,7 +25,7 @@ from ..ops import functional as F
 from .kvcache import KVCache
 from .linear import Linear, hooked
 from .llama import LlamaAttention, LlamaConfig, RMSNorm
-from .qlinear import QLinear
+from .qlinear import QLinear, gathers
 
 
 @dataclass
@@ -79,7 +80,7 @@ class MixtralExpert(nn.Module):
 # the grouped kernels address 4 GiB of 16-bit rows
 _ROWS_ELEMENTS = (1 << 31) - 1
 _PACKED = ("qweight", "scales", "qzeros")
-_STACKS = [(name, key) for name in ("w13", "w2") for key in _PACKED]
+_STACKING = threading.Lock()
 
 
 class MixtralMoE(nn.Module):
@@ -108,22 +109,50 @@ class MixtralMoE(nn.Module):
         weights = torch.softmax(weights, dim=-1)
         return weights, ids
 
-    def _packed(self) -> bool:
-        return all(isinstance(m, QLinear) for e in self.experts
-                   for m in (e.w13, e.w2))
+    def _layers(self):
+        """The experts' layers [w13, w2, w13, ..], or None if one of them is
+        not packed.  (Asked for in every forward: no module attributes.)"""
+        ms = [e._modules.get(name) for e in self.experts._modules.values()
+              for name in ("w13", "w2")]
+        for m in ms:
+            if not isinstance(m, QLinear):
+                return None
+        return ms
 
     def consolidate(self):
         """Stack the quantized experts' packed buffers for the grouped
         kernels: qweight [E, n, kw], scales [E, n, G], qzeros [E, n, zw].
         The experts' buffers become the stacks' parts: the weights are there
         once, and what is written to an expert is what the kernels read."""
-        if not self._packed():
+        ms = self._layers()
+        return None if ms is None else self._stacks(ms)
+
+    def _stacks(self, ms=None) -> dict:
+        """The stacks of the experts' buffers as they are now: replaced or
+        moved ones are stacked again."""
+        ms = ms or self._layers()
+        g = self._current(ms)
+        if g is None:
+            with _STACKING:
+                g = self._current(ms) or self._stack(ms)
+        return g
+
+    def _current(self, ms):
+        g = self._grouped
+        if g is None:
             return None
+        for key, stacked in zip(_PACKED, g["at"]):
+            if [m._buffers[key].data_ptr() for m in ms] != stacked or \
+                    g["w13"][key].data_ptr() != stacked[0] or \
+                    g["w2"][key].data_ptr() != stacked[1]:
+                return None
+        return g
+
+    def _stack(self, ms) -> dict:
         g = {}
         # (ordinary tensors, which may be written to, in any mode)
         with torch.inference_mode(False), torch.no_grad():
-            for name in ("w13", "w2"):
-                mods = [getattr(e, name) for e in self.experts]
+            for name, mods in (("w13", ms[::2]), ("w2", ms[1::2])):
                 g[name] = {key: torch.stack([getattr(m, key) for m in mods])
                            for key in _PACKED}
                 g[name].update(bits=mods[0].bits, g=mods[0].group_size,
@@ -134,24 +163,13 @@ class MixtralMoE(nn.Module):
                 return g         # the graph's: filled whenever it runs
             # before another stream reads the stacks
             torch.cuda.current_stream(device).synchronize()
-        for name, key in _STACKS:
-            for e, part in zip(self.experts, g[name][key]):
-                setattr(getattr(e, name), key, part)
+        for name, mods in (("w13", ms[::2]), ("w2", ms[1::2])):
+            for key in _PACKED:
+                for m, part in zip(mods, g[name][key]):
+                    setattr(m, key, part)
+        # where the layers' buffers are while they are parts of the stacks
+        g["at"] = [[m._buffers[key].data_ptr() for m in ms] for key in _PACKED]
         self._grouped = g
-        return g
-
-    def _stacks(self) -> dict:
-        """The stacks of the experts' buffers as they are now: replaced or
-        moved ones are stacked again."""
-        g = self._grouped
-        if g is None:
-            return self.consolidate()
-        for name, key in _STACKS:
-            t = g[name][key]
-            at, step = t.data_ptr(), t.stride(0) * t.element_size()
-            for i, e in enumerate(self.experts):
-                if getattr(getattr(e, name), key).data_ptr() != at + i * step:
-                    return self.consolidate()
         return g
 
     def forward(self, x):
@@ -160,19 +178,14 @@ class MixtralMoE(nn.Module):
         t = x2.shape[0]
         # up to 64 rows go through the grouped kernels whoever watches the
         # experts; more do where the experts are nothing but their matrices
-        if x.is_cuda and self._packed() and not self._gathers() and (
+        ms = self._layers() if x.is_cuda else None
+        if ms is not None and not any(map(gathers, ms)) and (
                 t * self.top_k <= 64 or self._plain()):
-            y2 = self._forward_grouped(x2)
+            y2 = self._forward_grouped(x2, self._stacks(ms))
         else:
             weights, ids = self.route(x2)
             y2 = self._forward_loop(x2, weights, ids)
         return y2.reshape(b, s, h)
-
-    def _gathers(self) -> bool:
-        """Experts have an act-order gather or a bias, which the grouped
-        kernels know nothing of."""
-        return any(hasattr(m, "perm") or m.bias is not None
-                   for e in self.experts for m in (e.w13, e.w2))
 
     def _plain(self) -> bool:
         """Routing and experts are what the grouped kernels do: no hook, class
@@ -207,13 +220,12 @@ class MixtralMoE(nn.Module):
             y[tok_mask] += ye * w.unsqueeze(-1).to(ye.dtype)
         return y
 
-    def _forward_grouped(self, x2):
+    def _forward_grouped(self, x2, g):
         """On the device from logits to sum, any number of tokens: routing
         and row tiles in one kernel, grouped products with silu·mul in the
         first one's epilogue, weighted sum of a token's rows."""
         from ..ops import hip_ext
         ext = hip_ext()
-        g = self._stacks()
         a, b = g["w13"], g["w2"]
         logits16 = self.gate(x2).contiguous()  # dense bf16 router GEMV
 

@@ -128,6 +128,14 @@ class QLinear(nn.Module):
                            self.bits, self.group_size, self.bias, resid=resid)
 
 
+def gathers(p: QLinear) -> bool:
+    """Whether p takes its input's columns in an order of its own (act-order),
+    or adds a bias: what products of stacked matrices know nothing of."""
+    b = p._buffers
+    return "perm" in b or "perm" in p.__dict__ or \
+        b.get("bias") is not None or p.__dict__.get("bias") is not None
+
+
 FEW_ROWS = 48        # rows of the kernel that has norm and gate epilogues
 
 

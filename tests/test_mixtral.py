@@ -229,3 +229,24 @@ def test_experts_made_in_inference_mode_consolidate(later):
             qm.consolidate_moe()
     qm.consolidate_moe()
     assert qm.layers[0].moe._stacks()["w13"]["qweight"].shape[0] == 4
+
+
+def test_experts_are_stacked_once_for_all_threads():
+    """Threads that use a model first at the same time read one copy."""
+    import threading
+    cfg = MixtralConfig.tiny(hidden_size=256, intermediate_size=1024)
+    qcfg = lfmq.QuantConfig(scheme="rtn", bits=4, group_size=32)
+    moe = lfmq.quantize(lfmq.build_model(cfg, seed=8), qcfg).layers[0].moe
+    got, start = [], threading.Barrier(8)
+
+    def first():
+        start.wait()
+        got.append(moe._stacks())
+
+    threads = [threading.Thread(target=first) for _ in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(got) == 8 and all(g is got[0] for g in got)
+    assert moe._stacks() is got[0]
