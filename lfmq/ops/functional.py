@@ -157,7 +157,9 @@ def attn_prefill(q, k, v, causal: bool = True, scale: Optional[float] = None):
         hkv = k.shape[1]
         rep = hq // hkv
         scale = scale or 1.0 / math.sqrt(d)
-        kt = k.transpose(-1, -2)                      # [b, hkv, d, s]
+        # [b, hkv, d, s], laid out so: the library's batched 16-bit product
+        # has faulted on a right operand that is a transposed view
+        kt = k.transpose(-1, -2).contiguous()
         out = torch.empty_like(q)
         CH = 512 if s > 512 else s
         for q0 in range(0, s, CH):

@@ -53,6 +53,24 @@ def test_prompt_attention_takes_any_scale(scale, s, pos0):
     assert float((got - want).abs().max() / want.abs().max()) < 2 ** -7
 
 
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("b,s", [(1, 7), (2, 3), (5, 9), (17, 2), (1, 130)])
+def test_prompt_attention_of_narrow_heads(d, b, s):
+    """Head sizes that the kernel does not take: products of the library,
+    whose operands are laid out for it.  Weights and result are rounded to 8
+    bits."""
+    from lfmq.ops import functional as F
+    torch.manual_seed(s)
+    hq, hkv = 8, 2
+    q = torch.randn(b, s, hq, d).to(BF).to(DEV).transpose(1, 2)
+    kc, vc = (torch.randn(b, hkv, s + 16, d).to(BF) for _ in range(2))
+    got = F.attn_prefill(q, kc.to(DEV)[:, :, :s], vc.to(DEV)[:, :, :s])
+    want = ref.attn_prefill(q.cpu().float(), kc[:, :, :s].float(),
+                            vc[:, :, :s].float())
+    assert float((got.float().cpu() - want).abs().max()
+                 / want.abs().max()) < 2 ** -6
+
+
 @pytest.mark.parametrize("T", [1, 33, 70, 300])
 @pytest.mark.parametrize("fused", [False, True])
 def test_decode_attention_of_an_infinite_value(T, fused):
