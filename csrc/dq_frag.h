@@ -24,6 +24,25 @@ __device__ __forceinline__ s16x8 codes8(const u32* w) {
   }
 }
 
+// The same eight codes of a dword in the order 0 2 4 6 1 3 5 7, which takes
+// seven instructions instead of eleven, and eight numbers of x in that order.
+__device__ __forceinline__ s16x8 codes8_dealt(u32 w) {
+  const u32 even = w & 0x0F0F0F0Fu, odd = (w >> 4) & 0x0F0F0F0Fu;
+  return __builtin_bit_cast(
+      s16x8, u32x4{__builtin_amdgcn_perm(0x43434343u, even, 0x04010400u),
+                   __builtin_amdgcn_perm(0x43434343u, even, 0x04030402u),
+                   __builtin_amdgcn_perm(0x43434343u, odd, 0x04010400u),
+                   __builtin_amdgcn_perm(0x43434343u, odd, 0x04030402u)});
+}
+__device__ __forceinline__ s16x8 deal8(s16x8 x) {
+  const u32x4 a = __builtin_bit_cast(u32x4, x);
+  return __builtin_bit_cast(
+      s16x8, u32x4{__builtin_amdgcn_perm(a[1], a[0], 0x05040100u),
+                   __builtin_amdgcn_perm(a[3], a[2], 0x05040100u),
+                   __builtin_amdgcn_perm(a[1], a[0], 0x07060302u),
+                   __builtin_amdgcn_perm(a[3], a[2], 0x07060302u)});
+}
+
 // zb of group gi from its word of packed zeros
 template <int BITS>
 __device__ __forceinline__ float zero_bias(u32 word, int gi) {

@@ -16,6 +16,10 @@ hipError_t lfmq_dq_rows(const void*, const void*, const void*, const void*,
                         void*, const void*, const void*, void*, int, int, int,
                         int, int, int, float,
                         bool, hipStream_t);
+bool lfmq_dq_row_ok(int, int, int);
+hipError_t lfmq_dq_row(const void*, const void*, const void*, const void*,
+                       void*, const void*, const void*, int, int, int, int,
+                       float, bool, hipStream_t);
 bool lfmq_dq_tile_ok(int, int);
 int lfmq_dq_tile_splits(int, int, int, int);
 hipError_t lfmq_dq_tile(const void*, const void*, const void*, const void*,
@@ -146,9 +150,10 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
   const int m = (int)x.size(0), k = (int)x.size(1);
   const int n = (int)qweight.size(0);
   TORCH_CHECK(qweight.size(1) == (long)k * bits / 32, "qweight/k mismatch");
-  // more groups than either kernel with the norm in it holds scales of (381
+  const bool one = cols_hint == 0 && m == 1 && lfmq_dq_row_ok(n, k, (int)g);
+  // more groups than the kernels with the norm in them hold scales of (381
   // and 128): the norm apart
-  if (rms_eps >= 0 && m <= 4 && k > 128 * g &&
+  if (rms_eps >= 0 && m <= 4 && k > 128 * g && !one &&
       !lfmq_dq_rows_ok(m, n, k, (int)g, true)) {
     x = rmsnorm(x, torch::ones({k}, x.options()), rms_eps, c10::nullopt);
     rms_eps = -1;
@@ -201,7 +206,12 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
                         x.options().dtype(torch::kFloat32));
     return part.data_ptr();
   };
-  if (by_rows) {
+  if (one) {
+    CHECK_HIP(lfmq_dq_row(qweight.data_ptr(), scales.data_ptr(),
+                          qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
+                          rptr, n, k, (int)g, (int)bits, (float)rms_eps, false,
+                          stream()));
+  } else if (by_rows) {
     const int splits = rms ? 1 : lfmq_dq_rows_splits(m, n, k, (int)g);
     CHECK_HIP(lfmq_dq_rows(qweight.data_ptr(), scales.data_ptr(),
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
@@ -397,6 +407,14 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
                            nullptr, nullptr,
                            splits > 1 ? part.data_ptr() : nullptr, m, n, k,
                            (int)g, (int)bits, splits, true, stream()));
+    return y;
+  }
+  if (cols_hint == 0 && n % 2 == 0 && m == 1 && lfmq_dq_row_ok(n, k, (int)g)) {
+    if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
+    CHECK_HIP(lfmq_dq_row(qweight.data_ptr(), scales.data_ptr(),
+                          qzeros.data_ptr(), x.data_ptr(), y.data_ptr(),
+                          nullptr, nullptr, n, k, (int)g, (int)bits,
+                          (float)rms_eps, true, stream()));
     return y;
   }
   if (cols_hint == 0 && m >= rows_from(bits, n, k, g) && m <= 48 &&

@@ -30,6 +30,7 @@ SOURCES = [
     "csrc/rope.hip",
     "csrc/elementwise.hip",
     "csrc/dq_gemv.hip",
+    "csrc/dq_row.hip",
     "csrc/dq_rows.hip",
     "csrc/dq_tile.hip",
     "csrc/hessian.hip",

@@ -1,0 +1,77 @@
+"""Packed products of a decode step against 64 bits: one row (dq_row) and up
+to sixteen (dq_wide), where their waves, groups and tiles end.
+
+Products of bf16 and codes are exact and summed in fp32, so a result is off
+by its own rounding, 2^-9 of a value, and by the sums' error where it is small
+beside its row."""
+import pytest
+import torch
+
+from lfmq.ops import hip_ext as ext
+from lfmq.ops import ref
+
+pytestmark = pytest.mark.gpu
+DEV, BF = "cuda", torch.bfloat16
+
+
+def matrix(bits, n, k, g, experts=()):
+    """Packed weights on the device, and what they stand for."""
+    codes = torch.randint(0, 1 << bits, (*experts, n, k), dtype=torch.int32)
+    zeros = torch.randint(0, 1 << bits, (*experts, n, k // g),
+                          dtype=torch.int32)
+    s = (torch.rand(*experts, n, k // g) * 0.02 + 0.01).to(BF)
+    flat = [t.flatten(0, -2) for t in (codes, zeros, s)]
+    w = ((flat[0].to(DEV).view(-1, k // g, g) - flat[1].to(DEV).unsqueeze(-1))
+         .double() * flat[2].to(DEV).double().unsqueeze(-1)).flatten(1)
+    packed = [ref.pack_codes(flat[0], bits), flat[2],
+              ref.pack_zeros(flat[1], bits)]
+    return [t.view(*experts, n, -1).to(DEV).contiguous() for t in packed], \
+        w.view(*experts, n, k)
+
+
+def close(y, want, rel=5e-3):
+    err = (y.double() - want).abs()
+    floor = 1e-3 * want.abs().amax(-1, keepdim=True) + 1e-30
+    assert y.shape == want.shape
+    assert float((err / (want.abs() + floor)).max()) < rel
+
+
+def normed(x, eps):
+    x = x.double()
+    return x * torch.rsqrt((x ** 2).mean(-1, keepdim=True) + eps)
+
+
+def gated(h):
+    a, u = h.chunk(2, -1)
+    return torch.nn.functional.silu(a) * u
+
+
+def check(bits, m, n, k, g):
+    p, w = matrix(bits, n, k, g)
+    x = torch.randn(m, k, device=DEV).to(BF)
+    if m > 1:
+        x[0] = 0
+    bias = torch.randn(n, device=DEV).to(BF)
+    resid = torch.randn(m, n, device=DEV).to(BF)
+    plain, rms = x.double() @ w.t(), normed(x, 1e-5) @ w.t()
+    close(ext().dq_linear(x, *p, bits, g, bias, None, 1e-5, 0),
+          rms + bias.double())
+    close(ext().dq_linear(x, *p, bits, g, None, resid, -1.0, 0),
+          plain + resid.double())
+    if n % 2 == 0:
+        # the gate turns its sum's error into at most its slope, 1.1, of it
+        close(ext().dq_gemv_gateup(x, *p, bits, g, 1e-5, 0), gated(rms), 1e-2)
+        close(ext().dq_gemv_gateup(x, *p, bits, g, -1.0, 0), gated(plain),
+              1e-2)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("n,k,g", [
+    (8198, 2048, 128), (8193, 2048, 64), (7946, 2112, 32), (4097, 4096, 128),
+    (28674, 4096, 128), (4106, 5120, 128), (2731, 6400, 64), (1542, 8192, 128),
+    (1030, 14336, 128), (774, 16384, 32)])
+def test_one_row(bits, n, k, g):
+    """One to eight waves along k, the last one short; rows that end inside a
+    group of four, gates inside a pair; several groups a wave."""
+    torch.manual_seed(n)
+    check(bits, 1, n, k, g)
