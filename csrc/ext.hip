@@ -20,6 +20,13 @@ bool lfmq_dq_row_ok(int, int, int);
 hipError_t lfmq_dq_row(const void*, const void*, const void*, const void*,
                        void*, const void*, const void*, int, int, int, int,
                        float, bool, hipStream_t);
+bool lfmq_dq_wide_ok(int, int, int, int);
+hipError_t lfmq_dq_wide(const void*, const void*, const void*, const void*,
+                        void*, const void*, const void*, int, int, int, int,
+                        int, float, bool, hipStream_t);
+hipError_t lfmq_dq_wide_experts(const void*, const void*, const void*,
+                                const void*, const void*, const void*, void*,
+                                int, int, int, int, int, bool, hipStream_t);
 bool lfmq_dq_tile_ok(int, int);
 int lfmq_dq_tile_splits(int, int, int, int);
 hipError_t lfmq_dq_tile(const void*, const void*, const void*, const void*,
@@ -132,6 +139,18 @@ bool tile_addresses(long n, long k, long bits) {
   return n * k / 8 * bits < 1l << 32;
 }
 
+// The kernel that keeps x and walks over columns, or rows.  us of rows / wide,
+// 4 bits: n 28672, k 4096 21.5 / 16.0 at 2 rows, 30.4 / 18.5 at 16; n 4096, k
+// 4096 6.6 / 6.1 and 9.0 / 8.7; n 2048, k 2048 4.9 / 4.1 and 6.3 / 5.6; n 8192,
+// k 8192 14.5 / 12.4 and 18.6 / 17.4; n 5120, k 5120 14.6 / 14.5 at 16.  A long
+// k of few columns is another matter: n 4096, k 14336 13.7 / 13.1 at 2 rows,
+// 19.5 / 22.9 at 16; n 2048, k 8192 (8 bits) 10.7 / 11.5 at 4.
+bool wide_rows(int m, int n, int k, long g) {
+  return m >= 2 && n >= 2048 && k >= 2048 &&
+         (k <= 4096 || n >= 8192 || (n >= 5120 && k <= 8192)) &&
+         lfmq_dq_wide_ok(m, n, k, (int)g);
+}
+
 torch::Tensor rmsnorm(torch::Tensor x, torch::Tensor w, double eps,
                       c10::optional<torch::Tensor> residual);
 torch::Tensor silu_mul_fused(torch::Tensor gate_up);
@@ -211,6 +230,11 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
                           qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                           rptr, n, k, (int)g, (int)bits, (float)rms_eps, false,
                           stream()));
+  } else if (cols_hint == 0 && wide_rows(m, n, k, g)) {
+    CHECK_HIP(lfmq_dq_wide(qweight.data_ptr(), scales.data_ptr(),
+                           qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
+                           rptr, m, n, k, (int)g, (int)bits, (float)rms_eps,
+                           false, stream()));
   } else if (by_rows) {
     const int splits = rms ? 1 : lfmq_dq_rows_splits(m, n, k, (int)g);
     CHECK_HIP(lfmq_dq_rows(qweight.data_ptr(), scales.data_ptr(),
@@ -409,12 +433,19 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
                            (int)g, (int)bits, splits, true, stream()));
     return y;
   }
-  if (cols_hint == 0 && n % 2 == 0 && m == 1 && lfmq_dq_row_ok(n, k, (int)g)) {
+  if (cols_hint == 0 && n % 2 == 0 &&
+      (m == 1 ? lfmq_dq_row_ok(n, k, (int)g) : wide_rows(m, n, k, g))) {
     if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
-    CHECK_HIP(lfmq_dq_row(qweight.data_ptr(), scales.data_ptr(),
-                          qzeros.data_ptr(), x.data_ptr(), y.data_ptr(),
-                          nullptr, nullptr, n, k, (int)g, (int)bits,
-                          (float)rms_eps, true, stream()));
+    if (m == 1)
+      CHECK_HIP(lfmq_dq_row(qweight.data_ptr(), scales.data_ptr(),
+                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(),
+                            nullptr, nullptr, n, k, (int)g, (int)bits,
+                            (float)rms_eps, true, stream()));
+    else
+      CHECK_HIP(lfmq_dq_wide(qweight.data_ptr(), scales.data_ptr(),
+                             qzeros.data_ptr(), x.data_ptr(), y.data_ptr(),
+                             nullptr, nullptr, m, n, k, (int)g, (int)bits,
+                             (float)rms_eps, true, stream()));
     return y;
   }
   if (cols_hint == 0 && m >= rows_from(bits, n, k, g) && m <= 48 &&
@@ -503,13 +534,22 @@ std::vector<torch::Tensor> moe_route(torch::Tensor logits, long topk) {
   return {src_tok, slot_w, offsets, active};
 }
 
+// Tiles of 16 rows of the grouped products that keep x and walk over columns.
+bool wide_experts(int n, int k, long g) {
+  return n >= 2048 && k >= 2048 && lfmq_dq_wide_ok(16, n, k, (int)g);
+}
+
 // Rows a tile of the grouped products for `slots` rows over E experts.  us of
-// a layer of 8 experts (4096, 14336, 4 bits) with 16 / 128: 280 / 377 at 12
-// rows an expert, 418 / 397 at 16, 669 / 403 at 32.
+// a layer of 8 experts (4096, 14336, 4 bits) with 16 / 128: 224 / 364 at 14
+// rows an expert, 330 / 368 at 24, 399 / 369 at 32 (2048, 8192: 123 / 150 at
+// 32, 155 / 150 at 48); 418 / 397 at 16 where tiles of 16 are dq_rows'.
 long moe_tile(long slots, long E, long k_in, long g_in, long k_out,
               long g_out) {
   TORCH_CHECK(g_in > 0 && g_out > 0, "groups have at least one column");
-  return slots > 14 * E && lfmq_dq_tile_ok((int)k_in, (int)g_in) &&
+  // (the first product has 2 k_out columns, the second k_in)
+  const bool wide = wide_experts(2048, (int)k_in, g_in) && k_out >= 1024;
+  return slots > (wide ? 26 : 14) * E &&
+                 lfmq_dq_tile_ok((int)k_in, (int)g_in) &&
                  lfmq_dq_tile_ok((int)k_out, (int)g_out)
              ? 128
              : 16;
@@ -566,6 +606,11 @@ torch::Tensor moe_linear(torch::Tensor x, c10::optional<torch::Tensor> src,
   if (nt == 0) return y;
   if (bm == 128)
     CHECK_HIP(lfmq_dq_tile_experts(
+        qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
+        sptr, tiles.data_ptr(), y.data_ptr(), nt, n, k, (int)g, (int)bits, glu,
+        stream()));
+  else if (wide_experts(n, k, g))
+    CHECK_HIP(lfmq_dq_wide_experts(
         qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
         sptr, tiles.data_ptr(), y.data_ptr(), nt, n, k, (int)g, (int)bits, glu,
         stream()));

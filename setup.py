@@ -31,6 +31,7 @@ SOURCES = [
     "csrc/elementwise.hip",
     "csrc/dq_gemv.hip",
     "csrc/dq_row.hip",
+    "csrc/dq_wide.hip",
     "csrc/dq_rows.hip",
     "csrc/dq_tile.hip",
     "csrc/hessian.hip",

@@ -75,3 +75,40 @@ def test_one_row(bits, n, k, g):
     group of four, gates inside a pair; several groups a wave."""
     torch.manual_seed(n)
     check(bits, 1, n, k, g)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,n,k,g", [
+    (2, 2049, 2048, 128), (3, 3074, 2304, 64), (4, 4098, 4096, 128),
+    (5, 2050, 2048, 64), (8, 28674, 4096, 128), (9, 8198, 4352, 128),
+    (12, 33000, 2048, 128), (16, 5126, 8192, 64), (16, 4110, 4096, 64)])
+def test_few_rows_many_columns(bits, m, n, k, g):
+    """Eight and sixteen waves along k, one and more steps of it; tiles that
+    end inside a workgroup's last one; 4, 8 and 16 rows of sums."""
+    torch.manual_seed(n)
+    check(bits, m, n, k, g)
+
+
+@pytest.mark.parametrize("bits,n,k,g", [(4, 2062, 2048, 128),
+                                        (8, 2048, 4352, 64),
+                                        (4, 4100, 4096, 128)])
+@pytest.mark.parametrize("counts", [(1, 0, 2), (16, 3, 0), (0, 21, 9)])
+def test_rows_by_expert(bits, n, k, g, counts):
+    """One to sixteen rows a tile, experts without any, tiles that are none."""
+    torch.manual_seed(n)
+    p, w = matrix(bits, n, k, g, (len(counts),))
+    ids = torch.tensor([e for e, c in enumerate(counts) for _ in range(c)],
+                       device=DEV)
+    src = torch.randperm(len(ids)).to(DEV)
+    x = torch.randn(len(ids), k, device=DEV).to(BF)
+    tiles, at = [], 0
+    for e, c in enumerate(counts):
+        tiles += [(e, at + i, min(16, c - i)) for i in range(0, c, 16)]
+        at += c
+    tiles.insert(1, (-1, 0, 0))
+    tiles = torch.tensor(tiles + [(-1, 0, 0)], dtype=torch.int32, device=DEV)
+    want = (x.double()[src].unsqueeze(1) @ w[ids].transpose(1, 2)).squeeze(1)
+    s32 = src.to(torch.int32)
+    close(ext().moe_linear(x, s32, tiles, *p, bits, g, True, 16), gated(want),
+          1e-2)
+    close(ext().moe_linear(x[src], None, tiles, *p, bits, g, False, 16), want)
