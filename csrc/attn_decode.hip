@@ -20,25 +20,30 @@
 // scratch, and the last workgroup of the head to arrive merges them (a
 // ticket counter) or, without tickets, a second kernel does.
 //
-// One layer of an 8B model (32 query heads on 8), one kernel, against a
-// workgroup a query head and 64 keys:
-//   b 1,  T 129       8.4 us (10.3)
-//   b 1,  T 7901     20.2 us (199)
-//   b 8,  T 1000     20.4 us (165)
-//   b 48, T 2047     117 us (2157), 3.4 TB/s
+// A launch that only reads 402 MB takes 66 us, one of 33 MB 6.5: the rest is a
+// chain from the length over the rotation to the keys, sums over the lanes, and
+// the merge's trips to memory.  One layer of an 8B model (32 query heads on 8),
+// us before and now (tickets that emptied the XCD's caches, two waves a SIMD,
+// ranges of 256 keys):
+//   b 1,  T 129        8.9 ->  8.2      b 8,  T 4000     66   -> 31
+//   b 1,  T 7901      21.4 -> 16.8      b 20, T 900      46   -> 21.8
+//   b 8,  T 1000      20.8 -> 14.3      b 48, T 2047    114   -> 77 (5.2 TB/s)
 #include "common.h"
 
 namespace {
 
 constexpr int TPB = 256, NW = 4, KT = 32;
 constexpr int MAX_SPLITS = 64;       // a wave merges them, one a lane
-// Two rounds of a wave's 32 keys cost 1.6 us more than one, a merge 4 us:
-// ranges of 128 / 256 / 512 keys take 10.0 / 8.4 / 8.4 us at 129 keys,
-// 13.4 / 13.6 / 17.2 at 2000, 23.7 / 20.2 / 19.1 at 7901 (b 1).
-constexpr int LEAST_KEYS = 256;
-// No more workgroups than are resident at once: 384 heads in 2 / 3 / 6
-// ranges take 117 / 143 / 199 us (b 48, 2047 keys).
-constexpr int FULL_WGS = 1024;
+// A merge costs 2 us, two rounds of a wave's 32 keys 1.5 more than one.  Up to
+// ONE_RANGE keys are one range; longer ranges than LEAST_KEYS where there would
+// be more than MANY of them.  us with least ranges of 128 / 256 keys (b 1): 9.2
+// / 8.2 at 129 keys, 9.7 / 11.3 at 700, 11.2 / 11.9 at 2000; 21.8 / 16.8 at
+// 7901, 62 and 31 ranges.
+constexpr int ONE_RANGE = 256, LEAST_KEYS = 128, MANY = 32;
+// Two workgroups a CU, three where a range has very many keys: us with 512 / 768
+// workgroups 14.3 / 15.2 (b 8, 1000 keys), 18.4 / 19.2 (b 16, 900), 81.5 / 77
+// (b 48, 2047).
+constexpr int FULL_WGS = 512, MORE_WGS = 768, LONG_RANGE = 1024;
 
 struct DArgs {
   const unsigned short* q;           // [b, hq, D], or [b, (hq + 2 hkv) D]
@@ -48,29 +53,64 @@ struct DArgs {
   const float* inv_freq;
   const i32* T_dev;
   u32* tickets;                      // [b * hkv * head tiles], zero
-  int hq, hkv, tmax, T, splits, least;
+  int hq, hkv, tmax, T, splits;
   float scale;
+  int group, htiles;                 // hq / hkv, workgroups a key/value head
+  u32 inv_splits;                    // 2^32 / splits, rounded up
 };
 
-// keys a range: all ranges alike, whole wave tiles, not below `least`
-__device__ __forceinline__ int range_keys(int T, int splits, int least) {
-  const int per = max((T + splits - 1) / splits, least);
-  return (per + KT - 1) / KT * KT;
+// keys a range: all ranges alike, whole wave tiles
+__device__ __forceinline__ int range_keys(const DArgs& A, int len) {
+  // (len + splits - 1) / splits, exact below 2^26 keys
+  const int per = A.splits == 1 ? len
+                                : (int)(((u64)(u32)(len + A.splits - 1) *
+                                         A.inv_splits) >> 32);
+  const int least = len <= ONE_RANGE ? ONE_RANGE : LEAST_KEYS;
+  return (max(per, least) + KT - 1) / KT * KT;
+}
+
+// the other half's value, or the other 16 lanes' of this half
+__device__ __forceinline__ float max_across(float v) {
+  const u32 x = __builtin_bit_cast(u32, v);
+  const auto p = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  const u32 p0 = p[0], p1 = p[1];
+  const u32 y = __builtin_bit_cast(u32, fmaxf(__builtin_bit_cast(float, p0),
+                                              __builtin_bit_cast(float, p1)));
+  const auto q = __builtin_amdgcn_permlane16_swap(y, y, false, false);
+  const u32 q0 = q[0], q1 = q[1];
+  return fmaxf(__builtin_bit_cast(float, q0), __builtin_bit_cast(float, q1));
+}
+
+// Two floats of a partial result, past the caches of the XCD: a workgroup of
+// another one may be the reader.
+__device__ __forceinline__ void put2(float* p, float a, float b) {
+  typedef __attribute__((address_space(1))) u64 gu64;
+  __hip_atomic_store((gu64*)p,
+                     (u64)__builtin_bit_cast(u32, b) << 32 |
+                         __builtin_bit_cast(u32, a),
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void get2(const float* p, float& a, float& b) {
+  typedef __attribute__((address_space(1))) u64 gu64;
+  const u64 v = __hip_atomic_load((gu64*)p, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+  a = __builtin_bit_cast(float, (u32)v);
+  b = __builtin_bit_cast(float, (u32)(v >> 32));
 }
 
 // weights of `used` partial results of one head: lane c holds range c's
 __device__ __forceinline__ float merge_weight(const float* p, int used,
                                               int stride, int D, int lane) {
   const bool on = lane < used;
-  const float m = on ? p[lane * stride + D] : -INFINITY;
-  const float l = on ? p[lane * stride + D + 1] : 0.f;
+  float m = -INFINITY, l = 0.f;
+  if (on) get2(p + lane * stride + D, m, l);
   const float M = wave_reduce_max(m);
   const float e = on ? __expf(m - M) : 0.f;
   return e / wave_reduce_sum(e * l);
 }
 
 template <int D, int GH, bool FUSED>
-__global__ __launch_bounds__(TPB) void attn_decode_kernel(DArgs A) {
+__global__ __launch_bounds__(TPB, D * GH > 512 ? 2 : 3) void attn_decode_kernel(DArgs A) {
   constexpr int KS = D / 32, LPR = D / 8;
   constexpr int RPP = 64 / LPR;          // value rows a pass
   constexpr int NP = KT / RPP;           // passes a tile
@@ -82,37 +122,49 @@ __global__ __launch_bounds__(TPB) void attn_decode_kernel(DArgs A) {
   __shared__ float s_new[GH];            // FUSED: scores of the new key
 
   const int T = A.T_dev != nullptr ? *A.T_dev : A.T;
-  const int group = A.hq / A.hkv, htiles = (group + GH - 1) / GH;
-  const int kh = blockIdx.y / htiles, ht = blockIdx.y % htiles;
+  const int group = A.group, htiles = A.htiles;
+  const int kh = htiles == 1 ? blockIdx.y : blockIdx.y / htiles;
+  const int ht = htiles == 1 ? 0 : blockIdx.y % htiles;
   const int bb = blockIdx.z;
   const int h0 = kh * group + ht * GH;             // first query head
   const int nh = min(GH, group - ht * GH);
-  const int len = min(T, A.tmax);
-  const int per = range_keys(len, A.splits, A.least);
-  const int used = (len + per - 1) / per;
-  const int lo = blockIdx.x * per, hi = min(len, lo + per);
-  if (lo >= hi) return;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int l15 = lane & 15, l4 = lane >> 4;
   const int vrow = lane / LPR, vcol = (lane % LPR) * 8;
-  unsigned short* K = A.kc + ((u64)bb * A.hkv + kh) * A.tmax * D;
-  unsigned short* V = A.vc + ((u64)bb * A.hkv + kh) * A.tmax * D;
   const s16x8 z8 = {0, 0, 0, 0, 0, 0, 0, 0};
 
   s16x8 qf[KS];
   u32x4 v_new = {0, 0, 0, 0};
-  const int pos = FUSED ? T - 1 : -1;    // the new key
+  // what does not depend on the number of keys is on its way with it: a wave
+  // rotates heads wave, wave + 4, one angle a lane
+  constexpr int QW = (GH + NW - 1) / NW;
+  float freq, k1, k2, q1[QW], q2[QW];
+  const int i = lane & (D / 2 - 1);
   if constexpr (FUSED) {
     const unsigned short* row = A.q + (u64)bb * (A.hq + 2 * A.hkv) * D;
     const unsigned short* kr = row + (u64)(A.hq + kh) * D;
-    const unsigned short* vr = row + (u64)(A.hq + A.hkv + kh) * D;
-    v_new = *(const u32x4*)(vr + vcol);
-    // a wave rotates heads wave, wave + 4, ..: one angle a lane
-    const int i = lane & (D / 2 - 1);
+    v_new = *(const u32x4*)(row + (u64)(A.hq + A.hkv + kh) * D + vcol);
+    freq = A.inv_freq[i];
+    k1 = bf16_bits_to_f32(kr[i]);
+    k2 = bf16_bits_to_f32(kr[i + D / 2]);
+#pragma unroll
+    for (int g = 0; g < QW; ++g) {
+      const unsigned short* qr =
+          row + (u64)(h0 + min(wave + g * NW, nh - 1)) * D;
+      q1[g] = bf16_bits_to_f32(qr[i]);
+      q2[g] = bf16_bits_to_f32(qr[i + D / 2]);
+    }
+  }
+  const int len = min(T, A.tmax);
+  const int per = range_keys(A, len);
+  const int lo = blockIdx.x * per, hi = min(len, lo + per);
+  if (lo >= hi) return;
+  unsigned short* K = A.kc + ((u64)bb * A.hkv + kh) * A.tmax * D;
+  unsigned short* V = A.vc + ((u64)bb * A.hkv + kh) * A.tmax * D;
+  const int pos = FUSED ? T - 1 : -1;    // the new key
+  if constexpr (FUSED) {
     float sn, cs;
-    __sincosf((float)pos * A.inv_freq[i], &sn, &cs);
-    const float k1 = bf16_bits_to_f32(kr[i]);
-    const float k2 = bf16_bits_to_f32(kr[i + D / 2]);
+    __sincosf((float)pos * freq, &sn, &cs);
     const float ka = k1 * cs - k2 * sn, kb = k1 * sn + k2 * cs;
     if (blockIdx.x == 0 && ht == 0 && wave == 0 && pos < A.tmax) {
       if (lane < D / 2) {
@@ -121,16 +173,17 @@ __global__ __launch_bounds__(TPB) void attn_decode_kernel(DArgs A) {
       }
       if (vrow == 0) *(u32x4*)(V + (u64)pos * D + vcol) = v_new;
     }
-    for (int g = wave; g < nh; g += NW) {
-      const unsigned short* qr = row + (u64)(h0 + g) * D;
-      const float q1 = bf16_bits_to_f32(qr[i]);
-      const float q2 = bf16_bits_to_f32(qr[i + D / 2]);
-      const float qa = q1 * cs - q2 * sn, qb = q1 * sn + q2 * cs;
+#pragma unroll
+    for (int j = 0; j < QW; ++j) {
+      const int g = wave + j * NW;
+      if (g >= nh) break;
+      const float qa = q1[j] * cs - q2[j] * sn, qb = q1[j] * sn + q2[j] * cs;
       if (lane < D / 2) {
         qs[g][i] = (unsigned short)f32_to_bf16_bits_rne(qa);
         qs[g][i + D / 2] = (unsigned short)f32_to_bf16_bits_rne(qb);
       }
-      const float s = wave_reduce_sum(lane < D / 2 ? qa * ka + qb * kb : 0.f);
+      const float s =
+          wave_reduce_sum_dpp(lane < D / 2 ? qa * ka + qb * kb : 0.f);
       if (lane == 0) s_new[g] = s;
     }
     __syncthreads();
@@ -179,9 +232,7 @@ __global__ __launch_bounds__(TPB) void attn_decode_kernel(DArgs A) {
         sc[mt][r] = t < hi ? s * A.scale : -INFINITY;
         mx = fmaxf(mx, sc[mt][r]);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float mn = fmaxf(m, mx);             // a tile has a visible key
+    const float mn = fmaxf(m, max_across(mx));  // a tile has a visible key
     const float al = __expf(m - mn);
     float sum = 0.f;
 #pragma unroll
@@ -192,9 +243,7 @@ __global__ __launch_bounds__(TPB) void attn_decode_kernel(DArgs A) {
         sum += p;
         if (l15 < GH) ps[wave][mt * 16 + l4 * 4 + r][l15] = p;
       }
-    sum += __shfl_xor(sum, 16, 64);
-    sum += __shfl_xor(sum, 32, 64);
-    l = l * al + sum;
+    l = l * al + sum;                          // this lane's keys only
     m = mn;
     if (lane < GH) al_s[wave][lane] = al;
     // wave-local slabs: LDS operations of a wave retire in order
@@ -230,7 +279,9 @@ __global__ __launch_bounds__(TPB) void attn_decode_kernel(DArgs A) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // ps is read
   }
 
-  // rows of one wave, then the waves
+  // lanes and rows of one wave, then the waves
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
 #pragma unroll
   for (int h = 0; h < GH; ++h)
 #pragma unroll
@@ -245,6 +296,7 @@ __global__ __launch_bounds__(TPB) void attn_decode_kernel(DArgs A) {
     ml[wave][lane][1] = l;
   }
   __syncthreads();
+  const int used = (len + per - 1) / per;
   float* part = A.part + (((u64)bb * A.hq + h0) * A.splits + blockIdx.x) *
                              (D + 2);
   const int hstep = A.splits * (D + 2);
@@ -266,32 +318,27 @@ __global__ __launch_bounds__(TPB) void attn_decode_kernel(DArgs A) {
       continue;
     }
     // written through to where the merging workgroup reads
-    typedef __attribute__((address_space(1))) float gfloat;
     float* p = part + (u64)h * hstep;
-    __hip_atomic_store((gfloat*)(p + e), o0, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store((gfloat*)(p + e + 1), o1, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-    if (e == 0) {
-      __hip_atomic_store((gfloat*)(p + D), M, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store((gfloat*)(p + D + 1), L, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    }
+    put2(p + e, o0, o1);
+    if (e == 0) put2(p + D, M, L);
   }
   if (used == 1 || A.tickets == nullptr) return;
 
-  // the last to arrive merges.  vmcnt is a per-wave counter: every wave
-  // drains its own stores, and the barrier orders all of them before the
-  // ticket.  The merging workgroup puts the ticket back to zero, so a
-  // replayed graph finds it as the first launch did.
+  // The last to arrive merges.  vmcnt is a per-wave counter: every wave
+  // drains its own stores, which are past the XCDs' caches when they are done,
+  // and the barrier orders all of them before the ticket; the merging workgroup
+  // reads past its caches, too.  So the ticket orders nothing: as a release and
+  // acquire it writes back and empties an XCD's L2, once for each of these
+  // workgroups (48 x 300 keys, 384 of them: 58 us).  The merging workgroup
+  // puts the ticket back to zero, so a replayed graph finds it as the first
+  // launch did.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   __shared__ int last_s;
   typedef __attribute__((address_space(1))) unsigned gu32;
   gu32* ticket = (gu32*)(A.tickets + (u64)bb * gridDim.y + blockIdx.y);
   if (tid == 0) {
-    const unsigned old = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL,
+    const unsigned old = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED,
                                                 __HIP_MEMORY_SCOPE_AGENT);
     last_s = (int)old == used - 1;
     if (last_s)
@@ -300,23 +347,37 @@ __global__ __launch_bounds__(TPB) void attn_decode_kernel(DArgs A) {
   }
   __syncthreads();
   if (!last_s) return;
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  // the first results of a thread are on their way with the weights
   const float* head = A.part + ((u64)bb * A.hq + h0) * hstep;
+  constexpr int AT = 32;                             // ranges at a time
+  float r0[AT], r1[AT];
+  auto fetch = [&](int id, int c0) {
+    const float* p = head + (u64)(id / (D / 2)) * hstep + id % (D / 2) * 2;
+#pragma unroll
+    for (int c = 0; c < AT; ++c)
+      if (c0 + c < used) get2(p + (c0 + c) * (D + 2), r0[c], r1[c]);
+  };
+  const int ids = nh * (D / 2);
+  if (tid < ids) fetch(tid, 0);
   float(*wt)[GH] = (float(*)[GH])&ps[0][0][0];       // [MAX_SPLITS][GH]
   static_assert(MAX_SPLITS <= NW * KT, "weights fit the slab");
   for (int g = wave; g < nh; g += NW)
     wt[lane][g] = merge_weight(head + (u64)g * hstep, used, D + 2, D, lane);
   __syncthreads();
-  for (int id = tid; id < nh * (D / 2); id += TPB) {
-    const int h = id / (D / 2), e = id % (D / 2) * 2;
-    const float* p = head + (u64)h * hstep + e;
+  for (int id = tid; id < ids; id += TPB) {
+    const int h = id / (D / 2);
     float a0 = 0.f, a1 = 0.f;
-#pragma unroll 8
-    for (int c = 0; c < used; ++c) {
-      a0 = fmaf(wt[c][h], p[c * (D + 2)], a0);
-      a1 = fmaf(wt[c][h], p[c * (D + 2) + 1], a1);
+    for (int c0 = 0; c0 < used; c0 += AT) {
+      if (id != tid || c0 > 0) fetch(id, c0);
+#pragma unroll
+      for (int c = 0; c < AT; ++c)
+        if (c0 + c < used) {
+          a0 = fmaf(wt[c0 + c][h], r0[c], a0);
+          a1 = fmaf(wt[c0 + c][h], r1[c], a1);
+        }
     }
-    A.o[((u64)bb * A.hq + h0 + h) * (D / 2) + e / 2] = pack_bf16x2(a0, a1);
+    A.o[((u64)bb * A.hq + h0 + h) * (D / 2) + id % (D / 2)] =
+        pack_bf16x2(a0, a1);
   }
 }
 
@@ -324,7 +385,7 @@ __global__ __launch_bounds__(TPB) void attn_decode_kernel(DArgs A) {
 template <int D>
 __global__ __launch_bounds__(64) void attn_decode_merge(DArgs A) {
   const int len = min(A.T_dev != nullptr ? *A.T_dev : A.T, A.tmax);
-  const int per = range_keys(len, A.splits, A.least);
+  const int per = range_keys(A, len);
   const int used = (len + per - 1) / per;
   if (used <= 1) return;
   __shared__ float wt[MAX_SPLITS];
@@ -348,9 +409,12 @@ int head_tile(int group) {
 }
 
 template <int D, bool FUSED>
-hipError_t launch(const DArgs& A, int b, hipStream_t stream) {
+hipError_t launch(DArgs A, int b, hipStream_t stream) {
   const int group = A.hq / A.hkv, gh = head_tile(group);
-  const dim3 grid(A.splits, A.hkv * ((group + gh - 1) / gh), b);
+  A.group = group;
+  A.htiles = (group + gh - 1) / gh;
+  A.inv_splits = (u32)(((1ull << 32) + A.splits - 1) / A.splits);
+  const dim3 grid(A.splits, A.hkv * A.htiles, b);
 #define GO(G)                                                               \
   hipLaunchKernelGGL((attn_decode_kernel<D, G, FUSED>), grid, dim3(TPB), 0, \
                      stream, A)
@@ -371,8 +435,10 @@ hipError_t launch(const DArgs& A, int b, hipStream_t stream) {
 int lfmq_attn_decode_splits(int b, int hq, int hkv, int T) {
   const int group = hq / hkv, gh = head_tile(group);
   const int wgs = b * hkv * ((group + gh - 1) / gh);
-  const int n = FULL_WGS / max(wgs, 1);
-  const int most = (T + LEAST_KEYS - 1) / LEAST_KEYS;
+  int n = FULL_WGS / max(wgs, 1);
+  if (T > max(n, 1) * LONG_RANGE) n = MORE_WGS / max(wgs, 1);
+  const int most = max(min((T + LEAST_KEYS - 1) / LEAST_KEYS, MANY),
+                       (T + 2 * LEAST_KEYS - 1) / (2 * LEAST_KEYS));
   return max(1, min(min(n, most), MAX_SPLITS));
 }
 
@@ -387,7 +453,7 @@ hipError_t lfmq_attn_decode(const void* q, const void* kc, const void* vc,
   const DArgs A{(const unsigned short*)q, (unsigned short*)kc,
                 (unsigned short*)vc, (float*)scratch, (u32*)o, nullptr,
                 (const i32*)T_dev, nullptr, hq, hkv, tmax, T, splits,
-                LEAST_KEYS, scale};
+                scale, 0, 0, 0};
   return d == 128 ? launch<128, false>(A, b, stream)
                   : launch<64, false>(A, b, stream);
 }
@@ -406,7 +472,7 @@ hipError_t lfmq_attn_decode_fused(const void* qkv, void* kc, void* vc,
   const DArgs A{(const unsigned short*)qkv, (unsigned short*)kc,
                 (unsigned short*)vc, (float*)scratch, (u32*)o,
                 (const float*)inv_freq, (const i32*)T_dev, (u32*)tickets, hq,
-                hkv, tmax, T, splits, LEAST_KEYS, scale};
+                hkv, tmax, T, splits, scale, 0, 0, 0};
   return d == 128 ? launch<128, true>(A, b, stream)
                   : launch<64, true>(A, b, stream);
 }
