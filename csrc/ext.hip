@@ -60,6 +60,8 @@ hipError_t lfmq_chol_inverse(const void*, void*, void*, void*, void*, void*,
 hipError_t lfmq_gptq_block(const void*, const void*, int, void*, void*, void*,
                            void*, int, int, int, int, int, int, int, bool,
                            hipStream_t);
+hipError_t lfmq_gptq_push(const void*, const void*, const void*, long, int, int,
+                          int, int, hipStream_t);
 hipError_t lfmq_dq_gemv_gateup(const void*, const void*, const void*,
                                const void*, void*, int, int, int, int, int,
                                float, int, hipStream_t);
@@ -852,6 +854,23 @@ torch::Tensor gptq_block(torch::Tensor w, torch::Tensor ub,
   return err;
 }
 
+// w[:, i1 + nb:] -= err U[i1:i1 + nb, i1 + nb:]
+void gptq_push(torch::Tensor w, torch::Tensor err, torch::Tensor u, long i1) {
+  check_t(w, torch::kFloat32, "w");
+  check_t(err, torch::kFloat32, "err");
+  TORCH_CHECK(w.dim() == 2 && err.dim() == 2 && err.size(0) == w.size(0),
+              "w [n, k], err [n, nb]");
+  const long n = w.size(0), k = w.size(1), nb = err.size(1);
+  TORCH_CHECK(u.is_cuda() && u.scalar_type() == torch::kFloat32 &&
+                  u.dim() == 2 && u.size(0) == k && u.size(1) == k &&
+                  u.stride(1) == 1 && u.stride(0) >= k,
+              "u must be [k, k], rows of fp32 on GPU");
+  TORCH_CHECK(i1 >= 0 && i1 + nb <= k, "block past the last column");
+  CHECK_HIP(lfmq_gptq_push(w.data_ptr(), err.data_ptr(),
+                           u.data_ptr<float>() + i1 * u.stride(0), u.stride(0),
+                           (int)n, (int)k, (int)(i1 + nb), (int)nb, stream()));
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -871,6 +890,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("hessian_accum", &hessian_accum, "H += 2 X^T X");
   m.def("chol_inverse", &chol_inverse,
         "upper Cholesky factor of the inverse, and whether there is none");
+  m.def("gptq_push", &gptq_push, "a GPTQ block's errors to later columns");
   m.def("gptq_block", &gptq_block, "one column block of the GPTQ solve");
   m.def("dq_gemv_gateup", &dq_gemv_gateup, "fused gate_up GEMV + silu*mul");
   m.def("qkv_rope_append", &qkv_rope_append, "fused rope + KV append");

@@ -95,6 +95,14 @@ def _gpu_block(w, ub, codes, scales, zeros, i1, cfg, g) -> torch.Tensor:
                                     cfg.bits, cfg.sym)
 
 
+def _gpu_push(w, err, U, i1) -> None:
+    """The columns behind the block from i1 on take over its errors
+    (csrc/gptq_block.hip)."""
+    from ..ops import hip_ext
+    with torch.cuda.device(w.device):
+        hip_ext().gptq_push(w, err, U, i1)
+
+
 @torch.no_grad()
 def gptq_quantize_layer(
     w: torch.Tensor, h: torch.Tensor, cfg: QuantConfig
@@ -134,11 +142,16 @@ def gptq_quantize_layer(
     scales = torch.zeros(n, G, dtype=torch.float32, device=dev)
     zeros = torch.zeros(n, G, dtype=torch.int32, device=dev)
 
-    block = _gpu_block if w.is_cuda and cfg.block_size <= GPU_BLOCK else _block
+    on_gpu = w.is_cuda and cfg.block_size <= GPU_BLOCK
+    block = _gpu_block if on_gpu else _block
+    if on_gpu and U.stride(1) != 1:        # the library's factor
+        U = U.contiguous()
     for i1 in range(0, k, cfg.block_size):
         i2 = min(i1 + cfg.block_size, k)
         err = block(w, U[i1:i2, i1:i2], codes, scales, zeros, i1, cfg, g)
-        if i2 < k:
+        if i2 < k and on_gpu:
+            _gpu_push(w, err, U, i1)
+        elif i2 < k:
             # in one pass over w, of the products' sums in fp32
             w[:, i2:].addmm_(err, U[i1:i2, i2:], alpha=-1)
 
