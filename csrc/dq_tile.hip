@@ -1,5 +1,5 @@
 // K3b/K4b — W4A16 / W8A16 product for prompts: y[m, n] = x[m, k] ·
-// dequant(W)[n, k]^T (+ bias).
+// dequant(W)[n, k]^T (+ bias).  Few rows, and groups that dq_block does not take.
 //
 // A workgroup computes 128 rows by 128 columns, four waves side by side in
 // the columns, each all 128 rows by 32 columns.  x goes through LDS (two

@@ -85,6 +85,7 @@ hipError_t lfmq_argmax_rows(const void*, void*, void*, void*, int, int,
                             hipStream_t);
 hipError_t lfmq_read_probe(const void*, void*, long, long, int, int, int,
                            hipStream_t);
+#include "dq_block.h"
 #include "engine_args.h"
 
 namespace {
@@ -151,6 +152,35 @@ bool wide_rows(int m, int n, int k, long g) {
   return m >= 2 && n >= 2048 && k >= 2048 &&
          (k <= 4096 || n >= 8192 || (n >= 5120 && k <= 8192)) &&
          lfmq_dq_wide_ok(m, n, k, (int)g);
+}
+
+// The product for many rows: tiles of 256 columns instead of 128.  us of
+// dq_tile / dq_block, 4 bits, k 4096: n 28672 38.5 / 34.3 at 49 rows, 438 / 368 at
+// 1500; n 6144 17.3 / 18.4 at 49, 22.0 / 20.5 at 77, 117.6 / 90.2 at 1500; n 4096,
+// k 14336 24.7 / 24.9 at 49, 30.4 / 28.7 at 77.  8 bits, groups of 64: n 16384, k
+// 2048 22.5 / 21.5 at 49; n 2048, k 8192 23.1 / 23.5 at 77, 25.4 / 24.7 at 120.  8
+// bits in groups of 128, n 32000, k 4096: 64.1 / 65.4 at 120, 96.4 / 93.0 at 200,
+// 535 / 495 at 1500.
+bool block_rows(const torch::Tensor& qweight, const torch::Tensor& scales,
+                long m, long n, long k, long g, long bits) {
+  return (m > (bits == 4 ? 64 : 96) || n * k >= 32l << 20) &&
+         (m > 128 || bits == 4 || g % 128 != 0) &&
+         lfmq_dq_block_ok(qweight.data_ptr(), scales.data_ptr(), n, k, g, bits);
+}
+
+void dq_block(const torch::Tensor& x, const torch::Tensor& qweight,
+              const torch::Tensor& scales, const torch::Tensor& qzeros,
+              const void* bias, torch::Tensor& y, long g, long bits, bool glu) {
+  const int m = (int)x.size(0), k = (int)x.size(1), n = (int)qweight.size(0);
+  const DqBlockPlan P =
+      lfmq_dq_block_plan(m, n, k, (int)g, (int)bits, glu);
+  torch::Tensor part;
+  if (P.part > 0)
+    part = torch::empty({P.part}, x.options().dtype(torch::kFloat32));
+  CHECK_HIP(lfmq_dq_block(qweight.data_ptr(), scales.data_ptr(),
+                          qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bias,
+                          P.part > 0 ? part.data_ptr() : nullptr, m, n, k,
+                          (int)g, (int)bits, glu, P, stream()));
 }
 
 torch::Tensor rmsnorm(torch::Tensor x, torch::Tensor w, double eps,
@@ -248,6 +278,9 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                            rptr, m, n, k, (int)g, (int)bits, (float)rms_eps,
                            (int)cols_hint, stream()));
+  } else if (rptr == nullptr &&
+             block_rows(qweight, scales, m, n, k, g, bits)) {
+    dq_block(x, qweight, scales, qzeros, bptr, y, g, bits, false);
   } else {
     const int splits = lfmq_dq_tile_splits(m, n, k, (int)g);
     CHECK_HIP(lfmq_dq_tile(qweight.data_ptr(), scales.data_ptr(),
@@ -423,6 +456,10 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
       lfmq_dq_tile_ok(k, (int)g)) {
     TORCH_CHECK(rms_eps < 0, "fused rms is a decode (m <= 48) path");
     if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
+    if (block_rows(qweight, scales, m, n, k, g, bits)) {
+      dq_block(x, qweight, scales, qzeros, nullptr, y, g, bits, true);
+      return y;
+    }
     const int splits = lfmq_dq_tile_splits(m, n, k, (int)g);
     torch::Tensor part;
     if (splits > 1)
@@ -606,7 +643,13 @@ torch::Tensor moe_linear(torch::Tensor x, c10::optional<torch::Tensor> src,
   TORCH_CHECK(bm == 16 || bm == 128, "tiles of 16 or 128 rows");
   const int nt = (int)tiles.size(0);
   if (nt == 0) return y;
-  if (bm == 128)
+  if (bm == 128 && lfmq_dq_block_ok(qweight.data_ptr(), scales.data_ptr(), n, k,
+                                    g, bits))
+    CHECK_HIP(lfmq_dq_block_experts(
+        qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
+        sptr, tiles.data_ptr(), y.data_ptr(), nt, n, k, (int)g, (int)bits, glu,
+        stream()));
+  else if (bm == 128)
     CHECK_HIP(lfmq_dq_tile_experts(
         qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
         sptr, tiles.data_ptr(), y.data_ptr(), nt, n, k, (int)g, (int)bits, glu,

@@ -34,6 +34,7 @@ SOURCES = [
     "csrc/dq_wide.hip",
     "csrc/dq_rows.hip",
     "csrc/dq_tile.hip",
+    "csrc/dq_block.hip",
     "csrc/hessian.hip",
     "csrc/gptq_block.hip",
     "csrc/chol_inverse.hip",

@@ -1,0 +1,66 @@
+"""Packed products of a prompt against 64 bits (dq_block), where its row tiles,
+column blocks, stages and parts end.  Tolerances: test_gpu_decode_products."""
+import pytest
+import torch
+
+from lfmq.ops import hip_ext as ext
+from test_gpu_decode_products import BF, DEV, close, gated, matrix
+
+pytestmark = pytest.mark.gpu
+
+
+# One to three row tiles of 64 to 128, also of sizes in between; column blocks
+# that end inside a wave's columns, or between pieces of 16 bytes; one group a
+# chunk and several; four chunks up, whole, split, and some tiles split.
+@pytest.mark.parametrize("bits,m,n,k,g", [
+    (4, 65, 264, 1024, 128), (4, 97, 1041, 2048, 128), (4, 128, 520, 1024, 64),
+    (4, 129, 2062, 5120, 128), (4, 300, 258, 8192, 512), (4, 70, 300, 512, 64),
+    (4, 2100, 4352, 1024, 128), (4, 1100, 8450, 1536, 64),
+    (8, 97, 264, 512, 64), (8, 128, 1030, 2048, 64), (8, 113, 519, 1024, 64),
+    (8, 193, 700, 2048, 128), (8, 2100, 4352, 1024, 64),
+    (4, 33, 33026, 1024, 128), (4, 49, 28674, 2048, 128)])
+def test_many_rows(bits, m, n, k, g):
+    torch.manual_seed(m + n)
+    p, w = matrix(bits, n, k, g)
+    x = torch.randn(m, k, device=DEV).to(BF)
+    x[0] = 0
+    bias = torch.randn(n, device=DEV).to(BF)
+    plain = x.double() @ w.t()
+    close(ext().dq_linear(x, *p, bits, g, bias, None, -1.0, 0),
+          plain + bias.double())
+    if n % 2 == 0:
+        close(ext().dq_gemv_gateup(x, *p, bits, g, -1.0, 0), gated(plain),
+              1e-2)
+
+
+def test_values_that_are_not_finite_stay_in_their_rows():
+    torch.manual_seed(0)
+    p, w = matrix(4, 512, 4096, 128)
+    x = torch.randn(200, 4096, device=DEV).to(BF)
+    x[3, 7], x[130, 4000] = float("inf"), float("nan")
+    y = ext().dq_linear(x, *p, 4, 128, None, None, -1.0, 0)
+    fine = torch.isfinite(x).all(1)
+    assert not bool(torch.isfinite(y[~fine]).any())
+    close(y[fine], x[fine].double() @ w.t())
+
+
+@pytest.mark.parametrize("bits,n,k,g", [(4, 2062, 2048, 128),
+                                        (8, 1040, 1024, 64),
+                                        (4, 516, 1536, 64)])
+def test_many_rows_by_expert(bits, n, k, g):
+    """One to 128 rows a tile, experts without any, tiles that are none."""
+    torch.manual_seed(n)
+    counts = (1, 0, 129, 80, 192, 17)
+    p, w = matrix(bits, n, k, g, (len(counts),))
+    src = torch.randperm(sum(counts)).to(DEV)
+    x = torch.randn(sum(counts), k, device=DEV).to(BF)
+    tiles, at, want = [(-1, 0, 0)], 0, []
+    for e, c in enumerate(counts):
+        tiles += [(e, at + i, min(128, c - i)) for i in range(0, c, 128)]
+        want.append(x.double()[src[at:at + c]] @ w[e].t())
+        at += c
+    tiles = torch.tensor(tiles + [(-1, 0, 0)], dtype=torch.int32, device=DEV)
+    want, s32 = torch.cat(want), src.to(torch.int32)
+    close(ext().moe_linear(x, s32, tiles, *p, bits, g, True, 128), gated(want),
+          1e-2)
+    close(ext().moe_linear(x[src], None, tiles, *p, bits, g, False, 128), want)
