@@ -71,17 +71,6 @@ __device__ __forceinline__ s16x8 codes8_exact(const u32* w) {
   }
 }
 
-// Swizzle of rows of 4, 8 or 16 16-byte slots for reads of 16 bytes where lane
-// group l4 reads slots l4 S / 4 ..: such a read takes 16 lanes at a time, lanes
-// 0-3, 12-15, 20-27 and 4-11, 16-19, 28-31 (and so on from 32), and each of
-// these sets finds its slots in different banks.
-template <int S>
-__device__ __forceinline__ int slot_key16(int row) {
-  static_assert(S == 4 || S == 8 || S == 16, "");
-  const int q = 0xD2 >> (row >> 1 & 6) & 3;      // 2 0 1 3 of row / 4
-  return S == 4 ? q : (S == 8 ? q * 2 + (row >> 1 & 1) : q * 4 + (row & 3));
-}
-
 // own loads but the last N have landed, and reads of LDS are done; then
 // everybody's
 template <int N>

@@ -49,7 +49,7 @@ __device__ __forceinline__ void dq_tile_body(const DqArgs& A, char* smem,
   const int c0 = (int)((long)C * sp / A.splits);
   const int c1 = (int)((long)C * (sp + 1) / A.splits);
   const int G = A.k / A.g, zw = (G + 32 / BITS - 1) / (32 / BITS);
-  auto key = [](int row) { return slot_key<SL>(row); };
+  auto key = [](int row) { return slot_key16<SL>(row); };
   // columns of this workgroup; GLU: a wave's first 16 are gate, the others up
   const int half = A.n / 2, n0 = nblk * (MODE == GLU ? BN / 2 : BN);
 

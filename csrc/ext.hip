@@ -155,15 +155,15 @@ bool wide_rows(int m, int n, int k, long g) {
 }
 
 // The product for many rows: tiles of 256 columns instead of 128.  us of
-// dq_tile / dq_block, 4 bits, k 4096: n 28672 38.5 / 34.3 at 49 rows, 438 / 368 at
-// 1500; n 6144 17.3 / 18.4 at 49, 22.0 / 20.5 at 77, 117.6 / 90.2 at 1500; n 4096,
-// k 14336 24.7 / 24.9 at 49, 30.4 / 28.7 at 77.  8 bits, groups of 64: n 16384, k
-// 2048 22.5 / 21.5 at 49; n 2048, k 8192 23.1 / 23.5 at 77, 25.4 / 24.7 at 120.  8
-// bits in groups of 128, n 32000, k 4096: 64.1 / 65.4 at 120, 96.4 / 93.0 at 200,
+// dq_tile / dq_block, 4 bits, k 4096: n 28672 39.4 / 35.1 at 49 rows, 438 / 368 at
+// 1500; n 6144 21.1 / 24.3 at 77, 25.8 / 22.0 at 120, 118 / 90 at 1500; n 4096, k
+// 14336 25.4 / 26.4 at 49, 30.2 / 30.0 at 77.  8 bits, groups of 64: n 32000, k
+// 2048 34.3 / 30.3 at 49; n 2048, k 8192 23.1 / 23.5 at 77, 25.4 / 24.8 at 120.  8
+// bits in groups of 128, n 32000, k 4096: 63.5 / 65.4 at 120, 96.4 / 93.0 at 200,
 // 535 / 495 at 1500.
 bool block_rows(const torch::Tensor& qweight, const torch::Tensor& scales,
                 long m, long n, long k, long g, long bits) {
-  return (m > (bits == 4 ? 64 : 96) || n * k >= 32l << 20) &&
+  return (m > 96 || n * k >= 62l << 20) &&
          (m > 128 || bits == 4 || g % 128 != 0) &&
          lfmq_dq_block_ok(qweight.data_ptr(), scales.data_ptr(), n, k, g, bits);
 }

@@ -13,12 +13,12 @@ pytestmark = pytest.mark.gpu
 # that end inside a wave's columns, or between pieces of 16 bytes; one group a
 # chunk and several; four chunks up, whole, split, and some tiles split.
 @pytest.mark.parametrize("bits,m,n,k,g", [
-    (4, 65, 264, 1024, 128), (4, 97, 1041, 2048, 128), (4, 128, 520, 1024, 64),
-    (4, 129, 2062, 5120, 128), (4, 300, 258, 8192, 512), (4, 70, 300, 512, 64),
+    (4, 101, 264, 1024, 128), (4, 97, 1041, 2048, 128), (4, 128, 520, 1024, 64),
+    (4, 129, 2062, 5120, 128), (4, 300, 258, 8192, 512), (4, 100, 300, 512, 64),
     (4, 2100, 4352, 1024, 128), (4, 1100, 8450, 1536, 64),
     (8, 97, 264, 512, 64), (8, 128, 1030, 2048, 64), (8, 113, 519, 1024, 64),
     (8, 193, 700, 2048, 128), (8, 2100, 4352, 1024, 64),
-    (4, 33, 33026, 1024, 128), (4, 49, 28674, 2048, 128)])
+    (4, 33, 33026, 2048, 128), (4, 49, 28674, 3072, 128)])
 def test_many_rows(bits, m, n, k, g):
     torch.manual_seed(m + n)
     p, w = matrix(bits, n, k, g)
