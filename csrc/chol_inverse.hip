@@ -12,15 +12,20 @@
 //   update  M_rc -= S_r S_c^T for r > j, c <= r; the first workgroup then
 //           factors M_j+1,j+1 and inverts the factor for the next panel
 //
+// Up to 2048 both are one launch: a tile's workgroup makes the two panels it
+// needs itself and reads one copy of M while it writes the other.  Above, three
+// products a tile instead of one would cost more than the launch.
+//
 // Both halves of the work share one square of memory, since column j of L is
 // read by its panel only.  Products are fp32 matrix instructions fed from
 // global memory (L2): a lane's 16 values of k lie side by side.
 //
 // Bound by the chain of the diagonal blocks (the factor of 64 in panels of 16
-// by one wave, inverse by blocks of 16: 15 us with its update) and two
-// launches a step; from 8192 on by the traffic of M.  n 2048: 0.70 ms, 12.7
-// for factor, inverse and factor from the library; 14336: 50 and 261.  The
-// error of U against 64 bits is a third of that path's (n 2048: 1.4e-7).
+// by one wave, inverse by blocks of 16: 15 us with its update, 20 with the
+// panels and the launch); from 8192 on by the traffic of M.  n 2048: 0.63 ms
+// (two launches a step 0.70), 12.7 for factor, inverse and factor from the
+// library; 14336: 50 and 261.  The error of U against 64 bits is a third of that
+// path's (n 2048: 1.4e-7).
 #include <float.h>
 
 #include "common.h"
@@ -177,12 +182,12 @@ __device__ __forceinline__ void load_rows(const float* p, f32x4 (&v)[4]) {
   for (int i = 0; i < 4; ++i) v[i] = ((const f32x4*)p)[i];
 }
 
-__global__ __launch_bounds__(TPB) void chol_panel_kernel(
-    const float* __restrict__ m, const float* __restrict__ inv,
-    float* __restrict__ s, float* __restrict__ u, int j, int n, int np) {
-  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+// S_b of step j: rows wave * 16 + l4 * 4 + i, columns t * 16 + l15
+__device__ __forceinline__ void panel(const float* __restrict__ m,
+                                      const float* __restrict__ inv, int b,
+                                      int j, int np, f32x4 (&acc)[4]) {
+  const int tid = threadIdx.x, lane = tid & 63;
   const int l15 = lane & 15, l4 = lane >> 4, row = (tid >> 6) * 16 + l15;
-  f32x4 acc[4];
   if (b == j) {
 #pragma unroll
     for (int t = 0; t < 4; ++t)
@@ -207,16 +212,116 @@ __global__ __launch_bounds__(TPB) void chol_panel_kernel(
         acc[t] = mfma(va[i / 4][i % 4], vb[i / 4][i % 4], acc[t]);
     }
   }
+}
+
+// S_b, b <= j: row j of L^-1, to U
+__device__ __forceinline__ void to_u(const f32x4 (&acc)[4],
+                                     float* __restrict__ u, int b, int j,
+                                     int n) {
+  const int tid = threadIdx.x, l15 = tid & 15, l4 = tid >> 4 & 3;
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int r = b * NB + (tid >> 6) * 16 + l4 * 4 + i, k = t * 16 + l15;
-      s[(size_t)r * NB + k] = acc[t][i];
-      const int at = j * NB + k;           // element (at, r) of L^-1
-      if (b <= j && at < n && r <= at)
+      const int r = b * NB + (tid >> 6) * 16 + l4 * 4 + i;
+      const int at = j * NB + t * 16 + l15;      // element (at, r) of L^-1
+      if (at < n && r <= at)
         u[(size_t)(n - 1 - at) * n + n - 1 - r] = acc[t][i];
     }
+}
+
+// A step in one launch: a tile's workgroup makes both panels it needs again,
+// so everything is read from one copy of M (and D) and written to another.
+__global__ __launch_bounds__(TPB, 4) void chol_step_kernel(
+    const float* __restrict__ m, float* __restrict__ mn,
+    const float* __restrict__ inv, float* __restrict__ invn,
+    float* __restrict__ u, int* __restrict__ info, int j, int n, int np) {
+  __shared__ Diag d;                       // S_r, S_c; then the next block
+  // rows from j on, tile (j + 1, j + 1), whose factor the next step waits for,
+  // first
+  const int first = (j + 1) * NB < np ? j + 1 : 0;
+  u32 id = blockIdx.x + first;
+  id = id < gridDim.x ? id : id - gridDim.x;
+  int r, c;
+  tile_of(id + j * (j + 1) / 2, r, c);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int l15 = lane & 15, l4 = lane >> 4;
+  f32x4 p[4];
+  if (r == j) {
+    panel(m, inv, c, j, np, p);
+    to_u(p, u, c, j, n);
+    return;
+  }
+  const int row0 = wave / 2 * 32, col0 = wave % 2 * 32;
+  const size_t mt = (size_t)(r * NB + row0 + l4 * 4) * np + c * NB + col0 + l15;
+  f32x4 old[2][2];                         // at c = j M still holds the panel
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        old[t][v][i] = c == j ? 0.f : m[mt + (size_t)(t * 16 + i) * np + v * 16];
+  auto keep = [&](float (*s)[LD]) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        s[wave * 16 + l4 * 4 + i][t * 16 + l15] = p[t][i];
+  };
+  panel(m, inv, r, j, np, p);
+  keep(d.a);
+  if (c != r) {
+    panel(m, inv, c, j, np, p);
+    keep(d.x);
+  }
+  __syncthreads();
+  const float (*sc)[LD] = c == r ? d.a : d.x;
+  f32x4 acc[2][2] = {};                    // summed apart (chol_update_kernel)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f32x4 a[2], b[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      a[t] = *(const f32x4*)&d.a[row0 + t * 16 + l15][l4 * 16 + i * 4];
+      b[t] = *(const f32x4*)&sc[col0 + t * 16 + l15][l4 * 16 + i * 4];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int v = 0; v < 2; ++v)
+          acc[t][v] = mfma(a[t][e], b[v][e], acc[t][v]);
+  }
+  const bool next = r == j + 1 && c == r;
+  if (next) __syncthreads();               // the panel is read
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float x = old[t][v][i] - acc[t][v][i];
+        if (next) d.a[row0 + t * 16 + l4 * 4 + i][col0 + v * 16 + l15] = x;
+        else mn[mt + (size_t)(t * 16 + i) * np + v * 16] = x;
+      }
+  if (next) factor(d, invn, info, false);
+}
+
+__global__ __launch_bounds__(TPB) void chol_panel_kernel(
+    const float* __restrict__ m, const float* __restrict__ inv,
+    float* __restrict__ s, float* __restrict__ u, int j, int n, int np) {
+  const int b = blockIdx.x, tid = threadIdx.x, l15 = tid & 15, l4 = tid >> 4 & 3;
+  f32x4 acc[4];
+  panel(m, inv, b, j, np, acc);
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      s[(size_t)(b * NB + (tid >> 6) * 16 + l4 * 4 + i) * NB + t * 16 + l15] =
+          acc[t][i];
+  if (b <= j) to_u(acc, u, b, j, n);
 }
 
 __global__ __launch_bounds__(TPB, 4) void chol_update_kernel(
@@ -282,25 +387,48 @@ __global__ __launch_bounds__(TPB, 4) void chol_update_kernel(
 
 int lfmq_chol_pad(int n) { return (n + NB - 1) / NB * NB; }
 
-// h [n, n] fp32 (its lower triangle), u [n, n] zeros.  m [np, np],
-// s [np, 64], inv [64, 64] scratch; info: 1 if a pivot was not positive.
-hipError_t lfmq_chol_inverse(const void* h, void* u, void* m, void* s,
-                             void* inv, void* info, int n,
-                             hipStream_t stream) {
+// One launch a step or two: us at n 512 130 / 156, 1024 256 / 314, 2048 629 / 701,
+// but 3072 1427 / 1174, where three products a tile are more than the chain.
+static bool one_launch(int N) { return N <= 32; }
+
+// floats of scratch memory: M and inverse twice where a step is one launch,
+// else M, inverse and panel
+long lfmq_chol_scratch(int n) {
+  const long np = lfmq_chol_pad(n), N = np / NB;
+  return one_launch((int)N) ? 2 * (np * np + NB * NB)
+                            : np * np + NB * NB + np * NB;
+}
+
+// h [n, n] fp32 (its lower triangle), u [n, n] zeros, scratch of
+// lfmq_chol_scratch; info: 1 if a pivot was not positive.
+hipError_t lfmq_chol_inverse(const void* h, void* u, void* scratch, void* info,
+                             int n, hipStream_t stream) {
   const int np = lfmq_chol_pad(n), N = np / NB;
   if (n < 1 || N > 32768) return hipErrorInvalidValue;
+  const size_t sq = (size_t)np * np;
+  float* m = (float*)scratch;
+  float* inv = m + sq;
+  float* s = inv + NB * NB;                // panel, or the other M and inverse
   hipLaunchKernelGGL(chol_begin_kernel, dim3(N * (N + 1) / 2), dim3(TPB), 0,
-                     stream, (const float*)h, (float*)m, (float*)inv,
-                     (int*)info, n, np);
+                     stream, (const float*)h, m, inv, (int*)info, n, np);
+  if (one_launch(N)) {
+    for (int j = 0; j < N; ++j) {
+      float* m1 = j & 1 ? s : m;
+      float* m2 = j & 1 ? m : s;
+      hipLaunchKernelGGL(chol_step_kernel,
+                         dim3(N * (N + 1) / 2 - j * (j + 1) / 2), dim3(TPB), 0,
+                         stream, m1, m2, m1 + sq, m2 + sq, (float*)u,
+                         (int*)info, j, n, np);
+    }
+    return hipGetLastError();
+  }
   for (int j = 0; j < N; ++j) {
-    hipLaunchKernelGGL(chol_panel_kernel, dim3(N), dim3(TPB), 0, stream,
-                       (const float*)m, (const float*)inv, (float*)s,
-                       (float*)u, j, n, np);
+    hipLaunchKernelGGL(chol_panel_kernel, dim3(N), dim3(TPB), 0, stream, m, inv,
+                       s, (float*)u, j, n, np);
     if (j + 1 < N)
       hipLaunchKernelGGL(chol_update_kernel,
                          dim3(N * (N + 1) / 2 - (j + 1) * (j + 2) / 2),
-                         dim3(TPB), 0, stream, (float*)m, (const float*)s,
-                         (float*)inv, (int*)info, j, np);
+                         dim3(TPB), 0, stream, m, s, inv, (int*)info, j, np);
   }
   return hipGetLastError();
 }

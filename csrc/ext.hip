@@ -54,9 +54,9 @@ hipError_t lfmq_attn_prefill(const void*, const void*, const void*, void*,
                              int, int, int, int, int, int, int, float,
                              hipStream_t);
 hipError_t lfmq_hessian_accum(const void*, void*, int, int, hipStream_t);
-int lfmq_chol_pad(int n);
-hipError_t lfmq_chol_inverse(const void*, void*, void*, void*, void*, void*,
-                             int, hipStream_t);
+long lfmq_chol_scratch(int n);
+hipError_t lfmq_chol_inverse(const void*, void*, void*, void*, int,
+                             hipStream_t);
 hipError_t lfmq_gptq_block(const void*, const void*, int, void*, void*, void*,
                            void*, int, int, int, int, int, int, int, bool,
                            hipStream_t);
@@ -856,13 +856,10 @@ std::vector<torch::Tensor> chol_inverse(torch::Tensor h) {
   TORCH_CHECK(h.dim() == 2 && h.size(0) == h.size(1) && h.size(0) > 0,
               "h must be [n, n]");
   const int n = (int)h.size(0);
-  const long np = lfmq_chol_pad(n);
   auto u = torch::zeros_like(h);
-  auto m = torch::empty({np, np}, h.options());
-  auto s = torch::empty({np + 64, 64}, h.options());
+  auto scratch = torch::empty({lfmq_chol_scratch(n)}, h.options());
   auto info = torch::empty({1}, h.options().dtype(torch::kInt32));
-  CHECK_HIP(lfmq_chol_inverse(h.data_ptr(), u.data_ptr(), m.data_ptr(),
-                              s.data_ptr(), s.data_ptr<float>() + np * 64,
+  CHECK_HIP(lfmq_chol_inverse(h.data_ptr(), u.data_ptr(), scratch.data_ptr(),
                               info.data_ptr(), n, stream()));
   return {u, info};
 }

@@ -48,3 +48,22 @@ def test_push(n, k, nb, i1):
     size[:, at:] += nb * (err.abs().double() @ ub[:, at:].abs())
     assert bool(((got - want).abs() <= size * 2 ** -24).all())
     assert torch.equal(got[:, :at], w[:, :at])
+
+
+# the largest of one launch a step, the smallest of two, and one in between
+@pytest.mark.parametrize("n", [2048, 2049, 1100])
+def test_inverse_factor_of_either_kind(n):
+    """First-order bound as in test_gpu_kernels: each rounding moves U by the
+    condition of H at most, sums of n of them in random directions."""
+    x = torch.randn(2 * n + 1, n, device=DEV) + torch.randn(n, device=DEV)
+    h = x.t() @ x + n * torch.eye(n, device=DEV)
+    u, failed = ext().chol_inverse(h)
+    h64 = h.double()
+    w = torch.linalg.cholesky(torch.linalg.inv(h64), upper=True)
+    e = torch.linalg.eigvalsh(h64)
+    tol = 2 * n ** 0.5 * 2 ** -24 * float(e[-1] / e[0])
+    assert failed.item() == 0
+    assert float((u.double() - w).norm() / w.norm()) <= tol
+    assert float(u.tril(-1).abs().max()) == 0.0
+    h[n - 1, n - 1] = -h[n - 1, n - 1]
+    assert ext().chol_inverse(h)[1].item() == 1
