@@ -153,7 +153,10 @@ class SequenceCache:
             self.lens_host[s] = 0
             self._free.append(s)
         if slots:
-            self.lens[upload(slots, torch.int64, self.device)] = 0
+            # (a number put by index is copied to the device first, and the
+            # host waits for that behind all that is queued)
+            self.lens.index_fill_(
+                0, upload(slots, torch.int64, self.device), 0)
 
     @property
     def free_slots(self) -> int:
