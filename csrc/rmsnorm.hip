@@ -1,8 +1,14 @@
 // K6 — fused RMSNorm: y = x · rsqrt(mean(x²)+ε) · w, optional fused
 // residual add in the same pass (one read, one write — the op is
 // HBM-bound).
-// One workgroup per row; bf16 loaded 8-wide (G13: scalar bf16 is 2×
-// slower); wave shuffle + LDS cross-wave reduction.
+// One workgroup per row, which it keeps in registers (rmsnorm_row_kernel): 16
+// bytes a load, the row, the residual and the weights on their way at once, one
+// barrier for the sum.  Bound by that one latency and the launch for few rows,
+// by the traffic for many.  us a call with the residual, 4096 wide, reading the
+// row twice by four bytes and this one: 1 row 4.1 / 2.1, 48 rows 5.0 / 2.5, 660
+// rows 9.6 / 5.4, 3001 rows 25.6 / 16.9 (5.8 TB/s); 14336 wide, 77 rows 17.5 / 4.6.
+// Rows that are no multiple of eight, unaligned or above 16384 wide take
+// the kernels below.
 #include "common.h"
 
 namespace {
@@ -11,6 +17,70 @@ constexpr int TPB = 256;
 
 // MODE: 0 = plain, 1 = fused residual-in (y = norm(x+r)),
 //       2 = fused residual-in + write new residual (r_out = x+r)
+// V: pieces of eight values a thread
+template <int MODE, int V>
+__global__ __launch_bounds__(TPB) void rmsnorm_row_kernel(
+    const u32x4* __restrict__ x, const u32x4* __restrict__ res_in,
+    const u32x4* __restrict__ w, u32x4* __restrict__ y,
+    u32x4* __restrict__ res_out, int hidden, float eps) {
+  const int n = hidden / 8, tid = threadIdx.x;
+  const u64 at = (u64)blockIdx.x * n;
+  u32x4 xv[V], rv[V], wv[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    // past the end the last piece again, not counted and not stored
+    const int c = min(tid + i * TPB, n - 1);
+    xv[i] = x[at + c];
+    if (MODE) rv[i] = res_in[at + c];
+    wv[i] = w[c];
+  }
+  __shared__ float red[TPB / LFMQ_WAVE];
+  float v[V][8], ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    float part = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float a, b;
+      bf16x2_to_f32(xv[i][e], a, b);
+      if (MODE) {
+        float c, d;
+        bf16x2_to_f32(rv[i][e], c, d);
+        a += c;
+        b += d;
+      }
+      v[i][2 * e] = a;
+      v[i][2 * e + 1] = b;
+      part = fmaf(a, a, part);
+      part = fmaf(b, b, part);
+    }
+    if (tid + i * TPB < n) ss += part;
+  }
+  ss = wave_reduce_sum_dpp(ss);
+  if (tid % LFMQ_WAVE == 0) red[tid / LFMQ_WAVE] = ss;
+  __syncthreads();
+  float t = 0.f;
+#pragma unroll
+  for (int i = 0; i < TPB / LFMQ_WAVE; ++i) t += red[i];
+  const float inv = rsqrtf(t / (float)hidden + eps);
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    const int c = tid + i * TPB;
+    if (c >= n) break;
+    u32x4 o, r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float a = v[i][2 * e], b = v[i][2 * e + 1];
+      float wa, wb;
+      bf16x2_to_f32(wv[i][e], wa, wb);
+      o[e] = pack_bf16x2(a * inv * wa, b * inv * wb);
+      if (MODE == 2) r[e] = pack_bf16x2(a, b);
+    }
+    y[at + c] = o;
+    if (MODE == 2) res_out[at + c] = r;
+  }
+}
+
 template <int MODE>
 __global__ __launch_bounds__(TPB) void rmsnorm_kernel(
     const u32* __restrict__ x, const u32* __restrict__ res_in,
@@ -118,6 +188,26 @@ __global__ __launch_bounds__(LFMQ_WAVE) void rmsnorm_wave_kernel(
 }
 
 template <int MODE>
+bool launch_row(const void* x, const void* r, const void* w, void* y, void* ro,
+                int rows, int hidden, float eps, hipStream_t stream) {
+  if (hidden % 8 || (((u64)x | (u64)r | (u64)w | (u64)y | (u64)ro) & 15))
+    return false;
+#define RCASE(V)                                                            \
+  if (hidden <= 8 * V * TPB) {                                              \
+    hipLaunchKernelGGL((rmsnorm_row_kernel<MODE, V>), dim3(rows), dim3(TPB), \
+                       0, stream, (const u32x4*)x, (const u32x4*)r,          \
+                       (const u32x4*)w, (u32x4*)y, (u32x4*)ro, hidden, eps); \
+    return true;                                                            \
+  }
+  RCASE(1)
+  RCASE(2)
+  RCASE(4)
+  RCASE(8)
+#undef RCASE
+  return false;
+}
+
+template <int MODE>
 bool launch_wave(const u32* x, const u32* r, const u32* w, u32* y, u32* ro,
                  int rows, int hidden, float eps, hipStream_t stream) {
   const int dw = hidden / 2;
@@ -139,6 +229,13 @@ hipError_t lfmq_rmsnorm(const void* x, const void* residual, const void* w,
                         void* y, void* res_out, int rows, int hidden,
                         float eps, hipStream_t stream) {
   if (hidden % 2) return hipErrorInvalidValue;
+  if (residual == nullptr
+          ? launch_row<0>(x, nullptr, w, y, nullptr, rows, hidden, eps, stream)
+          : (res_out == nullptr ? launch_row<1>(x, residual, w, y, nullptr, rows,
+                                                hidden, eps, stream)
+                                : launch_row<2>(x, residual, w, y, res_out, rows,
+                                                hidden, eps, stream)))
+    return hipGetLastError();
   if (rows <= 16 && hidden <= 1024) {  // tiny rows: wave-per-row path
     bool ok;
     if (residual == nullptr)
