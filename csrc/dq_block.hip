@@ -519,11 +519,9 @@ __global__ __launch_bounds__(256) void dq_block_sum(DqArgs A, Plan P) {
   if (row >= rows || col >= nout) return;
   // GLU: 16 of gate, 16 of up a wave
   const float* p = part + row * BN + (MODE == GLU ? (c >> 4) * 32 + (c & 15) : c);
-  f32x4 v = {}, u = {};
-  for (int s = 0; s < P.parts; ++s) {
-    v += *(const f32x4*)(p + (u64)s * (P.step * BN));
-    if (MODE == GLU) u += *(const f32x4*)(p + (u64)s * (P.step * BN) + 16);
-  }
+  const f32x4 v = sum_of_parts(p, P.step * BN, P.parts);
+  f32x4 u = {};
+  if constexpr (MODE == GLU) u = sum_of_parts(p + 16, P.step * BN, P.parts);
   unsigned short* y = A.y + (u64)(row0 + row) * nout + col;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {

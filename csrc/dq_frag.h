@@ -55,6 +55,29 @@ __device__ __forceinline__ s16x8 bf16_ones() {
       s16x8, u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
 }
 
+// The sum of `parts` results, `stride` floats apart, in order; up to eight of
+// them on their way at once.
+template <int B>
+__device__ __forceinline__ f32x4 sum_in(const float* p, u64 stride, int parts) {
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < parts; s0 += B) {
+    f32x4 t[B];
+#pragma unroll
+    for (int i = 0; i < B; ++i)
+      t[i] = *(const f32x4*)(p + (u64)min(s0 + i, parts - 1) * stride);
+#pragma unroll
+    for (int i = 0; i < B; ++i)
+      if (s0 + i < parts) v += t[i];
+  }
+  return v;
+}
+__device__ __forceinline__ f32x4 sum_of_parts(const float* p, u64 stride,
+                                              int parts) {
+  return parts <= 2 ? sum_in<2>(p, stride, parts)
+                    : (parts <= 4 ? sum_in<4>(p, stride, parts)
+                                  : sum_in<8>(p, stride, parts));
+}
+
 // what the packed-product kernels (dq_rows, dq_tile) take
 struct DqArgs {
   const char* w;                 // [n, k * BITS / 8] bytes
