@@ -47,38 +47,6 @@ constexpr int NW = 8, TPB = NW * LFMQ_WAVE, NT = 2, BN = NW * NT * 16;
 constexpr int ROWS = 128;                        // of a tile, at most
 constexpr int D = 3;                             // stages
 
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-
-// Eight codes as bf16, exact.  int4: a nibble c is the fp8 (e4m3) number
-// c 2^-9, denormal or not, which an instruction turns into bf16 two at a time.
-template <int BITS>
-__device__ __forceinline__ s16x8 codes8_exact(const u32* w) {
-  if constexpr (BITS == 8) {
-    return codes8<8>(w);
-  } else {
-    const u32 even = w[0] & 0x0F0F0F0Fu, odd = (w[0] >> 4) & 0x0F0F0F0Fu;
-    const u32 lo = __builtin_amdgcn_perm(odd, even, 0x05010400u);
-    const u32 hi = __builtin_amdgcn_perm(odd, even, 0x07030602u);
-    auto two = [](u32 v, auto up) {
-      return __builtin_bit_cast(
-          u32, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(
-                   v, 512.f, decltype(up)::value));
-    };
-    constexpr std::false_type l{};
-    constexpr std::true_type h{};
-    return __builtin_bit_cast(
-        s16x8, u32x4{two(lo, l), two(lo, h), two(hi, l), two(hi, h)});
-  }
-}
-
-// own loads but the last N have landed, and reads of LDS are done; then
-// everybody's
-template <int N>
-__device__ __forceinline__ void loads_but() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N)
-               : "memory");
-}
-
 __device__ __forceinline__ void load4_to_lds(const void* base, u32 off,
                                              u32 lds) {
   asm volatile(

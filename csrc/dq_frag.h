@@ -3,6 +3,8 @@
 // With a group's scale s and zero z,
 //   sum s (c - z) x = s (sum code x) - s zb sum x,  zb = z + 128 or z.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 
 template <int BITS>
@@ -41,6 +43,28 @@ __device__ __forceinline__ s16x8 deal8(s16x8 x) {
                    __builtin_amdgcn_perm(a[3], a[2], 0x05040100u),
                    __builtin_amdgcn_perm(a[1], a[0], 0x07060302u),
                    __builtin_amdgcn_perm(a[3], a[2], 0x07060302u)});
+}
+
+// Eight codes as bf16, exact.  int4: a nibble c is the fp8 (e4m3) number
+// c 2^-9, denormal or not, which an instruction turns into bf16 two at a time.
+template <int BITS>
+__device__ __forceinline__ s16x8 codes8_exact(const u32* w) {
+  if constexpr (BITS == 8) {
+    return codes8<8>(w);
+  } else {
+    const u32 even = w[0] & 0x0F0F0F0Fu, odd = (w[0] >> 4) & 0x0F0F0F0Fu;
+    const u32 lo = __builtin_amdgcn_perm(odd, even, 0x05010400u);
+    const u32 hi = __builtin_amdgcn_perm(odd, even, 0x07030602u);
+    auto two = [](u32 v, auto up) {
+      return __builtin_bit_cast(
+          u32, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(
+                   v, 512.f, decltype(up)::value));
+    };
+    constexpr std::false_type l{};
+    constexpr std::true_type h{};
+    return __builtin_bit_cast(
+        s16x8, u32x4{two(lo, l), two(lo, h), two(hi, l), two(hi, h)});
+  }
 }
 
 // zb of group gi from its word of packed zeros

@@ -29,6 +29,8 @@ hipError_t lfmq_dq_wide_experts(const void*, const void*, const void*,
                                 int, int, int, int, int, bool, hipStream_t);
 bool lfmq_dq_tile_ok(int, int);
 int lfmq_dq_tile_splits(int, int, int, int);
+hipError_t lfmq_dq_rows_sum(const void*, void*, const void*, const void*, int,
+                            int, int, bool, hipStream_t);
 hipError_t lfmq_dq_tile(const void*, const void*, const void*, const void*,
                         void*, const void*, const void*, void*, int, int, int,
                         int, int, int, bool, hipStream_t);
@@ -86,6 +88,7 @@ hipError_t lfmq_argmax_rows(const void*, void*, void*, void*, int, int,
 hipError_t lfmq_read_probe(const void*, void*, long, long, int, int, int,
                            hipStream_t);
 #include "dq_block.h"
+#include "dq_short.h"
 #include "engine_args.h"
 
 namespace {
@@ -183,6 +186,59 @@ void dq_block(const torch::Tensor& x, const torch::Tensor& qweight,
                           (int)g, (int)bits, glu, P, stream()));
 }
 
+// The product for 17 to 128 rows whose loads are several stages ahead.  us of
+// dq_rows, dq_tile or dq_block / dq_short (dq_short.hip has more): 20 rows, 4 bits,
+// n 4096, k 4096 11.0 / 10.5, but 8 bits, n 16384, k 2048 18.2 / 19.5 at 48 and n
+// 2048, k 8192 14.0 / 14.4 at 32; n 28672, k 4096 34.6 / 38.8 at 64; n 32000, k 2048
+// (8) 30.7 / 28.4 at 64, 35.8 / 36.8 at 96; 128 rows: n 4096, k 4096 21.5 / 18.9, n
+// 16384, k 2048 30.9 / 26.9, n 6144, k 4096 22.5 / 25.2, n 2048, k 8192 21.9 / 22.6.
+// Below 4 million weights rows of x in registers (n 2048, k 2048 10.6 / 11.5 at
+// 77) up to 96.
+bool short_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
+                long bits) {
+  const long size = n * k, M = 1l << 20;
+  const bool gains =
+      m <= 48 ? n >= 4096 && size >= 16 * M && (k >= 4096 || size >= 48 * M)
+      : m <= 96 ? size < 62 * M || (bits == 8 && g % 128 == 0)
+                : (k <= 4096 && size <= 17 * M) ||
+                      (k <= 2048 && size <= 34 * M) ||
+                      (bits == 8 && g % 128 == 0);
+  return m > 16 && m <= 128 && gains && tile_addresses(n, k, bits) &&
+         lfmq_dq_tile_ok((int)k, (int)g) &&
+         (uintptr_t)qweight.data_ptr() % 16 == 0;
+}
+
+void dq_short(const torch::Tensor& x, const torch::Tensor& qweight,
+              const torch::Tensor& scales, const torch::Tensor& qzeros,
+              const void* bias, const void* resid, torch::Tensor& y, long g,
+              long bits, bool glu) {
+  const int m = (int)x.size(0), k = (int)x.size(1), n = (int)qweight.size(0);
+  const DqShortPlan P = lfmq_dq_short_plan(m, n, k, (int)g, (int)bits, glu);
+  DqArgs A{};
+  torch::Tensor part;
+  if (P.splits > 1) {
+    part = torch::empty({(long)P.splits * m * n},
+                        x.options().dtype(torch::kFloat32));
+    A.part = part.data_ptr<float>();
+  }
+  A.w = (const char*)qweight.data_ptr();
+  A.scales = (const unsigned short*)scales.data_ptr();
+  A.zeros = (const u32*)qzeros.data_ptr();
+  A.x = (const unsigned short*)x.data_ptr();
+  A.y = (unsigned short*)y.data_ptr();
+  A.bias = (const unsigned short*)bias;
+  A.resid = (const unsigned short*)resid;
+  A.m = m;
+  A.n = n;
+  A.k = k;
+  A.g = (int)g;
+  A.splits = P.splits;
+  CHECK_HIP(lfmq_dq_short(A, P, (int)bits, glu, stream()));
+  if (P.splits > 1)
+    CHECK_HIP(lfmq_dq_rows_sum(part.data_ptr(), y.data_ptr(), bias, resid, m, n,
+                               P.splits, glu, stream()));
+}
+
 torch::Tensor rmsnorm(torch::Tensor x, torch::Tensor w, double eps,
                       c10::optional<torch::Tensor> residual);
 torch::Tensor silu_mul_fused(torch::Tensor gate_up);
@@ -243,6 +299,8 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
                                        : cols_hint == 6 && m > 4) &&
                        (!tile || m <= (large ? 32 : small ? 96 : 48)) &&
                        lfmq_dq_rows_ok(m, n, k, (int)g, rms);
+  const bool few = cols_hint == 0 && !rms && !(small && by_rows) &&
+                   short_rows(qweight, m, n, k, g, bits);
   if (m > 16) {
     TORCH_CHECK((by_rows || !rms) && (m <= 48 || rptr == nullptr),
                 "fused rms/resid is a decode (m <= 48) path");
@@ -267,6 +325,8 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                            rptr, m, n, k, (int)g, (int)bits, (float)rms_eps,
                            false, stream()));
+  } else if (few) {
+    dq_short(x, qweight, scales, qzeros, bptr, rptr, y, g, bits, false);
   } else if (by_rows) {
     const int splits = rms ? 1 : lfmq_dq_rows_splits(m, n, k, (int)g);
     CHECK_HIP(lfmq_dq_rows(qweight.data_ptr(), scales.data_ptr(),
@@ -452,6 +512,12 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
   const bool tile = tile_addresses(n, k, bits) && (long)m * k < 1l << 31;
   const bool large =
       tile && rms_eps < 0 && k >= 4096 && (long)n * k >= 24l << 20;
+  if (cols_hint == 0 && rms_eps < 0 && n % 2 == 0 &&
+      short_rows(qweight, m, n, k, g, bits)) {
+    if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
+    dq_short(x, qweight, scales, qzeros, nullptr, nullptr, y, g, bits, true);
+    return y;
+  }
   if (cols_hint == 0 && tile && n % 2 == 0 && m > (large ? 32 : 48) &&
       lfmq_dq_tile_ok(k, (int)g)) {
     TORCH_CHECK(rms_eps < 0, "fused rms is a decode (m <= 48) path");

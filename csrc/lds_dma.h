@@ -23,6 +23,14 @@ __device__ __forceinline__ void lds_loads_done() {
   __syncthreads();
 }
 
+// own loads but the last N have landed, and reads of LDS are done; then
+// everybody's
+template <int N>
+__device__ __forceinline__ void loads_but() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N)
+               : "memory");
+}
+
 // Swizzle of rows of 4, 8 or 16 16-byte slots: the slots of 16 consecutive
 // rows at one column fall into different banks.
 template <int SLOTS>

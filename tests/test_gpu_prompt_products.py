@@ -1,5 +1,5 @@
-"""Packed products of a prompt against 64 bits (dq_block), where its row tiles,
-column blocks, stages and parts end.  Tolerances: test_gpu_decode_products."""
+"""Packed products of a prompt against 64 bits (dq_block, dq_short), where their
+row tiles, column blocks, stages and parts end.  Tolerances: test_gpu_decode_products."""
 import pytest
 import torch
 
@@ -13,10 +13,10 @@ pytestmark = pytest.mark.gpu
 # that end inside a wave's columns, or between pieces of 16 bytes; one group a
 # chunk and several; four chunks up, whole, split, and some tiles split.
 @pytest.mark.parametrize("bits,m,n,k,g", [
-    (4, 101, 264, 1024, 128), (4, 97, 1041, 2048, 128), (4, 128, 520, 1024, 64),
-    (4, 129, 2062, 5120, 128), (4, 300, 258, 8192, 512), (4, 100, 300, 512, 64),
+    (4, 129, 264, 1024, 128), (4, 180, 1041, 2048, 128), (4, 256, 520, 1024, 64),
+    (4, 150, 2062, 5120, 128), (4, 300, 258, 8192, 512), (4, 130, 300, 512, 64),
     (4, 2100, 4352, 1024, 128), (4, 1100, 8450, 1536, 64),
-    (8, 97, 264, 512, 64), (8, 128, 1030, 2048, 64), (8, 113, 519, 1024, 64),
+    (8, 129, 264, 512, 64), (8, 256, 1030, 2048, 64), (8, 150, 519, 1024, 64),
     (8, 193, 700, 2048, 128), (8, 2100, 4352, 1024, 64),
     (4, 33, 33026, 2048, 128), (4, 49, 28674, 3072, 128)])
 def test_many_rows(bits, m, n, k, g):
@@ -64,3 +64,30 @@ def test_many_rows_by_expert(bits, n, k, g):
     close(ext().moe_linear(x, s32, tiles, *p, bits, g, True, 128), gated(want),
           1e-2)
     close(ext().moe_linear(x[src], None, tiles, *p, bits, g, False, 128), want)
+
+
+# Row tiles of 32 to 128, one to three of them; columns that end inside a wave's;
+# k whole and in parts, with more groups to a part than LDS holds and with
+# groups of 64's multiples; the residual, which a step of 48 sequences has.
+@pytest.mark.parametrize("bits,m,n,k,g", [
+    (4, 17, 4098, 4096, 128), (4, 33, 4104, 4160, 64), (8, 48, 4099, 4096, 128),
+    (8, 40, 24580, 2112, 64), (4, 49, 2100, 2112, 64), (4, 80, 4098, 1152, 128),
+    (4, 64, 5001, 1024, 256), (8, 65, 2062, 2112, 64), (8, 96, 16400, 2112, 64),
+    (4, 113, 4098, 1024, 128), (4, 128, 4102, 1152, 64), (8, 97, 2054, 2304, 128),
+    (8, 128, 16386, 2048, 64), (8, 77, 32770, 1024, 128)])
+def test_some_rows(bits, m, n, k, g):
+    torch.manual_seed(m + n)
+    p, w = matrix(bits, n, k, g)
+    x = torch.randn(m, k, device=DEV).to(BF)
+    x[0] = 0
+    bias = torch.randn(n, device=DEV).to(BF)
+    plain = x.double() @ w.t()
+    close(ext().dq_linear(x, *p, bits, g, bias, None, -1.0, 0),
+          plain + bias.double())
+    if m <= 48:
+        resid = torch.randn(m, n, device=DEV).to(BF)
+        close(ext().dq_linear(x, *p, bits, g, None, resid, -1.0, 0),
+              plain + resid.double())
+    if n % 2 == 0:
+        close(ext().dq_gemv_gateup(x, *p, bits, g, -1.0, 0), gated(plain),
+              1e-2)
