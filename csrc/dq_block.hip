@@ -323,7 +323,7 @@ __device__ __forceinline__ void dq_block_body(const DqArgs& A, char* smem,
         for (int nt = 0; nt < NT; ++nt)
           a[t & 1][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
               xa[t & 1][j], b[P][nt][j], a[t & 1][nt], 0, 0, 0);
-        if (t == 2)
+        if (t == (MT > 2 ? 2 : 1))
           xsm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xo1[j], ones, xsm, 0, 0,
                                                         0);
       }
@@ -460,14 +460,21 @@ __global__ __launch_bounds__(TPB, 2) void dq_block_kernel(DqArgs A, Plan P) {
     row0 = mt * P.step;
     rows = min(A.m - row0, P.step);
   }
-  if (rows <= 64)
-    dq_block_body<BITS, KC, MODE, 4>(A, smem, row0, rows, expert, nblk, sp,
+  if (rows > 96)
+    dq_block_body<BITS, KC, MODE, 8>(A, smem, row0, rows, expert, nblk, sp,
                                      parts, part);
-  else if (rows <= 96)
+  else if (rows > 64)
     dq_block_body<BITS, KC, MODE, 6>(A, smem, row0, rows, expert, nblk, sp,
                                      parts, part);
+  else if (MODE == DENSE || rows > 32)
+    dq_block_body<BITS, KC, MODE, 4>(A, smem, row0, rows, expert, nblk, sp,
+                                     parts, part);
   else
-    dq_block_body<BITS, KC, MODE, 8>(A, smem, row0, rows, expert, nblk, sp,
+    // experts with few rows, and what 128s leave of others: a layer of 8
+    // (k 4096, 14336) 257 us at 26 rows an expert, 597 at 140; 298 and 630
+    // with 64.  (Tested last: as the first of them it made the others 1 %
+    // slower.)
+    dq_block_body<BITS, KC, MODE, 2>(A, smem, row0, rows, expert, nblk, sp,
                                      parts, part);
 }
 

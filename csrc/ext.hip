@@ -645,15 +645,27 @@ bool wide_experts(int n, int k, long g) {
 }
 
 // Rows a tile of the grouped products for `slots` rows over E experts.  us of
-// a layer of 8 experts (4096, 14336, 4 bits) with 16 / 128: 224 / 364 at 14
-// rows an expert, 330 / 368 at 24, 399 / 369 at 32 (2048, 8192: 123 / 150 at
-// 32, 155 / 150 at 48); 418 / 397 at 16 where tiles of 16 are dq_rows'.
+// a layer with tiles of 16 / 128 (4 bits):
+//   rows an expert             14         18         26         40
+//   E 8,  k 4096, 14336    212 / 252  259 / 254  326 / 258  479 / 310
+//   E 64, k 2048, 2048     118 / 131  142 / 132  186 / 142
+//   E 8,  k 2048, 8192      63 / 100   67 / 101  100 / 119  126 / 123
+//   (of 8 bits: k 4096)     57 / 80    57 / 80    87 / 93   109 / 93
+//   E 16, k 1024, 2048      32 / 33    38 / 33    48 / 40
+// Few weights give dq_block too few workgroups to fill the chip: tiles of 16
+// win for longer there.  With dq_tile (for groups that dq_block does not take)
+// the first line's 128 wins from 26: 364 us at 14 rows, 369 at 32.
+// The last line's tiles of 16 are dq_rows', which reads x for each column.
 long moe_tile(long slots, long E, long k_in, long g_in, long k_out,
               long g_out) {
   TORCH_CHECK(g_in > 0 && g_out > 0, "groups have at least one column");
   // (the first product has 2 k_out columns, the second k_in)
   const bool wide = wide_experts(2048, (int)k_in, g_in) && k_out >= 1024;
-  return slots > (wide ? 26 : 14) * E &&
+  const bool many = E * k_in * k_out >= 1l << 28;
+  const bool block =
+      lfmq_dq_block_ok(nullptr, nullptr, 2 * k_out, k_in, g_in, 8) &&
+      lfmq_dq_block_ok(nullptr, nullptr, k_in, k_out, g_out, 8);
+  return slots > (!wide ? 14 : (!many ? 32 : (block ? 16 : 26))) * E &&
                  lfmq_dq_tile_ok((int)k_in, (int)g_in) &&
                  lfmq_dq_tile_ok((int)k_out, (int)g_out)
              ? 128

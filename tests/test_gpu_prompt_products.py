@@ -50,7 +50,7 @@ def test_values_that_are_not_finite_stay_in_their_rows():
 def test_many_rows_by_expert(bits, n, k, g):
     """One to 128 rows a tile, experts without any, tiles that are none."""
     torch.manual_seed(n)
-    counts = (1, 0, 129, 80, 192, 17)
+    counts = (1, 0, 129, 80, 192, 17, 32, 161)
     p, w = matrix(bits, n, k, g, (len(counts),))
     src = torch.randperm(sum(counts)).to(DEV)
     x = torch.randn(sum(counts), k, device=DEV).to(BF)
