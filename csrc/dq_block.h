@@ -23,10 +23,15 @@ hipError_t lfmq_dq_block(const void* qweight, const void* scales,
                          int g, int bits, bool glu, const DqBlockPlan& P,
                          hipStream_t stream);
 
+// parts of k that pay for an fp32 product of `slots` rows over E experts
+int lfmq_dq_block_slot_parts(long slots, long E, int n, int k, int g, int bits);
+
 // rows of x (or slots) by expert, tiles of up to 128 of them (DqArgs); glu:
-// y bf16 [slots, n / 2], else fp32 [slots, n]
+// y bf16 [slots, n / 2], else fp32 [parts][slots, n], the sum of the parts in
+// the first
 hipError_t lfmq_dq_block_experts(const void* qweight, const void* scales,
                                  const void* qzeros, const void* x,
                                  const void* src, const void* tiles, void* y,
                                  int n_tiles, int n, int k, int g, int bits,
-                                 bool glu, hipStream_t stream);
+                                 bool glu, int parts, long slots,
+                                 hipStream_t stream);

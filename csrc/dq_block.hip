@@ -446,6 +446,11 @@ __global__ __launch_bounds__(TPB, 2) void dq_block_kernel(DqArgs A, Plan P) {
     if (expert < 0) return;
     row0 = A.tiles[3 * mt + 1];
     rows = A.tiles[3 * mt + 2];
+    if (MODE == SLOTS) {
+      sp = blockIdx.y;
+      parts = P.parts;
+      A.y32 += (u64)sp * P.part;
+    }
   } else {
     u32 id = blockIdx.x;
     if ((int)id < P.full) {
@@ -472,8 +477,8 @@ __global__ __launch_bounds__(TPB, 2) void dq_block_kernel(DqArgs A, Plan P) {
   else
     // experts with few rows, and what 128s leave of others: a layer of 8
     // (k 4096, 14336) 257 us at 26 rows an expert, 597 at 140; 298 and 630
-    // with 64.  (Tested last: as the first of them it made the others 1 %
-    // slower.)
+    // with 64 (k whole).  Tested last: as the first of them it made the others
+    // 1 % slower.
     dq_block_body<BITS, KC, MODE, 2>(A, smem, row0, rows, expert, nblk, sp,
                                      parts, part);
 }
@@ -508,6 +513,15 @@ __global__ __launch_bounds__(256) void dq_block_sum(DqArgs A, Plan P) {
   }
 }
 
+// y [parts][4 n4]: the sum of the parts in place of the first
+__global__ __launch_bounds__(256) void dq_block_sum_slots(float* y, u32 n4,
+                                                          int parts) {
+  const u32 i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  float* p = y + (u64)i * 4;
+  *(f32x4*)p = sum_of_parts(p, (u64)n4 * 4, parts);
+}
+
 template <int BITS, int KC, DqMode MODE>
 hipError_t go(const DqArgs& A, const Plan& P, u32 wgs, hipStream_t stream) {
   constexpr int lds = Lds<BITS, KC>::BYTES;
@@ -518,8 +532,9 @@ hipError_t go(const DqArgs& A, const Plan& P, u32 wgs, hipStream_t stream) {
         hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     set = true;
   }
-  hipLaunchKernelGGL((dq_block_kernel<BITS, KC, MODE>), dim3(wgs), dim3(TPB),
-                     lds, stream, A, P);
+  hipLaunchKernelGGL((dq_block_kernel<BITS, KC, MODE>),
+                     dim3(wgs, MODE == SLOTS ? P.parts : 1), dim3(TPB), lds,
+                     stream, A, P);
   return hipGetLastError();
 }
 
@@ -613,12 +628,35 @@ hipError_t lfmq_dq_block(const void* qweight, const void* scales,
   return hipGetLastError();
 }
 
+// Without a gate an expert's few rows give few workgroups (n 4096, 8 experts: a
+// tile each, 128): their k is split where the parts still fit into one round.
+// Rows are taken to be shared out as 9 / 8 of the mean to each, and a part to
+// have 8 chunks at least, for what its first loads and the sum cost.  us of a
+// layer (gate and this), k whole and in parts, at 26 and 60 rows an expert:
+// 8 of 4096, 14336 276, 348 and 238, 304; 8 of 2048, 8192 119 and 76 at 32,
+// 145 and 93 at 60; 16 of 1024, 2048 49 and 42 at 60.
+int lfmq_dq_block_slot_parts(long slots, long E, int n, int k, int g,
+                             int bits) {
+  if (slots < 1 || n % 4 || slots * n >= 1l << 32) return 1;
+  const long each = (slots * 9 / 8 + E - 1) / E;
+  const long wgs = std::min(E, slots) * ((each + ROWS - 1) / ROWS) *
+                   column_blocks(n, false);
+  int parts = 1;
+  while (parts < 4 && wgs * parts * 2 <= 256 &&
+         k / chunk_of(bits, g) / (parts * 2) >= 8)
+    parts *= 2;
+  return parts;
+}
+
 hipError_t lfmq_dq_block_experts(const void* qweight, const void* scales,
                                  const void* qzeros, const void* x,
                                  const void* src, const void* tiles, void* y,
                                  int n_tiles, int n, int k, int g, int bits,
-                                 bool glu, hipStream_t stream) {
-  if (!lfmq_dq_block_ok(qweight, scales, n, k, g, bits) || (glu && n % 2))
+                                 bool glu, int parts, long slots,
+                                 hipStream_t stream) {
+  if (!lfmq_dq_block_ok(qweight, scales, n, k, g, bits) || (glu && n % 2) ||
+      parts < 1 ||
+      (parts > 1 && (glu || n % 4 || slots < 1 || slots * n >= 1l << 32)))
     return hipErrorInvalidValue;
   DqArgs A{};
   A.w = (const char*)qweight;
@@ -634,6 +672,14 @@ hipError_t lfmq_dq_block_experts(const void* qweight, const void* scales,
   A.g = g;
   A.splits = 1;
   const u32 wgs = n_tiles * column_blocks(n, glu);
-  return glu ? go_bits<GLU>(A, Plan{}, bits, wgs, stream)
-             : go_bits<SLOTS>(A, Plan{}, bits, wgs, stream);
+  Plan P{};
+  P.parts = parts;
+  P.part = slots * n;
+  if (glu) return go_bits<GLU>(A, P, bits, wgs, stream);
+  const hipError_t e = go_bits<SLOTS>(A, P, bits, wgs, stream);
+  if (e != hipSuccess || parts == 1) return e;
+  const u32 n4 = (u32)(slots * n / 4);
+  hipLaunchKernelGGL(dq_block_sum_slots, dim3(ceil_div_u32(n4, 256)), dim3(256),
+                     0, stream, A.y32, n4, parts);
+  return hipGetLastError();
 }

@@ -645,27 +645,25 @@ bool wide_experts(int n, int k, long g) {
 }
 
 // Rows a tile of the grouped products for `slots` rows over E experts.  us of
-// a layer with tiles of 16 / 128 (4 bits):
+// a layer with tiles of 16 / 128 (4 bits but the third):
 //   rows an expert             14         18         26         40
-//   E 8,  k 4096, 14336    212 / 252  259 / 254  326 / 258  479 / 310
-//   E 64, k 2048, 2048     118 / 131  142 / 132  186 / 142
-//   E 8,  k 2048, 8192      63 / 100   67 / 101  100 / 119  126 / 123
-//   (of 8 bits: k 4096)     57 / 80    57 / 80    87 / 93   109 / 93
-//   E 16, k 1024, 2048      32 / 33    38 / 33    48 / 40
-// Few weights give dq_block too few workgroups to fill the chip: tiles of 16
-// win for longer there.  With dq_tile (for groups that dq_block does not take)
-// the first line's 128 wins from 26: 364 us at 14 rows, 369 at 32.
-// The last line's tiles of 16 are dq_rows', which reads x for each column.
+//   E 8,  k 4096, 14336    214 / 218  259 / 223  340 / 230  461 / 272
+//   E 8,  k 2048, 8192      63 / 64    67 / 65    99 / 74   126 / 82
+//   E 8,  k 2048, 4096      57 / 53    56 / 53    88 / 60   110 / 62
+//   E 64, k 2048, 2048     118 / 133  142 / 131  186 / 145  246 / 165
+//   E 16, k 1024, 2048      32 / 29    39 / 29    49 / 34    63 / 35
+// With dq_tile (for groups that dq_block does not take) the first line's 128
+// wins from 26: 364 us at 14 rows, 369 at 32.  The last line's tiles of 16 are
+// dq_rows', which reads x for each column.
 long moe_tile(long slots, long E, long k_in, long g_in, long k_out,
               long g_out) {
   TORCH_CHECK(g_in > 0 && g_out > 0, "groups have at least one column");
   // (the first product has 2 k_out columns, the second k_in)
   const bool wide = wide_experts(2048, (int)k_in, g_in) && k_out >= 1024;
-  const bool many = E * k_in * k_out >= 1l << 28;
   const bool block =
       lfmq_dq_block_ok(nullptr, nullptr, 2 * k_out, k_in, g_in, 8) &&
       lfmq_dq_block_ok(nullptr, nullptr, k_in, k_out, g_out, 8);
-  return slots > (!wide ? 14 : (!many ? 32 : (block ? 16 : 26))) * E &&
+  return slots > (!wide ? 14 : (block ? 16 : 26)) * E &&
                  lfmq_dq_tile_ok((int)k_in, (int)g_in) &&
                  lfmq_dq_tile_ok((int)k_out, (int)g_out)
              ? 128
@@ -715,18 +713,26 @@ torch::Tensor moe_linear(torch::Tensor x, c10::optional<torch::Tensor> src,
     sptr = src->data_ptr();
     slots = src->numel();
   }
-  auto y = glu ? torch::empty({slots, (long)n / 2}, x.options())
-               : torch::empty({slots, (long)n},
-                              x.options().dtype(torch::kFloat32));
   TORCH_CHECK(bm == 16 || bm == 128, "tiles of 16 or 128 rows");
+  const bool block =
+      bm == 128 && lfmq_dq_block_ok(qweight.data_ptr(), scales.data_ptr(), n, k,
+                                    g, bits);
+  const int parts = block && !glu
+                        ? lfmq_dq_block_slot_parts(slots, qweight.size(0), n, k,
+                                                   (int)g, (int)bits)
+                        : 1;
+  // (with parts, the sum of them comes to lie in the first)
+  auto y = glu ? torch::empty({slots, (long)n / 2}, x.options())
+               : torch::empty({parts * slots, (long)n},
+                              x.options().dtype(torch::kFloat32))
+                     .narrow(0, 0, slots);
   const int nt = (int)tiles.size(0);
   if (nt == 0) return y;
-  if (bm == 128 && lfmq_dq_block_ok(qweight.data_ptr(), scales.data_ptr(), n, k,
-                                    g, bits))
+  if (block)
     CHECK_HIP(lfmq_dq_block_experts(
         qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
         sptr, tiles.data_ptr(), y.data_ptr(), nt, n, k, (int)g, (int)bits, glu,
-        stream()));
+        parts, slots, stream()));
   else if (bm == 128)
     CHECK_HIP(lfmq_dq_tile_experts(
         qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),

@@ -46,9 +46,11 @@ def test_values_that_are_not_finite_stay_in_their_rows():
 
 @pytest.mark.parametrize("bits,n,k,g", [(4, 2062, 2048, 128),
                                         (8, 1040, 1024, 64),
-                                        (4, 516, 1536, 64)])
+                                        (4, 516, 1536, 64),
+                                        (4, 260, 2560, 64)])
 def test_many_rows_by_expert(bits, n, k, g):
-    """One to 128 rows a tile, experts without any, tiles that are none."""
+    """One to 128 rows a tile, experts without any, tiles that are none; k whole
+    (n not in fours), in two and in four parts."""
     torch.manual_seed(n)
     counts = (1, 0, 129, 80, 192, 17, 32, 161)
     p, w = matrix(bits, n, k, g, (len(counts),))
