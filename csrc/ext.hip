@@ -203,7 +203,7 @@ bool short_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
                 : (k <= 4096 && size <= 17 * M) ||
                       (k <= 2048 && size <= 34 * M) ||
                       (bits == 8 && g % 128 == 0);
-  return m > 16 && m <= 128 && gains && tile_addresses(n, k, bits) &&
+  return m > 16 && m <= 128 && n > 0 && gains && tile_addresses(n, k, bits) &&
          lfmq_dq_tile_ok((int)k, (int)g) &&
          (uintptr_t)qweight.data_ptr() % 16 == 0;
 }

@@ -736,3 +736,17 @@ def test_step_of_a_batch_made_before_its_capture():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("m", [17, 49, 97, 100, 128, 129])
+def test_packed_product_of_no_columns(m):
+    """Refused with any number of rows, as a launch of nothing is."""
+    k, g = 4096, 128
+    p = [torch.zeros(0, k // 8, dtype=torch.int32, device=DEV),
+         torch.ones(0, k // g, dtype=BF, device=DEV),
+         torch.zeros(0, k // g // 8, dtype=torch.int32, device=DEV)]
+    x = torch.zeros(m, k, dtype=BF, device=DEV)
+    for call in (lambda: ext().dq_linear(x, *p, 4, g, None, None, -1.0, 0),
+                 lambda: ext().dq_gemv_gateup(x, *p, 4, g, -1.0, 0)):
+        with pytest.raises(RuntimeError, match="invalid configuration"):
+            call()
