@@ -637,7 +637,7 @@ hipError_t lfmq_dq_block(const void* qweight, const void* scales,
 // 145 and 93 at 60; 16 of 1024, 2048 49 and 42 at 60.
 int lfmq_dq_block_slot_parts(long slots, long E, int n, int k, int g,
                              int bits) {
-  if (slots < 1 || n % 4 || slots * n >= 1l << 32) return 1;
+  if (slots < 1 || E < 1 || n % 4 || slots * n >= 1l << 32) return 1;
   const long each = (slots * 9 / 8 + E - 1) / E;
   const long wgs = std::min(E, slots) * ((each + ROWS - 1) / ROWS) *
                    column_blocks(n, false);

@@ -750,3 +750,17 @@ def test_packed_product_of_no_columns(m):
                  lambda: ext().dq_gemv_gateup(x, *p, 4, g, -1.0, 0)):
         with pytest.raises(RuntimeError, match="invalid configuration"):
             call()
+
+
+@pytest.mark.parametrize("glu", [True, False])
+@pytest.mark.parametrize("bm", [16, 128])
+def test_grouped_product_of_no_experts(bm, glu):
+    """Without experts there are no tiles, and nothing is computed."""
+    k, n, g = 1024, 512, 128
+    p = [torch.zeros(0, n, k // 8, dtype=torch.int32, device=DEV),
+         torch.ones(0, n, k // g, dtype=BF, device=DEV),
+         torch.zeros(0, n, k // g // 8, dtype=torch.int32, device=DEV)]
+    x = torch.zeros(5, k, dtype=BF, device=DEV)
+    tiles = torch.zeros(0, 3, dtype=torch.int32, device=DEV)
+    y = ext().moe_linear(x, None, tiles, *p, 4, g, glu, bm)
+    assert y.shape == (5, n // 2 if glu else n)
