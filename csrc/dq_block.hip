@@ -557,8 +557,8 @@ int column_blocks(int n, bool glu) {
 
 bool lfmq_dq_block_ok(const void* qweight, const void* scales, long n, long k,
                       long g, long bits) {
-  return (bits == 4 || bits == 8) && g > 0 && g % 64 == 0 && k % g == 0 &&
-         k / g % 8 == 0 && n * k / 8 * bits < 1l << 32 &&
+  return (bits == 4 || bits == 8) && g > 0 && g <= k && g % 64 == 0 &&
+         k % g == 0 && k / g % 8 == 0 && n * k / 8 * bits < 1l << 32 &&
          ((u64)qweight | (u64)scales) % 16 == 0;
 }
 

@@ -764,3 +764,17 @@ def test_grouped_product_of_no_experts(bm, glu):
     tiles = torch.zeros(0, 3, dtype=torch.int32, device=DEV)
     y = ext().moe_linear(x, None, tiles, *p, 4, g, glu, bm)
     assert y.shape == (5, n // 2 if glu else n)
+
+
+@pytest.mark.parametrize("glu", [True, False])
+@pytest.mark.parametrize("bm", [16, 128])
+def test_grouped_product_of_no_groups(bm, glu):
+    """Rows of nothing have no chunk of k to begin with: refused."""
+    n, g = 512, 128
+    p = [torch.zeros(2, n, 0, dtype=torch.int32, device=DEV),
+         torch.ones(2, n, 0, dtype=BF, device=DEV),
+         torch.zeros(2, n, 0, dtype=torch.int32, device=DEV)]
+    x = torch.zeros(5, 0, dtype=BF, device=DEV)
+    tiles = torch.tensor([[0, 0, 5]], dtype=torch.int32, device=DEV)
+    with pytest.raises(RuntimeError, match="invalid argument"):
+        ext().moe_linear(x, None, tiles, *p, 4, g, glu, bm)
