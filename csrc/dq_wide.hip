@@ -244,13 +244,19 @@ size_t lds_bytes(int nt, int rows, int G, int zw, int NW) {
          (size_t)nt * NW * lanes_of(rows) * 16 + NW * 64;
 }
 
+int words_of(int G, int bits) { return (G + 32 / bits - 1) / (32 / bits); }
+
+// waves of a workgroup, and the LDS that it may take of a CU's
+int waves_of(int k) { return k <= 8 * KS ? 8 : 16; }
+size_t room_of(int NW) { return 160 * 1024 / (16 / NW); }
+
 // rows: the most that a tile of rows has; lists: tiles of rows
 template <int BITS, int KC, DqMode MODE, bool MORE, int NW>
 hipError_t go(const DqArgs& A, int rows, int lists, hipStream_t stream) {
   constexpr int TC = MODE == GLU ? 8 : 16;
   const int tiles = (int)ceil_div_u32(MODE == GLU ? A.n / 2 : A.n, TC);
-  const int G = A.k / KC, zw = (G + 32 / BITS - 1) / (32 / BITS);
-  const size_t room = 160 * 1024 / (16 / NW);
+  const int G = A.k / KC, zw = words_of(G, BITS);
+  const size_t room = room_of(NW);
   // Tiles of a workgroup, whose scales and sums lie in LDS: what takes the
   // fewest rounds of workgroups that run at once, a round as long as its tiles
   // and about two more.  (4 experts, n 28672, k 4096: 3.5 rounds of 8 tiles 61.1
@@ -308,10 +314,14 @@ hipError_t go_bits(const DqArgs& A, int bits, int rows, int lists,
 
 }  // namespace
 
-// groups of 64 or 128, an even number of them
-bool lfmq_dq_wide_ok(int m, int n, int k, int g) {
+// groups of 64 or 128, an even number of them, and as many as LDS holds the
+// scales of for a tile of columns (16 rows, groups of 64: k up to 233 000 with 4
+// bits, 194 000 with 8)
+bool lfmq_dq_wide_ok(int m, int n, int k, int g, int bits) {
   return m >= 1 && m <= 16 && n >= 1 && (g == 64 || g == 128) &&
-         k % (2 * g) == 0;
+         k % (2 * g) == 0 && (bits == 4 || bits == 8) &&
+         lds_bytes(1, m, k / g, words_of(k / g, bits), waves_of(k)) <=
+             room_of(waves_of(k));
 }
 
 // as lfmq_dq_rows, without splits of k
@@ -320,7 +330,7 @@ hipError_t lfmq_dq_wide(const void* qweight, const void* scales,
                         const void* bias, const void* resid, int m, int n,
                         int k, int g, int bits, float rms_eps, bool glu,
                         hipStream_t stream) {
-  if (!lfmq_dq_wide_ok(m, n, k, g) || (glu && n % 2))
+  if (!lfmq_dq_wide_ok(m, n, k, g, bits) || (glu && n % 2))
     return hipErrorInvalidValue;
   const DqArgs A{(const char*)qweight, (const unsigned short*)scales,
                  (const u32*)qzeros, (const unsigned short*)x,
@@ -337,7 +347,7 @@ hipError_t lfmq_dq_wide_experts(const void* qweight, const void* scales,
                                 const void* src, const void* tiles, void* y,
                                 int n_tiles, int n, int k, int g, int bits,
                                 bool glu, hipStream_t stream) {
-  if (!lfmq_dq_wide_ok(16, n, k, g) || (glu && n % 2) || n_tiles < 1)
+  if (!lfmq_dq_wide_ok(16, n, k, g, bits) || (glu && n % 2) || n_tiles < 1)
     return hipErrorInvalidValue;
   DqArgs A{};
   A.w = (const char*)qweight;

@@ -20,7 +20,7 @@ bool lfmq_dq_row_ok(int, int, int);
 hipError_t lfmq_dq_row(const void*, const void*, const void*, const void*,
                        void*, const void*, const void*, int, int, int, int,
                        float, bool, hipStream_t);
-bool lfmq_dq_wide_ok(int, int, int, int);
+bool lfmq_dq_wide_ok(int, int, int, int, int);
 hipError_t lfmq_dq_wide(const void*, const void*, const void*, const void*,
                         void*, const void*, const void*, int, int, int, int,
                         int, float, bool, hipStream_t);
@@ -151,10 +151,10 @@ bool tile_addresses(long n, long k, long bits) {
 // k 8192 14.5 / 12.4 and 18.6 / 17.4; n 5120, k 5120 14.6 / 14.5 at 16.  A long
 // k of few columns is another matter: n 4096, k 14336 13.7 / 13.1 at 2 rows,
 // 19.5 / 22.9 at 16; n 2048, k 8192 (8 bits) 10.7 / 11.5 at 4.
-bool wide_rows(int m, int n, int k, long g) {
+bool wide_rows(int m, int n, int k, long g, long bits) {
   return m >= 2 && n >= 2048 && k >= 2048 &&
          (k <= 4096 || n >= 8192 || (n >= 5120 && k <= 8192)) &&
-         lfmq_dq_wide_ok(m, n, k, (int)g);
+         lfmq_dq_wide_ok(m, n, k, (int)g, (int)bits);
 }
 
 // The product for many rows: tiles of 256 columns instead of 128.  us of
@@ -320,7 +320,7 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
                           qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                           rptr, n, k, (int)g, (int)bits, (float)rms_eps, false,
                           stream()));
-  } else if (cols_hint == 0 && wide_rows(m, n, k, g)) {
+  } else if (cols_hint == 0 && wide_rows(m, n, k, g, bits)) {
     CHECK_HIP(lfmq_dq_wide(qweight.data_ptr(), scales.data_ptr(),
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                            rptr, m, n, k, (int)g, (int)bits, (float)rms_eps,
@@ -539,7 +539,7 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
     return y;
   }
   if (cols_hint == 0 && n % 2 == 0 &&
-      (m == 1 ? lfmq_dq_row_ok(n, k, (int)g) : wide_rows(m, n, k, g))) {
+      (m == 1 ? lfmq_dq_row_ok(n, k, (int)g) : wide_rows(m, n, k, g, bits))) {
     if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
     if (m == 1)
       CHECK_HIP(lfmq_dq_row(qweight.data_ptr(), scales.data_ptr(),
@@ -640,8 +640,8 @@ std::vector<torch::Tensor> moe_route(torch::Tensor logits, long topk) {
 }
 
 // Tiles of 16 rows of the grouped products that keep x and walk over columns.
-bool wide_experts(int n, int k, long g) {
-  return n >= 2048 && k >= 2048 && lfmq_dq_wide_ok(16, n, k, (int)g);
+bool wide_experts(int n, int k, long g, long bits) {
+  return n >= 2048 && k >= 2048 && lfmq_dq_wide_ok(16, n, k, (int)g, (int)bits);
 }
 
 // Rows a tile of the grouped products for `slots` rows over E experts.  us of
@@ -659,7 +659,7 @@ long moe_tile(long slots, long E, long k_in, long g_in, long k_out,
               long g_out) {
   TORCH_CHECK(g_in > 0 && g_out > 0, "groups have at least one column");
   // (the first product has 2 k_out columns, the second k_in)
-  const bool wide = wide_experts(2048, (int)k_in, g_in) && k_out >= 1024;
+  const bool wide = wide_experts(2048, (int)k_in, g_in, 8) && k_out >= 1024;
   const bool block =
       lfmq_dq_block_ok(nullptr, nullptr, 2 * k_out, k_in, g_in, 8) &&
       lfmq_dq_block_ok(nullptr, nullptr, k_in, k_out, g_out, 8);
@@ -738,7 +738,7 @@ torch::Tensor moe_linear(torch::Tensor x, c10::optional<torch::Tensor> src,
         qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
         sptr, tiles.data_ptr(), y.data_ptr(), nt, n, k, (int)g, (int)bits, glu,
         stream()));
-  else if (wide_experts(n, k, g))
+  else if (wide_experts(n, k, g, bits))
     CHECK_HIP(lfmq_dq_wide_experts(
         qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
         sptr, tiles.data_ptr(), y.data_ptr(), nt, n, k, (int)g, (int)bits, glu,

@@ -112,3 +112,24 @@ def test_rows_by_expert(bits, n, k, g, counts):
     close(ext().moe_linear(x, s32, tiles, *p, bits, g, True, 16), gated(want),
           1e-2)
     close(ext().moe_linear(x[src], None, tiles, *p, bits, g, False, 16), want)
+
+
+# just below and above the number of groups whose scales dq_wide's LDS holds
+@pytest.mark.parametrize("bits,k", [(4, 232960), (4, 240000), (4, 262144),
+                                    (8, 194560), (8, 196608)])
+@pytest.mark.parametrize("m", [2, 16])
+def test_few_rows_of_more_groups_than_a_tile_holds(bits, k, m):
+    n, g, gen = 8192, 64, torch.Generator(DEV).manual_seed(k)
+    i32 = dict(dtype=torch.int32, device=DEV, generator=gen)
+    q = torch.randint(-2 ** 31, 2 ** 31, (n, k * bits // 32), **i32)
+    z = torch.randint(-2 ** 31, 2 ** 31, (n, -(-k // g * bits // 32)), **i32)
+    s = (torch.rand(n, k // g, device=DEV, generator=gen) * 0.02 + 0.01).to(BF)
+    x = torch.randn(m, k, device=DEV, generator=gen).to(BF)
+    y = ext().dq_linear(x, q, s, z, bits, g, None, None, -1.0, 0)
+    # the columns in parts, some of each
+    for c in range(0, n, 1024):
+        at = slice(c, c + 40)
+        w = ref.dequant_groupwise(
+            ref.unpack_codes(q[at], bits, k), s[at].float(),
+            ref.unpack_zeros(z[at], bits, k // g), g).double()
+        close(y[:, at], x.double() @ w.t())
