@@ -27,11 +27,11 @@ hipError_t lfmq_dq_block(const void* qweight, const void* scales,
 int lfmq_dq_block_slot_parts(long slots, long E, int n, int k, int g, int bits);
 
 // rows of x (or slots) by expert, tiles of up to 128 of them (DqArgs); glu:
-// y bf16 [slots, n / 2], else fp32 [parts][slots, n], the sum of the parts in
-// the first
+// y bf16 [slots, n / 2], else fp32 [slots, n]; part: parts > 1 only, fp32
+// [parts, slots, n]
 hipError_t lfmq_dq_block_experts(const void* qweight, const void* scales,
                                  const void* qzeros, const void* x,
                                  const void* src, const void* tiles, void* y,
-                                 int n_tiles, int n, int k, int g, int bits,
-                                 bool glu, int parts, long slots,
+                                 void* part, int n_tiles, int n, int k, int g,
+                                 int bits, bool glu, int parts, long slots,
                                  hipStream_t stream);

@@ -513,13 +513,14 @@ __global__ __launch_bounds__(256) void dq_block_sum(DqArgs A, Plan P) {
   }
 }
 
-// y [parts][4 n4]: the sum of the parts in place of the first
-__global__ __launch_bounds__(256) void dq_block_sum_slots(float* y, u32 n4,
+// y [4 n4]: the sum of part [parts][4 n4]
+__global__ __launch_bounds__(256) void dq_block_sum_slots(const float* part,
+                                                          float* y, u32 n4,
                                                           int parts) {
   const u32 i = blockIdx.x * 256 + threadIdx.x;
   if (i >= n4) return;
-  float* p = y + (u64)i * 4;
-  *(f32x4*)p = sum_of_parts(p, (u64)n4 * 4, parts);
+  *(f32x4*)(y + (u64)i * 4) =
+      sum_of_parts(part + (u64)i * 4, (u64)n4 * 4, parts);
 }
 
 template <int BITS, int KC, DqMode MODE>
@@ -651,12 +652,13 @@ int lfmq_dq_block_slot_parts(long slots, long E, int n, int k, int g,
 hipError_t lfmq_dq_block_experts(const void* qweight, const void* scales,
                                  const void* qzeros, const void* x,
                                  const void* src, const void* tiles, void* y,
-                                 int n_tiles, int n, int k, int g, int bits,
-                                 bool glu, int parts, long slots,
+                                 void* part, int n_tiles, int n, int k, int g,
+                                 int bits, bool glu, int parts, long slots,
                                  hipStream_t stream) {
   if (!lfmq_dq_block_ok(qweight, scales, n, k, g, bits) || (glu && n % 2) ||
       parts < 1 ||
-      (parts > 1 && (glu || n % 4 || slots < 1 || slots * n >= 1l << 32)))
+      (parts > 1 && (glu || part == nullptr || n % 4 || slots < 1 ||
+                     slots * n >= 1l << 32)))
     return hipErrorInvalidValue;
   DqArgs A{};
   A.w = (const char*)qweight;
@@ -664,7 +666,7 @@ hipError_t lfmq_dq_block_experts(const void* qweight, const void* scales,
   A.zeros = (const u32*)qzeros;
   A.x = (const unsigned short*)x;
   A.y = (unsigned short*)y;
-  A.y32 = (float*)y;
+  A.y32 = (float*)(parts > 1 ? part : y);
   A.src = (const i32*)src;
   A.tiles = (const i32*)tiles;
   A.n = n;
@@ -680,6 +682,6 @@ hipError_t lfmq_dq_block_experts(const void* qweight, const void* scales,
   if (e != hipSuccess || parts == 1) return e;
   const u32 n4 = (u32)(slots * n / 4);
   hipLaunchKernelGGL(dq_block_sum_slots, dim3(ceil_div_u32(n4, 256)), dim3(256),
-                     0, stream, A.y32, n4, parts);
+                     0, stream, (const float*)part, (float*)y, n4, parts);
   return hipGetLastError();
 }

@@ -721,17 +721,18 @@ torch::Tensor moe_linear(torch::Tensor x, c10::optional<torch::Tensor> src,
                         ? lfmq_dq_block_slot_parts(slots, qweight.size(0), n, k,
                                                    (int)g, (int)bits)
                         : 1;
-  // (with parts, the sum of them comes to lie in the first)
+  const auto f32 = x.options().dtype(torch::kFloat32);
   auto y = glu ? torch::empty({slots, (long)n / 2}, x.options())
-               : torch::empty({parts * slots, (long)n},
-                              x.options().dtype(torch::kFloat32))
-                     .narrow(0, 0, slots);
+               : torch::empty({slots, (long)n}, f32);
   const int nt = (int)tiles.size(0);
   if (nt == 0) return y;
+  torch::Tensor part;
+  if (parts > 1) part = torch::empty({parts * slots, (long)n}, f32);
   if (block)
     CHECK_HIP(lfmq_dq_block_experts(
         qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
-        sptr, tiles.data_ptr(), y.data_ptr(), nt, n, k, (int)g, (int)bits, glu,
+        sptr, tiles.data_ptr(), y.data_ptr(),
+        parts > 1 ? part.data_ptr() : nullptr, nt, n, k, (int)g, (int)bits, glu,
         parts, slots, stream()));
   else if (bm == 128)
     CHECK_HIP(lfmq_dq_tile_experts(

@@ -93,3 +93,16 @@ def test_some_rows(bits, m, n, k, g):
     if n % 2 == 0:
         close(ext().dq_gemv_gateup(x, *p, bits, g, -1.0, 0), gated(plain),
               1e-2)
+
+
+@torch.no_grad()
+def test_rows_by_expert_in_parts_are_all_that_is_kept():
+    """k in four parts, whose scratch memory is not the result's."""
+    k, n, g, E, each = 2560, 256, 64, 8, 20
+    p, w = matrix(4, n, k, g, (E,))
+    x = torch.randn(E * each, k, device=DEV).to(BF)
+    tiles = torch.tensor([(e, e * each, each) for e in range(E)],
+                         dtype=torch.int32, device=DEV)
+    y = ext().moe_linear(x, None, tiles, *p, 4, g, False, 128)
+    close(y, (x.double().view(E, each, k) @ w.transpose(1, 2)).flatten(0, 1))
+    assert y.untyped_storage().nbytes() == y.numel() * 4
