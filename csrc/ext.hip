@@ -145,16 +145,51 @@ bool tile_addresses(long n, long k, long bits) {
   return n * k / 8 * bits < 1l << 32;
 }
 
-// The kernel that keeps x and walks over columns, or rows.  us of rows / wide,
-// 4 bits: n 28672, k 4096 21.5 / 16.0 at 2 rows, 30.4 / 18.5 at 16; n 4096, k
-// 4096 6.6 / 6.1 and 9.0 / 8.7; n 2048, k 2048 4.9 / 4.1 and 6.3 / 5.6; n 8192,
-// k 8192 14.5 / 12.4 and 18.6 / 17.4; n 5120, k 5120 14.6 / 14.5 at 16.  A long
-// k of few columns is another matter: n 4096, k 14336 13.7 / 13.1 at 2 rows,
-// 19.5 / 22.9 at 16; n 2048, k 8192 (8 bits) 10.7 / 11.5 at 4.
-bool wide_rows(int m, int n, int k, long g, long bits) {
-  return m >= 2 && n >= 2048 && k >= 2048 &&
-         (k <= 4096 || n >= 8192 || (n >= 5120 && k <= 8192)) &&
-         lfmq_dq_wide_ok(m, n, k, (int)g, (int)bits);
+// The kernel that keeps x and walks over columns (dq_wide), or rows.  Its 8 or
+// 16 waves hold 256 values of k each and as many steps of them as k takes, so
+// what counts first is how full the last step is; then, that rows runs one
+// column tile of 16 to 32 a workgroup, in whole rounds of them up to 8192
+// columns (10240: one and a quarter).  us of rows / wide:
+//   4 bits, groups of 128        4 rows         16 rows
+//     n 4096, k 4096 (full)    7.2 / 6.7       9.2 / 8.5
+//     n 4096, k 2560 (0.62)    6.2 / 6.5       7.2 / 8.2
+//     n 8192, k 2560           7.7 / 7.9       8.8 / 9.7
+//     n 10240, k 2560         10.3 / 9.1      12.5 / 11.0
+//     n 6144, k 5120 (0.62)   10.9 / 11.0     13.3 / 14.6
+//     n 28672, k 4096         22.4 / 16.2     30.2 / 18.1
+// With groups of 64 the bodies for several steps spill (gate, 4 rows: n 5120, k
+// 5120 14.9 / 20.7; n 10240, k 8192 31.3 / 26.9).  A gate makes twice the tiles:
+// of 5120 to 8192 columns and k 2048, where that is one a workgroup, 7.0 / 6.7
+// at 4 rows, 7.6 / 8.5 at 16.  With k of many groups rows has the gate apart (n
+// 8192, k 28672, groups of 64: 94 / 68).  Two rows of a smaller matrix of 4 bits
+// are otherwise the GEMV's, which takes, groups of 128, 0.9 of wide's time at n
+// 2048, 1.1 at n 4096; of 64, 0.75 to 1.05 up to 10240 columns, with a gate 0.9
+// to 1.1, and 0.65 to 0.7 for several steps.
+bool wide_rows(int m, int n, int k, long g, long bits, bool glu) {
+  if (m < 2 || n < 2048 || k < 2048 ||
+      !lfmq_dq_wide_ok(m, n, k, (int)g, (int)bits))
+    return false;
+  const bool more = k > 4096;                    // than one step
+  if (more && n < (k <= 8192 ? 5120 : 8192)) return false;
+  if (m == 2 && rows_from(bits, n, k, g) > 2)
+    return g == 128 ? glu || n > 2048 : (glu ? !more : n >= 12288);
+  const int step = k <= 2048 ? 2048 : 4096;
+  const int full = (int)(100l * k / (((long)k + step - 1) / step * step));
+  int least;                                     // percent of the steps
+  if (n > 8192) {
+    least = !more || g == 128 ? 50 : (glu && n <= 16384 ? 70 : 60);
+  } else if (more && g == 64) {
+    if (glu) return !lfmq_dq_rows_ok(m, n, k, (int)g, true);
+    if (bits == 8 && k > 8192) return false;
+    least = bits == 4 ? 70 : 80;
+  } else if (glu && k <= 2048 && n > 4096) {
+    return m <= 8;
+  } else if (glu ? n <= 4096 : n > 4096 && n < 6144) {
+    least = glu ? 50 : 60;
+  } else {
+    least = bits == 8 || (more && !glu) ? 70 : 80;
+  }
+  return full >= least;
 }
 
 // The product for many rows: tiles of 256 columns instead of 128.  us of
@@ -320,7 +355,7 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
                           qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                           rptr, n, k, (int)g, (int)bits, (float)rms_eps, false,
                           stream()));
-  } else if (cols_hint == 0 && wide_rows(m, n, k, g, bits)) {
+  } else if (cols_hint == 0 && wide_rows(m, n, k, g, bits, false)) {
     CHECK_HIP(lfmq_dq_wide(qweight.data_ptr(), scales.data_ptr(),
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                            rptr, m, n, k, (int)g, (int)bits, (float)rms_eps,
@@ -539,7 +574,7 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
     return y;
   }
   if (cols_hint == 0 && n % 2 == 0 &&
-      (m == 1 ? lfmq_dq_row_ok(n, k, (int)g) : wide_rows(m, n, k, g, bits))) {
+      (m == 1 ? lfmq_dq_row_ok(n, k, (int)g) : wide_rows(m, n, k, g, bits, true))) {
     if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
     if (m == 1)
       CHECK_HIP(lfmq_dq_row(qweight.data_ptr(), scales.data_ptr(),

@@ -81,7 +81,8 @@ def test_one_row(bits, n, k, g):
 @pytest.mark.parametrize("m,n,k,g", [
     (2, 2049, 2048, 128), (3, 3074, 2304, 64), (4, 4098, 4096, 128),
     (5, 2050, 2048, 64), (8, 28674, 4096, 128), (9, 8198, 4352, 128),
-    (12, 33000, 2048, 128), (16, 5126, 8192, 64), (16, 4110, 4096, 64)])
+    (12, 33000, 2048, 128), (16, 5126, 8192, 64), (16, 4110, 4096, 64),
+    (6, 8210, 6144, 64)])
 def test_few_rows_many_columns(bits, m, n, k, g):
     """Eight and sixteen waves along k, one and more steps of it; tiles that
     end inside a workgroup's last one; 4, 8 and 16 rows of sums."""
