@@ -192,18 +192,35 @@ bool wide_rows(int m, int n, int k, long g, long bits, bool glu) {
   return full >= least;
 }
 
-// The product for many rows: tiles of 256 columns instead of 128.  us of
-// dq_tile / dq_block, 4 bits, k 4096: n 28672 39.4 / 35.1 at 49 rows, 438 / 368 at
-// 1500; n 6144 21.1 / 24.3 at 77, 25.8 / 22.0 at 120, 118 / 90 at 1500; n 4096, k
-// 14336 25.4 / 26.4 at 49, 30.2 / 30.0 at 77.  8 bits, groups of 64: n 32000, k
-// 2048 34.3 / 30.3 at 49; n 2048, k 8192 23.1 / 23.5 at 77, 25.4 / 24.8 at 120.  8
-// bits in groups of 128, n 32000, k 4096: 63.5 / 65.4 at 120, 96.4 / 93.0 at 200,
-// 535 / 495 at 1500.
+// The product for many rows: tiles of 256 columns instead of 128, which few
+// columns leave most of the chip without.  The time of dq_tile / of this one, the
+// mean over 4400 measured calls of 129 to 700 rows and 6700 of 17 to 128, by n k
+// in millions (2^20):
+//   4 bits, 128  49-96 rows: 0.85 to 1.05 up to 66, 1.08 from 67 on.  129-160:
+//                0.97 up to 10, 1.08 from there on; 161 and more: 1.05 to 1.3
+//   4 bits, 64   49-96: 1.05 from 26 on, 1.15 from 50 on (n 12288, k 3072 at 96
+//                rows 29.4 / 26.6 us).  129-160: 0.97 up to 7, then 1.1 to 1.4
+//   8 bits, 64   49-96: 1.08 from 50 on.  129 and more as 4 bits
+//   8 bits, 128  up to 128 rows 0.85 to 1.0.  129-160: 0.86 to 0.99 up to 66,
+//                then 1.03; 161-256: 0.9 to 1.0 up to 34, then 1.04; 257 and
+//                more: 1.0 to 1.1.  With a gate up to 256 rows 1.0 up to 120 and
+//                1.1 at 224, but n 16384, k 8192 82 / 116 us at 144 rows
+// us, 4 bits, k 4096: n 28672 438 / 368 at 1500 rows; n 6144 118 / 90.
 bool block_rows(const torch::Tensor& qweight, const torch::Tensor& scales,
-                long m, long n, long k, long g, long bits) {
-  return (m > 96 || n * k >= 62l << 20) &&
-         (m > 128 || bits == 4 || g % 128 != 0) &&
-         lfmq_dq_block_ok(qweight.data_ptr(), scales.data_ptr(), n, k, g, bits);
+                long m, long n, long k, long g, long bits, bool glu) {
+  const long size = n * k, M = 1l << 20;
+  const bool wide = g % 128 == 0;                // groups
+  bool gains;
+  if (bits == 8 && wide)
+    gains = m > 256 ||
+            (m > 128 && size > (glu ? 160 : m <= 160 ? 66 : 34) * M);
+  else if (m > 128)
+    gains = m > 160 || size > (wide ? 10 : 7) * M;
+  else
+    gains = m > 96 || size >= 62 * M ||
+            (m > 64 && bits == 4 && !wide && size > 26 * M);
+  return gains && lfmq_dq_block_ok(qweight.data_ptr(), scales.data_ptr(), n, k,
+                                   g, bits);
 }
 
 void dq_block(const torch::Tensor& x, const torch::Tensor& qweight,
@@ -221,23 +238,46 @@ void dq_block(const torch::Tensor& x, const torch::Tensor& qweight,
                           (int)g, (int)bits, glu, P, stream()));
 }
 
-// The product for 17 to 128 rows whose loads are several stages ahead.  us of
-// dq_rows, dq_tile or dq_block / dq_short (dq_short.hip has more): 20 rows, 4 bits,
-// n 4096, k 4096 11.0 / 10.5, but 8 bits, n 16384, k 2048 18.2 / 19.5 at 48 and n
-// 2048, k 8192 14.0 / 14.4 at 32; n 28672, k 4096 34.6 / 38.8 at 64; n 32000, k 2048
-// (8) 30.7 / 28.4 at 64, 35.8 / 36.8 at 96; 128 rows: n 4096, k 4096 21.5 / 18.9, n
-// 16384, k 2048 30.9 / 26.9, n 6144, k 4096 22.5 / 25.2, n 2048, k 8192 21.9 / 22.6.
+// The product for 17 to 128 rows whose loads are several stages ahead: where it
+// is faster than dq_rows (up to 48 rows), dq_tile and dq_block.  The time of
+// those / of this one (m rows), the mean over 6700 measured calls by size, that
+// is n k in millions (2^20):
+//   4 bits, 128  49-96 rows: 1.05 to 1.2 up to 66 (dq_block 0.97 to 1.05), 0.94
+//                from 67 on (1.08).  97-128: 1.25 up to 17, then dq_block
+//   4 bits, 64   49-64: 1.1 (and so dq_block).  65-96: 1.08 up to 26, then 1.02
+//                and dq_block 1.12
+//   8 bits, 64   49-64: 1.15 to 1.3, dq_block 1.0 to 1.15.  65-96: 1.1 up to 60,
+//                then the same as dq_block.  97-128: 1.08 up to 34, 1.04 (1.07)
+//   8 bits, 128  49-128: 1.1 up to 58 and for k 2048 (n 32000 1.2), 0.93 from 64
+//                on (dq_block 0.98)
+// Up to 48 rows of 16 million weights, groups of 64: n 4096, k 4096 10.9 / 12.6
+// at 17 rows, with a gate 24 / 13.  81 to 104 blocks of 128 columns in groups of
+// 128 fill two thirds of the CUs with two parts, and gain nothing by a third: n
+// 11008, k 4096 27.0 / 30.8 at 80 rows, 10240 29.3 / 23.8.  97 rows of short k,
+// groups of 128: n 24576, k 1024 18.1 / 23.8 (dq_block 16.1).
+// block: dq_block would take the call.
 // Below 4 million weights rows of x in registers (n 2048, k 2048 10.6 / 11.5 at
 // 77) up to 96.
 bool short_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
-                long bits) {
+                long bits, bool glu, bool block) {
   const long size = n * k, M = 1l << 20;
-  const bool gains =
-      m <= 48 ? n >= 4096 && size >= 16 * M && (k >= 4096 || size >= 48 * M)
-      : m <= 96 ? size < 62 * M || (bits == 8 && g % 128 == 0)
-                : (k <= 4096 && size <= 17 * M) ||
-                      (k <= 2048 && size <= 34 * M) ||
-                      (bits == 8 && g % 128 == 0);
+  const bool wide = g % 128 == 0;                // groups
+  bool gains;
+  if (m <= 48)
+    gains = n >= 4096 && size >= (wide || glu ? 16 : 20) * M &&
+            (k >= 4096 || size >= 48 * M);
+  else if (bits == 8 && wide)
+    gains = k <= 2048 || size < (m <= 96 ? 58 : 63) * M;
+  else if (m > 96)
+    gains = (k <= 4096 && size <= 17 * M) ||
+            (size <= 34 * M &&
+             (bits == 8 || (k <= 2048 && (n <= 16384 || !wide))));
+  else if (bits == 8)
+    gains = m <= 64 || size < (m <= 80 ? 66 : 62) * M;
+  else
+    gains = wide || m <= 64 ? size < 66 * M : size < 62 * M && !block;
+  const long blocks = (n + 127) / 128;
+  if (wide && m > 48 && k >= 4096 && blocks > 80 && blocks <= 104) gains = false;
   return m > 16 && m <= 128 && n > 0 && gains && tile_addresses(n, k, bits) &&
          lfmq_dq_tile_ok((int)k, (int)g) &&
          (uintptr_t)qweight.data_ptr() % 16 == 0;
@@ -334,8 +374,10 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
                                        : cols_hint == 6 && m > 4) &&
                        (!tile || m <= (large ? 32 : small ? 96 : 48)) &&
                        lfmq_dq_rows_ok(m, n, k, (int)g, rms);
+  const bool block = rptr == nullptr &&
+                     block_rows(qweight, scales, m, n, k, g, bits, false);
   const bool few = cols_hint == 0 && !rms && !(small && by_rows) &&
-                   short_rows(qweight, m, n, k, g, bits);
+                   short_rows(qweight, m, n, k, g, bits, false, block);
   if (m > 16) {
     TORCH_CHECK((by_rows || !rms) && (m <= 48 || rptr == nullptr),
                 "fused rms/resid is a decode (m <= 48) path");
@@ -373,8 +415,7 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                            rptr, m, n, k, (int)g, (int)bits, (float)rms_eps,
                            (int)cols_hint, stream()));
-  } else if (rptr == nullptr &&
-             block_rows(qweight, scales, m, n, k, g, bits)) {
+  } else if (block) {
     dq_block(x, qweight, scales, qzeros, bptr, y, g, bits, false);
   } else {
     const int splits = lfmq_dq_tile_splits(m, n, k, (int)g);
@@ -547,8 +588,9 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
   const bool tile = tile_addresses(n, k, bits) && (long)m * k < 1l << 31;
   const bool large =
       tile && rms_eps < 0 && k >= 4096 && (long)n * k >= 24l << 20;
+  const bool block = block_rows(qweight, scales, m, n, k, g, bits, true);
   if (cols_hint == 0 && rms_eps < 0 && n % 2 == 0 &&
-      short_rows(qweight, m, n, k, g, bits)) {
+      short_rows(qweight, m, n, k, g, bits, true, block)) {
     if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
     dq_short(x, qweight, scales, qzeros, nullptr, nullptr, y, g, bits, true);
     return y;
@@ -557,7 +599,7 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
       lfmq_dq_tile_ok(k, (int)g)) {
     TORCH_CHECK(rms_eps < 0, "fused rms is a decode (m <= 48) path");
     if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
-    if (block_rows(qweight, scales, m, n, k, g, bits)) {
+    if (block) {
       dq_block(x, qweight, scales, qzeros, nullptr, y, g, bits, true);
       return y;
     }

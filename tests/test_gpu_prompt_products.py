@@ -18,7 +18,7 @@ pytestmark = pytest.mark.gpu
     (4, 2100, 4352, 1024, 128), (4, 1100, 8450, 1536, 64),
     (8, 129, 264, 512, 64), (8, 256, 1030, 2048, 64), (8, 150, 519, 1024, 64),
     (8, 193, 700, 2048, 128), (8, 2100, 4352, 1024, 64),
-    (4, 33, 33026, 2048, 128), (4, 49, 28674, 3072, 128)])
+    (8, 257, 1030, 2048, 128), (4, 66, 9002, 3072, 64), (4, 49, 28674, 3072, 128)])
 def test_many_rows(bits, m, n, k, g):
     torch.manual_seed(m + n)
     p, w = matrix(bits, n, k, g)
@@ -76,7 +76,8 @@ def test_many_rows_by_expert(bits, n, k, g):
     (8, 40, 24580, 2112, 64), (4, 49, 2100, 2112, 64), (4, 80, 4098, 1152, 128),
     (4, 64, 5001, 1024, 256), (8, 65, 2062, 2112, 64), (8, 96, 16400, 2112, 64),
     (4, 113, 4098, 1024, 128), (4, 128, 4102, 1152, 64), (8, 97, 2054, 2304, 128),
-    (8, 128, 16386, 2048, 64), (8, 77, 32770, 1024, 128)])
+    (8, 128, 16386, 2048, 64), (8, 77, 32770, 1024, 128), (4, 33, 33026, 2048, 128),
+    (4, 33, 5128, 4160, 64)])
 def test_some_rows(bits, m, n, k, g):
     torch.manual_seed(m + n)
     p, w = matrix(bits, n, k, g)
