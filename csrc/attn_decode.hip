@@ -25,9 +25,12 @@
 // the merge's trips to memory.  One layer of an 8B model (32 query heads on 8),
 // us before and now (tickets that emptied the XCD's caches, two waves a SIMD,
 // ranges of 256 keys):
-//   b 1,  T 129        8.9 ->  8.2      b 8,  T 4000     66   -> 31
-//   b 1,  T 7901      21.4 -> 16.8      b 20, T 900      46   -> 21.8
-//   b 8,  T 1000      20.8 -> 14.3      b 48, T 2047    114   -> 77 (5.2 TB/s)
+//   b 1,  T 129        9.0 ->  8.4      b 8,  T 4000     64   -> 29.1
+//   b 1,  T 7901      20.9 -> 16.1      b 20, T 900      42   -> 20.1
+//   b 8,  T 1000      20.2 -> 13.7      b 48, T 2047    117   -> 77 (5.2 TB/s)
+// Still slower than before: 8 query heads on one, b 1 and 2, 6000 keys and more
+// (20.3 -> 21.9 at 8000), and some 800 workgroups of one range (8 heads, b 100,
+// 8000 keys: 568 -> 601), whose second round is all but empty.
 #include "common.h"
 
 namespace {
@@ -36,10 +39,12 @@ constexpr int TPB = 256, NW = 4, KT = 32;
 constexpr int MAX_SPLITS = 64;       // a wave merges them, one a lane
 // A merge costs 2 us, two rounds of a wave's 32 keys 1.5 more than one.  Up to
 // ONE_RANGE keys are one range; longer ranges than LEAST_KEYS where there would
-// be more than MANY of them.  us with least ranges of 128 / 256 keys (b 1): 9.2
-// / 8.2 at 129 keys, 9.7 / 11.3 at 700, 11.2 / 11.9 at 2000; 21.8 / 16.8 at
-// 7901, 62 and 31 ranges.
-constexpr int ONE_RANGE = 256, LEAST_KEYS = 128, MANY = 32;
+// be more than MANY of them, of the keys that there are: a cache that is half
+// full has as many.  us with least ranges of 128 / 256 keys (b 1): 9.2 / 8.2 at
+// 129 keys, 9.7 / 11.3 at 700, 11.2 / 11.9 at 2000, 13.7 / 13.2 at 4000; 21.0 /
+// 16.1 at 8000 of 16100, 63 and 32 ranges; 25.7 / 23.0 with 8 heads a workgroup
+// (b 2, 4000), but 18.2 / 19.2 with one workgroup a range (3200).
+constexpr int ONE_RANGE = 256, LEAST_KEYS = 128, MANY = 24;
 // Two workgroups a CU, three where a range has very many keys: us with 512 / 768
 // workgroups 14.3 / 15.2 (b 8, 1000 keys), 18.4 / 19.2 (b 16, 900), 81.5 / 77
 // (b 48, 2047).
@@ -65,7 +70,8 @@ __device__ __forceinline__ int range_keys(const DArgs& A, int len) {
   const int per = A.splits == 1 ? len
                                 : (int)(((u64)(u32)(len + A.splits - 1) *
                                          A.inv_splits) >> 32);
-  const int least = len <= ONE_RANGE ? ONE_RANGE : LEAST_KEYS;
+  const int least = len <= ONE_RANGE ? ONE_RANGE
+                    : len <= MANY * LEAST_KEYS ? LEAST_KEYS : 2 * LEAST_KEYS;
   return (max(per, least) + KT - 1) / KT * KT;
 }
 

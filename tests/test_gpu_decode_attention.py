@@ -13,7 +13,9 @@ DEV, BF = "cuda", torch.bfloat16
 @pytest.mark.parametrize("b,T,room,hq,hkv,d", [
     (1, 256, 600, 32, 8, 128), (1, 257, 0, 32, 8, 128), (48, 300, 200, 32, 8, 128),
     (20, 900, 0, 32, 8, 128), (1, 4129, 0, 8, 2, 128), (3, 9000, 7900, 8, 1, 128),
-    (1, 16300, 0, 16, 2, 64), (5, 700, 90, 12, 2, 64), (2, 3000, 0, 3, 3, 128)])
+    (1, 16300, 0, 16, 2, 64), (5, 700, 90, 12, 2, 64), (2, 3000, 0, 3, 3, 128),
+    # the most ranges of 128 keys, and one key more
+    (2, 3072, 5000, 8, 2, 128), (2, 3073, 5000, 8, 2, 128)])
 def test_merge_in_the_launch(b, T, room, hq, hkv, d):
     """Same ranges, same order of sums: the same bits, launch after launch on
     other values, with results of other workgroups, of other XCDs most of them,
