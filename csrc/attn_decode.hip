@@ -47,7 +47,8 @@ constexpr int MAX_SPLITS = 64;       // a wave merges them, one a lane
 constexpr int ONE_RANGE = 256, LEAST_KEYS = 128, MANY = 24;
 // Two workgroups a CU, three where a range has very many keys: us with 512 / 768
 // workgroups 14.3 / 15.2 (b 8, 1000 keys), 18.4 / 19.2 (b 16, 900), 81.5 / 77
-// (b 48, 2047).
+// (b 48, 2047).  Not where a workgroup has eight heads, of which two fit: 23.3 /
+// 32.8 (28 heads on 4, b 13, 2000 keys of 16384).
 constexpr int FULL_WGS = 512, MORE_WGS = 768, LONG_RANGE = 1024;
 
 struct DArgs {
@@ -446,7 +447,8 @@ int lfmq_attn_decode_splits(int b, int hq, int hkv, int T) {
   const int group = hq / hkv, gh = head_tile(group);
   const int wgs = b * hkv * ((group + gh - 1) / gh);
   int n = FULL_WGS / max(wgs, 1);
-  if (T > max(n, 1) * LONG_RANGE) n = MORE_WGS / max(wgs, 1);
+  // (eight heads a workgroup: two of them a CU)
+  if (gh < 8 && T > max(n, 1) * LONG_RANGE) n = MORE_WGS / max(wgs, 1);
   const int most = max(min((T + LEAST_KEYS - 1) / LEAST_KEYS, MANY),
                        (T + 2 * LEAST_KEYS - 1) / (2 * LEAST_KEYS));
   return max(1, min(min(n, most), MAX_SPLITS));
