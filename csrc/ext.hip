@@ -716,9 +716,21 @@ std::vector<torch::Tensor> moe_route(torch::Tensor logits, long topk) {
   return {src_tok, slot_w, offsets, active};
 }
 
-// Tiles of 16 rows of the grouped products that keep x and walk over columns.
-bool wide_experts(int n, int k, long g, long bits) {
-  return n >= 2048 && k >= 2048 && lfmq_dq_wide_ok(16, n, k, (int)g, (int)bits);
+// Tiles of 16 rows, `lists` of them, of the grouped products that keep x and walk
+// over columns, against those of dq_rows.  The time of rows / wide: k 2048 to
+// 4096 and 8192 1.05 to 1.5, up to 4 lists up to 1.9; where k leaves many waves
+// without a step (wide_rows) k 5632, n 2048 0.7 to 0.9 from 9 lists on, 1.1 with
+// 4 bits in groups of 128; k 5120, n 16384 with a gate, groups of 64 0.8 to 0.95;
+// k 3072, 4 bits in groups of 64 0.9 from 17 lists on.
+bool wide_experts(int n, int k, long g, long bits, bool glu, long lists) {
+  if (n < 2048 || k < 2048 ||
+      !lfmq_dq_wide_ok(16, n, k, (int)g, (int)bits))
+    return false;
+  const int step = k <= 2048 ? 2048 : 4096;
+  const int full = (int)(100l * k / (((long)k + step - 1) / step * step));
+  if (k > 4096 && full < 70)
+    return g == 128 ? bits == 4 || glu || lists <= 8 : !glu && lists <= 8;
+  return bits == 8 || g == 128 || full >= 80 || lists <= 16;
 }
 
 // Rows a tile of the grouped products for `slots` rows over E experts.  us of
@@ -736,7 +748,8 @@ long moe_tile(long slots, long E, long k_in, long g_in, long k_out,
               long g_out) {
   TORCH_CHECK(g_in > 0 && g_out > 0, "groups have at least one column");
   // (the first product has 2 k_out columns, the second k_in)
-  const bool wide = wide_experts(2048, (int)k_in, g_in, 8) && k_out >= 1024;
+  const bool wide =
+      wide_experts(2048, (int)k_in, g_in, 8, true, 1) && k_out >= 1024;
   const bool block =
       lfmq_dq_block_ok(nullptr, nullptr, 2 * k_out, k_in, g_in, 8) &&
       lfmq_dq_block_ok(nullptr, nullptr, k_in, k_out, g_out, 8);
@@ -816,7 +829,7 @@ torch::Tensor moe_linear(torch::Tensor x, c10::optional<torch::Tensor> src,
         qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
         sptr, tiles.data_ptr(), y.data_ptr(), nt, n, k, (int)g, (int)bits, glu,
         stream()));
-  else if (wide_experts(n, k, g, bits))
+  else if (wide_experts(n, k, g, bits, glu, nt))
     CHECK_HIP(lfmq_dq_wide_experts(
         qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
         sptr, tiles.data_ptr(), y.data_ptr(), nt, n, k, (int)g, (int)bits, glu,

@@ -92,6 +92,7 @@ def test_few_rows_many_columns(bits, m, n, k, g):
 
 @pytest.mark.parametrize("bits,n,k,g", [(4, 2062, 2048, 128),
                                         (8, 2048, 4352, 64),
+                                        (4, 2048, 6144, 64),
                                         (4, 4100, 4096, 128)])
 @pytest.mark.parametrize("counts", [(1, 0, 2), (16, 3, 0), (0, 21, 9)])
 def test_rows_by_expert(bits, n, k, g, counts):
