@@ -804,9 +804,12 @@ torch::Tensor moe_linear(torch::Tensor x, c10::optional<torch::Tensor> src,
     slots = src->numel();
   }
   TORCH_CHECK(bm == 16 || bm == 128, "tiles of 16 or 128 rows");
+  // Tiles of 128 rows.  The time of dq_tile / dq_block is 1.1 to 4 but for 8 bits
+  // in groups of 128: with a gate 0.8 to 1.0 from 25 rows an expert on, without
+  // one (k in parts) 1.0 to 2.5, but 0.7 to 0.95 at k 1024.
   const bool block =
-      bm == 128 && lfmq_dq_block_ok(qweight.data_ptr(), scales.data_ptr(), n, k,
-                                    g, bits);
+      bm == 128 && !(bits == 8 && g % 128 == 0 && (glu || k <= 1024)) &&
+      lfmq_dq_block_ok(qweight.data_ptr(), scales.data_ptr(), n, k, g, bits);
   const int parts = block && !glu
                         ? lfmq_dq_block_slot_parts(slots, qweight.size(0), n, k,
                                                    (int)g, (int)bits)
