@@ -742,8 +742,10 @@ bool wide_experts(int n, int k, long g, long bits, bool glu, long lists) {
 //   E 64, k 2048, 2048     118 / 133  142 / 131  186 / 145  246 / 165
 //   E 16, k 1024, 2048      32 / 29    39 / 29    49 / 34    63 / 35
 // With dq_tile (for groups that dq_block does not take) the first line's 128
-// wins from 26: 364 us at 14 rows, 369 at 32.  The last line's tiles of 16 are
-// dq_rows', which reads x for each column.
+// wins from 26: 364 us at 14 rows, 369 at 32; where there are more experts, and
+// so tiles, from 18 (k 3072, 1536, 8 bits in groups of 128, at 19 rows: E 16 116
+// / 83, E 64 387 / 282; E 8 at 16 0.9 of the time, at 25 1.1).  The last line's
+// tiles of 16 are dq_rows', which reads x for each column.
 long moe_tile(long slots, long E, long k_in, long g_in, long k_out,
               long g_out) {
   TORCH_CHECK(g_in > 0 && g_out > 0, "groups have at least one column");
@@ -753,7 +755,7 @@ long moe_tile(long slots, long E, long k_in, long g_in, long k_out,
   const bool block =
       lfmq_dq_block_ok(nullptr, nullptr, 2 * k_out, k_in, g_in, 8) &&
       lfmq_dq_block_ok(nullptr, nullptr, k_in, k_out, g_out, 8);
-  return slots > (!wide ? 14 : (block ? 16 : 26)) * E &&
+  return slots > (!wide ? 14 : block ? 16 : E > 8 ? 18 : 26) * E &&
                  lfmq_dq_tile_ok((int)k_in, (int)g_in) &&
                  lfmq_dq_tile_ok((int)k_out, (int)g_out)
              ? 128
