@@ -130,6 +130,11 @@ torch::Tensor unpack(torch::Tensor packed, long bits, long k) {
   return out;
 }
 
+// dq_row and dq_wide read scales two at a time
+bool in_pairs(const torch::Tensor& scales) {
+  return (uintptr_t)scales.data_ptr() % 4 == 0;
+}
+
 // rows from which the rows kernel is taken and not the GEMV, whose lanes hold
 // the scales of 128 groups at most.  us of both at 2 rows: 8 bits 12.5 / 13.3
 // (n 6144, k 4096), 22.9 / 20.5 (4096, 14336), 44.6 / 32.7 (28672, 4096); 4
@@ -332,7 +337,8 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
   const int m = (int)x.size(0), k = (int)x.size(1);
   const int n = (int)qweight.size(0);
   TORCH_CHECK(qweight.size(1) == (long)k * bits / 32, "qweight/k mismatch");
-  const bool one = cols_hint == 0 && m == 1 && lfmq_dq_row_ok(n, k, (int)g);
+  const bool one = cols_hint == 0 && m == 1 && in_pairs(scales) &&
+                   lfmq_dq_row_ok(n, k, (int)g);
   // more groups than the kernels with the norm in them hold scales of (381
   // and 128): the norm apart
   if (rms_eps >= 0 && m <= 4 && k > 128 * g && !one &&
@@ -397,7 +403,8 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
                           qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                           rptr, n, k, (int)g, (int)bits, (float)rms_eps, false,
                           stream()));
-  } else if (cols_hint == 0 && wide_rows(m, n, k, g, bits, false)) {
+  } else if (cols_hint == 0 && in_pairs(scales) &&
+             wide_rows(m, n, k, g, bits, false)) {
     CHECK_HIP(lfmq_dq_wide(qweight.data_ptr(), scales.data_ptr(),
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                            rptr, m, n, k, (int)g, (int)bits, (float)rms_eps,
@@ -615,7 +622,7 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
                            (int)g, (int)bits, splits, true, stream()));
     return y;
   }
-  if (cols_hint == 0 && n % 2 == 0 &&
+  if (cols_hint == 0 && n % 2 == 0 && in_pairs(scales) &&
       (m == 1 ? lfmq_dq_row_ok(n, k, (int)g) : wide_rows(m, n, k, g, bits, true))) {
     if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
     if (m == 1)
@@ -834,7 +841,7 @@ torch::Tensor moe_linear(torch::Tensor x, c10::optional<torch::Tensor> src,
         qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
         sptr, tiles.data_ptr(), y.data_ptr(), nt, n, k, (int)g, (int)bits, glu,
         stream()));
-  else if (wide_experts(n, k, g, bits, glu, nt))
+  else if (in_pairs(scales) && wide_experts(n, k, g, bits, glu, nt))
     CHECK_HIP(lfmq_dq_wide_experts(
         qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
         sptr, tiles.data_ptr(), y.data_ptr(), nt, n, k, (int)g, (int)bits, glu,

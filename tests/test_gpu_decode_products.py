@@ -135,3 +135,21 @@ def test_few_rows_of_more_groups_than_a_tile_holds(bits, k, m):
             ref.unpack_codes(q[at], bits, k), s[at].float(),
             ref.unpack_zeros(z[at], bits, k // g), g).double()
         close(y[:, at], x.double() @ w.t())
+
+
+@pytest.mark.parametrize("m", [1, 8])
+def test_scales_that_start_on_an_odd_number(m):
+    """dq_row and dq_wide read them in pairs: such a matrix is another kernel's."""
+    bits, n, k, g = 4, 8194, 2048, 128
+    (q, s, z), w = matrix(bits, n, k, g)
+    odd = torch.zeros(s.numel() + 1, dtype=BF, device=DEV)[1:].view_as(s)
+    odd.copy_(s)
+    assert odd.data_ptr() % 4 == 2
+    x = torch.randn(m, k, device=DEV).to(BF)
+    want = x.double() @ w.t()
+    close(ext().dq_linear(x, q, odd, z, bits, g, None, None, -1.0, 0), want)
+    close(ext().dq_gemv_gateup(x, q, odd, z, bits, g, -1.0, 0), gated(want),
+          1e-2)
+    tiles = torch.tensor([[0, 0, m]], dtype=torch.int32, device=DEV)
+    close(ext().moe_linear(x, None, tiles, q.unsqueeze(0), odd.unsqueeze(0),
+                           z.unsqueeze(0), bits, g, False, 16), want)
