@@ -153,3 +153,31 @@ def test_scales_that_start_on_an_odd_number(m):
     tiles = torch.tensor([[0, 0, m]], dtype=torch.int32, device=DEV)
     close(ext().moe_linear(x, None, tiles, q.unsqueeze(0), odd.unsqueeze(0),
                            z.unsqueeze(0), bits, g, False, 16), want)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_one_row_of_values_that_are_not_finite(value):
+    """Every column takes part in every value: no result is finite."""
+    p, _ = matrix(4, 8198, 2048, 128)
+    x = torch.randn(1, 2048, device=DEV).to(BF)
+    x[0, 1000] = value
+    for eps in (-1.0, 1e-5):
+        y = ext().dq_linear(x, *p, 4, 128, None, None, eps, 0)
+        assert not bool(torch.isfinite(y).any())
+
+
+# matrices past 4 GiB (k 16384, 8 bits: 262144 rows are), whose last rows a
+# 32-bit offset would not reach
+@pytest.mark.parametrize("m", [1, 4])
+def test_few_rows_past_4_gib(m):
+    bits, n, k, g = 8, 263168, 16384, 128
+    q = torch.zeros(n, k // 4, dtype=torch.int32, device=DEV)
+    s = torch.zeros(n, k // g, dtype=BF, device=DEV)
+    z = torch.zeros(n, k // g // 4, dtype=torch.int32, device=DEV)
+    part, w = matrix(bits, 1024, k, g)
+    for t, u in zip((q, s, z), part):
+        t[-1024:] = u
+    x = torch.randn(m, k, device=DEV).to(BF)
+    y = ext().dq_linear(x, q, s, z, bits, g, None, None, -1.0, 0)
+    close(y[:, -1024:], x.double() @ w.t())
+    assert not bool(y[:, :-1024].any())

@@ -33,11 +33,14 @@ def test_many_rows(bits, m, n, k, g):
               1e-2)
 
 
-def test_values_that_are_not_finite_stay_in_their_rows():
+# dq_wide, dq_short (k whole, and in parts) and dq_block
+@pytest.mark.parametrize("m,n,k", [(8, 8200, 2048), (40, 4104, 4096),
+                                   (100, 4104, 2048), (200, 512, 4096)])
+def test_values_that_are_not_finite_stay_in_their_rows(m, n, k):
     torch.manual_seed(0)
-    p, w = matrix(4, 512, 4096, 128)
-    x = torch.randn(200, 4096, device=DEV).to(BF)
-    x[3, 7], x[130, 4000] = float("inf"), float("nan")
+    p, w = matrix(4, n, k, 128)
+    x = torch.randn(m, k, device=DEV).to(BF)
+    x[3, 7], x[m * 2 // 3, k - 96] = float("inf"), float("nan")
     y = ext().dq_linear(x, *p, 4, 128, None, None, -1.0, 0)
     fine = torch.isfinite(x).all(1)
     assert not bool(torch.isfinite(y[~fine]).any())
