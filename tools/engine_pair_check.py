@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Validate the record-pair ILP engine path in one short GPU pass:
 parity vs the launched fused path (teacher-forced), bit-determinism,
-and per-phase prof deltas.  Designed to fit one small gpurun call."""
+and per-phase prof deltas, in one short run."""
 import os
 import sys
 import time
