@@ -556,6 +556,33 @@ def test_unequal_batch_and_slots_used_again(name, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+def test_requests_end_on_another_stream(dtype):
+    """Slots are given back behind steps that are still queued elsewhere, and
+    serve again: the numbers of `end` outlive the call that brings them."""
+    m, cfg, w = model("mixed", dtype)
+    st, steps, ends = stepper(m, 400, 2), torch.cuda.Stream(), \
+        torch.cuda.Stream()
+    got, want = [], []
+    for rnd in range(6):
+        req = {i: util.tokens(cfg, n, 100 * rnd + n)
+               for i, n in enumerate((70 - 9 * rnd, 5 + rnd))}
+        with torch.cuda.stream(steps):
+            got.append(st.step([(i, t[:-1], list(range(len(t) - 1)))
+                                for i, t in req.items()]))
+            got.append(st.step([(i, t[-1:], [0]) for i, t in req.items()]))
+        ends.wait_stream(steps)
+        with torch.cuda.stream(ends):
+            st.end(list(req))
+        steps.wait_stream(ends)
+        full = [util.expected(w, cfg, t) for t in req.values()]
+        want += [torch.cat([x[:-1] for x in full]),
+                 torch.cat([x[-1:] for x in full])]
+    torch.cuda.synchronize()
+    for g, x in zip(got, want):
+        assert util.rel(g, x) < TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_mixed_step_of_prompts_and_single_tokens(dtype):
     """A step may bring portions for some sequences, one token for others."""
     m, cfg, w = model("mixed", dtype)
