@@ -335,8 +335,9 @@ __global__ __launch_bounds__(TPB, D * GH > 512 ? 2 : 3) void attn_decode_kernel(
   // drains its own stores, which are past the XCDs' caches when they are done,
   // and the barrier orders all of them before the ticket; the merging workgroup
   // reads past its caches, too.  So the ticket orders nothing: as a release and
-  // acquire it writes back and empties an XCD's L2, once for each of these
-  // workgroups (48 x 300 keys, 384 of them: 58 us).  The merging workgroup
+  // acquire, which any chip would need that keeps agent scope in its L2s, it
+  // writes back and empties an XCD's L2, once for each of these workgroups (48 x
+  // 300 keys, 384 of them: 58 us).  The merging workgroup
   // puts the ticket back to zero, so a replayed graph finds it as the first
   // launch did.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

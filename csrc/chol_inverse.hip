@@ -24,8 +24,8 @@
 // by one wave, inverse by blocks of 16: 15 us with its update, 20 with the
 // panels and the launch); from 8192 on by the traffic of M.  n 2048: 0.63 ms
 // (two launches a step 0.70), 12.7 for factor, inverse and factor from the
-// library; 14336: 50 and 261.  The error of U against 64 bits is a third of that
-// path's (n 2048: 1.4e-7).
+// library; 14336: 50 and 261.  The error of U against 64 bits is a third to a
+// half of that path's (n 2048: 1.4e-7, condition 3600: 4.6e-6).
 #include <float.h>
 
 #include "common.h"

@@ -1,4 +1,4 @@
-// K3c/K4c — W4A16 / W8A16 product for a few to a few hundred rows of x:
+// K3c/K4c — W4A16 / W8A16 product for a few to a hundred rows of x:
 // y[m, n] = x[m, k] · dequant(W)[n, k]^T (+ bias) (+ residual).
 //
 // Between the GEMV (m <= 4) and the large product the packed weights are
@@ -21,13 +21,11 @@
 // and scales the sums; silu(gate) * up; bias and residual.
 //
 // us a call, before (16-column GEMV tiles up to 16 rows, 128 x 128 tiles
-// above) and now:
+// above) and now, of what is not dq_wide's or dq_short's:
 //                       8 rows       24 rows       48 rows
-//   n 28672, k 4096   70.0 -> 24.1  108 -> 31.6   107 -> 49.3
-//   n 4096, k 14336   45.0 -> 17.4  362 -> 20.6   366 -> 29.7   (4 bits)
-//   n 4096, k 4096    13.7 ->  8.0  101 -> 11.6   101 -> 14.4
-//   n 16384, k 2048   75.5 -> 12.9   57 -> 15.1    58 -> 18.2   (8 bits,
-//   n 2048, k 8192    25.5 -> 12.0  203 -> 14.1   203 -> 16.6    group 64)
+//   n 4096, k 14336   45.0 -> 17.4
+//   n 2048, k 8192    25.5 -> 12.0  203 -> 14.1   203 -> 16.6   (8 bits,
+//   n 16384, k 2048                  57 -> 15.1    58 -> 18.2   group 64)
 #include "dq_frag.h"
 
 namespace {

@@ -1,4 +1,4 @@
-// K3e/K4e — W4A16 / W8A16 product for a few tens to a hundred rows: y[m, n] =
+// K3g/K4g — W4A16 / W8A16 product for a few tens to a hundred rows: y[m, n] =
 // x[m, k] · dequant(W)[n, k]^T (+ bias) (+ residual), or the gated half of a
 // fused gate and up projection.
 //

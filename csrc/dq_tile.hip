@@ -1,5 +1,6 @@
 // K3b/K4b — W4A16 / W8A16 product for prompts: y[m, n] = x[m, k] ·
-// dequant(W)[n, k]^T (+ bias).  Few rows, and groups that dq_block does not take.
+// dequant(W)[n, k]^T (+ bias).  Groups that dq_block does not take, 8 bits in
+// groups of 128 up to some 200 rows, small matrices a few rows above 128.
 //
 // A workgroup computes 128 rows by 128 columns, four waves side by side in
 // the columns, each all 128 rows by 32 columns.  x goes through LDS (two
@@ -12,16 +13,14 @@
 // of the rows' with products by ones, and all waves apply them a chunk later.
 //
 // Bound by latencies between the stages of two waves a SIMD (matrix cores
-// busy 41 % of the time, vector units 46 %, LDS half): 832 TFLOP/s at 3001 x
-// 28672 x 4096 (4 bits, groups of 128), where 128 x 128 tiles of weights
-// unpacked into LDS reached 418.  128 x 256 tiles with one wave a SIMD: 570.
-// LDS slots without bank conflicts: the same time.  us a call, before and now:
-//                       64 rows      256 rows      3001 rows
-//   n 28672, k 4096   107 -> 40.2   178 -> 87.5   1690 -> 847
-//   n 4096, k 14336   369 -> 26.4   361 -> 52.2    890 -> 459   (4 bits)
-//   n 6144, k 4096    101 -> 19.5   103 -> 32.6    422 -> 210
-//   n 16384, k 2048    58 -> 24.2    59 -> 46.2    501 -> 336   (8 bits,
-//   n 2048, k 8192    203 -> 20.8   203 -> 31.1    343 -> 213    group 64)
+// busy 41 % of the time, vector units 46 %, LDS half: 3001 rows of n 28672, k
+// 4096, which are dq_block's now).  128 x 256 tiles with one wave a SIMD: 570
+// TFLOP/s and not 832.  slot_key's order of LDS slots, which pairs of lanes
+// share: the same within 2 %.  us a call (TFLOP/s):
+//                                  100 rows   256 rows   1500 rows   3001 rows
+//   n 4096, k 11008 (4 bits)          37         48       195 (692)   403 (672)
+//   n 5120, k 13824                   41         67       274 (776)   536 (793)
+//   n 28672, k 4096 (8, group 128)    57         95
 #include "dq_frag.h"
 #include "lds_dma.h"
 

@@ -25,6 +25,8 @@
 // 130.6 -> 110.8, 72.5 -> 70.9.  Two steps of weights in flight a wave: 17.1
 // us instead of 16.9 at 8 rows; eight waves with twice the k 17.9; batches of
 // tiles whose sums are taken during the next batch: registers spill, 20 % slower.
+// (Groups of 64 with k above 4096 spill 2 to 20 registers: ext.hip's rules were
+// measured with that.)
 #include "dq_frag.h"
 
 namespace {

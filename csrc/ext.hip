@@ -136,10 +136,9 @@ bool in_pairs(const torch::Tensor& scales) {
 }
 
 // rows from which the rows kernel is taken and not the GEMV, whose lanes hold
-// the scales of 128 groups at most.  us of both at 2 rows: 8 bits 12.5 / 13.3
-// (n 6144, k 4096), 22.9 / 20.5 (4096, 14336), 44.6 / 32.7 (28672, 4096); 4
-// bits 8.8 / 9.3, 17.0 / 15.1 and 27.3 / 22.0.  At 1 row the GEMV: 6.9 / 9.2,
-// 13.5 / 15.1, 18.1 / 22.5 (4 bits).
+// the scales of 128 groups at most.  us of both (4 bits, groups of 128): n 4096, k
+// 14336 11.3 / 13.0 at 1 row, 15.6 / 13.1 at 2; n 2048, k 8192 5.9 / 8.4, 7.6 / 8.3
+// and 9.3 / 8.5 at 3 (8 bits, groups of 64: 8.1 / 11.0, 10.8 / 10.8).
 int rows_from(long bits, long n, long k, long g) {
   if (k > 128 * g) return 1;
   return bits == 8 || n * k >= 32l << 20 ? 2 : 3;
@@ -261,8 +260,8 @@ void dq_block(const torch::Tensor& x, const torch::Tensor& qweight,
 // 11008, k 4096 27.0 / 30.8 at 80 rows, 10240 29.3 / 23.8.  97 rows of short k,
 // groups of 128: n 24576, k 1024 18.1 / 23.8 (dq_block 16.1).
 // block: dq_block would take the call.
-// Below 4 million weights rows of x in registers (n 2048, k 2048 10.6 / 11.5 at
-// 77) up to 96.
+// Below 4 million weights rows of x in registers up to 96 (n 2048, k 2048 9.7 /
+// 9.9 at 96 rows).
 bool short_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
                 long bits, bool glu, bool block) {
   const long size = n * k, M = 1l << 20;
@@ -358,23 +357,18 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
     rptr = resid->data_ptr();
   }
   auto y = torch::empty({m, n}, x.options());
-  // Which kernel: a wave a few columns (GEMV), rows of x in registers, or x
-  // through LDS.  us of the first two, n 28672, k 4096, 4 bits: 24.6 / 21.5 at
-  // 2 rows but 8.5 / 9.6 at n 6144; 36 / 22 and 11.9 / 9.8 at 4.  8 bits,
-  // n 32000, k 2048: 18.5 / 18.7 at 1 row, 29 / 19 at 2.  The last two, 4
-  // bits, k 4096: n 28672 35.0 / 35.4 at 32 rows, 42 / 35 at 33; n 6144
-  // 15.8 / 16.1 and 18.1 / 16.4; n 4096 still 14.5 / 15.4 at 48.  k 2048, n
-  // 16384 (8 bits): 19.9 / 21.6 at 48.
-  // With the norm, GEMV / rows (n 6144, k 4096, 4 bits): 8.8 / 9.1 at 2 rows,
-  // 12.9 / 9.8 at 4, and norm and product apart: 13.6 / 10.0 at 8, 23.8 /
-  // 20.2 at 48.
+  // What is left by dq_row, dq_wide, dq_short and dq_block, whose rules go
+  // first: a wave a few columns (GEMV), rows of x in registers, x through LDS.  us
+  // of the last two: n 3072, k 8192 (4 bits) 14.5 / 17.1 at 32 rows, 17.7 / 17.1 at
+  // 33, 25.5 / 18.7 at 49; n 16384, k 2048 (8 bits, groups of 64) 18.4 / 21.4 at 48,
+  // 30.7 / 21.6 at 49.
   const bool rms = rms_eps >= 0;
   const bool tile = tile_addresses(n, k, bits);
   const bool large = tile && !rms && k >= 4096 && (long)n * k >= 24l << 20 &&
                      (rptr == nullptr ||
                       lfmq_dq_tile_splits(m, n, k, (int)g) > 1);
-  // a product that a few workgroups do whole: n 2048, k 2048 11.2 / 14.7 at 77
-  // rows, 15.1 / 17.0 at 120, but 21 / 16.6 at 129; n 3072 15.6 / 16.0
+  // a product that a few workgroups do whole: n 2048, k 2048 9.7 / 12.9 at 77
+  // rows; n 3072 14.1 / 13.6
   const bool small = !rms && rptr == nullptr && (long)n * k <= 4l << 20;
   const bool by_rows = (cols_hint == 0 ? m >= rows_from(bits, n, k, g)
                                        : cols_hint == 6 && m > 4) &&
@@ -589,9 +583,7 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
   const int n = (int)qweight.size(0);
   TORCH_CHECK(qweight.size(1) == (long)k * bits / 32, "qweight/k mismatch");
   auto y = torch::empty({m, n / 2}, x.options());
-  // as dq_linear.  us with the norm, GEMV / rows, n 28672, k 4096, 4 bits:
-  // 37.5 / 24.0 at 4 rows; norm, product and gate apart / rows: 32.5 / 26.4 at
-  // 8, 44.0 / 37.6 at 32 (n 16384, k 2048 at 48: 21.4 / 15.6)
+  // as dq_linear
   const bool tile = tile_addresses(n, k, bits) && (long)m * k < 1l << 31;
   const bool large =
       tile && rms_eps < 0 && k >= 4096 && (long)n * k >= 24l << 20;

@@ -274,10 +274,10 @@ __global__ __launch_bounds__(512) void gptq_block_kernel(BlockArgs A) {
 // A workgroup 64 x 64, K in 64s through LDS, fp32 matrix instructions, the
 // product summed apart and rounded once at the size of w.  Bound by the load
 // of both operands before the products and, from some 1000 workgroups on, by
-// the products: 2048 x 1920 17.4 us (6.4 at the instructions' rate; the
-// library 15.6), 4096 rows 28.6 (32.9), 8192 50.5 (61); over the blocks of
-// 2048 x 2048 11.4 on average (16.5).  K whole in LDS, two workgroups a CU:
-// 15.1.
+// the products.  Over the blocks of 2048 x 2048 11.0 us a product on average
+// (the library 14.5), of 4096 x 4096 28.6 (37.4), of 8192 x 2048 28.6 (35.3).  A
+// small product repeated on operands that the caches hold takes the library
+// less (4.6, here 6.9).  K whole in LDS, two workgroups a CU: 15.1 for 11.4.
 constexpr int PT = 64, PK = 64, LA = PK + 4, LB = PT + 16;
 
 __global__ __launch_bounds__(256, 3) void gptq_push_kernel(

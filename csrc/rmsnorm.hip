@@ -96,8 +96,7 @@ __global__ __launch_bounds__(TPB) void rmsnorm_kernel(
   __shared__ float red[TPB / LFMQ_WAVE];
 
   float ss = 0.f;
-  // pass 1: sum of squares (values kept in registers when hidden small
-  // enough; re-read from L1 otherwise — rows are <= 16 KB, L1-resident)
+  // the row is read twice, the second time mostly from the caches
   for (int i = threadIdx.x; i < dw; i += TPB) {
     float a, b;
     bf16x2_to_f32(xr[i], a, b);
@@ -135,11 +134,9 @@ __global__ __launch_bounds__(TPB) void rmsnorm_kernel(
   }
 }
 
-// Single-WAVE variant for the decode shape (few rows): no LDS, no
-// barriers — 64 lanes, values held in registers between the reduce and
-// the scale pass (hidden <= 8192: <= 32 dwords/lane).  The 256-thread
-// two-barrier version measured 6.1 us/call on [1,4096]; the decode step
-// runs 64 of these per token.
+// A wave a row, which it keeps in registers: no LDS, no barrier.  Up to 16 rows
+// of up to 1024 that rmsnorm_row_kernel does not take (widths not in eights,
+// rows not on 16 bytes).
 template <int MODE, int DWPL>  // dwords per lane
 __global__ __launch_bounds__(LFMQ_WAVE) void rmsnorm_wave_kernel(
     const u32* __restrict__ x, const u32* __restrict__ res_in,
