@@ -10,11 +10,19 @@
 // A workgroup = 128 x 128, 4 waves of 64 x 64, tokens in steps of 64 through
 // two LDS buffers.  Tiles run in blocks of 4 x 4, a range of blocks to an XCD,
 // whose L2 then serves a row of tiles four times (8 x 8 leave more of the
-// triangle's edge empty: 102 x 7416 99 us, 82 so).  Bound by the LDS
-// reads of the fragments and by reading and writing H (in whole lines,
-// through LDS), one after the other.  2048 x 14336: 653 us (645 TFLOP/s of
-// the half computed), against 2102 for the full square staged through
-// transposing 2-byte LDS writes; 2048 x 2048: 33 (70), 64 x 512: 9.3 (8.5).
+// triangle's edge empty: 102 x 7416 99 us, 82 so).
+//
+// Where H is large its traffic is as long as the products (128 x 14336: 346 us
+// at 4.8 TB/s; the products of 2048 x 14336 alone: 465), and the two overlap
+// only as far as a workgroup's loads are under way before it needs them and
+// leave X in the L2.  So elements of the tile's own place load beside the last
+// two steps, those of the mirror while the result goes through LDS, and H
+// passes by the caches where its rows are whole lines.  2048 x 14336: 673 us
+// with H read after the products, 629 with loads ahead, 545 past the caches
+// too (772 TFLOP/s of the half computed); 512 x 8192: 122 and 100;
+// 2048 x 4096: 78 and 70; 2048 x 2048: 33, 64 x 512: 9.3 (one round of
+// workgroups, below).  Matrix cores are busy 40 % of the time, memory 65 %:
+// two workgroups of one wave a SIMD each hide no more of each other.
 #include "lds_dma.h"
 
 namespace {
@@ -35,9 +43,17 @@ __device__ __forceinline__ int chunk_key(int token) {
   return (token & 7) ^ ((token >> 1) & 4);
 }
 
+// How H is read and written.  DIRECT: a single round of workgroups, which wait
+// for memory once, straight from the fragments (64 x 512: 9.3 us, 13.9 through
+// LDS).  WHOLE: more workgroups, rows of H whole lines, past the caches.
+// CACHED: the same where neighbouring tiles share lines, which then have to
+// meet in a cache (102 x 7416: 81 us, 107 past it).
+enum Way { DIRECT, WHOLE, CACHED };
+
+template <Way WAY>
 __global__ __launch_bounds__(TPB, 2) void hessian_kernel(
     const unsigned short* __restrict__ x, float* __restrict__ h, int t,
-    int k, bool direct) {
+    int k) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   // block (bi, bj) of the lower triangle, tile (r, c) of it
   const u32 id = xcd_swizzle(blockIdx.x, gridDim.x);
@@ -91,20 +107,20 @@ __global__ __launch_bounds__(TPB, 2) void hessian_kernel(
     }
     return f;
   };
-  f32x4 acc[4][4] = {};
-  stage(0, 0);
-  for (int t0 = 0, par = 0; t0 < t; t0 += BK, par ^= 1) {
-    lds_loads_done();
-    if (t0 + BK < t) {
-      stage(t0 + BK, par ^ 1);
-    } else if (t0 + BK > t) {
-      const u32x4 z = {0, 0, 0, 0};
-      for (int i = (t - t0) * 16 + tid; i < BK * 16; i += TPB) {
-        *(u32x4*)(smem + par * BUF + i * 16) = z;
-        *(u32x4*)(smem + par * BUF + BUF / 2 + i * 16) = z;
-      }
-      __syncthreads();
+  // rows of a tile of H in fours of a thread: 512 bytes of a row together
+  constexpr int NF = BC * BC / 4 / TPB;
+  const int c4 = tid % (BC / 4) * 4, r0 = tid / (BC / 4);
+  auto fours_load = [&](f32x4 (&v)[NF], int row0, int col0) {
+    const float* p = h + (u64)row0 * k + min(col0 + c4, k - 4);
+#pragma unroll
+    for (int e = 0; e < NF; ++e) {
+      const int r = min(r0 + e * (TPB * 4 / BC), k - 1 - row0);
+      const f32x4* q = (const f32x4*)(p + (u32)(r * k));
+      v[e] = WAY == WHOLE ? __builtin_nontemporal_load(q) : *q;
     }
+  };
+  f32x4 acc[4][4] = {}, own[NF];
+  auto products = [&](int par) {
     const char* la = smem + par * BUF;
     const char* lb = la + BUF / 2;
 #pragma unroll
@@ -122,11 +138,30 @@ __global__ __launch_bounds__(TPB, 2) void hessian_kernel(
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
               a[i], b[j], acc[i][j], 0, 0, 0);
     }
+  };
+  // the last step by itself: behind its loads those of H are on their way (in
+  // the same loop their registers are copied at each turn: 724 us for 545)
+  const int end = (t - 1) / BK * BK;
+  int par = 0;
+  stage(0, 0);
+  for (int t0 = 0; t0 < end; t0 += BK, par ^= 1) {
+    loads_but<0>();
+    stage(t0 + BK, par ^ 1);
+    products(par);
   }
-  // H += 2 acc, here and mirrored.  A single round of workgroups waits for
-  // memory once, straight from the fragments (64 x 512: 9.3 us, 13.9 through
-  // LDS) ...
-  if (direct) {
+  if (WAY != DIRECT) fours_load(own, i0, j0);
+  loads_but<WAY == DIRECT ? 0 : NF>();
+  if (end + BK > t) {
+    const u32x4 z = {0, 0, 0, 0};
+    for (int i = (t - end) * 16 + tid; i < BK * 16; i += TPB) {
+      *(u32x4*)(smem + par * BUF + i * 16) = z;
+      *(u32x4*)(smem + par * BUF + BUF / 2 + i * 16) = z;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+  products(par);
+  // H += 2 acc, here and mirrored
+  if constexpr (WAY == DIRECT) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int row = i0 + wi * 64 + i * 16 + l4 * 4;
@@ -152,48 +187,44 @@ __global__ __launch_bounds__(TPB, 2) void hessian_kernel(
         if (ti != tj) *(f32x4*)(h + (u64)col * k + row) = u[j];
       }
     }
-    return;
+  } else {
+    // (LD: rows and columns both spread over the banks)
+    float* out = (float*)smem;
+    loads_but<NF>();
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          out[(wi * 64 + i * 16 + l4 * 4 + r) * LD + wj * 64 + j * 16 + l15] =
+              acc[i][j][r];
+    f32x4 mirror[NF];
+    if (ti != tj) fours_load(mirror, j0, i0);
+    // only LDS: the loads stay under way
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // v + 2 out at (row0, col0) of H; out by ro a row and co a column
+    auto add = [&](const f32x4 (&v)[NF], int row0, int col0, int ro, int co) {
+      if (col0 + c4 >= k) return;            // k in eights: four columns alike
+      float* p = h + (u64)row0 * k + col0 + c4;
+#pragma unroll
+      for (int e = 0; e < NF; ++e) {
+        const int r = r0 + e * (TPB * 4 / BC);
+        f32x4 w;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          w[q] = fmaf(2.f, out[r * ro + (c4 + q) * co], v[e][q]);
+        if (row0 + r >= k) continue;
+        f32x4* to = (f32x4*)(p + (u32)(r * k));
+        if (WAY == WHOLE)
+          __builtin_nontemporal_store(w, to);
+        else
+          *to = w;
+      }
+    };
+    add(own, i0, j0, LD, 1);
+    if (ti != tj) add(mirror, j0, i0, 1, LD);
   }
-  // ... more are bound by the traffic: through LDS, so that 512 bytes of a row
-  // are read and written together either way, 32 elements a thread in flight
-  // (128 x 14336: 350 us, 707 from the fragments; with halves of the tile and
-  // 256 bytes of the mirror, 102 x 7416, whose rows do not start lines, is 5 %
-  // slower.  LD: rows and columns both spread over the banks)
-  float* out = (float*)smem;
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        out[(wi * 64 + i * 16 + l4 * 4 + r) * LD + wj * 64 + j * 16 + l15] =
-            acc[i][j][r];
-  __syncthreads();
-  // BC x BC results at (row0, col0) of H, U of a thread at once
-  auto add = [&](int row0, int col0, int ro, int co) {
-    constexpr int U = 32;
-    const int c = tid & (BC - 1), rs = TPB / BC;
-    if (col0 + c >= k) return;
-    const int R = min(BC, k - row0);
-    float* p = h + (u64)row0 * k + col0;
-    for (int r = tid / BC; r < R; r += rs * U) {
-      float v[U];
-#pragma unroll
-      for (int e = 0; e < U; ++e) {
-        const int rr = r + e * rs;
-        if (rr < R) v[e] = p[(u32)(rr * k + c)];
-      }
-#pragma unroll
-      for (int e = 0; e < U; ++e) {
-        const int rr = r + e * rs;
-        if (rr < R)
-          p[(u32)(rr * k + c)] = fmaf(2.f, out[rr * ro + c * co], v[e]);
-      }
-    }
-  };
-  add(i0, j0, LD, 1);
-  if (ti != tj) add(j0, i0, 1, LD);
 }
 
 }  // namespace
@@ -205,8 +236,11 @@ hipError_t lfmq_hessian_accum(const void* x, void* h, int t, int k,
   const u32 n = ceil_div_u32(k, BC * SB), tiles = ceil_div_u32(k, BC);
   const bool direct = tiles * (tiles + 1) / 2 <= 256;
   const int lds = direct ? 2 * BUF : max(2 * BUF, BC * LD * 4);
-  hipLaunchKernelGGL(hessian_kernel, dim3(n * (n + 1) / 2 * SB * SB),
-                     dim3(TPB), lds, stream, (const unsigned short*)x,
-                     (float*)h, t, k, direct);
+  auto* kernel = direct ? hessian_kernel<DIRECT>
+                        : (k % 32 == 0 && (u64)h % 128 == 0
+                               ? hessian_kernel<WHOLE>
+                               : hessian_kernel<CACHED>);
+  hipLaunchKernelGGL(kernel, dim3(n * (n + 1) / 2 * SB * SB), dim3(TPB), lds,
+                     stream, (const unsigned short*)x, (float*)h, t, k);
   return hipGetLastError();
 }

@@ -404,6 +404,27 @@ def test_hessian_accum_tiles(t, k):
                  <= (t + 1) * bound.double()).all())
 
 
+@pytest.mark.parametrize("t,k,off", [(1, 2944, 0), (64, 3104, 0),
+                                     (65, 2824, 0), (130, 2944, 1)])
+def test_hessian_accum_past_caches(t, k, off):
+    """More than a round of tiles: rows of H whole lines and not, an H that
+    begins within a line; what lies before and behind it stays.  Bound as
+    above."""
+    torch.manual_seed(t + k)
+    x = torch.randn(t, k).to(torch.bfloat16)
+    room = torch.randn(off + k * k + 8)
+    got = room.to(DEV)
+    ext().hessian_accum(got[off:off + k * k].view(k, k), x.to(DEV))
+    got = got.cpu()
+    h = room[off:off + k * k].view(k, k)
+    want = h.double() + 2 * x.double().t() @ x.double()
+    bound = (h.abs() + 2 * x.float().abs().t() @ x.float().abs()) * 2 ** -24
+    assert bool(((got[off:off + k * k].view(k, k).double() - want).abs()
+                 <= (t + 1) * bound.double()).all())
+    assert torch.equal(got[:off], room[:off])
+    assert torch.equal(got[off + k * k:], room[off + k * k:])
+
+
 @pytest.mark.parametrize("b,T,hq,hkv,d", [
     (1, 1, 4, 4, 128), (2, 32, 4, 2, 64), (1, 33, 8, 2, 128),
     (3, 256, 8, 1, 128), (1, 257, 16, 1, 64), (2, 513, 6, 2, 128),
