@@ -12,7 +12,7 @@
 //   update  M_rc -= S_r S_c^T for r > j, c <= r; the first workgroup then
 //           factors M_j+1,j+1 and inverts the factor for the next panel
 //
-// Up to 2048 both are one launch: a tile's workgroup makes the two panels it
+// Up to 3072 both are one launch: a tile's workgroup makes the two panels it
 // needs itself and reads one copy of M while it writes the other.  Above, three
 // products a tile instead of one would cost more than the launch.
 //
@@ -20,13 +20,20 @@
 // read by its panel only.  Products are fp32 matrix instructions fed from
 // global memory (L2): a lane's 16 values of k lie side by side.
 //
-// Bound by the chain of the diagonal blocks (the factor of 64 in panels of 16
-// by one wave, inverse by blocks of 16: 15 us with its update, 20 with the
-// panels and the launch); from 8192 on by the traffic of M.  n 2048: 0.63 ms
-// (two launches a step 0.70), 12.7 for factor, inverse and factor from the
-// library; 14336: 50 and 261.  The error of U against 64 bits is a third to a
-// half of that path's (n 2048: 1.4e-7, condition 3600: 4.6e-6).
+// Bound by the chain of the diagonal blocks, 15 us a step at n 2048: 4 from the
+// end of a launch to the next one's first workgroup, 2.5 until its panel's
+// operands are there (other XCDs wrote them), 2 of products, 6.5 of factor and
+// inverse; from 8192 on by the traffic of M.  In the factor every wave carries
+// the diagonal block's 16 columns, a lane a column, beside 16 rows of its own,
+// so that a column is a reciprocal and one instruction a row, and the inverse
+// grows beside it (a lane a row in one wave, other waves waiting, then the
+// inverse: 10 us).  n 512: 101 us (133 so), 1024 192 (256), 2048 470 (638; 12.7
+// ms for factor, inverse and factor from the library), 3072 975 (1170), 4096
+// 1615 (1732), 8192 8140 (8250).  The error of U against 64 bits is a third of
+// that path's (n 2048: 2.1e-7 of its norm; 2.5e-7 with the factor before).
 #include <float.h>
+
+#include <utility>
 
 #include "common.h"
 
@@ -43,110 +50,142 @@ __device__ __forceinline__ float lane_value(float v, int lane) {
 }
 
 struct Diag {
-  float a[NB][LD];   // the block, its lower triangle becomes L
-  float x[NB][LD];   // L^-1
+  float a[NB][LD];           // the block; its lower blocks of 16 become L's
+  float x[NB][LD];           // L^-T, its upper blocks of 16
+  float diag[4][16][20];     // a wave's diagonal block (20: over all banks)
 };
 
-// d.a: factor and inverse; the inverse to inv [64, 64], upper part zero
+// lane J's value of each row of 16 lanes
+template <int J>
+__device__ __forceinline__ float row_lane(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                         0x150 + J, 0xf, 0xf, true));
+}
+
+// v[i] += f * lane J's v[i], one instruction each (the compiler makes a move
+// and a sum of it, with waits between).  Lanes of a register may be read two
+// instructions after it was written: the wait in front covers what comes before
+// a block, and within a block no register is written and read again.
+#define LFMQ_ADD(i, f, J)                                       \
+  "v_fmac_f32_dpp %" #i ", %" #i ", %" #f " row_newbcast:%" #J \
+  " row_mask:0xf bank_mask:0xf\n\t"
+
+template <int J, int N>
+__device__ __forceinline__ void add_lane(float* v, float f) {
+  if constexpr (N >= 6) {
+    asm("s_nop 1\n\t" LFMQ_ADD(0, 6, 7) LFMQ_ADD(1, 6, 7) LFMQ_ADD(2, 6, 7)
+            LFMQ_ADD(3, 6, 7) LFMQ_ADD(4, 6, 7) LFMQ_ADD(5, 6, 7)
+        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]),
+          "+v"(v[5])
+        : "v"(f), "n"(J));
+    add_lane<J, N - 6>(v + 6, f);
+  } else if constexpr (N >= 3) {
+    asm("s_nop 1\n\t" LFMQ_ADD(0, 3, 4) LFMQ_ADD(1, 3, 4) LFMQ_ADD(2, 3, 4)
+        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2])
+        : "v"(f), "n"(J));
+    add_lane<J, N - 3>(v + 3, f);
+  } else if constexpr (N == 2) {
+    asm("s_nop 1\n\t" LFMQ_ADD(0, 2, 3) LFMQ_ADD(1, 2, 3)
+        : "+v"(v[0]), "+v"(v[1])
+        : "v"(f), "n"(J));
+  } else if constexpr (N == 1) {
+    asm("s_nop 1\n\t" LFMQ_ADD(0, 1, 2) : "+v"(v[0]) : "v"(f), "n"(J));
+  }
+}
+
+// Column J of a panel leaves the columns behind it, without square roots: the
+// diagonal block's rows v, and four rows o of another block.  A lane is a
+// column; piv is the pivot, then the next one (read four instructions after it
+// was written: the chain of a panel runs through it).
+template <int J>
+__device__ __forceinline__ void column(float (&v)[16], float (&o)[4],
+                                       float& piv, int l15) {
+  if constexpr (J < 15) {
+    float r = __builtin_amdgcn_rcpf(piv);
+    r = fmaf(fmaf(-piv, r, 1.f), r, r);
+    const float f = l15 > J ? -v[J] * r : 0.f;
+    asm("s_nop 1\n\t" LFMQ_ADD(0, 6, 7) LFMQ_ADD(1, 6, 7) LFMQ_ADD(2, 6, 7)
+            LFMQ_ADD(3, 6, 7)
+        "v_mov_b32_dpp %5, %0 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
+            LFMQ_ADD(4, 6, 7)
+        : "+v"(v[J + 1]), "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]),
+          "=&v"(piv)
+        : "v"(f), "n"(J), "n"(J + 1));
+    add_lane<J, 14 - J>(v + J + 2, f);
+  }
+}
+template <int... J>
+__device__ __forceinline__ void columns(float (&v)[16], float (&o)[4], int l15,
+                                        std::integer_sequence<int, J...>) {
+  float piv = row_lane<0>(v[0]);
+  (column<J>(v, o, piv, l15), ...);
+}
+
+// d.a = L L^T; L^-1 to inv [64, 64], upper part zero.  The columns of L act on
+// the rows of the identity too, which become L^-T: in panel p a wave has one
+// block of 16 rows, of d.a below the diagonal block or of the identity beside
+// and above it (below that it is still zero), and everybody the diagonal block.
+// A panel's blocks first take what the panels before it leave them.
 __device__ __forceinline__ void factor(Diag& d, float* inv, int* info, bool first) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l15 = lane & 15, l4 = lane >> 4;
   bool bad = false;
-  __syncthreads();
 #pragma unroll 1
   for (int p = 0; p < 4; ++p) {
-    if (wave == 0) {                       // a lane a row, 16 columns
-      f32x4 v[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = *(f32x4*)&d.a[lane][16 * p + 4 * i];
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const float piv = lane_value(v[j / 4][j % 4], 16 * p + j);
-        bad |= !(piv >= FLT_MIN && piv <= FLT_MAX);
-        float rs = __builtin_amdgcn_rsqf(piv);
-        rs = fmaf(fmaf(-piv * rs, rs, 1.f), 0.5f * rs, rs);
-        const float l = v[j / 4][j % 4] * rs;
-        v[j / 4][j % 4] = l;
-#pragma unroll
-        for (int c = j + 1; c < 16; ++c)
-          v[c / 4][c % 4] -= l * lane_value(l, 16 * p + c);
-      }
-      if (lane >= 16 * p)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) *(f32x4*)&d.a[lane][16 * p + 4 * i] = v[i];
-    }
     __syncthreads();
-    int t = 0;
-    for (int r = p + 1; r < 4; ++r)
-      for (int c = p + 1; c <= r; ++c, ++t) {
-        if ((t & 3) != wave) continue;
-        const f32x4 va = *(f32x4*)&d.a[16 * r + l15][16 * p + 4 * l4];
-        const f32x4 vb = *(f32x4*)&d.a[16 * c + l15][16 * p + 4 * l4];
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc = mfma(va[i], vb[i], acc);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          d.a[16 * r + l4 * 4 + i][16 * c + l15] -= acc[i];
-      }
-    __syncthreads();
-  }
-  if (tid == 0 && (first || bad)) *info = bad;
-
-  {                                        // a wave a diagonal block of 16
-    f32x4 l[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      l[i] = *(f32x4*)&d.a[16 * wave + l15][16 * wave + 4 * i];
-    const float rd = 1.f / d.a[16 * wave + l15][16 * wave + l15];
-    f32x4 x[4];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) x[i / 4][i % 4] = i == l15 ? 1.f : 0.f;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const float xk = x[k / 4][k % 4] * lane_value(rd, k);
-      x[k / 4][k % 4] = xk;
-#pragma unroll
-      for (int i = k + 1; i < 16; ++i)
-        x[i / 4][i % 4] -= lane_value(l[k / 4][k % 4], i) * xk;
-    }
+    const bool below = wave > p;
+    float (*rows)[LD] = below ? d.a : d.x;
+    f32x4 dg, sd = {0.f, 0.f, 0.f, 0.f}, so = sd;
+    float o[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      float v = x[i][0];
-      v = l4 == 1 ? x[i][1] : v;
-      v = l4 == 2 ? x[i][2] : v;
-      v = l4 == 3 ? x[i][3] : v;
-      d.x[16 * wave + 4 * i + l4][16 * wave + l15] = v;
+      dg[i] = d.a[16 * p + 4 * l4 + i][16 * p + l15];
+      o[i] = below ? d.a[16 * wave + 4 * l4 + i][16 * p + l15]
+                   : (wave == p && l15 == 4 * l4 + i ? 1.f : 0.f);
     }
-  }
+    f32x4 va[3], vb[3];
 #pragma unroll
-  for (int dist = 1; dist < 4; ++dist) {   // X_rc = -X_rr sum L_rm X_mc
-    __syncthreads();
-    const int c = wave, r = c + dist;
-    if (r < 4) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-      for (int m = c; m < r; ++m) {
-        const f32x4 l = *(f32x4*)&d.a[16 * r + l15][16 * m + 4 * l4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          acc = mfma(l[i], d.x[16 * m + 4 * l4 + i][16 * c + l15], acc);
+    for (int m = 0; m < 3; ++m)
+      if (m < p) {
+        vb[m] = *(f32x4*)&d.a[16 * p + l15][16 * m + 4 * l4];
+        va[m] = *(f32x4*)&rows[16 * wave + l15][16 * m + 4 * l4];
       }
-      const f32x4 xr = *(f32x4*)&d.x[16 * r + l15][16 * r + 4 * l4];
-      f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o = mfma(xr[i], acc[i], o);
+    for (int m = 0; m < 3; ++m)
+      if (m < p)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        d.x[16 * r + l4 * 4 + i][16 * c + l15] = -o[i];
+        for (int i = 0; i < 4; ++i) {
+          sd = mfma(vb[m][i], vb[m][i], sd);
+          if (below || m >= wave) so = mfma(va[m][i], vb[m][i], so);
+        }
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      o[i] -= so[i];
+      d.diag[wave][4 * l4 + i][l15] = dg[i] - sd[i];
     }
-  }
-  __syncthreads();
 #pragma unroll
-  for (int t = 0; t < NB * NB / 4; t += TPB) {
-    const int r = (t + tid) / (NB / 4), c = (t + tid) % (NB / 4) * 4;
-    ((f32x4*)inv)[t + tid] = c / 16 <= r / 16 ? *(f32x4*)&d.x[r][c]
-                                              : f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < 16; ++i) v[i] = d.diag[wave][i][l15];
+    columns(v, o, l15, std::make_integer_sequence<int, 16>());
+    float piv = v[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) piv = l15 == i ? v[i] : piv;
+    // (above, its reciprocal leaves the normal range)
+    bad |= !(piv >= FLT_MIN && piv <= 0x1p125f);
+    float rs = __builtin_amdgcn_rsqf(piv);
+    rs = fmaf(fmaf(-piv * rs, rs, 1.f), 0.5f * rs, rs);
+    f32x4 out;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      out[i] = o[i] * rs;
+      rows[16 * wave + 4 * l4 + i][16 * p + l15] = out[i];
+    }
+    *(f32x4*)(inv + (16 * p + l15) * NB + 16 * wave + 4 * l4) =
+        below ? f32x4{0.f, 0.f, 0.f, 0.f} : out;
   }
+  bad = __any(bad);
+  if (tid == 0 && (first || bad)) *info = bad;
 }
 
 // tile t of the lower triangle, a row's tiles from the diagonal to the left
@@ -182,36 +221,58 @@ __device__ __forceinline__ void load_rows(const float* p, f32x4 (&v)[4]) {
   for (int i = 0; i < 4; ++i) v[i] = ((const f32x4*)p)[i];
 }
 
-// S_b of step j: rows wave * 16 + l4 * 4 + i, columns t * 16 + l15
-__device__ __forceinline__ void panel(const float* __restrict__ m,
-                                      const float* __restrict__ inv, int b,
-                                      int j, int np, f32x4 (&acc)[4]) {
+// S_b of step j: rows wave * 16 + l4 * 4 + i, columns t * 16 + l15.  SIDE: where
+// b lies from j; each has its loads and products to itself, or the compiler
+// waits for the first loads before it issues the rest.
+enum Side { LEFT, AT, BELOW };
+
+template <Side SIDE>
+__device__ __forceinline__ void panel_of(const float* __restrict__ m,
+                                         const float* __restrict__ inv, int b,
+                                         int j, int np, f32x4 (&acc)[4]) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int l15 = lane & 15, l4 = lane >> 4, row = (tid >> 6) * 16 + l15;
-  if (b == j) {
+  if constexpr (SIDE == AT) {
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         acc[t][i] = inv[(t * 16 + l15) * NB + (tid >> 6) * 16 + l4 * 4 + i];
   } else {
-    f32x4 va[4], vb[4];
-    if (b > j) {
-      load_rows(m + (size_t)(b * NB + row) * np + j * NB + l4 * 16, va);
-    } else {
+    f32x4 va[4], vb[4][4];
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
-        va[i / 4][i % 4] = m[(size_t)(j * NB + l4 * 16 + i) * np + b * NB + row];
-    }
+    for (int q = 0; q < 4; ++q)
+      if constexpr (SIDE == BELOW) {
+        va[q] = *(const f32x4*)(m + (size_t)(b * NB + row) * np + j * NB +
+                                q * 16 + l4 * 4);
+      } else {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      load_rows(inv + (t * 16 + l15) * NB + l4 * 16, vb);
-      acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < 4; ++i)
+          va[q][i] = m[(size_t)(j * NB + q * 16 + l4 * 4 + i) * np + b * NB + row];
+      }
+    // D is lower triangular: its rows of block t end with block t of k
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
-        acc[t] = mfma(va[i / 4][i % 4], vb[i / 4][i % 4], acc[t]);
-    }
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int q = 0; q <= t; ++q)
+        vb[t][q] = *(const f32x4*)(inv + (t * 16 + l15) * NB + q * 16 + l4 * 4);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = q; t < 4; ++t)
+          acc[t] = mfma(va[q][i], vb[t][q][i], acc[t]);
   }
+}
+__device__ __forceinline__ void panel(const float* __restrict__ m,
+                                      const float* __restrict__ inv, int b,
+                                      int j, int np, f32x4 (&acc)[4]) {
+  if (b > j) panel_of<BELOW>(m, inv, b, j, np, acc);
+  else if (b < j) panel_of<LEFT>(m, inv, b, j, np, acc);
+  else panel_of<AT>(m, inv, b, j, np, acc);
 }
 
 // S_b, b <= j: row j of L^-1, to U
@@ -261,7 +322,7 @@ __global__ __launch_bounds__(TPB, 4) void chol_step_kernel(
     for (int v = 0; v < 2; ++v)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        old[t][v][i] = c == j ? 0.f : m[mt + (size_t)(t * 16 + i) * np + v * 16];
+        old[t][v][i] = m[mt + (size_t)(t * 16 + i) * np + v * 16];
   auto keep = [&](float (*s)[LD]) {
 #pragma unroll
     for (int t = 0; t < 4; ++t)
@@ -269,7 +330,7 @@ __global__ __launch_bounds__(TPB, 4) void chol_step_kernel(
       for (int i = 0; i < 4; ++i)
         s[wave * 16 + l4 * 4 + i][t * 16 + l15] = p[t][i];
   };
-  panel(m, inv, r, j, np, p);
+  panel_of<BELOW>(m, inv, r, j, np, p);
   keep(d.a);
   if (c != r) {
     panel(m, inv, c, j, np, p);
@@ -302,7 +363,7 @@ __global__ __launch_bounds__(TPB, 4) void chol_step_kernel(
     for (int v = 0; v < 2; ++v)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float x = old[t][v][i] - acc[t][v][i];
+        const float x = (c == j ? 0.f : old[t][v][i]) - acc[t][v][i];
         if (next) d.a[row0 + t * 16 + l4 * 4 + i][col0 + v * 16 + l15] = x;
         else mn[mt + (size_t)(t * 16 + i) * np + v * 16] = x;
       }
@@ -387,9 +448,10 @@ __global__ __launch_bounds__(TPB, 4) void chol_update_kernel(
 
 int lfmq_chol_pad(int n) { return (n + NB - 1) / NB * NB; }
 
-// One launch a step or two: us at n 512 130 / 156, 1024 256 / 314, 2048 629 / 701,
-// but 3072 1427 / 1174, where three products a tile are more than the chain.
-static bool one_launch(int N) { return N <= 32; }
+// One launch a step or two: us at n 512 101 / 127, 1024 192 / 251, 2048 470 / 575,
+// 2560 720 / 806, 3072 975 / 1043, but 3584 1340 / 1315 and 4096 1790 / 1630,
+// where three products a tile are more than the chain.
+static bool one_launch(int N) { return N <= 48; }
 
 // floats of scratch memory: M and inverse twice where a step is one launch,
 // else M, inverse and panel

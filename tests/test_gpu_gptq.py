@@ -1,4 +1,6 @@
 """GPTQ's column blocks, and the products that carry their errors on."""
+import math
+
 import pytest
 import torch
 
@@ -87,4 +89,35 @@ def test_inverse_factor_of_either_kind(n):
     gone[:64, 64:128] = 0
     assert worst_tile(gone, w) > 2e-4 and worst_tile(w.bfloat16(), w) > 2e-4
     h[n - 1, n - 1] = -h[n - 1, n - 1]
+    assert ext().chol_inverse(h)[1].item() == 1
+
+
+# the most steps of one launch, the least of two
+@pytest.mark.parametrize("n", [3072, 3073])
+def test_inverse_factor_at_the_line(n):
+    test_inverse_factor_of_either_kind(n)
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 31, 33, 48, 63, 64])
+def test_inverse_factor_of_one_block(n):
+    """Every panel of a diagonal block, columns of unequal size.  A rounding
+    moves U by the condition times 2^-24 at most, sums of n of them in random
+    directions (the scales of rows and columns cancel)."""
+    torch.manual_seed(n)
+    x = torch.randn(4 * n, n, device=DEV)
+    size = torch.exp(2 * torch.randn(n, device=DEV))
+    h64 = (x.t() @ x).double()
+    tol = 2 * math.sqrt(n) * 2 ** -24 * float(torch.linalg.cond(h64))
+    h = (h64 * size * size[:, None]).float()
+    u, failed = ext().chol_inverse(h)
+    w = torch.linalg.cholesky(torch.linalg.inv(h.double()), upper=True)
+    assert failed.item() == 0
+    assert float(u.tril(-1).abs().max()) == 0.0
+    away = (u.double() - w) * size
+    assert float(away.norm() / (w * size).norm()) <= tol
+    for i in range(n):
+        bad = h.clone()
+        bad[i, i] = -bad[i, i]
+        assert ext().chol_inverse(bad)[1].item() == 1
+    h[n // 2, n // 2] = 2.0 ** 126         # no reciprocal in the normal range
     assert ext().chol_inverse(h)[1].item() == 1
