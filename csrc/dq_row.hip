@@ -12,11 +12,21 @@
 // of all, into LDS; and four rows are summed over the lanes at once.  A row of
 // W is read by KW waves, 1 or 2 KiB in a piece, four rows ahead.
 //
-// us a call, the GEMV and this one (4 bits; the last two 8 bits):
-//   n 28672, k 4096, norm and gate  18.3 / 13.2    n 2048, k 8192   6.2 / 5.5
-//   n 4096, k 14336, residual       11.2 /  9.2    n 6144, k 4096   6.6 / 6.4
-//   n 32000, k 4096                 33.3 / 26.1    n 2048, k 8192   8.0 / 6.8
-// Eight rows ahead: 15.4; 1024 workgroups: 14.8 (n 28672).
+// Loads wait by count: x, scales and weights are asked for in this order and
+// without conditions (past an end the buffer's bounds give zeros), or the
+// compiler waits for all of them at every turn.
+//
+// us a call, the GEMV, this one with conditions and now (4 bits; the last three 8):
+//   n 28672, k 4096, norm and gate  18.3 / 13.1 / 12.8
+//   n 4096, k 14336, residual       11.2 /  9.7 /  8.9
+//   n 6144, k 4096, norm             6.6 /  6.4 /  5.8
+//   n 4096, k 4096, residual         5.2 /      /  4.6
+//   n 2048, k 8192                   6.2 /  5.5 /  4.9
+//   n 32000, k 4096                 33.3 / 27.6 / 27.0
+//   n 16384, k 2048, norm and gate       /  9.7 /  9.1
+//   n 2048, k 8192                   8.0 /  7.1 /  6.3
+// (a launch that only reads: 10.0 for n 28672, k 4096.)  Eight rows ahead: 15.4;
+// 1024 workgroups: 14.8 (n 28672).
 #include "dq_frag.h"
 
 namespace {
@@ -29,6 +39,7 @@ struct Row {
   int q, r;                              // groups of four rows of a workgroup:
                                          // q, or q + 1 of the first r
   int G, zw;
+  int kw, cw;                            // waves along k, groups at a time
 };
 
 // sums over the 64 lanes of four values: in the n-th 16 lanes the n-th one's
@@ -60,7 +71,7 @@ __global__ __launch_bounds__(MOST * 64, 4) void dq_row_kernel(Row W) {
   constexpr int WB = BITS / 4;                   // 16-byte pieces a lane
   constexpr int H = GATE ? 2 : 1, TC = 4 / H;    // columns of a group
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int lane = threadIdx.x, KW = blockDim.y, CW = blockDim.z;
+  const int lane = threadIdx.x, KW = W.kw, CW = W.cw;
   const int kw = __builtin_amdgcn_readfirstlane(threadIdx.y);
   const int cw = __builtin_amdgcn_readfirstlane(threadIdx.z);
   const int tid = (cw * KW + kw) * 64 + lane, T = KW * CW * 64;
@@ -80,43 +91,45 @@ __global__ __launch_bounds__(MOST * 64, 4) void dq_row_kernel(Row W) {
   float* sqs = part + KW * ng * 4;               // [KW]
   const u32* S0 = (const u32*)(A.scales + (u64)r0 * G);
   const u32* Z0 = A.zeros + (u64)r0 * zw;
+  // (selects, no branches, and a load for everybody: waits by count)
   auto meta_at = [&](int i) {
-    if (i < H * sd)
-      return GATE && i >= sd ? S0[(u64)nout * G / 2 + i - sd] : S0[i];
-    i -= H * sd;
-    return GATE && i >= zd ? Z0[(u64)nout * zw + i - zd] : Z0[i];
+    const bool zero = i >= H * sd;
+    i -= zero ? H * sd : 0;
+    const int one = zero ? zd : sd;
+    const u64 up = zero ? (u64)nout * zw : (u64)nout * G / 2;
+    const u32* p = zero ? Z0 : S0;
+    return p[GATE && i >= one ? up + (u64)(i - one) : (u64)i];
   };
-  constexpr int MQ = 4;
-  u32 mq[MQ];
-#pragma unroll
-  for (int i = 0; i < MQ; ++i)
-    if (tid + i * T < all) mq[i] = meta_at(tid + i * T);
-  for (int i = tid + MQ * T; i < all; i += T) meta[i] = meta_at(i);
   // this lane's 32 values of x: none past the end
   const int k0 = kw * 2048 + lane * 32;
   const bool in = k0 < k;
-  u32x4 xv[4] = {};
-  if (in) {
+  const auto xr = make_rsrc(A.x, k * 2);
+  u32x4 xv[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) xv[i] = ((const u32x4*)(A.x + k0))[i];
-  }
+  for (int i = 0; i < 4; ++i)
+    xv[i] = __builtin_amdgcn_raw_buffer_load_b128(xr, k0 * 2 + i * 16, 0, 0);
+  constexpr int MQ = 4;
+  u32 mq[MQ];
+#pragma unroll
+  for (int i = 0; i < MQ; ++i) mq[i] = meta_at(min(tid + i * T, all - 1));
+  for (int i = tid + MQ * T; i < all; i += T) meta[i] = meta_at(i);
   // row j of group g, inside the workgroup's: gate, gate, up, up
   auto column = [&](int g, int j) { return g * TC + (GATE ? j & 1 : j); };
   const u32 pitch = k * BITS / 8;
   const u32 byte = kw * 256 * BITS + lane * (BITS * 4);
   u32x4 w[AHEAD][WB];
+  // (past the last group nothing is read, but the load is there: where loads of
+  // a loop depend on conditions the compiler waits for all of them)
   auto fetch = [&](int g, int j, u32x4 (&b)[WB]) {
     const u64 row = (u64)(r0 + min(column(g, j), nr - 1)) +
                     (GATE ? (u64)(j >> 1) * nout : 0);
-    const auto rsrc = make_rsrc_uniform(A.w + row * pitch, pitch);
+    const auto rsrc = make_rsrc_uniform(A.w + row * pitch, g < ng ? pitch : 0);
 #pragma unroll
     for (int i = 0; i < WB; ++i)
       b[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, byte + i * 16, 0, 2);
   };
-  if (cw < ng) {
 #pragma unroll
-    for (int j = 0; j < AHEAD; ++j) fetch(cw, j, w[j]);
-  }
+  for (int j = 0; j < AHEAD; ++j) fetch(cw, j, w[j]);
 #pragma unroll
   for (int i = 0; i < MQ; ++i)
     if (tid + i * T < all) meta[tid + i * T] = mq[i];
@@ -182,14 +195,18 @@ __global__ __launch_bounds__(MOST * 64, 4) void dq_row_kernel(Row W) {
             c1 = fmaf((float)(d >> 24), x[3], c1);
           }
       }
-      if (g + CW < ng) fetch(g + CW, j, w[j]);
+      // (above the products it would go to other registers, and be waited for)
+      __builtin_amdgcn_sched_barrier(0);
+      fetch(g + CW, j, w[j]);
       const int lr = min(column(g, j), nr - 1) + (GATE ? (j >> 1) * nr : 0);
       const float s = bf16_bits_to_f32(ms[lr * G + gi]);
       const u32 z = (mz[lr * zw + zi] >> zs) & ((1u << BITS) - 1);
       // the bits of 128 + z, and z
       const float zb = BITS == 4 ? __builtin_bit_cast(float, z << 16 | 0x43000000u)
                                  : (float)z;
-      v[j] = in ? s * fmaf(-zb, xs, c0 + c1) : 0.f;
+      float t = s * fmaf(-zb, xs, c0 + c1);
+      asm volatile("" : "+v"(t));                // a select, no branch
+      v[j] = in ? t : 0.f;
     }
     const float t = sum4(v[0], v[1], v[2], v[3]);
     if ((lane & 15) == 0) part[(kw * ng + g) * 4 + (lane >> 4)] = t;
@@ -246,7 +263,7 @@ hipError_t go(const DqArgs& A, hipStream_t stream) {
     if (lds <= 64 * 1024 || wgs >= groups) break;
   }
   if (lds > 64 * 1024) return hipErrorInvalidValue;
-  const Row W{A, groups / grid, groups % grid, G, zw};
+  const Row W{A, groups / grid, groups % grid, G, zw, KW, CW};
   hipLaunchKernelGGL((dq_row_kernel<BITS, GATE>), dim3(grid), dim3(64, KW, CW),
                      lds, stream, W);
   return hipGetLastError();
@@ -255,11 +272,12 @@ hipError_t go(const DqArgs& A, hipStream_t stream) {
 }  // namespace
 
 // Up to eight waves along k; an even number of groups, each a lane's values or
-// more.  Smaller matrices are the GEMV's: n 4096, k 4096 5.3 us either way, n
-// 3072, k 2048 3.7 there and 4.1 here.
+// more.  Smaller matrices are the GEMV's, us of both: n 2048, k 2048 3.4 / 3.4, n
+// 1024, k 4096 3.4 / 3.4 (from there on this one: n 3072, k 2048 3.7 / 3.5, n 1024, k
+// 8192 5.2 / 3.7, n 4096, k 2048 with norm and gate 5.0 / 3.8).
 bool lfmq_dq_row_ok(int n, int k, int g) {
   return n >= 1 && k <= MOST * 2048 && g % 32 == 0 && k % (2 * g) == 0 &&
-         (k >= 8192 ? (long)n * k > 12l << 20 : (long)n * k > 16l << 20);
+         (long)n * k >= 4l << 20;
 }
 
 // rms_eps >= 0: x over its root mean square; glu: y [n / 2] = silu(gate) up of

@@ -78,6 +78,17 @@ def test_one_row(bits, n, k, g):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("n,k,g", [
+    (2050, 2048, 32), (1366, 3072, 128), (1027, 4096, 64), (514, 8192, 128),
+    (259, 16384, 64)])
+def test_one_row_of_few_weights(bits, n, k, g):
+    """The least that is not the GEMV's: fewer groups than waves, waves without
+    any, a short last wave."""
+    torch.manual_seed(n + bits)
+    check(bits, 1, n, k, g)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("m,n,k,g", [
     (2, 2049, 2048, 128), (3, 3074, 2304, 64), (4, 4098, 4096, 128),
     (5, 2050, 2048, 64), (8, 28674, 4096, 128), (9, 8198, 4352, 128),
