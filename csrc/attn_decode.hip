@@ -21,29 +21,30 @@
 // ticket counter) or, without tickets, a second kernel does.
 //
 // A launch that only reads 402 MB takes 66 us, one of 33 MB 6.5: the rest is a
-// chain from the length over the rotation to the keys, sums over the lanes, and
-// the merge's trips to memory.  One layer of an 8B model (32 query heads on 8),
-// us before and now (tickets that emptied the XCD's caches, two waves a SIMD,
-// ranges of 256 keys):
-//   b 1,  T 129        9.0 ->  8.4      b 8,  T 4000     64   -> 29.1
-//   b 1,  T 7901      20.9 -> 16.1      b 20, T 900      42   -> 20.1
-//   b 8,  T 1000      20.2 -> 13.7      b 48, T 2047    117   -> 77 (5.2 TB/s)
-// Still slower than before: 8 query heads on one, b 1 and 2, 6000 keys and more
-// (20.3 -> 21.9 at 8000), and some 800 workgroups of one range (8 heads, b 100,
-// 8000 keys: 568 -> 601), whose second round is all but empty.
+// chain from the length over the keys and the rotation to the scores, sums over
+// the lanes, and the merge's trips to memory.  So a wave's first keys and values
+// are on their way before the rotation and the next ones during a round, by loads
+// that stop at the range's end and wait by count; sums over the lanes are taken two
+// at a time by exchanges of lanes and not through LDS.  One layer of an 8B model
+// (32 query heads on 8), us before (loads in the round that needs them) and now:
+//   b 1,  T 129         8.1 ->  6.3      b 8,  T 4000     30.9 -> 28.5
+//   b 1,  T 7901       16.0 -> 13.8      b 20, T 900      21.6 -> 19.4
+//   b 8,  T 1000       13.4 -> 11.5      b 48, T 2047     80.2 -> 76.6 (5.2 TB/s)
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
 
-constexpr int TPB = 256, NW = 4, KT = 32;
+constexpr int KT = 32;               // keys of a wave and round
 constexpr int MAX_SPLITS = 64;       // a wave merges them, one a lane
 // A merge costs 2 us, two rounds of a wave's 32 keys 1.5 more than one.  Up to
 // ONE_RANGE keys are one range; longer ranges than LEAST_KEYS where there would
 // be more than MANY of them, of the keys that there are: a cache that is half
-// full has as many.  us with least ranges of 128 / 256 keys (b 1): 9.2 / 8.2 at
-// 129 keys, 9.7 / 11.3 at 700, 11.2 / 11.9 at 2000, 13.7 / 13.2 at 4000; 21.0 /
-// 16.1 at 8000 of 16100, 63 and 32 ranges; 25.7 / 23.0 with 8 heads a workgroup
-// (b 2, 4000), but 18.2 / 19.2 with one workgroup a range (3200).
+// full has as many.  us (32 heads on 8, b 1) with one range up to 128 / 256 keys
+// 6.6 / 6.2 at 150 keys (b 4 7.0 / 6.3); with least ranges of 128 / 256 7.0 / 8.1
+// at 700, 8.0 / 8.8 at 1500, 10.3 / 10.3 at 4000, but b 12 10.4 / 9.4 at 400 and
+// 12.4 / 13.2 at 700.
 constexpr int ONE_RANGE = 256, LEAST_KEYS = 128, MANY = 24;
 // Two workgroups a CU, three where a range has very many keys: us with 512 / 768
 // workgroups 14.3 / 15.2 (b 8, 1000 keys), 18.4 / 19.2 (b 16, 900), 81.5 / 77
@@ -66,12 +67,13 @@ struct DArgs {
 };
 
 // keys a range: all ranges alike, whole wave tiles
+template <int NW>
 __device__ __forceinline__ int range_keys(const DArgs& A, int len) {
   // (len + splits - 1) / splits, exact below 2^26 keys
   const int per = A.splits == 1 ? len
                                 : (int)(((u64)(u32)(len + A.splits - 1) *
                                          A.inv_splits) >> 32);
-  const int least = len <= ONE_RANGE ? ONE_RANGE
+  const int least = NW == 8 || len <= ONE_RANGE ? ONE_RANGE
                     : len <= MANY * LEAST_KEYS ? LEAST_KEYS : 2 * LEAST_KEYS;
   return (max(per, least) + KT - 1) / KT * KT;
 }
@@ -86,6 +88,31 @@ __device__ __forceinline__ float max_across(float v) {
   const auto q = __builtin_amdgcn_permlane16_swap(y, y, false, false);
   const u32 q0 = q[0], q1 = q[1];
   return fmaxf(__builtin_bit_cast(float, q0), __builtin_bit_cast(float, q1));
+}
+
+__device__ __forceinline__ float sum_across(float v) {
+  const u32 x = __builtin_bit_cast(u32, v);
+  const auto p = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  const u32 p0 = p[0], p1 = p[1];
+  const u32 y = __builtin_bit_cast(u32, __builtin_bit_cast(float, p0) +
+                                            __builtin_bit_cast(float, p1));
+  const auto q = __builtin_amdgcn_permlane16_swap(y, y, false, false);
+  const u32 q0 = q[0], q1 = q[1];
+  return __builtin_bit_cast(float, q0) + __builtin_bit_cast(float, q1);
+}
+// a of both halves in the lower one, b in the upper one
+__device__ __forceinline__ float sum_halves(float a, float b) {
+  const auto p = __builtin_amdgcn_permlane32_swap(
+      __builtin_bit_cast(u32, a), __builtin_bit_cast(u32, b), false, false);
+  const u32 p0 = p[0], p1 = p[1];
+  return __builtin_bit_cast(float, p0) + __builtin_bit_cast(float, p1);
+}
+// the same in each half: 16 lanes and 16
+__device__ __forceinline__ float sum_quarters(float a, float b) {
+  const auto p = __builtin_amdgcn_permlane16_swap(
+      __builtin_bit_cast(u32, a), __builtin_bit_cast(u32, b), false, false);
+  const u32 p0 = p[0], p1 = p[1];
+  return __builtin_bit_cast(float, p0) + __builtin_bit_cast(float, p1);
 }
 
 // Two floats of a partial result, past the caches of the XCD: a workgroup of
@@ -111,13 +138,15 @@ __device__ __forceinline__ float merge_weight(const float* p, int used,
   const bool on = lane < used;
   float m = -INFINITY, l = 0.f;
   if (on) get2(p + lane * stride + D, m, l);
-  const float M = wave_reduce_max(m);
+  const float M = wave_reduce_max_dpp(m);
   const float e = on ? __expf(m - M) : 0.f;
-  return e / wave_reduce_sum(e * l);
+  return e / wave_reduce_sum_dpp(e * l);
 }
 
-template <int D, int GH, bool FUSED>
-__global__ __launch_bounds__(TPB, D * GH > 512 ? 2 : 3) void attn_decode_kernel(DArgs A) {
+template <int D, int GH, bool FUSED, int NW>
+__global__ __launch_bounds__(NW * 64, NW == 8 || D * GH > 512 ? 2 : 3)
+void attn_decode_kernel(DArgs A) {
+  constexpr int TPB = NW * 64;
   constexpr int KS = D / 32, LPR = D / 8;
   constexpr int RPP = 64 / LPR;          // value rows a pass
   constexpr int NP = KT / RPP;           // passes a tile
@@ -163,11 +192,40 @@ __global__ __launch_bounds__(TPB, D * GH > 512 ? 2 : 3) void attn_decode_kernel(
     }
   }
   const int len = min(T, A.tmax);
-  const int per = range_keys(A, len);
+  const int per = range_keys<NW>(A, len);
   const int lo = range * per, hi = min(len, lo + per);
   if (lo >= hi) return;
   unsigned short* K = A.kc + ((u64)bb * A.hkv + kh) * A.tmax * D;
   unsigned short* V = A.vc + ((u64)bb * A.hkv + kh) * A.tmax * D;
+  // A wave's keys and values from t0 on, zeros past the range.  The first are on
+  // their way beside the rotation, the next ones as soon as there is room for
+  // them; the loads are there without keys too, or the compiler waits for all.
+  s16x8 kf[2][KS];
+  u32x4 vv[NP];
+  auto rows_of = [&](const unsigned short* base, int t0) {
+    const int n = max(0, min(KT, hi - t0));
+    return make_rsrc_uniform(base + (u64)(n > 0 ? t0 : 0) * D, (u32)n * D * 2);
+  };
+  auto load_keys = [&](int t0) {
+    const auto r = rows_of(K, t0);
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        kf[mt][ks] = __builtin_bit_cast(
+            s16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                       r, ((mt * 16 + l15) * D + ks * 32 + l4 * 8) * 2, 0, 0));
+  };
+  auto load_values = [&](int t0) {
+    const auto r = rows_of(V, t0);
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      vv[i] = __builtin_amdgcn_raw_buffer_load_b128(
+          r, ((i * RPP + vrow) * D + vcol) * 2, 0, 0);
+  };
+  const int first = lo + __builtin_amdgcn_readfirstlane(wave) * KT;
+  load_keys(first);
+  load_values(first);
   const int pos = FUSED ? T - 1 : -1;    // the new key
   if constexpr (FUSED) {
     float sn, cs;
@@ -208,20 +266,7 @@ __global__ __launch_bounds__(TPB, D * GH > 512 ? 2 : 3) void attn_decode_kernel(
 
   float m = -INFINITY, l = 0.f;          // of head l15
   float acc[GH][8] = {};
-  for (int t0 = lo + wave * KT; t0 < hi; t0 += NW * KT) {
-    s16x8 kf[2][KS];
-    u32x4 vv[NP];
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-      const unsigned short* kr = K + (u64)min(t0 + mt * 16 + l15, hi - 1) * D;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        kf[mt][ks] = *(const s16x8*)(kr + ks * 32 + l4 * 8);
-    }
-#pragma unroll
-    for (int i = 0; i < NP; ++i)
-      vv[i] = *(const u32x4*)(V + (u64)min(t0 + i * RPP + vrow, hi - 1) * D +
-                              vcol);
+  for (int t0 = first; t0 < hi; t0 += NW * KT) {
     f32x4 sc[2] = {};
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
@@ -229,6 +274,8 @@ __global__ __launch_bounds__(TPB, D * GH > 512 ? 2 : 3) void attn_decode_kernel(
       for (int mt = 0; mt < 2; ++mt)
         sc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[mt][ks], qf[ks],
                                                          sc[mt], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);         // not before: other registers
+    load_keys(t0 + NW * KT);
     float mx = -INFINITY;
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
@@ -261,13 +308,7 @@ __global__ __launch_bounds__(TPB, D * GH > 512 ? 2 : 3) void attn_decode_kernel(
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc[h][e] *= a;
     }
-    // rows past the range are the last one again: 0, which their weight of 0
-    // leaves 0 (an infinite value would be NaN)
-    if (t0 + KT > hi) {
-#pragma unroll
-      for (int i = 0; i < NP; ++i)
-        if (t0 + i * RPP + vrow >= hi) vv[i] = u32x4{0, 0, 0, 0};
-    }
+    // (rows past the range are zeros, which their weight of 0 leaves 0)
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
       if (FUSED && t0 + i * RPP + vrow == pos) vv[i] = v_new;
@@ -283,21 +324,30 @@ __global__ __launch_bounds__(TPB, D * GH > 512 ? 2 : 3) void attn_decode_kernel(
         for (int e = 0; e < 8; ++e) acc[h][e] = fmaf(p, v[e], acc[h][e]);
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
+    load_values(t0 + NW * KT);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // ps is read
   }
 
-  // lanes and rows of one wave, then the waves
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  // lanes and rows of one wave, then the waves.  Two sums at a time: halves, then
+  // quarters of the wave end up with one each, in all R of GH * 8
+  l = sum_across(l);
+  constexpr int NV = GH * 8, R = NV / 4;
+  float* a1 = &acc[0][0];
+  if constexpr (LPR == 8)
 #pragma unroll
-  for (int h = 0; h < GH; ++h)
+    for (int v = 0; v < NV; ++v)
+      a1[v] += __builtin_bit_cast(
+          float, __builtin_amdgcn_update_dpp(
+                     0, __builtin_bit_cast(int, a1[v]), 0x128, 0xf, 0xf, true));
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
+  for (int v = 0; v < NV / 2; ++v) a1[v] = sum_halves(a1[v], a1[v + NV / 2]);
 #pragma unroll
-      for (int o = LPR; o < 64; o <<= 1)
-        acc[h][e] += __shfl_xor(acc[h][e], o, 64);
-      if (lane < LPR) ws[wave][h][vcol + e] = acc[h][e];
-    }
+  for (int v = 0; v < R; ++v) {
+    const float x = sum_quarters(a1[v], a1[v + R]);
+    const int at = l4 * R + v;               // of the heads' columns
+    if (l15 < LPR) ws[wave][at / 8][vcol + at % 8] = x;
+  }
   if (lane < GH) {
     ml[wave][lane][0] = m;
     ml[wave][lane][1] = l;
@@ -309,8 +359,9 @@ __global__ __launch_bounds__(TPB, D * GH > 512 ? 2 : 3) void attn_decode_kernel(
   const int hstep = A.splits * (D + 2);
   for (int id = tid; id < nh * (D / 2); id += TPB) {
     const int h = id / (D / 2), e = id % (D / 2) * 2;
-    const float M = fmaxf(fmaxf(ml[0][h][0], ml[1][h][0]),
-                          fmaxf(ml[2][h][0], ml[3][h][0]));
+    float M = ml[0][h][0];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) M = fmaxf(M, ml[w][h][0]);
     float o0 = 0.f, o1 = 0.f, L = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
@@ -390,10 +441,10 @@ __global__ __launch_bounds__(TPB, D * GH > 512 ? 2 : 3) void attn_decode_kernel(
 }
 
 // the merge as a kernel of its own: one head a wave
-template <int D>
+template <int D, int NW>
 __global__ __launch_bounds__(64) void attn_decode_merge(DArgs A) {
   const int len = min(A.T_dev != nullptr ? *A.T_dev : A.T, A.tmax);
-  const int per = range_keys(A, len);
+  const int per = range_keys<NW>(A, len);
   const int used = (len + per - 1) / per;
   if (used <= 1) return;
   __shared__ float wt[MAX_SPLITS];
@@ -416,6 +467,16 @@ int head_tile(int group) {
   return group <= 1 ? 1 : (group <= 2 ? 2 : (group <= 4 ? 4 : 8));
 }
 
+// Eight waves a workgroup, ranges of one round of theirs: eight heads of 128,
+// whose rounds are the longest, where that is a workgroup a CU or less.  us with
+// four / eight (8 heads on one key head, of 128): 11.9 / 10.2 at 1500 keys (b 1, 4
+// key heads), 18.5 / 14.1 at 8000, 16.6 / 13.8 (b 3, 4000), 5.7 / 6.1 at 60; of 64
+// 10.6 / 9.6 to 7.0 / 7.8; 4 heads of 128 7.0 / 8.4 at 600 keys, 10.2 / 10.5 at 4000.
+bool eight_waves(int d, int gh, int wgs, int T) {
+  return d == 128 && gh == 8 && T <= MAX_SPLITS * ONE_RANGE &&
+         (long)wgs * ((T + ONE_RANGE - 1) / ONE_RANGE) <= 256;
+}
+
 template <int D, bool FUSED>
 hipError_t launch(DArgs A, int b, hipStream_t stream) {
   const int group = A.hq / A.hkv, gh = head_tile(group);
@@ -427,26 +488,32 @@ hipError_t launch(DArgs A, int b, hipStream_t stream) {
   // would get all of those.  us with ranges first / second / last: 32 heads on
   // 32, b 4, 200 keys of 500 9.6 / 8.4 / 7.2; 28 on 4, b 20 15.7 / 15.1 / 13.4.
   const dim3 grid(A.hkv * A.htiles, b, A.splits);
-#define GO(G)                                                               \
-  hipLaunchKernelGGL((attn_decode_kernel<D, G, FUSED>), grid, dim3(TPB), 0, \
-                     stream, A)
-  if (gh == 1) GO(1);
-  else if (gh == 2) GO(2);
-  else if (gh == 4) GO(4);
-  else GO(8);
-#undef GO
-  if (A.splits > 1 && A.tickets == nullptr)
-    hipLaunchKernelGGL((attn_decode_merge<D>), dim3(b * A.hq), dim3(64), 0,
-                       stream, A);
+  auto go = [&](auto heads, auto waves) {
+    constexpr int G = decltype(heads)::value, NW = decltype(waves)::value;
+    hipLaunchKernelGGL((attn_decode_kernel<D, G, FUSED, NW>), grid,
+                       dim3(NW * 64), 0, stream, A);
+    if (A.splits > 1 && A.tickets == nullptr)
+      hipLaunchKernelGGL((attn_decode_merge<D, NW>), dim3(b * A.hq), dim3(64), 0,
+                         stream, A);
+  };
+  constexpr std::integral_constant<int, 4> four{};
+  if (gh == 1) go(std::integral_constant<int, 1>(), four);
+  else if (gh == 2) go(std::integral_constant<int, 2>(), four);
+  else if (gh == 4) go(four, four);
+  else if (eight_waves(D, gh, b * A.hkv * A.htiles, A.T))
+    go(std::integral_constant<int, 8>(), std::integral_constant<int, 8>());
+  else
+    go(std::integral_constant<int, 8>(), four);
   return hipGetLastError();
 }
 
 }  // namespace
 
 // Key ranges a head for up to T keys.
-int lfmq_attn_decode_splits(int b, int hq, int hkv, int T) {
+int lfmq_attn_decode_splits(int b, int hq, int hkv, int T, int d) {
   const int group = hq / hkv, gh = head_tile(group);
   const int wgs = b * hkv * ((group + gh - 1) / gh);
+  if (eight_waves(d, gh, wgs, T)) return max(1, (T + ONE_RANGE - 1) / ONE_RANGE);
   int n = FULL_WGS / max(wgs, 1);
   // (eight heads a workgroup: two of them a CU)
   if (gh < 8 && T > max(n, 1) * LONG_RANGE) n = MORE_WGS / max(wgs, 1);

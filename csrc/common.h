@@ -102,6 +102,25 @@ __device__ __forceinline__ float wave_reduce_sum_dpp(float v) {
   return __builtin_bit_cast(
       float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
+__device__ __forceinline__ float wave_reduce_max_dpp(float v) {
+#define LFMQ_DPP_MAX(ctrl)                                                  \
+  v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(       \
+                       __builtin_bit_cast(int, v),                          \
+                       __builtin_bit_cast(int, v), (ctrl), 0xf, 0xf, false)))
+  LFMQ_DPP_MAX(0xB1);   // the neighbour
+  LFMQ_DPP_MAX(0x4E);   // the other two of four
+  LFMQ_DPP_MAX(0x141);  // eight, mirrored
+  LFMQ_DPP_MAX(0x140);  // sixteen, mirrored
+#undef LFMQ_DPP_MAX
+  const u32 x = __builtin_bit_cast(u32, v);
+  const auto p = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  const u32 p0 = p[0], p1 = p[1];
+  const u32 y = __builtin_bit_cast(u32, fmaxf(__builtin_bit_cast(float, p0),
+                                              __builtin_bit_cast(float, p1)));
+  const auto q = __builtin_amdgcn_permlane16_swap(y, y, false, false);
+  const u32 q0 = q[0], q1 = q[1];
+  return fmaxf(__builtin_bit_cast(float, q0), __builtin_bit_cast(float, q1));
+}
 __device__ __forceinline__ float wave_reduce_max(float v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));

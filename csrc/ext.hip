@@ -51,7 +51,7 @@ hipError_t lfmq_attn_decode_fused(const void*, void*, void*, void*, void*,
                                   const void*, int, int, int, int, int,
                                   const void*, int, int, float, void*,
                                   hipStream_t);
-int lfmq_attn_decode_splits(int, int, int, int);
+int lfmq_attn_decode_splits(int, int, int, int, int);
 hipError_t lfmq_attn_prefill(const void*, const void*, const void*, void*,
                              int, int, int, int, int, int, int, float,
                              hipStream_t);
@@ -533,7 +533,7 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
   const int hkv = (int)kc.size(1), tmax = (int)kc.size(2);
   // graph mode (t_dev set): seq_len is MAX T; grid fixed, T read on device
   TORCH_CHECK(hq % hkv == 0, "query heads must share key heads evenly");
-  const int splits = lfmq_attn_decode_splits(b, hq, hkv, (int)seq_len);
+  const int splits = lfmq_attn_decode_splits(b, hq, hkv, (int)seq_len, d);
   auto scratch = torch::empty({(long)b * hq * splits * (d + 2)},
                               q.options().dtype(torch::kFloat32));
   auto o = torch::empty_like(q);
@@ -934,7 +934,7 @@ torch::Tensor attn_decode_fused(torch::Tensor qkv, torch::Tensor kc,
   const int b = (int)kc.size(0), hkv = (int)kc.size(1);
   const int tmax = (int)kc.size(2), d = (int)kc.size(3);
   TORCH_CHECK(hq % hkv == 0, "query heads must share key heads evenly");
-  const int splits = lfmq_attn_decode_splits(b, (int)hq, hkv, (int)seq_len);
+  const int splits = lfmq_attn_decode_splits(b, (int)hq, hkv, (int)seq_len, d);
   auto scratch = torch::empty({(long)b * hq * splits * (d + 2)},
                               qkv.options().dtype(torch::kFloat32));
   auto o = torch::empty({(long)b, 1L, hq * (long)d}, qkv.options());
