@@ -20,7 +20,7 @@
 // passes by the caches where its rows are whole lines.  2048 x 14336: 673 us
 // with H read after the products, 629 with loads ahead, 545 past the caches
 // too (772 TFLOP/s of the half computed); 512 x 8192: 122 and 100;
-// 2048 x 4096: 78 and 70; 2048 x 2048: 33, 64 x 512: 9.3 (one round of
+// 2048 x 4096: 78 and 65; 2048 x 2048: 33, 64 x 512: 7.9 (one round of
 // workgroups, below).  Matrix cores are busy 40 % of the time, memory 65 %:
 // two workgroups of one wave a SIMD each hide no more of each other.
 #include "lds_dma.h"
@@ -43,15 +43,16 @@ __device__ __forceinline__ int chunk_key(int token) {
   return (token & 7) ^ ((token >> 1) & 4);
 }
 
-// How H is read and written.  DIRECT: a single round of workgroups, which wait
-// for memory once, straight from the fragments (64 x 512: 9.3 us, 13.9 through
-// LDS).  WHOLE: more workgroups, rows of H whole lines, past the caches.
+// How H is read and written.  DIRECT: a single round of workgroups, one a CU, which
+// wait for memory once, straight from the fragments, with registers for all of a
+// thread's elements (64 x 512 with clearing H: 9.6 us, 11.0 row by row in half the
+// registers; 478 x 1616 21.8, 23.3).  WHOLE: more workgroups, rows of H whole lines, past the caches.
 // CACHED: the same where neighbouring tiles share lines, which then have to
 // meet in a cache (102 x 7416: 81 us, 107 past it).
 enum Way { DIRECT, WHOLE, CACHED };
 
 template <Way WAY>
-__global__ __launch_bounds__(TPB, 2) void hessian_kernel(
+__global__ __launch_bounds__(TPB, WAY == DIRECT ? 1 : 2) void hessian_kernel(
     const unsigned short* __restrict__ x, float* __restrict__ h, int t,
     int k) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -139,54 +140,82 @@ __global__ __launch_bounds__(TPB, 2) void hessian_kernel(
               a[i], b[j], acc[i][j], 0, 0, 0);
     }
   };
-  // the last step by itself: behind its loads those of H are on their way (in
-  // the same loop their registers are copied at each turn: 724 us for 545)
-  const int end = (t - 1) / BK * BK;
-  int par = 0;
-  stage(0, 0);
-  for (int t0 = 0; t0 < end; t0 += BK, par ^= 1) {
-    loads_but<0>();
-    stage(t0 + BK, par ^ 1);
-    products(par);
-  }
-  if (WAY != DIRECT) fours_load(own, i0, j0);
-  loads_but<WAY == DIRECT ? 0 : NF>();
-  if (end + BK > t) {
+  // tokens past the end of the last step
+  auto clear = [&](int t0, int par) {
+    if (t0 + BK <= t) return;
     const u32x4 z = {0, 0, 0, 0};
-    for (int i = (t - end) * 16 + tid; i < BK * 16; i += TPB) {
+    for (int i = (t - t0) * 16 + tid; i < BK * 16; i += TPB) {
       *(u32x4*)(smem + par * BUF + i * 16) = z;
       *(u32x4*)(smem + par * BUF + BUF / 2 + i * 16) = z;
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  int par = 0;
+  stage(0, 0);
+  if constexpr (WAY == DIRECT) {
+    for (int t0 = 0; t0 < t; t0 += BK, par ^= 1) {
+      loads_but<0>();
+      if (t0 + BK < t) stage(t0 + BK, par ^ 1);
+      else clear(t0, par);
+      products(par);
+    }
+  } else {
+    // The last step by itself: behind its loads those of H are on their way (in
+    // the same loop their registers are copied at each turn: 724 us for 545).  A
+    // second copy of the products costs a single round 1.2 us of fetching it.
+    const int end = (t - 1) / BK * BK;
+    for (int t0 = 0; t0 < end; t0 += BK, par ^= 1) {
+      loads_but<0>();
+      stage(t0 + BK, par ^ 1);
+      products(par);
+    }
+    fours_load(own, i0, j0);
+    loads_but<NF>();
+    clear(end, par);
+    products(par);
   }
-  products(par);
   // H += 2 acc, here and mirrored
   if constexpr (WAY == DIRECT) {
+    // All of a thread's elements on their way at once, places past the end out of
+    // the buffer's bounds (by rows of fragments, in conditions: 1.1 us more)
+    const auto hr = make_rsrc(h, (u32)k * (u32)k * 4);
+    float v[4][4][4];
+    f32x4 u[4][4];
+    auto place = [&](int row, int col, bool in) {
+      return in && row < k && col < k ? (u32)(row * k + col) * 4 : ~0u;
+    };
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = i0 + wi * 64 + i * 16 + l4 * 4;
-      float v[4][4];
-      f32x4 u[4];
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
+        const int row = i0 + wi * 64 + i * 16 + l4 * 4;
         const int col = j0 + wj * 64 + j * 16 + l15;
-        if (row >= k || col >= k) continue;  // k in eights: four rows alike
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[j][r] = h[(u64)(row + r) * k + col];
-        if (ti != tj) u[j] = *(const f32x4*)(h + (u64)col * k + row);
+        for (int r = 0; r < 4; ++r)
+          v[i][j][r] = __builtin_bit_cast(
+              float, __builtin_amdgcn_raw_buffer_load_b32(
+                         hr, place(row + r, col, true), 0, 0));
+        u[i][j] = __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                       hr, place(col, row, ti != tj), 0, 0));
       }
 #pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
       for (int j = 0; j < 4; ++j) {
+        const int row = i0 + wi * 64 + i * 16 + l4 * 4;
         const int col = j0 + wj * 64 + j * 16 + l15;
-        if (row >= k || col >= k) continue;
+        f32x4 w;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          h[(u64)(row + r) * k + col] = fmaf(2.f, acc[i][j][r], v[j][r]);
-          u[j][r] = fmaf(2.f, acc[i][j][r], u[j][r]);
+          __builtin_amdgcn_raw_buffer_store_b32(
+              __builtin_bit_cast(u32, fmaf(2.f, acc[i][j][r], v[i][j][r])), hr,
+              place(row + r, col, true), 0, 0);
+          w[r] = fmaf(2.f, acc[i][j][r], u[i][j][r]);
         }
-        if (ti != tj) *(f32x4*)(h + (u64)col * k + row) = u[j];
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, w), hr,
+                                               place(col, row, ti != tj), 0, 0);
       }
-    }
   } else {
     // (LD: rows and columns both spread over the banks)
     float* out = (float*)smem;
@@ -233,14 +262,16 @@ hipError_t lfmq_hessian_accum(const void* x, void* h, int t, int k,
                               hipStream_t stream) {
   if (k % 8) return hipErrorInvalidValue;
   if (t == 0 || k == 0) return hipSuccess;
-  const u32 n = ceil_div_u32(k, BC * SB), tiles = ceil_div_u32(k, BC);
-  const bool direct = tiles * (tiles + 1) / 2 <= 256;
+  const u32 n = ceil_div_u32(k, BC * SB), wgs = n * (n + 1) / 2 * SB * SB;
+  // (of 336, 231 with a tile, some XCD has more than CUs: 1469 x 2584 59 us, 51
+  // the other way)
+  const bool direct = wgs <= 256;
   const int lds = direct ? 2 * BUF : max(2 * BUF, BC * LD * 4);
   auto* kernel = direct ? hessian_kernel<DIRECT>
                         : (k % 32 == 0 && (u64)h % 128 == 0
                                ? hessian_kernel<WHOLE>
                                : hessian_kernel<CACHED>);
-  hipLaunchKernelGGL(kernel, dim3(n * (n + 1) / 2 * SB * SB), dim3(TPB), lds,
+  hipLaunchKernelGGL(kernel, dim3(wgs), dim3(TPB), lds,
                      stream, (const unsigned short*)x, (float*)h, t, k);
   return hipGetLastError();
 }

@@ -404,12 +404,13 @@ def test_hessian_accum_tiles(t, k):
                  <= (t + 1) * bound.double()).all())
 
 
-@pytest.mark.parametrize("t,k,off", [(1, 2944, 0), (64, 3104, 0),
-                                     (65, 2824, 0), (130, 2944, 1)])
+@pytest.mark.parametrize("t,k,off", [
+    (1, 2944, 0), (64, 3104, 0), (65, 2824, 0), (130, 2944, 1), (70, 2568, 0),
+    (33, 2560, 0), (129, 2552, 1), (5, 136, 3)])
 def test_hessian_accum_past_caches(t, k, off):
-    """More than a round of tiles: rows of H whole lines and not, an H that
-    begins within a line; what lies before and behind it stays.  Bound as
-    above."""
+    """The most tiles of a single round, and more: rows of H whole lines and
+    not, an H that begins within a line; what lies before and behind it stays.
+    Bound as above."""
     torch.manual_seed(t + k)
     x = torch.randn(t, k).to(torch.bfloat16)
     room = torch.randn(off + k * k + 8)
