@@ -196,10 +196,12 @@ __device__ __forceinline__ void tile_of(int t, int& r, int& c) {
   c = r - (t - r * (r + 1) / 2);
 }
 
-// M = J H J, lower triangle (of H also), identity past n; factors block 0
+// M = J H J, lower triangle (of H also), identity past n; factors block 0.
+// diag: H's diagonal instead of its own, or null
 __global__ __launch_bounds__(TPB, 4) void chol_begin_kernel(
-    const float* __restrict__ h, float* __restrict__ m,
-    float* __restrict__ inv, int* __restrict__ info, int n, int np) {
+    const float* __restrict__ h, const float* __restrict__ diag,
+    float* __restrict__ m, float* __restrict__ inv, int* __restrict__ info,
+    int n, int np) {
   __shared__ Diag d;
   int r, c;
   tile_of(blockIdx.x, r, c);
@@ -207,8 +209,10 @@ __global__ __launch_bounds__(TPB, 4) void chol_begin_kernel(
     // neighbouring threads: neighbouring i, which H's rows run along
     const int i = r * NB + t % NB, k = c * NB + t / NB;
     const int lo = max(i, k), hi = min(i, k);
-    const float v = lo < n ? h[(size_t)(n - 1 - hi) * n + n - 1 - lo]
-                           : (i == k ? 1.f : 0.f);
+    const float* p = i == k && diag != nullptr
+                         ? diag + (n - 1 - i)
+                         : h + (size_t)(n - 1 - hi) * n + n - 1 - lo;
+    const float v = lo < n ? *p : (i == k ? 1.f : 0.f);
     if (r == 0) d.a[t % NB][t / NB] = v;
     else m[(size_t)i * np + k] = v;
   }
@@ -461,10 +465,12 @@ long lfmq_chol_scratch(int n) {
                             : np * np + NB * NB + np * NB;
 }
 
-// h [n, n] fp32 (its lower triangle), u [n, n] zeros, scratch of
-// lfmq_chol_scratch; info: 1 if a pivot was not positive.
-hipError_t lfmq_chol_inverse(const void* h, void* u, void* scratch, void* info,
-                             int n, hipStream_t stream) {
+// h [n, n] fp32 (its lower triangle), diag [n] to take its diagonal's place or
+// null, u [n, n] zeros, scratch of lfmq_chol_scratch; info: 1 if a pivot was not
+// positive.
+hipError_t lfmq_chol_inverse(const void* h, const void* diag, void* u,
+                             void* scratch, void* info, int n,
+                             hipStream_t stream) {
   const int np = lfmq_chol_pad(n), N = np / NB;
   if (n < 1 || N > 32768) return hipErrorInvalidValue;
   const size_t sq = (size_t)np * np;
@@ -472,7 +478,8 @@ hipError_t lfmq_chol_inverse(const void* h, void* u, void* scratch, void* info,
   float* inv = m + sq;
   float* s = inv + NB * NB;                // panel, or the other M and inverse
   hipLaunchKernelGGL(chol_begin_kernel, dim3(N * (N + 1) / 2), dim3(TPB), 0,
-                     stream, (const float*)h, m, inv, (int*)info, n, np);
+                     stream, (const float*)h, (const float*)diag, m, inv,
+                     (int*)info, n, np);
   if (one_launch(N)) {
     for (int j = 0; j < N; ++j) {
       float* m1 = j & 1 ? s : m;

@@ -57,13 +57,19 @@ hipError_t lfmq_attn_prefill(const void*, const void*, const void*, void*,
                              hipStream_t);
 hipError_t lfmq_hessian_accum(const void*, void*, int, int, hipStream_t);
 long lfmq_chol_scratch(int n);
-hipError_t lfmq_chol_inverse(const void*, void*, void*, void*, int,
+hipError_t lfmq_chol_inverse(const void*, const void*, void*, void*, void*, int,
                              hipStream_t);
+hipError_t lfmq_gptq_prepare(const void*, const void*, void*, void*, int, int,
+                             float, hipStream_t);
 hipError_t lfmq_gptq_block(const void*, const void*, int, void*, void*, void*,
                            void*, int, int, int, int, int, int, int, bool,
                            hipStream_t);
 hipError_t lfmq_gptq_push(const void*, const void*, const void*, long, int, int,
                           int, int, hipStream_t);
+bool lfmq_gptq_step_ok(const void*, long, int, int, int);
+hipError_t lfmq_gptq_step(const void*, const void*, long, void*, void*, void*,
+                          const void*, void*, int, int, int, int, int, int, bool,
+                          hipStream_t);
 hipError_t lfmq_dq_gemv_gateup(const void*, const void*, const void*,
                                const void*, void*, int, int, int, int, int,
                                float, int, hipStream_t);
@@ -1029,18 +1035,43 @@ void hessian_accum(torch::Tensor h, torch::Tensor x) {
 }
 
 // U upper triangular, U^T U = h^-1, and [1]: not 0 if h (its lower triangle)
-// is not positive definite in fp32
-std::vector<torch::Tensor> chol_inverse(torch::Tensor h) {
+// is not positive definite in fp32.  diag takes the place of h's diagonal
+std::vector<torch::Tensor> chol_inverse(torch::Tensor h,
+                                        c10::optional<torch::Tensor> diag) {
   check_t(h, torch::kFloat32, "h");
   TORCH_CHECK(h.dim() == 2 && h.size(0) == h.size(1) && h.size(0) > 0,
               "h must be [n, n]");
   const int n = (int)h.size(0);
+  const void* dptr = nullptr;
+  if (diag.has_value()) {
+    check_t(*diag, torch::kFloat32, "diag");
+    TORCH_CHECK(diag->numel() == n, "diag must be [n]");
+    dptr = diag->data_ptr();
+  }
   auto u = torch::zeros_like(h);
   auto scratch = torch::empty({lfmq_chol_scratch(n)}, h.options());
   auto info = torch::empty({1}, h.options().dtype(torch::kInt32));
-  CHECK_HIP(lfmq_chol_inverse(h.data_ptr(), u.data_ptr(), scratch.data_ptr(),
-                              info.data_ptr(), n, stream()));
+  CHECK_HIP(lfmq_chol_inverse(h.data_ptr(), dptr, u.data_ptr(),
+                              scratch.data_ptr(), info.data_ptr(), n, stream()));
   return {u, info};
+}
+
+// w, a copy without columns that have no inputs (zeros on h's diagonal), and [3, k]:
+// h's diagonal with ones there, the same damped, whether a column has inputs
+std::vector<torch::Tensor> gptq_prepare(torch::Tensor w, torch::Tensor h,
+                                        double percent) {
+  check_t(w, torch::kFloat32, "w");
+  check_t(h, torch::kFloat32, "h");
+  TORCH_CHECK(w.dim() == 2 && h.dim() == 2 && w.size(1) > 0 &&
+                  h.size(0) == w.size(1) && h.size(1) == w.size(1) &&
+                  h.device() == w.device(),
+              "w [n, k], h [k, k] on one device");
+  auto to = torch::empty_like(w);
+  auto d = torch::empty({3, w.size(1)}, w.options());
+  CHECK_HIP(lfmq_gptq_prepare(w.data_ptr(), h.data_ptr(), to.data_ptr(),
+                              d.data_ptr(), (int)w.size(0), (int)w.size(1),
+                              (float)percent, stream()));
+  return {to, d};
 }
 
 // one column block of the GPTQ solve; returns its errors [n, nb]
@@ -1090,6 +1121,46 @@ void gptq_push(torch::Tensor w, torch::Tensor err, torch::Tensor u, long i1) {
                            (int)n, (int)k, (int)(i1 + nb), (int)nb, stream()));
 }
 
+// All columns of a solve, `block` at a time: w, which changes, with the factor u
+// to codes, scales and zeros
+void gptq_columns(torch::Tensor w, torch::Tensor u, torch::Tensor codes,
+                  torch::Tensor scales, torch::Tensor zeros, long block, long g,
+                  long bits, bool sym) {
+  check_t(w, torch::kFloat32, "w");
+  check_t(u, torch::kFloat32, "u");
+  check_t(codes, torch::kInt32, "codes");
+  check_t(scales, torch::kFloat32, "scales");
+  check_t(zeros, torch::kInt32, "zeros");
+  TORCH_CHECK(w.dim() == 2 && codes.sizes() == w.sizes(),
+              "w and codes must be [n, k]");
+  const long n = w.size(0), k = w.size(1);
+  TORCH_CHECK(u.dim() == 2 && u.size(0) == k && u.size(1) == k,
+              "u must be [k, k]");
+  TORCH_CHECK(g > 0 && k % g == 0 && scales.numel() == n * (k / g) &&
+                  zeros.numel() == n * (k / g),
+              "scales and zeros must be [n, k / g]");
+  TORCH_CHECK(block > 0, "a block has columns");
+  const bool steps = block == 128 && lfmq_gptq_step_ok(u.data_ptr(), k, (int)n,
+                                                       (int)k, (int)g);
+  torch::Tensor before, other;             // errors of the last two blocks
+  for (long i1 = 0; i1 < k; i1 += block) {
+    const long nb = std::min(block, k - i1);
+    if (i1 > 0 && steps && nb == block) {
+      if (!other.defined()) other = torch::empty_like(before);
+      CHECK_HIP(lfmq_gptq_step(w.data_ptr(), u.data_ptr(), k, codes.data_ptr(),
+                               scales.data_ptr(), zeros.data_ptr(),
+                               before.data_ptr(), other.data_ptr(), (int)n,
+                               (int)k, (int)(k / g), (int)i1, (int)g, (int)bits,
+                               sym, stream()));
+      std::swap(before, other);
+      continue;
+    }
+    if (i1 > 0) gptq_push(w, before, u, i1 - block);
+    before = gptq_block(w, u.narrow(0, i1, nb).narrow(1, i1, nb), codes, scales,
+                        zeros, i1, g, bits, sym);
+  }
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -1107,9 +1178,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prefill", &attn_prefill,
         "flash prefill attention (LFMQ_FLASH_PREFILL)");
   m.def("hessian_accum", &hessian_accum, "H += 2 X^T X");
+  m.def("gptq_prepare", &gptq_prepare, "weights and diagonal of a GPTQ solve");
   m.def("chol_inverse", &chol_inverse,
-        "upper Cholesky factor of the inverse, and whether there is none");
+        "upper Cholesky factor of the inverse, and whether there is none",
+        pybind11::arg("h"), pybind11::arg("diag") = pybind11::none());
   m.def("gptq_push", &gptq_push, "a GPTQ block's errors to later columns");
+  m.def("gptq_columns", &gptq_columns, "all column blocks of the GPTQ solve");
   m.def("gptq_block", &gptq_block, "one column block of the GPTQ solve");
   m.def("dq_gemv_gateup", &dq_gemv_gateup, "fused gate_up GEMV + silu*mul");
   m.def("qkv_rope_append", &qkv_rope_append, "fused rope + KV append");

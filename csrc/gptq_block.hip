@@ -11,17 +11,19 @@
 // in 16-byte pieces side by side, the same address for all four rows.  The
 // columns in turn are always the first lane's, which a lane permutation hands
 // to the others (through LDS, as from any lane, it is 100 cycles of the chain).
-// Bound by the chain broadcast -> quotients -> update, 128 times 0.18 us, so
-// rows of U are read a column ahead, nothing in the loop waits for stores, and
-// few rows go to workgroups of two waves, a wave a SIMD: 2048 rows take 25.1
-// us a block of 128 (35.1 in eight waves with the reads in the chain), 8192
-// rows 27.2 (35.9), 28672 72 (87).  Four rows that meet numbers whose quotients
-// need a division are done again with divisions.
+// Bound by the chain broadcast -> quotients -> update, 128 times 0.13 us, so
+// rows of U are read a column ahead (held there, or the compiler reads them where
+// they are needed), nothing in the loop waits for stores, blocks of whole chunks
+// have no tests of their end, and few rows go to workgroups of two waves, a wave a
+// SIMD: 2048 rows take 20.6 us a block of 128 (25.9 with rows of U read late, a test
+// a column, and a group's fit from one load after the other).  Four rows that meet
+// numbers whose quotients need a division are done again with divisions.
 //
 // Every operation rounds on its own, in the order of the tensor expressions
 // above, so that results are those of a GPU tensor loop, bit by bit: no
 // contraction, and a division by a constant is a product with its
 // reciprocal.
+#include <algorithm>
 #include <type_traits>
 
 #include "lds_dma.h"
@@ -84,18 +86,65 @@ struct BlockArgs {
   int ldu, n, k, G, i1, nb, g;
   float qmax, inv_range;
   bool sym, wide;          // wide: codes and errors in pieces of 16 bytes
+  // gptq_step: errors [n, nb] of the block before and its rows of U, from this
+  // block's first column on
+  const float *before, *ubefore;
 };
 
-// DMA: U comes by 16-byte pieces straight into LDS (nb whole chunks)
-template <int NC, bool DMA>  // chunks of 64 columns
-__global__ __launch_bounds__(512) void gptq_block_kernel(BlockArgs A) {
-  constexpr int BS = NC * 64;
+// w [rows, columns] -= before U, sixteen rows and 128 columns of four waves, as
+// gptq_push takes it off (the same sums in the same order), but into LDS
+template <int LD>
+__device__ __forceinline__ void take_off(const BlockArgs& A, int row0,
+                                         float* to) {
+  const int lane = threadIdx.x & 63, l15 = lane & 15, l4 = lane >> 4;
+  const int c0 = (threadIdx.x >> 6) * 32, nb = A.nb;
+  const int R = min(16, A.n - row0);
+  const auto er = make_rsrc(A.before + (size_t)row0 * nb, (u32)R * nb * 4);
+  const auto wr = make_rsrc(A.w + (size_t)row0 * A.k, (u32)R * A.k * 4);
+  auto load = [](__amdgpu_buffer_rsrc_t r, int at) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_raw_buffer_load_b32(r, at * 4, 0, 0));
+  };
+  constexpr int K = 128 / 4;               // products, 4 of k each
+  float e[K], u[2][K], w[2][4];
+#pragma unroll
+  for (int s = 0; s < K; ++s) {
+    e[s] = load(er, l15 * nb + s * 4 + l4);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      u[t][s] = A.ubefore[(size_t)(s * 4 + l4) * A.ldu + c0 + t * 16 + l15];
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      w[t][i] = load(wr, (l4 * 4 + i) * A.k + A.i1 + c0 + t * 16 + l15);
+  f32x4 acc[2] = {};
+#pragma unroll
+  for (int s = 0; s < K; ++s)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(e[s], u[t][s], acc[t], 0, 0, 0);
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      to[(l4 * 4 + i) * LD + c0 + t * 16 + l15] = w[t][i] - acc[t][i];
+}
+
+// DMA: U comes by 16-byte pieces straight into LDS (nb whole chunks), and groups
+// start on every fourth column at most.  BEFORE: the
+// block's columns of w still want the errors of the block before (take_off)
+template <int NC, bool DMA, bool BEFORE>   // chunks of 64 columns
+__device__ __forceinline__ void block_rows(const BlockArgs& A, int tpb) {
+  constexpr int BS = NC * 64, WL = BS + 4;
   const int n = A.n, k = A.k, G = A.G, i1 = A.i1, nb = A.nb, g = A.g;
-  const int tpb = blockDim.x, tid = threadIdx.x;
+  const int tid = threadIdx.x;
   const float qmax = A.qmax;
-  // U [nb][BS], then {u_jj, 1 / u_jj}
+  // U [nb][BS], then {u_jj, 1 / u_jj}; BEFORE: then w [16][WL]
   extern __shared__ __attribute__((aligned(16))) float us[];
   f32x2* diag = (f32x2*)(us + nb * BS);
+  float* ws = (float*)(diag + nb);
   if constexpr (DMA) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr int RL = 256 / BS;           // rows of U a load
@@ -120,7 +169,13 @@ __global__ __launch_bounds__(512) void gptq_block_kernel(BlockArgs A) {
   const int lane = tid & 63, c16 = lane & 15;
   const int row = blockIdx.x * (tpb / 16) + (tid >> 6) * RPW + (lane >> 4);
   const bool live = row < n;
-  const float* wr = A.w + (u64)(live ? row : n - 1) * k;
+  if constexpr (BEFORE) {
+    take_off<WL>(A, blockIdx.x * 16, ws);
+    __syncthreads();
+  }
+  // the row's columns from i1 on
+  const float* wr = BEFORE ? ws + (tid >> 4) * WL
+                           : A.w + (u64)(live ? row : n - 1) * k + i1;
 
   struct Fit {
     float s, z, rs;
@@ -128,10 +183,16 @@ __global__ __launch_bounds__(512) void gptq_block_kernel(BlockArgs A) {
   // scale and zero of the group from column j of the block on
   auto fit = [&](int j) {
     float lo = INFINITY, hi = -INFINITY;
-    for (int t = c16; t < g; t += 16) {
-      const float x = wr[i1 + j + t];
-      lo = nmin(lo, x);
-      hi = nmax(hi, x);
+    constexpr int IN = 8;                  // on their way at once
+    for (int t0 = c16; t0 < g; t0 += 16 * IN) {
+      float x[IN];
+#pragma unroll
+      for (int e = 0; e < IN; ++e) x[e] = wr[j + (t0 + 16 * e < g ? t0 + 16 * e : t0)];
+#pragma unroll
+      for (int e = 0; e < IN; ++e) {
+        lo = nmin(lo, x[e]);
+        hi = nmax(hi, x[e]);
+      }
     }
 #pragma unroll
     for (int o = 8; o > 0; o >>= 1) {
@@ -181,7 +242,7 @@ __global__ __launch_bounds__(512) void gptq_block_kernel(BlockArgs A) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int c = i * 64 + c16 * 4 + r;
-        v[i * 4 + r] = c < nb ? wr[i1 + c] : 0.f;
+        v[i * 4 + r] = c < nb ? wr[c] : 0.f;
         // here, or every round waits for the stores of the one before
         asm volatile("" : "+v"(v[i * 4 + r]));
       }
@@ -210,13 +271,13 @@ __global__ __launch_bounds__(512) void gptq_block_kernel(BlockArgs A) {
     for (int i = 0; i < NC; ++i)
       for (int c = 0; c < 16; ++c) {
         const int j0 = i * 64 + c * 4;
-        if (j0 >= nb) break;
+        if (!DMA && j0 >= nb) break;
         float q4[4] = {}, e4[4] = {};
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int j = j0 + r;
-          if (j >= nb) break;
-          if (j == start) {
+          if (!DMA && j >= nb) break;
+          if ((!DMA || r == 0) && j == start) {
             f = starts == 0 ? ahead[0] : (starts == 1 ? ahead[1] : fit(j));
             ++starts;
             start += g;
@@ -226,6 +287,7 @@ __global__ __launch_bounds__(512) void gptq_block_kernel(BlockArgs A) {
             }
           }
           read(next, j + 1, i);
+          __builtin_amdgcn_sched_barrier(0);   // here, not where it is needed
           const float x = first_lane(v[i * 4 + r]);
           const float t = EXACT ? x / f.s : quotient(x, f.s, f.rs);
           // (the median of a NaN is not NaN: seen by `finite`)
@@ -270,6 +332,11 @@ __global__ __launch_bounds__(512) void gptq_block_kernel(BlockArgs A) {
   if (__any(!columns(std::false_type{}))) columns(std::true_type{});
 }
 
+template <int NC, bool DMA>
+__global__ __launch_bounds__(512) void gptq_block_kernel(BlockArgs A) {
+  block_rows<NC, DMA, false>(A, blockDim.x);
+}
+
 // w[:, i2:] -= err U[i1:i2, i2:]: the later columns learn of a block's errors.
 // A workgroup 64 x 64, K in 64s through LDS, fp32 matrix instructions, the
 // product summed apart and rounded once at the size of w.  Bound by the load
@@ -280,14 +347,24 @@ __global__ __launch_bounds__(512) void gptq_block_kernel(BlockArgs A) {
 // less (4.6, here 6.9).  K whole in LDS, two workgroups a CU: 15.1 for 11.4.
 constexpr int PT = 64, PK = 64, LA = PK + 4, LB = PT + 16;
 
-__global__ __launch_bounds__(256, 3) void gptq_push_kernel(
-    float* __restrict__ w, const float* __restrict__ err,
-    const float* __restrict__ u, long ldu, int n, int k, int i2, int nb) {
-  // [row][k], banks row * 4 + k; [k][column], banks k * 16 + column
-  __shared__ float a[PT * LA], b[PK * LB];
+struct PushArgs {
+  float* w;
+  const float *err, *u;
+  long ldu;
+  int n, k, i2, nb;
+};
+
+// a, b: PT * LA and PK * LB floats of LDS, [row][k], banks row * 4 + k, and
+// [k][column], banks k * 16 + column
+__device__ __forceinline__ void push_tile(const PushArgs& A, float* a, float* b,
+                                          int bx, int by) {
+  float* w = A.w;
+  const float *err = A.err, *u = A.u;
+  const long ldu = A.ldu;
+  const int n = A.n, k = A.k, i2 = A.i2, nb = A.nb;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l15 = lane & 15, l4 = lane >> 4;
-  const int r0 = blockIdx.x * PT, c0 = i2 + blockIdx.y * PT;
+  const int r0 = bx * PT, c0 = i2 + by * PT;
   const int ro = wave / 2 * 32, co = wave % 2 * 32;
   constexpr int PL = PT * PK / 256;
   // loads with bounds: rows past the last one are zeros (columns past it, the
@@ -366,6 +443,78 @@ __global__ __launch_bounds__(256, 3) void gptq_push_kernel(
       }
 }
 
+__global__ __launch_bounds__(256, 3) void gptq_push_kernel(PushArgs A) {
+  __shared__ float a[PT * LA], b[PK * LB];
+  push_tile(A, a, b, blockIdx.x, blockIdx.y);
+}
+
+// A block's columns and what is left of the block before's push, in one launch:
+// its first `rows16` workgroups take the errors off their own columns and go
+// through them, a wave a SIMD, while the others carry the errors to the columns
+// behind this block.  The chain of columns hides the products: a step of 2048
+// x 2048 23 us at the end and 29 with all of the push, one after the other 20.6 + 6
+// to 17.
+__global__ __launch_bounds__(256, 2) void gptq_step_kernel(BlockArgs A,
+                                                           PushArgs P,
+                                                           int rows16) {
+  extern __shared__ __attribute__((aligned(16))) float us[];
+  if ((int)blockIdx.x < rows16) {
+    __builtin_amdgcn_s_setprio(3);         // before products on the same SIMD
+    block_rows<2, true, true>(A, 256);
+    return;
+  }
+  const int id = blockIdx.x - rows16, tiles = (P.n + PT - 1) / PT;
+  push_tile(P, us, us + PT * LA, id % tiles, id / tiles);
+}
+
+// The diagonal of h [k, k] as the solve wants it: d[0] with ones for zeros (columns
+// without inputs), d[1] damped by `percent` of its mean, d[2] whether a column has
+// inputs.  One workgroup.
+__global__ __launch_bounds__(1024) void gptq_diag_kernel(
+    const float* __restrict__ h, float* __restrict__ d, int k, float percent) {
+  const int tid = threadIdx.x;
+  __shared__ float part[16];
+  float sum = 0.f;
+#pragma unroll 4
+  for (int i = tid; i < k; i += 1024) {
+    const float x = h[(size_t)i * k + i];
+    const float y = x == 0.f ? 1.f : x;
+    d[i] = y;
+    d[2 * (size_t)k + i] = x == 0.f ? 0.f : 1.f;
+    sum += y;
+  }
+  sum = wave_reduce_sum(sum);
+  if ((tid & 63) == 0) part[tid >> 6] = sum;
+  __syncthreads();
+  float all = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) all += part[i];
+  const float damp = percent * (all / (float)k);
+  for (int i = tid; i < k; i += 1024) d[(size_t)k + i] = d[i] + damp;
+}
+
+// to = w, zeros in columns without inputs; a row of workgroups a row
+__global__ __launch_bounds__(256) void gptq_copy_kernel(
+    const float* __restrict__ w, const float* __restrict__ on,
+    float* __restrict__ to, int n, int k) {
+  const int c = (blockIdx.x * 256 + threadIdx.x) * 4;
+  if (c >= k) return;
+  for (int r = blockIdx.y; r < n; r += gridDim.y) {
+    const float* p = w + (size_t)r * k + c;
+    float* q = to + (size_t)r * k + c;
+    if (k % 4 == 0 && ((u64)w | (u64)to | (u64)on) % 16 == 0) {
+      const f32x4 x = *(const f32x4*)p, o = *(const f32x4*)(on + c);
+      f32x4 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = o[e] == 0.f ? 0.f : x[e];
+      *(f32x4*)q = y;
+    } else {
+      for (int e = 0; e < 4 && c + e < k; ++e)
+        q[e] = on[c + e] == 0.f ? 0.f : p[e];
+    }
+  }
+}
+
 }  // namespace
 
 // w [n, k] fp32 (read only), ub [nb, nb] the block of U on the diagonal, its
@@ -386,14 +535,14 @@ hipError_t lfmq_gptq_block(const void* w, const void* ub, int ldu, void* codes,
                     ((u64)codes | (u64)err) % 16 == 0;
   const BlockArgs A{(const float*)w, (const float*)ub, (i32*)codes,
                     (float*)scales, (i32*)zeros, (float*)err, ldu, n, k, G, i1,
-                    nb, g, qmax, inv, sym, wide};
+                    nb, g, qmax, inv, sym, wide, nullptr, nullptr};
   // a wave a SIMD while they last (2048 rows 31 us in eight waves, 26 in two),
   // then U read less often
   const int tpb = n <= 4096 ? 128 : (n <= 8192 ? 256 : 512);
   const dim3 grid((n + tpb / 16 - 1) / (tpb / 16));
   const int bs = nb <= 64 ? 64 : 128;
   const size_t lds = ((size_t)nb * bs + 2 * nb) * sizeof(float);
-  const bool dma = nb == bs && ldu % 4 == 0 && (u64)ub % 16 == 0 &&
+  const bool dma = nb == bs && g % 4 == 0 && i1 % 4 == 0 && ldu % 4 == 0 && (u64)ub % 16 == 0 &&
                    (u64)nb * ldu * 4 < 1ull << 32;
 #define GO(NC, DMA)                                                          \
   do {                                                                       \
@@ -428,7 +577,71 @@ hipError_t lfmq_gptq_push(const void* w, const void* err, const void* u, long ld
   if (n == 0 || i2 == k) return hipSuccess;
   hipLaunchKernelGGL(gptq_push_kernel,
                      dim3((n + PT - 1) / PT, (k - i2 + PT - 1) / PT), dim3(256),
-                     0, stream, (float*)w, (const float*)err,
-                     (const float*)u, ldu, n, k, i2, nb);
+                     0, stream,
+                     PushArgs{(float*)w, (const float*)err, (const float*)u,
+                              ldu, n, k, i2, nb});
+  return hipGetLastError();
+}
+
+// Whether whole blocks of 128 columns go by lfmq_gptq_step: groups that start in a
+// block end in it, since the columns behind it change meanwhile; U for 16-byte
+// pieces; rows of a workgroup a CU at most (8192 rows: 27 us a block in 256
+// workgroups of two waves a SIMD, which leave the products no room).
+bool lfmq_gptq_step_ok(const void* u, long ldu, int n, int k, int g) {
+  return n >= 1 && n <= 4096 && g >= 4 && 128 % g == 0 && ldu % 4 == 0 &&
+         (u64)u % 16 == 0 && 128ull * ldu * 4 < 1ull << 32 &&
+         (u64)16 * k * 4 < 1ull << 31 && k / PT <= 65535;
+}
+
+// The columns i1 .. i1 + 127 (i1 >= 128), whose w wants the errors `before` [n,
+// 128] of the 128 columns in front, and these errors' push to the columns behind.
+// u: the whole factor; err another buffer than before.  Otherwise as
+// lfmq_gptq_block.
+hipError_t lfmq_gptq_step(const void* w, const void* u, long ldu, void* codes,
+                          void* scales, void* zeros, const void* before,
+                          void* err, int n, int k, int G, int i1, int g,
+                          int bits, bool sym, hipStream_t stream) {
+  if (!lfmq_gptq_step_ok(u, ldu, n, k, g) || i1 < 128 || i1 + 128 > k ||
+      i1 % g != 0 || G * (long)g != k)
+    return hipErrorInvalidValue;
+  const float qmax = (float)((1 << bits) - 1);
+  const float inv = sym ? 1.f / ((qmax - 1.f) / 2.f) : 1.f / qmax;
+  const bool wide = k % 4 == 0 && ((u64)codes | (u64)err) % 16 == 0;
+  const float* ut = (const float*)u;
+  const float* prow = ut + (size_t)(i1 - 128) * ldu;
+  const BlockArgs A{(const float*)w, ut + (size_t)i1 * ldu + i1, (i32*)codes,
+                    (float*)scales, (i32*)zeros, (float*)err, (int)ldu, n, k, G,
+                    i1, 128, g, qmax, inv, sym, wide, (const float*)before,
+                    prow + i1};
+  const PushArgs P{(float*)w, (const float*)before, prow, ldu, n, k, i1 + 128, 128};
+  const int rows16 = (n + 15) / 16;
+  const int tiles = (n + PT - 1) / PT * ((k - i1 - 128 + PT - 1) / PT);
+  const size_t lds = (128 * 128 + 2 * 128 + 16 * 132) * sizeof(float);
+  static_assert(PT * LA + PK * LB <= 128 * 128, "a push fits");
+  static bool set = false;
+  if (!set) {
+    LFMQ_CHECK_HIP(hipFuncSetAttribute(
+        (const void*)gptq_step_kernel,
+        hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024));
+    set = true;
+  }
+  hipLaunchKernelGGL(gptq_step_kernel, dim3(rows16 + tiles), dim3(256), lds,
+                     stream, A, P, rows16);
+  return hipGetLastError();
+}
+
+// d [3, k] of h [k, k] (gptq_diag_kernel); to = w [n, k] without the columns that
+// have no inputs.  Two launches, where tensor operations take twelve and a wait
+// for the device.
+hipError_t lfmq_gptq_prepare(const void* w, const void* h, void* to, void* d,
+                             int n, int k, float percent, hipStream_t stream) {
+  if (n < 0 || k < 1) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(gptq_diag_kernel, dim3(1), dim3(1024), 0, stream,
+                     (const float*)h, (float*)d, k, percent);
+  if (n > 0)
+    hipLaunchKernelGGL(gptq_copy_kernel,
+                       dim3((k + 1023) / 1024, std::min(n, 65535)), dim3(256), 0,
+                       stream, (const float*)w, (const float*)d + 2 * (size_t)k,
+                       (float*)to, n, k);
   return hipGetLastError();
 }

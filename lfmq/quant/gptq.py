@@ -68,6 +68,12 @@ def _block(w, ub, codes, scales, zeros, i1, cfg, g) -> torch.Tensor:
     return err
 
 
+def _library_factor(h: torch.Tensor) -> torch.Tensor:
+    L = torch.linalg.cholesky(h)
+    hinv = torch.cholesky_inverse(L)
+    return torch.linalg.cholesky(hinv, upper=True)
+
+
 def _inverse_factor(h: torch.Tensor) -> torch.Tensor:
     """U upper triangular with UᵀU = h⁻¹."""
     if h.is_cuda:
@@ -77,9 +83,7 @@ def _inverse_factor(h: torch.Tensor) -> torch.Tensor:
         if not failed.item():
             return U
         # a pivot is not positive in this order of elimination
-    L = torch.linalg.cholesky(h)
-    hinv = torch.cholesky_inverse(L)
-    return torch.linalg.cholesky(hinv, upper=True)
+    return _library_factor(h)
 
 
 GPU_BLOCK = 128        # widest block of the HIP kernel: its U fits in LDS
@@ -95,12 +99,44 @@ def _gpu_block(w, ub, codes, scales, zeros, i1, cfg, g) -> torch.Tensor:
                                     cfg.bits, cfg.sym)
 
 
-def _gpu_push(w, err, U, i1) -> None:
-    """The columns behind the block from i1 on take over its errors
-    (csrc/gptq_block.hip)."""
+def _gpu_layer(w, h, cfg, g):
+    """gptq_quantize_layer in the HIP kernels, which leave w and h as they
+    are; the host waits for one number while the columns run."""
     from ..ops import hip_ext
-    with torch.cuda.device(w.device):
-        hip_ext().gptq_push(w, err, U, i1)
+    ext = hip_ext()
+    (n, k), dev = w.shape, w.device
+    w, h = w.float().contiguous(), h.float().contiguous()
+
+    def columns(wq, U):
+        out = (torch.empty(n, k, dtype=torch.int32, device=dev),
+               torch.empty(n, k // g, dtype=torch.float32, device=dev),
+               torch.empty(n, k // g, dtype=torch.int32, device=dev))
+        # (the library's factor is not contiguous)
+        ext.gptq_columns(wq, U.contiguous(), *out, cfg.block_size, g,
+                         cfg.bits, cfg.sym)
+        return out
+
+    wq, diag = ext.gptq_prepare(w, h, cfg.damp_percent)
+    perm, damped = None, diag[1]
+    if cfg.act_order:
+        perm = torch.argsort(diag[0], descending=True)
+        w = wq[:, perm].contiguous()
+        wq, h, damped = w.clone(), h[perm][:, perm], damped[perm]
+    U, failed = ext.chol_inverse(h, damped)
+    # read once the factor is there, while its columns run
+    failed = failed.to("cpu", non_blocking=True)
+    known = torch.cuda.Event()
+    known.record()
+    out = columns(wq, U)
+    known.synchronize()
+    if failed.item():
+        # a pivot is not positive in this order of elimination
+        if perm is None:
+            w = ext.gptq_prepare(w, h, cfg.damp_percent)[0]
+        h = h.clone()
+        h.diagonal().copy_(damped)
+        out = columns(w, _library_factor(h))
+    return *out, perm
 
 
 @torch.no_grad()
@@ -118,6 +154,9 @@ def gptq_quantize_layer(
     n, k = w.shape
     g = k if cfg.group_size == -1 else cfg.group_size
     G = k // g
+    if w.is_cuda and 0 < cfg.block_size <= GPU_BLOCK and k > 0:
+        with torch.cuda.device(w.device):
+            return _gpu_layer(w, h, cfg, g)
     w = w.float().clone(memory_format=torch.contiguous_format)
     h = h.float().clone()
     dev = w.device
@@ -142,16 +181,10 @@ def gptq_quantize_layer(
     scales = torch.zeros(n, G, dtype=torch.float32, device=dev)
     zeros = torch.zeros(n, G, dtype=torch.int32, device=dev)
 
-    on_gpu = w.is_cuda and cfg.block_size <= GPU_BLOCK
-    block = _gpu_block if on_gpu else _block
-    if on_gpu and U.stride(1) != 1:        # the library's factor
-        U = U.contiguous()
     for i1 in range(0, k, cfg.block_size):
         i2 = min(i1 + cfg.block_size, k)
-        err = block(w, U[i1:i2, i1:i2], codes, scales, zeros, i1, cfg, g)
-        if i2 < k and on_gpu:
-            _gpu_push(w, err, U, i1)
-        elif i2 < k:
+        err = _block(w, U[i1:i2, i1:i2], codes, scales, zeros, i1, cfg, g)
+        if i2 < k:
             # in one pass over w, of the products' sums in fp32
             w[:, i2:].addmm_(err, U[i1:i2, i2:], alpha=-1)
 

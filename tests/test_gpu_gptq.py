@@ -121,3 +121,85 @@ def test_inverse_factor_of_one_block(n):
         assert ext().chol_inverse(bad)[1].item() == 1
     h[n // 2, n // 2] = 2.0 ** 126         # no reciprocal in the normal range
     assert ext().chol_inverse(h)[1].item() == 1
+
+
+# rows that end inside a workgroup's sixteen and inside a product's 64; a last
+# block of 64; one, two and many groups a block; too many rows, and groups that do
+# not end with a block, which go block by block
+@pytest.mark.parametrize("n,k,g,bits,sym", [
+    (1, 256, 128, 4, False), (2048, 512, 128, 4, False), (17, 384, 64, 8, True),
+    (4096, 320, 64, 4, False), (1000, 640, 16, 4, True), (4097, 384, 128, 4, False),
+    (70, 768, 384, 4, False), (33, 520, 104, 8, False)])
+def test_all_columns_are_block_by_block(n, k, g, bits, sym):
+    """A launch that takes a block's errors off the next one's columns while it
+    carries them on: bit by bit what a launch each leaves."""
+    gen = torch.Generator(DEV).manual_seed(n)
+    w = torch.randn(n, k, generator=gen, device=DEV)
+    w[0] *= 1e-39                          # quotients that need divisions
+    w[n // 2, 3] = float("inf")
+    u = torch.randn(k, k, generator=gen, device=DEV).triu_() * 0.05
+    u.diagonal().copy_(torch.rand(k, generator=gen, device=DEV) + 0.5)
+
+    def out():
+        return (torch.zeros(n, k, dtype=torch.int32, device=DEV),
+                torch.zeros(n, k // g, device=DEV),
+                torch.zeros(n, k // g, dtype=torch.int32, device=DEV))
+
+    got, want = out(), out()
+    ext().gptq_columns(w.clone(), u, *got, 128, g, bits, sym)
+    cfg = QuantConfig(scheme="gptq", bits=bits, group_size=g, sym=sym)
+    for i1 in range(0, k, 128):
+        i2 = min(i1 + 128, k)
+        err = _gpu_block(w, u[i1:i2, i1:i2], *want, i1, cfg, g)
+        if i2 < k:
+            ext().gptq_push(w, err, u, i1)
+    finite = torch.isfinite(want[1]).all(1)
+    assert int(finite.sum()) >= n - 1
+    for a, b in zip(got, want):
+        assert torch.equal(a[finite], b[finite])
+
+
+@pytest.mark.parametrize("n,k", [(1, 1), (3, 7), (70, 1030), (5, 2048)])
+def test_weights_and_diagonal_of_a_solve(n, k):
+    """Columns without inputs: ones on the diagonal, zeros (whatever w holds) in
+    the weights; the damping is a mean of k sums in fp32."""
+    gen = torch.Generator(DEV).manual_seed(k)
+    w = torch.randn(n, k, generator=gen, device=DEV)
+    h = torch.rand(k, k, generator=gen, device=DEV) + 0.5
+    dead = torch.rand(k, generator=gen, device=DEV) < 0.3
+    h.diagonal()[dead] = 0
+    w[:, dead] = float("nan")
+    kept = w.clone(), h.clone()
+    to, d = ext().gptq_prepare(w, h, 0.01)
+    assert torch.equal(w.nan_to_num(7.0), kept[0].nan_to_num(7.0))
+    assert torch.equal(h, kept[1])
+    diag = torch.where(dead, torch.ones_like(h.diagonal()), h.diagonal())
+    assert torch.equal(to, torch.where(dead, torch.zeros_like(w), w))
+    assert torch.equal(d[0], diag) and torch.equal(d[2] == 0, dead)
+    want = diag.double() + 0.01 * diag.double().mean()
+    # a sum of k in trees of 64 and 16 and runs of k / 1024, and three roundings
+    bound = (26 + k / 1024) * 2 ** -24
+    assert float(((d[1].double() - want) / want).abs().max()) <= bound
+
+
+@pytest.mark.parametrize("act_order", [False, True])
+def test_solve_by_the_library_factor(act_order):
+    """Pivots that the factor does not take (from 2^125): the library's factor,
+    of weights that the columns have not changed.  Without elements beside the
+    diagonal nothing is carried on, whatever its size."""
+    from lfmq.quant.gptq import gptq_quantize_layer
+    torch.manual_seed(3)
+    w = torch.randn(40, 256, device=DEV)
+    cfg = QuantConfig(scheme="gptq", bits=4, group_size=64, act_order=act_order)
+    h = torch.diag(torch.rand(256, device=DEV) + 1)
+    h[5, 5] = 0
+    h[9, 9] = 3
+    want = gptq_quantize_layer(w, h, cfg)
+    h[9, 9] = 1.5 * 2.0 ** 125
+    assert ext().chol_inverse(h + torch.eye(256, device=DEV))[1].item()
+    got = gptq_quantize_layer(w, h, cfg)
+    for a, b in zip(got[:3], want[:3]):
+        assert torch.equal(a, b)
+    assert act_order == (got[3] is not None)
+    if act_order:
+        assert got[3].dtype == torch.int64 and torch.equal(got[3], want[3])
