@@ -102,6 +102,16 @@ __device__ __forceinline__ f32x4 sum_of_parts(const float* p, u64 stride,
                                   : sum_in<8>(p, stride, parts));
 }
 
+// What follows a whole row of the result, r = sum + bias (+ residual) in bf16.
+// normed: y = r + to in bf16, normed = (r + to) w over its root mean square;
+// else scale: y = r, scale = 1 / its root mean square (mean square + eps).
+struct DqRowEnd {
+  float* scale;                  // [m]
+  unsigned short* normed;        // [m, n]
+  const unsigned short *to, *w;  // [m, n], [n]
+  float eps;
+};
+
 // what the packed-product kernels (dq_rows, dq_tile) take
 struct DqArgs {
   const char* w;                 // [n, k * BITS / 8] bytes
@@ -118,6 +128,8 @@ struct DqArgs {
   const i32* src;                // row of x for a slot, or null: the slot
   float* y32;                    // [slots, n]
   float rms_eps = -1.f;          // >= 0: rows of x over their root mean square
+  const float* row_scale = nullptr;  // [m] x's rows times this
+  DqRowEnd end{};
 };
 
 // DENSE: y = x W^T (+ bias) (+ residual).  Of an expert's rows, GLU: W is
@@ -127,3 +139,15 @@ enum DqMode { DENSE, GLU, SLOTS };
 __device__ __forceinline__ float silu_mul_f(float g, float u) {
   return g / (1.f + __expf(-g)) * u;
 }
+
+// The rows of the result that a workgroup of the sum of parts can hold whole.
+bool lfmq_dq_row_end_ok(int n);
+
+// y = sum of part [splits, m, n] (row_scale: times that of its row) (+ bias)
+// (+ residual), or the gate of it; end: without a gate, n that row_end_ok takes,
+// vectors on 8 bytes
+hipError_t lfmq_dq_rows_sum(const void* part, void* y, const void* bias,
+                            const void* resid, int m, int n, int splits,
+                            bool glu, hipStream_t stream,
+                            const float* row_scale = nullptr,
+                            const DqRowEnd* end = nullptr);

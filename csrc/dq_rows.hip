@@ -229,13 +229,18 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(DqArgs A) {
       return v;
     };
     f32x4 v = sum(c4);
-    const float scale = rms ? rs[row] : 1.f;
+    // of parts: after their sum
+    const float scale =
+        rms ? rs[row]
+            : (MODE != SLOTS && A.row_scale != nullptr && gridDim.y == 1
+                   ? A.row_scale[gr]
+                   : 1.f);
     if constexpr (MODE == GLU) {
       const f32x4 up = sum(HT * 16 + c4);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         v[e] = silu_mul_f(v[e] * scale, up[e] * scale);
-    } else if (rms) {
+    } else if (MODE == DENSE) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] *= scale;
     }
@@ -281,9 +286,10 @@ __global__ __launch_bounds__(256) void dq_rows_sum(DqArgs A) {
       if constexpr (!GLU)
 #pragma unroll
         for (int e = 0; e < 4; ++e) add[e] = epilogue(A, 0.f, row, col + e);
-      f32x4 v = sum_of_parts(p, part, A.splits);
+      const float scale = A.row_scale != nullptr ? A.row_scale[row] : 1.f;
+      f32x4 v = sum_of_parts(p, part, A.splits) * scale;
       if constexpr (GLU) {
-        const f32x4 up = sum_of_parts(p + nout, part, A.splits);
+        const f32x4 up = sum_of_parts(p + nout, part, A.splits) * scale;
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = silu_mul_f(v[e], up[e]);
       } else if (A.bias != nullptr || A.resid != nullptr) {
@@ -303,12 +309,122 @@ __global__ __launch_bounds__(256) void dq_rows_sum(DqArgs A) {
       v += A.part[s * part + (u64)row * A.n + col];
       if (GLU) up += A.part[s * part + (u64)row * A.n + nout + col];
     }
+    const float scale = A.row_scale != nullptr ? A.row_scale[row] : 1.f;
+    v *= scale;
     A.y[id] = (unsigned short)f32_to_bf16_bits_rne(
-        GLU ? silu_mul_f(v, up) : epilogue(A, v, row, col));
+        GLU ? silu_mul_f(v, up * scale) : epilogue(A, v, row, col));
   }
 }
 
+// A whole row of the result a workgroup, and what DqRowEnd says of it: the sum of
+// parts, the residual and the norm in one launch.  V pieces of four columns a
+// thread, B parts of them on their way at once.  Bound as dq_rows_sum by launch
+// and latency: 48 rows of 4096, six parts, 4.7 us (dq_rows_sum 4.8, and the norm
+// of its rows 5.0, or in the next product the squares of every workgroup's rows,
+// n 6144, k 4096 22 us where the product without is 10.5).
+constexpr int ROW_TPB = 512;
+
+template <int V, int B, bool NORM>
+__global__ __launch_bounds__(ROW_TPB) void dq_rows_sum_row(DqArgs A) {
+  typedef u32 u32x2 __attribute__((ext_vector_type(2)));
+  const u64 part = (u64)A.m * A.n;
+  const int n4 = A.n / 4, tid = threadIdx.x;
+  const u64 at = (u64)blockIdx.x * A.n;
+  auto four = [](const u32x2 t) {
+    float a, b, c, d;
+    bf16x2_to_f32(t[0], a, b);
+    bf16x2_to_f32(t[1], c, d);
+    return f32x4{a, b, c, d};
+  };
+  const float scale = A.row_scale != nullptr ? A.row_scale[blockIdx.x] : 1.f;
+  const unsigned short* resid = NORM ? A.end.to : A.resid;
+  u32x2 add[V] = {}, wv[V];
+  f32x4 v[V] = {}, bias[V] = {};
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    // past the end the last piece again, not counted and not stored
+    const int c = min(tid + i * ROW_TPB, n4 - 1);
+    if (resid != nullptr) add[i] = ((const u32x2*)(resid + at))[c];
+    if (NORM) wv[i] = ((const u32x2*)A.end.w)[c];
+    if (A.bias != nullptr) bias[i] = four(((const u32x2*)A.bias)[c]);
+  }
+  for (int s0 = 0; s0 < A.splits; s0 += B) {
+    f32x4 t[B][V];
+#pragma unroll
+    for (int s = 0; s < B; ++s)
+#pragma unroll
+      for (int i = 0; i < V; ++i)
+        t[s][i] = ((const f32x4*)(A.part + at + min(s0 + s, A.splits - 1) * part))
+            [min(tid + i * ROW_TPB, n4 - 1)];
+#pragma unroll
+    for (int s = 0; s < B; ++s)
+#pragma unroll
+      for (int i = 0; i < V; ++i)
+        if (s0 + s < A.splits) v[i] += t[s][i];
+  }
+  __shared__ float red[ROW_TPB / LFMQ_WAVE];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    const int c = tid + i * ROW_TPB;
+    f32x4 r = v[i] * scale + bias[i];
+    if (!NORM) r += four(add[i]);
+    const u32x2 out = {pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3])};
+    v[i] = four(out);                      // the result as it is stored
+    if (NORM) v[i] += four(add[i]);
+    if (c < n4) {
+      if (!NORM) ((u32x2*)(A.y + at))[c] = out;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ss = fmaf(v[i][e], v[i][e], ss);
+    }
+  }
+  ss = wave_reduce_sum_dpp(ss);
+  if (tid % LFMQ_WAVE == 0) red[tid / LFMQ_WAVE] = ss;
+  __syncthreads();
+  ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < ROW_TPB / LFMQ_WAVE; ++i) ss += red[i];
+  const float inv = rsqrtf(ss / (float)A.n + A.end.eps);
+  if constexpr (NORM) {
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const int c = tid + i * ROW_TPB;
+      if (c >= n4) break;
+      const f32x4 w = four(wv[i]);
+      ((u32x2*)(A.y + at))[c] =
+          u32x2{pack_bf16x2(v[i][0], v[i][1]), pack_bf16x2(v[i][2], v[i][3])};
+      ((u32x2*)(A.end.normed + at))[c] =
+          u32x2{pack_bf16x2(v[i][0] * inv * w[0], v[i][1] * inv * w[1]),
+                pack_bf16x2(v[i][2] * inv * w[2], v[i][3] * inv * w[3])};
+    }
+  } else if (tid == 0) {
+    A.end.scale[blockIdx.x] = inv;
+  }
+}
+
+template <bool NORM>
+void sum_row(const DqArgs& A, hipStream_t stream) {
+#define GO(V, B)                                                          \
+  hipLaunchKernelGGL((dq_rows_sum_row<V, B, NORM>), dim3(A.m), dim3(ROW_TPB), \
+                     0, stream, A)
+  const int v = (int)ceil_div_u32(A.n, 4 * ROW_TPB);
+  if (v <= 1) {
+    if (A.splits <= 4) GO(1, 4);
+    else GO(1, 8);
+  } else if (v == 2) {
+    if (A.splits <= 4) GO(2, 4);
+    else GO(2, 8);
+  } else if (v <= 4) {
+    GO(4, 4);
+  } else {
+    GO(8, 2);
+  }
+#undef GO
+}
+
 void sum_parts(const DqArgs& A, bool glu, hipStream_t stream) {
+  if (A.end.normed != nullptr) return sum_row<true>(A, stream);
+  if (A.end.scale != nullptr) return sum_row<false>(A, stream);
   const int nout = glu ? A.n / 2 : A.n;
   const dim3 grid =
       nout % 4 == 0
@@ -446,12 +562,14 @@ int lfmq_dq_rows_splits(int m, int n, int k, int g) {
 
 // part: splits > 1 only, [splits, m, n] fp32.  rms_eps >= 0: rows of x are
 // scaled by 1 / sqrt(mean x^2 + eps) first; glu: y [m, n / 2] = silu(gate)
-// up of W = [gate | up].  Both with splits 1.
+// up of W = [gate | up].  Both with splits 1.  row_scale: rows of x times it.
+// end: with splits only, what lfmq_dq_rows_sum takes.
 hipError_t lfmq_dq_rows(const void* qweight, const void* scales,
                         const void* qzeros, const void* x, void* y,
                         const void* bias, const void* resid, void* part,
                         int m, int n, int k, int g, int bits, int splits,
-                        float rms_eps, bool glu, hipStream_t stream) {
+                        float rms_eps, bool glu, hipStream_t stream,
+                        const float* row_scale, const DqRowEnd* end) {
   const bool fused = glu || rms_eps >= 0.f;
   if (!lfmq_dq_rows_ok(m, n, k, g, fused) || (fused && splits != 1) ||
       (glu && n % 2))
@@ -461,7 +579,8 @@ hipError_t lfmq_dq_rows(const void* qweight, const void* scales,
                  (const u32*)qzeros, (const unsigned short*)x,
                  (unsigned short*)y, (const unsigned short*)bias,
                  (const unsigned short*)resid, (float*)part, m, n, k, g,
-                 splits, nullptr, nullptr, nullptr, rms_eps};
+                 splits, nullptr, nullptr, nullptr, rms_eps, row_scale,
+                 end != nullptr ? *end : DqRowEnd{}};
   const int kc = chunk_of(g);
   if (bits == 4) {
     if (kc == 128) return go_tile<4, 128>(A, glu, stream);
@@ -473,10 +592,12 @@ hipError_t lfmq_dq_rows(const void* qweight, const void* scales,
   return go_tile<8, 32>(A, glu, stream);
 }
 
-// y = sum of part [splits, m, n] (+ bias) (+ residual), or the gate of it
+bool lfmq_dq_row_end_ok(int n) { return n % 8 == 0 && n <= 32 * ROW_TPB; }
+
 hipError_t lfmq_dq_rows_sum(const void* part, void* y, const void* bias,
                             const void* resid, int m, int n, int splits,
-                            bool glu, hipStream_t stream) {
+                            bool glu, hipStream_t stream,
+                            const float* row_scale, const DqRowEnd* end) {
   DqArgs A{};
   A.part = (float*)part;
   A.y = (unsigned short*)y;
@@ -485,6 +606,8 @@ hipError_t lfmq_dq_rows_sum(const void* part, void* y, const void* bias,
   A.m = m;
   A.n = n;
   A.splits = splits;
+  A.row_scale = row_scale;
+  if (end != nullptr) A.end = *end;
   sum_parts(A, glu, stream);
   return hipGetLastError();
 }

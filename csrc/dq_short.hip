@@ -287,9 +287,13 @@ __global__ __launch_bounds__(TPB, 2) void dq_short_kernel(DqArgs A, int mb,
     for (int t = 0; t < MT; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        float v = MODE == GLU ? silu_mul_f(acc[t][0][r], acc[t][1][r])
-                              : acc[t][nt][r] + bias;
         const int row = t * 16 + l4 * 4 + r;
+        const float scale = A.row_scale != nullptr && row < rows
+                                ? A.row_scale[row0 + row]
+                                : 1.f;
+        float v = MODE == GLU
+                      ? silu_mul_f(acc[t][0][r] * scale, acc[t][1][r] * scale)
+                      : acc[t][nt][r] * scale + bias;
         if (MODE == DENSE && A.resid != nullptr && row < rows && n0 + c < A.n)
           v += bf16_bits_to_f32(A.resid[(u64)(row0 + row) * A.n + n0 + c]);
         out[(t * 16 + l4 * 4 + r) * LD + c] =

@@ -414,17 +414,13 @@ int lfmq_dq_tile_splits(int m, int n, int k, int g) {
   return 512 / wgs <= C / 6 ? max(s, 512 / wgs) : s;
 }
 
-hipError_t lfmq_dq_rows_sum(const void* part, void* y, const void* bias,
-                            const void* resid, int m, int n, int splits,
-                            bool glu, hipStream_t stream);
-
 // glu: y [m, n / 2] = silu(gate) up of W = [gate | up], without bias and
-// residual
+// residual.  end: with splits only, what lfmq_dq_rows_sum takes.
 hipError_t lfmq_dq_tile(const void* qweight, const void* scales,
                         const void* qzeros, const void* x, void* y,
                         const void* bias, const void* resid, void* part,
                         int m, int n, int k, int g, int bits, int splits,
-                        bool glu, hipStream_t stream) {
+                        bool glu, hipStream_t stream, const DqRowEnd* end) {
   if (resid != nullptr && splits == 1) return hipErrorInvalidValue;
   if (glu && (n % 2 || bias != nullptr || resid != nullptr ||
               (u64)m * k * 2 >= 1ull << 32))
@@ -448,7 +444,8 @@ hipError_t lfmq_dq_tile(const void* qweight, const void* scales,
     e = step <= 96 ? go_bits<DENSE, false>(A, bits, mb, step, stream)
                    : go_bits<DENSE, true>(A, bits, mb, step, stream);
   if (e != hipSuccess || splits == 1) return e;
-  return lfmq_dq_rows_sum(part, y, bias, resid, m, n, splits, glu, stream);
+  return lfmq_dq_rows_sum(part, y, bias, resid, m, n, splits, glu, stream,
+                          nullptr, end);
 }
 
 // rows of x (or slots) by expert, tiles of up to 128 of them (DqArgs); glu:

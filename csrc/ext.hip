@@ -5,6 +5,8 @@
 #include <ATen/cuda/CUDAContext.h>
 #include <hip/hip_runtime.h>
 
+#include "dq_short.h"
+
 hipError_t lfmq_pack(const void*, void*, long, int, int, hipStream_t);
 hipError_t lfmq_unpack(const void*, void*, long, int, int, hipStream_t);
 hipError_t lfmq_dq_gemv(const void*, const void*, const void*, const void*,
@@ -15,7 +17,8 @@ int lfmq_dq_rows_splits(int, int, int, int);
 hipError_t lfmq_dq_rows(const void*, const void*, const void*, const void*,
                         void*, const void*, const void*, void*, int, int, int,
                         int, int, int, float,
-                        bool, hipStream_t);
+                        bool, hipStream_t, const float* row_scale = nullptr,
+                        const DqRowEnd* end = nullptr);
 bool lfmq_dq_row_ok(int, int, int);
 hipError_t lfmq_dq_row(const void*, const void*, const void*, const void*,
                        void*, const void*, const void*, int, int, int, int,
@@ -29,11 +32,11 @@ hipError_t lfmq_dq_wide_experts(const void*, const void*, const void*,
                                 int, int, int, int, int, bool, hipStream_t);
 bool lfmq_dq_tile_ok(int, int);
 int lfmq_dq_tile_splits(int, int, int, int);
-hipError_t lfmq_dq_rows_sum(const void*, void*, const void*, const void*, int,
-                            int, int, bool, hipStream_t);
 hipError_t lfmq_dq_tile(const void*, const void*, const void*, const void*,
                         void*, const void*, const void*, void*, int, int, int,
-                        int, int, int, bool, hipStream_t);
+                        int, int, int, bool, hipStream_t,
+                        const DqRowEnd* end = nullptr);
+hipError_t lfmq_row_scale(const void*, void*, int, int, float, hipStream_t);
 hipError_t lfmq_rmsnorm(const void*, const void*, const void*, void*, void*,
                         int, int, float, hipStream_t);
 hipError_t lfmq_rope(void*, void*, const void*, const void*, int, int, int,
@@ -94,7 +97,6 @@ hipError_t lfmq_argmax_rows(const void*, void*, void*, void*, int, int,
 hipError_t lfmq_read_probe(const void*, void*, long, long, int, int, int,
                            hipStream_t);
 #include "dq_block.h"
-#include "dq_short.h"
 #include "engine_args.h"
 
 namespace {
@@ -293,10 +295,22 @@ bool short_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
          (uintptr_t)qweight.data_ptr() % 16 == 0;
 }
 
+// What goes with whole rows of a product: a factor of x's rows, and what follows
+// rows of the result, which the sum of parts takes along if there is one.
+struct RowWays {
+  const float* scale = nullptr;
+  const DqRowEnd* end = nullptr;
+  bool* ended = nullptr;
+  const DqRowEnd* ends() const {           // for a launch that sums parts
+    if (end != nullptr) *ended = true;
+    return end;
+  }
+};
+
 void dq_short(const torch::Tensor& x, const torch::Tensor& qweight,
               const torch::Tensor& scales, const torch::Tensor& qzeros,
               const void* bias, const void* resid, torch::Tensor& y, long g,
-              long bits, bool glu) {
+              long bits, bool glu, const RowWays& ways) {
   const int m = (int)x.size(0), k = (int)x.size(1), n = (int)qweight.size(0);
   const DqShortPlan P = lfmq_dq_short_plan(m, n, k, (int)g, (int)bits, glu);
   DqArgs A{};
@@ -318,21 +332,23 @@ void dq_short(const torch::Tensor& x, const torch::Tensor& qweight,
   A.k = k;
   A.g = (int)g;
   A.splits = P.splits;
+  A.row_scale = ways.scale;
   CHECK_HIP(lfmq_dq_short(A, P, (int)bits, glu, stream()));
   if (P.splits > 1)
     CHECK_HIP(lfmq_dq_rows_sum(part.data_ptr(), y.data_ptr(), bias, resid, m, n,
-                               P.splits, glu, stream()));
+                               P.splits, glu, stream(), ways.scale,
+                               ways.ends()));
 }
 
 torch::Tensor rmsnorm(torch::Tensor x, torch::Tensor w, double eps,
                       c10::optional<torch::Tensor> residual);
 torch::Tensor silu_mul_fused(torch::Tensor gate_up);
 
-torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
-                        torch::Tensor scales, torch::Tensor qzeros, long bits,
-                        long g, c10::optional<torch::Tensor> bias,
-                        c10::optional<torch::Tensor> resid, double rms_eps,
-                        long cols_hint) {
+torch::Tensor linear(torch::Tensor x, const torch::Tensor& qweight,
+                     const torch::Tensor& scales, const torch::Tensor& qzeros,
+                     long bits, long g, const c10::optional<torch::Tensor>& bias,
+                     const c10::optional<torch::Tensor>& resid, double rms_eps,
+                     long cols_hint, const RowWays& ways) {
   check_t(x, torch::kBFloat16, "x");
   check_t(qweight, torch::kInt32, "qweight");
   check_t(scales, torch::kBFloat16, "scales");
@@ -368,7 +384,7 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
   // of the last two: n 3072, k 8192 (4 bits) 14.5 / 17.1 at 32 rows, 17.7 / 17.1 at
   // 33, 25.5 / 18.7 at 49; n 16384, k 2048 (8 bits, groups of 64) 18.4 / 21.4 at 48,
   // 30.7 / 21.6 at 49.
-  const bool rms = rms_eps >= 0;
+  const bool rms = rms_eps >= 0, scaled = ways.scale != nullptr;
   const bool tile = tile_addresses(n, k, bits);
   const bool large = tile && !rms && k >= 4096 && (long)n * k >= 24l << 20 &&
                      (rptr == nullptr ||
@@ -378,12 +394,14 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
   const bool small = !rms && rptr == nullptr && (long)n * k <= 4l << 20;
   const bool by_rows = (cols_hint == 0 ? m >= rows_from(bits, n, k, g)
                                        : cols_hint == 6 && m > 4) &&
-                       (!tile || m <= (large ? 32 : small ? 96 : 48)) &&
+                       (!tile || m <= (scaled ? 48 : large ? 32 : small ? 96 : 48)) &&
                        lfmq_dq_rows_ok(m, n, k, (int)g, rms);
-  const bool block = rptr == nullptr &&
+  const bool block = rptr == nullptr && !scaled &&
                      block_rows(qweight, scales, m, n, k, g, bits, false);
   const bool few = cols_hint == 0 && !rms && !(small && by_rows) &&
                    short_rows(qweight, m, n, k, g, bits, false, block);
+  TORCH_CHECK(!scaled || (m > 16 && m <= 48 && (by_rows || few)),
+              "factors of rows are for 17 to 48 of them");
   if (m > 16) {
     TORCH_CHECK((by_rows || !rms) && (m <= 48 || rptr == nullptr),
                 "fused rms/resid is a decode (m <= 48) path");
@@ -410,13 +428,15 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
                            rptr, m, n, k, (int)g, (int)bits, (float)rms_eps,
                            false, stream()));
   } else if (few) {
-    dq_short(x, qweight, scales, qzeros, bptr, rptr, y, g, bits, false);
+    dq_short(x, qweight, scales, qzeros, bptr, rptr, y, g, bits, false,
+             ways);
   } else if (by_rows) {
     const int splits = rms ? 1 : lfmq_dq_rows_splits(m, n, k, (int)g);
     CHECK_HIP(lfmq_dq_rows(qweight.data_ptr(), scales.data_ptr(),
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                            rptr, parts(splits), m, n, k, (int)g, (int)bits,
-                           splits, (float)rms_eps, false, stream()));
+                           splits, (float)rms_eps, false, stream(), ways.scale,
+                           splits > 1 ? ways.ends() : nullptr));
   } else if (m <= 16) {
     CHECK_HIP(lfmq_dq_gemv(qweight.data_ptr(), scales.data_ptr(),
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
@@ -429,10 +449,78 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
     CHECK_HIP(lfmq_dq_tile(qweight.data_ptr(), scales.data_ptr(),
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                            rptr, parts(splits), m, n, k, (int)g, (int)bits,
-                           splits, false, stream()));
+                           splits, false, stream(),
+                           splits > 1 ? ways.ends() : nullptr));
   }
   return y;
 }
+
+torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
+                        torch::Tensor scales, torch::Tensor qzeros, long bits,
+                        long g, c10::optional<torch::Tensor> bias,
+                        c10::optional<torch::Tensor> resid, double rms_eps,
+                        long cols_hint) {
+  return linear(x, qweight, scales, qzeros, bits, g, bias, resid, rms_eps,
+                cols_hint, {});
+}
+
+// 1 / sqrt(mean x^2 + eps) of each row, fp32
+torch::Tensor row_scale(torch::Tensor x, double eps) {
+  check_t(x, torch::kBFloat16, "x");
+  TORCH_CHECK(x.dim() == 2, "x must be [m, k]");
+  auto s = torch::empty({x.size(0)}, x.options().dtype(torch::kFloat32));
+  CHECK_HIP(lfmq_row_scale(x.data_ptr(), s.data_ptr(), (int)x.size(0),
+                           (int)x.size(1), (float)eps, stream()));
+  return s;
+}
+
+const float* factors(const c10::optional<torch::Tensor>& scale, long m) {
+  if (!scale.has_value()) return nullptr;
+  check_t(*scale, torch::kFloat32, "row scale");
+  TORCH_CHECK(scale->numel() == m, "one factor a row");
+  return scale->data_ptr<float>();
+}
+
+// whether a workgroup of the sum of parts can hold a row and read beside it
+bool rows_end(int n, const c10::optional<torch::Tensor>& bias,
+              const c10::optional<torch::Tensor>& add, const void* w) {
+  auto even = [](const c10::optional<torch::Tensor>& t) {
+    return !t.has_value() || (uintptr_t)t->data_ptr() % 8 == 0;
+  };
+  return lfmq_dq_row_end_ok(n) && even(bias) && even(add) &&
+         (uintptr_t)w % 8 == 0;
+}
+
+// Rows of x times their factors (17 to 48 rows); eps >= 0: also row_scale of the
+// result, with the sum of the product's parts where it has some
+std::vector<torch::Tensor> dq_linear_scaled(
+    torch::Tensor x, c10::optional<torch::Tensor> scale, torch::Tensor qweight,
+    torch::Tensor scales, torch::Tensor qzeros, long bits, long g,
+    c10::optional<torch::Tensor> bias, c10::optional<torch::Tensor> resid,
+    double eps) {
+  const int m = (int)x.size(0), n = (int)qweight.size(0);
+  if (resid.has_value())
+    TORCH_CHECK(resid->numel() == (long)m * n, "one residual a result");
+  RowWays ways{factors(scale, m)};
+  DqRowEnd end{};
+  bool ended = false;
+  torch::Tensor out;
+  if (eps >= 0) {
+    out = torch::empty({m}, x.options().dtype(torch::kFloat32));
+    end.scale = out.data_ptr<float>();
+    end.eps = (float)eps;
+    ways.ended = &ended;
+    if (rows_end(n, bias, resid, nullptr)) ways.end = &end;
+  }
+  auto y = linear(x, qweight, scales, qzeros, bits, g, bias, resid, -1.0, 0,
+                  ways);
+  if (eps < 0) return {y};
+  if (!ended)
+    CHECK_HIP(lfmq_row_scale(y.data_ptr(), out.data_ptr(), m, n, (float)eps,
+                             stream()));
+  return {y, out};
+}
+
 
 torch::Tensor rmsnorm(torch::Tensor x, torch::Tensor w, double eps,
                       c10::optional<torch::Tensor> residual) {
@@ -597,7 +685,7 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
   if (cols_hint == 0 && rms_eps < 0 && n % 2 == 0 &&
       short_rows(qweight, m, n, k, g, bits, true, block)) {
     if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
-    dq_short(x, qweight, scales, qzeros, nullptr, nullptr, y, g, bits, true);
+    dq_short(x, qweight, scales, qzeros, nullptr, nullptr, y, g, bits, true, {});
     return y;
   }
   if (cols_hint == 0 && tile && n % 2 == 0 && m > (large ? 32 : 48) &&
@@ -652,6 +740,36 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
                                 qzeros.data_ptr(), x.data_ptr(), y.data_ptr(),
                                 m, n, k, (int)g, (int)bits, (float)rms_eps,
                                 (int)cols_hint, stream()));
+  return y;
+}
+
+// dq_gemv_gateup of rows of x times their factors (17 to 48 rows)
+torch::Tensor dq_gateup_scaled(torch::Tensor x, torch::Tensor scale,
+                               torch::Tensor qweight, torch::Tensor scales,
+                               torch::Tensor qzeros, long bits, long g) {
+  check_t(x, torch::kBFloat16, "x");
+  check_t(qweight, torch::kInt32, "qweight");
+  check_t(scales, torch::kBFloat16, "scales");
+  check_t(qzeros, torch::kInt32, "qzeros");
+  TORCH_CHECK(x.dim() == 2, "x must be [m, k]");
+  TORCH_CHECK(g > 0, "groups have at least one column");
+  const int m = (int)x.size(0), k = (int)x.size(1);
+  const int n = (int)qweight.size(0);
+  TORCH_CHECK(qweight.size(1) == (long)k * bits / 32, "qweight/k mismatch");
+  TORCH_CHECK(m > 16 && m <= 48 && n % 2 == 0 &&
+                  lfmq_dq_rows_ok(m, n, k, (int)g, true),
+              "factors of rows are for 17 to 48 of them");
+  RowWays ways{factors(scale, m)};
+  if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
+  auto y = torch::empty({m, n / 2}, x.options());
+  if (short_rows(qweight, m, n, k, g, bits, true, false))
+    dq_short(x, qweight, scales, qzeros, nullptr, nullptr, y, g, bits, true,
+             ways);
+  else
+    CHECK_HIP(lfmq_dq_rows(qweight.data_ptr(), scales.data_ptr(),
+                           qzeros.data_ptr(), x.data_ptr(), y.data_ptr(),
+                           nullptr, nullptr, nullptr, m, n, k, (int)g,
+                           (int)bits, 1, -1.f, true, stream(), ways.scale));
   return y;
 }
 
@@ -1167,6 +1285,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("pack", &pack, "pack int codes");
   m.def("unpack", &unpack, "unpack int codes");
   m.def("dq_linear", &dq_linear, "fused dequant GEMV/GEMM");
+  m.def("row_scale", &row_scale, "1 / root mean square of rows");
+  m.def("dq_linear_scaled", &dq_linear_scaled,
+        "dq_linear of rows times factors, and the result's own");
+  m.def("dq_gateup_scaled", &dq_gateup_scaled,
+        "dq_gemv_gateup of rows times factors");
   m.def("rmsnorm", &rmsnorm, "fused rmsnorm");
   m.def("rmsnorm_residual", &rmsnorm_residual, "fused rmsnorm + residual");
   m.def("rope", &rope, "fused rope (in-place)");

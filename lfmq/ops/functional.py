@@ -88,6 +88,34 @@ def dq_linear(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor,
     return ref.dq_linear(x, qweight, scales, qzeros, bits, group_size, bias).to(x.dtype)
 
 
+def row_scale(x: torch.Tensor, eps: float) -> torch.Tensor:
+    """GPU-only 1 / sqrt(mean x^2 + eps) of each row, fp32."""
+    return hip_ext().row_scale(x.reshape(-1, x.shape[-1]), eps)
+
+
+def dq_linear_scaled(x: torch.Tensor, scale: Optional[torch.Tensor], p,
+                     resid: Optional[torch.Tensor] = None, eps: float = -1.0):
+    """GPU-only dq_linear of the packed layer p for 17 to 48 rows: x's rows
+    times scale (its row_scale, for an RMSNorm without weights in front); with
+    eps >= 0 the result and its own row_scale."""
+    r2 = resid.reshape(-1, resid.shape[-1]).contiguous() \
+        if resid is not None else None
+    y, *own = hip_ext().dq_linear_scaled(
+        x.reshape(-1, x.shape[-1]), scale, p.qweight, p.scales, p.qzeros,
+        p.bits, p.group_size, p.bias, r2, eps)
+    y = _guard(y, "dq_linear").reshape(*x.shape[:-1], y.shape[-1])
+    return (y, *own) if own else y
+
+
+def dq_gateup_scaled(x: torch.Tensor, scale: torch.Tensor, p) -> torch.Tensor:
+    """GPU-only dq_gemv_gateup of the packed layer p for 17 to 48 rows, which
+    are multiplied by scale."""
+    y = hip_ext().dq_gateup_scaled(x.reshape(-1, x.shape[-1]), scale,
+                                   p.qweight, p.scales, p.qzeros, p.bits,
+                                   p.group_size)
+    return _guard(y, "dq_gemv_gateup").reshape(*x.shape[:-1], y.shape[-1])
+
+
 def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     if gate.is_cuda:
         return hip_ext().silu_mul(gate.contiguous(), up.contiguous())

@@ -192,3 +192,32 @@ def test_few_rows_past_4_gib(m):
     y = ext().dq_linear(x, q, s, z, bits, g, None, None, -1.0, 0)
     close(y[:, -1024:], x.double() @ w.t())
     assert not bool(y[:, :-1024].any())
+
+
+@pytest.mark.parametrize("m,n,k,g,bits", [
+    (17, 2048, 4096, 64, 4), (48, 4096, 14336, 128, 4), (33, 4104, 2048, 64, 8),
+    (20, 8192, 4096, 128, 8), (48, 16384, 2048, 128, 4), (48, 512, 512, 64, 4),
+    (31, 1028, 1024, 128, 8), (47, 1030, 2048, 64, 4), (18, 24576, 2048, 64, 4)])
+def test_rows_times_their_factors(m, n, k, g, bits):
+    """A norm as factors of x's rows, and the result's own factors from the sum
+    of parts (rows of up to 2048, 4096, 8192 and 16384 columns, few and many
+    parts), from whole products and from rows that no workgroup holds."""
+    p, w = matrix(bits, n, k, g)
+    x = torch.randn(m, k, device=DEV).to(BF)
+    x[0] = 0
+    bias = torch.randn(n, device=DEV).to(BF)
+    resid = torch.randn(m, n, device=DEV).to(BF)
+    scale = ext().row_scale(x, 1e-5)
+    rms = normed(x, 1e-5) @ w.t()
+    # a sum of k squares in fp32 and a reciprocal root
+    own = torch.rsqrt((x.double() ** 2).mean(-1) + 1e-5)
+    assert float((scale.double() / own - 1).abs().max()) < 1e-5
+    y, = ext().dq_linear_scaled(x, scale, *p, bits, g, bias, None, -1.0)
+    close(y, rms + bias.double())
+    for s, want in ((None, x.double() @ w.t()), (scale, rms)):
+        y, out = ext().dq_linear_scaled(x, s, *p, bits, g, None, resid, 1e-6)
+        close(y, want + resid.double())
+        own = torch.rsqrt((y.double() ** 2).mean(-1) + 1e-6)
+        assert float((out.double() / own - 1).abs().max()) < 1e-5
+    if n % 2 == 0:
+        close(ext().dq_gateup_scaled(x, scale, *p, bits, g), gated(rms), 1e-2)
