@@ -20,16 +20,20 @@
 // scratch, and the last workgroup of the head to arrive merges them (a
 // ticket counter) or, without tickets, a second kernel does.
 //
-// A launch that only reads 402 MB takes 66 us, one of 33 MB 6.5: the rest is a
+// A launch that only reads 402 MB takes 66 us, one of 33 MB 6.5, and so does this
+// one from some 60 MB on since its loads are whole lines that pass the caches by
+// (b 48, T 2047 by half lines of keys 76.6, values past the caches 69, keys too
+// 72, keys by whole lines alike 67).  Below, the rest is a
 // chain from the length over the keys and the rotation to the scores, sums over
 // the lanes, and the merge's trips to memory.  So a wave's first keys and values
 // are on their way before the rotation and the next ones during a round, by loads
 // that stop at the range's end and wait by count; sums over the lanes are taken two
 // at a time by exchanges of lanes and not through LDS.  One layer of an 8B model
-// (32 query heads on 8), us before (loads in the round that needs them) and now:
-//   b 1,  T 129         8.1 ->  6.3      b 8,  T 4000     30.9 -> 28.5
-//   b 1,  T 7901       16.0 -> 13.8      b 20, T 900      21.6 -> 19.4
-//   b 8,  T 1000       13.4 -> 11.5      b 48, T 2047     80.2 -> 76.6 (5.2 TB/s)
+// (32 query heads on 8), cold, us before (loads in the round that needs them, in the
+// caches' way) and now:
+//   b 1,  T 129         8.1 ->  6.0      b 8,  T 4000     31.3 -> 26.5
+//   b 1,  T 7901       16.8 -> 13.9      b 20, T 900      21.9 -> 18.1
+//   b 8,  T 1000       14.3 -> 11.8      b 48, T 2047     80.0 -> 67.7 (5.9 TB/s)
 #include <type_traits>
 
 #include "common.h"
@@ -47,8 +51,8 @@ constexpr int MAX_SPLITS = 64;       // a wave merges them, one a lane
 // 12.4 / 13.2 at 700.
 constexpr int ONE_RANGE = 256, LEAST_KEYS = 128, MANY = 24;
 // Two workgroups a CU, three where a range has very many keys: us with 512 / 768
-// workgroups 14.3 / 15.2 (b 8, 1000 keys), 18.4 / 19.2 (b 16, 900), 81.5 / 77
-// (b 48, 2047).  Not where a workgroup has eight heads, of which two fit: 23.3 /
+// workgroups 26.5 / 27.6 (b 8, 4000 keys), 15.6 / 16.2 (b 16, 900), 71.6 / 67.7
+// (b 48, 2047; with 1536 70.4).  Not where a workgroup has eight heads, of which two fit: 23.3 /
 // 32.8 (28 heads on 4, b 13, 2000 keys of 16384).
 constexpr int FULL_WGS = 512, MORE_WGS = 768, LONG_RANGE = 1024;
 
@@ -115,6 +119,16 @@ __device__ __forceinline__ float sum_quarters(float a, float b) {
   return __builtin_bit_cast(float, p0) + __builtin_bit_cast(float, p1);
 }
 
+// a's lower half and b's, plus the upper halves eight columns away
+__device__ __forceinline__ float sum_pieces(float a, float b) {
+  const auto p = __builtin_amdgcn_permlane32_swap(
+      __builtin_bit_cast(u32, a), __builtin_bit_cast(u32, b), false, false);
+  const u32 p0 = p[0], p1 = p[1];
+  return __builtin_bit_cast(float, p0) +
+         __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                                       0, (int)p1, 0x128, 0xf, 0xf, true));
+}
+
 // Two floats of a partial result, past the caches of the XCD: a workgroup of
 // another one may be the reader.
 __device__ __forceinline__ void put2(float* p, float a, float b) {
@@ -143,11 +157,12 @@ __device__ __forceinline__ float merge_weight(const float* p, int used,
   return e / wave_reduce_sum_dpp(e * l);
 }
 
-template <int D, int GH, bool FUSED, int NW>
+// NT: keys and values pass the caches by (cache policy 2)
+template <int D, int GH, bool FUSED, int NW, bool NT>
 __global__ __launch_bounds__(NW * 64, NW == 8 || D * GH > 512 ? 2 : 3)
 void attn_decode_kernel(DArgs A) {
-  constexpr int TPB = NW * 64;
-  constexpr int KS = D / 32, LPR = D / 8;
+  constexpr int TPB = NW * 64, AUX = NT ? 2 : 0;
+  constexpr int KL = D / 64, LPR = D / 8;  // lines of 128 bytes a key
   constexpr int RPP = 64 / LPR;          // value rows a pass
   constexpr int NP = KT / RPP;           // passes a tile
   __shared__ __attribute__((aligned(16))) float ps[NW][KT][GH];
@@ -165,11 +180,12 @@ void attn_decode_kernel(DArgs A) {
   const int h0 = kh * group + ht * GH;             // first query head
   const int nh = min(GH, group - ht * GH);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int l15 = lane & 15, l4 = lane >> 4;
+  const int l15 = lane & 15, l4 = lane >> 4, lh = l15 & 7;
   const int vrow = lane / LPR, vcol = (lane % LPR) * 8;
   const s16x8 z8 = {0, 0, 0, 0, 0, 0, 0, 0};
 
-  s16x8 qf[KS];
+  s16x8 qf[KL];
+  auto piece = [&](int j) { return j * 64 + (l4 * 2 + (l15 >> 3)) * 8; };
   u32x4 v_new = {0, 0, 0, 0};
   // what does not depend on the number of keys is on its way with it: a wave
   // rotates heads wave, wave + 4, one angle a lane
@@ -200,7 +216,11 @@ void attn_decode_kernel(DArgs A) {
   // A wave's keys and values from t0 on, zeros past the range.  The first are on
   // their way beside the rotation, the next ones as soon as there is room for
   // them; the loads are there without keys too, or the compiler waits for all.
-  s16x8 kf[2][KS];
+  // A load of keys takes a whole line of 128 bytes of 8 of them: lane l15 has key
+  // l15 % 8, piece l4 * 2 of the line below l15 8 and l4 * 2 + 1 from there.  As
+  // rows of a product, keys' first pieces and keys' second ones; its columns are
+  // heads' first pieces and, 8 on, heads' second ones.
+  s16x8 kf[KT / 8][KL];
   u32x4 vv[NP];
   auto rows_of = [&](const unsigned short* base, int t0) {
     const int n = max(0, min(KT, hi - t0));
@@ -209,19 +229,19 @@ void attn_decode_kernel(DArgs A) {
   auto load_keys = [&](int t0) {
     const auto r = rows_of(K, t0);
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
+    for (int g = 0; g < KT / 8; ++g)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        kf[mt][ks] = __builtin_bit_cast(
+      for (int j = 0; j < KL; ++j)
+        kf[g][j] = __builtin_bit_cast(
             s16x8, __builtin_amdgcn_raw_buffer_load_b128(
-                       r, ((mt * 16 + l15) * D + ks * 32 + l4 * 8) * 2, 0, 0));
+                       r, ((g * 8 + (l15 & 7)) * D + piece(j)) * 2, 0, AUX));
   };
   auto load_values = [&](int t0) {
     const auto r = rows_of(V, t0);
 #pragma unroll
     for (int i = 0; i < NP; ++i)
       vv[i] = __builtin_amdgcn_raw_buffer_load_b128(
-          r, ((i * RPP + vrow) * D + vcol) * 2, 0, 0);
+          r, ((i * RPP + vrow) * D + vcol) * 2, 0, AUX);
   };
   const int first = lo + __builtin_amdgcn_readfirstlane(wave) * KT;
   load_keys(first);
@@ -253,29 +273,36 @@ void attn_decode_kernel(DArgs A) {
     }
     __syncthreads();
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      qf[ks] = l15 < nh ? *(const s16x8*)&qs[l15 < GH ? l15 : 0][ks * 32 + l4 * 8]
-                        : z8;
+    for (int j = 0; j < KL; ++j)
+      qf[j] = lh < nh ? *(const s16x8*)&qs[lh < GH ? lh : 0][piece(j)] : z8;
   } else {
-    const unsigned short* qr = A.q + ((u64)bb * A.hq + h0 + l15) * D;
+    const unsigned short* qr = A.q + ((u64)bb * A.hq + h0 + lh) * D;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      qf[ks] = l15 < nh ? *(const s16x8*)(qr + ks * 32 + l4 * 8) : z8;
+    for (int j = 0; j < KL; ++j)
+      qf[j] = lh < nh ? *(const s16x8*)(qr + piece(j)) : z8;
   }
   const float sn_h = FUSED && l15 < nh ? s_new[l15 < GH ? l15 : 0] : 0.f;
 
   float m = -INFINITY, l = 0.f;          // of head l15
   float acc[GH][8] = {};
   for (int t0 = first; t0 < hi; t0 += NW * KT) {
-    f32x4 sc[2] = {};
+    f32x4 pt[KT / 8] = {};
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
+    for (int j = 0; j < KL; ++j)
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
-        sc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[mt][ks], qf[ks],
-                                                         sc[mt], 0, 0, 0);
+      for (int g = 0; g < KT / 8; ++g)
+        pt[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[g][j], qf[j], pt[g],
+                                                        0, 0, 0);
     __builtin_amdgcn_sched_barrier(0);         // not before: other registers
     load_keys(t0 + NW * KT);
+    // a result's rows: first pieces in the lower half of the wave, second ones in
+    // the upper half; what pairs a first with a second stays in lanes from 8 on
+    f32x4 sc[2];
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        sc[mt][r] = sum_pieces(pt[mt * 2][r], pt[mt * 2 + 1][r]);
     float mx = -INFINITY;
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
@@ -477,6 +504,12 @@ bool eight_waves(int d, int gh, int wgs, int T) {
          (long)wgs * ((T + ONE_RANGE - 1) / ONE_RANGE) <= 256;
 }
 
+// From how many bytes of keys and values on they pass the caches by: less than
+// this, of all layers, may still be there at the next token (b 1, 129 keys in a
+// step of four layers 0.25 us a launch).  us in the caches' way / past them, cold: b 1, 600 keys (2.5 MB) 7.1 / 7.1, b 4,
+// 300 (4.9 MB) 7.4 / 7.3, b 16, 129 (8.5 MB) 7.2 / 6.8, b 48, 300 16.5 / 15.3.
+constexpr long PAST_CACHES = 4l << 20;
+
 template <int D, bool FUSED>
 hipError_t launch(DArgs A, int b, hipStream_t stream) {
   const int group = A.hq / A.hkv, gh = head_tile(group);
@@ -488,10 +521,15 @@ hipError_t launch(DArgs A, int b, hipStream_t stream) {
   // would get all of those.  us with ranges first / second / last: 32 heads on
   // 32, b 4, 200 keys of 500 9.6 / 8.4 / 7.2; 28 on 4, b 20 15.7 / 15.1 / 13.4.
   const dim3 grid(A.hkv * A.htiles, b, A.splits);
+  const bool nt = (long)b * A.hkv * A.T * D * 4 >= PAST_CACHES;
   auto go = [&](auto heads, auto waves) {
     constexpr int G = decltype(heads)::value, NW = decltype(waves)::value;
-    hipLaunchKernelGGL((attn_decode_kernel<D, G, FUSED, NW>), grid,
-                       dim3(NW * 64), 0, stream, A);
+    if (nt)
+      hipLaunchKernelGGL((attn_decode_kernel<D, G, FUSED, NW, true>), grid,
+                         dim3(NW * 64), 0, stream, A);
+    else
+      hipLaunchKernelGGL((attn_decode_kernel<D, G, FUSED, NW, false>), grid,
+                         dim3(NW * 64), 0, stream, A);
     if (A.splits > 1 && A.tickets == nullptr)
       hipLaunchKernelGGL((attn_decode_merge<D, NW>), dim3(b * A.hq), dim3(64), 0,
                          stream, A);

@@ -80,3 +80,11 @@ def test_rows_past_the_keys(b, T, room, hq, hkv, d):
     want = (torch.softmax(q @ k.transpose(2, 3) * d ** -0.5, -1) @ v).view(b, -1)
     # roundings of q, k and o, as above
     assert float((o.view(b, -1).double() - want).norm() / want.norm()) < 6e-3
+
+
+# up to 4 MiB of keys and values by the caches, from there on past them
+@pytest.mark.parametrize("b,T,room,hq,hkv,d", [
+    (2, 511, 0, 8, 8, 128), (2, 512, 0, 32, 8, 128), (2, 500, 13, 16, 8, 128),
+    (3, 1366, 0, 16, 2, 128), (4, 513, 0, 16, 8, 64), (5, 1100, 77, 8, 8, 64)])
+def test_keys_past_the_caches(b, T, room, hq, hkv, d):
+    test_rows_past_the_keys(b, T, room, hq, hkv, d)
