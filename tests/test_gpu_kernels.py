@@ -939,6 +939,19 @@ def test_linear_rows(m, n, k, glu):
                  <= 2 ** -8 * want.abs() + slack + 1e-30).all())
 
 
+# tiles of 8, 16, 32, 48 and 64 columns, one or two of a wave's chunks in flight,
+# below and from 4 MiB of weights on, a last tile that is not full
+@pytest.mark.parametrize("m,n,k,glu", [
+    (1, 8193, 3200, False), (2, 5001, 2304, False), (5, 2001, 1152, False),
+    (8, 1023, 2048, False), (8, 1025, 2048, False), (12, 3001, 1152, False),
+    (16, 4097, 4224, False), (8, 8189, 1152, False), (6, 8161, 2304, False),
+    (6, 12283, 1152, False), (9, 16375, 2304, False), (16, 16383, 384, False),
+    (4, 2 * 4099, 2304, True), (6, 2 * 1001, 2176, True),
+    (8, 2 * 8191, 1152, True), (3, 2 * 4097, 3200, True)])
+def test_linear_rows_by_tiles(m, n, k, glu):
+    test_linear_rows(m, n, k, glu)
+
+
 def test_linear_rows_leaves_the_rest_to_the_library():
     from lfmq.ops import functional as F
     from lfmq.ops import seq_ext
