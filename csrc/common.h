@@ -81,6 +81,14 @@ __device__ __forceinline__ float wave_reduce_sum(float v) {
   return v;
 }
 
+// y of the lane eight further of its sixteen in the upper eight lanes (HI) or the
+// lower ones, x in the others
+template <bool HI>
+__device__ __forceinline__ u32 other8(u32 x, u32 y) {
+  return (u32)__builtin_amdgcn_update_dpp((int)x, (int)y, 0x128, 0xf,
+                                          HI ? 0xc : 0x3, false);
+}
+
 // DPP-based wave sum: ~6 VALU ops instead of 6 LDS-unit bpermute round
 // trips (~20 vs ~500 cycles — decisive at 1 wave/SIMD where nothing hides
 // the bpermute latency).  rocPRIM's classic CDNA ladder: row_shr 1/2/4/8

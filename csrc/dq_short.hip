@@ -288,7 +288,8 @@ __global__ __launch_bounds__(TPB, 2) void dq_short_kernel(DqArgs A, int mb,
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = t * 16 + l4 * 4 + r;
-        const float scale = A.row_scale != nullptr && row < rows
+        // (of up to 48 rows)
+        const float scale = MT <= 3 && A.row_scale != nullptr && row < rows
                                 ? A.row_scale[row0 + row]
                                 : 1.f;
         float v = MODE == GLU

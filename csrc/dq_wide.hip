@@ -20,7 +20,7 @@
 //   n 6144, k 4096, norm           8.9 /  7.6   9.4 /  8.7  10.8 / 10.0
 //   n 2048, k 2048, residual       4.9 /  4.1   5.5 /  4.9   6.3 /  5.6
 //   n 16384, k 2048, norm, gate    9.8 /  8.3  10.4 /  9.3  11.4 / 10.5
-//   n 32000, k 4096 (8 bits)      31.0 / 28.3  34.5 / 29.2  40.5 / 30.6
+//   n 32000, k 4096 (8 bits)      31.0 / 26.2  34.5 / 27.0  40.5 / 27.3
 // 8 experts of n 28672, k 4096 and n 4096, k 14336, one to four rows each:
 // 130.6 -> 110.8, 72.5 -> 70.9.  Two steps of weights in flight a wave: 17.1
 // us instead of 16.9 at 8 rows; eight waves with twice the k 17.9; batches of
@@ -45,8 +45,10 @@ __host__ __device__ __forceinline__ int lanes_of(int rows) {
   return rows <= 4 ? 16 : (rows <= 8 ? 32 : 64);
 }
 
-// MORE: more than one step of k
-template <int BITS, int KC, DqMode MODE, bool MORE, int NW>
+// MORE: more than one step of k.  LINES: a load takes a whole 128-byte line of eight
+// rows of W, past the caches: pieces of two chunks (PAIR), or the halves of one;
+// lanes of the two eights exchange theirs on the way into the operands.
+template <int BITS, int KC, DqMode MODE, bool MORE, int NW, bool LINES>
 __global__ __launch_bounds__(NW * 64, 4) void dq_wide_kernel(Wide W) {
   const DqArgs& A = W.A;
   constexpr int TPB = NW * 64;
@@ -94,7 +96,11 @@ __global__ __launch_bounds__(NW * 64, 4) void dq_wide_kernel(Wide W) {
   // rows past the last one repeat it
   int xr = row0 + min(l15, rows - 1);
   if (MODE != DENSE && A.src != nullptr) xr = A.src[xr];
-  const char* xp = (const char*)A.x + ((u64)xr * A.k + l4 * (KC / 4)) * 2;
+  // halves of a chunk: its values of x are read in that order
+  constexpr bool PAIR = LINES && WD == 4, HALVES = LINES && WD == 8;
+  static_assert(!LINES || PAIR || HALVES, "");
+  constexpr int XP = HALVES ? 16 : KC / 4;         // values of x in a piece
+  const char* xp = (const char*)A.x + ((u64)xr * A.k + l4 * XP) * 2;
   auto chunk = [&](int p) { return (p * NW + wave) * S; };
   s16x8 xq[S][J];
   auto fetch_x = [&](int p) {
@@ -103,7 +109,8 @@ __global__ __launch_bounds__(NW * 64, 4) void dq_wide_kernel(Wide W) {
       const int c = min(chunk(p) + s, C - 1);
 #pragma unroll
       for (int j = 0; j < J; ++j)
-        xq[s][j] = *(const s16x8*)(xp + (u32)(c * KC + j * 8) * 2);
+        xq[s][j] = *(const s16x8*)(
+            xp + (u32)(c * KC + (HALVES ? j / 2 * 64 + j % 2 * 8 : j * 8)) * 2);
     }
   };
   // this lane's row of W in tile t, from r0 on (GLU: gate, then up)
@@ -111,27 +118,54 @@ __global__ __launch_bounds__(NW * 64, 4) void dq_wide_kernel(Wide W) {
     return min(t * TC + (H == 2 ? l15 & 7 : l15), nr - 1);
   };
   const u64 wrow = (u64)A.k * BITS / 8;
-  const char* wp = A.w + (first + r0 + (H == 2 ? (l15 >> 3) * nout : 0)) * wrow +
-                   l4 * (WD * 4);
-  u32 w[S][WD];
+  const int l7 = l15 & 7, odd = l15 >> 3;
+  const char* wp = A.w + (first + r0 + (H == 2 && !LINES ? odd * nout : 0)) * wrow +
+                   l4 * (LINES ? 16 : WD * 4) + (HALVES ? odd * 64 : 0);
+  u32 w[S][WD];                          // LINES: of rows l7, then of l7 + 8
   auto fetch_w = [&](int p, int t) {
-    const char* row = wp + local(t) * wrow;
+    if constexpr (LINES) {
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      const u32* a =
-          (const u32*)(row + (u32)min(chunk(p) + s, C - 1) * (KC * BITS / 8));
-      if constexpr (WD >= 4) {
+      for (int h = 0; h < 2; ++h) {
+        const char* row =
+            wp + (u64)(min(t * TC + (H == 2 ? l7 : h * 8 + l7), nr - 1) +
+                       (H == 2 ? h * nout : 0)) * wrow;
 #pragma unroll
-        for (int i = 0; i < WD / 4; ++i) {
-          const u32x4 v = ((const u32x4*)a)[i];
+        for (int s = 0; s < (PAIR ? S / 2 : S); ++s) {
+          const int c = min(chunk(p) + (PAIR ? 2 * s + odd : s), C - 1);
+          const u32x4 v = __builtin_nontemporal_load(
+              (const u32x4*)(row + (u32)c * (KC * BITS / 8)));
 #pragma unroll
-          for (int e = 0; e < 4; ++e) w[s][i * 4 + e] = v[e];
+          for (int e = 0; e < 4; ++e)
+            w[PAIR ? 2 * s + h : s][(PAIR ? 0 : h * 4) + e] = v[e];
         }
-      } else {
+      }
+    } else {
+      const char* row = wp + local(t) * wrow;
 #pragma unroll
-        for (int e = 0; e < WD; ++e) w[s][e] = a[e];
+      for (int s = 0; s < S; ++s) {
+        const u32* a = (const u32*)(
+            row + (u32)min(chunk(p) + s, C - 1) * (KC * BITS / 8));
+        if constexpr (WD >= 4) {
+#pragma unroll
+          for (int i = 0; i < WD / 4; ++i) {
+            const u32x4 v = ((const u32x4*)a)[i];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[s][i * 4 + e] = v[e];
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < WD; ++e) w[s][e] = a[e];
+        }
       }
     }
+  };
+  // this lane's row's dword e of chunk s
+  auto word = [&](int s, int e) {
+    if constexpr (!LINES) return w[s][e];
+    const bool hi = PAIR ? s & 1 : e >= 4;
+    const u32 x = PAIR ? w[s & ~1][e] : w[s][e & 3];
+    const u32 y = PAIR ? w[s | 1][e] : w[s][e | 4];
+    return hi ? other8<false>(y, x) : other8<true>(x, y);
   };
   fetch_x(0);
   fetch_w(0, 0);
@@ -179,8 +213,8 @@ __global__ __launch_bounds__(NW * 64, 4) void dq_wide_kernel(Wide W) {
           f32x4 a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int j = 0; j < J; ++j) {
-            const s16x8 b = BITS == 4 ? codes8_dealt(w[s][j * UW])
-                                      : codes8<BITS>(&w[s][j * UW]);
+            const u32 two[2] = {word(s, j * UW), word(s, j * UW + UW - 1)};
+            const s16x8 b = BITS == 4 ? codes8_dealt(two[0]) : codes8<BITS>(two);
             a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[s][j], b, a, 0, 0, 0);
           }
           const float sc = bf16_bits_to_f32(ms[lr * G + c]);
@@ -253,7 +287,7 @@ int waves_of(int k) { return k <= 8 * KS ? 8 : 16; }
 size_t room_of(int NW) { return 160 * 1024 / (16 / NW); }
 
 // rows: the most that a tile of rows has; lists: tiles of rows
-template <int BITS, int KC, DqMode MODE, bool MORE, int NW>
+template <int BITS, int KC, DqMode MODE, bool MORE, int NW, bool LINES = false>
 hipError_t go(const DqArgs& A, int rows, int lists, hipStream_t stream) {
   constexpr int TC = MODE == GLU ? 8 : 16;
   const int tiles = (int)ceil_div_u32(MODE == GLU ? A.n / 2 : A.n, TC);
@@ -278,7 +312,7 @@ hipError_t go(const DqArgs& A, int rows, int lists, hipStream_t stream) {
   }
   if (nt == 0) return hipErrorInvalidValue;
   const int grid = (int)ceil_div_u32(tiles, nt);
-  const auto kernel = dq_wide_kernel<BITS, KC, MODE, MORE, NW>;
+  const auto kernel = dq_wide_kernel<BITS, KC, MODE, MORE, NW, LINES>;
   static bool set = false;
   if (!set) {
     LFMQ_CHECK_HIP(hipFuncSetAttribute(
@@ -296,6 +330,22 @@ hipError_t go(const DqArgs& A, int rows, int lists, hipStream_t stream) {
 
 template <int BITS, int KC, DqMode MODE>
 hipError_t go_k(const DqArgs& A, int rows, int lists, hipStream_t stream) {
+  // Whole lines from 8 MiB on: below, the exchange costs more.  us by 64 bytes of 16
+  // rows / by lines: n 28672, k 4096 (4 bits, norm and gate, 16 rows) 18.8 / 18.7, n
+  // 6144, k 4096 (12 MiB) 10.3 / 10.0, n 4096, k 4096 (8) 8.8 / 8.7; n 32000, k 4096 (8
+  // bits, groups of 128) 30.4 / 27.3, n 16384, k 2048 (32 MiB) 13.4 / 13.1; n 3072, k
+  // 2048 (6, 2 rows) 5.1 / 5.3.  With more steps there is no room for it (n 10240, k
+  // 8192, 4 bits 15.4 / 16.3); 4 bits in groups of 64 have 32 bytes a chunk; and an
+  // expert's second tile of rows reads again what the first one has read (8 experts, 120
+  // rows, n 28672, k 4096 164 / 170).
+  if constexpr (BITS * KC >= 512 && MODE != SLOTS) {
+    if (A.tiles == nullptr && (u64)A.n * A.k * BITS / 8 >= 8u << 20) {
+      if (A.k <= 8 * KS)
+        return go<BITS, KC, MODE, false, 8, true>(A, rows, lists, stream);
+      if (A.k <= 16 * KS)
+        return go<BITS, KC, MODE, false, 16, true>(A, rows, lists, stream);
+    }
+  }
   if (A.k <= 8 * KS) return go<BITS, KC, MODE, false, 8>(A, rows, lists, stream);
   if (A.k <= 16 * KS)
     return go<BITS, KC, MODE, false, 16>(A, rows, lists, stream);

@@ -33,16 +33,12 @@ struct LArgs {
   int m, n, k;
 };
 
-// b of the lane eight further of its sixteen in the upper eight lanes (HI) or the
-// lower ones, a in the others
 template <bool HI>
 __device__ __forceinline__ s16x8 other8(s16x8 a, s16x8 b) {
   const u32x4 x = __builtin_bit_cast(u32x4, a), y = __builtin_bit_cast(u32x4, b);
   u32x4 o;
 #pragma unroll
-  for (int e = 0; e < 4; ++e)
-    o[e] = (u32)__builtin_amdgcn_update_dpp((int)x[e], (int)y[e], 0x128, 0xf,
-                                            HI ? 0xc : 0x3, false);
+  for (int e = 0; e < 4; ++e) o[e] = ::other8<HI>(x[e], y[e]);
   return __builtin_bit_cast(s16x8, o);
 }
 

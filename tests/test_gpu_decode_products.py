@@ -194,6 +194,17 @@ def test_few_rows_past_4_gib(m):
     assert not bool(y[:, :-1024].any())
 
 
+@pytest.mark.parametrize("bits,m,n,k,g", [
+    (4, 2, 8191, 2048, 128), (4, 16, 8194, 2048, 128), (4, 9, 7290, 2304, 128),
+    (4, 5, 4110, 4096, 128), (8, 3, 4095, 2048, 128), (8, 12, 4098, 2048, 64),
+    (8, 16, 3650, 2304, 128), (8, 7, 2050, 4096, 64), (8, 4, 3300, 2688, 64)])
+def test_few_rows_by_whole_lines(bits, m, n, k, g):
+    """From 8 MiB of weights on, and just below: both pieces of a line, columns
+    that end inside an eight, waves with a part of their chunks."""
+    torch.manual_seed(n)
+    check(bits, m, n, k, g)
+
+
 @pytest.mark.parametrize("m,n,k,g,bits", [
     (17, 2048, 4096, 64, 4), (48, 4096, 14336, 128, 4), (33, 4104, 2048, 64, 8),
     (20, 8192, 4096, 128, 8), (48, 16384, 2048, 128, 4), (48, 512, 512, 64, 4),
