@@ -22,9 +22,12 @@
 //   n 6144, k 4096, norm             6.6 /  6.4 /  5.8
 //   n 4096, k 4096, residual         5.2 /      /  4.6
 //   n 2048, k 8192                   6.2 /  5.5 /  4.9
-//   n 32000, k 4096                 33.3 / 27.6 / 27.0
-//   n 16384, k 2048, norm and gate       /  9.7 /  9.1
+//   n 32000, k 4096                 33.3 / 27.6 / 23.9
+//   n 16384, k 2048, norm and gate       /  9.7 /  8.5
 //   n 2048, k 8192                   8.0 /  7.1 /  6.3
+// 8 bits, where a load took 16 of every 32 bytes and each line was asked for twice:
+// 26.1 for n 32000, 9.3 for n 16384, 24.6 for n 28672, k 4096, norm and gate (21.7;
+// the loads as they were, but by way of the caches 22.8).
 // (a launch that only reads: 10.0 for n 28672, k 4096.)  Eight rows ahead: 15.4;
 // 1024 workgroups: 14.8 (n 28672).
 #include "dq_frag.h"
@@ -62,6 +65,16 @@ __device__ __forceinline__ float sum4(float a, float b, float c, float d) {
   LFMQ_ADD(0x140);                       // sixteen, mirrored
 #undef LFMQ_ADD
   return v;
+}
+
+// the lower four of eight lanes a, the upper ones b
+__device__ __forceinline__ u32 own16(u32 a, u32 b) {
+  return (u32)__builtin_amdgcn_update_dpp((int)a, (int)b, 0xE4, 0xf, 0xa, false);
+}
+// the same of the lane that mirrors this one in eight
+__device__ __forceinline__ u32 mirrored16(u32 a, u32 b) {
+  const int lo = __builtin_amdgcn_update_dpp((int)a, (int)a, 0x141, 0xf, 0x5, false);
+  return (u32)__builtin_amdgcn_update_dpp(lo, (int)b, 0x141, 0xf, 0xa, false);
 }
 
 // block (64, KW, CW): KW waves along k, CW groups of rows at a time
@@ -116,7 +129,12 @@ __global__ __launch_bounds__(MOST * 64, 4) void dq_row_kernel(Row W) {
   // row j of group g, inside the workgroup's: gate, gate, up, up
   auto column = [&](int g, int j) { return g * TC + (GATE ? j & 1 : j); };
   const u32 pitch = k * BITS / 8;
-  const u32 byte = kw * 256 * BITS + lane * (BITS * 4);
+  // 8 bits: a load takes whole lines of 128 bytes, by eight lanes; a lane has 16 of
+  // its own 32 bytes and 16 of those of the lane that mirrors it
+  const int l7 = lane & 7;
+  const u32 byte = kw * 256 * BITS + (BITS == 4 ? lane * 16 : lane / 8 * 256);
+  const u32 at[2] = {BITS == 4 ? 0u : (l7 < 4 ? 2 * l7 : 15 - 2 * l7) * 16u,
+                     128 + (l7 < 4 ? 7 - 2 * l7 : 2 * l7 - 8) * 16u};
   u32x4 w[AHEAD][WB];
   // (past the last group nothing is read, but the load is there: where loads of
   // a loop depend on conditions the compiler waits for all of them)
@@ -126,7 +144,7 @@ __global__ __launch_bounds__(MOST * 64, 4) void dq_row_kernel(Row W) {
     const auto rsrc = make_rsrc_uniform(A.w + row * pitch, g < ng ? pitch : 0);
 #pragma unroll
     for (int i = 0; i < WB; ++i)
-      b[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, byte + i * 16, 0, 2);
+      b[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, byte + at[i], 0, 2);
   };
 #pragma unroll
   for (int j = 0; j < AHEAD; ++j) fetch(cw, j, w[j]);
@@ -187,7 +205,8 @@ __global__ __launch_bounds__(MOST * 64, 4) void dq_row_kernel(Row W) {
         for (int b = 0; b < WB; ++b)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const u32 d = w[j][b][e];
+            const u32 d = b == 0 ? own16(w[j][0][e], w[j][WB - 1][e])
+                                 : mirrored16(w[j][0][e], w[j][WB - 1][e]);
             const float* x = xf + (b * 16 + e * 4) % (BITS == 8 ? 32 : 1);
             c0 = fmaf((float)(d & 0xFFu), x[0], c0);
             c1 = fmaf((float)((d >> 8) & 0xFFu), x[1], c1);
