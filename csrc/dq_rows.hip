@@ -319,7 +319,8 @@ __global__ __launch_bounds__(256) void dq_rows_sum(DqArgs A) {
 // A whole row of the result a workgroup, and what DqRowEnd says of it: the sum of
 // parts, the residual and the norm in one launch.  V pieces of four columns a
 // thread, B parts of them on their way at once.  Bound as dq_rows_sum by launch
-// and latency: 48 rows of 4096, six parts, 4.7 us (dq_rows_sum 4.8, and the norm
+// and latency: 77 rows of 2048 with the norm 4.0 us (dq_rows_sum 3.9, the norm
+// alone 3.2); 48 rows of 4096, six parts, 4.7 us (dq_rows_sum 4.8, and the norm
 // of its rows 5.0, or in the next product the squares of every workgroup's rows,
 // n 6144, k 4096 22 us where the product without is 10.5).
 constexpr int ROW_TPB = 512;

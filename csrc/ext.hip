@@ -491,6 +491,37 @@ bool rows_end(int n, const c10::optional<torch::Tensor>& bias,
          (uintptr_t)w % 8 == 0;
 }
 
+// y = x W^T (+ bias) in bf16, then {rmsnorm(y + residual) w, y + residual}: in the
+// launch that adds up the product's parts where it has some
+std::vector<torch::Tensor> dq_linear_norm(
+    torch::Tensor x, torch::Tensor qweight, torch::Tensor scales,
+    torch::Tensor qzeros, long bits, long g, c10::optional<torch::Tensor> bias,
+    torch::Tensor residual, torch::Tensor w, double eps) {
+  check_t(residual, torch::kBFloat16, "residual");
+  check_t(w, torch::kBFloat16, "w");
+  const int m = (int)x.size(0), n = (int)qweight.size(0);
+  TORCH_CHECK(residual.numel() == (long)m * n && w.numel() == n,
+              "a residual and a weight for each column of the result");
+  auto h = torch::empty({m, n}, x.options());
+  RowWays ways{};
+  DqRowEnd end{};
+  bool ended = false;
+  end.normed = (unsigned short*)h.data_ptr();
+  end.to = (const unsigned short*)residual.data_ptr();
+  end.w = (const unsigned short*)w.data_ptr();
+  end.eps = (float)eps;
+  ways.ended = &ended;
+  if (rows_end(n, bias, residual, w.data_ptr())) ways.end = &end;
+  auto y = linear(x, qweight, scales, qzeros, bits, g, bias, c10::nullopt, -1.0,
+                  0, ways);
+  if (ended) return {h, y};
+  auto sum = torch::empty_like(y);
+  CHECK_HIP(lfmq_rmsnorm(y.data_ptr(), residual.data_ptr(), w.data_ptr(),
+                         h.data_ptr(), sum.data_ptr(), m, n, (float)eps,
+                         stream()));
+  return {h, sum};
+}
+
 // Rows of x times their factors (17 to 48 rows); eps >= 0: also row_scale of the
 // result, with the sum of the product's parts where it has some
 std::vector<torch::Tensor> dq_linear_scaled(
@@ -1288,6 +1319,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("row_scale", &row_scale, "1 / root mean square of rows");
   m.def("dq_linear_scaled", &dq_linear_scaled,
         "dq_linear of rows times factors, and the result's own");
+  m.def("dq_linear_norm", &dq_linear_norm,
+        "dq_linear, the residual and the next norm");
   m.def("dq_gateup_scaled", &dq_gateup_scaled,
         "dq_gemv_gateup of rows times factors");
   m.def("rmsnorm", &rmsnorm, "fused rmsnorm");

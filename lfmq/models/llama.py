@@ -79,6 +79,16 @@ class RMSNorm(nn.Module):
         return F.rmsnorm(x, self.weight, self.eps, residual)
 
 
+def linear_norm(p: nn.Module, x, residual, norm: RMSNorm):
+    """F.rmsnorm_residual(p(x), residual) of the norm, and what it norms: in the
+    product's own launches where p is a packed layer as it is.  (us, 77 rows of
+    2048: the sum of parts 3.9 and the norm 3.2, both in one 4.0)"""
+    if x.is_cuda and type(p) is QLinear and not hasattr(p, "perm") and \
+            not hooked(p):
+        return F.dq_linear_norm(x, p, residual, norm.weight, norm.eps)
+    return F.rmsnorm_residual(p(x), residual, norm.weight, norm.eps)
+
+
 class LlamaAttention(nn.Module):
     def __init__(self, cfg: LlamaConfig, dtype):
         super().__init__()
@@ -95,6 +105,11 @@ class LlamaAttention(nn.Module):
     def forward(self, x: torch.Tensor, cache_k: torch.Tensor,
                 cache_v: torch.Tensor, positions: torch.Tensor,
                 seq_len_after: int) -> torch.Tensor:
+        return self.o_proj(self.attend(x, cache_k, cache_v, positions,
+                                       seq_len_after))
+
+    def attend(self, x, cache_k, cache_v, positions, seq_len_after):
+        """What o_proj projects."""
         b, s, _ = x.shape
         hq, hkv, d = self.n_heads, self.n_kv_heads, self.head_dim
         qkv = self.qkv_proj(x)
@@ -121,7 +136,7 @@ class LlamaAttention(nn.Module):
                 else:
                     o = self._chunk_attn(qh, cache_k, cache_v, pos0, seq_len_after)
                 o = o.transpose(1, 2).reshape(b, s, hq * d)
-            return self.o_proj(o)
+            return o
         q, k, v = qkv.split([hq * d, hkv * d, hkv * d], dim=-1)
         q = q.reshape(b, s, hq, d)
         k = k.reshape(b, s, hkv, d)
@@ -136,8 +151,17 @@ class LlamaAttention(nn.Module):
                                causal=True, scale=self.scale)
         else:  # chunked continuation: attend to full cache, causal inside chunk
             o = self._chunk_attn(qh, cache_k, cache_v, pos0, seq_len_after)
-        o = o.transpose(1, 2).reshape(b, s, hq * d)
-        return self.o_proj(o)
+        return o.transpose(1, 2).reshape(b, s, hq * d)
+
+    def norm_after(self, x, cache_k, cache_v, positions, seq_len_after,
+                   residual, norm):
+        """F.rmsnorm_residual of the result, and what it norms."""
+        if type(self).forward is LlamaAttention.forward and not hooked(self):
+            return linear_norm(self.o_proj, self.attend(
+                x, cache_k, cache_v, positions, seq_len_after), residual, norm)
+        return F.rmsnorm_residual(
+            self(x, cache_k, cache_v, positions, seq_len_after), residual,
+            norm.weight, norm.eps)
 
     def forward_decode_graph(self, x, cache_k, cache_v, state, max_seq,
                              tickets=None):
@@ -190,6 +214,10 @@ class LlamaMLP(nn.Module):
         self.inter = cfg.intermediate_size
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        return self.down_proj(self.gated(x))
+
+    def gated(self, x: torch.Tensor) -> torch.Tensor:
+        """What down_proj projects."""
         gp = self.gate_up_proj
         m = x.numel() // x.shape[-1]
         if (x.is_cuda and isinstance(gp, QLinear)
@@ -197,11 +225,15 @@ class LlamaMLP(nn.Module):
                 and not hasattr(gp, "perm")
                 and (m <= 4 or (gp.bias is None and rows_fused(gp)))):
             # fused gate_up product + silu·mul epilogue (no separate pass)
-            h = F.dq_gemv_gateup(x, gp.qweight, gp.scales, gp.qzeros,
-                                 gp.bits, gp.group_size)
-            return self.down_proj(h)
-        gu = gp(x)
-        return self.down_proj(F.silu_mul_gateup(gu, self.inter))
+            return F.dq_gemv_gateup(x, gp.qweight, gp.scales, gp.qzeros,
+                                    gp.bits, gp.group_size)
+        return F.silu_mul_gateup(gp(x), self.inter)
+
+    def norm_after(self, x, residual, norm):
+        """F.rmsnorm_residual of the result, and what it norms."""
+        if type(self).forward is LlamaMLP.forward and not hooked(self):
+            return linear_norm(self.down_proj, self.gated(x), residual, norm)
+        return F.rmsnorm_residual(self(x), residual, norm.weight, norm.eps)
 
 
 class LlamaDecoderLayer(nn.Module):
@@ -224,12 +256,20 @@ class LlamaDecoderLayer(nn.Module):
             h, residual = F.rmsnorm_residual(x, residual,
                                              self.input_layernorm.weight,
                                              self.input_layernorm.eps)
-        h = self.self_attn(h, cache_k, cache_v, positions, seq_len_after)
-        h, residual = F.rmsnorm_residual(h, residual,
-                                         self.post_attention_layernorm.weight,
-                                         self.post_attention_layernorm.eps)
+        h, residual = self.self_attn.norm_after(
+            h, cache_k, cache_v, positions, seq_len_after, residual,
+            self.post_attention_layernorm)
         h = self.mlp(h)
         return h, residual
+
+    def forward_normed(self, h, residual, cache_k, cache_v, positions,
+                       seq_len_after, norm):
+        """forward between norms: of the layer's normed input and what that
+        was to the same of the next layer, whose norm it is."""
+        h, residual = self.self_attn.norm_after(
+            h, cache_k, cache_v, positions, seq_len_after, residual,
+            self.post_attention_layernorm)
+        return self.mlp.norm_after(h, residual, norm)
 
     def forward_decode_step(self, x, cache_k, cache_v, state, max_seq,
                             residual=None, tickets=None):
@@ -327,19 +367,36 @@ class LlamaForCausalLM(nn.Module):
         b, s = input_ids.shape
         pos0 = cache.seq_len
         if positions is None:
-            positions = torch.arange(pos0, pos0 + s, device=input_ids.device)
+            positions = torch.arange(
+                pos0, pos0 + s, device=input_ids.device,
+                dtype=torch.int32 if input_ids.is_cuda else None)
         if positions.is_cuda:
             positions = positions.to(torch.int32)    # once, not in every layer
         seq_after = pos0 + s
         x = self.embed_tokens(input_ids)
-        residual = None
-        for i, layer in enumerate(self.layers):
-            x, residual = layer(x, cache.k[i], cache.v[i], positions,
-                                seq_after, residual)
-        x = self.norm(x, residual=residual)
+        if self._norms_ride(x):
+            norms = [l.input_layernorm for l in self.layers] + [self.norm]
+            x, residual = norms[0](x), x
+            for i, layer in enumerate(self.layers):
+                x, residual = layer.forward_normed(
+                    x, residual, cache.k[i], cache.v[i], positions, seq_after,
+                    norms[i + 1])
+        else:
+            residual = None
+            for i, layer in enumerate(self.layers):
+                x, residual = layer(x, cache.k[i], cache.v[i], positions,
+                                    seq_after, residual)
+            x = self.norm(x, residual=residual)
         logits = self.lm_head(x)
         cache.advance(s)
         return logits
+
+    def _norms_ride(self, x) -> bool:
+        """Whether a layer's last product may take the next norm with it."""
+        return x.is_cuda and len(self.layers) > 0 and all(
+            type(l).forward is LlamaDecoderLayer.forward for l in self.layers
+        ) and type(self.norm).forward is RMSNorm.forward and not hooked(
+            self.norm, *self.layers)
 
     def _engine_for(self, cache, batch: int) -> bool:
         """Build/bind the persistent decode engine for this cache (lazy;

@@ -268,10 +268,9 @@ class MixtralDecoderLayer(nn.Module):
             h, residual = F.rmsnorm_residual(x, residual,
                                              self.input_layernorm.weight,
                                              self.input_layernorm.eps)
-        h = self.self_attn(h, cache_k, cache_v, positions, seq_len_after)
-        h, residual = F.rmsnorm_residual(h, residual,
-                                         self.post_attention_layernorm.weight,
-                                         self.post_attention_layernorm.eps)
+        h, residual = self.self_attn.norm_after(
+            h, cache_k, cache_v, positions, seq_len_after, residual,
+            self.post_attention_layernorm)
         h = self.moe(h)
         return h, residual
 
@@ -329,7 +328,9 @@ class MixtralForCausalLM(nn.Module):
         b, s = input_ids.shape
         pos0 = cache.seq_len
         if positions is None:
-            positions = torch.arange(pos0, pos0 + s, device=input_ids.device)
+            positions = torch.arange(
+                pos0, pos0 + s, device=input_ids.device,
+                dtype=torch.int32 if input_ids.is_cuda else None)
         if positions.is_cuda:
             positions = positions.to(torch.int32)    # once, not in every layer
         x = self.embed_tokens(input_ids)

@@ -107,6 +107,18 @@ def dq_linear_scaled(x: torch.Tensor, scale: Optional[torch.Tensor], p,
     return (y, *own) if own else y
 
 
+def dq_linear_norm(x: torch.Tensor, p, residual: torch.Tensor,
+                   weight: torch.Tensor, eps: float):
+    """GPU-only rmsnorm_residual(y, residual, weight, eps) of the product y of
+    the packed layer p, added up, normed and stored by one launch where k was
+    split."""
+    n = residual.shape[-1]
+    h, s = hip_ext().dq_linear_norm(
+        x.reshape(-1, x.shape[-1]), p.qweight, p.scales, p.qzeros, p.bits,
+        p.group_size, p.bias, residual.reshape(-1, n).contiguous(), weight, eps)
+    return _guard(h, "dq_linear").view(residual.shape), s.view(residual.shape)
+
+
 def dq_gateup_scaled(x: torch.Tensor, scale: torch.Tensor, p) -> torch.Tensor:
     """GPU-only dq_gemv_gateup of the packed layer p for 17 to 48 rows, which
     are multiplied by scale."""

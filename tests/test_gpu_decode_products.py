@@ -232,3 +232,28 @@ def test_rows_times_their_factors(m, n, k, g, bits):
         assert float((out.double() / own - 1).abs().max()) < 1e-5
     if n % 2 == 0:
         close(ext().dq_gateup_scaled(x, scale, *p, bits, g), gated(rms), 1e-2)
+
+
+@pytest.mark.parametrize("m,n,k,g,bits", [
+    (77, 2048, 8192, 64, 8), (40, 4096, 14336, 128, 4), (64, 4104, 4096, 64, 4),
+    (50, 8192, 4096, 128, 8), (33, 16384, 2048, 128, 4), (100, 1032, 4096, 128, 4),
+    (20, 2044, 8192, 64, 4), (60, 2046, 2048, 64, 8), (3, 2048, 2048, 128, 4),
+    (300, 2048, 2048, 64, 4)])
+@pytest.mark.parametrize("shift", [0, 2])
+def test_norm_after_a_product(m, n, k, g, bits, shift):
+    """The sum of parts with residual and norm (rows of up to 2048, 4096, 8192 and
+    16384 columns), a product in one piece, and rows that no workgroup holds or
+    that lie off 8 bytes: as the product and the norm apart."""
+    torch.manual_seed(n + m)
+    p, w = matrix(bits, n, k, g)
+    x = torch.randn(m, k, device=DEV).to(BF)
+    bias = torch.randn(n, device=DEV).to(BF)
+    to = torch.randn(m * n + shift, device=DEV).to(BF)[shift:].view(m, n)
+    weight = torch.randn(n, device=DEV).to(BF)
+    h, s = ext().dq_linear_norm(x, *p, bits, g, bias, to, weight, 1e-5)
+    y = ext().dq_linear(x, *p, bits, g, bias, None, -1.0, 0)
+    close(y, x.double() @ w.t() + bias.double())
+    assert torch.equal(s, (y.float() + to.float()).to(BF))
+    want = normed(y.double() + to.double(), 1e-5) * weight.double()
+    # its own rounding, and a sum of n squares in fp32
+    assert float(((h.double() - want).abs() / (want.abs() + 1e-6)).max()) < 4.1e-3
