@@ -266,10 +266,28 @@ class LlamaDecoderLayer(nn.Module):
                        seq_len_after, norm):
         """forward between norms: of the layer's normed input and what that
         was to the same of the next layer, whose norm it is."""
+        att, mlp, post = self.self_attn, self.mlp, self.post_attention_layernorm
+        products = att.qkv_proj, att.o_proj, mlp.gate_up_proj, mlp.down_proj
+        if h.shape[1] > 1 and self._in_one_call(products):
+            return F.prompt_layer(h, residual, cache_k, cache_v, positions,
+                                  seq_len_after - h.shape[1], att.n_heads,
+                                  att.cfg.rope_theta, att.scale, products,
+                                  post, norm)
         h, residual = self.self_attn.norm_after(
             h, cache_k, cache_v, positions, seq_len_after, residual,
             self.post_attention_layernorm)
         return self.mlp.norm_after(h, residual, norm)
+
+    def _in_one_call(self, products) -> bool:
+        att, mlp = self.self_attn, self.mlp
+        return (F.USE_FLASH_PREFILL and att.head_dim == 128
+                and not F._NANCHECK
+                and all(type(p) is QLinear and "perm" not in p._buffers
+                        and "perm" not in p.__dict__ for p in products)
+                and products[2].bias is None and rows_fused(products[2])
+                and type(att).forward is LlamaAttention.forward
+                and type(mlp).forward is LlamaMLP.forward
+                and not hooked(att, mlp, *products))
 
     def forward_decode_step(self, x, cache_k, cache_v, state, max_seq,
                             residual=None, tickets=None):

@@ -243,6 +243,23 @@ def attn_prefill_fused(q: torch.Tensor, k_cache: torch.Tensor,
 USE_FLASH_PREFILL = os.environ.get("LFMQ_FLASH_PREFILL", "1") == "1"
 
 
+def prompt_layer(h, residual, k_cache, v_cache, positions, pos0: int, hq: int,
+                 theta: float, scale: float, products, post_norm, next_norm):
+    """GPU-only layer between norms for a prompt, in one call: products are the
+    packed layers qkv, o, gate and up (no bias), down; heads of 128."""
+    packed, forms = [], []
+    for p in products:
+        b = p._buffers
+        packed += (b["qweight"], b["scales"], b["qzeros"])
+        forms += (p.bits, p.group_size)
+    qkv, o, _, down = products
+    return hip_ext().prompt_layer(
+        h, residual, k_cache, v_cache, positions,
+        _inv_freq(k_cache.shape[-1], theta, h.device), hq, pos0, scale, packed,
+        forms, [qkv.bias, o.bias, down.bias], post_norm.weight, post_norm.eps,
+        next_norm.weight, next_norm.eps)
+
+
 def qkv_rope_append(qkv: torch.Tensor, k_cache: torch.Tensor,
                     v_cache: torch.Tensor, positions: torch.Tensor,
                     pos0: int, hq: int, theta: float = 500000.0) -> torch.Tensor:

@@ -285,3 +285,39 @@ def test_decode_matches_prefill_gpu_d128():
     outs2 = [qm(more[:, t:t + 1], cache2).float() for t in range(40)]
     rel2 = (cont - torch.cat(outs2, dim=1)).abs().max() / cont.abs().max()
     assert rel2 < 0.05, f"continuation mismatch rel={float(rel2)}"
+
+
+@pytest.mark.parametrize("b,s,past,bits,gs,bias", [
+    (1, 2, 0, 4, 64, False), (1, 77, 5, 8, 64, False), (3, 40, 0, 4, 128, True),
+    (2, 150, 33, 4, 64, False)])
+def test_prompt_layer_in_one_call(b, s, past, bits, gs, bias, monkeypatch):
+    """A layer's kernels called from one place are those called one by one:
+    the same logits and cache; a hook on a layer is still called."""
+    from lfmq.models.llama import LlamaDecoderLayer
+    cfg = LlamaConfig(vocab_size=512, hidden_size=512, intermediate_size=1024,
+                      n_layers=2, n_heads=4, n_kv_heads=2, head_dim=128,
+                      max_seq=256)
+    m = lfmq.quantize(lfmq.build_model(cfg, seed=7), lfmq.QuantConfig(
+        scheme="rtn", bits=bits, group_size=gs)).to(DEV)
+    if bias:
+        for layer in m.layers:
+            for p in (layer.self_attn.qkv_proj, layer.mlp.down_proj):
+                p.bias = torch.randn(p.out_features, device=DEV).bfloat16()
+    ids = torch.randint(0, 512, (b, past + s), device=DEV)
+    out, calls = [], []
+    for way in ("one call", "one by one", "watched"):
+        if way == "one by one":
+            monkeypatch.setattr(LlamaDecoderLayer, "_in_one_call",
+                                lambda *a: False)
+        if way == "watched":
+            monkeypatch.undo()
+            m.layers[1].mlp.register_forward_hook(lambda *a: calls.append(1))
+        c = m.make_cache(b, 256)
+        with torch.no_grad():
+            if past:
+                m(ids[:, :past], c)
+            out.append((m(ids[:, past:], c), c.k_all.clone(), c.v_all.clone()))
+    assert all(torch.equal(x, y) for x, y in zip(*out[:2]))
+    assert calls
+    a, z = out[0][0].float(), out[2][0].float()
+    assert float((a - z).norm() / z.norm()) < 0.02   # 2 layers of 2^-9 roundings
