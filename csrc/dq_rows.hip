@@ -38,7 +38,8 @@ __device__ __forceinline__ float epilogue(const DqArgs& A, float v, int row,
   return v;
 }
 
-template <int BITS, int MT, int NT, int NW, int KC, DqMode MODE>
+// SCALED: whole sums of rows of x times A.row_scale
+template <int BITS, int MT, int NT, int NW, int KC, DqMode MODE, bool SCALED>
 __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(DqArgs A) {
   constexpr int TPB = NW * 64;
   constexpr int J = KC / 32;                 // products a chunk
@@ -198,6 +199,8 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(DqArgs A) {
         red[((u32)wave * BM + t * 16 + l4 * 4 + r) * LD + nt * 16 + l15] =
             acc[t][nt][r];
   float* rs = red + NW * BM * LD;            // [BM], after [NW][BM]
+  if (SCALED && threadIdx.x < BM)
+    rs[threadIdx.x] = A.row_scale[row0 + min((int)threadIdx.x, rows - 1)];
   if (rms) {
 #pragma unroll
     for (int t = 0; t < MT; ++t)
@@ -229,18 +232,13 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(DqArgs A) {
       return v;
     };
     f32x4 v = sum(c4);
-    // of parts: after their sum
-    const float scale =
-        rms ? rs[row]
-            : (MODE != SLOTS && A.row_scale != nullptr && gridDim.y == 1
-                   ? A.row_scale[gr]
-                   : 1.f);
+    const float scale = SCALED || rms ? rs[row] : 1.f;
     if constexpr (MODE == GLU) {
       const f32x4 up = sum(HT * 16 + c4);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         v[e] = silu_mul_f(v[e] * scale, up[e] * scale);
-    } else if (MODE == DENSE) {
+    } else if (SCALED || rms) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] *= scale;
     }
@@ -272,7 +270,7 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(DqArgs A) {
 // the sums, y half as wide.  Bound by the launch and one latency: all parts on
 // their way at once, no division for a place (48 x 4096: 5.1 us with a grid over
 // all elements and parts four by four, 4.8 so).
-template <bool GLU>
+template <bool GLU, bool SCALED>
 __global__ __launch_bounds__(256) void dq_rows_sum(DqArgs A) {
   const u64 part = (u64)A.m * A.n;
   const int nout = GLU ? A.n / 2 : A.n;
@@ -286,10 +284,11 @@ __global__ __launch_bounds__(256) void dq_rows_sum(DqArgs A) {
       if constexpr (!GLU)
 #pragma unroll
         for (int e = 0; e < 4; ++e) add[e] = epilogue(A, 0.f, row, col + e);
-      const float scale = A.row_scale != nullptr ? A.row_scale[row] : 1.f;
-      f32x4 v = sum_of_parts(p, part, A.splits) * scale;
+      f32x4 v = sum_of_parts(p, part, A.splits);
+      if constexpr (SCALED) v *= A.row_scale[row];
       if constexpr (GLU) {
-        const f32x4 up = sum_of_parts(p + nout, part, A.splits) * scale;
+        f32x4 up = sum_of_parts(p + nout, part, A.splits);
+        if constexpr (SCALED) up *= A.row_scale[row];
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = silu_mul_f(v[e], up[e]);
       } else if (A.bias != nullptr || A.resid != nullptr) {
@@ -309,10 +308,12 @@ __global__ __launch_bounds__(256) void dq_rows_sum(DqArgs A) {
       v += A.part[s * part + (u64)row * A.n + col];
       if (GLU) up += A.part[s * part + (u64)row * A.n + nout + col];
     }
-    const float scale = A.row_scale != nullptr ? A.row_scale[row] : 1.f;
-    v *= scale;
+    if constexpr (SCALED) {
+      v *= A.row_scale[row];
+      up *= A.row_scale[row];
+    }
     A.y[id] = (unsigned short)f32_to_bf16_bits_rne(
-        GLU ? silu_mul_f(v, up * scale) : epilogue(A, v, row, col));
+        GLU ? silu_mul_f(v, up) : epilogue(A, v, row, col));
   }
 }
 
@@ -431,10 +432,12 @@ void sum_parts(const DqArgs& A, bool glu, hipStream_t stream) {
       nout % 4 == 0
           ? dim3(ceil_div_u32(nout, 1024), min(A.m, 65535))
           : dim3((u32)min(((u64)A.m * nout + 255) / 256, (u64)1024));
-  if (glu)
-    hipLaunchKernelGGL(dq_rows_sum<true>, grid, dim3(256), 0, stream, A);
-  else
-    hipLaunchKernelGGL(dq_rows_sum<false>, grid, dim3(256), 0, stream, A);
+  const bool scaled = A.row_scale != nullptr;
+  const auto kernel = glu ? (scaled ? dq_rows_sum<true, true>
+                                    : dq_rows_sum<true, false>)
+                          : (scaled ? dq_rows_sum<false, true>
+                                    : dq_rows_sum<false, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, A);
 }
 
 int chunk_of(int g) { return g % 128 == 0 ? 128 : (g % 64 == 0 ? 64 : 32); }
@@ -446,8 +449,12 @@ size_t meta_bytes(int k, int g, int splits, int nt) {
   return ((size_t)chunks * kc / g + 2) * nt * 16 * 4;
 }
 
-template <int BITS, int MT, int NT, int NW, int KC, DqMode MODE = DENSE>
+template <int BITS, int MT, int NT, int NW, int KC, DqMode MODE = DENSE,
+          bool SCALED = false>
 hipError_t go(const DqArgs& A, int tiles, hipStream_t stream) {
+  if constexpr (!SCALED && MT > 1 && MODE != SLOTS)
+    if (A.row_scale != nullptr && A.splits == 1)
+      return go<BITS, MT, NT, NW, KC, MODE, true>(A, tiles, stream);
   const size_t sums =
       ((size_t)NW * MT * 16 * (NT * 16 + 4) + (NW + 1) * MT * 16) * 4;
   const size_t lds = max(sums, meta_bytes(A.k, A.g, A.splits, NT));
@@ -455,14 +462,14 @@ hipError_t go(const DqArgs& A, int tiles, hipStream_t stream) {
   static size_t set = 64 * 1024;
   if (lds > set) {
     LFMQ_CHECK_HIP(hipFuncSetAttribute(
-        (const void*)dq_rows_kernel<BITS, MT, NT, NW, KC, MODE>,
+        (const void*)dq_rows_kernel<BITS, MT, NT, NW, KC, MODE, SCALED>,
         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     set = 160 * 1024;
   }
   const int cols = MODE == GLU ? NT * 8 : NT * 16;
   const dim3 grid(ceil_div_u32(MODE == GLU ? A.n / 2 : A.n, cols), A.splits,
                   tiles);
-  hipLaunchKernelGGL((dq_rows_kernel<BITS, MT, NT, NW, KC, MODE>), grid, dim3(NW * 64),
+  hipLaunchKernelGGL((dq_rows_kernel<BITS, MT, NT, NW, KC, MODE, SCALED>), grid, dim3(NW * 64),
                      lds, stream, A);
   if (A.splits > 1) sum_parts(A, false, stream);
   return hipGetLastError();

@@ -39,7 +39,8 @@ struct Lds {
   static constexpr int BYTES = ALL > OUT ? ALL : OUT;
 };
 
-template <int BITS, int KC, int MT, int D, DqMode MODE>
+// SCALED: rows of x times A.row_scale, whole sums
+template <int BITS, int KC, int MT, int D, DqMode MODE, bool SCALED>
 __global__ __launch_bounds__(TPB, 2) void dq_short_kernel(DqArgs A, int mb,
                                                           int step) {
   typedef Lds<BITS, KC, MT, D> L;
@@ -272,6 +273,17 @@ __global__ __launch_bounds__(TPB, 2) void dq_short_kernel(DqArgs A, int mb,
       }
     return;
   }
+  if constexpr (SCALED) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float scale =
+            A.row_scale[row0 + min(t * 16 + l4 * 4 + r, rows - 1)];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[t][nt][r] *= scale;
+      }
+  }
   // through LDS, so that rows are written in 16-byte pieces
   constexpr int BO = MODE == GLU ? BN / 2 : BN, LD = BO + 8;
   const int nout = MODE == GLU ? half : A.n;
@@ -288,13 +300,8 @@ __global__ __launch_bounds__(TPB, 2) void dq_short_kernel(DqArgs A, int mb,
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = t * 16 + l4 * 4 + r;
-        // (of up to 48 rows)
-        const float scale = MT <= 3 && A.row_scale != nullptr && row < rows
-                                ? A.row_scale[row0 + row]
-                                : 1.f;
-        float v = MODE == GLU
-                      ? silu_mul_f(acc[t][0][r] * scale, acc[t][1][r] * scale)
-                      : acc[t][nt][r] * scale + bias;
+        float v = MODE == GLU ? silu_mul_f(acc[t][0][r], acc[t][1][r])
+                              : acc[t][nt][r] + bias;
         if (MODE == DENSE && A.resid != nullptr && row < rows && n0 + c < A.n)
           v += bf16_bits_to_f32(A.resid[(u64)(row0 + row) * A.n + n0 + c]);
         out[(t * 16 + l4 * 4 + r) * LD + c] =
@@ -327,21 +334,26 @@ constexpr int depth() {
   return d < m ? m : (d > 6 ? 6 : d);
 }
 
-template <int BITS, int KC, int MT, DqMode MODE>
+template <int BITS, int KC, int MT, DqMode MODE, bool SCALED = false>
 hipError_t go(const DqArgs& A, int mb, int step, hipStream_t stream) {
+  // (17 to 48 rows)
+  if (!SCALED && A.row_scale != nullptr && A.splits == 1) {
+    if constexpr (MT <= 3) return go<BITS, KC, MT, MODE, true>(A, mb, step, stream);
+    return hipErrorInvalidValue;
+  }
   constexpr int D = depth<BITS, KC, MT>();
   constexpr int lds = Lds<BITS, KC, MT, D>::BYTES;
   static_assert(lds <= 160 * 1024, "");
   static bool set = false;
   if (!set && lds > 64 * 1024) {
     LFMQ_CHECK_HIP(hipFuncSetAttribute(
-        (const void*)dq_short_kernel<BITS, KC, MT, D, MODE>,
+        (const void*)dq_short_kernel<BITS, KC, MT, D, MODE, SCALED>,
         hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     set = true;
   }
   const u32 nb = MODE == GLU ? ceil_div_u32(A.n / 2, 64)
                              : ceil_div_u32(A.n, 128);
-  hipLaunchKernelGGL((dq_short_kernel<BITS, KC, MT, D, MODE>),
+  hipLaunchKernelGGL((dq_short_kernel<BITS, KC, MT, D, MODE, SCALED>),
                      dim3(mb * nb * A.splits), dim3(TPB), lds, stream, A, mb,
                      step);
   return hipGetLastError();
