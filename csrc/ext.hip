@@ -5,6 +5,7 @@
 #include <ATen/cuda/CUDAContext.h>
 #include <hip/hip_runtime.h>
 
+#include "dq_mid.h"
 #include "dq_short.h"
 
 hipError_t lfmq_pack(const void*, void*, long, int, int, hipStream_t);
@@ -295,6 +296,42 @@ bool short_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
          (uintptr_t)qweight.data_ptr() % 16 == 0;
 }
 
+// The product of 8 bits whose workgroups share k among eight waves (dq_mid): where
+// it is faster than dq_short, dq_rows, dq_tile and dq_block.  Of 437 random shapes of
+// 17 to 128 rows, 3 to 120 million weights, this takes 180, whose time before / now is
+// 1.24 in the mean and 0.95 to 1.65.  Long k
+// pays where the columns are few, so that parts of it fill the chip: n 4096, k 4096
+// 20.6 / 15.2 us at 96 rows, n 2048, k 8192 18.2 / 14.9 at 61; n 20480, k 4096 35.3 /
+// 39.2 at 50.  A gate has no parts: n 6144, k 8192 24.0 / 34.3 at 54.  Above 96 rows
+// there are two tiles of them, and many columns are read twice: n 28672, k 2048 34.2 /
+// 41.8 at 109, n 6144, k 8192 33.2 / 41.6 at 110; 16384 to 28672 columns leave a
+// third of the chip (n 20480, k 2560 24.6 / 27.5 at 40).  Few rows of few columns are dq_rows': n 4096, k 1024 6.4 / 7.7 at 36.
+bool mid_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
+              long bits, bool glu) {
+  if (bits != 8 || m <= 16 || m > 128 || n <= 0 || n % 8 ||
+      !tile_addresses(n, k, bits) || !lfmq_dq_tile_ok((int)k, (int)g) ||
+      (uintptr_t)qweight.data_ptr() % 16)
+    return false;
+  bool gains;
+  if (glu)
+    gains = k <= 3072 && (m <= 96 || n <= 8192) && (m <= 48 || n >= 4096) &&
+            (k <= 2048 || n <= 16384 || n >= 24576);
+  else if (m > 96 && n > (k <= 3072 ? 8192 : 3072))
+    gains = false;
+  else if (k <= 3072 && n > 16384 && n < 28672)
+    gains = m > 64 || (m <= 48 && k <= 2048);
+  else if (k <= 3072)
+    gains = m <= 48 ? n >= 5120 && (m > 24 || n * k >= 16l << 20)
+                    : n * k >= 3l << 20;
+  else if (n <= 6144)
+    gains = m > (g == 64 && k <= 8192 ? 48 : 64) && m <= 112 &&
+            (k <= 8192 || g == 64);
+  else
+    gains = m > 48 && k <= 4096 && n >= 10240 && n <= 16384;
+  return gains &&
+         lfmq_dq_mid_plan((int)m, (int)n, (int)k, (int)g, glu).mb > 0;
+}
+
 // What goes with whole rows of a product: a factor of x's rows, and what follows
 // rows of the result, which the sum of parts takes along if there is one.
 struct RowWays {
@@ -337,6 +374,39 @@ void dq_short(const torch::Tensor& x, const torch::Tensor& qweight,
   if (P.splits > 1)
     CHECK_HIP(lfmq_dq_rows_sum(part.data_ptr(), y.data_ptr(), bias, resid, m, n,
                                P.splits, glu, stream(), ways.scale,
+                               ways.ends()));
+}
+
+void dq_mid(const torch::Tensor& x, const torch::Tensor& qweight,
+            const torch::Tensor& scales, const torch::Tensor& qzeros,
+            const void* bias, const void* resid, torch::Tensor& y, long g,
+            bool glu, const RowWays& ways) {
+  const int m = (int)x.size(0), k = (int)x.size(1), n = (int)qweight.size(0);
+  const DqMidPlan P = lfmq_dq_mid_plan(m, n, k, (int)g, glu);
+  DqArgs A{};
+  torch::Tensor part;
+  if (P.splits > 1) {
+    part = torch::empty({(long)P.splits * m * n},
+                        x.options().dtype(torch::kFloat32));
+    A.part = part.data_ptr<float>();
+  }
+  A.w = (const char*)qweight.data_ptr();
+  A.scales = (const unsigned short*)scales.data_ptr();
+  A.zeros = (const u32*)qzeros.data_ptr();
+  A.x = (const unsigned short*)x.data_ptr();
+  A.y = (unsigned short*)y.data_ptr();
+  A.bias = (const unsigned short*)bias;
+  A.resid = (const unsigned short*)resid;
+  A.m = m;
+  A.n = n;
+  A.k = k;
+  A.g = (int)g;
+  A.splits = P.splits;
+  A.row_scale = ways.scale;
+  CHECK_HIP(lfmq_dq_mid(A, P, glu, stream()));
+  if (P.splits > 1)
+    CHECK_HIP(lfmq_dq_rows_sum(part.data_ptr(), y.data_ptr(), bias, resid, m, n,
+                               P.splits, false, stream(), ways.scale,
                                ways.ends()));
 }
 
@@ -398,9 +468,11 @@ torch::Tensor linear(torch::Tensor x, const torch::Tensor& qweight,
                        lfmq_dq_rows_ok(m, n, k, (int)g, rms);
   const bool block = rptr == nullptr && !scaled &&
                      block_rows(qweight, scales, m, n, k, g, bits, false);
+  const bool mid = cols_hint == 0 && !rms &&
+                   mid_rows(qweight, m, n, k, g, bits, false);
   const bool few = cols_hint == 0 && !rms && !(small && by_rows) &&
                    short_rows(qweight, m, n, k, g, bits, false, block);
-  TORCH_CHECK(!scaled || (m > 16 && m <= 48 && (by_rows || few)),
+  TORCH_CHECK(!scaled || (m > 16 && m <= 48 && (by_rows || few || mid)),
               "factors of rows are for 17 to 48 of them");
   if (m > 16) {
     TORCH_CHECK((by_rows || !rms) && (m <= 48 || rptr == nullptr),
@@ -427,6 +499,8 @@ torch::Tensor linear(torch::Tensor x, const torch::Tensor& qweight,
                            qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bptr,
                            rptr, m, n, k, (int)g, (int)bits, (float)rms_eps,
                            false, stream()));
+  } else if (mid) {
+    dq_mid(x, qweight, scales, qzeros, bptr, rptr, y, g, false, ways);
   } else if (few) {
     dq_short(x, qweight, scales, qzeros, bptr, rptr, y, g, bits, false,
              ways);
@@ -713,6 +787,11 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
   const bool large =
       tile && rms_eps < 0 && k >= 4096 && (long)n * k >= 24l << 20;
   const bool block = block_rows(qweight, scales, m, n, k, g, bits, true);
+  if (cols_hint == 0 && rms_eps < 0 && mid_rows(qweight, m, n, k, g, bits, true)) {
+    if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
+    dq_mid(x, qweight, scales, qzeros, nullptr, nullptr, y, g, true, {});
+    return y;
+  }
   if (cols_hint == 0 && rms_eps < 0 && n % 2 == 0 &&
       short_rows(qweight, m, n, k, g, bits, true, block)) {
     if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
@@ -793,7 +872,9 @@ torch::Tensor dq_gateup_scaled(torch::Tensor x, torch::Tensor scale,
   RowWays ways{factors(scale, m)};
   if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
   auto y = torch::empty({m, n / 2}, x.options());
-  if (short_rows(qweight, m, n, k, g, bits, true, false))
+  if (mid_rows(qweight, m, n, k, g, bits, true))
+    dq_mid(x, qweight, scales, qzeros, nullptr, nullptr, y, g, true, ways);
+  else if (short_rows(qweight, m, n, k, g, bits, true, false))
     dq_short(x, qweight, scales, qzeros, nullptr, nullptr, y, g, bits, true,
              ways);
   else

@@ -36,6 +36,7 @@ SOURCES = [
     "csrc/dq_tile.hip",
     "csrc/dq_block.hip",
     "csrc/dq_short.hip",
+    "csrc/dq_mid.hip",
     "csrc/hessian.hip",
     "csrc/gptq_block.hip",
     "csrc/chol_inverse.hip",

@@ -257,3 +257,35 @@ def test_norm_after_a_product(m, n, k, g, bits, shift):
     want = normed(y.double() + to.double(), 1e-5) * weight.double()
     # its own rounding, and a sum of n squares in fp32
     assert float(((h.double() - want).abs() / (want.abs() + 1e-6)).max()) < 4.1e-3
+
+
+@pytest.mark.parametrize("m,n,k,g", [
+    (17, 5120, 256, 128), (48, 8200, 2112, 64), (33, 32008, 192, 64),
+    (49, 3072, 1024, 64), (64, 2056, 2048, 128), (77, 16384, 2048, 64),
+    (81, 1544, 2688, 192), (96, 2048, 2048, 64), (97, 2048, 3072, 64),
+    (113, 2504, 2560, 256), (128, 8192, 1024, 128), (49, 2048, 8192, 64),
+    (96, 4104, 4224, 128), (112, 1536, 4096, 64), (65, 1032, 14336, 64),
+    (80, 10240, 4096, 128)])
+def test_eight_waves_along_k(m, n, k, g):
+    """8 bits, some tens of rows: 2 to 6 sixteens of rows and two tiles of them,
+    2 and 4 waves side by side, parts of k and none, groups that the waves do
+    not share evenly, columns that end inside a wave's; bias, residual, gate
+    and factors of rows."""
+    torch.manual_seed(n + m)
+    p, w = matrix(8, n, k, g)
+    x = torch.randn(m, k, device=DEV).to(BF)
+    x[0] = 0
+    bias = torch.randn(n, device=DEV).to(BF)
+    plain = x.double() @ w.t()
+    close(ext().dq_linear(x, *p, 8, g, bias, None, -1.0, 0),
+          plain + bias.double())
+    close(ext().dq_gemv_gateup(x, *p, 8, g, -1.0, 0), gated(plain), 1e-2)
+    if m <= 48:
+        resid = torch.randn(m, n, device=DEV).to(BF)
+        scale = torch.rand(m, device=DEV) + 0.5
+        close(ext().dq_linear(x, *p, 8, g, bias, resid, -1.0, 0),
+              plain + bias.double() + resid.double())
+        want = plain * scale.double().unsqueeze(1)
+        y, _ = ext().dq_linear_scaled(x, scale, *p, 8, g, None, resid, 1e-5)
+        close(y, want + resid.double())
+        close(ext().dq_gateup_scaled(x, scale, *p, 8, g), gated(want), 1e-2)
