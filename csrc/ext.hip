@@ -97,6 +97,9 @@ hipError_t lfmq_argmax_rows(const void*, void*, void*, void*, int, int,
                             hipStream_t);
 hipError_t lfmq_read_probe(const void*, void*, long, long, int, int, int,
                            hipStream_t);
+hipError_t lfmq_qkv_sum_rope_append(const void*, int, const void*, void*, void*,
+                                    void*, const void*, const void*, int, int,
+                                    int, int, int, int, int, hipStream_t);
 #include "dq_block.h"
 #include "engine_args.h"
 
@@ -338,6 +341,15 @@ struct RowWays {
   const float* scale = nullptr;
   const DqRowEnd* end = nullptr;
   bool* ended = nullptr;
+  // where the parts go that a launch of the caller's adds up (dq_mid, dq_short)
+  torch::Tensor* parts = nullptr;
+  int* count = nullptr;
+  bool keeps(const torch::Tensor& part, int splits) const {
+    if (parts == nullptr) return false;
+    *parts = part;
+    *count = splits;
+    return true;
+  }
   const DqRowEnd* ends() const {           // for a launch that sums parts
     if (end != nullptr) *ended = true;
     return end;
@@ -371,7 +383,7 @@ void dq_short(const torch::Tensor& x, const torch::Tensor& qweight,
   A.splits = P.splits;
   A.row_scale = ways.scale;
   CHECK_HIP(lfmq_dq_short(A, P, (int)bits, glu, stream()));
-  if (P.splits > 1)
+  if (P.splits > 1 && !ways.keeps(part, P.splits))
     CHECK_HIP(lfmq_dq_rows_sum(part.data_ptr(), y.data_ptr(), bias, resid, m, n,
                                P.splits, glu, stream(), ways.scale,
                                ways.ends()));
@@ -404,7 +416,7 @@ void dq_mid(const torch::Tensor& x, const torch::Tensor& qweight,
   A.splits = P.splits;
   A.row_scale = ways.scale;
   CHECK_HIP(lfmq_dq_mid(A, P, glu, stream()));
-  if (P.splits > 1)
+  if (P.splits > 1 && !ways.keeps(part, P.splits))
     CHECK_HIP(lfmq_dq_rows_sum(part.data_ptr(), y.data_ptr(), bias, resid, m, n,
                                P.splits, false, stream(), ways.scale,
                                ways.ends()));
@@ -930,10 +942,33 @@ std::vector<torch::Tensor> prompt_layer(
   const auto sizes = h.sizes().vec();
   const long b = sizes[0], s = sizes[1];
   auto rows = [&](const torch::Tensor& t) { return t.view({b * s, t.size(-1)}); };
+  torch::Tensor part, q;
+  int splits = 0;
+  RowWays ways{};
+  const long d = kc.size(3), hkv = kc.size(1);
+  if (d % 8 == 0 && b * s <= 65535 && packed[0].size(0) == (hq + 2 * hkv) * d &&
+      ((uintptr_t)kc.data_ptr() | (uintptr_t)vc.data_ptr() |
+       (uintptr_t)inv_freq.data_ptr()) % 16 == 0) {
+    ways.parts = &part;
+    ways.count = &splits;
+  }
   auto qkv = linear(rows(h), packed[0], packed[1], packed[2], forms[0], forms[1],
-                    biases[0], c10::nullopt, -1.0, 0, {});
-  auto q = qkv_rope_append(qkv, kc, vc, positions, inv_freq, hq, pos0,
-                           c10::nullopt);
+                    biases[0], c10::nullopt, -1.0, 0, ways);
+  if (splits > 1) {
+    check_t(kc, torch::kBFloat16, "k_cache");
+    check_t(vc, torch::kBFloat16, "v_cache");
+    check_t(positions, torch::kInt32, "positions");
+    check_t(inv_freq, torch::kFloat32, "inv_freq");
+    q = torch::empty({b, s, hq, d}, h.options());
+    CHECK_HIP(lfmq_qkv_sum_rope_append(
+        part.data_ptr(), splits,
+        biases[0].has_value() ? biases[0]->data_ptr() : nullptr, q.data_ptr(),
+        kc.data_ptr(), vc.data_ptr(), positions.data_ptr(), inv_freq.data_ptr(),
+        (int)b, (int)s, (int)hq, (int)hkv, (int)d, (int)kc.size(2), (int)pos0,
+        stream()));
+  } else {
+    q = qkv_rope_append(qkv, kc, vc, positions, inv_freq, hq, pos0, c10::nullopt);
+  }
   auto o = attn_prefill(q.view({b, s, hq * q.size(3)}), kc, vc, hq, pos0, scale);
   auto r = dq_linear_norm(rows(o), packed[3], packed[4], packed[5], forms[2],
                           forms[3], biases[1], residual, post_norm, post_eps);

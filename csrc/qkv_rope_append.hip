@@ -72,7 +72,98 @@ __global__ void qkv_rope_append_kernel(
   }
 }
 
+// The same from the parts of the projection, part [splits, b s, n] fp32 (+ bias),
+// whose sums are rounded to bf16 as a launch of their own would store them: one
+// launch and the projection's way to memory and back less.  A thread has four
+// values of each half of a head, up to four parts of them on their way at once.
+// 77 tokens of 3072, us: the sum of parts 3.8 and the rotation 3.4, both here 3.8.
+__global__ __launch_bounds__(256) void qkv_sum_rope_append_kernel(
+    const float* __restrict__ part, int splits,
+    const unsigned short* __restrict__ bias, u64* __restrict__ q_out,
+    u64* __restrict__ kc, u64* __restrict__ vc,
+    const i32* __restrict__ positions, const float* __restrict__ inv_freq,
+    int s, int hq, int hkv, int d, int tmax, int pos0) {
+  const int item = blockIdx.x * 256 + threadIdx.x, per = d / 8;
+  const int head = item / per, j = item % per, tok = blockIdx.y;
+  if (head >= hq + 2 * hkv) return;
+  const int n = (hq + 2 * hkv) * d, c0 = head * d + j * 4, c1 = c0 + d / 2;
+  const int si = tok % s, bb = tok / s;
+  const u64 stride = (u64)gridDim.y * n;
+  const float* row = part + (u64)tok * n;
+  const float pos = (float)positions[si];
+  const f32x4 freq = *(const f32x4*)(inv_freq + j * 4);
+  f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
+  for (int s0 = 0; s0 < splits; s0 += 4) {
+    f32x4 ta[4], tb[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float* p = row + (u64)min(s0 + i, splits - 1) * stride;
+      ta[i] = *(const f32x4*)(p + c0);
+      tb[i] = *(const f32x4*)(p + c1);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (s0 + i < splits) {
+        a += ta[i];
+        b += tb[i];
+      }
+  }
+  if (bias != nullptr)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      a[e] += bf16_bits_to_f32(bias[c0 + e]);
+      b[e] += bf16_bits_to_f32(bias[c1 + e]);
+    }
+  u32 lo[2], hi[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    lo[e] = pack_bf16x2(a[2 * e], a[2 * e + 1]);
+    hi[e] = pack_bf16x2(b[2 * e], b[2 * e + 1]);
+  }
+  const bool rotated = head < hq + hkv;
+  if (rotated) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      float a0, a1, b0, b1, sn0, cs0, sn1, cs1;
+      bf16x2_to_f32(lo[e], a0, a1);
+      bf16x2_to_f32(hi[e], b0, b1);
+      __sincosf(pos * freq[2 * e], &sn0, &cs0);
+      __sincosf(pos * freq[2 * e + 1], &sn1, &cs1);
+      lo[e] = pack_bf16x2(a0 * cs0 - b0 * sn0, a1 * cs1 - b1 * sn1);
+      hi[e] = pack_bf16x2(a0 * sn0 + b0 * cs0, a1 * sn1 + b1 * cs1);
+    }
+  }
+  u64* dst;
+  if (head < hq)
+    dst = q_out + ((u64)tok * hq + head) * (d / 4);
+  else
+    dst = (rotated ? kc : vc) +
+          (((u64)bb * hkv + (head - hq) % hkv) * tmax + pos0 + si) * (d / 4);
+  dst[j] = lo[0] | (u64)lo[1] << 32;
+  dst[j + per] = hi[0] | (u64)hi[1] << 32;
+}
+
 }  // namespace
+
+// part [splits, b s, (hq + 2 hkv) d]; heads in eights, caches and frequencies on 16
+// bytes
+hipError_t lfmq_qkv_sum_rope_append(const void* part, int splits,
+                                    const void* bias, void* q_out, void* kc,
+                                    void* vc, const void* positions,
+                                    const void* inv_freq, int b, int s, int hq,
+                                    int hkv, int d, int tmax, int pos0,
+                                    hipStream_t stream) {
+  const int items = (hq + 2 * hkv) * (d / 8);
+  if (d % 8 || splits < 1 || b < 1 || s < 1 || (long)b * s > 65535 ||
+      (((u64)kc | (u64)vc | (u64)q_out | (u64)inv_freq) & 15))
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL(qkv_sum_rope_append_kernel,
+                     dim3((items + 255) / 256, b * s), dim3(256), 0, stream,
+                     (const float*)part, splits, (const unsigned short*)bias,
+                     (u64*)q_out, (u64*)kc, (u64*)vc, (const i32*)positions,
+                     (const float*)inv_freq, s, hq, hkv, d, tmax, pos0);
+  return hipGetLastError();
+}
 
 hipError_t lfmq_qkv_rope_append(const void* qkv, void* q_out, void* kc,
                                 void* vc, const void* positions,

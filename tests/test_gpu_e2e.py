@@ -289,14 +289,17 @@ def test_decode_matches_prefill_gpu_d128():
 
 @pytest.mark.parametrize("b,s,past,bits,gs,bias", [
     (1, 2, 0, 4, 64, False), (1, 77, 5, 8, 64, False), (3, 40, 0, 4, 128, True),
-    (2, 150, 33, 4, 64, False)])
+    (2, 150, 33, 4, 64, False), (1, 60, 0, 4, 64, True), (2, 33, 9, 8, 128, True),
+    (1, 77, 3, 8, 64, True), (2, 50, 0, 8, 64, False), (1, 96, 1, 4, 128, True)])
 def test_prompt_layer_in_one_call(b, s, past, bits, gs, bias, monkeypatch):
     """A layer's kernels called from one place are those called one by one:
-    the same logits and cache; a hook on a layer is still called."""
+    the same logits and cache, also where the rotation adds up the projection's
+    parts (from 2048 wide on); a hook on a layer is still called."""
     from lfmq.models.llama import LlamaDecoderLayer
-    cfg = LlamaConfig(vocab_size=512, hidden_size=512, intermediate_size=1024,
-                      n_layers=2, n_heads=4, n_kv_heads=2, head_dim=128,
-                      max_seq=256)
+    heads = 16 if s in (50, 77, 96) else 4
+    cfg = LlamaConfig(vocab_size=512, hidden_size=heads * 128,
+                      intermediate_size=1024, n_layers=2, n_heads=heads,
+                      n_kv_heads=heads // 4 * 2, head_dim=128, max_seq=256)
     m = lfmq.quantize(lfmq.build_model(cfg, seed=7), lfmq.QuantConfig(
         scheme="rtn", bits=bits, group_size=gs)).to(DEV)
     if bias:
