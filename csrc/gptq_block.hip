@@ -536,7 +536,8 @@ hipError_t lfmq_gptq_block(const void* w, const void* ub, int ldu, void* codes,
   const BlockArgs A{(const float*)w, (const float*)ub, (i32*)codes,
                     (float*)scales, (i32*)zeros, (float*)err, ldu, n, k, G, i1,
                     nb, g, qmax, inv, sym, wide, nullptr, nullptr};
-  // a wave a SIMD while they last (2048 rows 31 us in eight waves, 26 in two),
+  // a wave a SIMD while they last (2048 rows, with rows of U read
+  // late, 31 us in eight waves, 26 in two),
   // then U read less often
   const int tpb = n <= 4096 ? 128 : (n <= 8192 ? 256 : 512);
   const dim3 grid((n + tpb / 16 - 1) / (tpb / 16));
