@@ -1,6 +1,6 @@
 """GPU parity tests: every HIP kernel vs its CPU reference twin.
 
-All run in ONE gpurun call (`pytest -m gpu`).  Tolerances: exact for
+All run with `pytest -m gpu`.  Tolerances: exact for
 pack/unpack/kv_append; bf16-accumulation tolerances vs the fp32 reference
 for the compute kernels.  Inputs are random and ASYMMETRIC (guide §3:
 symmetric operands mask transposed-output bugs).
