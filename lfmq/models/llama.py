@@ -89,6 +89,14 @@ def linear_norm(p: nn.Module, x, residual, norm: RMSNorm):
     return F.rmsnorm_residual(p(x), residual, norm.weight, norm.eps)
 
 
+def takes_factors(p: QLinear) -> bool:
+    """Whether a norm in front of p is worth a launch of its own for 17 to 48
+    rows: where a product without it may split k (`dq_mid`, `dq_short`).  A step of
+    17 rows of four layers of 2048, groups of 128: 4 bits 217.7 us with it, 209.3
+    without; 8 bits 228 and 231."""
+    return p.bits == 8 or p.in_features >= 4096
+
+
 class LlamaAttention(nn.Module):
     def __init__(self, cfg: LlamaConfig, dtype):
         super().__init__()
@@ -333,19 +341,24 @@ class LlamaDecoderLayer(nn.Module):
                             next_eps: float, tickets=None):
         """forward_decode_fused for 17 to 48 rows: an RMSNorm is a factor of
         each row, which the product before it leaves beside its result
-        (x, scale -> the same of the next layer).  The products, which do not
+        (x, scale, or None -> the same of the next layer).  The products, which do not
         have to see whole rows any more, may split k.  us a step of four
         layers, norms in the products and this way: hidden 4096, 4 bits 410 /
         372 at 17 rows, 452 / 378 at 32, 459 / 425 at 48; 8 bits 551 / 473 at
-        32; hidden 2048 260 / 256.  Up to 16 rows the product that walks over
+        32; hidden 2048 268 / 260 at 48.  Up to 16 rows the product that walks over
         columns has the norm for nothing (with a gate 18 us at 16 rows of
         28672 x 4096, 26 for this way's at 17)."""
         att, mlp = self.self_attn, self.mlp
+        gp, eps = mlp.gate_up_proj, self.post_attention_layernorm.eps
         o = att.decode_qkv_attn(x, cache_k, cache_v, state, max_seq,
-                                tickets=tickets, row_scale=scale)
-        x, scale = F.dq_linear_scaled(o, None, att.o_proj, x,
-                                      self.post_attention_layernorm.eps)
-        h = F.dq_gateup_scaled(x, scale, mlp.gate_up_proj)
+                                self.input_layernorm.eps, tickets, scale)
+        if takes_factors(gp):
+            x, scale = F.dq_linear_scaled(o, None, att.o_proj, x, eps)
+            h = F.dq_gateup_scaled(x, scale, gp)
+        else:
+            x = att.o_proj.forward_resid(o, x)
+            h = F.dq_gemv_gateup(x, gp.qweight, gp.scales, gp.qzeros, gp.bits,
+                                 gp.group_size, rms_eps=eps)
         return F.dq_linear_scaled(h, None, mlp.down_proj, x, next_eps)
 
 
@@ -494,7 +507,8 @@ class LlamaForCausalLM(nn.Module):
                                               and self._rows_fused())):
             if b > 16 and self._rows_scaled():
                 eps = [l.input_layernorm.eps for l in self.layers]
-                scale = F.row_scale(x, eps[0])
+                scale = F.row_scale(x, eps[0]) if takes_factors(
+                    self.layers[0].self_attn.qkv_proj) else None
                 for i, layer in enumerate(self.layers):
                     x, scale = layer.forward_decode_rows(
                         x, scale, cache.k[i], cache.v[i], state, max_seq,

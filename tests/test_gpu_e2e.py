@@ -324,3 +324,27 @@ def test_prompt_layer_in_one_call(b, s, past, bits, gs, bias, monkeypatch):
     assert calls
     a, z = out[0][0].float(), out[2][0].float()
     assert float((a - z).norm() / z.norm()) < 0.02   # 2 layers of 2^-9 roundings
+
+
+@pytest.mark.parametrize("b,gs", [(17, 64), (48, 128)])
+def test_factors_of_rows_match_norms_apart(b, gs):
+    """8 bits: norms as factors that a product leaves for the next one, against
+    kernels of their own: logits agree to the rounding of the values between."""
+    cfg = LlamaConfig(vocab_size=512, hidden_size=512, intermediate_size=1024,
+                      n_layers=2, n_heads=8, n_kv_heads=2, head_dim=64,
+                      max_seq=64)
+    m = lfmq.quantize(lfmq.build_model(cfg, seed=7), lfmq.QuantConfig(
+        scheme="rtn", bits=8, group_size=gs, fold_rms=True)).to(DEV)
+    ids = torch.randint(0, cfg.vocab_size, (b, 5), device=DEV)
+    out = []
+    for fused in (True, False):
+        if not fused:
+            assert m._fused_decode and m._rows_fused() and m._rows_scaled()
+            m._fused_decode = False
+        c = m.make_cache(b, 32)
+        with torch.no_grad():
+            m(ids, c)
+            state = torch.tensor([5, 6, 0], dtype=torch.int32, device=DEV)
+            out.append(m.forward_decode_step(ids[:, :1], c, state, 32).float())
+    d = (out[0] - out[1]).norm() / out[1].norm()
+    assert float(d) < 0.02, float(d)     # 2 layers of 2^-9 roundings
