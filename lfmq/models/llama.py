@@ -161,16 +161,6 @@ class LlamaAttention(nn.Module):
             o = self._chunk_attn(qh, cache_k, cache_v, pos0, seq_len_after)
         return o.transpose(1, 2).reshape(b, s, hq * d)
 
-    def norm_after(self, x, cache_k, cache_v, positions, seq_len_after,
-                   residual, norm):
-        """F.rmsnorm_residual of the result, and what it norms."""
-        if type(self).forward is LlamaAttention.forward and not hooked(self):
-            return linear_norm(self.o_proj, self.attend(
-                x, cache_k, cache_v, positions, seq_len_after), residual, norm)
-        return F.rmsnorm_residual(
-            self(x, cache_k, cache_v, positions, seq_len_after), residual,
-            norm.weight, norm.eps)
-
     def forward_decode_graph(self, x, cache_k, cache_v, state, max_seq,
                              tickets=None):
         """hipGraph-capturable decode step (s == 1, GPU only)."""
@@ -237,11 +227,29 @@ class LlamaMLP(nn.Module):
                                     gp.bits, gp.group_size)
         return F.silu_mul_gateup(gp(x), self.inter)
 
-    def norm_after(self, x, residual, norm):
-        """F.rmsnorm_residual of the result, and what it norms."""
-        if type(self).forward is LlamaMLP.forward and not hooked(self):
-            return linear_norm(self.down_proj, self.gated(x), residual, norm)
-        return F.rmsnorm_residual(self(x), residual, norm.weight, norm.eps)
+
+def forwards_as(m, cls: type) -> bool:
+    """Whether m's call is what cls does, and no module's that a caller has put
+    in its place (of such a one only the call is known)."""
+    return getattr(type(m), "forward", None) is cls.forward
+
+
+def attention_norm(att: nn.Module, x, cache_k, cache_v, positions,
+                   seq_len_after, residual, norm: RMSNorm):
+    """F.rmsnorm_residual of att's result, and what it norms."""
+    if forwards_as(att, LlamaAttention) and not hooked(att):
+        return linear_norm(att.o_proj, att.attend(
+            x, cache_k, cache_v, positions, seq_len_after), residual, norm)
+    return F.rmsnorm_residual(
+        att(x, cache_k, cache_v, positions, seq_len_after), residual,
+        norm.weight, norm.eps)
+
+
+def mlp_norm(mlp: nn.Module, x, residual, norm: RMSNorm):
+    """The same of the feed-forward's."""
+    if forwards_as(mlp, LlamaMLP) and not hooked(mlp):
+        return linear_norm(mlp.down_proj, mlp.gated(x), residual, norm)
+    return F.rmsnorm_residual(mlp(x), residual, norm.weight, norm.eps)
 
 
 class LlamaDecoderLayer(nn.Module):
@@ -264,9 +272,9 @@ class LlamaDecoderLayer(nn.Module):
             h, residual = F.rmsnorm_residual(x, residual,
                                              self.input_layernorm.weight,
                                              self.input_layernorm.eps)
-        h, residual = self.self_attn.norm_after(
-            h, cache_k, cache_v, positions, seq_len_after, residual,
-            self.post_attention_layernorm)
+        h, residual = attention_norm(
+            self.self_attn, h, cache_k, cache_v, positions, seq_len_after,
+            residual, self.post_attention_layernorm)
         h = self.mlp(h)
         return h, residual
 
@@ -275,16 +283,18 @@ class LlamaDecoderLayer(nn.Module):
         """forward between norms: of the layer's normed input and what that
         was to the same of the next layer, whose norm it is."""
         att, mlp, post = self.self_attn, self.mlp, self.post_attention_layernorm
-        products = att.qkv_proj, att.o_proj, mlp.gate_up_proj, mlp.down_proj
-        if h.shape[1] > 1 and self._in_one_call(products):
-            return F.prompt_layer(h, residual, cache_k, cache_v, positions,
-                                  seq_len_after - h.shape[1], att.n_heads,
-                                  att.cfg.rope_theta, att.scale, products,
-                                  post, norm)
-        h, residual = self.self_attn.norm_after(
-            h, cache_k, cache_v, positions, seq_len_after, residual,
-            self.post_attention_layernorm)
-        return self.mlp.norm_after(h, residual, norm)
+        if h.shape[1] > 1 and forwards_as(att, LlamaAttention) and \
+                forwards_as(mlp, LlamaMLP):
+            products = (att.qkv_proj, att.o_proj, mlp.gate_up_proj,
+                        mlp.down_proj)
+            if self._in_one_call(products):
+                return F.prompt_layer(h, residual, cache_k, cache_v, positions,
+                                      seq_len_after - h.shape[1], att.n_heads,
+                                      att.cfg.rope_theta, att.scale, products,
+                                      post, norm)
+        h, residual = attention_norm(att, h, cache_k, cache_v, positions,
+                                     seq_len_after, residual, post)
+        return mlp_norm(mlp, h, residual, norm)
 
     def _in_one_call(self, products) -> bool:
         att, mlp = self.self_attn, self.mlp
@@ -293,8 +303,6 @@ class LlamaDecoderLayer(nn.Module):
                 and all(type(p) is QLinear and "perm" not in p._buffers
                         and "perm" not in p.__dict__ for p in products)
                 and products[2].bias is None and rows_fused(products[2])
-                and type(att).forward is LlamaAttention.forward
-                and type(mlp).forward is LlamaMLP.forward
                 and not hooked(att, mlp, *products))
 
     def forward_decode_step(self, x, cache_k, cache_v, state, max_seq,

@@ -24,7 +24,7 @@ import torch.nn as nn
 from ..ops import functional as F
 from .kvcache import KVCache
 from .linear import Linear, hooked
-from .llama import LlamaAttention, LlamaConfig, RMSNorm
+from .llama import LlamaAttention, LlamaConfig, RMSNorm, attention_norm
 from .qlinear import QLinear, gathers
 
 
@@ -268,9 +268,9 @@ class MixtralDecoderLayer(nn.Module):
             h, residual = F.rmsnorm_residual(x, residual,
                                              self.input_layernorm.weight,
                                              self.input_layernorm.eps)
-        h, residual = self.self_attn.norm_after(
-            h, cache_k, cache_v, positions, seq_len_after, residual,
-            self.post_attention_layernorm)
+        h, residual = attention_norm(
+            self.self_attn, h, cache_k, cache_v, positions, seq_len_after,
+            residual, self.post_attention_layernorm)
         h = self.moe(h)
         return h, residual
 

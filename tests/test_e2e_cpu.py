@@ -4,10 +4,13 @@ Config #1: OPT-125m-shaped per-tensor int8 RTN quantize +
 CPU matmul decode — quantize -> save -> load -> greedy decode equivalence
 vs fp32 within tolerance.  Plus tiny-Llama GPTQ/AWQ end-to-end fidelity.
 """
+import pytest
 import torch
 
 from lfmq import QuantConfig, build_model, load, quantize, save
-from lfmq.models.llama import LlamaConfig
+from lfmq.models.kvcache import KVCache
+from lfmq.models.llama import LlamaConfig, LlamaForCausalLM
+from lfmq.models.mixtral import MixtralConfig
 from lfmq.models.opt import OPTConfig
 from lfmq.quant.calib import CalibStream
 
@@ -154,3 +157,42 @@ def test_caches_own_their_arrival_counters():
         a, b = m.make_cache(3, 16), m.make_cache(3, 16)
         assert a.tickets.data_ptr() != b.tickets.data_ptr()
         assert a.tickets.tolist() == [0] * 3 * cfg.n_heads
+
+
+class Standin(torch.nn.Module):
+    """A caller's module in the place of a layer's: a call, and nothing else."""
+
+    def __init__(self, of):
+        super().__init__()
+        self.of = of
+
+    def forward(self, *args):
+        return self.of(*args)
+
+
+@pytest.mark.parametrize("arch", ["llama", "mixtral"])
+@pytest.mark.parametrize("names", [("self_attn",), ("mlp",), ("self_attn", "mlp")])
+@pytest.mark.parametrize("norms_ride", [False, True])
+def test_replaced_modules_are_called(arch, names, norms_ride, monkeypatch):
+    """Attention and feed-forward that a caller has replaced take prompts and
+    tokens, also where a layer's last product takes the next norm along (on the
+    GPU)."""
+    cfg = (LlamaConfig if arch == "llama" else MixtralConfig).tiny()
+    m = build_model(cfg, seed=3)
+    if norms_ride:
+        monkeypatch.setattr(LlamaForCausalLM, "_norms_ride", lambda *a: True)
+    ids = torch.randint(0, cfg.vocab_size, (2, 9))
+
+    def logits():
+        cache = m.make_cache(2, 16)
+        return m(ids, cache), m(ids[:, :1], cache)
+
+    want = logits()
+    m.make_cache = lambda b, n: KVCache(
+        cfg.n_layers, b, cfg.n_kv_heads, n, cfg.head_dim, "cpu", dtype=m.dtype)
+    for layer in m.layers:
+        for name in names:
+            name = "moe" if arch == "mixtral" and name == "mlp" else name
+            setattr(layer, name, Standin(getattr(layer, name)))
+    for a, b in zip(logits(), want):
+        assert torch.equal(a, b)
