@@ -897,18 +897,35 @@ torch::Tensor dq_gateup_scaled(torch::Tensor x, torch::Tensor scale,
   return y;
 }
 
+// s rows from pos0 on for caches [b, hkv, tmax, d], before anything writes them:
+// their places in the caches, an angle's factors and positions are there
+void check_append(const torch::Tensor& kc, const torch::Tensor& vc,
+                  const torch::Tensor& positions, const torch::Tensor& inv_freq,
+                  long s, long pos0) {
+  check_t(kc, torch::kBFloat16, "k_cache");
+  check_t(vc, torch::kBFloat16, "v_cache");
+  check_t(positions, torch::kInt32, "positions");
+  check_t(inv_freq, torch::kFloat32, "inv_freq");
+  TORCH_CHECK(kc.dim() == 4 && kc.sizes() == vc.sizes(),
+              "caches must be [b, hkv, tmax, d]");
+  TORCH_CHECK(pos0 >= 0 && s <= kc.size(2) && pos0 <= kc.size(2) - s,
+              "KV cache overflow: ", pos0, " + ", s, " > ", kc.size(2));
+  TORCH_CHECK(positions.numel() >= s, "positions must have s entries");
+  TORCH_CHECK(inv_freq.numel() >= kc.size(3) / 2,
+              "inv_freq must have d / 2 entries");
+}
+
 torch::Tensor qkv_rope_append(torch::Tensor qkv, torch::Tensor kc,
                               torch::Tensor vc, torch::Tensor positions,
                               torch::Tensor inv_freq, long hq, long pos0,
                               c10::optional<torch::Tensor> pos_dev) {
   check_t(qkv, torch::kBFloat16, "qkv");
-  check_t(kc, torch::kBFloat16, "k_cache");
-  check_t(vc, torch::kBFloat16, "v_cache");
-  check_t(positions, torch::kInt32, "positions");
-  check_t(inv_freq, torch::kFloat32, "inv_freq");
+  TORCH_CHECK(kc.dim() == 4 && kc.size(0) > 0 && (hq + 2 * kc.size(1)) * kc.size(3) > 0,
+              "caches must be [b, hkv, tmax, d]");
   const int b = (int)kc.size(0), hkv = (int)kc.size(1);
   const int tmax = (int)kc.size(2), d = (int)kc.size(3);
   const int s = (int)(qkv.numel() / ((hq + 2 * hkv) * d)) / b;
+  check_append(kc, vc, positions, inv_freq, s, pos0);
   auto q_out = torch::empty({b, s, hq, (long)d}, qkv.options());
   const void* pdev = nullptr;
   if (pos_dev.has_value()) {
@@ -941,6 +958,8 @@ std::vector<torch::Tensor> prompt_layer(
               "a layer has four packed products");
   const auto sizes = h.sizes().vec();
   const long b = sizes[0], s = sizes[1];
+  check_append(kc, vc, positions, inv_freq, s, pos0);
+  TORCH_CHECK(kc.size(0) == b, "a cache of ", kc.size(0), " for ", b, " sequences");
   auto rows = [&](const torch::Tensor& t) { return t.view({b * s, t.size(-1)}); };
   torch::Tensor part, q;
   int splits = 0;
@@ -955,10 +974,6 @@ std::vector<torch::Tensor> prompt_layer(
   auto qkv = linear(rows(h), packed[0], packed[1], packed[2], forms[0], forms[1],
                     biases[0], c10::nullopt, -1.0, 0, ways);
   if (splits > 1) {
-    check_t(kc, torch::kBFloat16, "k_cache");
-    check_t(vc, torch::kBFloat16, "v_cache");
-    check_t(positions, torch::kInt32, "positions");
-    check_t(inv_freq, torch::kFloat32, "inv_freq");
     q = torch::empty({b, s, hq, d}, h.options());
     CHECK_HIP(lfmq_qkv_sum_rope_append(
         part.data_ptr(), splits,

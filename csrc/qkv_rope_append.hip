@@ -155,6 +155,7 @@ hipError_t lfmq_qkv_sum_rope_append(const void* part, int splits,
                                     hipStream_t stream) {
   const int items = (hq + 2 * hkv) * (d / 8);
   if (d % 8 || splits < 1 || b < 1 || s < 1 || (long)b * s > 65535 ||
+      pos0 < 0 || pos0 > tmax - s ||
       (((u64)kc | (u64)vc | (u64)q_out | (u64)inv_freq) & 15))
     return hipErrorInvalidValue;
   hipLaunchKernelGGL(qkv_sum_rope_append_kernel,

@@ -287,7 +287,7 @@ class LlamaDecoderLayer(nn.Module):
                 forwards_as(mlp, LlamaMLP):
             products = (att.qkv_proj, att.o_proj, mlp.gate_up_proj,
                         mlp.down_proj)
-            if self._in_one_call(products):
+            if cache_k.shape[0] == h.shape[0] and self._in_one_call(products):
                 return F.prompt_layer(h, residual, cache_k, cache_v, positions,
                                       seq_len_after - h.shape[1], att.n_heads,
                                       att.cfg.rope_theta, att.scale, products,

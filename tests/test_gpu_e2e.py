@@ -348,3 +348,37 @@ def test_factors_of_rows_match_norms_apart(b, gs):
             out.append(m.forward_decode_step(ids[:, :1], c, state, 32).float())
     d = (out[0] - out[1]).norm() / out[1].norm()
     assert float(d) < 0.02, float(d)     # 2 layers of 2^-9 roundings
+
+
+@pytest.mark.parametrize("one_call", [True, False])
+@pytest.mark.parametrize("past,s,given", [(0, 77, None), (60, 5, None),
+                                          (0, 50, 49), (3, 61, 64)])
+def test_prompts_that_do_not_fit_write_nothing(one_call, past, s, given,
+                                               monkeypatch):
+    """Rows past the cache's end, and positions that are too few, are refused
+    before any layer writes to the cache."""
+    from lfmq.models.llama import LlamaDecoderLayer
+    cfg = LlamaConfig(vocab_size=512, hidden_size=2048, intermediate_size=1024,
+                      n_layers=1, n_heads=16, n_kv_heads=8, head_dim=128,
+                      max_seq=64)
+    m = lfmq.quantize(lfmq.build_model(cfg, seed=7), lfmq.QuantConfig(
+        scheme="rtn", bits=8, group_size=64)).to(DEV)
+    if not one_call:
+        monkeypatch.setattr(LlamaDecoderLayer, "_in_one_call",
+                            lambda *a: False)
+    c = m.make_cache(2, 64)
+    c.k_all.fill_(7)
+    c.v_all.fill_(7)
+    c.seq_len = past
+    ids = torch.randint(0, 512, (2, s), device=DEV)
+    pos = None if given is None else torch.arange(given, device=DEV)
+    with torch.no_grad():
+        if past + s > 64 or (given or s) < s:
+            with pytest.raises(RuntimeError):
+                m(ids, c, pos)
+            assert bool((c.k_all == 7).all()) and bool((c.v_all == 7).all())
+            assert c.seq_len == past
+        else:
+            m(ids, c, pos)
+            assert bool((c.k_all[..., :past, :] == 7).all())
+            assert c.seq_len == past + s
