@@ -609,12 +609,13 @@ std::vector<torch::Tensor> dq_linear_norm(
 }
 
 // Rows of x times their factors (17 to 48 rows); eps >= 0: also row_scale of the
-// result, with the sum of the product's parts where it has some
+// result, from the sum of the product's parts where it has some, else by a launch
+// of its own, and not at all without `apart`
 std::vector<torch::Tensor> dq_linear_scaled(
     torch::Tensor x, c10::optional<torch::Tensor> scale, torch::Tensor qweight,
     torch::Tensor scales, torch::Tensor qzeros, long bits, long g,
     c10::optional<torch::Tensor> bias, c10::optional<torch::Tensor> resid,
-    double eps) {
+    double eps, bool apart) {
   const int m = (int)x.size(0), n = (int)qweight.size(0);
   if (resid.has_value())
     TORCH_CHECK(resid->numel() == (long)m * n, "one residual a result");
@@ -631,7 +632,7 @@ std::vector<torch::Tensor> dq_linear_scaled(
   }
   auto y = linear(x, qweight, scales, qzeros, bits, g, bias, resid, -1.0, 0,
                   ways);
-  if (eps < 0) return {y};
+  if (eps < 0 || (!ended && !apart)) return {y};
   if (!ended)
     CHECK_HIP(lfmq_row_scale(y.data_ptr(), out.data_ptr(), m, n, (float)eps,
                              stream()));
@@ -1482,7 +1483,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("dq_linear", &dq_linear, "fused dequant GEMV/GEMM");
   m.def("row_scale", &row_scale, "1 / root mean square of rows");
   m.def("dq_linear_scaled", &dq_linear_scaled,
-        "dq_linear of rows times factors, and the result's own");
+        "dq_linear of rows times factors, and the result's own",
+        pybind11::arg("x"), pybind11::arg("scale"), pybind11::arg("qweight"),
+        pybind11::arg("scales"), pybind11::arg("qzeros"), pybind11::arg("bits"),
+        pybind11::arg("g"), pybind11::arg("bias"), pybind11::arg("resid"),
+        pybind11::arg("eps"), pybind11::arg("apart") = true);
   m.def("prompt_layer", &prompt_layer, "a layer's kernels for a prompt");
   m.def("dq_linear_norm", &dq_linear_norm,
         "dq_linear, the residual and the next norm");

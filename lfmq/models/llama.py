@@ -346,10 +346,12 @@ class LlamaDecoderLayer(nn.Module):
         return x
 
     def forward_decode_rows(self, x, scale, cache_k, cache_v, state, max_seq,
-                            next_eps: float, tickets=None):
+                            following: Optional["LlamaDecoderLayer"],
+                            tickets=None):
         """forward_decode_fused for 17 to 48 rows: an RMSNorm is a factor of
         each row, which the product before it leaves beside its result
-        (x, scale, or None -> the same of the next layer).  The products, which do not
+        (x, scale, or None -> the same of the following layer, if there is
+        one).  The products, which do not
         have to see whole rows any more, may split k.  us a step of four
         layers, norms in the products and this way: hidden 4096, 4 bits 410 /
         372 at 17 rows, 452 / 378 at 32, 459 / 425 at 48; 8 bits 551 / 473 at
@@ -367,7 +369,11 @@ class LlamaDecoderLayer(nn.Module):
             x = att.o_proj.forward_resid(o, x)
             h = F.dq_gemv_gateup(x, gp.qweight, gp.scales, gp.qzeros, gp.bits,
                                  gp.group_size, rms_eps=eps)
-        return F.dq_linear_scaled(h, None, mlp.down_proj, x, next_eps)
+        if following is None:              # nobody reads the last one's
+            return mlp.down_proj.forward_resid(h, x), None
+        return F.dq_linear_scaled(
+            h, None, mlp.down_proj, x, following.input_layernorm.eps,
+            takes_factors(following.self_attn.qkv_proj))
 
 
 class LlamaForCausalLM(nn.Module):
@@ -514,13 +520,14 @@ class LlamaForCausalLM(nn.Module):
         if self._fused_decode and (b <= 4 or (b <= FEW_ROWS
                                               and self._rows_fused())):
             if b > 16 and self._rows_scaled():
-                eps = [l.input_layernorm.eps for l in self.layers]
-                scale = F.row_scale(x, eps[0]) if takes_factors(
-                    self.layers[0].self_attn.qkv_proj) else None
-                for i, layer in enumerate(self.layers):
+                first, scale = self.layers[0], None
+                if takes_factors(first.self_attn.qkv_proj):
+                    scale = F.row_scale(x, first.input_layernorm.eps)
+                for i, (layer, following) in enumerate(
+                        zip(self.layers, [*self.layers[1:], None])):
                     x, scale = layer.forward_decode_rows(
                         x, scale, cache.k[i], cache.v[i], state, max_seq,
-                        eps[min(i + 1, len(eps) - 1)], tickets)
+                        following, tickets)
             else:
                 for i, layer in enumerate(self.layers):
                     x = layer.forward_decode_fused(x, cache.k[i], cache.v[i],

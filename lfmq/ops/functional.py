@@ -94,17 +94,19 @@ def row_scale(x: torch.Tensor, eps: float) -> torch.Tensor:
 
 
 def dq_linear_scaled(x: torch.Tensor, scale: Optional[torch.Tensor], p,
-                     resid: Optional[torch.Tensor] = None, eps: float = -1.0):
+                     resid: Optional[torch.Tensor] = None, eps: float = -1.0,
+                     apart: bool = True):
     """GPU-only dq_linear of the packed layer p for 17 to 48 rows: x's rows
     times scale (its row_scale, for an RMSNorm without weights in front); with
-    eps >= 0 the result and its own row_scale."""
+    eps >= 0 the result and its own row_scale, or None where that would take a
+    launch of its own and apart is not set."""
     r2 = resid.reshape(-1, resid.shape[-1]).contiguous() \
         if resid is not None else None
     y, *own = hip_ext().dq_linear_scaled(
         x.reshape(-1, x.shape[-1]), scale, p.qweight, p.scales, p.qzeros,
-        p.bits, p.group_size, p.bias, r2, eps)
+        p.bits, p.group_size, p.bias, r2, eps, apart)
     y = _guard(y, "dq_linear").reshape(*x.shape[:-1], y.shape[-1])
-    return (y, *own) if own else y
+    return (y, own[0] if own else None) if eps >= 0 else y
 
 
 def dq_linear_norm(x: torch.Tensor, p, residual: torch.Tensor,

@@ -196,3 +196,56 @@ def test_replaced_modules_are_called(arch, names, norms_ride, monkeypatch):
             setattr(layer, name, Standin(getattr(layer, name)))
     for a, b in zip(logits(), want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("bits,parts", [(4, True), (4, False), (8, False)])
+def test_factors_of_rows_that_somebody_reads(bits, parts, monkeypatch):
+    """A step of 17 rows asks for the factors of a norm's rows only where a
+    product reads them, and for a launch of their own only where the next product
+    is worth one; what a product in parts leaves is taken anyhow."""
+    from lfmq.ops import functional as F
+    cfg = LlamaConfig.tiny()
+    m = quantize(build_model(cfg, seed=3), QuantConfig(
+        scheme="rtn", bits=bits, group_size=64, fold_rms=True))
+    b, asked, given, read = 17, [], [], []
+    names = {id(p): f"{i}.{n}" for i, l in enumerate(m.layers) for n, p in
+             (("qkv", l.self_attn.qkv_proj), ("o", l.self_attn.o_proj),
+              ("gate_up", l.mlp.gate_up_proj), ("down", l.mlp.down_proj))}
+
+    def out(x, n):
+        return torch.zeros(*x.shape[:-1], n, dtype=x.dtype)
+
+    def factors(name):
+        given.append(name)
+        return name
+
+    def linear_scaled(x, scale, p, resid=None, eps=-1.0, apart=True):
+        y, name = out(x, p.out_features), names[id(p)]
+        if scale is not None:
+            read.append(scale)
+        if eps < 0:
+            return y
+        asked.append((name, apart))
+        return y, factors(name) if parts or apart else None
+
+    monkeypatch.setattr(F, "row_scale", lambda x, eps: factors("embedding"))
+    monkeypatch.setattr(F, "dq_linear_scaled", linear_scaled)
+    monkeypatch.setattr(F, "dq_gateup_scaled", lambda x, scale, p: (
+        read.append(scale), out(x, p.out_features // 2))[1])
+    monkeypatch.setattr(F, "dq_gemv_gateup", lambda x, q, *a, **kw: out(
+        x, q.shape[0] // 2))
+    monkeypatch.setattr(F, "dq_linear", lambda x, q, *a, **kw: out(x, q.shape[0]))
+    monkeypatch.setattr(F, "attn_decode_fused", lambda qkv, k, v, st, n, sc, hq,
+                        *a: torch.zeros(len(qkv), hq * cfg.head_dim,
+                                        dtype=qkv.dtype))
+    state = torch.zeros(3, dtype=torch.int32)
+    m.forward_decode_step(torch.zeros(b, 1, dtype=torch.long),
+                          m.make_cache(b, 8), state, 8)
+    assert m._fused_decode and m._rows_fused() and m._rows_scaled()
+    last = len(m.layers) - 1
+    assert last > 0
+    assert given == read
+    assert ("embedding" in given) == (bits == 8)
+    assert asked == [(f"{i}.{n}", bits == 8) for i in range(last + 1)
+                     for n in ("o", "down")
+                     if (n == "o" and bits == 8) or (n == "down" and i < last)]

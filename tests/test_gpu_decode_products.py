@@ -234,6 +234,22 @@ def test_rows_times_their_factors(m, n, k, g, bits):
         close(ext().dq_gateup_scaled(x, scale, *p, bits, g), gated(rms), 1e-2)
 
 
+@pytest.mark.parametrize("m,n,k,g,bits,parts", [
+    (17, 2048, 2048, 64, 4, False), (32, 2048, 4096, 128, 4, False),
+    (48, 4096, 14336, 128, 4, True), (33, 4104, 2048, 64, 8, None),
+    (47, 1030, 2048, 64, 4, None), (18, 24576, 2048, 64, 4, None)])
+def test_factors_without_a_launch_of_their_own(m, n, k, g, bits, parts):
+    """Where the product's parts are summed the same factors, elsewhere none."""
+    p, _ = matrix(bits, n, k, g)
+    x = torch.randn(m, k, device=DEV).to(BF)
+    resid = torch.randn(m, n, device=DEV).to(BF)
+    y, want = ext().dq_linear_scaled(x, None, *p, bits, g, None, resid, 1e-6)
+    z, *own = ext().dq_linear_scaled(x, None, *p, bits, g, None, resid, 1e-6,
+                                     False)
+    assert torch.equal(y, z) and all(torch.equal(t, want) for t in own)
+    assert parts is None or bool(own) == parts
+
+
 @pytest.mark.parametrize("m,n,k,g,bits", [
     (77, 2048, 8192, 64, 8), (40, 4096, 14336, 128, 4), (64, 4104, 4096, 64, 4),
     (50, 8192, 4096, 128, 8), (33, 16384, 2048, 128, 4), (100, 1032, 4096, 128, 4),
