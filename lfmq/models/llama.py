@@ -228,16 +228,17 @@ class LlamaMLP(nn.Module):
         return F.silu_mul_gateup(gp(x), self.inter)
 
 
-def forwards_as(m, cls: type) -> bool:
-    """Whether m's call is what cls does, and no module's that a caller has put
-    in its place (of such a one only the call is known)."""
-    return getattr(type(m), "forward", None) is cls.forward
+def unchanged(m, cls: type, *names: str) -> bool:
+    """Whether these calls of m are what cls does, and not a caller's: of a module
+    or a method put in their place only the call is known."""
+    return all(getattr(type(m), n, None) is getattr(cls, n)
+               and n not in getattr(m, "__dict__", ()) for n in names)
 
 
 def attention_norm(att: nn.Module, x, cache_k, cache_v, positions,
                    seq_len_after, residual, norm: RMSNorm):
     """F.rmsnorm_residual of att's result, and what it norms."""
-    if forwards_as(att, LlamaAttention) and not hooked(att):
+    if unchanged(att, LlamaAttention, "forward") and not hooked(att):
         return linear_norm(att.o_proj, att.attend(
             x, cache_k, cache_v, positions, seq_len_after), residual, norm)
     return F.rmsnorm_residual(
@@ -247,7 +248,7 @@ def attention_norm(att: nn.Module, x, cache_k, cache_v, positions,
 
 def mlp_norm(mlp: nn.Module, x, residual, norm: RMSNorm):
     """The same of the feed-forward's."""
-    if forwards_as(mlp, LlamaMLP) and not hooked(mlp):
+    if unchanged(mlp, LlamaMLP, "forward") and not hooked(mlp):
         return linear_norm(mlp.down_proj, mlp.gated(x), residual, norm)
     return F.rmsnorm_residual(mlp(x), residual, norm.weight, norm.eps)
 
@@ -283,8 +284,8 @@ class LlamaDecoderLayer(nn.Module):
         """forward between norms: of the layer's normed input and what that
         was to the same of the next layer, whose norm it is."""
         att, mlp, post = self.self_attn, self.mlp, self.post_attention_layernorm
-        if h.shape[1] > 1 and forwards_as(att, LlamaAttention) and \
-                forwards_as(mlp, LlamaMLP):
+        if h.shape[1] > 1 and unchanged(att, LlamaAttention, "forward") \
+                and unchanged(mlp, LlamaMLP, "forward"):
             products = (att.qkv_proj, att.o_proj, mlp.gate_up_proj,
                         mlp.down_proj)
             if cache_k.shape[0] == h.shape[0] and self._in_one_call(products):
@@ -501,10 +502,13 @@ class LlamaForCausalLM(nn.Module):
 
     def _rows_scaled(self) -> bool:
         """Whether norms may also be left to the product before them."""
-        return all(type(p).forward_resid is QLinear.forward_resid
-                   and type(p).forward is QLinear.forward
-                   for layer in self.layers
-                   for p in (layer.self_attn.o_proj, layer.mlp.down_proj))
+        return all(
+            unchanged(layer, LlamaDecoderLayer, "forward_decode_fused")
+            and unchanged(layer.self_attn, LlamaAttention, "decode_qkv_attn")
+            and unchanged(layer.self_attn.qkv_proj, QLinear, "forward_rms")
+            and all(unchanged(p, QLinear, "forward", "forward_resid")
+                    for p in (layer.self_attn.o_proj, layer.mlp.down_proj))
+            for layer in self.layers)
 
     def forward_decode_step(self, input_ids, cache, state, max_seq):
         """One hipGraph-capturable decode step: [b,1] ids -> [b,1,vocab]."""

@@ -4,6 +4,8 @@ Config #1: OPT-125m-shaped per-tensor int8 RTN quantize +
 CPU matmul decode — quantize -> save -> load -> greedy decode equivalence
 vs fp32 within tolerance.  Plus tiny-Llama GPTQ/AWQ end-to-end fidelity.
 """
+import types
+
 import pytest
 import torch
 
@@ -198,6 +200,32 @@ def test_replaced_modules_are_called(arch, names, norms_ride, monkeypatch):
         assert torch.equal(a, b)
 
 
+def out(x, n):
+    return torch.zeros(*x.shape[:-1], n, dtype=x.dtype)
+
+
+def shapes_alone(m, monkeypatch):
+    """A captured step's products and attention (GPU only) as their shapes."""
+    from lfmq.ops import functional as F
+    d = m.cfg.head_dim
+    monkeypatch.setattr(F, "dq_gemv_gateup", lambda x, q, *a, **kw: out(
+        x, q.shape[0] // 2))
+    monkeypatch.setattr(F, "dq_linear", lambda x, q, *a, **kw: out(x, q.shape[0]))
+    monkeypatch.setattr(F, "attn_decode_fused", lambda qkv, k, v, st, n, sc, hq,
+                        *a: torch.zeros(len(qkv), hq * d, dtype=qkv.dtype))
+    monkeypatch.setattr(F, "row_scale", lambda x, eps: "embedding")
+    monkeypatch.setattr(F, "dq_linear_scaled", lambda x, scale, p, resid=None,
+                        eps=-1.0, apart=True: out(x, p.out_features)
+                        if eps < 0 else (out(x, p.out_features), "product"))
+    monkeypatch.setattr(F, "dq_gateup_scaled", lambda x, scale, p: out(
+        x, p.out_features // 2))
+
+
+def step(m, b):
+    m.forward_decode_step(torch.zeros(b, 1, dtype=torch.long), m.make_cache(b, 8),
+                          torch.zeros(3, dtype=torch.int32), 8)
+
+
 @pytest.mark.parametrize("bits,parts", [(4, True), (4, False), (8, False)])
 def test_factors_of_rows_that_somebody_reads(bits, parts, monkeypatch):
     """A step of 17 rows asks for the factors of a norm's rows only where a
@@ -207,13 +235,10 @@ def test_factors_of_rows_that_somebody_reads(bits, parts, monkeypatch):
     cfg = LlamaConfig.tiny()
     m = quantize(build_model(cfg, seed=3), QuantConfig(
         scheme="rtn", bits=bits, group_size=64, fold_rms=True))
-    b, asked, given, read = 17, [], [], []
+    asked, given, read = [], [], []
     names = {id(p): f"{i}.{n}" for i, l in enumerate(m.layers) for n, p in
              (("qkv", l.self_attn.qkv_proj), ("o", l.self_attn.o_proj),
               ("gate_up", l.mlp.gate_up_proj), ("down", l.mlp.down_proj))}
-
-    def out(x, n):
-        return torch.zeros(*x.shape[:-1], n, dtype=x.dtype)
 
     def factors(name):
         given.append(name)
@@ -228,19 +253,12 @@ def test_factors_of_rows_that_somebody_reads(bits, parts, monkeypatch):
         asked.append((name, apart))
         return y, factors(name) if parts or apart else None
 
+    shapes_alone(m, monkeypatch)
     monkeypatch.setattr(F, "row_scale", lambda x, eps: factors("embedding"))
     monkeypatch.setattr(F, "dq_linear_scaled", linear_scaled)
     monkeypatch.setattr(F, "dq_gateup_scaled", lambda x, scale, p: (
         read.append(scale), out(x, p.out_features // 2))[1])
-    monkeypatch.setattr(F, "dq_gemv_gateup", lambda x, q, *a, **kw: out(
-        x, q.shape[0] // 2))
-    monkeypatch.setattr(F, "dq_linear", lambda x, q, *a, **kw: out(x, q.shape[0]))
-    monkeypatch.setattr(F, "attn_decode_fused", lambda qkv, k, v, st, n, sc, hq,
-                        *a: torch.zeros(len(qkv), hq * cfg.head_dim,
-                                        dtype=qkv.dtype))
-    state = torch.zeros(3, dtype=torch.int32)
-    m.forward_decode_step(torch.zeros(b, 1, dtype=torch.long),
-                          m.make_cache(b, 8), state, 8)
+    step(m, 17)
     assert m._fused_decode and m._rows_fused() and m._rows_scaled()
     last = len(m.layers) - 1
     assert last > 0
@@ -249,3 +267,30 @@ def test_factors_of_rows_that_somebody_reads(bits, parts, monkeypatch):
     assert asked == [(f"{i}.{n}", bits == 8) for i in range(last + 1)
                      for n in ("o", "down")
                      if (n == "o" and bits == 8) or (n == "down" and i < last)]
+
+
+@pytest.mark.parametrize("where", ["class", "instance"])
+@pytest.mark.parametrize("b", [3, 17])
+@pytest.mark.parametrize("name", ["forward_decode_fused", "decode_qkv_attn"])
+def test_a_callers_own_step_is_called(name, b, where, monkeypatch):
+    """A layer's step, or its attention's, that a caller has overridden takes
+    batches of every size, by the call that it knows."""
+    cfg = LlamaConfig.tiny()
+    m = quantize(build_model(cfg, seed=3), QuantConfig(
+        scheme="rtn", bits=8, group_size=64, fold_rms=True))
+    shapes_alone(m, monkeypatch)
+    layer, calls = m.layers[1], []
+    on = layer if name == "forward_decode_fused" else layer.self_attn
+    old = getattr(type(on), name)
+
+    def own(self, x, cache_k, cache_v, state, max_seq, *more):
+        assert len(more) <= 2
+        calls.append(x.shape[0])
+        return old(self, x, cache_k, cache_v, state, max_seq, *more)
+
+    if where == "class":
+        on.__class__ = type("Own", (type(on),), {name: own})
+    else:
+        setattr(on, name, types.MethodType(own, on))
+    step(m, b)
+    assert m._fused_decode and calls == [b]
