@@ -53,8 +53,7 @@ enum Way { DIRECT, WHOLE, CACHED };
 
 template <Way WAY>
 __global__ __launch_bounds__(TPB, WAY == DIRECT ? 1 : 2) void hessian_kernel(
-    const unsigned short* __restrict__ x, float* __restrict__ h, int t,
-    int k) {
+    const unsigned short* __restrict__ x, float* h, int t, int k) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   // block (bi, bj) of the lower triangle, tile (r, c) of it
   const u32 id = xcd_swizzle(blockIdx.x, gridDim.x);
@@ -169,7 +168,11 @@ __global__ __launch_bounds__(TPB, WAY == DIRECT ? 1 : 2) void hessian_kernel(
       stage(t0 + BK, par ^ 1);
       products(par);
     }
+    // counted: what comes between the stage's loads and the wait is these NF (h is
+    // not __restrict__, so that the waits' memory clobbers hold for them as well)
+    __builtin_amdgcn_sched_barrier(0);
     fours_load(own, i0, j0);
+    __builtin_amdgcn_sched_barrier(0);
     loads_but<NF>();
     clear(end, par);
     products(par);
