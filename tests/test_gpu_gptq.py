@@ -135,8 +135,9 @@ def test_all_columns_are_block_by_block(n, k, g, bits, sym):
     carries them on: bit by bit what a launch each leaves."""
     gen = torch.Generator(DEV).manual_seed(n)
     w = torch.randn(n, k, generator=gen, device=DEV)
-    w[0] *= 1e-39                          # quotients that need divisions
-    w[n // 2, 3] = float("inf")
+    if n > 1:
+        w[0] *= 1e-39                      # quotients that need divisions
+        w[n // 2, 3] = float("inf")
     u = torch.randn(k, k, generator=gen, device=DEV).triu_() * 0.05
     u.diagonal().copy_(torch.rand(k, generator=gen, device=DEV) + 0.5)
 
@@ -154,7 +155,7 @@ def test_all_columns_are_block_by_block(n, k, g, bits, sym):
         if i2 < k:
             ext().gptq_push(w, err, u, i1)
     finite = torch.isfinite(want[1]).all(1)
-    assert int(finite.sum()) >= n - 1
+    assert int(finite.sum()) == max(n - 1, 1)
     for a, b in zip(got, want):
         assert torch.equal(a[finite], b[finite])
 
