@@ -44,10 +44,6 @@ constexpr int NB = 64, TPB = 256, LD = NB + 4;
 __device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ float lane_value(float v, int lane) {
-  return __builtin_bit_cast(
-      float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
-}
 
 struct Diag {
   float a[NB][LD];           // the block; its lower blocks of 16 become L's

@@ -89,16 +89,6 @@ def _inverse_factor(h: torch.Tensor) -> torch.Tensor:
 GPU_BLOCK = 128        # widest block of the HIP kernel: its U fits in LDS
 
 
-def _gpu_block(w, ub, codes, scales, zeros, i1, cfg, g) -> torch.Tensor:
-    """_block in one launch (csrc/gptq_block.hip), the same bit by bit."""
-    from ..ops import hip_ext
-    if ub.stride(1) != 1:
-        ub = ub.contiguous()
-    with torch.cuda.device(w.device):
-        return hip_ext().gptq_block(w, ub, codes, scales, zeros, i1, g,
-                                    cfg.bits, cfg.sym)
-
-
 def _gpu_layer(w, h, cfg, g):
     """gptq_quantize_layer in the HIP kernels, which leave w and h as they
     are; the host waits for one number while the columns run."""

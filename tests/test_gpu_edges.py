@@ -322,6 +322,8 @@ def test_gptq_block_of_numbers_below_the_normal_range(tiny):
     the normal range: still the tensor loop's quotients."""
     from lfmq import QuantConfig
     from lfmq.quant import gptq
+
+    from gptq_util import gpu_block
     torch.manual_seed(5)
     n, k, g = 40, 128, 64
     w = torch.randn(n, k, device=DEV)
@@ -341,7 +343,7 @@ def test_gptq_block_of_numbers_below_the_normal_range(tiny):
                torch.zeros(n, k // g, dtype=torch.int32, device=DEV))
         return (*out, f(w, u, *out, 0, cfg, g))
 
-    for got, want in zip(solve(gptq._gpu_block), solve(gptq._block)):
+    for got, want in zip(solve(gpu_block), solve(gptq._block)):
         assert torch.equal(got, want)
 
 

@@ -6,7 +6,9 @@ import torch
 
 from lfmq import QuantConfig
 from lfmq.ops import hip_ext as ext
-from lfmq.quant.gptq import _block, _gpu_block
+from lfmq.quant.gptq import _block
+
+from gptq_util import gpu_block
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -24,7 +26,7 @@ def test_block_is_the_tensor_loop(n, k, nb, i1, g):
     u = torch.randn(k, k, device=DEV).mul_(0.1).triu_()
     u.diagonal().uniform_(0.5, 2.0)
     got = []
-    for fn in (_block, _gpu_block):
+    for fn in (_block, gpu_block):
         out = [torch.zeros(n, k, dtype=torch.int32, device=DEV),
                torch.full((n, k // g), 0.4, device=DEV),
                torch.full((n, k // g), 5, dtype=torch.int32, device=DEV)]
@@ -151,7 +153,7 @@ def test_all_columns_are_block_by_block(n, k, g, bits, sym):
     cfg = QuantConfig(scheme="gptq", bits=bits, group_size=g, sym=sym)
     for i1 in range(0, k, 128):
         i2 = min(i1 + 128, k)
-        err = _gpu_block(w, u[i1:i2, i1:i2], *want, i1, cfg, g)
+        err = gpu_block(w, u[i1:i2, i1:i2], *want, i1, cfg, g)
         if i2 < k:
             ext().gptq_push(w, err, u, i1)
     finite = torch.isfinite(want[1]).all(1)

@@ -476,7 +476,9 @@ def test_gptq_block_is_the_tensor_loop(n, k, nb, i1, g, bits, sym):
     """Bit by bit: partial blocks, groups longer and shorter than a block,
     an all-zero group, a row that is not finite."""
     from lfmq import QuantConfig
-    from lfmq.quant.gptq import _block, _gpu_block
+    from lfmq.quant.gptq import _block
+
+    from gptq_util import gpu_block
     torch.manual_seed(n + k)
     cfg = QuantConfig(scheme="gptq", bits=bits, group_size=g, sym=sym)
     w = torch.randn(n, k, device=DEV)
@@ -486,7 +488,7 @@ def test_gptq_block_is_the_tensor_loop(n, k, nb, i1, g, bits, sym):
     ub = torch.randn(nb, nb, device=DEV).mul_(0.1).triu_()
     ub.diagonal().uniform_(0.5, 2.0)
     got = []
-    for fn in (_block, _gpu_block):
+    for fn in (_block, gpu_block):
         out = [torch.zeros(n, k, dtype=torch.int32, device=DEV),
                torch.full((n, k // g), 0.4, device=DEV),
                torch.full((n, k // g), 5, dtype=torch.int32, device=DEV)]
