@@ -255,8 +255,9 @@ def prompt_layer(h, residual, k_cache, v_cache, positions, pos0: int, hq: int,
         packed += (b["qweight"], b["scales"], b["qzeros"])
         forms += (p.bits, p.group_size)
     qkv, o, _, down = products
+    # (contiguous: a caller's own norm may lay its rows out otherwise)
     return hip_ext().prompt_layer(
-        h, residual, k_cache, v_cache, positions,
+        h.contiguous(), residual, k_cache, v_cache, positions,
         _inv_freq(k_cache.shape[-1], theta, h.device), hq, pos0, scale, packed,
         forms, [qkv.bias, o.bias, down.bias], post_norm.weight, post_norm.eps,
         next_norm.weight, next_norm.eps)

@@ -382,3 +382,26 @@ def test_prompts_that_do_not_fit_write_nothing(one_call, past, s, given,
             m(ids, c, pos)
             assert bool((c.k_all[..., :past, :] == 7).all())
             assert c.seq_len == past + s
+
+
+def test_normed_input_in_another_layout():
+    """A caller's own norm may leave tokens before sequences in memory."""
+    cfg = LlamaConfig(vocab_size=512, hidden_size=512, intermediate_size=1024,
+                      n_layers=2, n_heads=4, n_kv_heads=2, head_dim=128,
+                      max_seq=64)
+    m = lfmq.quantize(lfmq.build_model(cfg, seed=7), lfmq.QuantConfig(
+        scheme="rtn", bits=8, group_size=64)).to(DEV)
+    ids = torch.randint(0, 512, (2, 40), device=DEV)
+
+    class Norm(torch.nn.Module):
+        def __init__(self, of):
+            super().__init__()
+            self.of, self.weight, self.eps = of, of.weight, of.eps
+
+        def forward(self, x):
+            return self.of(x).transpose(0, 1).contiguous().transpose(0, 1)
+
+    with torch.no_grad():
+        want = m(ids, m.make_cache(2, 64))
+        m.layers[0].input_layernorm = Norm(m.layers[0].input_layernorm)
+        assert torch.equal(m(ids, m.make_cache(2, 64)), want)
