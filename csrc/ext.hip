@@ -300,15 +300,22 @@ bool short_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
 }
 
 // The product of 8 bits whose workgroups share k among eight waves (dq_mid): where
-// it is faster than dq_short, dq_rows, dq_tile and dq_block.  Of 437 random shapes of
-// 17 to 128 rows, 3 to 120 million weights, this takes 180, whose time before / now is
-// 1.24 in the mean and 0.95 to 1.65.  Long k
+// it is faster than dq_short, dq_rows, dq_tile and dq_block.  Long k
 // pays where the columns are few, so that parts of it fill the chip: n 4096, k 4096
 // 20.6 / 15.2 us at 96 rows, n 2048, k 8192 18.2 / 14.9 at 61; n 20480, k 4096 35.3 /
 // 39.2 at 50.  A gate has no parts: n 6144, k 8192 24.0 / 34.3 at 54.  Above 96 rows
 // there are two tiles of them, and many columns are read twice: n 28672, k 2048 34.2 /
 // 41.8 at 109, n 6144, k 8192 33.2 / 41.6 at 110; 16384 to 28672 columns leave a
-// third of the chip (n 20480, k 2560 24.6 / 27.5 at 40).  Few rows of few columns are dq_rows': n 4096, k 1024 6.4 / 7.7 at 36.
+// third of the chip (n 20480, k 2560 24.6 / 27.5 at 40).  Few rows of few columns are
+// dq_rows': n 4096, k 1024 6.4 / 7.7 at 36; and up to 32 rows of 6144 to 8192 columns,
+// 192 to 256 of its workgroups: n 8192, k 2048 9.8 / 12.1 at 17, 10.7 / 12.2 at 24, n
+// 7680, k 768 6.6 / 8.1 at 25.  49 to 64 rows of short k are dq_short's from 28672
+// columns on (n 34816, k 1024 22.1 / 29.2 at 60).  From 32769 columns on a second
+// round begins, and what is left over these lines is what gains there (n 36864, k
+// 1024, gate 21.1 / 23.9 at 18 rows; n 33088, k 960 29.4 / 33.3 at 83).
+// Of 5785 random calls of 17 to 128 rows, 768 to 40000 columns, k 768 to 10000, groups
+// of 64 to 256, that all but the last three lines take: 1.19 times as fast in the mean,
+// 6 % of them slower by more than 4 %; with these lines 2.3 % (2.5 % of 1997 others).
 bool mid_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
               long bits, bool glu) {
   if (bits != 8 || m <= 16 || m > 128 || n <= 0 || n % 8 ||
@@ -322,7 +329,7 @@ bool mid_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
   else if (m > 96 && n > (k <= 3072 ? 8192 : 3072))
     gains = false;
   else if (k <= 3072 && n > 16384 && n < 28672)
-    gains = m > 64 || (m <= 48 && k <= 2048);
+    gains = m > 64 ? k <= 2048 || n > 24576 : m <= 48 && k <= 2048;
   else if (k <= 3072)
     gains = m <= 48 ? n >= 5120 && (m > 24 || n * k >= 16l << 20)
                     : n * k >= 3l << 20;
@@ -331,6 +338,14 @@ bool mid_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
             (k <= 8192 || g == 64);
   else
     gains = m > 48 && k <= 4096 && n >= 10240 && n <= 16384;
+  if (n > 32768)
+    gains = gains && (m <= 32   ? !glu && (g > 64 || k > 2048)
+                      : m <= 48 ? k < 1280 || (!glu && g > 64)
+                                : m > 64 && k >= 1536 && (glu || k <= 2560));
+  else if (m <= 32)
+    gains = gains && (glu || n < 6144 || n > 8192);
+  else if (m > 48 && m <= 64)
+    gains = gains && (n < 28672 || k > 2048);
   return gains &&
          lfmq_dq_mid_plan((int)m, (int)n, (int)k, (int)g, glu).mb > 0;
 }

@@ -305,3 +305,15 @@ def test_eight_waves_along_k(m, n, k, g):
         y, _ = ext().dq_linear_scaled(x, scale, *p, 8, g, None, resid, 1e-5)
         close(y, want + resid.double())
         close(ext().dq_gateup_scaled(x, scale, *p, 8, g), gated(want), 1e-2)
+
+
+@pytest.mark.parametrize("m,n,k,g", [
+    (32, 6136, 1024, 64), (32, 6144, 1024, 64), (25, 8192, 768, 128),
+    (25, 8200, 768, 128), (17, 8192, 2048, 64), (17, 8200, 2048, 64),
+    (64, 28664, 1024, 64), (64, 28672, 1024, 64), (50, 28672, 2112, 64),
+    (96, 24576, 2112, 64), (65, 24584, 2112, 64), (32, 32768, 512, 64),
+    (32, 32776, 512, 64), (32, 32776, 512, 128), (48, 32776, 1216, 64),
+    (33, 32776, 1280, 64), (65, 32776, 1472, 64), (65, 32776, 1536, 64)])
+def test_eight_waves_at_the_lines(m, n, k, g):
+    """On both sides of the lines where other products are the faster ones."""
+    test_eight_waves_along_k(m, n, k, g)
