@@ -20,7 +20,8 @@
 // read by its panel only.  Products are fp32 matrix instructions fed from
 // global memory (L2): a lane's 16 values of k lie side by side.
 //
-// Bound by the chain of the diagonal blocks, 15 us a step at n 2048: 4 from the
+// Bound by the chain of the diagonal blocks, 15 us a step at n 2048 as clocks within
+// count it, 14.2 timed: 4 from the
 // end of a launch to the next one's first workgroup, 2.5 until its panel's
 // operands are there (other XCDs wrote them), 2 of products, 6.5 of factor and
 // inverse; from 8192 on by the traffic of M.  In the factor every wave carries

@@ -16,7 +16,7 @@
 // at 4.8 TB/s; the products of 2048 x 14336 alone: 465), and the two overlap
 // only as far as a workgroup's loads are under way before it needs them and
 // leave X in the L2.  So elements of the tile's own place load beside the last
-// two steps, those of the mirror while the result goes through LDS, and H
+// step, those of the mirror while the result goes through LDS, and H
 // passes by the caches where its rows are whole lines.  2048 x 14336: 673 us
 // with H read after the products, 629 with loads ahead, 545 past the caches
 // too (772 TFLOP/s of the half computed); 512 x 8192: 122 and 100;

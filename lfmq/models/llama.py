@@ -337,7 +337,8 @@ class LlamaDecoderLayer(nn.Module):
         h, eps = x, self.post_attention_layernorm.eps
         if x.shape[0] > 32 and gp.in_features >= 4096 and \
                 gp.in_features * gp.out_features >= 24 << 20:
-            # (layers of several ranks; others by forward_decode_rows)
+            # (several ranks, steps of a caller's own; others by
+            # forward_decode_rows)
             # the product for prompts, which takes normed rows, is faster
             # (28672 x 4096 at 48 rows: 41 us with its norm, 50)
             h, eps = self.post_attention_layernorm(x), -1.0
