@@ -408,28 +408,7 @@ __device__ __forceinline__ void dq_block_body(const DqArgs& A, char* smem,
       }
   }
   __syncthreads();
-  const bool wide = nout % 8 == 0;
-  for (int i = tid; i < BM * BO / 8; i += TPB) {
-    const int row = i / (BO / 8), c = i % (BO / 8) * 8;
-    const int gc0 = n0 + c;
-    if (row >= rows || gc0 >= nout) continue;
-    unsigned short* p = A.y + (u64)(row0 + row) * nout + gc0;
-    const unsigned short* q = out + row * LD + c;
-    if (wide) {
-      *(u32x4*)p = *(const u32x4*)q;
-    } else {
-      for (int e = 0; e < 8 && gc0 + e < nout; ++e) p[e] = q[e];
-    }
-  }
-}
-
-// row tile and column block of a tile: bands of 8 row tiles, row tiles fastest
-__device__ __forceinline__ void place(u32 id, int mb, u32 nb, int& mt,
-                                      int& nblk) {
-  const u32 band = id / (8 * nb), in = id - band * 8 * nb;
-  const u32 w = min(8u, (u32)mb - band * 8);
-  mt = band * 8 + in % w;
-  nblk = in / w;
+  dq_block_store(out, LD, BM, BO, A.y, row0, rows, n0, nout, tid, TPB);
 }
 
 template <int BITS, int KC, DqMode MODE>
@@ -437,34 +416,11 @@ __global__ __launch_bounds__(TPB, 2) void dq_block_kernel(DqArgs A, Plan P) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const u32 nb = MODE == GLU ? (A.n / 2 + BN / 2 - 1) / (BN / 2)
                              : (A.n + BN - 1) / BN;
-  int mt, nblk, sp = 0, parts = 1, expert = 0, row0, rows;
-  float* part = nullptr;
-  if (MODE != DENSE && A.tiles != nullptr) {
-    nblk = blockIdx.x % nb;
-    mt = blockIdx.x / nb;
-    expert = A.tiles[3 * mt];
-    if (expert < 0) return;
-    row0 = A.tiles[3 * mt + 1];
-    rows = A.tiles[3 * mt + 2];
-    if (MODE == SLOTS) {
-      sp = blockIdx.y;
-      parts = P.parts;
-      A.y32 += (u64)sp * P.part;
-    }
-  } else {
-    u32 id = blockIdx.x;
-    if ((int)id < P.full) {
-      id = xcd_swizzle(id, P.full);
-    } else {
-      parts = P.parts;
-      part = A.part + (u64)(id - P.full) * (P.step * BN);
-      sp = (id - P.full) % parts;
-      id = P.full + (id - P.full) / parts;
-    }
-    place(id, P.mb, nb, mt, nblk);
-    row0 = mt * P.step;
-    rows = min(A.m - row0, P.step);
-  }
+  DqBlockTile T;
+  if (!dq_block_tile<MODE>(A, P, nb, BN, T)) return;
+  const int nblk = T.nblk, sp = T.sp, parts = T.parts, expert = T.expert;
+  const int row0 = T.row0, rows = T.rows;
+  float* part = T.part;
   if (rows > 96)
     dq_block_body<BITS, KC, MODE, 8>(A, smem, row0, rows, expert, nblk, sp,
                                      parts, part);
@@ -489,7 +445,7 @@ __global__ __launch_bounds__(256) void dq_block_sum(DqArgs A, Plan P) {
   const u32 nb = MODE == GLU ? (A.n / 2 + BN / 2 - 1) / (BN / 2)
                              : (A.n + BN - 1) / BN;
   int mt, nblk;
-  place(P.full + blockIdx.x, P.mb, nb, mt, nblk);
+  dq_block_place(P.full + blockIdx.x, P.mb, nb, mt, nblk);
   const int row0 = mt * P.step, rows = min(A.m - row0, P.step);
   const int nout = MODE == GLU ? A.n / 2 : A.n;
   constexpr int BO = MODE == GLU ? BN / 2 : BN, Q = BO / 4;
@@ -604,8 +560,8 @@ DqBlockPlan lfmq_dq_block_plan(int m, int n, int k, int g, int bits, bool glu) {
 
 hipError_t lfmq_dq_block(const void* qweight, const void* scales,
                          const void* qzeros, const void* x, void* y,
-                         const void* bias, void* part, int m, int n, int k,
-                         int g, int bits, bool glu, const DqBlockPlan& P,
+                         const void* bias, void* part, void* sums, int m, int n,
+                         int k, int g, int bits, bool glu, const DqBlockPlan& P,
                          hipStream_t stream) {
   if (!lfmq_dq_block_ok(qweight, scales, n, k, g, bits) || m < 1 ||
       (glu && (n % 2 || bias != nullptr || (u64)m * k * 2 >= 1ull << 32)))
@@ -617,8 +573,11 @@ hipError_t lfmq_dq_block(const void* qweight, const void* scales,
   const int rest = P.mb * column_blocks(n, glu) - P.full;
   if (rest > 0 && part == nullptr) return hipErrorInvalidValue;
   const u32 wgs = P.full + rest * P.parts;
-  const hipError_t e = glu ? go_bits<GLU>(A, P, bits, wgs, stream)
-                           : go_bits<DENSE>(A, P, bits, wgs, stream);
+  const hipError_t e =
+      sums != nullptr
+          ? lfmq_dq_panel(A, P, bits, glu ? GLU : DENSE, wgs, sums, m, stream)
+      : glu ? go_bits<GLU>(A, P, bits, wgs, stream)
+            : go_bits<DENSE>(A, P, bits, wgs, stream);
   if (e != hipSuccess || rest == 0) return e;
   if (glu)
     hipLaunchKernelGGL(dq_block_sum<GLU>, dim3(rest, ceil_div_u32(P.step, 8)),
@@ -652,9 +611,9 @@ int lfmq_dq_block_slot_parts(long slots, long E, int n, int k, int g,
 hipError_t lfmq_dq_block_experts(const void* qweight, const void* scales,
                                  const void* qzeros, const void* x,
                                  const void* src, const void* tiles, void* y,
-                                 void* part, int n_tiles, int n, int k, int g,
-                                 int bits, bool glu, int parts, long slots,
-                                 hipStream_t stream) {
+                                 void* part, void* sums, long rows, int n_tiles,
+                                 int n, int k, int g, int bits, bool glu,
+                                 int parts, long slots, hipStream_t stream) {
   if (!lfmq_dq_block_ok(qweight, scales, n, k, g, bits) || (glu && n % 2) ||
       parts < 1 ||
       (parts > 1 && (glu || part == nullptr || n % 4 || slots < 1 ||
@@ -677,8 +636,11 @@ hipError_t lfmq_dq_block_experts(const void* qweight, const void* scales,
   Plan P{};
   P.parts = parts;
   P.part = slots * n;
-  if (glu) return go_bits<GLU>(A, P, bits, wgs, stream);
-  const hipError_t e = go_bits<SLOTS>(A, P, bits, wgs, stream);
+  const hipError_t e =
+      sums != nullptr
+          ? lfmq_dq_panel(A, P, bits, glu ? GLU : SLOTS, wgs, sums, rows, stream)
+      : glu ? go_bits<GLU>(A, P, bits, wgs, stream)
+            : go_bits<SLOTS>(A, P, bits, wgs, stream);
   if (e != hipSuccess || parts == 1) return e;
   const u32 n4 = (u32)(slots * n / 4);
   hipLaunchKernelGGL(dq_block_sum_slots, dim3(ceil_div_u32(n4, 256)), dim3(256),

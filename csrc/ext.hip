@@ -239,6 +239,14 @@ bool block_rows(const torch::Tensor& qweight, const torch::Tensor& scales,
                                    g, bits);
 }
 
+// room for the sums of x's groups, where a product of `rows` rows gains by them
+torch::Tensor panel_sums(const torch::Tensor& x, long rows, long n, long g,
+                         long bits) {
+  const long k = x.size(1), groups = x.size(0) * (k / g);
+  if (!lfmq_dq_panel_gains(rows, n, k, g, bits) || groups * 8 >= 1l << 32) return {};
+  return torch::empty({groups}, x.options().dtype(torch::kInt64));
+}
+
 void dq_block(const torch::Tensor& x, const torch::Tensor& qweight,
               const torch::Tensor& scales, const torch::Tensor& qzeros,
               const void* bias, torch::Tensor& y, long g, long bits, bool glu) {
@@ -248,9 +256,11 @@ void dq_block(const torch::Tensor& x, const torch::Tensor& qweight,
   torch::Tensor part;
   if (P.part > 0)
     part = torch::empty({P.part}, x.options().dtype(torch::kFloat32));
+  const torch::Tensor sums = panel_sums(x, m, n, g, bits);
   CHECK_HIP(lfmq_dq_block(qweight.data_ptr(), scales.data_ptr(),
                           qzeros.data_ptr(), x.data_ptr(), y.data_ptr(), bias,
-                          P.part > 0 ? part.data_ptr() : nullptr, m, n, k,
+                          P.part > 0 ? part.data_ptr() : nullptr,
+                          sums.defined() ? sums.data_ptr() : nullptr, m, n, k,
                           (int)g, (int)bits, glu, P, stream()));
 }
 
@@ -1157,13 +1167,15 @@ torch::Tensor moe_linear(torch::Tensor x, c10::optional<torch::Tensor> src,
   if (nt == 0) return y;
   torch::Tensor part;
   if (parts > 1) part = torch::empty({parts * slots, (long)n}, f32);
-  if (block)
+  if (block) {
+    const torch::Tensor sums = panel_sums(x, slots, n, g, bits);
     CHECK_HIP(lfmq_dq_block_experts(
         qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
         sptr, tiles.data_ptr(), y.data_ptr(),
-        parts > 1 ? part.data_ptr() : nullptr, nt, n, k, (int)g, (int)bits, glu,
-        parts, slots, stream()));
-  else if (bm == 128)
+        parts > 1 ? part.data_ptr() : nullptr,
+        sums.defined() ? sums.data_ptr() : nullptr, x.size(0), nt, n, k, (int)g,
+        (int)bits, glu, parts, slots, stream()));
+  } else if (bm == 128)
     CHECK_HIP(lfmq_dq_tile_experts(
         qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
         sptr, tiles.data_ptr(), y.data_ptr(), nt, n, k, (int)g, (int)bits, glu,

@@ -31,12 +31,16 @@ __device__ __forceinline__ void loads_but() {
                : "memory");
 }
 
-// Swizzle of rows of 4, 8 or 16 16-byte slots: the slots of 16 consecutive
-// rows at one column fall into different banks.
+// Swizzle of rows of 2, 4, 8 or 16 16-byte slots: the slots of 16 consecutive
+// rows at one column fall into different banks, and so do those of the two halves
+// of 32 rows that a 16-byte read of a row a lane takes together (below).
 template <int SLOTS>
 __device__ __forceinline__ int slot_key(int row) {
-  static_assert(SLOTS == 4 || SLOTS == 8 || SLOTS == 16, "");
-  return SLOTS == 16 ? row & 15 : (SLOTS == 8 ? (row >> 1) & 7 : (row >> 2) & 3);
+  static_assert(SLOTS == 2 || SLOTS == 4 || SLOTS == 8 || SLOTS == 16, "");
+  return SLOTS == 16  ? row & 15
+         : SLOTS == 8 ? (row >> 1) & 7
+         : SLOTS == 4 ? (row >> 2) & 3
+                      : (row >> 3) & 1;
 }
 
 // Swizzle of rows of 4, 8 or 16 16-byte slots for reads of 16 bytes where lane

@@ -35,6 +35,7 @@ SOURCES = [
     "csrc/dq_rows.hip",
     "csrc/dq_tile.hip",
     "csrc/dq_block.hip",
+    "csrc/dq_panel.hip",
     "csrc/dq_short.hip",
     "csrc/dq_mid.hip",
     "csrc/hessian.hip",

@@ -33,9 +33,21 @@ def test_many_rows(bits, m, n, k, g):
               1e-2)
 
 
-# dq_wide, dq_short (k whole, and in parts) and dq_block
+# What is large enough for dq_panel: row tiles of 64 to 128; columns that end inside
+# a wave's; sums of 16 to 108 groups, 32 at a time; several chunks a group; some tiles
+# split, the groups of a part then as they fall.
+@pytest.mark.parametrize("bits,m,n,k,g", [
+    (4, 1100, 8450, 2048, 128), (4, 130, 20002, 6144, 128), (4, 60, 28674, 9216, 128),
+    (4, 150, 16390, 8192, 512), (4, 2100, 4352, 3072, 128), (8, 140, 16390, 4608, 64),
+    (4, 140, 16391, 4608, 64), (8, 300, 9030, 8192, 128), (8, 700, 4100, 6912, 64)])
+def test_many_rows_of_large_products(bits, m, n, k, g):
+    test_many_rows(bits, m, n, k, g)
+
+
+# dq_wide, dq_short (k whole, and in parts), dq_block and dq_panel
 @pytest.mark.parametrize("m,n,k", [(8, 8200, 2048), (40, 4104, 4096),
-                                   (100, 4104, 2048), (200, 512, 4096)])
+                                   (100, 4104, 2048), (200, 512, 4096),
+                                   (300, 8200, 8192)])
 def test_values_that_are_not_finite_stay_in_their_rows(m, n, k):
     torch.manual_seed(0)
     p, w = matrix(4, n, k, 128)
@@ -50,7 +62,10 @@ def test_values_that_are_not_finite_stay_in_their_rows(m, n, k):
 @pytest.mark.parametrize("bits,n,k,g", [(4, 2062, 2048, 128),
                                         (8, 1040, 1024, 64),
                                         (4, 516, 1536, 64),
-                                        (4, 260, 2560, 64)])
+                                        (4, 260, 2560, 64),
+                                        # dq_panel: whole, and in two parts
+                                        (4, 6162, 5120, 128),
+                                        (8, 4096, 7168, 64)])
 def test_many_rows_by_expert(bits, n, k, g):
     """One to 128 rows a tile, experts without any, tiles that are none; k whole
     (n not in fours), in two and in four parts."""
