@@ -27,19 +27,59 @@
 // tiles whose sums are taken during the next batch: registers spill, 20 % slower.
 // (Groups of 64 with k above 4096 spill 2 to 20 registers: ext.hip's rules were
 // measured with that.)
+//
+// Where k is longer than a workgroup's 4096, it may also be shared by workgroups of
+// which the last one to end adds up: a merge by way of memory costs 2 to 3 us, one
+// part after the other of a tile more from some 50 million weights on.  us a call,
+// dq_rows or several steps a workgroup, and in parts (4 bits; 5120 x 17408 of 8 bits):
+//                                   3 rows       8 rows       16 rows
+//   n 4096, k 14336               13.6 / 13.5  16.4 / 14.4  18.7 / 15.7
+//   n 6144, k 8192                12.3 / 11.2  13.9 / 12.2  16.7 / 13.4
+//   n 5120, k 17408               26.1 / 19.0  33.3 / 20.3  27.3 / 21.7
+//   n 5120, k 17408 (8 bits)      37.6 / 25.3  45.5 / 26.4  35.5 / 28.0
 #include "dq_frag.h"
+
+int lfmq_dq_wide_part_blocks(int n, int parts);
 
 namespace {
 
 constexpr int KS = 256;                  // values of k of a wave and step
 constexpr int MAX_TILES = 8;             // of a workgroup
+constexpr int MOST_PARTS = 5;            // of k
 
 struct Wide {
   DqArgs A;
   int q, r;                              // tiles of a workgroup: q, or q + 1
                                          // of the first r
   int G, zw, steps;                      // groups, words of zeros; steps of k
+  u32* tickets;                          // PARTS: a counter a workgroup, zero
 };
+
+// A partial result, past the caches of the XCD: a workgroup of another one may be
+// the reader.
+__device__ __forceinline__ void put4(float* p, f32x4 v) {
+  typedef __attribute__((address_space(1))) u64 gu64;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float a = v[2 * i], b = v[2 * i + 1];
+    __hip_atomic_store((gu64*)p + i,
+                       (u64)__builtin_bit_cast(u32, b) << 32 |
+                           __builtin_bit_cast(u32, a),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+__device__ __forceinline__ f32x4 get4(const float* p) {
+  typedef __attribute__((address_space(1))) u64 gu64;
+  f32x4 v;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const u64 b = __hip_atomic_load((gu64*)p + i, __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT);
+    v[2 * i] = __builtin_bit_cast(float, (u32)b);
+    v[2 * i + 1] = __builtin_bit_cast(float, (u32)(b >> 32));
+  }
+  return v;
+}
 
 __host__ __device__ __forceinline__ int lanes_of(int rows) {
   return rows <= 4 ? 16 : (rows <= 8 ? 32 : 64);
@@ -47,8 +87,9 @@ __host__ __device__ __forceinline__ int lanes_of(int rows) {
 
 // MORE: more than one step of k.  LINES: a load takes a whole 128-byte line of eight
 // rows of W, past the caches: pieces of two chunks (PAIR), or the halves of one;
-// lanes of the two eights exchange theirs on the way into the operands.
-template <int BITS, int KC, DqMode MODE, bool MORE, int NW, bool LINES>
+// lanes of the two eights exchange theirs on the way into the operands.  PARTS: k is
+// shared by A.splits workgroups, of which the last one to end adds up.
+template <int BITS, int KC, DqMode MODE, bool MORE, int NW, bool LINES, bool PARTS>
 __global__ __launch_bounds__(NW * 64, 4) void dq_wide_kernel(Wide W) {
   const DqArgs& A = W.A;
   constexpr int TPB = NW * 64;
@@ -66,7 +107,11 @@ __global__ __launch_bounds__(NW * 64, 4) void dq_wide_kernel(Wide W) {
     rows = A.tiles[3 * blockIdx.y + 2];
   }
   const bool rms = MODE != SLOTS && A.rms_eps >= 0.f;
-  const int nout = A.n / H, G = W.G, zw = W.zw, C = A.k / KC;
+  const int nout = A.n / H, G = W.G, zw = W.zw;
+  // (parts end with a line, two chunks)
+  const int c0 = PARTS ? A.k / KC / 2 * (int)blockIdx.y / A.splits * 2 : 0;
+  const int C = PARTS ? A.k / KC / 2 * (int)(blockIdx.y + 1) / A.splits * 2
+                      : A.k / KC;
   const int bi = blockIdx.x, ta = bi * W.q + min(bi, W.r);
   const int nt = W.q + (bi < W.r ? 1 : 0);
   // rows of W of this workgroup: r0 .. (GLU: of either half)
@@ -101,7 +146,7 @@ __global__ __launch_bounds__(NW * 64, 4) void dq_wide_kernel(Wide W) {
   static_assert(!LINES || PAIR || HALVES, "");
   constexpr int XP = HALVES ? 16 : KC / 4;         // values of x in a piece
   const char* xp = (const char*)A.x + ((u64)xr * A.k + l4 * XP) * 2;
-  auto chunk = [&](int p) { return (p * NW + wave) * S; };
+  auto chunk = [&](int p) { return c0 + (p * NW + wave) * S; };
   s16x8 xq[S][J];
   auto fetch_x = [&](int p) {
 #pragma unroll
@@ -237,7 +282,7 @@ __global__ __launch_bounds__(NW * 64, 4) void dq_wide_kernel(Wide W) {
   }
   __syncthreads();
   // a wave a tile: column l15, rows l4 * 4 + e
-  if (wave >= nt) return;
+  if (!PARTS && wave >= nt) return;
   float inv = 1.f;                                       // of row l15
   if (rms) {
     float v = 0.f;
@@ -247,9 +292,39 @@ __global__ __launch_bounds__(NW * 64, 4) void dq_wide_kernel(Wide W) {
   }
   const int t = wave;
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
-  if (lane < lanes) {
+  if (lane < lanes && (!PARTS || t < nt)) {
 #pragma unroll
     for (int i = 0; i < NW; ++i) v += red[(t * NW + i) * lanes + lane];
+  }
+  if constexpr (PARTS) {
+    // As the decode attention's merge: results are written through to where the
+    // workgroup that adds up reads, every wave waits for its own, and the barrier
+    // stands before the ticket, which is put back to zero.
+    float* part = A.part + ((u64)(ta + t) * A.splits * 64 + lane) * 4;
+    if (t < nt && lane < lanes) put4(part + blockIdx.y * 256, v);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int* last_s = (int*)smem;              // (scales, read)
+    typedef __attribute__((address_space(1))) unsigned gu32;
+    gu32* ticket = (gu32*)(W.tickets + blockIdx.x);
+    if (tid == 0) {
+      const unsigned old = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT);
+      *last_s = (int)old == A.splits - 1;
+      if (*last_s)
+        __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!*last_s || t >= nt) return;
+    f32x4 all[MOST_PARTS];
+    const bool on = lane < lanes;
+#pragma unroll
+    for (int i = 0; i < MOST_PARTS; ++i)
+      if (i < A.splits && on) all[i] = get4(part + i * 256);
+    v = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < MOST_PARTS; ++i)
+      if (i < A.splits && on) v += all[i];
   }
   const int col = (ta + t) * TC + (H == 2 ? l15 & 7 : l15);
 #pragma unroll
@@ -312,7 +387,7 @@ hipError_t go(const DqArgs& A, int rows, int lists, hipStream_t stream) {
   }
   if (nt == 0) return hipErrorInvalidValue;
   const int grid = (int)ceil_div_u32(tiles, nt);
-  const auto kernel = dq_wide_kernel<BITS, KC, MODE, MORE, NW, LINES>;
+  const auto kernel = dq_wide_kernel<BITS, KC, MODE, MORE, NW, LINES, false>;
   static bool set = false;
   if (!set) {
     LFMQ_CHECK_HIP(hipFuncSetAttribute(
@@ -321,7 +396,7 @@ hipError_t go(const DqArgs& A, int rows, int lists, hipStream_t stream) {
     set = true;
   }
   const Wide W{A, tiles / grid, tiles % grid, G, zw,
-               (int)ceil_div_u32(A.k, NW * KS)};
+               (int)ceil_div_u32(A.k, NW * KS), nullptr};
   hipLaunchKernelGGL(kernel, dim3(grid, lists), dim3(NW * 64),
                      lds_bytes((int)ceil_div_u32(tiles, grid), rows, G, zw, NW),
                      stream, W);
@@ -350,6 +425,31 @@ hipError_t go_k(const DqArgs& A, int rows, int lists, hipStream_t stream) {
   if (A.k <= 16 * KS)
     return go<BITS, KC, MODE, false, 16>(A, rows, lists, stream);
   return go<BITS, KC, MODE, true, 16>(A, rows, lists, stream);
+}
+
+// column tiles of a workgroup where k is in parts of up to 4096: a workgroup a CU
+int part_tiles(int n, int parts) {
+  return (int)ceil_div_u32(ceil_div_u32(n, 16) * parts, 256);
+}
+
+template <int BITS, int KC>
+hipError_t go_parts(const DqArgs& A, void* tickets, hipStream_t stream) {
+  constexpr int NW = 16;
+  constexpr bool LINES = BITS * KC >= 512;
+  const int tiles = (int)ceil_div_u32(A.n, 16), G = A.k / KC, zw = words_of(G, BITS);
+  const int grid = lfmq_dq_wide_part_blocks(A.n, A.splits);
+  const size_t lds = lds_bytes((int)ceil_div_u32(tiles, grid), A.m, G, zw, NW);
+  const auto kernel = dq_wide_kernel<BITS, KC, DENSE, false, NW, LINES, true>;
+  static bool set = false;
+  if (!set) {
+    LFMQ_CHECK_HIP(hipFuncSetAttribute(
+        (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+        (int)room_of(NW)));
+    set = true;
+  }
+  const Wide W{A, tiles / grid, tiles % grid, G, zw, 1, (u32*)tickets};
+  hipLaunchKernelGGL(kernel, dim3(grid, A.splits), dim3(NW * 64), lds, stream, W);
+  return hipGetLastError();
 }
 
 template <DqMode MODE>
@@ -391,6 +491,45 @@ hipError_t lfmq_dq_wide(const void* qweight, const void* scales,
                  nullptr, nullptr, rms_eps};
   return glu ? go_bits<GLU>(A, bits, m, 1, stream)
              : go_bits<DENSE>(A, bits, m, 1, stream);
+}
+
+// Workgroups of a part of k.
+int lfmq_dq_wide_part_blocks(int n, int parts) {
+  return (int)ceil_div_u32(ceil_div_u32(n, 16), part_tiles(n, parts));
+}
+
+// Parts of k of a product that one launch does in parts; 0: it does not.
+int lfmq_dq_wide_parts(int m, int n, int k, int g, int bits) {
+  const int parts = (int)ceil_div_u32(k, 16 * KS);
+  if (parts < 2 || parts > MOST_PARTS || !lfmq_dq_wide_ok(m, n, k, g, bits)) return 0;
+  const int nt = part_tiles(n, parts), G = k / g;
+  return nt <= MAX_TILES &&
+                 lds_bytes(nt, m, G, words_of(G, bits), 16) <= room_of(16)
+             ? parts
+             : 0;
+}
+
+// as lfmq_dq_wide, without a norm; part: [n / 16, rounded up][parts][256] floats of
+// scratch memory; tickets: a zero a workgroup of a part, which no other launch uses
+// meanwhile, and zeros again afterwards
+hipError_t lfmq_dq_wide_in_parts(const void* qweight, const void* scales,
+                                 const void* qzeros, const void* x, void* y,
+                                 const void* bias, const void* resid, void* part,
+                                 void* tickets, int m, int n, int k, int g, int bits,
+                                 hipStream_t stream) {
+  const int parts = lfmq_dq_wide_parts(m, n, k, g, bits);
+  if (parts == 0 || part == nullptr || tickets == nullptr)
+    return hipErrorInvalidValue;
+  const DqArgs A{(const char*)qweight, (const unsigned short*)scales,
+                 (const u32*)qzeros, (const unsigned short*)x,
+                 (unsigned short*)y, (const unsigned short*)bias,
+                 (const unsigned short*)resid, (float*)part, m, n, k, g, parts,
+                 nullptr, nullptr, nullptr};
+  if (bits == 4)
+    return g == 128 ? go_parts<4, 128>(A, tickets, stream)
+                    : go_parts<4, 64>(A, tickets, stream);
+  return g == 128 ? go_parts<8, 128>(A, tickets, stream)
+                  : go_parts<8, 64>(A, tickets, stream);
 }
 
 // as lfmq_dq_rows_experts

@@ -28,6 +28,11 @@ bool lfmq_dq_wide_ok(int, int, int, int, int);
 hipError_t lfmq_dq_wide(const void*, const void*, const void*, const void*,
                         void*, const void*, const void*, int, int, int, int,
                         int, float, bool, hipStream_t);
+int lfmq_dq_wide_parts(int, int, int, int, int);
+int lfmq_dq_wide_part_blocks(int, int);
+hipError_t lfmq_dq_wide_in_parts(const void*, const void*, const void*, const void*,
+                                 void*, const void*, const void*, void*, void*, int,
+                                 int, int, int, int, hipStream_t);
 hipError_t lfmq_dq_wide_experts(const void*, const void*, const void*,
                                 const void*, const void*, const void*, void*,
                                 int, int, int, int, int, bool, hipStream_t);
@@ -206,6 +211,20 @@ bool wide_rows(int m, int n, int k, long g, long bits, bool glu) {
     least = bits == 8 || (more && !glu) ? 70 : 80;
   }
   return full >= least;
+}
+
+// Whether that kernel gains by k in parts, of up to 4096 each, which its last
+// workgroup adds up (dq_wide).  us of the other way / this one: n 4096, k 8192 (4 bits,
+// groups of 128) 11.4 / 10.9 at 8 rows, 13.6 / 12.1 at 16, 10.1 / 10.4 at 4; n 4096, k
+// 14336 14.2 / 13.7 at 4; n 2048, k 8192 9.9 / 10.7 at 16; n 4096, k 5120 10.9 / 12.1; n
+// 12288, k 8192 17.0 / 16.0 at 3, groups of 64 21.5 / 21.9; seven parts, n 4096, k 27648
+// 26.7 / 34.6 at 7, of few columns n 1904, k 25600 20.9 / 22.6 at 13.  Of 65 random
+// calls that it takes 1.26 times as fast in the mean.
+bool part_rows(long m, long n, long k, long g, long bits) {
+  const long size = n * k, M = 1l << 20, parts = (k + 4095) / 4096;
+  return m >= 3 && m <= 16 && n >= 2048 && k >= 8192 && parts <= 5 && size >= (m > 8 ? 32 : 48) * M &&
+         10 * k >= 7 * 4096 * parts && (bits == 8 || g != 64 || n <= 8192) &&
+         tile_addresses(n, k, bits);
 }
 
 // The product for many rows: tiles of 256 columns instead of 128, which few
@@ -573,6 +592,46 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
                         long cols_hint) {
   return linear(x, qweight, scales, qzeros, bits, g, bias, resid, rms_eps,
                 cols_hint, {});
+}
+
+// dq_linear of 2 to 16 rows whose k is in parts that one launch adds up, with
+// `tickets` (zeros before and afterwards, of nobody else meanwhile); None: it gains
+// nothing by them.
+c10::optional<torch::Tensor> dq_linear_parts(
+    torch::Tensor x, torch::Tensor qweight, torch::Tensor scales,
+    torch::Tensor qzeros, long bits, long g, c10::optional<torch::Tensor> bias,
+    c10::optional<torch::Tensor> resid, torch::Tensor tickets) {
+  check_t(x, torch::kBFloat16, "x");
+  check_t(qweight, torch::kInt32, "qweight");
+  check_t(scales, torch::kBFloat16, "scales");
+  check_t(qzeros, torch::kInt32, "qzeros");
+  check_t(tickets, torch::kInt32, "tickets");
+  TORCH_CHECK(x.dim() == 2, "x must be [m, k]");
+  TORCH_CHECK(g > 0, "groups have at least one column");
+  const long m = x.size(0), k = x.size(1), n = qweight.size(0);
+  TORCH_CHECK(qweight.size(1) == k * bits / 32, "qweight/k mismatch");
+  if (!part_rows(m, n, k, g, bits) || !in_pairs(scales) ||
+      (uintptr_t)x.data_ptr() % 16 || (uintptr_t)qweight.data_ptr() % 16)
+    return c10::nullopt;
+  const int parts = lfmq_dq_wide_parts((int)m, (int)n, (int)k, (int)g, (int)bits);
+  if (parts == 0 || tickets.numel() < lfmq_dq_wide_part_blocks((int)n, parts))
+    return c10::nullopt;
+  auto vector = [&](const c10::optional<torch::Tensor>& t, const char* name,
+                    long size) -> const void* {
+    if (!t.has_value()) return nullptr;
+    check_t(*t, torch::kBFloat16, name);
+    TORCH_CHECK(t->numel() == size, name, " has another size");
+    return t->data_ptr();
+  };
+  const void* b = vector(bias, "bias", n);
+  const void* r = vector(resid, "resid", m * n);
+  auto y = torch::empty({m, n}, x.options());
+  auto part = torch::empty({(n + 15) / 16 * parts * 256}, x.options().dtype(torch::kFloat32));
+  CHECK_HIP(lfmq_dq_wide_in_parts(
+      qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
+      y.data_ptr(), b, r, part.data_ptr(), tickets.data_ptr(), (int)m, (int)n, (int)k,
+      (int)g, (int)bits, stream()));
+  return y;
 }
 
 // 1 / sqrt(mean x^2 + eps) of each row, fp32
@@ -1508,6 +1567,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("pack", &pack, "pack int codes");
   m.def("unpack", &unpack, "unpack int codes");
   m.def("dq_linear", &dq_linear, "fused dequant GEMV/GEMM");
+  m.def("dq_linear_parts", &dq_linear_parts, "dq_linear with k in parts, or None");
   m.def("row_scale", &row_scale, "1 / root mean square of rows");
   m.def("dq_linear_scaled", &dq_linear_scaled,
         "dq_linear of rows times factors, and the result's own",

@@ -97,6 +97,22 @@ def takes_factors(p: QLinear) -> bool:
     return p.bits == 8 or p.in_features >= 4096
 
 
+def shares_k(p: nn.Module) -> bool:
+    """Whether p's forward_resid is a packed layer's product and nothing else."""
+    return type(p) is QLinear and not hasattr(p, "perm") \
+        and unchanged(p, QLinear, "forward", "forward_resid") and not hooked(p)
+
+
+def resid_product(p: QLinear, x, resid, tickets):
+    """p.forward_resid(x, resid), by the kernel that shares k among workgroups where
+    that gains."""
+    if x.is_cuda and 2 < x.shape[0] <= 16 and shares_k(p):
+        y = F.dq_linear_parts(x, p, resid, tickets)
+        if y is not None:
+            return y
+    return p.forward_resid(x, resid)
+
+
 class LlamaAttention(nn.Module):
     def __init__(self, cfg: LlamaConfig, dtype):
         super().__init__()
@@ -344,8 +360,7 @@ class LlamaDecoderLayer(nn.Module):
             h, eps = self.post_attention_layernorm(x), -1.0
         h = F.dq_gemv_gateup(h, gp.qweight, gp.scales, gp.qzeros, gp.bits,
                              gp.group_size, rms_eps=eps)
-        x = mlp.down_proj.forward_resid(h, x)
-        return x
+        return resid_product(mlp.down_proj, h, x, tickets)
 
     def forward_decode_rows(self, x, scale, cache_k, cache_v, state, max_seq,
                             following: Optional["LlamaDecoderLayer"],

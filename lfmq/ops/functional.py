@@ -88,6 +88,21 @@ def dq_linear(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor,
     return ref.dq_linear(x, qweight, scales, qzeros, bits, group_size, bias).to(x.dtype)
 
 
+def dq_linear_parts(x: torch.Tensor, p, resid: torch.Tensor,
+                    tickets: Optional[torch.Tensor]):
+    """GPU-only dq_linear of the packed layer p for a few rows with the residual,
+    whose k is shared by workgroups of one launch, or None where that gains
+    nothing.  tickets: as attn_decode_fused's."""
+    if tickets is None:
+        return None
+    y = hip_ext().dq_linear_parts(
+        x.reshape(-1, x.shape[-1]), p.qweight, p.scales, p.qzeros, p.bits,
+        p.group_size, p.bias, resid.reshape(-1, resid.shape[-1]).contiguous(),
+        tickets)
+    return None if y is None else \
+        _guard(y, "dq_linear").reshape(*x.shape[:-1], y.shape[-1])
+
+
 def row_scale(x: torch.Tensor, eps: float) -> torch.Tensor:
     """GPU-only 1 / sqrt(mean x^2 + eps) of each row, fp32."""
     return hip_ext().row_scale(x.reshape(-1, x.shape[-1]), eps)

@@ -269,6 +269,28 @@ def test_factors_of_rows_that_somebody_reads(bits, parts, monkeypatch):
                      if (n == "o" and bits == 8) or (n == "down" and i < last)]
 
 
+def test_products_that_share_k_are_a_packed_layers_own():
+    """A caller's forward_resid or forward, hooks and gathers keep the call."""
+    from lfmq.models.llama import shares_k
+    from lfmq.models.qlinear import QLinear
+
+    def layer():
+        return QLinear(64, 8, 4, 64)
+    assert shares_k(layer())
+    own = type("Own", (QLinear,), {"forward_resid": lambda self, x, r: r})
+    assert not shares_k(own(64, 8, 4, 64))
+    for name in ("forward", "forward_resid"):
+        p = layer()
+        setattr(p, name, types.MethodType(lambda self, *a: a[-1], p))
+        assert not shares_k(p)
+    p = layer()
+    p.register_forward_hook(lambda *a: None)
+    assert not shares_k(p)
+    p = layer()
+    p.register_buffer("perm", torch.arange(64))
+    assert not shares_k(p)
+
+
 @pytest.mark.parametrize("where", ["class", "instance"])
 @pytest.mark.parametrize("b", [3, 17])
 @pytest.mark.parametrize("name", ["forward_decode_fused", "decode_qkv_attn"])

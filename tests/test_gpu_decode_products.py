@@ -65,6 +65,30 @@ def check(bits, m, n, k, g):
               1e-2)
 
 
+# k in two to five parts, also of unequal length; columns that end inside a tile, and
+# workgroups with a tile less than others; without a residual, and with a bias.
+@pytest.mark.parametrize("bits,m,n,k,g", [
+    (4, 3, 6148, 8192, 128), (4, 16, 4099, 8704, 64), (4, 8, 4096, 14336, 128),
+    (8, 5, 5001, 12288, 128), (8, 16, 2050, 20352, 64), (4, 9, 4200, 17408, 128),
+    (8, 4, 6160, 8704, 64), (4, 12, 4112, 11904, 64)])
+def test_k_in_parts_that_one_launch_adds_up(bits, m, n, k, g):
+    torch.manual_seed(m + n)
+    p, w = matrix(bits, n, k, g)
+    tickets = torch.zeros(256, dtype=torch.int32, device=DEV)
+    bias = torch.randn(n, device=DEV).to(BF)
+    resid = torch.randn(m, n, device=DEV).to(BF)
+    x = torch.randn(m, k, device=DEV).to(BF)
+    x[0] = 0
+    for _ in range(3):                       # the counters are as they were
+        y = ext().dq_linear_parts(x, *p, bits, g, bias, resid, tickets)
+        close(y, x.double() @ w.t() + bias.double() + resid.double())
+        y = ext().dq_linear_parts(x, *p, bits, g, None, None, tickets)
+        close(y, x.double() @ w.t())
+        assert not bool(tickets.any())
+        x = torch.randn(m, k, device=DEV).to(BF)
+    assert ext().dq_linear_parts(x, *p, bits, g, None, None, tickets[:8]) is None
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("n,k,g", [
     (8198, 2048, 128), (8193, 2048, 64), (7946, 2112, 32), (4097, 4096, 128),
