@@ -328,57 +328,6 @@ bool short_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
          (uintptr_t)qweight.data_ptr() % 16 == 0;
 }
 
-// The product of 8 bits whose workgroups share k among eight waves (dq_mid): where
-// it is faster than dq_short, dq_rows, dq_tile and dq_block.  Long k
-// pays where the columns are few, so that parts of it fill the chip: n 4096, k 4096
-// 20.6 / 15.2 us at 96 rows, n 2048, k 8192 18.2 / 14.9 at 61; n 20480, k 4096 35.3 /
-// 39.2 at 50.  A gate has no parts: n 6144, k 8192 24.0 / 34.3 at 54.  Above 96 rows
-// there are two tiles of them, and many columns are read twice: n 28672, k 2048 34.2 /
-// 41.8 at 109, n 6144, k 8192 33.2 / 41.6 at 110; 16384 to 28672 columns leave a
-// third of the chip (n 20480, k 2560 24.6 / 27.5 at 40).  Few rows of few columns are
-// dq_rows': n 4096, k 1024 6.4 / 7.7 at 36; and up to 32 rows of 6144 to 8192 columns,
-// 192 to 256 of its workgroups: n 8192, k 2048 9.8 / 12.1 at 17, 10.7 / 12.2 at 24, n
-// 7680, k 768 6.6 / 8.1 at 25.  49 to 64 rows of short k are dq_short's from 28672
-// columns on (n 34816, k 1024 22.1 / 29.2 at 60).  From 32769 columns on a second
-// round begins, and what is left over these lines is what gains there (n 36864, k
-// 1024, gate 21.1 / 23.9 at 18 rows; n 33088, k 960 29.4 / 33.3 at 83).
-// Of 5785 random calls of 17 to 128 rows, 768 to 40000 columns, k 768 to 10000, groups
-// of 64 to 256, that all but the last three lines take: 1.19 times as fast in the mean,
-// 6 % of them slower by more than 4 %; with these lines 2.3 % (2.5 % of 1997 others).
-bool mid_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
-              long bits, bool glu) {
-  if (bits != 8 || m <= 16 || m > 128 || n <= 0 || n % 8 ||
-      !tile_addresses(n, k, bits) || !lfmq_dq_tile_ok((int)k, (int)g) ||
-      (uintptr_t)qweight.data_ptr() % 16)
-    return false;
-  bool gains;
-  if (glu)
-    gains = k <= 3072 && (m <= 96 || n <= 8192) && (m <= 48 || n >= 4096) &&
-            (k <= 2048 || n <= 16384 || n >= 24576);
-  else if (m > 96 && n > (k <= 3072 ? 8192 : 3072))
-    gains = false;
-  else if (k <= 3072 && n > 16384 && n < 28672)
-    gains = m > 64 ? k <= 2048 || n > 24576 : m <= 48 && k <= 2048;
-  else if (k <= 3072)
-    gains = m <= 48 ? n >= 5120 && (m > 24 || n * k >= 16l << 20)
-                    : n * k >= 3l << 20;
-  else if (n <= 6144)
-    gains = m > (g == 64 && k <= 8192 ? 48 : 64) && m <= 112 &&
-            (k <= 8192 || g == 64);
-  else
-    gains = m > 48 && k <= 4096 && n >= 10240 && n <= 16384;
-  if (n > 32768)
-    gains = gains && (m <= 32   ? !glu && (g > 64 || k > 2048)
-                      : m <= 48 ? k < 1280 || (!glu && g > 64)
-                                : m > 64 && k >= 1536 && (glu || k <= 2560));
-  else if (m <= 32)
-    gains = gains && (glu || n < 6144 || n > 8192);
-  else if (m > 48 && m <= 64)
-    gains = gains && (n < 28672 || k > 2048);
-  return gains &&
-         lfmq_dq_mid_plan((int)m, (int)n, (int)k, (int)g, glu).mb > 0;
-}
-
 // What goes with whole rows of a product: a factor of x's rows, and what follows
 // rows of the result, which the sum of parts takes along if there is one.
 struct RowWays {
@@ -399,6 +348,17 @@ struct RowWays {
     return end;
   }
 };
+
+// The product whose workgroups share k among eight waves (dq_mid), where it is faster.
+bool mid_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
+              long bits, bool glu) {
+  if (m <= 16 || m > 128 || n <= 0 || n % 8 || !tile_addresses(n, k, bits) ||
+      !lfmq_dq_tile_ok((int)k, (int)g) || (uintptr_t)qweight.data_ptr() % 16)
+    return false;
+  return lfmq_dq_mid_gains(
+      lfmq_dq_mid_plan((int)m, (int)n, (int)k, (int)g, (int)bits, glu), m, n, k,
+      (int)bits, glu);
+}
 
 void dq_short(const torch::Tensor& x, const torch::Tensor& qweight,
               const torch::Tensor& scales, const torch::Tensor& qzeros,
@@ -436,9 +396,9 @@ void dq_short(const torch::Tensor& x, const torch::Tensor& qweight,
 void dq_mid(const torch::Tensor& x, const torch::Tensor& qweight,
             const torch::Tensor& scales, const torch::Tensor& qzeros,
             const void* bias, const void* resid, torch::Tensor& y, long g,
-            bool glu, const RowWays& ways) {
+            long bits, bool glu, const RowWays& ways) {
   const int m = (int)x.size(0), k = (int)x.size(1), n = (int)qweight.size(0);
-  const DqMidPlan P = lfmq_dq_mid_plan(m, n, k, (int)g, glu);
+  const DqMidPlan P = lfmq_dq_mid_plan(m, n, k, (int)g, (int)bits, glu);
   DqArgs A{};
   torch::Tensor part;
   if (P.splits > 1) {
@@ -459,7 +419,7 @@ void dq_mid(const torch::Tensor& x, const torch::Tensor& qweight,
   A.g = (int)g;
   A.splits = P.splits;
   A.row_scale = ways.scale;
-  CHECK_HIP(lfmq_dq_mid(A, P, glu, stream()));
+  CHECK_HIP(lfmq_dq_mid(A, P, (int)bits, glu, stream()));
   if (P.splits > 1 && !ways.keeps(part, P.splits))
     CHECK_HIP(lfmq_dq_rows_sum(part.data_ptr(), y.data_ptr(), bias, resid, m, n,
                                P.splits, false, stream(), ways.scale,
@@ -556,7 +516,7 @@ torch::Tensor linear(torch::Tensor x, const torch::Tensor& qweight,
                            rptr, m, n, k, (int)g, (int)bits, (float)rms_eps,
                            false, stream()));
   } else if (mid) {
-    dq_mid(x, qweight, scales, qzeros, bptr, rptr, y, g, false, ways);
+    dq_mid(x, qweight, scales, qzeros, bptr, rptr, y, g, bits, false, ways);
   } else if (few) {
     dq_short(x, qweight, scales, qzeros, bptr, rptr, y, g, bits, false,
              ways);
@@ -884,9 +844,10 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
   const bool large =
       tile && rms_eps < 0 && k >= 4096 && (long)n * k >= 24l << 20;
   const bool block = block_rows(qweight, scales, m, n, k, g, bits, true);
-  if (cols_hint == 0 && rms_eps < 0 && mid_rows(qweight, m, n, k, g, bits, true)) {
+  if (cols_hint == 0 && rms_eps < 0 &&
+      mid_rows(qweight, m, n, k, g, bits, true)) {
     if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
-    dq_mid(x, qweight, scales, qzeros, nullptr, nullptr, y, g, true, {});
+    dq_mid(x, qweight, scales, qzeros, nullptr, nullptr, y, g, bits, true, {});
     return y;
   }
   if (cols_hint == 0 && rms_eps < 0 && n % 2 == 0 &&
@@ -970,7 +931,7 @@ torch::Tensor dq_gateup_scaled(torch::Tensor x, torch::Tensor scale,
   if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
   auto y = torch::empty({m, n / 2}, x.options());
   if (mid_rows(qweight, m, n, k, g, bits, true))
-    dq_mid(x, qweight, scales, qzeros, nullptr, nullptr, y, g, true, ways);
+    dq_mid(x, qweight, scales, qzeros, nullptr, nullptr, y, g, bits, true, ways);
   else if (short_rows(qweight, m, n, k, g, bits, true, false))
     dq_short(x, qweight, scales, qzeros, nullptr, nullptr, y, g, bits, true,
              ways);

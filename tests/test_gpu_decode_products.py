@@ -332,6 +332,35 @@ def test_eight_waves_along_k(m, n, k, g):
 
 
 @pytest.mark.parametrize("m,n,k,g", [
+    (17, 28680, 1024, 128), (48, 8200, 2112, 64), (33, 32008, 832, 64),
+    (25, 1024, 768, 64), (33, 2008, 896, 128), (40, 28672, 4096, 128),
+    (48, 6144, 4096, 128), (64, 2056, 2048, 128), (77, 16384, 2048, 64),
+    (81, 1544, 2688, 192), (90, 8200, 896, 128), (97, 2048, 3072, 64),
+    (100, 512, 4992, 128), (113, 2504, 2560, 256), (128, 8192, 1024, 128),
+    (65, 1032, 14336, 64), (80, 10240, 4096, 128)])
+def test_eight_waves_along_k_of_four_bits(m, n, k, g):
+    """The same of 4 bits, whose sums of x waves side by side share and add two
+    steps later: one and two steps a group, one turn and many, last turns with
+    fewer groups than waves, more row tiles than waves side by side and fewer."""
+    torch.manual_seed(n + m)
+    p, w = matrix(4, n, k, g)
+    x = torch.randn(m, k, device=DEV).to(BF)
+    x[0] = 0
+    bias = torch.randn(n, device=DEV).to(BF)
+    plain = x.double() @ w.t()
+    close(ext().dq_linear(x, *p, 4, g, bias, None, -1.0, 0),
+          plain + bias.double())
+    close(ext().dq_gemv_gateup(x, *p, 4, g, -1.0, 0), gated(plain), 1e-2)
+    if m <= 48:
+        resid = torch.randn(m, n, device=DEV).to(BF)
+        scale = torch.rand(m, device=DEV) + 0.5
+        want = plain * scale.double().unsqueeze(1)
+        y, _ = ext().dq_linear_scaled(x, scale, *p, 4, g, None, resid, 1e-5)
+        close(y, want + resid.double())
+        close(ext().dq_gateup_scaled(x, scale, *p, 4, g), gated(want), 1e-2)
+
+
+@pytest.mark.parametrize("m,n,k,g", [
     (32, 6136, 1024, 64), (32, 6144, 1024, 64), (25, 8192, 768, 128),
     (25, 8200, 768, 128), (17, 8192, 2048, 64), (17, 8200, 2048, 64),
     (64, 28664, 1024, 64), (64, 28672, 1024, 64), (50, 28672, 2112, 64),
