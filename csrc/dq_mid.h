@@ -1,4 +1,4 @@
-// Packed product for some tens of rows (dq_mid.hip).
+// Packed product for some tens to hundreds of rows (dq_mid.hip).
 #pragma once
 #include "dq_frag.h"
 

@@ -1,4 +1,4 @@
-// K3h/K4h — W4A16 / W8A16 product for some tens of rows: y[m, n] = x[m, k] ·
+// K3h/K4h — W4A16 / W8A16 product for some tens to hundreds of rows: y[m, n] = x[m, k] ·
 // dequant(W)[n, k]^T (+ bias) (+ residual), or the gated half of a fused gate and up
 // projection.
 //
@@ -532,7 +532,7 @@ DqMidPlan lfmq_dq_mid_plan(int m, int n, int k, int g, int bits, bool glu) {
   static const float us[4][2] = {
       {0.244f, 0.169f}, {0.222f, 0.153f}, {0.409f, 0.148f}, {0.446f, 0.106f}};
   const int part = part_of(g), G = k / part;
-  for (int mb = 1; mb <= 4; ++mb) {
+  for (int mb = 1; mb <= 8; ++mb) {
     const int step =
         max(32, (int)ceil_div_u32(ceil_div_u32(m, mb), 16) * 16);
     // (every row tile has a row)
@@ -577,9 +577,19 @@ DqMidPlan lfmq_dq_mid_plan(int m, int n, int k, int g, int bits, bool glu) {
 // 4096, k 14336 at 126 rows 31.1 / 33.7.  Of 9600 random calls of 17 to 128 rows, 768 to
 // 36000 columns, k 512 to 14336, groups of 64 and 128, 8 in 10 taken: 1.19 times as fast
 // in the mean, 3.5 % of them slower by more than 4 %.
+//
+// 129 to 512 rows, where dq_block's and dq_tile's tiles of 128 rows are few: n 2048, k
+// 2048 at 300 rows 16.7 / 12.0, n 3072, k 2048 at 160 15.9 / 10.0, n 4096, k 4096 at 256
+// 24.2 / 19.4, n 16384, k 2048, gate (8), at 160 33.1 / 22.6; but long chains, n 4096, k
+// 14336 at 200 41.2 / 49.7, more than a round, n 16384, k 2048, gate, at 256 25.0 / 33.9,
+// and short k, n 12000, k 640 2 %.  Of 9200 random calls more than half are taken: 1.36
+// times as fast in the mean, 0.8 % slower by more than 4 %.
 bool lfmq_dq_mid_gains(const DqMidPlan& P, long m, long n, long k, int bits, bool glu) {
   const long size = n * k, M = 1l << 20;
   if (P.mb < 1 || P.wgs > 256) return false;
+  if (m > 128)
+    return k >= 768 && P.steps * P.mb * 256l <=
+                           (bits == 4 && size > 32 * M ? 100l : 200l) * P.wgs;
   const long most = bits == 4 && !glu && m <= 32 ? 40 : 120;
   if (!(glu && m <= 48) && P.steps * P.mb * 256l > most * P.wgs) return false;
   if (k < 768 && (m <= 32 || (bits == 4 && glu && m > 64 && n > 8192))) return false;

@@ -360,6 +360,22 @@ def test_eight_waves_along_k_of_four_bits(m, n, k, g):
         close(ext().dq_gateup_scaled(x, scale, *p, 4, g), gated(want), 1e-2)
 
 
+@pytest.mark.parametrize("bits,m,n,k,g", [
+    (4, 129, 2048, 2048, 64), (8, 161, 16384, 2048, 64), (4, 200, 4104, 4096, 128),
+    (8, 300, 2048, 2048, 128), (4, 511, 1032, 1920, 64), (8, 512, 2056, 2688, 192),
+    (4, 385, 520, 4992, 128), (8, 256, 4096, 4096, 64), (4, 512, 3072, 768, 128)])
+def test_eight_waves_of_many_rows(bits, m, n, k, g):
+    """The same of 129 to 512 rows: up to seven row tiles, last ones of one row."""
+    torch.manual_seed(n + m)
+    p, w = matrix(bits, n, k, g)
+    x = torch.randn(m, k, device=DEV).to(BF)
+    bias = torch.randn(n, device=DEV).to(BF)
+    plain = x.double() @ w.t()
+    close(ext().dq_linear(x, *p, bits, g, bias, None, -1.0, 0),
+          plain + bias.double())
+    close(ext().dq_gemv_gateup(x, *p, bits, g, -1.0, 0), gated(plain), 1e-2)
+
+
 @pytest.mark.parametrize("m,n,k,g", [
     (32, 6136, 1024, 64), (32, 6144, 1024, 64), (25, 8192, 768, 128),
     (25, 8200, 768, 128), (17, 8192, 2048, 64), (17, 8200, 2048, 64),
