@@ -578,11 +578,12 @@ DqMidPlan lfmq_dq_mid_plan(int m, int n, int k, int g, int bits, bool glu) {
 // 36000 columns, k 512 to 14336, groups of 64 and 128, 8 in 10 taken: 1.19 times as fast
 // in the mean, 3.5 % of them slower by more than 4 %.
 //
-// 129 to 512 rows, where dq_block's and dq_tile's tiles of 128 rows are few: n 2048, k
+// 129 to 768 rows (the most that were measured with these tiles), where dq_block's and dq_tile's tiles of 128 rows are few: n 2048, k
 // 2048 at 300 rows 16.7 / 12.0, n 3072, k 2048 at 160 15.9 / 10.0, n 4096, k 4096 at 256
 // 24.2 / 19.4, n 16384, k 2048, gate (8), at 160 33.1 / 22.6; but long chains, n 4096, k
 // 14336 at 200 41.2 / 49.7, more than a round, n 16384, k 2048, gate, at 256 25.0 / 33.9,
-// and short k, n 12000, k 640 2 %.  Of 9200 random calls more than half are taken: 1.36
+// and short k, n 12000, k 640 2 %; n 2048, k 2048 (8) at 768 26.6 / 15.9, but n 2048, k
+// 8192 (4 bits) at 660 37.2 / 42.7.  Of 9700 random calls more than half are taken: 1.36
 // times as fast in the mean, 0.8 % slower by more than 4 %.
 bool lfmq_dq_mid_gains(const DqMidPlan& P, long m, long n, long k, int bits, bool glu) {
   const long size = n * k, M = 1l << 20;

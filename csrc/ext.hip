@@ -352,7 +352,7 @@ struct RowWays {
 // The product whose workgroups share k among eight waves (dq_mid), where it is faster.
 bool mid_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
               long bits, bool glu) {
-  if (m <= 16 || m > 512 || n <= 0 || n % 8 || !tile_addresses(n, k, bits) ||
+  if (m <= 16 || m > 768 || n <= 0 || n % 8 || !tile_addresses(n, k, bits) ||
       !lfmq_dq_tile_ok((int)k, (int)g) || (uintptr_t)qweight.data_ptr() % 16)
     return false;
   return lfmq_dq_mid_gains(

@@ -363,9 +363,10 @@ def test_eight_waves_along_k_of_four_bits(m, n, k, g):
 @pytest.mark.parametrize("bits,m,n,k,g", [
     (4, 129, 2048, 2048, 64), (8, 161, 16384, 2048, 64), (4, 200, 4104, 4096, 128),
     (8, 300, 2048, 2048, 128), (4, 511, 1032, 1920, 64), (8, 512, 2056, 2688, 192),
-    (4, 385, 520, 4992, 128), (8, 256, 4096, 4096, 64), (4, 512, 3072, 768, 128)])
+    (4, 385, 520, 4992, 128), (8, 256, 4096, 4096, 64), (4, 512, 3072, 768, 128),
+    (8, 768, 2048, 2048, 64), (4, 673, 2048, 2048, 128)])
 def test_eight_waves_of_many_rows(bits, m, n, k, g):
-    """The same of 129 to 512 rows: up to seven row tiles, last ones of one row."""
+    """The same of 129 to 768 rows: up to eight row tiles, last ones of one row."""
     torch.manual_seed(n + m)
     p, w = matrix(bits, n, k, g)
     x = torch.randn(m, k, device=DEV).to(BF)
