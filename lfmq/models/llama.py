@@ -91,10 +91,10 @@ def linear_norm(p: nn.Module, x, residual, norm: RMSNorm):
 
 def takes_factors(p: QLinear) -> bool:
     """Whether a norm in front of p is worth a launch of its own for 17 to 48
-    rows: where a product without it may split k (`dq_mid`, `dq_short`).  A step of
-    17 rows of four layers of 2048, groups of 128: 4 bits 217.7 us with it, 209.3
-    without; 8 bits 228 and 231."""
-    return p.bits == 8 or p.in_features >= 4096
+    rows: where a product without it may be `dq_mid`'s or `dq_short`'s.  A step of
+    four layers of 2048, 4 bits: 17 rows 217 us with it, 219 without (groups of 64
+    230 and 238), 48 rows 255 and 260; 8 bits 228 and 231 at 17."""
+    return p.bits == 8 or p.in_features >= 2048
 
 
 def shares_k(p: nn.Module) -> bool:
