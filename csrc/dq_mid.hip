@@ -541,9 +541,10 @@ DqMidPlan lfmq_dq_mid_plan(int m, int n, int k, int g, int bits, bool glu) {
       const int kw = NWV / nc, bo = nc * NT * 16;
       const int nb = (int)(glu ? ceil_div_u32(n / 2, bo / 2) : ceil_div_u32(n, bo));
       const float* t0 = us[(bits == 8 ? 2 : 0) + (nc == 4 ? 1 : 0)];
-      for (int wgs = 0; wgs <= 512; wgs += wgs == 0 ? 256 : 128) {
+      for (int wgs = 0, before = 0; wgs <= 512; wgs += wgs == 0 ? 256 : 128) {
         const int sp = max(1, wgs / (nb * mb));
-        if (sp > 1 && (glu || sp > G)) continue;
+        if (sp == before || (sp > 1 && (glu || sp > G))) continue;
+        before = sp;
         const int ng = (int)ceil_div_u32(G, sp), all = mb * nb * sp;
         if (lds_of(bits, part, step / 16, nc, ng) > MOST_LDS) continue;
         const int u = (int)ceil_div_u32(all, 256);

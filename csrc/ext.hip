@@ -349,15 +349,16 @@ struct RowWays {
   }
 };
 
-// The product whose workgroups share k among eight waves (dq_mid), where it is faster.
-bool mid_rows(const torch::Tensor& qweight, long m, long n, long k, long g,
-              long bits, bool glu) {
+// The product whose workgroups share k among eight waves (dq_mid), where it is faster;
+// mb 0: it is not.
+DqMidPlan mid_plan(const torch::Tensor& qweight, long m, long n, long k, long g,
+                   long bits, bool glu) {
   if (m <= 16 || m > 768 || n <= 0 || n % 8 || !tile_addresses(n, k, bits) ||
       !lfmq_dq_tile_ok((int)k, (int)g) || (uintptr_t)qweight.data_ptr() % 16)
-    return false;
-  return lfmq_dq_mid_gains(
-      lfmq_dq_mid_plan((int)m, (int)n, (int)k, (int)g, (int)bits, glu), m, n, k,
-      (int)bits, glu);
+    return {};
+  const DqMidPlan P =
+      lfmq_dq_mid_plan((int)m, (int)n, (int)k, (int)g, (int)bits, glu);
+  return lfmq_dq_mid_gains(P, m, n, k, (int)bits, glu) ? P : DqMidPlan{};
 }
 
 void dq_short(const torch::Tensor& x, const torch::Tensor& qweight,
@@ -393,12 +394,11 @@ void dq_short(const torch::Tensor& x, const torch::Tensor& qweight,
                                ways.ends()));
 }
 
-void dq_mid(const torch::Tensor& x, const torch::Tensor& qweight,
+void dq_mid(const DqMidPlan& P, const torch::Tensor& x, const torch::Tensor& qweight,
             const torch::Tensor& scales, const torch::Tensor& qzeros,
             const void* bias, const void* resid, torch::Tensor& y, long g,
             long bits, bool glu, const RowWays& ways) {
   const int m = (int)x.size(0), k = (int)x.size(1), n = (int)qweight.size(0);
-  const DqMidPlan P = lfmq_dq_mid_plan(m, n, k, (int)g, (int)bits, glu);
   DqArgs A{};
   torch::Tensor part;
   if (P.splits > 1) {
@@ -484,8 +484,10 @@ torch::Tensor linear(torch::Tensor x, const torch::Tensor& qweight,
                        lfmq_dq_rows_ok(m, n, k, (int)g, rms);
   const bool block = rptr == nullptr && !scaled &&
                      block_rows(qweight, scales, m, n, k, g, bits, false);
-  const bool mid = cols_hint == 0 && !rms &&
-                   mid_rows(qweight, m, n, k, g, bits, false);
+  const DqMidPlan plan = cols_hint == 0 && !rms
+                             ? mid_plan(qweight, m, n, k, g, bits, false)
+                             : DqMidPlan{};
+  const bool mid = plan.mb > 0;
   const bool few = cols_hint == 0 && !rms && !(small && by_rows) &&
                    short_rows(qweight, m, n, k, g, bits, false, block);
   TORCH_CHECK(!scaled || (m > 16 && m <= 48 && (by_rows || few || mid)),
@@ -516,7 +518,7 @@ torch::Tensor linear(torch::Tensor x, const torch::Tensor& qweight,
                            rptr, m, n, k, (int)g, (int)bits, (float)rms_eps,
                            false, stream()));
   } else if (mid) {
-    dq_mid(x, qweight, scales, qzeros, bptr, rptr, y, g, bits, false, ways);
+    dq_mid(plan, x, qweight, scales, qzeros, bptr, rptr, y, g, bits, false, ways);
   } else if (few) {
     dq_short(x, qweight, scales, qzeros, bptr, rptr, y, g, bits, false,
              ways);
@@ -844,10 +846,12 @@ torch::Tensor dq_gemv_gateup(torch::Tensor x, torch::Tensor qweight,
   const bool large =
       tile && rms_eps < 0 && k >= 4096 && (long)n * k >= 24l << 20;
   const bool block = block_rows(qweight, scales, m, n, k, g, bits, true);
-  if (cols_hint == 0 && rms_eps < 0 &&
-      mid_rows(qweight, m, n, k, g, bits, true)) {
+  const DqMidPlan plan = cols_hint == 0 && rms_eps < 0
+                             ? mid_plan(qweight, m, n, k, g, bits, true)
+                             : DqMidPlan{};
+  if (plan.mb > 0) {
     if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
-    dq_mid(x, qweight, scales, qzeros, nullptr, nullptr, y, g, bits, true, {});
+    dq_mid(plan, x, qweight, scales, qzeros, nullptr, nullptr, y, g, bits, true, {});
     return y;
   }
   if (cols_hint == 0 && rms_eps < 0 && n % 2 == 0 &&
@@ -930,8 +934,9 @@ torch::Tensor dq_gateup_scaled(torch::Tensor x, torch::Tensor scale,
   RowWays ways{factors(scale, m)};
   if ((uintptr_t)x.data_ptr() % 16) x = x.clone();
   auto y = torch::empty({m, n / 2}, x.options());
-  if (mid_rows(qweight, m, n, k, g, bits, true))
-    dq_mid(x, qweight, scales, qzeros, nullptr, nullptr, y, g, bits, true, ways);
+  const DqMidPlan plan = mid_plan(qweight, m, n, k, g, bits, true);
+  if (plan.mb > 0)
+    dq_mid(plan, x, qweight, scales, qzeros, nullptr, nullptr, y, g, bits, true, ways);
   else if (short_rows(qweight, m, n, k, g, bits, true, false))
     dq_short(x, qweight, scales, qzeros, nullptr, nullptr, y, g, bits, true,
              ways);
