@@ -12,7 +12,8 @@ struct DqMidPlan {
 DqMidPlan lfmq_dq_mid_plan(int m, int n, int k, int g, int bits, bool glu);
 
 // whether that is the faster way
-bool lfmq_dq_mid_gains(const DqMidPlan& P, long m, long n, long k, int bits, bool glu);
+bool lfmq_dq_mid_gains(const DqMidPlan& P, long m, long n, long k, long g, int bits,
+                       bool glu);
 
 // a matrix below 4 GiB that starts on 16 bytes; splits > 1 (not with glu): A.part
 // gets [splits, m, n] fp32, and nothing else is done; else rows of x times

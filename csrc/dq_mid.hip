@@ -522,10 +522,16 @@ int part_of(int g) { return g % 128 == 0 ? 128 : 64; }
 
 // Row tiles, columns of a workgroup and parts of k by the time these would take: 256
 // workgroups a round, one after the other on a CU; a step 0.5 to 1.3 us, and the
-// traffic of the parts and 0.8 us for their launch, of 2.2: mostly a norm, the rotation
-// or factors of rows, which are a launch anyway, take the sum along.  Fitted to half of
-// 101000 measured plans of 9700 calls, 17 to 128 rows (off by 7 % rms; the plan it takes
-// is 0.5 % slower than the best).
+// traffic of the parts and 0.8 us for their launch: mostly a norm, the rotation or
+// factors of rows, which are a launch anyway, take the sum along.  A call with nothing
+// behind it has the same plan, so that its results are the same bits, and pays 1.6 us
+// in a graph and 3.0 called from Python (means of 840 calls).  us in a graph / called /
+// with a norm, with this plan and with one that charges 2.2: n 2048, k 2048 (4 bits) at
+// 77 rows 10.2 / 12.7 / 10.6, 9.8 / 10.2 / 12.2; n 4096, k 4096 (4) at 77 15.8 / 16.7 /
+// 16.5, 14.3 / 14.3 / 16.9; n 3072, k 2048 (8) at 96 12.5 / 13.5 / 13.6, 11.5 / 11.7 /
+// 14.2.
+// Fitted to half of 101000 measured plans of 9700 calls, 17 to 128 rows (off by 7 %
+// rms; the plan it takes is 0.5 % slower than the best); not to more rows.
 DqMidPlan lfmq_dq_mid_plan(int m, int n, int k, int g, int bits, bool glu) {
   DqMidPlan best{};
   float least = INFINITY;
@@ -566,39 +572,73 @@ DqMidPlan lfmq_dq_mid_plan(int m, int n, int k, int g, int bits, bool glu) {
 
 // Whether that is faster than the other kernels for these rows (dq_rows, dq_short,
 // dq_tile, dq_block): one round of workgroups, whose chain (steps, times row tiles and
-// idle CUs) is not long for what it does.  us of the best of those / of this one: two
-// rounds, n 32000, k 4096 (4 bits, groups of 128) at 128 rows 43.4 / 59.9; few
-// workgroups and no parts, as a gate has none, n 6592, k 9216 (8) at 105 rows 44.1 /
-// 50.6; few rows of 4 bits, where those lose less by it, n 16832, k 6400 at 32 27.6 /
-// 31.6.  Few rows of a small matrix are dq_rows': n 3712, k 3072 at 19 rows 9.0 / 11.4,
-// n 4096, k 4096 (8) at 17 11.1 / 12.6, n 3072, k 2048 at 32 8.3 / 9.5; short k: n 7424,
-// k 640, gate, 19 rows 6.8 / 8.0, and n 27200, k 512, gate, at 88 10.2 / 11.7.  From
-// 16384 to 20480 columns a workgroup of 128 leaves 96 CUs: n 18688, k 4096 at 55 rows
-// 26.3 / 30.1, n 17536, k 1536 at 82 16.6 / 18.7.  Many rows of very long k, 4 bits: n
-// 4096, k 14336 at 126 rows 31.1 / 33.7.  Of 9600 random calls of 17 to 128 rows, 768 to
-// 36000 columns, k 512 to 14336, groups of 64 and 128, 8 in 10 taken: 1.19 times as fast
-// in the mean, 3.5 % of them slower by more than 4 %.
+// idle CUs) is not long for what it does.  us of the best of those / of this one:
+// - two rounds: n 32000, k 4096 (4 bits, groups of 128) at 128 rows 43.4 / 59.9
+// - few rows of 4 bits, where those lose less by idle CUs: n 16832, k 6400 at 32 27.6 /
+//   31.6.  A gate has no parts here, nor in dq_rows, but in dq_short and dq_tile: n 8112,
+//   k 9728 (8) at 19 29.4 / 49.8, n 2256, k 12032 at 46 21.3 / 31.1; n 2416, k 3840 at
+//   40, which dq_rows has, 24.0 / 15.8
+// - few rows of a short k, which does not make up for the first loads: n 12584, k 768,
+//   gate, at 28 7.9 / 8.6, n 7424, k 640, gate, at 19 6.8 / 8.0; of a small matrix n
+//   3712, k 3072 at 19 9.0 / 11.4, n 3072, k 2048 at 32 8.3 / 9.5, but n 25496, k 640 (8)
+//   at 32 16.3 / 10.8.  6144 to 8192 columns are 192 to 256 workgroups of dq_rows, which
+//   has up to 32 rows at once: n 6944, k 1664 (8) at 26 9.8 / 11.8, n 7440, k 640 (8) at
+//   42 10.3 / 8.5
+// - groups of 128 of a short k, two steps each: n 16264, k 640 (8) at 119 11.1 / 12.7;
+//   n 27200, k 512, gate, at 88 10.2 / 11.7
+// - 16384 to 20480 columns, where a workgroup of 128 leaves 96 CUs: n 18688, k 4096 at
+//   55 26.3 / 30.1, n 17536, k 1536 at 82 16.6 / 18.7
+// - many rows of very long k, 4 bits: n 4096, k 14336 at 126 31.1 / 33.7
+// Of 5400 random calls of 17 to 128 rows, 768 to 36000 columns, k 1024 to 14336, groups
+// of 64 and 128, 8 in 10 are taken: 1.18 times as fast in the mean, 1.13 with a norm
+// behind them, 5 % of them slower by more than 4 %.  (97 to 128 rows of k below 2048
+// without parts, on half of the chip: 10 % faster, 8 % slower with a norm, which the sum
+// of dq_tile's parts takes along.)
 //
-// 129 to 768 rows (the most that were measured with these tiles), where dq_block's and dq_tile's tiles of 128 rows are few: n 2048, k
-// 2048 at 300 rows 16.7 / 12.0, n 3072, k 2048 at 160 15.9 / 10.0, n 4096, k 4096 at 256
-// 24.2 / 19.4, n 16384, k 2048, gate (8), at 160 33.1 / 22.6; but long chains, n 4096, k
-// 14336 at 200 41.2 / 49.7, more than a round, n 16384, k 2048, gate, at 256 25.0 / 33.9,
-// and short k, n 12000, k 640 2 %; n 2048, k 2048 (8) at 768 26.6 / 15.9, but n 2048, k
-// 8192 (4 bits) at 660 37.2 / 42.7.  Of 9700 random calls more than half are taken: 1.36
-// times as fast in the mean, 0.8 % slower by more than 4 %.
-bool lfmq_dq_mid_gains(const DqMidPlan& P, long m, long n, long k, int bits, bool glu) {
+// 129 to 768 rows (the most that were measured with these tiles), where dq_block's and
+// dq_tile's tiles of 128 rows are few: n 2048, k 2048 at 300 rows 16.7 / 12.0, n 3072, k
+// 2048 at 160 15.9 / 10.0, n 4096, k 4096 at 256 24.2 / 19.4, n 16384, k 2048, gate (8),
+// at 160 33.1 / 22.6; but long chains, n 4096, k 14336 at 200 41.2 / 49.7, more than a
+// round, n 16384, k 2048, gate, at 256 25.0 / 33.9, and short k, n 12000, k 640 2 %; n
+// 2048, k 2048 (8) at 768 26.6 / 15.9, but n 2048, k 8192 (4 bits) at 660 37.2 / 42.7.
+// Of 9700 random calls more than half are taken: 1.36 times as fast in the mean, 0.8 %
+// slower by more than 4 %.
+bool lfmq_dq_mid_gains(const DqMidPlan& P, long m, long n, long k, long g, int bits,
+                       bool glu) {
   const long size = n * k, M = 1l << 20;
+  const bool four = bits == 4, wide = g % 128 == 0;
   if (P.mb < 1 || P.wgs > 256) return false;
+  const int work = P.steps * (P.step / 16);      // of a wave
   if (m > 128)
-    return k >= 768 && P.steps * P.mb * 256l <=
-                           (bits == 4 && size > 32 * M ? 100l : 200l) * P.wgs;
-  const long most = bits == 4 && !glu && m <= 32 ? 40 : 120;
-  if (!(glu && m <= 48) && P.steps * P.mb * 256l > most * P.wgs) return false;
-  if (k < 768 && (m <= 32 || (bits == 4 && glu && m > 64 && n > 8192))) return false;
-  if (!glu && n > 2016 && (m <= 24 ? size < 20 * M : m <= 48 && size <= 8 * M))
+    return k >= 768 &&
+           P.steps * P.mb * 256l <= (four && size > 32 * M ? 100l : 200l) * P.wgs;
+  const long most = four && !glu && m <= 32 ? 40 : 120;
+  if (glu && m <= 48) {
+    // (dq_rows with its gate has no parts either, dq_short and dq_tile do)
+    const bool others = (n >= 4096 && size >= 16 * M && (k >= 4096 || size >= 48 * M)) ||
+                        (m > 32 && k >= 4096 && size >= 24 * M);
+    if (others && P.steps * P.mb * 256l > 56l * P.wgs) return false;
+  } else if (P.steps * P.mb * 256l > most * P.wgs) {
+    return false;
+  }
+  if (m <= 32) {
+    if (four ? P.splits == 1 && P.steps <= (glu ? 5 : 4)
+             : glu && wide && P.steps <= 4 && size < 10 * M)
+      return false;
+    if (k < 768 && (four || size < 10 * M)) return false;
+  } else if (m > 48 && k < 1024) {
+    if (wide && n > (four && glu ? 2304 : 6144) && work > (k < 768 ? 7 : four ? 9 : 12))
+      return false;
+    if (k < 768 && four && glu && m > 64 && n > 8192) return false;
+  }
+  if (!glu && n > 2016 &&
+      (m <= 24 ? size < (four ? 20 : 10) * M
+               : m <= 48 && size <= (four ? 8 : 6) * M && (four || n < 6144)))
+    return false;
+  if (!glu && m <= 32 && n >= 6144 && n <= 8192 && size < (four ? 21 : 16) * M)
     return false;
   if (n > 16384 && n <= 20480 && (k <= 2048 ? m > 80 : !glu && k >= 4096)) return false;
-  return !(bits == 4 && m > 96 && k >= 12000);
+  return !(four && m > 96 && k >= 12000);
 }
 
 hipError_t lfmq_dq_mid(const DqArgs& A, const DqMidPlan& P, int bits, bool glu,

@@ -358,7 +358,7 @@ DqMidPlan mid_plan(const torch::Tensor& qweight, long m, long n, long k, long g,
     return {};
   const DqMidPlan P =
       lfmq_dq_mid_plan((int)m, (int)n, (int)k, (int)g, (int)bits, glu);
-  return lfmq_dq_mid_gains(P, m, n, k, (int)bits, glu) ? P : DqMidPlan{};
+  return lfmq_dq_mid_gains(P, m, n, k, g, (int)bits, glu) ? P : DqMidPlan{};
 }
 
 void dq_short(const torch::Tensor& x, const torch::Tensor& qweight,

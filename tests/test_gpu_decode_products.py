@@ -4,8 +4,11 @@ to sixteen (dq_wide), where their waves, groups and tiles end.
 Products of bf16 and codes are exact and summed in fp32, so a result is off
 by its own rounding, 2^-9 of a value, and by the sums' error where it is small
 beside its row."""
+import re
+
 import pytest
 import torch
+from torch.profiler import ProfilerActivity, profile
 
 from lfmq.ops import hip_ext as ext
 from lfmq.ops import ref
@@ -34,6 +37,17 @@ def close(y, want, rel=5e-3):
     floor = 1e-3 * want.abs().amax(-1, keepdim=True) + 1e-30
     assert y.shape == want.shape
     assert float((err / (want.abs() + floor)).max()) < rel
+
+
+def launched(call):
+    """Names of the kernels that it launches."""
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        call()
+        torch.cuda.synchronize()
+    names = (re.search(r"(\w+)[<(]", e.key.replace("(anonymous namespace)", ""))
+             for e in p.key_averages())
+    return {n.group(1) for n in names if n}
 
 
 def normed(x, eps):
@@ -377,13 +391,51 @@ def test_eight_waves_of_many_rows(bits, m, n, k, g):
     close(ext().dq_gemv_gateup(x, *p, bits, g, -1.0, 0), gated(plain), 1e-2)
 
 
-@pytest.mark.parametrize("m,n,k,g", [
-    (32, 6136, 1024, 64), (32, 6144, 1024, 64), (25, 8192, 768, 128),
-    (25, 8200, 768, 128), (17, 8192, 2048, 64), (17, 8200, 2048, 64),
-    (64, 28664, 1024, 64), (64, 28672, 1024, 64), (50, 28672, 2112, 64),
-    (96, 24576, 2112, 64), (65, 24584, 2112, 64), (32, 32768, 512, 64),
-    (32, 32776, 512, 64), (32, 32776, 512, 128), (48, 32776, 1216, 64),
-    (33, 32776, 1280, 64), (65, 32776, 1472, 64), (65, 32776, 1536, 64)])
-def test_eight_waves_at_the_lines(m, n, k, g):
+# (bits, gate, rows, n, k, group): taken, and the neighbour that is not
+LINES = [
+    # rows, columns in eights, one round of workgroups
+    ((4, 0, 768, 2048, 2048, 128), (4, 0, 769, 2048, 2048, 128)),
+    ((4, 0, 100, 4104, 2048, 128), (4, 0, 100, 4102, 2048, 128)),
+    ((8, 0, 96, 32768, 2048, 64), (8, 0, 96, 32776, 2048, 64)),
+    ((4, 0, 80, 32768, 1024, 128), (4, 0, 80, 32776, 1024, 128)),
+    # a gate's chain, where the other kernel has parts, and above 48 rows
+    ((4, 1, 48, 10240, 4096, 128), (4, 1, 48, 10240, 9216, 128)),
+    ((4, 1, 40, 4088, 6144, 128), (4, 1, 40, 4104, 6144, 128)),
+    ((8, 1, 48, 1024, 6144, 64), (8, 1, 49, 1024, 6144, 64)),
+    # few rows: short chains, small matrices, 6144 to 8192 columns
+    ((4, 1, 28, 16384, 1280, 128), (4, 1, 28, 16384, 1024, 128)),
+    ((8, 1, 28, 4096, 1280, 128), (8, 1, 28, 4096, 1024, 128)),
+    ((4, 0, 32, 16384, 1280, 64), (4, 0, 32, 16384, 1024, 64)),
+    ((8, 0, 25, 9000, 1024, 64), (8, 0, 24, 9000, 1024, 64)),
+    ((8, 0, 49, 3000, 1024, 64), (8, 0, 48, 3000, 1024, 64)),
+    ((8, 0, 40, 2016, 1024, 64), (8, 0, 40, 2024, 1024, 64)),
+    ((8, 0, 40, 6144, 640, 64), (8, 0, 40, 6136, 640, 64)),
+    ((8, 0, 32, 6136, 1536, 64), (8, 0, 32, 6144, 1536, 64)),
+    ((8, 0, 32, 8200, 1024, 64), (8, 0, 32, 8192, 1024, 64)),
+    ((4, 0, 32, 8200, 2048, 128), (4, 0, 32, 8192, 2048, 128)),
+    # short k
+    ((8, 0, 200, 2048, 768, 64), (8, 0, 200, 2048, 704, 64)),
+    ((8, 0, 32, 9000, 768, 64), (8, 0, 32, 9000, 704, 64)),
+    ((8, 0, 64, 6144, 640, 128), (8, 0, 64, 6152, 640, 128)),
+    # 16385 to 20480 columns, long k
+    ((8, 0, 96, 16384, 1024, 64), (8, 0, 96, 16392, 1024, 64)),
+    ((8, 0, 96, 20488, 1024, 64), (8, 0, 96, 20480, 1024, 64)),
+    ((4, 0, 55, 16384, 4096, 64), (4, 0, 55, 16392, 4096, 64)),
+    ((4, 0, 96, 4096, 12032, 128), (4, 0, 97, 4096, 12032, 128))]
+
+
+@pytest.mark.parametrize("call,taken", [(c, i == 0) for pair in LINES
+                                        for i, c in enumerate(pair)])
+def test_eight_waves_at_the_lines(call, taken):
     """On both sides of the lines where other products are the faster ones."""
-    test_eight_waves_along_k(m, n, k, g)
+    bits, gate, m, n, k, g = call
+    torch.manual_seed(n + m)
+    p, w = matrix(bits, n, k, g)
+    x = torch.randn(m, k, device=DEV).to(BF)
+    want = x.double() @ w.t()
+    got = []
+    names = launched(lambda: got.append(
+        ext().dq_gemv_gateup(x, *p, bits, g, -1.0, 0) if gate else
+        ext().dq_linear(x, *p, bits, g, None, None, -1.0, 0)))
+    assert ("dq_mid_kernel" in names) == taken, names
+    close(got[0], gated(want) if gate else want, 1e-2 if gate else 5e-3)
