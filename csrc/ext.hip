@@ -218,13 +218,14 @@ bool wide_rows(int m, int n, int k, long g, long bits, bool glu) {
 // groups of 128) 11.4 / 10.9 at 8 rows, 13.6 / 12.1 at 16, 10.1 / 10.4 at 4; n 4096, k
 // 14336 14.2 / 13.7 at 4; n 2048, k 8192 9.9 / 10.7 at 16; n 4096, k 5120 10.9 / 12.1; n
 // 12288, k 8192 17.0 / 16.0 at 3, groups of 64 21.5 / 21.9; seven parts, n 4096, k 27648
-// 26.7 / 34.6 at 7, of few columns n 1904, k 25600 20.9 / 22.6 at 13.  Of 65 random
-// calls that it takes 1.26 times as fast in the mean.
+// 26.7 / 34.6 at 7, of few columns n 1904, k 25600 20.9 / 22.6 at 13.  Of 22000 random
+// calls that it takes 1.23 times as fast in the mean, 0.8 % slower by more than 4 %:
+// groups of 64 below 44 million weights, n 2136, k 16384 at 16 17.1 / 18.8.
 bool part_rows(long m, long n, long k, long g, long bits) {
   const long size = n * k, M = 1l << 20, parts = (k + 4095) / 4096;
-  return m >= 3 && m <= 16 && n >= 2048 && k >= 8192 && parts <= 5 && size >= (m > 8 ? 32 : 48) * M &&
-         10 * k >= 7 * 4096 * parts && (bits == 8 || g != 64 || n <= 8192) &&
-         tile_addresses(n, k, bits);
+  return m >= 3 && m <= 16 && n >= 2048 && k >= 8192 && parts <= 5 &&
+         size >= (m > 8 ? 32 : 48) * M && 10 * k >= 7 * 4096 * parts &&
+         (bits == 8 || g != 64 || n <= 8192) && tile_addresses(n, k, bits);
 }
 
 // The product for many rows: tiles of 256 columns instead of 128, which few
@@ -556,7 +557,7 @@ torch::Tensor dq_linear(torch::Tensor x, torch::Tensor qweight,
                 cols_hint, {});
 }
 
-// dq_linear of 2 to 16 rows whose k is in parts that one launch adds up, with
+// dq_linear of 3 to 16 rows whose k is in parts that one launch adds up, with
 // `tickets` (zeros before and afterwards, of nobody else meanwhile); None: it gains
 // nothing by them.
 c10::optional<torch::Tensor> dq_linear_parts(

@@ -103,6 +103,20 @@ def test_k_in_parts_that_one_launch_adds_up(bits, m, n, k, g):
     assert ext().dq_linear_parts(x, *p, bits, g, None, None, tickets[:8]) is None
 
 
+@pytest.mark.parametrize("n,k,rounds", [(8176, 8960, 1), (10912, 9984, 2)])
+def test_k_in_parts_is_one_round_of_workgroups(n, k, rounds):
+    """Three parts of 511 column tiles, six of which a workgroup would leave 258 of
+    them (seven do not), and of 682, which eight a workgroup would."""
+    torch.manual_seed(n)
+    p, w = matrix(4, n, k, 128)
+    x = torch.randn(5, k, device=DEV).to(BF)
+    tickets = torch.zeros(256, dtype=torch.int32, device=DEV)
+    y = ext().dq_linear_parts(x, *p, 4, 128, None, None, tickets)
+    assert (y is None) == (rounds > 1)
+    if y is not None:
+        close(y, x.double() @ w.t())
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("n,k,g", [
     (8198, 2048, 128), (8193, 2048, 64), (7946, 2112, 32), (4097, 4096, 128),
