@@ -23,9 +23,13 @@ class KVCache:
                                  head_dim, device=device, dtype=dtype)
         self.k = [self.k_all[i] for i in range(n_layers)]
         self.v = [self.v_all[i] for i in range(n_layers)]
-        # arrivals of the key ranges of a query head (decode attention), back
-        # at zero after every layer.  The cache's, as its rows are: steps that
-        # overlap, or that two graphs hold, run on caches of their own.
+        # arrivals of workgroups that share a result, whose last one adds up:
+        # the key ranges of a query head (decode attention), then the parts of
+        # k of a few rows' down projection, if there are as many as it has
+        # workgroups a part (128 at most; without them it takes k whole).  One
+        # launch after the other, each of which leaves zeros.  The cache's, as
+        # its rows are: steps that overlap, or that two graphs hold, run on
+        # caches of their own.
         self.tickets = torch.zeros(batch * (n_heads or n_kv_heads),
                                    dtype=torch.int32, device=device)
 

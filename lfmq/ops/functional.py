@@ -92,7 +92,8 @@ def dq_linear_parts(x: torch.Tensor, p, resid: torch.Tensor,
                     tickets: Optional[torch.Tensor]):
     """GPU-only dq_linear of the packed layer p for a few rows with the residual,
     whose k is shared by workgroups of one launch, or None where that gains
-    nothing.  tickets: as attn_decode_fused's."""
+    nothing, or there are fewer tickets (as attn_decode_fused's) than a part
+    has workgroups."""
     if tickets is None:
         return None
     y = hip_ext().dq_linear_parts(

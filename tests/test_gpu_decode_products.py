@@ -10,6 +10,9 @@ import pytest
 import torch
 from torch.profiler import ProfilerActivity, profile
 
+import lfmq
+from lfmq.models.llama import LlamaConfig
+from lfmq.ops import functional as F
 from lfmq.ops import hip_ext as ext
 from lfmq.ops import ref
 
@@ -453,3 +456,56 @@ def test_eight_waves_at_the_lines(call, taken):
         ext().dq_linear(x, *p, bits, g, None, None, -1.0, 0)))
     assert ("dq_mid_kernel" in names) == taken, names
     close(got[0], gated(want) if gate else want, 1e-2 if gate else 5e-3)
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("batch,heads,hidden,inner", [
+    (8, 32, 4096, 14336), (3, 48, 6144, 8192), (16, 32, 2048, 20480)])
+def test_a_step_whose_down_projection_is_in_parts(batch, heads, hidden, inner,
+                                                  monkeypatch):
+    """Its counters are those of decode attention, in each layer and in a graph's
+    replays; results to the bit, as a layer's launches are the same then."""
+    T = 300
+    torch.manual_seed(hidden)
+    with torch.device(DEV):
+        cfg = LlamaConfig(vocab_size=512, hidden_size=hidden, intermediate_size=inner,
+                          n_layers=2, n_heads=heads, n_kv_heads=8, head_dim=128)
+        m = lfmq.build_model(cfg)
+        for p in m.parameters():
+            if p.dim() > 1:
+                p.normal_(0, p.shape[-1] ** -0.5)
+    m = lfmq.quantize(m, lfmq.QuantConfig(scheme="rtn", bits=4, group_size=128,
+                                          skip_modules=("lm_head",)))
+    cache = m.make_cache(batch, max_seq=T + 8)
+    for t in (cache.k_all, cache.v_all):
+        t[:, :, :, :T].normal_()
+    state = torch.tensor([T, T + 1, 0], dtype=torch.int32, device=DEV)
+    ids = torch.randint(512, (batch, 1), device=DEV)
+    step = lambda: m.forward_decode_step(ids, cache, state, T + 8)
+    step()
+    found = []
+    parts = F.dq_linear_parts
+    monkeypatch.setattr(F, "dq_linear_parts",
+                        lambda *a: found.append(parts(*a)) or found[-1])
+    want = step()
+    assert len(found) == 2 and all(y is not None for y in found)
+    assert not bool(cache.tickets.any())
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        logits = step()
+    for _ in range(3):
+        logits.zero_()
+        graph.replay()
+        assert torch.equal(logits, want)
+        assert torch.equal(step(), want)
+        assert not bool(cache.tickets.any())
+    monkeypatch.setattr(F, "dq_linear_parts", lambda *a: None)
+    plain = step()
+    # roundings of 2^-9 in two layers' products and the head's
+    assert not torch.equal(plain, want)
+    assert float((plain.double() - want.double()).norm() / want.double().norm()) < 2e-2
