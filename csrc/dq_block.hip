@@ -47,17 +47,6 @@ constexpr int NW = 8, TPB = NW * LFMQ_WAVE, NT = 2, BN = NW * NT * 16;
 constexpr int ROWS = 128;                        // of a tile, at most
 constexpr int D = 3;                             // stages
 
-__device__ __forceinline__ void load4_to_lds(const void* base, u32 off,
-                                             u32 lds) {
-  asm volatile(
-      "s_mov_b32 m0, %0\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dword %1, %2"
-      :
-      : "s"(lds), "v"(off), "s"(base)
-      : "memory", "m0");
-}
-
 // LDS: x [D][rows][KC], weights [D][NW][..], two blocks of scales and of zeros
 // of eight groups, eight chunks' sums of x
 template <int BITS, int KC>

@@ -10,8 +10,13 @@
 //
 // - sum s (c - z) x = s (sum c x) - (s z) (sum x), and the sums of x's groups come from
 //   a launch before, instead of from each of the workgroups of its rows.  The second
-//   term is a product of bf16 parts, exact but for the last (times_sums), before the
-//   loop: 8 k a group of 128 and at the rate of the first, an eighth of that in fp32.
+//   term is a product of bf16 parts, exact but for the last (times_sums): 8 k a group of
+//   128 and at the rate of the first, an eighth of that in fp32.  It is taken off eight
+//   groups at a time, halfway through them, so that what cancels stays small; all of it
+//   before the loop is 1 % faster with 8 bits, but of x with a mean of one deviation, k
+//   14336, the result was 2.4e-5 off (8 bits, groups of 64; 4 bits, of 128 3.5e-6) and
+//   is 6.8e-7 (3.0e-7), with a mean of zero 6.9e-7 and 4.0e-7 (dq_block: 6.6e-7, 1.6e-7
+//   and 4.0e-7).
 // - 32 x 32 products, half as many instructions; a wave's 32 columns are one, and two
 //   row tiles go side by side over half a chunk's k.  A half's products hide the
 //   scaling of the chunk before or the unpacking of the half to come.
@@ -24,11 +29,11 @@
 //
 // us a call, dq_block and this one with the sums (groups of 128; 8 bits, of 64):
 //                            2048 rows     3001 rows
-//   n 28672, k 4096          481 / 451     720 / 663
-//   n 6144, k 4096           122 / 116     164 / 155
-//   n 4096, k 14336          231 / 223     345 / 331
-//   n 28672, k 4096 (8)      595 / 547     893 / 836
-//   n 8192, k 8192 (8)       327 / 307     489 / 452
+//   n 28672, k 4096          471 / 445     705 / 657
+//   n 6144, k 4096           116 / 115     167 / 157
+//   n 4096, k 14336          228 / 219     338 / 332
+//   n 28672, k 4096 (8)      595 / 562     887 / 838
+//   n 8192, k 8192 (8)       341 / 329     486 / 468
 #include "dq_block.h"
 #include "lds_dma.h"
 
@@ -41,16 +46,16 @@ typedef u32 u32x2 __attribute__((ext_vector_type(2)));
 constexpr int NW = 8, TPB = NW * LFMQ_WAVE, BN = NW * 32;
 constexpr int ROWS = 128;                        // of a tile, at most
 constexpr int D = 3;                             // stages
+constexpr int SUMS = 48;                         // bytes of eight groups' sums
 
 // LDS: x [D][rows][KC], weights [D][BN][..], two blocks of scales of eight groups;
-// sums of x of 32 groups, where x's last stage comes or beside it
+// zeros and sums of x of one
 template <int BITS, int KC>
 struct Lds {
   static constexpr int XB = ROWS * KC * 2, WB = BN * KC * BITS / 8;
   static constexpr int W = D * XB, S = W + D * WB;
-  static constexpr int SB = BN * 16, END = S + 2 * SB;
-  static constexpr int SUM = KC == 128 ? (D - 1) * XB : END;
-  static constexpr int BYTES = KC == 128 ? END : END + ROWS * 256;
+  static constexpr int SB = BN * 16, Z = S + 2 * SB, SUM = Z + BN * BITS;
+  static constexpr int BYTES = SUM + ROWS * SUMS;
   static_assert(BYTES <= 160 * 1024 && BYTES >= ROWS * (BN + 8) * 2, "");
 };
 
@@ -64,11 +69,11 @@ __device__ __forceinline__ s16x8 times_sums(float v) {
   return __builtin_bit_cast(s16x8, u32x4{h | h << 16, h, l | l << 16, l});
 }
 
-// sums [m, k / g] of x's groups, each as -(a, b, c, 0) in bf16 with a + b + c the sum
-// in fp32.  Eight lanes a group, 128 bytes of a row.  Bound by reading x:
-// 3001 x 4096 7 us.
+// sums [m, k / g] of x's groups, each as -(a, b, c) in bf16 with a + b + c the sum in
+// fp32: of eight groups a and b, and then c.  Eight lanes a group, 128 bytes of a row.
+// Bound by reading x: 3001 x 4096 7 us.
 __global__ __launch_bounds__(256) void dq_panel_sums(
-    const unsigned short* __restrict__ x, u64* __restrict__ sums, u32 groups,
+    const unsigned short* __restrict__ x, char* __restrict__ sums, u32 groups,
     int g) {
   const u32 id = blockIdx.x * 32 + threadIdx.x / 8;
   if (id >= groups) return;
@@ -87,14 +92,15 @@ __global__ __launch_bounds__(256) void dq_panel_sums(
   const float ra = -sum - bf16_bits_to_f32(a);
   const u32 b = f32_to_bf16_bits_rne(ra);
   const u32 c = f32_to_bf16_bits_rne(ra - bf16_bits_to_f32(b));
-  sums[id] = a | b << 16 | (u64)c << 32;
+  char* to = sums + (u64)(id / 8) * SUMS;
+  ((u32*)to)[id % 8] = a | b << 16;
+  ((unsigned short*)to)[16 + id % 8] = (unsigned short)c;
 }
 
-// the result's tile of column block nblk, part of it
 // the result's tile of column block nblk, part of it: MT row tiles of 32
 template <int BITS, int KC, DqMode MODE, int MT>
 __device__ __forceinline__ void dq_panel_body(const DqArgs& A,
-                                              const u64* sums_of_x, char* smem,
+                                              const char* sums_of_x, char* smem,
                                               const DqBlockTile& T) {
   typedef Lds<BITS, KC> L;
   constexpr int BM = MT * 32, J = KC / 16;       // products of 16 k a chunk
@@ -166,55 +172,48 @@ __device__ __forceinline__ void dq_panel_body(const DqArgs& A,
                   L::S + (q & 1) * L::SB + wave * 1024);
   };
 
-  f32x16 acc[MT] = {};
-  // acc -= (scale times zero) (sums of x) of this part's share of the groups, two
-  // to a product, 32 at a time by way of LDS
-  // (a division leaves them in vector registers)
-  const int q0 = __builtin_amdgcn_readfirstlane(G / 8 * sp / parts);
-  const int q1 = __builtin_amdgcn_readfirstlane(G / 8 * (sp + 1) / parts);
+  // zeros of groups 8 q .. 8 q + 7, and sums of x
+  constexpr int NS = (BM * SUMS + 1023) / 1024;  // 1 KiB loads
+  const u32 zo = mcol * (zw * 4) + (wave >> 2) * 4;
+  u32 so;
+  {
+    const int e = min(wave * 64 + lane, BM * 3 - 1);
+    so = (u32)x_row(e / 3) * (G / 8 * SUMS) + e % 3 * 16;
+  }
   auto load_sums = [&](int q) {
+    if (BITS == 8 || wave < 4)
+      load4_to_lds((const char*)(A.zeros + first * zw) + q * BITS, zo,
+                   L::Z + wave * 256);
+    if (wave < NS) load_to_lds(sums_of_x + q * SUMS, so, L::SUM + wave * 1024);
+  };
+  f32x16 acc[MT] = {};
+  // acc -= (scale times zero) (sums of x) of these groups, two to a product
+  u32x4 ab[MT];                                  // a and b of this lane's four, and c
+  u32x2 ec[MT], zs;
+  u32 zz;
+  auto read_zeros = [&](int q) {
+    const int col = wave * 32 + l31;
+    zs = *(const u32x2*)(smem + L::S + (q & 1) * L::SB + col * 16 + hi * 8);
+    zz = *(const u32*)(smem + L::Z + col * 4 + (BITS == 8 ? hi * 1024 : 0));
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const int at = (i * NW + wave) * 4 + lane / 16;
-      const int slot = (lane % 16) ^ slot_key<16>(at);
-      load_to_lds(sums_of_x,
-                  (u32)x_row(at) * (G * 8) + min(q * 4 + slot, q1 * 4 - 1) * 16,
-                  L::SUM + (i * NW + wave) * 1024);
+    for (int t = 0; t < MT; ++t) {
+      const char* p = smem + L::SUM + (t * 32 + l31) * SUMS;
+      ab[t] = *(const u32x4*)(p + hi * 16);
+      ec[t] = *(const u32x2*)(p + 32 + hi * 8);
     }
   };
-  u32x2 zs[4];                                   // four groups' scales, eights
-  u32 zz[4];                                     // and zeros
-  auto load_zeros = [&](int q) {
-    const u64 col = first + column(wave * 32 + l31);
+  auto zeros_term = [&]() {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int qi = min(q + i, q1 - 1);
-      zs[i] = *(const u32x2*)(A.scales + col * G + qi * 8 + hi * 4);
-      zz[i] = A.zeros[col * zw + (BITS == 8 ? qi * 2 + hi : qi)];
-    }
-  };
-  auto zeros_term = [&](int q) {
+    for (int e = 0; e < 4; ++e) {
+      const u32 zero = BITS == 4 ? unpack4(zz, hi * 4 + e) : unpack8(zz, e);
+      const u32 scale = e & 1 ? zs[e / 2] >> 16 : zs[e / 2] & 0xFFFFu;
+      const s16x8 w = times_sums(bf16_bits_to_f32(scale) * (float)zero);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (q + i >= q1) break;
-      u32x4 v[MT][2];
-#pragma unroll
-      for (int t = 0; t < MT; ++t)
-#pragma unroll
-        for (int e = 0; e < 2; ++e)
-          v[t][e] = *(const u32x4*)(smem + L::SUM + (t * 32 + l31) * 256 +
-                                    (((i * 4 + hi * 2 + e) ^ slot_key<16>(l31)) << 4));
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const u32 zero = BITS == 4 ? unpack4(zz[i], hi * 4 + e) : unpack8(zz[i], e);
-        const u32 scale = e & 1 ? zs[i][e / 2] >> 16 : zs[i][e / 2] & 0xFFFFu;
-        const s16x8 w = times_sums(bf16_bits_to_f32(scale) * (float)zero);
-#pragma unroll
-        for (int t = 0; t < MT; ++t) {
-          const u32 lo = v[t][e / 2][e % 2 * 2], up = v[t][e / 2][e % 2 * 2 + 1];
-          acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              __builtin_bit_cast(s16x8, u32x4{lo, up, lo, up}), w, acc[t], 0, 0, 0);
-        }
+      for (int t = 0; t < MT; ++t) {
+        const u32 lo = ab[t][e];
+        const u32 up = e & 1 ? ec[t][e / 2] >> 16 : ec[t][e / 2] & 0xFFFFu;
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            __builtin_bit_cast(s16x8, u32x4{lo, up, lo, up}), w, acc[t], 0, 0, 0);
       }
     }
   };
@@ -255,11 +254,9 @@ __device__ __forceinline__ void dq_panel_body(const DqArgs& A,
 
   int gi = c0 / cpg, gc = c0 % cpg;              // group, chunk in it
   const int m0 = gi >> 3;
+  const int first_q = (c0 + 4 * cpg - 1) / (8 * cpg);  // half of it in this part
   {
-    if (q0 < q1) {
-      load_zeros(q0);
-      load_sums(q0);
-    }
+    load_sums(min(first_q, G / 8 - 1));
 #pragma unroll
     for (int i = 0; i < NL; ++i) load_w(c0, 0, i);
     load_meta(m0);
@@ -271,19 +268,7 @@ __device__ __forceinline__ void dq_panel_body(const DqArgs& A,
 #pragma unroll
       for (int i = 0; i < NL; ++i) load_w(min(c0 + t + 1, c1 - 1), t + 1, i);
     }
-    for (int q = q0;;) {
-      loads_but<0>();
-      if (q >= q1) break;
-      zeros_term(q);
-      q += 4;
-      if (q >= q1) {
-        __syncthreads();                         // the sums are read
-        break;
-      }
-      load_zeros(q);
-      __syncthreads();
-      load_sums(q);
-    }
+    loads_but<0>();
     read_w(0);
     read_meta(gi);
     read_x(0, 0, 0, xa[0]);
@@ -303,6 +288,17 @@ __device__ __forceinline__ void dq_panel_body(const DqArgs& A,
     const int b1 = buf == D - 1 ? 0 : buf + 1, b2 = b1 == D - 1 ? 0 : b1 + 1;
     if (gc == 0 && (gi & 7) == 0 && gi >> 3 != m0 && gi + 8 < G)
       load_meta((gi >> 3) + 1);
+    // Zeros' terms of eight groups halfway through them (behind the first products, where
+    // there are registers for their operands: 8 bits 2 % slower than without a term in
+    // the loop, 1 % so), and the next ones' operands a chunk later, when all waves have
+    // read these.
+    const int cz = ((gi & 7) - 4) * cpg + gc;
+    if (cz == 0) {
+      read_zeros(gi >> 3);
+      if (KC == 128) zeros_term();
+    } else if (cz == 1 && (gi | 7) + 1 < G) {
+      load_sums((gi >> 3) + 1);
+    }
     if (++gc == cpg) {
       gc = 0;
       ++gi;
@@ -344,6 +340,7 @@ __device__ __forceinline__ void dq_panel_body(const DqArgs& A,
         }
 #pragma unroll
       for (int j = g * JH / NG; j < (g + 1) * JH / NG; ++j) unpack(h ^ 1, j);
+      if (KC == 64 && u == 0 && cz == 0) zeros_term();
       if (u == NG - 1) s = bf16_bits_to_f32(meta);
       if (u == U - 1) read_meta(gi);
       __builtin_amdgcn_sched_barrier(0);
@@ -415,7 +412,7 @@ __device__ __forceinline__ void dq_panel_body(const DqArgs& A,
 
 template <int BITS, int KC, DqMode MODE>
 __global__ __launch_bounds__(TPB, 2) void dq_panel_kernel(DqArgs A, Plan P,
-                                                          const u64* sums) {
+                                                          const char* sums) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const u32 nb = MODE == GLU ? (A.n / 2 + BN / 2 - 1) / (BN / 2)
                              : (A.n + BN - 1) / BN;
@@ -433,7 +430,7 @@ __global__ __launch_bounds__(TPB, 2) void dq_panel_kernel(DqArgs A, Plan P,
 }
 
 template <int BITS, int KC, DqMode MODE>
-hipError_t go(const DqArgs& A, const Plan& P, u32 wgs, const u64* sums,
+hipError_t go(const DqArgs& A, const Plan& P, u32 wgs, const char* sums,
               hipStream_t stream) {
   constexpr int lds = Lds<BITS, KC>::BYTES;
   static bool set = false;
@@ -451,7 +448,7 @@ hipError_t go(const DqArgs& A, const Plan& P, u32 wgs, const u64* sums,
 
 template <DqMode MODE>
 hipError_t go_bits(const DqArgs& A, const Plan& P, int bits, u32 wgs,
-                   const u64* sums, hipStream_t stream) {
+                   const char* sums, hipStream_t stream) {
   if (bits == 4)
     return A.g % 128 == 0 ? go<4, 128, MODE>(A, P, wgs, sums, stream)
                           : go<4, 64, MODE>(A, P, wgs, sums, stream);
@@ -475,9 +472,9 @@ hipError_t lfmq_dq_panel(const DqArgs& A, const DqBlockPlan& P, int bits, DqMode
   const long groups = rows * (A.k / A.g);
   if (groups < 1 || groups * 8 >= 1l << 32) return hipErrorInvalidValue;
   hipLaunchKernelGGL(dq_panel_sums, dim3(ceil_div_u32((u32)groups, 32)), dim3(256), 0,
-                     stream, (const unsigned short*)A.x, (u64*)sums, (u32)groups, A.g);
+                     stream, (const unsigned short*)A.x, (char*)sums, (u32)groups, A.g);
   LFMQ_CHECK_HIP(hipGetLastError());
-  const u64* s = (const u64*)sums;
+  const char* s = (const char*)sums;
   return mode == DENSE ? go_bits<DENSE>(A, P, bits, wgs, s, stream)
          : mode == GLU ? go_bits<GLU>(A, P, bits, wgs, s, stream)
                        : go_bits<SLOTS>(A, P, bits, wgs, s, stream);

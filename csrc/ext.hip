@@ -264,7 +264,7 @@ torch::Tensor panel_sums(const torch::Tensor& x, long rows, long n, long g,
                          long bits) {
   const long k = x.size(1), groups = x.size(0) * (k / g);
   if (!lfmq_dq_panel_gains(rows, n, k, g, bits) || groups * 8 >= 1l << 32) return {};
-  return torch::empty({groups}, x.options().dtype(torch::kInt64));
+  return torch::empty({groups * 3 / 2}, x.options().dtype(torch::kInt32));
 }
 
 void dq_block(const torch::Tensor& x, const torch::Tensor& qweight,

@@ -17,6 +17,18 @@ __device__ __forceinline__ void load_to_lds(const void* base, u32 off,
       : "memory", "m0");
 }
 
+// the same with 4 bytes a lane
+__device__ __forceinline__ void load4_to_lds(const void* base, u32 off,
+                                             u32 lds) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dword %1, %2"
+      :
+      : "s"(lds), "v"(off), "s"(base)
+      : "memory", "m0");
+}
+
 // own loads have landed, everybody's after the barrier
 __device__ __forceinline__ void lds_loads_done() {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
