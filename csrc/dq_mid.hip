@@ -359,12 +359,11 @@ __global__ __launch_bounds__(TPB, 2) void dq_mid_kernel(DqArgs A, int mb, int st
         unpack(b[PAR ^ 1], i);
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (FIRST) {                                 // a's group (none past the last)
-      const bool in = turn * KW + kw < ng;
+    if (FIRST) {                                 // a's group
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         zp[t] = z[t];
-        sc[t] = in ? __builtin_bit_cast(float, m0[t] & 0xFFFF0000u) : 0.f;
+        sc[t] = __builtin_bit_cast(float, m0[t] & 0xFFFF0000u);
         z[t] = sc[t] * (float)(m0[t] & 0xFFFFu);
       }
     }
@@ -399,8 +398,13 @@ __global__ __launch_bounds__(TPB, 2) void dq_mid_kernel(DqArgs A, int mb, int st
     }
     if (i < turns) one(i, even, yes);
   }
+  // (waves past the last group have nothing of it, which is not 0 times what they have:
+  // that may be infinite)
+  const bool in = kw < left;
+  if (in) {
 #pragma unroll
-  for (int t = 0; t < MT; ++t) fold(t);
+    for (int t = 0; t < MT; ++t) fold(t);
+  }
   loads_but<0>();
   if constexpr (BITS == 4) {
     if (GS == 1) {
@@ -408,9 +412,11 @@ __global__ __launch_bounds__(TPB, 2) void dq_mid_kernel(DqArgs A, int mb, int st
 #pragma unroll
       for (int t = 0; t < MT; ++t) fold_zeros(t, zp);
     }
-    read_sums(turns - 1);
+    if (in) {
+      read_sums(turns - 1);
 #pragma unroll
-    for (int t = 0; t < MT; ++t) fold_zeros(t, z);
+      for (int t = 0; t < MT; ++t) fold_zeros(t, z);
+    }
   }
   // the k waves' sums
   constexpr int LD = BN + 4;

@@ -44,19 +44,61 @@ def test_many_rows_of_large_products(bits, m, n, k, g):
     assert "dq_panel_kernel" in launched(lambda: test_many_rows(bits, m, n, k, g))
 
 
-# dq_wide, dq_short (k whole, and in parts), dq_block and dq_panel
-@pytest.mark.parametrize("m,n,k", [(8, 8200, 2048), (40, 4104, 4096),
-                                   (100, 4104, 2048), (200, 512, 4096),
-                                   (300, 8200, 8192)])
-def test_values_that_are_not_finite_stay_in_their_rows(m, n, k):
+# (k whole, and in parts)
+@pytest.mark.parametrize("kernel,bits,m,n,k,g", [
+    ("dq_wide_kernel", 4, 8, 8200, 2048, 128), ("dq_mid_kernel", 4, 40, 4104, 4096, 128),
+    ("dq_mid_kernel", 4, 100, 4104, 2048, 128), ("dq_mid_kernel", 4, 200, 512, 4096, 128),
+    ("dq_mid_kernel", 8, 40, 4104, 4160, 64), ("dq_mid_kernel", 8, 200, 512, 4224, 128),
+    ("dq_short_kernel", 4, 40, 4098, 4096, 128),
+    ("dq_short_kernel", 4, 100, 4102, 2048, 128),
+    ("dq_short_kernel", 8, 100, 4102, 2048, 64),
+    ("dq_block_kernel", 4, 200, 514, 4096, 128), ("dq_block_kernel", 8, 200, 514, 4096, 64),
+    ("dq_panel_kernel", 4, 300, 8200, 8192, 128),
+    ("dq_panel_kernel", 8, 300, 8200, 8192, 64)])
+def test_values_that_are_not_finite_stay_in_their_rows(kernel, bits, m, n, k, g):
     torch.manual_seed(0)
-    p, w = matrix(4, n, k, 128)
+    p, w = matrix(bits, n, k, g)
     x = torch.randn(m, k, device=DEV).to(BF)
     x[3, 7], x[m * 2 // 3, k - 96] = float("inf"), float("nan")
-    y = ext().dq_linear(x, *p, 4, 128, None, None, -1.0, 0)
+    got = []
+    assert kernel in launched(lambda: got.append(
+        ext().dq_linear(x, *p, bits, g, None, None, -1.0, 0)))
+    fine = torch.isfinite(x).all(1)
+    assert not bool(torch.isfinite(got[0][~fine]).any())
+    close(got[0][fine], x[fine].double() @ w.t())
+
+
+@pytest.mark.parametrize("bits,m,g", [(4, 8, 128), (8, 16, 64)])
+def test_values_that_are_not_finite_and_k_in_parts(bits, m, g):
+    n, k = 4096, 14336
+    torch.manual_seed(0)
+    p, w = matrix(bits, n, k, g)
+    x = torch.randn(m, k, device=DEV).to(BF)
+    x[3, 7], x[m * 2 // 3, k - 96] = float("inf"), float("nan")
+    tickets = torch.zeros(128, dtype=torch.int32, device=DEV)
+    y = ext().dq_linear_parts(x, *p, bits, g, None, None, tickets)
     fine = torch.isfinite(x).all(1)
     assert not bool(torch.isfinite(y[~fine]).any())
     close(y[fine], x[fine].double() @ w.t())
+
+
+@pytest.mark.parametrize("m,n,k,g", [(40, 4104, 4160, 64), (40, 4104, 4224, 128),
+                                     (100, 2056, 2112, 64), (200, 512, 4160, 64)])
+def test_an_infinite_value_gives_infinite_products(m, n, k, g):
+    """8 bits, whose codes less their zeros are exact: what IEEE 754 has for them, and
+    nothing of a group that a wave has beside others' (the last of a part)."""
+    torch.manual_seed(m)
+    p, w = matrix(8, n, k, g)
+    x = torch.randn(m, k, device=DEV).to(BF)
+    at = torch.arange(m, device=DEV) * (k // g - 1) // (m - 1) * g + 5
+    x[torch.arange(m, device=DEV), at] = float("inf")
+    got = []
+    assert "dq_mid_kernel" in launched(lambda: got.append(
+        ext().dq_linear(x, *p, 8, g, None, None, -1.0, 0)))
+    sign = w.t()[at].sign()                      # of the product with infinity
+    want = torch.where(sign == 0, float("nan"), sign * float("inf"))
+    assert torch.equal(got[0].isnan(), want.isnan())
+    assert bool((got[0].double() == want)[sign != 0].all())
 
 
 @pytest.mark.parametrize("bits,n,k,g", [(4, 2062, 2048, 128),
