@@ -331,7 +331,7 @@ def test_norm_after_a_product(m, n, k, g, bits, shift):
 
 
 @pytest.mark.parametrize("m,n,k,g", [
-    (17, 5120, 256, 128), (48, 8200, 2112, 64), (33, 32008, 192, 64),
+    (40, 10240, 256, 128), (48, 8200, 2112, 64), (33, 32008, 192, 64),
     (49, 3072, 1024, 64), (64, 2056, 2048, 128), (77, 16384, 2048, 64),
     (81, 1544, 2688, 192), (96, 2048, 2048, 64), (97, 2048, 3072, 64),
     (113, 2504, 2560, 256), (128, 8192, 1024, 128), (49, 2048, 8192, 64),
@@ -348,8 +348,8 @@ def test_eight_waves_along_k(m, n, k, g):
     x[0] = 0
     bias = torch.randn(n, device=DEV).to(BF)
     plain = x.double() @ w.t()
-    close(ext().dq_linear(x, *p, 8, g, bias, None, -1.0, 0),
-          plain + bias.double())
+    assert "dq_mid_kernel" in launched(lambda: close(
+        ext().dq_linear(x, *p, 8, g, bias, None, -1.0, 0), plain + bias.double()))
     close(ext().dq_gemv_gateup(x, *p, 8, g, -1.0, 0), gated(plain), 1e-2)
     if m <= 48:
         resid = torch.randn(m, n, device=DEV).to(BF)
@@ -364,9 +364,9 @@ def test_eight_waves_along_k(m, n, k, g):
 
 @pytest.mark.parametrize("m,n,k,g", [
     (17, 28680, 1024, 128), (48, 8200, 2112, 64), (33, 32008, 832, 64),
-    (25, 1024, 768, 64), (33, 2008, 896, 128), (40, 28672, 4096, 128),
+    (25, 1024, 1280, 64), (33, 2008, 896, 128), (50, 4096, 256, 128), (40, 28672, 4096, 128),
     (48, 6144, 4096, 128), (64, 2056, 2048, 128), (77, 16384, 2048, 64),
-    (81, 1544, 2688, 192), (90, 8200, 896, 128), (97, 2048, 3072, 64),
+    (81, 1544, 2688, 192), (90, 6136, 896, 128), (97, 2048, 3072, 64),
     (100, 512, 4992, 128), (113, 2504, 2560, 256), (128, 8192, 1024, 128),
     (65, 1032, 14336, 64), (80, 10240, 4096, 128)])
 def test_eight_waves_along_k_of_four_bits(m, n, k, g):
@@ -379,8 +379,8 @@ def test_eight_waves_along_k_of_four_bits(m, n, k, g):
     x[0] = 0
     bias = torch.randn(n, device=DEV).to(BF)
     plain = x.double() @ w.t()
-    close(ext().dq_linear(x, *p, 4, g, bias, None, -1.0, 0),
-          plain + bias.double())
+    assert "dq_mid_kernel" in launched(lambda: close(
+        ext().dq_linear(x, *p, 4, g, bias, None, -1.0, 0), plain + bias.double()))
     close(ext().dq_gemv_gateup(x, *p, 4, g, -1.0, 0), gated(plain), 1e-2)
     if m <= 48:
         resid = torch.randn(m, n, device=DEV).to(BF)
@@ -392,7 +392,7 @@ def test_eight_waves_along_k_of_four_bits(m, n, k, g):
 
 
 @pytest.mark.parametrize("bits,m,n,k,g", [
-    (4, 129, 2048, 2048, 64), (8, 161, 16384, 2048, 64), (4, 200, 4104, 4096, 128),
+    (4, 129, 2048, 2048, 64), (8, 161, 16384, 2048, 64), (4, 200, 4104, 3072, 128),
     (8, 300, 2048, 2048, 128), (4, 511, 1032, 1920, 64), (8, 512, 2056, 2688, 192),
     (4, 385, 520, 4992, 128), (8, 256, 4096, 4096, 64), (4, 512, 3072, 768, 128),
     (8, 768, 2048, 2048, 64), (4, 673, 2048, 2048, 128)])
@@ -403,8 +403,8 @@ def test_eight_waves_of_many_rows(bits, m, n, k, g):
     x = torch.randn(m, k, device=DEV).to(BF)
     bias = torch.randn(n, device=DEV).to(BF)
     plain = x.double() @ w.t()
-    close(ext().dq_linear(x, *p, bits, g, bias, None, -1.0, 0),
-          plain + bias.double())
+    assert "dq_mid_kernel" in launched(lambda: close(
+        ext().dq_linear(x, *p, bits, g, bias, None, -1.0, 0), plain + bias.double()))
     close(ext().dq_gemv_gateup(x, *p, bits, g, -1.0, 0), gated(plain), 1e-2)
 
 

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 # that end inside a wave's columns, or between pieces of 16 bytes; one group a
 # chunk and several; four chunks up, whole, split, and some tiles split.
 @pytest.mark.parametrize("bits,m,n,k,g", [
-    (4, 129, 264, 1024, 128), (4, 180, 1041, 2048, 128), (4, 256, 520, 1024, 64),
+    (4, 129, 264, 1024, 128), (4, 180, 1041, 2048, 128), (4, 256, 522, 1024, 64), (4, 256, 520, 1024, 64),
     (4, 150, 2062, 5120, 128), (4, 300, 258, 8192, 512), (4, 130, 300, 512, 64),
     (4, 2100, 4352, 1024, 128), (4, 1100, 8450, 1536, 64),
     (8, 129, 264, 512, 64), (8, 256, 1030, 2048, 64), (8, 150, 519, 1024, 64),
@@ -123,21 +123,23 @@ def test_many_rows_by_expert(bits, n, k, g):
         at += c
     tiles = torch.tensor(tiles + [(-1, 0, 0)], dtype=torch.int32, device=DEV)
     want, s32 = torch.cat(want), src.to(torch.int32)
-    close(ext().moe_linear(x, s32, tiles, *p, bits, g, True, 128), gated(want),
-          1e-2)
-    close(ext().moe_linear(x[src], None, tiles, *p, bits, g, False, 128), want)
+    names = launched(lambda: close(
+        ext().moe_linear(x, s32, tiles, *p, bits, g, True, 128), gated(want), 1e-2))
+    names |= launched(lambda: close(
+        ext().moe_linear(x[src], None, tiles, *p, bits, g, False, 128), want))
+    assert ("dq_panel_kernel" in names) == (n * k > 20 << 20), names
 
 
 # Row tiles of 32 to 128, one to three of them; columns that end inside a wave's;
 # k whole and in parts, with more groups to a part than LDS holds and with
 # groups of 64's multiples; the residual, which a step of 48 sequences has.
 @pytest.mark.parametrize("bits,m,n,k,g", [
-    (4, 17, 4098, 4096, 128), (4, 33, 4104, 4160, 64), (8, 48, 4099, 4096, 128),
+    (4, 17, 4098, 4096, 128), (4, 33, 5130, 4160, 64), (8, 48, 4099, 4096, 128),
     (8, 40, 24580, 2112, 64), (4, 49, 2100, 2112, 64), (4, 80, 4098, 1152, 128),
-    (4, 64, 5001, 1024, 256), (8, 65, 2062, 2112, 64), (8, 96, 16400, 2112, 64),
+    (4, 64, 5001, 1024, 256), (8, 65, 2062, 2112, 64), (8, 96, 16402, 2112, 64),
     (4, 113, 4098, 1024, 128), (4, 128, 4102, 1152, 64), (8, 97, 2054, 2304, 128),
     (8, 128, 16386, 2048, 64), (8, 77, 32770, 1024, 128), (4, 33, 33026, 2048, 128),
-    (4, 33, 5128, 4160, 64)])
+    (4, 33, 4104, 4160, 64), (8, 96, 16400, 2112, 64), (4, 33, 5128, 4160, 64)])
 def test_some_rows(bits, m, n, k, g):
     torch.manual_seed(m + n)
     p, w = matrix(bits, n, k, g)
@@ -145,8 +147,10 @@ def test_some_rows(bits, m, n, k, g):
     x[0] = 0
     bias = torch.randn(n, device=DEV).to(BF)
     plain = x.double() @ w.t()
-    close(ext().dq_linear(x, *p, bits, g, bias, None, -1.0, 0),
-          plain + bias.double())
+    # (columns in eights are dq_mid's)
+    kernel = "dq_mid_kernel" if n % 8 == 0 else "dq_short_kernel"
+    assert kernel in launched(lambda: close(
+        ext().dq_linear(x, *p, bits, g, bias, None, -1.0, 0), plain + bias.double()))
     if m <= 48:
         resid = torch.randn(m, n, device=DEV).to(BF)
         close(ext().dq_linear(x, *p, bits, g, None, resid, -1.0, 0),
