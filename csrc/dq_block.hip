@@ -21,15 +21,19 @@
 // split and a second launch adds the parts (3001 rows: n 4096, k 14336 399 us,
 // 343 so; n 6144, k 4096 172, 164).
 //
+// What is large (rows k (n - 2048) from 12 2^30 on, 8 2^30 with stages of 64) is
+// dq_panel's now, which measures itself against this kernel; the calls below that
+// are marked * are among it, and so is what the next lines are about.
+//
 // Bound by the matrix cores (busy 57 % of the time), by what the two waves of a
 // SIMD wait for together at the barrier, and by 7 us of first loads and last
 // stores of a tile of 66 that nothing covers.  us a call, dq_tile and this one
 // (4 bits; 8 bits with groups of 64 at k 2048 and 8192):
 //                       200 rows      500 rows      1500 rows     3001 rows
-//   n 28672, k 4096   80.2 / 63.4   155 / 137     438 / 368     815 / 703
-//   n 6144, k 4096    33.0 / 28.6   51.1 / 41.8   118 / 90.2    205 / 164
-//   n 4096, k 14336   51.8 / 41.3   91.5 / 77.8   230 / 180     451 / 343
-//   n 16384, k 2048   42.6 / 34.7   60.9 / 48.6   176 / 141     330 / 272
+//   n 28672, k 4096   80.2 / 63.4*  155 / 137*    438 / 368*    815 / 703*
+//   n 6144, k 4096    33.0 / 28.6   51.1 / 41.8   118 / 90.2*   205 / 164*
+//   n 4096, k 14336   51.8 / 41.3   91.5 / 77.8*  230 / 180*    451 / 343*
+//   n 16384, k 2048   42.6 / 34.7   60.9 / 48.6*  176 / 141*    330 / 272*
 //   n 2048, k 8192    30.5 / 27.6   45.5 / 37.8   125 / 88.5    199 / 146
 // Without effect: the order of products and sums, wave priorities, x fetched two
 // row tiles ahead.  LDS slots that pairs of lanes share (slot_key): 767 us

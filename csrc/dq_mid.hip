@@ -111,7 +111,8 @@ __global__ __launch_bounds__(TPB, 2) void dq_mid_kernel(DqArgs A, int mb, int st
   const int S = turns * GS;                      // steps
   const int half = A.n / 2, n0 = nblk * BO;
   auto column = [&](int c) {
-    if (MODE == GLU) return (c >> 4 & 1) * half + min(n0 + (c >> 5) * 16 + (c & 15), half - 1);
+    if (MODE == GLU)
+      return (c >> 4 & 1) * half + min(n0 + (c >> 5) * 16 + (c & 15), half - 1);
     return min(n0 + c, A.n - 1);
   };
   const char* xb = (const char*)(A.x + (u64)row0 * A.k);
@@ -428,7 +429,8 @@ __global__ __launch_bounds__(TPB, 2) void dq_mid_kernel(DqArgs A, int mb, int st
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        red[(kw * BM + t * 16 + l4 * 4 + r) * LD + (wc * NT + nt) * 16 + l15] = acc[t][nt][r];
+        red[(kw * BM + t * 16 + l4 * 4 + r) * LD + (wc * NT + nt) * 16 + l15] =
+            acc[t][nt][r];
   __syncthreads();
   for (int i = tid; i < BM * BO / 4; i += TPB) {
     const int row = i / (BO / 4), c = i % (BO / 4) * 4;

@@ -466,7 +466,7 @@ torch::Tensor linear(torch::Tensor x, const torch::Tensor& qweight,
     rptr = resid->data_ptr();
   }
   auto y = torch::empty({m, n}, x.options());
-  // What is left by dq_row, dq_wide, dq_short and dq_block, whose rules go
+  // What is left by dq_row, dq_wide, dq_mid, dq_short and dq_block, whose rules go
   // first: a wave a few columns (GEMV), rows of x in registers, x through LDS.  us
   // of the last two: n 3072, k 8192 (4 bits) 14.5 / 17.1 at 32 rows, 17.7 / 17.1 at
   // 33, 25.5 / 18.7 at 49; n 16384, k 2048 (8 bits, groups of 64) 18.4 / 21.4 at 48,
