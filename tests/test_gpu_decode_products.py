@@ -330,6 +330,30 @@ def test_norm_after_a_product(m, n, k, g, bits, shift):
     assert float(((h.double() - want).abs() / (want.abs() + 1e-6)).max()) < 4.1e-3
 
 
+def with_its_ways(bits, m, n, k, g):
+    """A product with a bias; with the gate; of up to 48 rows, with a residual and
+    with factors of rows.  Returns the first one's kernels."""
+    torch.manual_seed(n + m)
+    p, w = matrix(bits, n, k, g)
+    x = torch.randn(m, k, device=DEV).to(BF)
+    x[0] = 0
+    bias = torch.randn(n, device=DEV).to(BF)
+    plain = x.double() @ w.t()
+    names = launched(lambda: close(
+        ext().dq_linear(x, *p, bits, g, bias, None, -1.0, 0), plain + bias.double()))
+    close(ext().dq_gemv_gateup(x, *p, bits, g, -1.0, 0), gated(plain), 1e-2)
+    if m <= 48:
+        resid = torch.randn(m, n, device=DEV).to(BF)
+        scale = torch.rand(m, device=DEV) + 0.5
+        close(ext().dq_linear(x, *p, bits, g, bias, resid, -1.0, 0),
+              plain + bias.double() + resid.double())
+        want = plain * scale.double().unsqueeze(1)
+        y, _ = ext().dq_linear_scaled(x, scale, *p, bits, g, None, resid, 1e-5)
+        close(y, want + resid.double())
+        close(ext().dq_gateup_scaled(x, scale, *p, bits, g), gated(want), 1e-2)
+    return names
+
+
 @pytest.mark.parametrize("m,n,k,g", [
     (40, 10240, 256, 128), (48, 8200, 2112, 64), (33, 32008, 192, 64),
     (49, 3072, 1024, 64), (64, 2056, 2048, 128), (77, 16384, 2048, 64),
@@ -342,24 +366,7 @@ def test_eight_waves_along_k(m, n, k, g):
     2 and 4 waves side by side, parts of k and none, groups that the waves do
     not share evenly, columns that end inside a wave's; bias, residual, gate
     and factors of rows."""
-    torch.manual_seed(n + m)
-    p, w = matrix(8, n, k, g)
-    x = torch.randn(m, k, device=DEV).to(BF)
-    x[0] = 0
-    bias = torch.randn(n, device=DEV).to(BF)
-    plain = x.double() @ w.t()
-    assert "dq_mid_kernel" in launched(lambda: close(
-        ext().dq_linear(x, *p, 8, g, bias, None, -1.0, 0), plain + bias.double()))
-    close(ext().dq_gemv_gateup(x, *p, 8, g, -1.0, 0), gated(plain), 1e-2)
-    if m <= 48:
-        resid = torch.randn(m, n, device=DEV).to(BF)
-        scale = torch.rand(m, device=DEV) + 0.5
-        close(ext().dq_linear(x, *p, 8, g, bias, resid, -1.0, 0),
-              plain + bias.double() + resid.double())
-        want = plain * scale.double().unsqueeze(1)
-        y, _ = ext().dq_linear_scaled(x, scale, *p, 8, g, None, resid, 1e-5)
-        close(y, want + resid.double())
-        close(ext().dq_gateup_scaled(x, scale, *p, 8, g), gated(want), 1e-2)
+    assert "dq_mid_kernel" in with_its_ways(8, m, n, k, g)
 
 
 @pytest.mark.parametrize("m,n,k,g", [
@@ -373,22 +380,22 @@ def test_eight_waves_along_k_of_four_bits(m, n, k, g):
     """The same of 4 bits, whose sums of x waves side by side share and add two
     steps later: one and two steps a group, one turn and many, last turns with
     fewer groups than waves, more row tiles than waves side by side and fewer."""
-    torch.manual_seed(n + m)
-    p, w = matrix(4, n, k, g)
-    x = torch.randn(m, k, device=DEV).to(BF)
-    x[0] = 0
-    bias = torch.randn(n, device=DEV).to(BF)
-    plain = x.double() @ w.t()
-    assert "dq_mid_kernel" in launched(lambda: close(
-        ext().dq_linear(x, *p, 4, g, bias, None, -1.0, 0), plain + bias.double()))
-    close(ext().dq_gemv_gateup(x, *p, 4, g, -1.0, 0), gated(plain), 1e-2)
-    if m <= 48:
-        resid = torch.randn(m, n, device=DEV).to(BF)
-        scale = torch.rand(m, device=DEV) + 0.5
-        want = plain * scale.double().unsqueeze(1)
-        y, _ = ext().dq_linear_scaled(x, scale, *p, 4, g, None, resid, 1e-5)
-        close(y, want + resid.double())
-        close(ext().dq_gateup_scaled(x, scale, *p, 4, g), gated(want), 1e-2)
+    assert "dq_mid_kernel" in with_its_ways(4, m, n, k, g)
+
+
+@pytest.mark.parametrize("bits,m,n,k,g", [
+    (8, 17, 5120, 256, 128), (8, 32, 6136, 1024, 64), (8, 32, 6144, 1024, 64),
+    (8, 25, 8192, 768, 128), (8, 25, 8200, 768, 128), (8, 17, 8192, 2048, 64),
+    (8, 17, 8200, 2048, 64), (8, 64, 28664, 1024, 64), (8, 64, 28672, 1024, 64),
+    (8, 50, 28672, 2112, 64), (8, 96, 24576, 2112, 64), (8, 65, 24584, 2112, 64),
+    (8, 32, 32768, 512, 64), (8, 32, 32776, 512, 64), (8, 32, 32776, 512, 128),
+    (8, 48, 32776, 1216, 64), (8, 33, 32776, 1280, 64), (8, 65, 32776, 1472, 64),
+    (8, 65, 32776, 1536, 64), (4, 25, 1024, 768, 64), (4, 90, 8200, 896, 128),
+    (4, 200, 4104, 4096, 128), (8, 700, 4100, 6912, 64)])
+def test_some_tens_of_rows_by_any_kernel(bits, m, n, k, g):
+    """Sizes about the edges of several kernels' ranges, which one of them has at a
+    time: all that goes with a product is taken there by whichever it is."""
+    with_its_ways(bits, m, n, k, g)
 
 
 @pytest.mark.parametrize("bits,m,n,k,g", [
