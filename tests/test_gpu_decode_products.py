@@ -465,14 +465,8 @@ def test_eight_waves_at_the_lines(call, taken):
     close(got[0], gated(want) if gate else want, 1e-2 if gate else 5e-3)
 
 
-@torch.no_grad()
-@pytest.mark.parametrize("batch,heads,hidden,inner", [
-    (8, 32, 4096, 14336), (3, 48, 6144, 8192), (16, 32, 2048, 20480)])
-def test_a_step_whose_down_projection_is_in_parts(batch, heads, hidden, inner,
-                                                  monkeypatch):
-    """Its counters are those of decode attention, in each layer and in a graph's
-    replays; results to the bit, as a layer's launches are the same then."""
-    T = 300
+def step_of(batch, heads, hidden, inner, T=300):
+    """A cache of T keys, and a decode step behind it of two layers of 4 bits."""
     torch.manual_seed(hidden)
     with torch.device(DEV):
         cfg = LlamaConfig(vocab_size=512, hidden_size=hidden, intermediate_size=inner,
@@ -488,7 +482,17 @@ def test_a_step_whose_down_projection_is_in_parts(batch, heads, hidden, inner,
         t[:, :, :, :T].normal_()
     state = torch.tensor([T, T + 1, 0], dtype=torch.int32, device=DEV)
     ids = torch.randint(512, (batch, 1), device=DEV)
-    step = lambda: m.forward_decode_step(ids, cache, state, T + 8)
+    return cache, lambda: m.forward_decode_step(ids, cache, state, T + 8)
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("batch,heads,hidden,inner", [
+    (8, 32, 4096, 14336), (3, 48, 6144, 8192), (16, 32, 2048, 20480)])
+def test_a_step_whose_down_projection_is_in_parts(batch, heads, hidden, inner,
+                                                  monkeypatch):
+    """Its counters are those of decode attention, in each layer and in a graph's
+    replays; results to the bit, as a layer's launches are the same then."""
+    cache, step = step_of(batch, heads, hidden, inner)
     step()
     found = []
     parts = F.dq_linear_parts
@@ -516,3 +520,15 @@ def test_a_step_whose_down_projection_is_in_parts(batch, heads, hidden, inner,
     # roundings of 2^-9 in two layers' products and the head's
     assert not torch.equal(plain, want)
     assert float((plain.double() - want.double()).norm() / want.double().norm()) < 2e-2
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("batch,inner", [(8, 8192), (3, 16256), (2, 20480)])
+def test_a_step_asks_for_parts_only_where_there_may_be_some(batch, inner, monkeypatch):
+    """A step of two layers of 2048 without a graph waits for the host, which the
+    question takes 5 us a layer."""
+    _, step = step_of(batch, 16, 2048, inner)
+    asked = []
+    monkeypatch.setattr(F, "dq_linear_parts", lambda *a: asked.append(1))
+    step()
+    assert not asked
