@@ -93,7 +93,9 @@ def takes_factors(p: QLinear) -> bool:
     """Whether a norm in front of p is worth a launch of its own for 17 to 48
     rows: where a product without it may be `dq_mid`'s or `dq_short`'s.  A step of
     four layers of 2048, 4 bits: 17 rows 217 us with it, 219 without (groups of 64
-    230 and 238), 48 rows 255 and 260; 8 bits 228 and 231 at 17."""
+    230 and 238), 32 rows 216 and 230, 48 rows 249 and 261; 8 bits 228 and 231 at 17.
+    In a graph, that is: one by one the launches cost the host 4 us a layer (20 rows
+    347 and 330)."""
     return p.bits == 8 or p.in_features >= 2048
 
 
